@@ -108,6 +108,7 @@ int tl_scratch(int slot, size_t bytes, void** out) {
     void* p = nullptr;
     TL_HIP(hipMalloc(&p, bytes));
     TL_HIP(hipMemset(p, 0, bytes));
+    TL_HIP(hipDeviceSynchronize());  // the caller's stream need not be ordered behind the null stream the clear runs on
     e = {p, bytes};
   }
   *out = e.first;
