@@ -321,3 +321,29 @@ def test_prefill_attention_writes_the_gemm_planes_bit_identically(E, pkg, monkey
             m.free()
         for a, b in zip(got["0"], got["1"]):
             assert a.shape == b.shape and np.array_equal(a, b), (shape, np.abs(a - b).max())
+
+
+@pytest.mark.parametrize("name,rows,cols,T", [
+    ("q4_k", 1, 256, 8), ("q4_k", 65, 512, 16), ("q4_k", 129, 4096, 17), ("q4_k", 300, 14336, 32), ("q6_k", 63, 256, 9),
+    ("q6_k", 130, 2304, 16), ("q6_k", 97, 768, 31), ("q8_0", 31, 64, 8), ("q8_0", 70, 320, 13), ("q8_0", 129, 448, 27),
+    ("q8_0", 64, 1088, 32), ("q8_k", 127, 512, 11), ("q8_k", 33, 1280, 30)])
+def test_half_plane_gemm_edges(E, pkg, name, rows, cols, T):
+    """tl_hgemm.hip through tl_matmul_q (16- and 32-token tiles): rows and tokens off the tiles, one and several super-blocks,
+    K slices, Q8_0 rows that end inside a super-block; magnitudes 2^-20 .. 2^20 apart from super-block to super-block and
+    rows of zeros. Against float64 over the dequantized weights: an activation is held to 2^-22 of its super-block's largest
+    value at worst, a running sum of 256 products is rounded 16 to 48 times (2^-24 each), their sum once per super-block: with
+    |w| . |x| as the scale of a row's dot, 2^-22 + 48 * 2^-24 + (cols / 256) * 2^-24 bounds the error; measured a tenth."""
+    t, S = TYPES[name], pkg.synth
+    rng = np.random.default_rng(rows + 7 * cols + T)
+    w = E.QWeight(t, S.random_blocks(t, rows * cols // S.BLOCK_ELEMS[t], rng, w_std=1.0 / np.sqrt(cols)), rows, cols)
+    x = rng.standard_normal((T, cols)).astype(np.float32)
+    x *= np.exp2(rng.integers(-20, 21, (T, -(-cols // 256)))).astype(np.float32).repeat(256, axis=1)[:, :cols]
+    x[T // 2] = 0.0
+    W = w.dequantize().astype(np.float64)
+    want = x.astype(np.float64) @ W.T
+    # (Q4_K: the scale q and minimum m parts are summed apart, their sizes are what rounds)
+    scale = np.abs(x).astype(np.float64) @ (np.abs(W) + 4.0 * np.abs(W).max(axis=1, keepdims=True)).T
+    y = _matmul(E, w, x)
+    assert (np.abs(y - want) <= (2.0 ** -22 + 48 * 2.0 ** -24 + cols / 256 * 2.0 ** -24) * scale).all(), (np.abs(y - want) / np.maximum(scale, 1e-30)).max()
+    assert not y[T // 2].any()
+    w.free()

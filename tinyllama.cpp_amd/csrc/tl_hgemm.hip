@@ -1,0 +1,760 @@
+// tl_hgemm.hip — batched GEMM over the quantized plane layout with f16 matrix instructions:
+//   Y[T][rows] (+ resid) = X[T][cols] . W[rows][cols]^T      for the batched paths (prompts, multi-sequence steps)
+//
+// The same product as tl_gemm.hip's kernels (smart_gemm_batch_cuda, model.cpp:2141-2249; numerics target
+// matmul_f32_f32_batch_cpu, utils.cpp:730-782) at the same 32-bit grade, with fewer matrix instructions and fewer vector
+// instructions per weight:
+//   - an activation is held as two f16 parts of x * 2^k, k chosen per token and super-block (256 columns) so that the
+//     largest value there lies in [2^9, 2^10): x = hi + lo to 22 bits and sign, and to 2^-35 of that largest value where lo
+//     is sub-normal. Two matrix instructions per weight operand instead of the three that bf16 parts need;
+//   - what a weight operand holds is exact in f16, which has 11 bits: Q4_K's sub-block scale times the nibble (<= 945), the
+//     bytes of Q8, and of Q6_K the product scale * q (13 bits) as a rounded part plus its remainder. A running sum
+//     therefore spans a whole 256-column super-block (Q8_0: a 32-column block) before a vector FMA applies the
+//     super-block's factor to it: 16 FMAs per 33 matrix instructions (Q4_K) where integer operands need 16 per 3;
+//   - Q4_K's minima: sum_j m_j * (sum of x over sub-block j) is one more K = 16 matrix instruction per super-block, with
+//     the eight sub-block sums' two f16 parts side by side along K and the same eight m_j against either half.
+// Weights go from HBM straight into registers (a super-block ahead), are unpacked there and never touch LDS; the
+// activation tile is staged through LDS, a super-block ahead as well, with one barrier per super-block.
+//
+// The order of the columns inside an operand is free as long as both sides agree. Lane half h of a Q4_K / Q6_K step takes
+// the 32-weight chunk 2 s + h (one 16-byte load), of a Q8 step 16 of the 32 bytes of a chunk; the eight columns of an
+// operand are in the order [0 2 1 3 4 6 5 7], which is what masking a dword into 16-bit halves gives without moving a
+// byte, and which the activation planes are written in.
+#include <type_traits>
+
+#include "tl_internal.h"
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+
+namespace {
+
+// ---- activation planes: [2][ps] f16 (hi, lo), then per super-block the block sums [cols / 256][tpad][hi 8 | lo 8] f16,
+//      then 2^-k [cols / 256][tpad] (tpad: padded tokens)
+struct HAct {
+  const _Float16* x;
+  size_t ps;
+  const _Float16* bs;
+  const float* inv;
+  int tpad;
+};
+inline HAct hact(const void* planes, size_t ps, int T) {
+  const _Float16* x = static_cast<const _Float16*>(planes);
+  const _Float16* bs = x + 2 * ps;
+  return HAct{x, ps, bs, reinterpret_cast<const float*>(bs + ps / 16), (int)tl_gemm_padded_tokens(T)};
+}
+
+__device__ __forceinline__ float h2f(unsigned h) { return (float)__builtin_bit_cast(_Float16, (unsigned short)h); }
+__device__ __forceinline__ float h2f_scale(unsigned h) {  // |d| for finite negatives (quantization.cpp:85-87)
+  const float d = h2f(h);
+  return (d < 0.0f && d > -INFINITY) ? -d : d;
+}
+__device__ __forceinline__ f16x2 as_h2(unsigned u) { return __builtin_bit_cast(f16x2, u); }
+__device__ __forceinline__ f16x2 h2(float v) { return f16x2{(_Float16)v, (_Float16)v}; }
+__device__ __forceinline__ f16x8 join(f16x2 a, f16x2 b, f16x2 c, f16x2 d) {
+  return f16x8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+}
+
+// A matrix instruction covers TK tokens x TK weight rows: 32 x 32 x 16 columns, or 16 x 16 x 32 for 16 tokens and fewer. The
+// 64 / TK = NG lane groups hold eight columns each.
+template <int TK>
+struct Tile {
+  typedef f32x16 Acc;
+  static constexpr int E = 16;
+  static __device__ __forceinline__ Acc mfma(f16x8 a, f16x8 b, Acc c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
+  static __device__ __forceinline__ int quad(int q, int g) { return 8 * q + 4 * g; }  // token of element 4 q
+};
+template <>
+struct Tile<16> {
+  typedef f32x4 Acc;
+  static constexpr int E = 4;
+  static __device__ __forceinline__ Acc mfma(f16x8 a, f16x8 b, Acc c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+  static __device__ __forceinline__ int quad(int, int g) { return 4 * g; }
+};
+
+// what one lane holds of a step (NG 32-weight chunks of one row, four operands), and of a super-block
+template <int TYPE>
+struct WStep {
+  u32x4 q;       // Q4_K / Q6_K: chunk NG u + group; Q8: the lane's eight bytes of operands 0 and 1
+  u32x4 q1;      // Q8: of operands 2 and 3
+  u32x2 hi;      // Q6_K: high bits of the chunk
+  unsigned d[2]; // Q8_0: d of the step's chunks
+};
+template <int TYPE>
+struct WHead {
+  u32x4 h;     // Q4_K: super-block header; Q6_K: the 16 sub-block scales
+  unsigned d;  // Q6_K / Q8_K: d
+};
+// step u of super-block sb; steps past the end of a Q8_0 row (not a whole number of super-blocks) read its last chunks
+template <int TYPE, int TK>
+__device__ __forceinline__ void load_step(WStep<TYPE>& g, const QW& w, unsigned R, int sb, int u, int fg) {
+  constexpr int NG = 64 / TK;
+  const unsigned K = (unsigned)w.cols;
+  if (TYPE == TL_Q4_K || TYPE == TL_Q6_K) {
+    const unsigned c = sb * 8 + NG * u + fg;
+    g.q = *reinterpret_cast<const u32x4*>(w.p0 + (size_t)(R * (K >> 1) + c * 16));
+    if (TYPE == TL_Q6_K) g.hi = *reinterpret_cast<const u32x2*>(w.p1 + (size_t)(R * (K >> 2) + c * 8));
+  } else {
+    const unsigned last = (K >> 6) - 1;  // (pairs of chunks: K is a multiple of 64)
+    const unsigned s = (TK == 32 ? sb * 4 + u : sb * 4 + 2 * u), s0 = s < last ? s : last, s1 = s + 1 < last ? s + 1 : last;
+    if (TK == 32) {
+      g.q = *reinterpret_cast<const u32x4*>(w.p0 + (size_t)(R * K + s0 * 64 + fg * 16));
+      g.q1 = *reinterpret_cast<const u32x4*>(w.p0 + (size_t)(R * K + s0 * 64 + fg * 16 + 32));
+    } else {
+      const u32x2 a = *reinterpret_cast<const u32x2*>(w.p0 + (size_t)(R * K + s0 * 64 + fg * 8));
+      const u32x2 b = *reinterpret_cast<const u32x2*>(w.p0 + (size_t)(R * K + s0 * 64 + fg * 8 + 32));
+      const u32x2 c = *reinterpret_cast<const u32x2*>(w.p0 + (size_t)(R * K + s1 * 64 + fg * 8));
+      const u32x2 d = *reinterpret_cast<const u32x2*>(w.p0 + (size_t)(R * K + s1 * 64 + fg * 8 + 32));
+      g.q = u32x4{a[0], a[1], b[0], b[1]};
+      g.q1 = u32x4{c[0], c[1], d[0], d[1]};
+    }
+    if (TYPE == TL_Q8_0) {
+      g.d[0] = *reinterpret_cast<const unsigned*>(w.p1 + (size_t)((R * (K >> 5) + 2 * s0) * 2));
+      if (TK == 16) g.d[1] = *reinterpret_cast<const unsigned*>(w.p1 + (size_t)((R * (K >> 5) + 2 * s1) * 2));
+    }
+  }
+}
+template <int TYPE>
+__device__ __forceinline__ void load_head(WHead<TYPE>& g, const QW& w, unsigned R, int sb) {
+  const unsigned K = (unsigned)w.cols;
+  if (TYPE == TL_Q4_K) g.h = *reinterpret_cast<const u32x4*>(w.p1 + (size_t)(R * (K >> 4) + sb * 16));
+  if (TYPE == TL_Q6_K) {
+    g.h = *reinterpret_cast<const u32x4*>(w.p2 + (size_t)(R * (K >> 4) + sb * 16));
+    g.d = *reinterpret_cast<const uint16_t*>(w.p3 + (size_t)((R * (K >> 8) + sb) * 2));
+  }
+  if (TYPE == TL_Q8_K) g.d = *reinterpret_cast<const uint16_t*>(w.p1 + (size_t)((R * (K >> 8) + sb) * 2));
+}
+
+// the eight weights of operand w (0..3) of step u (0..3 inside the super-block), in operand order
+constexpr unsigned MAGIC = 0x64006400u;  // f16 1024: a small integer or-ed into the mantissa is 1024 + itself
+// (v & mask) | MAGIC in one instruction: v_and_or_b32 takes no literals, so both constants have to sit in registers
+__device__ __forceinline__ unsigned pick(unsigned v, unsigned mask) {
+  unsigned r;
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(mask), "v"(MAGIC));
+  return r;
+}
+struct Scale4 {
+  f16x2 c, cn, c16, cn16;  // sc, -1024 sc, sc / 16, -64 sc
+};
+__device__ __forceinline__ Scale4 q4_scale(unsigned h1, unsigned h3, int c) {  // h1, h3 already shifted to the lane group's chunk
+  const unsigned sc = ((h1 >> (4 * c)) & 15u) | (((h3 >> (2 * c)) & 3u) << 4);
+  Scale4 r;
+  r.c = as_h2(sc | (sc << 16) | MAGIC) - h2(1024.f);
+  r.cn = r.c * h2(-1024.f);
+  r.c16 = r.c * h2(0.0625f);
+  r.cn16 = r.c * h2(-64.f);
+  return r;
+}
+__device__ __forceinline__ f16x8 q4_operand(unsigned u, const Scale4& s) {
+  const unsigned v = u >> 8;
+  // (1024 + q) sc - 1024 sc and (1024 + 16 q) sc / 16 - 64 sc: one rounding each, of a value that needs none
+  return join(__builtin_elementwise_fma(as_h2(pick(u, 0x000F000Fu)), s.c, s.cn),
+              __builtin_elementwise_fma(as_h2(pick(v, 0x000F000Fu)), s.c, s.cn),
+              __builtin_elementwise_fma(as_h2(pick(u, 0x00F000F0u)), s.c16, s.cn16),
+              __builtin_elementwise_fma(as_h2(pick(v, 0x00F000F0u)), s.c16, s.cn16));
+}
+// the minima m_0..m_7 of a super-block in the order [0 4 1 5 2 6 3 7] (the block sums' order)
+__device__ __forceinline__ f16x8 q4_minima(unsigned m_lo, unsigned hi) {
+  const unsigned hh = ((hi >> 16) & 0xFFu) | ((hi >> 8) & 0x00FF0000u);
+  f16x2 r[4];
+#pragma unroll
+  for (int p = 0; p < 4; ++p) r[p] = as_h2(((m_lo >> (4 * p)) & 0x000F000Fu) | (((hh >> (2 * p)) & 0x00030003u) << 4) | MAGIC) - h2(1024.f);
+  return join(r[0], r[1], r[2], r[3]);
+}
+__device__ __forceinline__ void q6_operand(unsigned u, unsigned hv, int odd, f16x2 sc, f16x8& hi, f16x8& lo) {
+  f16x2 a[4], b[4];
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {  // pairs (0 2) (1 3) (4 6) (5 7): byte shift 8 (p & 1), part p >> 1
+    // low nibbles to bits 0..3, high bits to bits 4..5 of the 16-bit halves
+    const int at = 8 * (p & 1) + 2 * (2 * odd + (p >> 1)) - 4;
+    const unsigned h = pick(at < 0 ? hv << -at : hv >> at, 0x00300030u);
+    unsigned l = u >> (8 * (p & 1) + 4 * (p >> 1));
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(l) : "v"(l), "s"(0x000F000Fu), "v"(h));
+    const f16x2 q = as_h2(l) - h2(1056.f);
+    a[p] = q * sc;                                      // 13 bits rounded to 11
+    b[p] = __builtin_elementwise_fma(q, sc, -a[p]);     // the remainder, exact
+  }
+  hi = join(a[0], a[1], a[2], a[3]);
+  lo = join(b[0], b[1], b[2], b[3]);
+}
+__device__ __forceinline__ f16x8 q8_operand(unsigned a, unsigned b) {
+  const unsigned x = a ^ 0x80808080u, y = b ^ 0x80808080u;
+  const f16x2 off = h2(1152.f);
+  return join(as_h2(pick(x, 0x00FF00FFu)) - off, as_h2(pick(x >> 8, 0x00FF00FFu)) - off,
+              as_h2(pick(y, 0x00FF00FFu)) - off, as_h2(pick(y >> 8, 0x00FF00FFu)) - off);
+}
+
+struct HSegs {  // up to three matrices over the same activations (q | k | v, gate | up): row tiles follow each other
+  QW w[3];
+  float* y[3];
+  int mt_end[3];
+};
+
+// Workgroup: NW waves of TK MI rows each x TK NI tokens. LDS: two buffers of a super-block's activation tile, [4 x 64
+// columns][2 parts][tokens][64] f16, the 16-byte pieces of a token's 128 bytes at piece ^ (token / 2 & 7): the 16
+// consecutive tokens of a fragment read and the 2 x 8 pieces of a staging write cover the 64 banks once; behind them the
+// super-block's block sums and powers of two.
+template <int TYPE, int TK, int NI, int MI, int NW, int WPE>
+__global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct act, const float* __restrict__ resid, int T, int mtiles,
+                                                           int ntiles, int nslices) {
+  typedef Tile<TK> TL;
+  typedef typename TL::Acc Acc;
+  constexpr int NG = 64 / TK, US = 8 / NG;                        // lane groups, steps of a super-block
+  constexpr int BN = TK * NI, NT = 64 * NW, STEP = 2 * BN * 64;   // STEP: halfs of 64 columns
+  constexpr int XR = 2 * BN * 8 / NT;                             // 16-byte pieces of 64 columns per thread
+  constexpr int AUXH = 18 * BN;                                   // halfs of a super-block's block sums and 2^-k (float)
+  constexpr int BUF = 4 * STEP + AUXH;                            // !RINGED: halfs of a buffer
+  constexpr bool CHUNKED = TYPE == TL_Q4_K || TYPE == TL_Q6_K;
+  constexpr bool RINGED = BN > 32;                                // the tile goes through a ring of three 64-column steps
+  extern __shared__ __attribute__((aligned(16))) _Float16 hlds[];
+  // consecutive workgroups go to the 8 XCDs in turn: each XCD walks a contiguous range, token tiles fastest, so that the
+  // workgroups that read the same weights share an L2
+  const int total = mtiles * ntiles * nslices, per8 = total >> 3, rem8 = total & 7;
+  const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+  const int v = xcd * per8 + (xcd < rem8 ? xcd : rem8) + at;
+  const int nt = v % ntiles, rest = v / ntiles;
+  int mt = rest % mtiles;
+  const int slice = rest / mtiles;
+  const int seg = (mt >= segs.mt_end[0]) + (mt >= segs.mt_end[1]);
+  if (seg) mt -= segs.mt_end[seg - 1];
+  const QW w = segs.w[seg];
+  float* __restrict__ y = segs.y[seg];
+  const int M = w.rows, K = w.cols;
+  const int nsb_all = (K + 255) >> 8, per = (nsb_all + nslices - 1) / nslices;
+  const int sb0 = slice * per, nsb = nsb_all - sb0 < per ? nsb_all - sb0 : per;
+  const int slast = K / 64 - 1;
+  if (nslices > 1) y += (size_t)slice * (size_t)T * (size_t)M;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int fr = lane & (TK - 1), fg = lane / TK;
+  const int n0 = nt * BN, m0 = mt * (TK * MI * NW) + wave * (TK * MI);
+  unsigned R[MI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int r = m0 + TK * i + fr;
+    R[i] = (unsigned)(r < M ? r : M - 1);
+  }
+  // staging: this thread's pieces of 64 columns (padding tokens repeat the last one: lines that are read anyway)
+  unsigned xg[XR];
+  int xl[XR];
+#pragma unroll
+  for (int r = 0; r < XR; ++r) {
+    const int id = tid + r * NT, q = id & 7, row = id >> 3, tok = row % BN, part = row / BN;
+    xg[r] = (unsigned)((size_t)part * act.ps + (size_t)(n0 + tok < T ? n0 + tok : T - 1) * K + q * 8);
+    xl[r] = row * 64 + ((q ^ ((tok >> 1) & 7)) << 3);
+  }
+  auto load_x = [&](int r, int sb, int c) {  // 64-column piece c of super-block sb
+    const int s = sb * 4 + c;
+    return *reinterpret_cast<const f16x8*>(act.x + (size_t)(xg[r] + (unsigned)((s < slast ? s : slast) * 64)));
+  };
+  // 16-byte pieces of a super-block's block sums (2 BN) and powers of two (BN / 4); spare threads copy a piece again
+  constexpr int AUX = 2 * BN + BN / 4;
+  const int ap = tid % AUX;
+  const unsigned char* ag = ap < 2 * BN ? reinterpret_cast<const unsigned char*>(act.bs + (size_t)n0 * 16) + ap * 16
+                                        : reinterpret_cast<const unsigned char*>(act.inv + n0) + (ap - 2 * BN) * 16;
+  const size_t astride = (size_t)act.tpad * (ap < 2 * BN ? 32 : 4);
+  // fragment reads: where the lane's eight columns of operand k lie in a step's part of the tile
+  int xo[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int col = CHUNKED ? 32 * fg + 8 * k : TK == 32 ? 32 * (k >> 1) + 16 * fg + 8 * (k & 1) : 32 * k + 8 * fg;
+    xo[k] = (col >> 6) * STEP + fr * 64 + ((((col & 63) >> 3) ^ ((fr >> 1) & 7)) << 3);
+  }
+
+  constexpr bool APART = MI == 1;
+  constexpr int WD = US == 4 && NI * MI == 4 ? 2 : US;  // steps the weight loads run ahead: a super-block
+  WStep<TYPE> W[MI][WD];
+  WHead<TYPE> H[MI], Hn[MI];
+  // (in the order in which the first super-block waits for them: the counted waits of the loop depend on it)
+#pragma unroll
+  for (int i = 0; i < MI; ++i) load_head<TYPE>(H[i], w, R[i], sb0);
+  {
+    const u32x4 aux = *reinterpret_cast<const u32x4*>(ag + (size_t)sb0 * astride);
+    constexpr int FIRST = RINGED ? 2 : 4;
+    f16x8 xr[FIRST][XR];
+#pragma unroll
+    for (int c = 0; c < FIRST; ++c)
+#pragma unroll
+      for (int r = 0; r < XR; ++r) xr[c][r] = load_x(r, sb0, c);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < WD; ++u)
+#pragma unroll
+      for (int i = 0; i < MI; ++i) load_step<TYPE, TK>(W[i][u], w, R[i], sb0, u, fg);
+    __builtin_amdgcn_sched_barrier(0);
+    *reinterpret_cast<u32x4*>(hlds + (RINGED ? 3 : 4) * STEP + ap * 8) = aux;
+#pragma unroll
+    for (int c = 0; c < FIRST; ++c)
+#pragma unroll
+      for (int r = 0; r < XR; ++r) *reinterpret_cast<f16x8*>(hlds + c * STEP + xl[r]) = xr[c][r];
+  }
+  int slot = 0;  // RINGED: where the step in hand lies
+  const Acc zero = {};
+  Acc acc[NI][MI];
+#pragma unroll
+  for (int n = 0; n < NI; ++n)
+#pragma unroll
+    for (int i = 0; i < MI; ++i) acc[n][i] = zero;
+  __syncthreads();
+
+  auto superblock = [&](int b, auto next_c) __attribute__((always_inline)) {
+    constexpr bool NEXT = decltype(next_c)::value;  // another super-block follows: fetch it on the way
+    const int sb = sb0 + b, cur = b & 1;
+    const _Float16* xb = hlds + cur * BUF;
+    _Float16* xn = hlds + (cur ^ 1) * BUF;
+    const _Float16* ab = RINGED ? hlds + 3 * STEP + cur * AUXH : xb + 4 * STEP;
+    _Float16* an = RINGED ? hlds + 3 * STEP + (cur ^ 1) * AUXH : xn + 4 * STEP;
+    u32x4 aux;
+    if (NEXT) {
+      aux = *reinterpret_cast<const u32x4*>(ag + (size_t)(sb + 1) * astride);
+#pragma unroll
+      for (int i = 0; i < MI; ++i) load_head<TYPE>(Hn[i], w, R[i], sb + 1);
+    }
+    // sums of the hi part's products and of the small ones (lo part; Q6_K's remainders): apart where registers are not
+    // short, so that only the former's 16 additions round at the sum's own size, and as two chains. Q8_0: of a 32-column
+    // block, c8 adds up the blocks
+    Acc t[NI][MI], tl[NI][MI], c8[NI][MI];
+    f16x8 xr[RINGED ? 1 : 4][XR];
+    unsigned h1[MI], h3[MI];
+    if (TYPE == TL_Q4_K) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        h1[i] = H[i].h[1] >> (4 * fg);
+        h3[i] = H[i].h[3] >> (2 * fg);
+      }
+    }
+    // fragment reads run RD operands ahead of their matrix instructions. The compiler's scheduler would sink every load to
+    // its use (measured: all of a super-block's loads behind its last matrix instruction); the barriers keep them here
+    constexpr int RD = NI == 1 ? 3 : MI == 1 ? 2 : 1, RING = RD + 1, NF = 4 * US * NI;
+    f16x8 fa[RING][2];
+    auto read_frags = [&](int f, int u) __attribute__((always_inline)) {  // in step u: operand f / NI, token fragment f % NI
+      const int kk = f / NI, n = f % NI;
+      const _Float16* base = !RINGED ? xb + (kk >> 2) * (NG / 2) * STEP
+                                     : hlds + ((kk >> 2) == u ? slot : slot == 2 ? 0 : slot + 1) * STEP;
+#pragma unroll
+      for (int p = 0; p < 2; ++p) fa[f % RING][p] = *reinterpret_cast<const f16x8*>(base + (p * BN + TK * n) * 64 + xo[kk & 3]);
+    };
+#pragma unroll
+    for (int f = 0; f < RD; ++f) read_frags(f, 0);
+#pragma unroll
+    for (int u = 0; u < US; ++u) {
+      if (RINGED && (NEXT || u + 2 < US)) {  // two steps on
+#pragma unroll
+        for (int r = 0; r < XR; ++r) xr[0][r] = load_x(r, sb, u + 2);
+      } else if (NEXT && u == 0) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int r = 0; r < XR; ++r) xr[c][r] = load_x(r, sb + 1, c);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      Scale4 sc[MI];
+      f16x2 s6[MI][2];
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        if (TYPE == TL_Q4_K) sc[i] = q4_scale(h1[i], h3[i], NG * u);
+        if (TYPE == TL_Q6_K) {
+          const unsigned hs = NG == 2 ? H[i].h[u] : (fg & 2) ? H[i].h[(2 * u + 1) & 3] : H[i].h[(2 * u) & 3];
+          const unsigned sw = hs >> (16 * (fg & 1));
+          const _Float16 a = (_Float16)(short)(signed char)(sw & 0xFFu), c = (_Float16)(short)(signed char)((sw >> 8) & 0xFFu);
+          s6[i][0] = f16x2{a, a};
+          s6[i][1] = f16x2{c, c};
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int kk = 4 * u + k;
+        f16x8 bh[MI], bl[MI];
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+          const WStep<TYPE>& g = W[i][u % WD];
+          if (TYPE == TL_Q4_K) bh[i] = q4_operand(g.q[k], sc[i]);
+          else if (TYPE == TL_Q6_K) q6_operand(g.q[k], g.hi[k >> 1], k & 1, s6[i][k >> 1], bh[i], bl[i]);
+          else bh[i] = k < 2 ? q8_operand(g.q[2 * (k & 1)], g.q[2 * (k & 1) + 1]) : q8_operand(g.q1[2 * (k & 1)], g.q1[2 * (k & 1) + 1]);
+        }
+        // Q8_0: a 32-column block is two operands (TK 32) or one (TK 16)
+        const bool fresh = TYPE == TL_Q8_0 ? TK == 16 || (k & 1) == 0 : kk == 0;
+#pragma unroll
+        for (int n = 0; n < NI; ++n) {
+          const int f = kk * NI + n;
+          __builtin_amdgcn_sched_barrier(0);
+          if (f + RD < NF) read_frags(f + RD, u);
+          __builtin_amdgcn_sched_barrier(0);
+          const f16x8 a0 = fa[f % RING][0], a1 = fa[f % RING][1];
+#pragma unroll
+          for (int i = 0; i < MI; ++i) {
+            Acc& c = APART ? tl[n][i] : t[n][i];
+            c = TL::mfma(a1, bh[i], fresh ? zero : c);
+          }
+#pragma unroll
+          for (int i = 0; i < MI; ++i) t[n][i] = TL::mfma(a0, bh[i], APART && fresh ? zero : t[n][i]);
+          if (TYPE == TL_Q6_K) {
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+              Acc& c = APART ? tl[n][i] : t[n][i];
+              c = TL::mfma(a0, bl[i], c);
+            }
+          }
+        }
+        if (TYPE == TL_Q8_0 && (TK == 16 || (k & 1))) {
+          const int blk = TK == 16 ? 4 * u + k : 2 * u + (k >> 1), pair = TK == 16 ? k >> 1 : 0;  // block of the super-block
+          const unsigned live = sb * 4 + (blk >> 1) <= slast ? 0xFFFFu : 0u;  // (the row may end inside the super-block)
+#pragma unroll
+          for (int i = 0; i < MI; ++i) {
+            const float d = h2f_scale((W[i][u % WD].d[pair] >> (16 * (blk & 1))) & live);
+#pragma unroll
+            for (int n = 0; n < NI; ++n) {
+#pragma unroll
+              for (int e = 0; e < TL::E; ++e) {
+                const float c = APART ? t[n][i][e] + tl[n][i][e] : t[n][i][e];
+                c8[n][i][e] = blk == 0 ? d * c : fmaf(d, c, c8[n][i][e]);
+              }
+              asm volatile("" : "+v"(c8[n][i]));  // here, not behind the loop (eight blocks' sums would stay live)
+            }
+          }
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (NEXT || u + WD < US) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) load_step<TYPE, TK>(W[i][u % WD], w, R[i], sb + (u + WD) / US, (u + WD) % US, fg);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (RINGED) {
+        if (NEXT || u + 2 < US) {  // into the slot that everybody left at the last barrier
+#pragma unroll
+          for (int r = 0; r < XR; ++r) *reinterpret_cast<f16x8*>(hlds + (slot == 0 ? 2 : slot - 1) * STEP + xl[r]) = xr[0][r];
+        }
+        slot = slot == 2 ? 0 : slot + 1;
+        if (u < US - 1) __syncthreads();
+      } else if (NEXT && u == US - 1) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int r = 0; r < XR; ++r) *reinterpret_cast<f16x8*>(xn + c * STEP + xl[r]) = xr[c][r];
+      }
+    }
+    // the super-block's sums times the rows' factors and the tokens' powers of two
+    float d[MI], dm[MI];
+    f16x8 mn[MI];
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      d[i] = TYPE == TL_Q4_K ? h2f(H[i].h[0] & 0xFFFFu) : TYPE == TL_Q6_K ? h2f(H[i].d) : TYPE == TL_Q8_K ? h2f_scale(H[i].d) : 1.f;
+      if (TYPE == TL_Q4_K) {
+        mn[i] = q4_minima(H[i].h[2], H[i].h[3]);
+        dm[i] = -h2f(H[i].h[0] >> 16);
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < NI; ++n) {
+      f16x8 bs;
+      if (TYPE == TL_Q4_K) {
+        bs = *reinterpret_cast<const f16x8*>(ab + (TK * n + fr) * 16 + (fg & 1) * 8);
+        if (NG == 4 && fg >= 2) bs = f16x8{};  // (the instruction's columns 16..31: nothing)
+      }
+      const float* inv = reinterpret_cast<const float*>(ab + 16 * BN) + TK * n;
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        Acc s;
+        if (TYPE == TL_Q4_K) s = TL::mfma(bs, mn[i], zero);
+#pragma unroll
+        for (int q = 0; q < TL::E / 4; ++q) {
+          const f32x4 iv = *reinterpret_cast<const f32x4*>(inv + TL::quad(q, fg));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            float x = TYPE == TL_Q8_0 ? c8[n][i][4 * q + e] : d[i] * (APART ? t[n][i][4 * q + e] + tl[n][i][4 * q + e] : t[n][i][4 * q + e]);
+            if (TYPE == TL_Q4_K) x = fmaf(dm[i], s[4 * q + e], x);
+            acc[n][i][4 * q + e] = fmaf(iv[e], x, acc[n][i][4 * q + e]);
+          }
+        }
+      }
+    }
+    if (NEXT) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i) H[i] = Hn[i];
+      *reinterpret_cast<u32x4*>(an + ap * 8) = aux;
+      __syncthreads();
+    }
+  };
+  for (int b = 0; b + 1 < nsb; ++b) superblock(b, std::true_type{});
+  superblock(nsb - 1, std::false_type{});
+
+#pragma unroll
+  for (int n = 0; n < NI; ++n)
+#pragma unroll
+    for (int q = 0; q < TL::E / 4; ++q) {
+      const int t0 = n0 + TK * n + TL::quad(q, fg);
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        const int r = m0 + TK * i + fr;
+        if (r >= M) continue;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (t0 + e < T) {
+            const size_t o = (size_t)(t0 + e) * M + r;
+            const float val = acc[n][i][4 * q + e];
+            y[o] = resid ? resid[o] + val : val;
+          }
+        }
+      }
+    }
+}
+
+// ---- producer of the activation planes ----------------------------------------------------------------------------------
+// MODE 0: x; 1: rmsnorm_batch(x, aux = weight, eps) (utils.cpp:613-646); 2: swiglu(x, aux) (cpu_batch_processor.cpp:252-256).
+// a / b: pending K-split sums (see tl_launch_split); RMSNORM with a pending projection writes the new residual row to xout.
+// 8 columns per thread, so a super-block is half a wave. RMSNORM: one workgroup per token, NIT pieces of 8 columns per
+// thread; else grid.y covers the row.
+// (S <= 8; the loads of all slices are in flight together, four at a time: one after another they are S round trips to L2)
+__device__ __forceinline__ f32x4 hparts4(const GemmParts& g, size_t o) {
+  auto ld = [&](int z) { return *reinterpret_cast<const f32x4*>(g.part + (size_t)z * g.n + o); };
+  f32x4 acc = ld(0);
+  int z = 1;
+  for (; z + 4 <= g.S; z += 4) {
+    const f32x4 a = ld(z), b = ld(z + 1), c = ld(z + 2), d = ld(z + 3);
+    acc = acc + a + b + c + d;
+  }
+  if (z + 2 <= g.S) {
+    const f32x4 a = ld(z), b = ld(z + 1);
+    acc = acc + a + b;
+    z += 2;
+  }
+  if (z < g.S) acc += ld(z);
+  return acc;
+}
+// eight columns i0.. of token t (all lanes of a half wave on one super-block): both parts, the power of two, the block sum
+__device__ __forceinline__ void hsplit8(const float* v, _Float16* __restrict__ planes, size_t ps, int t, int K, int i0, int tpad) {
+  float top = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) top = fmaxf(top, fabsf(v[e]));
+#pragma unroll
+  for (int o = 16; o >= 1; o >>= 1) top = fmaxf(top, __shfl_xor(top, o));
+  if (i0 >= K) return;  // (whole quads of threads: K is a multiple of 32)
+  // top * 2^k in [512, 1024); zeros, and sub-normals or infinities, keep k in the normal range
+  int ex = (int)((__builtin_bit_cast(unsigned, top) >> 23) & 255u) - 127;
+  ex = top == 0.f ? 0 : ex < -110 ? -110 : ex > 120 ? 120 : ex;
+  const float scale = __builtin_bit_cast(float, (unsigned)(127 + 9 - ex) << 23);
+  _Float16* bs = planes + 2 * ps;
+  float* inv = reinterpret_cast<float*>(bs + ps / 16);
+  const int sb = i0 >> 8;
+  if ((i0 & 255) == 0) inv[(size_t)sb * tpad + t] = __builtin_bit_cast(float, (unsigned)(127 - 9 + ex) << 23);
+  float s = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+  s += __shfl_xor(s, 1);
+  s += __shfl_xor(s, 2);
+  if ((i0 & 31) == 0 && (K & 255) == 0) {  // sum of the 32-column block, at the place of its minimum in the operand
+    const int j = (i0 >> 5) & 7, at = j < 4 ? 2 * j : 2 * (j - 4) + 1;
+    _Float16* o = bs + ((size_t)sb * tpad + t) * 16 + at;
+    s *= scale;
+    const _Float16 h = (_Float16)s;
+    o[0] = h;
+    o[8] = (_Float16)(s - (float)h);
+  }
+  constexpr int ORDER[8] = {0, 2, 1, 3, 4, 6, 5, 7};
+  f16x8 hi, lo;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float xv = v[ORDER[e]] * scale;
+    hi[e] = (_Float16)xv;
+    lo[e] = (_Float16)(xv - (float)hi[e]);
+  }
+  *reinterpret_cast<f16x8*>(planes + (size_t)t * K + i0) = hi;
+  *reinterpret_cast<f16x8*>(planes + ps + (size_t)t * K + i0) = lo;
+}
+constexpr int HNORM_THREADS = 512, HMAX_COLS = 8 * 8 * HNORM_THREADS;
+template <int NIT>
+__global__ __launch_bounds__(HNORM_THREADS) void hsplit_norm_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                    _Float16* __restrict__ planes, size_t ps, int K, float eps,
+                                                                    GemmParts a, float* __restrict__ xout, int tpad) {
+  __shared__ float red[HNORM_THREADS / 64];
+  const int t = blockIdx.x, tid = threadIdx.x;
+  const size_t row = (size_t)t * K;
+  float v[NIT][8];
+  float ssq = 0.f;
+#pragma unroll
+  for (int it = 0; it < NIT; ++it) {
+    const int i0 = (it * HNORM_THREADS + tid) * 8;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      f32x4 p = {0.f, 0.f, 0.f, 0.f};
+      if (i0 < K) {
+        const size_t o = row + i0 + 4 * h;
+        p = *reinterpret_cast<const f32x4*>(x + o);
+        if (a.S) {
+          p += hparts4(a, o);
+          *reinterpret_cast<f32x4*>(xout + o) = p;
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[it][4 * h + e] = p[e];
+        ssq = fmaf(p[e], p[e], ssq);
+      }
+    }
+  }
+  for (int o = 32; o >= 1; o >>= 1) ssq += __shfl_xor(ssq, o);
+  if ((tid & 63) == 0) red[tid >> 6] = ssq;
+  __syncthreads();
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < HNORM_THREADS / 64; ++i) sum += red[i];
+  const float nf = 1.0f / sqrtf(sum / (float)K + eps);
+#pragma unroll
+  for (int it = 0; it < NIT; ++it) {
+    const int i0 = (it * HNORM_THREADS + tid) * 8;
+    if (i0 < K) {
+      const f32x4 w0 = *reinterpret_cast<const f32x4*>(w + i0), w1 = *reinterpret_cast<const f32x4*>(w + i0 + 4);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[it][e] = v[it][e] * nf * (e < 4 ? w0[e] : w1[e - 4]);
+    }
+    hsplit8(v[it], planes, ps, t, K, i0, tpad);
+  }
+}
+template <int MODE>
+__global__ __launch_bounds__(256) void hsplit_kernel(const float* __restrict__ x, const float* __restrict__ aux,
+                                                     _Float16* __restrict__ planes, size_t ps, int K, GemmParts a, GemmParts b,
+                                                     int tpad) {
+  const int t = blockIdx.x, i0 = (blockIdx.y * 256 + threadIdx.x) * 8;
+  float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (i0 < K) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const size_t o = (size_t)t * K + i0 + 4 * h;
+      f32x4 p = MODE == 2 && a.S ? hparts4(a, o) : *reinterpret_cast<const f32x4*>(x + o);
+      if (MODE == 2) {
+        const f32x4 up = b.S ? hparts4(b, o) : *reinterpret_cast<const f32x4*>(aux + o);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) p[e] = (p[e] / (1.0f + expf(-p[e]))) * up[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[4 * h + e] = p[e];
+    }
+  }
+  hsplit8(v, planes, ps, t, K, i0, tpad);
+}
+
+// The shapes of a workgroup. Up to 16 tokens: 64 rows, four workgroups (sixteen waves) on a CU, which keeps the most weight
+// bytes in flight: a step of 16 sequences of the 8B shape (8 layers) 0.96 ms against 0.98 with the 32-token shape (Q8_0 of
+// 1.1B 0.58 against 0.63). Up to 64: 128 rows x 32 tokens, two on a CU (32 sequences 1.04 ms; 64: 1.46 against 1.49 with
+// 64-token tiles). More: 64-token tiles, each operand unpacked once for two token fragments. There the matrix cores set the
+// pace: without unpacking, fragment reads and scale FMAs a 512-token chunk is 20 % shorter, no more, and the clock falls to
+// 1.9 GHz under them; which of the three shapes is taken is a matter of filling the chip, so the plan below weighs them.
+// (8 layers of the 8B shape in ms, this kernel / the bf16 kernels it replaced: 8 sequences 0.86 / 1.56, 32: 1.05 / 1.62,
+// 64: 1.52 / 2.03, 128: 2.2 / 2.7; a prompt of 512: 5.3 / 7.0.)
+struct HShape {
+  int tk, ni, mi, nw, wpe, percu;
+};
+constexpr HShape SHAPE[] = {{16, 1, 1, 4, 4, 4}, {32, 1, 1, 4, 2, 2}, {32, 2, 1, 8, 2, 1}, {32, 2, 2, 4, 2, 2}, {32, 2, 1, 4, 2, 2}};
+// us of a super-block of a workgroup on a full chip (measured; Q6_K's third product and longer unpacking)
+float hgemm_us(int type, int shape) {
+  constexpr float US[] = {1.2f, 2.0f, 4.9f, 9.0f, 5.0f};
+  return US[shape] * (type == TL_Q6_K ? 1.37f : 1.f);
+}
+struct HPlan {
+  int shape, bm, bn, S;
+};
+// The shape and the K slices with the least of: rounds over the chip x (a workgroup's super-blocks + its start and end) + the
+// partial sums written and read once at about 4 TB/s.
+HPlan hgemm_plan(const QW* w, int n, int T) {
+  const int nsb = (w[0].cols + 255) / 256, type = w[0].type;
+  const int lo = T <= 16 ? 0 : T <= 64 ? 1 : type == TL_Q8_0 ? 4 : 2, hi = T <= 64 ? lo : 4;
+  HPlan best = {lo, 0, 0, 1};
+  float least = -1.f;
+  for (int v = lo; v <= hi; ++v) {
+    if (v == 3 && type == TL_Q6_K) continue;  // (spills)
+    const HShape& q = SHAPE[v];
+    const int bm = q.tk * q.mi * q.nw, bn = q.tk * q.ni, ntiles = (T + bn - 1) / bn, slots = tl_num_cus() * q.percu;
+    long tiles = 0, rows = 0;
+    for (int i = 0; i < n; ++i) {
+      tiles += (long)((w[i].rows + bm - 1) / bm) * ntiles;
+      rows += w[i].rows;
+    }
+    for (int S = 1; S <= 8 && S <= nsb; ++S) {
+      const int per = (nsb + S - 1) / S;
+      if ((nsb + per - 1) / per != S) continue;  // (no empty slice)
+      const float cost = (float)((tiles * S + slots - 1) / slots) * (float)(per + (v < 2 ? 2 : 1)) * hgemm_us(type, v) +
+                         (S > 1 ? (float)S * (0.3f + (float)T * (float)rows * 2e-6f) : 0.f);
+      if (least < 0.f || cost < least) {
+        least = cost;
+        best = {v, bm, bn, S};
+      }
+    }
+  }
+  return best;
+}
+
+template <int TYPE, int V>
+int hgemm_go(const HSegs& g, int mt, const HAct& act, const float* resid, int T, int S, hipStream_t s) {
+  constexpr HShape q = SHAPE[V];
+  constexpr int BN = q.tk * q.ni;
+  constexpr size_t lds = (size_t)(BN > 32 ? 3 * 2 * 64 + 2 * 18 : 2 * (4 * 2 * 64 + 18)) * BN * sizeof(_Float16);
+  static TlDeviceOnce lds_raised;
+  auto kernel = hgemm_kernel<TYPE, q.tk, q.ni, q.mi, q.nw, q.wpe>;
+  TL_TRY(tl_raise_lds_limit(kernel, (int)lds, lds_raised));
+  const int ntiles = (T + BN - 1) / BN;
+  kernel<<<dim3((unsigned)(mt * ntiles * S)), dim3(64 * q.nw), lds, s>>>(g, act, resid, T, mt, ntiles, S);
+  TL_HIP(hipGetLastError());
+  return 0;
+}
+template <int TYPE>
+int hgemm_typed(const QW* w, int n, const HPlan& p, const HAct& act, float* const* out, const float* resid, int T, hipStream_t s) {
+  HSegs g = {};
+  int mt = 0;
+  for (int i = 0; i < 3; ++i) {
+    const int k = i < n ? i : n - 1;  // (unused slots repeat the last matrix; their tile range is empty)
+    g.w[i] = w[k];
+    g.y[i] = out[k];
+    if (i < n) mt += (w[i].rows + p.bm - 1) / p.bm;
+    g.mt_end[i] = mt;
+  }
+  if (p.shape == 0) return hgemm_go<TYPE, 0>(g, mt, act, resid, T, p.S, s);
+  if (p.shape == 1) return hgemm_go<TYPE, 1>(g, mt, act, resid, T, p.S, s);
+  if constexpr (TYPE != TL_Q8_0)
+    if (p.shape == 2) return hgemm_go<TYPE, 2>(g, mt, act, resid, T, p.S, s);
+  if constexpr (TYPE == TL_Q4_K || TYPE == TL_Q8_K)
+    if (p.shape == 3) return hgemm_go<TYPE, 3>(g, mt, act, resid, T, p.S, s);
+  return hgemm_go<TYPE, 4>(g, mt, act, resid, T, p.S, s);
+}
+
+}  // namespace
+
+bool tl_hgemm_supported(const QW& w) {
+  const bool k256 = w.type == TL_Q4_K || w.type == TL_Q6_K || w.type == TL_Q8_K;
+  return (k256 || w.type == TL_Q8_0) && w.cols % (k256 ? 256 : 64) == 0 && w.cols <= HMAX_COLS && w.rows > 0 &&
+         (size_t)w.rows * w.cols < ((size_t)1 << 32);  // (32-bit byte offsets)
+}
+int tl_hgemm_slices(const QW* w, int n, int T) { return hgemm_plan(w, n, T).S; }
+int tl_launch_hgemm(const QW* w, int n, const void* planes, size_t ps, float* const* out, const float* resid, int T, int S, hipStream_t s) {
+  for (int i = 0; i < n; ++i)
+    TL_REQUIRE(tl_hgemm_supported(w[i]) && w[i].type == w[0].type && w[i].cols == w[0].cols, "half-plane GEMM: matrix %d does not fit", i);
+  TL_REQUIRE(n >= 1 && n <= 3 && T > 0 && S >= 1 && ps < ((size_t)1 << 31) && ps >= tl_gemm_padded_tokens(T) * (size_t)w[0].cols, "half-plane GEMM: bad argument");
+  HPlan p = hgemm_plan(w, n, T);
+  p.S = S;
+  const HAct act = hact(planes, ps, T);
+  switch (w[0].type) {
+    case TL_Q4_K: return hgemm_typed<TL_Q4_K>(w, n, p, act, out, resid, T, s);
+    case TL_Q6_K: return hgemm_typed<TL_Q6_K>(w, n, p, act, out, resid, T, s);
+    case TL_Q8_0: return hgemm_typed<TL_Q8_0>(w, n, p, act, out, resid, T, s);
+    default: return hgemm_typed<TL_Q8_K>(w, n, p, act, out, resid, T, s);
+  }
+}
+int tl_launch_hsplit(int mode, const float* x, const float* aux, void* planes, size_t ps, int T, int K, float eps, hipStream_t s,
+                     const GemmParts& a, const GemmParts& b, float* xout) {
+  TL_REQUIRE(K > 0 && K % 32 == 0 && K <= HMAX_COLS && T > 0 && T <= 65535, "half-plane split: bad shape %d x %d", T, K);
+  _Float16* pl = static_cast<_Float16*>(planes);
+  const int tpad = (int)tl_gemm_padded_tokens(T);
+  if (mode == 1) {
+    const int nit = (K + 8 * HNORM_THREADS - 1) / (8 * HNORM_THREADS);
+    if (nit <= 1) hsplit_norm_kernel<1><<<T, HNORM_THREADS, 0, s>>>(x, aux, pl, ps, K, eps, a, xout, tpad);
+    else if (nit <= 2) hsplit_norm_kernel<2><<<T, HNORM_THREADS, 0, s>>>(x, aux, pl, ps, K, eps, a, xout, tpad);
+    else hsplit_norm_kernel<8><<<T, HNORM_THREADS, 0, s>>>(x, aux, pl, ps, K, eps, a, xout, tpad);
+  } else {
+    const dim3 grid(T, (K + 2047) / 2048);
+    if (mode == 2) hsplit_kernel<2><<<grid, 256, 0, s>>>(x, aux, pl, ps, K, a, b, tpad);
+    else hsplit_kernel<0><<<grid, 256, 0, s>>>(x, aux, pl, ps, K, a, b, tpad);
+  }
+  TL_HIP(hipGetLastError());
+  return 0;
+}

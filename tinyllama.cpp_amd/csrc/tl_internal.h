@@ -269,6 +269,15 @@ int tl_launch_gemm_q(const QW& w, const void* planes, size_t plane_stride, float
 // was launched
 int tl_launch_gemm_q_multi(const QW* w, int n, const void* planes, size_t plane_stride, float* const* y, int T, int terms,
                            hipStream_t s, GemmDefer* const* defer, bool* merged);
+// the f16 form of the same (tl_hgemm.hip), selected in tl_launch_split / tl_launch_gemm_q / _multi by terms ==
+// TL_TERMS_HALF: activations as two f16 parts + a power of two per token, any supported format, 32-bit grade
+constexpr int TL_TERMS_HALF = 2;
+bool tl_hgemm_supported(const QW& w);
+int tl_hgemm_slices(const QW* w, int n, int T);
+int tl_launch_hgemm(const QW* w, int n, const void* planes, size_t plane_stride, float* const* out, const float* resid, int T, int S,
+                    hipStream_t s);
+int tl_launch_hsplit(int mode, const float* x, const float* aux, void* planes, size_t plane_stride, int T, int K, float eps,
+                     hipStream_t s, const GemmParts& a, const GemmParts& b, float* xout);
 // y = (resid ? resid : 0) + the pending sums (what the GEMM launch would have run itself)
 int tl_launch_ksplit_reduce(const GemmParts& g, const float* resid, float* y, hipStream_t s);
 

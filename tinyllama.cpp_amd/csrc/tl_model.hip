@@ -77,6 +77,7 @@ struct tl_model {
   float* attn_ws = nullptr;    // split-attention partials
   float* xn = nullptr;         // normalised input of the unfused (F32-matrix) projections
   bool has_f32 = false;        // some projection matrix is F32 (set by finalize): no MFMA prefill, no multi-sequence step
+  bool half_planes = false;    // every projection matrix has the f16 form of the chunk GEMMs (tl_hgemm.hip; set by finalize)
   bool attn_split = false;
   int* state = nullptr;  // DevState header + history ring
   int hist_cap = 0;
@@ -746,12 +747,13 @@ static int plan_chain(tl_model* m) {
   m->chain.on = true;
   return 0;
 }
-// Expanded prefill planes for every quantized matrix of the model (tl_gemm.hip, gemm_px_kernel), when they are affordable:
-// at most a quarter of the device's memory and what is free now less 4 GiB (TL_PREFILL_PLANES=0 / 1: never / always).
+// Expanded prefill planes for every quantized matrix of a model whose chunks go through bf16 parts (tl_gemm.hip,
+// gemm_px_kernel), when they are affordable: at most a quarter of the device's memory and what is free now less 4 GiB
+// (TL_PREFILL_PLANES=0 / 1: never / always).
 static int expand_prefill_planes(tl_model* m) {
   const char* e = getenv("TL_PREFILL_PLANES");
   const int mode = e ? (atoi(e) != 0 ? 1 : 0) : -1;
-  if (mode == 0) return 0;
+  if (mode == 0 || (mode < 0 && m->half_planes)) return 0;  // (the f16 form reads the quantized planes themselves)
   std::vector<const tl_qweight*> ws;
   for (auto& l : m->layers)
     for (auto* w : l.q)
@@ -1096,6 +1098,9 @@ extern "C" int tl_model_finalize(tl_model* m) {
   TL_HIP(hipMemsetAsync(m->kv_base, 0, sizeof(float) * 2 * m->kv_layer_elems * c.num_hidden_layers, m->stream));
   TL_HIP(hipMalloc(&m->x, sizeof(float) * H));
   m->has_f32 = m->out->type == TL_F32;
+  m->half_planes = tl_hgemm_supported(qw_view(m->out));
+  for (const LayerW& L : m->layers)
+    for (int k = 0; k < 7; ++k) m->half_planes = m->half_planes && tl_hgemm_supported(qw_view(L.q[k]));
   for (int l = 0; l < c.num_hidden_layers; ++l)
     for (int k = 0; k < 7; ++k) m->has_f32 |= m->layers[l].q[k]->type == TL_F32;
   if (m->has_f32) TL_HIP(hipMalloc(&m->xn, sizeof(float) * (H > (size_t)m->qd_l ? H : (size_t)m->qd_l)));
@@ -1285,6 +1290,13 @@ constexpr int kPrefillChunk = 512;
 
 __global__ void set_token_kernel(int* state, const int* tokens, int i) { state[0] = tokens[i]; }
 
+// how a chunk's products are formed: 1 = plain bf16; 3 and 6 both as the f16 form of the 32-bit grade where every matrix has
+// it (tl_hgemm.hip: two matrix instructions a product, what 3 terms of bf16 parts cost, at the grade of 6), else bf16 parts
+static int chunk_terms(const tl_model* m) {
+  const int terms = m->prefill_terms ? m->prefill_terms : tl_gemm_default_terms();
+  return terms != 1 && m->half_planes ? TL_TERMS_HALF : terms;
+}
+
 static int ensure_prefill_ws(tl_model* m, bool all_logits) {
   const tl_model_config& c = m->cfg;
   tl_model::Prefill& p = m->pf;
@@ -1333,7 +1345,7 @@ static int prefill_embed(tl_model* m, const int* toks_dev, int T, hipStream_t s)
 // RMSNorm of the residual stream -> activation planes; a projection still pending as K-split partials is added on the way
 static int split_residual(tl_model* m, const float* norm_w, int T, hipStream_t s) {
   tl_model::Prefill& p = m->pf;
-  const int terms = m->prefill_terms ? m->prefill_terms : tl_gemm_default_terms();
+  const int terms = chunk_terms(m);
   if (!p.pend.S) return tl_launch_split(1, p.xb, norm_w, p.planes, p.plane_stride, T, m->cfg.hidden_size, terms, m->cfg.rms_norm_eps, s);
   TL_TRY(tl_launch_split(1, p.xb, norm_w, p.planes, p.plane_stride, T, m->cfg.hidden_size, terms, m->cfg.rms_norm_eps, s,
                          &p.pend, nullptr, p.xb2));
@@ -1352,7 +1364,7 @@ static int flush_residual(tl_model* m, hipStream_t s) {
 // a row-split projection (attn_output, ffn_down) added to the residual stream: now, or pending
 static int project_residual(tl_model* m, const tl_qweight* w, int T, hipStream_t s) {
   tl_model::Prefill& p = m->pf;
-  const int terms = m->prefill_terms ? m->prefill_terms : tl_gemm_default_terms();
+  const int terms = chunk_terms(m);
   if (m->tp > 1 || !p.part_cap)
     return tl_launch_gemm_q(qw_view(w), p.planes, p.plane_stride, m->tp > 1 ? p.xpart : p.xb, m->rank == 0 ? p.xb : nullptr, T,
                             terms, s);
@@ -1365,7 +1377,7 @@ static int project_residual(tl_model* m, const tl_qweight* w, int T, hipStream_t
 // tiles described by pf.dq / dk / dv .got for the RoPE + cache-write kernel to sum
 static int qkv_deferred(tl_model* m, LayerW& L, int T, hipStream_t s) {
   tl_model::Prefill& p = m->pf;
-  const int terms = m->prefill_terms ? m->prefill_terms : tl_gemm_default_terms();
+  const int terms = chunk_terms(m);
   const size_t ps = p.plane_stride;
   p.dq = {p.part[0], p.part_cap, {nullptr, 0, 0}};
   p.dk = {p.part[1], p.part_cap, {nullptr, 0, 0}};
@@ -1397,7 +1409,7 @@ static int prefill_attn_half(tl_model* m, int l, int T, int start_pos, hipStream
   tl_model::Prefill& p = m->pf;
   LayerW& L = m->layers[l];
   const int H = c.hidden_size, hd = m->head_dim;
-  const int terms = m->prefill_terms ? m->prefill_terms : tl_gemm_default_terms();
+  const int terms = chunk_terms(m);
   const size_t ps = p.plane_stride;
   const float scale = 1.0f / sqrtf((float)hd);
   (void)H;
@@ -1423,7 +1435,7 @@ static int prefill_attn_half(tl_model* m, int l, int T, int start_pos, hipStream
   // the attention output goes straight into the planes of the attn_output GEMM where the MFMA kernel serves the head shape
   // (no split launch; TL_ATTN_PLANES=0 keeps the launch, for A/B runs and the bit-identity test)
   const char* ap = getenv("TL_ATTN_PLANES");
-  if (tl_attn_prefill_mfma_supported(m->nh_l, m->nkv_l, hd) && !(ap && atoi(ap) == 0)) {
+  if (terms != TL_TERMS_HALF && tl_attn_prefill_mfma_supported(m->nh_l, m->nkv_l, hd) && !(ap && atoi(ap) == 0)) {
     TL_TRY(tl_launch_attn_prefill_mfma(p.qb, m->kc(l), m->vc(l), p.ab, T, start_pos, m->nh_l, m->nkv_l, hd, scale, s, p.planes,
                                        ps, terms));
   } else {
@@ -1437,7 +1449,7 @@ static int prefill_mlp_half(tl_model* m, int l, int T, hipStream_t s) {
   const tl_model_config& c = m->cfg;
   tl_model::Prefill& p = m->pf;
   LayerW& L = m->layers[l];
-  const int terms = m->prefill_terms ? m->prefill_terms : tl_gemm_default_terms();
+  const int terms = chunk_terms(m);
   const size_t ps = p.plane_stride;
   (void)c;
   TL_TRY(split_residual(m, L.ffn_norm, T, s));
@@ -1499,7 +1511,6 @@ static int prefill_batched(tl_model* m, const int* tokens_host, int num_tokens, 
   hipStream_t s = m->stream;
   TL_TRY(prepare_prefill(m, tokens_host, num_tokens, all_logits_host != nullptr, s));
   const size_t H = c.hidden_size, V = c.vocab_size;
-  const int terms = m->prefill_terms ? m->prefill_terms : tl_gemm_default_terms();
   for (int c0 = 0; c0 < num_tokens; c0 += p.cap) {
     const int T = num_tokens - c0 < p.cap ? num_tokens - c0 : p.cap;
     TL_TRY(prefill_embed(m, p.toks + c0, T, s));
@@ -1510,6 +1521,7 @@ static int prefill_batched(tl_model* m, const int* tokens_host, int num_tokens, 
       TL_TRY(prefill_all_reduce(m, T, s));
     }
     TL_TRY(flush_residual(m, s));
+    const int terms = chunk_terms(m);
     if (all_logits_host) {  // final norm + lm_head for every token of the chunk (forward_cpu_logits_batch, model.cpp:1094-1156)
       TL_TRY(tl_launch_split(1, p.xb, m->out_norm, p.planes, p.plane_stride, T, (int)H, terms, c.rms_norm_eps, s));
       TL_TRY(tl_launch_gemm_q(qw_view(m->out), p.planes, p.plane_stride, p.logits_all, nullptr, T, terms, s));
@@ -1613,7 +1625,7 @@ static int batch_attn_half(tl_model* m, int l, int T, hipStream_t s) {
   tl_model::Prefill& p = m->pf;
   LayerW& L = m->layers[l];
   const int H = c.hidden_size, hd = m->head_dim;
-  const int terms = m->prefill_terms ? m->prefill_terms : tl_gemm_default_terms();
+  const int terms = chunk_terms(m);
   const size_t ps = p.plane_stride;
   const float scale = 1.0f / sqrtf((float)hd);
   (void)H;
@@ -1625,7 +1637,7 @@ static int batch_attn_half(tl_model* m, int l, int T, hipStream_t s) {
   // the attention output goes straight into the planes of the attn_output GEMM (no split launch; TL_ATTN_PLANES=0 keeps
   // the launch, for A/B runs and the bit-identity test)
   const char* ap = getenv("TL_ATTN_PLANES");
-  if (ap && atoi(ap) == 0) {
+  if (terms == TL_TERMS_HALF || (ap && atoi(ap) == 0)) {
     TL_TRY(tl_launch_batch_attn(p.qb, m->bkc(l), m->bvc(l), m->kv_layer_elems, p.ab, m->bt.pos, m->bt.seq, T, m->nh_l,
                                 m->nkv_l, hd, c.max_position_embeddings, m->bt.max_batch, scale, s));
     TL_TRY(tl_launch_split(0, p.ab, nullptr, p.planes, ps, T, m->qd_l, terms, 0.f, s));
@@ -1748,7 +1760,7 @@ static int batch_head(tl_model* m, const float* hidden, int R, hipStream_t s) {
     f.eps = c.rms_norm_eps;
     return tl_launch_gemv_nv(f, R, s);
   }
-  const int terms = m->prefill_terms ? m->prefill_terms : tl_gemm_default_terms();
+  const int terms = chunk_terms(m);
   TL_TRY(tl_launch_split(1, hidden, m->out_norm, p.planes, p.plane_stride, R, c.hidden_size, terms, c.rms_norm_eps, s));
   return tl_launch_gemm_q(qw_view(m->out), p.planes, p.plane_stride, p.logits_all, nullptr, R, terms, s);
 }
