@@ -52,6 +52,23 @@ def test_device_sampler_matches_oracle(E, oracle, V, T, k, pp):
         assert got == int(ids[oracle.discrete_draw(probs, u)]), (u, got)
 
 
+@pytest.mark.parametrize("V,k,levels", [(127, 40, 0), (128, 128, 0), (129, 129, 0), (1024, 0, 0), (1025, 128, 0), (33000, 128, 0),
+                                        (33000, 129, 0), (32000, 40, 3), (32000, 1, 2), (4097, 1024, 5)])
+def test_device_sampler_slices_and_fallback(E, oracle, V, k, levels):
+    """The list of candidates is taken from 128 slices and bounded by the k-th largest slice maximum: vocabularies around one
+    entry per slice, k around the number of slices (a larger one lists everything), and `levels` distinct logits, whose ties at
+    the bound overflow the list and take the whole-vector selection. Ids exactly: equal logits have equal probabilities."""
+    rng = np.random.default_rng(V + k + levels)
+    logits = (rng.integers(0, levels, V) if levels else rng.standard_normal(V) * 3).astype(np.float32)
+    wi, wp = oracle.sample_candidates(logits, 0.9, k, 1.0)
+    u = 0.40625  # the same in FP32 and FP64, and between two partial sums of 40 equal probabilities
+    got, ids, probs = E.sample_top_k_top_p(logits, 0.9, k, 1.0, u)
+    _same_candidates(ids, probs, wi, wp)
+    if levels:
+        assert np.array_equal(ids, wi)
+    assert got == int(ids[oracle.discrete_draw(probs, u)])
+
+
 def test_device_sampler_edge_cases(E):
     from tinyllama_cpp_amd.capi import TlError
     rng = np.random.default_rng(1)

@@ -299,6 +299,7 @@ struct TlSampleParams {  // lives in device memory; `counter` is advanced by the
   unsigned counter;
   unsigned long long seed;
 };
+size_t tl_sample_scratch_bytes(int n);  // probabilities + the slices' maxima and sums + the list of candidates
 int tl_launch_sample_topk(float* logits, int n, float* probs_scratch, int* state, int state_header, int hist_cap,
                           TlSampleParams* params_dev, int* out_id, int* cand_ids, float* cand_probs, int* n_cand,
                           hipStream_t s);

@@ -1248,7 +1248,7 @@ extern "C" int tl_model_generate_sampled(tl_model* m, int first_token, int start
   TL_REQUIRE(keep + n_steps <= m->hist_cap, "tl_model_generate_sampled: %d steps exceed the id history capacity", n_steps);
   if (!m->sparams) {
     TL_HIP(hipMalloc(&m->sparams, sizeof(TlSampleParams)));
-    TL_HIP(hipMalloc(&m->sample_probs, sizeof(float) * (size_t)V));
+    TL_HIP(hipMalloc(&m->sample_probs, tl_sample_scratch_bytes((int)V)));
   }
   TlSampleParams h = {};
   h.temperature = temperature;
