@@ -347,3 +347,35 @@ def test_half_plane_gemm_edges(E, pkg, name, rows, cols, T):
     assert (np.abs(y - want) <= (2.0 ** -22 + 48 * 2.0 ** -24 + cols / 256 * 2.0 ** -24) * scale).all(), (np.abs(y - want) / np.maximum(scale, 1e-30)).max()
     assert not y[T // 2].any()
     w.free()
+
+
+@pytest.mark.parametrize("heads,kv,hd,start,T", [
+    (4, 2, 64, 0, 8), (8, 1, 64, 33, 95), (16, 16, 64, 31, 33), (4, 1, 64, 900, 129), (6, 2, 128, 0, 129), (2, 2, 128, 63, 64),
+    (6, 2, 128, 1000, 300), (8, 8, 128, 7, 150), (16, 2, 128, 2000, 9)])
+def test_half_attention_edges(E, pkg, monkeypatch, heads, kv, hd, start, T):
+    """tl_hattn.hip against the FP32 matrix kernel (TL_HATTN=0): groups of 1 to 8 heads, rows and keys on and off the tiles of
+    128 and 32, one and several pieces of the keys, tiles whose values are 2^-9 .. 2^9 apart (the common exponent of the running
+    sum) and an all-zero tile. A score's error is at most 2^-21 |q| |k| scale from the parts and hd 2^-24 of it from the sums;
+    with |q| |k| scale below 16 here, and as much again from the values, the outputs agree to 2 * 16 * (2^-21 + hd 2^-24) < 3e-4
+    at worst; errors are independent, so the L2 distance of the logits is held to 1e-5."""
+    cfg = dict(hidden=heads * hd, inter=256, n_heads=heads, n_kv_heads=kv, n_layers=1, vocab=64, max_pos=start + T, eps=1e-5,
+               rope_theta=10000.0)
+    _, tensors = pkg.synth.build_model(cfg, "q8_0", seed=heads + T)
+    m = E.Model(cfg).load(tensors)
+    m.set_prefill(terms=6, min_batch=8)
+    rng = np.random.default_rng(start + T)
+    K = rng.standard_normal((start, kv * hd)).astype(np.float32)
+    V = rng.standard_normal((start, kv * hd)).astype(np.float32)
+    V *= np.exp2(rng.integers(-9, 10, -(-start // 32))).astype(np.float32).repeat(32)[:start, None]
+    K[32:64] = V[32:64] = 0.0
+    toks = rng.integers(0, cfg["vocab"], T).astype(np.int32)
+    got = []
+    for route in ("0", "1"):
+        monkeypatch.setenv("TL_HATTN", route)
+        m.reset_kv()
+        if start:
+            m.set_kv_cache(0, K, V)
+        got.append(np.array(m.prefill(toks, start, all_logits=True)[1], np.float64))
+    m.free()
+    assert np.isfinite(got[1]).all() and not np.array_equal(got[0], got[1])
+    assert np.linalg.norm(got[1] - got[0]) <= 1e-5 * np.linalg.norm(got[0]), np.linalg.norm(got[1] - got[0]) / np.linalg.norm(got[0])

@@ -281,6 +281,11 @@ int tl_launch_hsplit(int mode, const float* x, const float* aux, void* planes, s
 // y = (resid ? resid : 0) + the pending sums (what the GEMM launch would have run itself)
 int tl_launch_ksplit_reduce(const GemmParts& g, const float* resid, float* y, hipStream_t s);
 
+// causal prefill attention in two-part f16 over a workspace of converted K/V tiles (tl_hattn.hip)
+bool tl_hattn_supported(int nh, int nkv, int hd);
+size_t tl_hattn_bytes(int max_len, int nkv, int hd);
+int tl_launch_hattn(const float* q, const float* kc, const float* vc, float* out, int T, int start_pos, int nh, int nkv, int hd,
+                    float scale, void* ws, size_t ws_bytes, hipStream_t s);
 // causal prefill attention on the FP32 matrix instruction (tl_prefill.hip)
 bool tl_attn_prefill_mfma_supported(int nh, int nkv, int hd);
 // planes != NULL: the output as the attn_output GEMM's activation planes (tl_launch_split's layout) instead of `out`

@@ -112,6 +112,8 @@ struct tl_model {
     int rows_cap = 0;
     int* toks = nullptr;
     int toks_cap = 0;
+    void* hattn = nullptr;     // converted K/V tiles and partial outputs of the f16 attention (tl_hattn.hip)
+    size_t hattn_bytes = 0;
     // independent GEMMs of a layer (q | k, v and gate | up) run on two streams so that their workgroups share the chip
     hipStream_t side = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
@@ -259,6 +261,7 @@ extern "C" int tl_model_free(tl_model* m) {
   for (float* b : pbufs) hipFree(b);
   hipFree(m->pf.planes);
   hipFree(m->pf.toks);
+  hipFree(m->pf.hattn);
   hipFree(m->pf.rows);
   hipFree(m->bt.kv);
   hipFree(m->bt.toks);
@@ -1435,7 +1438,16 @@ static int prefill_attn_half(tl_model* m, int l, int T, int start_pos, hipStream
   // the attention output goes straight into the planes of the attn_output GEMM where the MFMA kernel serves the head shape
   // (no split launch; TL_ATTN_PLANES=0 keeps the launch, for A/B runs and the bit-identity test)
   const char* ap = getenv("TL_ATTN_PLANES");
-  if (terms != TL_TERMS_HALF && tl_attn_prefill_mfma_supported(m->nh_l, m->nkv_l, hd) && !(ap && atoi(ap) == 0)) {
+  const char* ha = getenv("TL_HATTN");  // 0: the FP32 attention kernel everywhere (A/B runs and tests)
+  if (terms == TL_TERMS_HALF && tl_hattn_supported(m->nh_l, m->nkv_l, hd) && !(ha && atoi(ha) == 0)) {
+    if (!p.hattn) {
+      const size_t bytes = tl_hattn_bytes(c.max_position_embeddings, m->nkv_l, hd);
+      TL_HIP(hipMalloc(&p.hattn, bytes));
+      p.hattn_bytes = bytes;
+    }
+    TL_TRY(tl_launch_hattn(p.qb, m->kc(l), m->vc(l), p.ab, T, start_pos, m->nh_l, m->nkv_l, hd, scale, p.hattn, p.hattn_bytes, s));
+    TL_TRY(tl_launch_split(0, p.ab, nullptr, p.planes, ps, T, m->qd_l, terms, 0.f, s));
+  } else if (terms != TL_TERMS_HALF && tl_attn_prefill_mfma_supported(m->nh_l, m->nkv_l, hd) && !(ap && atoi(ap) == 0)) {
     TL_TRY(tl_launch_attn_prefill_mfma(p.qb, m->kc(l), m->vc(l), p.ab, T, start_pos, m->nh_l, m->nkv_l, hd, scale, s, p.planes,
                                        ps, terms));
   } else {
