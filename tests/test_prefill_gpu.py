@@ -379,3 +379,22 @@ def test_half_attention_edges(E, pkg, monkeypatch, heads, kv, hd, start, T):
     m.free()
     assert np.isfinite(got[1]).all() and not np.array_equal(got[0], got[1])
     assert np.linalg.norm(got[1] - got[0]) <= 1e-5 * np.linalg.norm(got[0]), np.linalg.norm(got[1] - got[0]) / np.linalg.norm(got[0])
+
+
+@pytest.mark.parametrize("T", [2048, 2049, 2600])
+def test_prefill_chunks_of_2048(E, pkg, T):
+    """Prompts around the largest chunk: the last logits of the whole prompt against the last row of an all-logits prefill, which
+    walks the prompt in chunks of 512. The same products in the same grade; only which K slices and key pieces are summed apart
+    differs: 32-bit rounding, some 2^-22 a layer. And the packed form of the same prompt."""
+    cfg = dict(hidden=256, inter=512, n_heads=4, n_kv_heads=2, n_layers=2, vocab=64, max_pos=2700, eps=1e-5, rope_theta=10000.0)
+    _, tensors = pkg.synth.build_model(cfg, "q4_k_m", seed=T)
+    m = E.Model(cfg).load(tensors)
+    m.batch_init(3)
+    toks = np.random.default_rng(T).integers(0, cfg["vocab"], T).astype(np.int32)
+    last = np.array(m.prefill(toks, 0), np.float64)
+    m.reset_kv()
+    rows = np.array(m.prefill(toks, 0, all_logits=True)[1], np.float64)
+    packed = np.array(m.batch_prefill_packed([toks], slots=[2])[0][0], np.float64)
+    for got in (last, packed):
+        assert np.linalg.norm(got - rows[-1]) <= 4e-6 * np.linalg.norm(rows[-1])
+    m.free()

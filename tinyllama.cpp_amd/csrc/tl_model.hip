@@ -1289,7 +1289,11 @@ extern "C" int tl_model_generate_sampled(tl_model* m, int first_token, int start
 // the matrix cores (tl_gemm.hip), batched RoPE + KV write, causal attention from the cache (tl_prefill.hip), O GEMM +
 // residual, RMSNorm -> planes, gate/up GEMMs, SwiGLU -> planes, down GEMM + residual. Longer prompts are walked chunk by
 // chunk over the growing cache. Short prompts (< prefill_min_batch) replay the decode graph token by token instead (same positions, KV contents and logits to ~1e-6).
-constexpr int kPrefillChunk = 512;
+// Unsharded models whose products take the f16 form: 2048, where a projection has four times the tiles and no K slices, and the
+// attention converts the cache and sums its pieces a quarter as often (3B Q6_K, 3989 tokens: 98 ms in chunks of 512, 92 in these;
+// more would only grow the workspaces). The bf16 routes and tensor-parallel shards keep the 512 that they were tuned at, which
+// is also the most sequences of a step and the most logits rows of a chunk.
+constexpr int kPrefillChunk = 2048, kChunkRows = 512;
 
 __global__ void set_token_kernel(int* state, const int* tokens, int i) { state[0] = tokens[i]; }
 
@@ -1300,11 +1304,16 @@ static int chunk_terms(const tl_model* m) {
   return terms != 1 && m->half_planes ? TL_TERMS_HALF : terms;
 }
 
+// tokens that a chunk takes now (tl_model_set_prefill may have chosen plain bf16)
+static int chunk_tokens(const tl_model* m) {
+  return chunk_terms(m) == TL_TERMS_HALF ? m->pf.cap : m->pf.cap < kChunkRows ? m->pf.cap : kChunkRows;
+}
 static int ensure_prefill_ws(tl_model* m, bool all_logits) {
   const tl_model_config& c = m->cfg;
   tl_model::Prefill& p = m->pf;
   if (p.cap == 0) {
-    const int cap = c.max_position_embeddings < kPrefillChunk ? c.max_position_embeddings : kPrefillChunk;
+    const int most = m->half_planes && m->tp == 1 ? kPrefillChunk : kChunkRows;
+    const int cap = c.max_position_embeddings < most ? c.max_position_embeddings : most;
     const size_t H = c.hidden_size, maxk = H > (size_t)m->I_l ? H : (size_t)m->I_l;
     const size_t kmax = maxk > (size_t)m->qd_l ? maxk : (size_t)m->qd_l;
     p.plane_stride = tl_gemm_padded_tokens(cap) * kmax;
@@ -1333,7 +1342,10 @@ static int ensure_prefill_ws(tl_model* m, bool all_logits) {
     TL_HIP(hipEventCreateWithFlags(&p.join, hipEventDisableTiming));
     p.cap = cap;
   }
-  if (all_logits && !p.logits_all) TL_HIP(hipMalloc(&p.logits_all, sizeof(float) * p.cap * (size_t)c.vocab_size));
+  if (all_logits && !p.logits_all) {
+    const size_t rows = p.cap < kChunkRows ? p.cap : kChunkRows;
+    TL_HIP(hipMalloc(&p.logits_all, sizeof(float) * rows * (size_t)c.vocab_size));
+  }
   return 0;
 }
 
@@ -1523,8 +1535,9 @@ static int prefill_batched(tl_model* m, const int* tokens_host, int num_tokens, 
   hipStream_t s = m->stream;
   TL_TRY(prepare_prefill(m, tokens_host, num_tokens, all_logits_host != nullptr, s));
   const size_t H = c.hidden_size, V = c.vocab_size;
-  for (int c0 = 0; c0 < num_tokens; c0 += p.cap) {
-    const int T = num_tokens - c0 < p.cap ? num_tokens - c0 : p.cap;
+  const int chunk = all_logits_host && p.cap > kChunkRows ? kChunkRows : chunk_tokens(m);
+  for (int c0 = 0; c0 < num_tokens; c0 += chunk) {
+    const int T = num_tokens - c0 < chunk ? num_tokens - c0 : chunk;
     TL_TRY(prefill_embed(m, p.toks + c0, T, s));
     for (int l = 0; l < c.num_hidden_layers; ++l) {
       TL_TRY(prefill_attn_half(m, l, T, start_pos + c0, s));
@@ -1589,7 +1602,7 @@ extern "C" int tl_tp_local_group_prefill(tl_model* const* ms, int n, const int* 
   auto all = [&](auto&& f) {
     for (int r = 0; r < n && rc == 0; ++r) rc = f(ms[r]);
   };
-  const int cap = m0->pf.cap, H = m0->cfg.hidden_size, V = m0->cfg.vocab_size;
+  const int cap = chunk_tokens(m0), H = m0->cfg.hidden_size, V = m0->cfg.vocab_size;
   for (int c0 = 0; c0 < num_tokens && rc == 0; c0 += cap) {
     const int T = num_tokens - c0 < cap ? num_tokens - c0 : cap;
     const size_t len = (size_t)T * H;
@@ -1759,7 +1772,8 @@ static int batch_layers(tl_model* m, int T, hipStream_t s) {
 }
 // final RMSNorm + lm_head of R hidden rows -> pf.logits_all [R][vocab]
 static int batch_head(tl_model* m, const float* hidden, int R, hipStream_t s) {
-  TL_REQUIRE(R >= 1 && R <= m->pf.cap, "tl_model: %d logits rows exceed the chunk workspaces (%d)", R, m->pf.cap);
+  TL_REQUIRE(R >= 1 && R <= m->pf.cap && R <= kChunkRows, "tl_model: %d logits rows exceed the chunk workspaces (%d)", R,
+             m->pf.cap < kChunkRows ? m->pf.cap : kChunkRows);
   const tl_model_config& c = m->cfg;
   tl_model::Prefill& p = m->pf;
   if (R <= m->bt.gemv_max) {
@@ -1795,12 +1809,12 @@ extern "C" int tl_model_batch_init(tl_model* m, int max_batch) {
   TL_REQUIRE(m->tp == 1, "tl_model_batch_init: multi-sequence decode is not available on tensor-parallel shards");
   TL_REQUIRE(!m->has_f32, "tl_model_batch_init: a model with F32 / BF16 projection matrices has no multi-sequence step "
                           "(its matrices run the unfused F32 route; decode the sequences one by one)");
-  TL_REQUIRE(max_batch >= 1 && max_batch <= kPrefillChunk, "tl_model_batch_init: max_batch %d outside 1..%d", max_batch,
-             kPrefillChunk);
+  TL_REQUIRE(max_batch >= 1 && max_batch <= kChunkRows, "tl_model_batch_init: max_batch %d outside 1..%d", max_batch,
+             kChunkRows);
   TL_REQUIRE(tl_batch_attn_supported(m->nh_l, m->nkv_l, m->head_dim),
              "tl_model_batch_init: head configuration %d/%d/%d is not supported by the batched decode attention", m->nh_l,
              m->nkv_l, m->head_dim);
-  TL_REQUIRE(max_batch <= (m->cfg.max_position_embeddings < kPrefillChunk ? m->cfg.max_position_embeddings : kPrefillChunk),
+  TL_REQUIRE(max_batch <= (m->cfg.max_position_embeddings < kChunkRows ? m->cfg.max_position_embeddings : kChunkRows),
              "tl_model_batch_init: max_batch %d exceeds the chunk capacity of this model", max_batch);
   TL_HIP(hipStreamSynchronize(m->stream));
   tl_model::Batch& b = m->bt;
@@ -1901,7 +1915,7 @@ extern "C" int tl_model_batch_prefill_packed(tl_model* m, int n_tokens, const in
                last_rows_host[j]);
   hipStream_t s = m->stream;
   const size_t H = c.hidden_size;
-  const int chunk = m->pf.cap;  // tokens the chunk workspaces hold: min(kPrefillChunk, max_position_embeddings)
+  const int chunk = chunk_tokens(m);
   TL_REQUIRE(chunk >= 1 && chunk <= kPrefillChunk, "tl_model_batch_prefill_packed: workspaces are missing");
   for (int c0 = 0; c0 < n_tokens; c0 += chunk) {
     const int T = n_tokens - c0 < chunk ? n_tokens - c0 : chunk;
