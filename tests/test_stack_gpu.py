@@ -383,3 +383,42 @@ def test_generation_through_the_host_session(env, tmp_path):
     synth.write_stack_dir(str(tmp_path / "bad"), bad, tensors)
     with pytest.raises(hostapi.TlHostError, match="Ralasun"):
         hostapi.Session(str(tmp_path / "bad"), 0, 64)
+
+
+@pytest.mark.parametrize("family", ["windows", "sink", "latent", "chunk"])
+def test_half_attention_routes(pkg, monkeypatch, family):
+    """The two-part f16 attention of a chunk against the FP32 matrix kernel (TL_HATTN=0): windows that end inside a tile and head
+    sizes 64, 128 and 128 over 64, a sink with unequal groups, expanded latent rows of 96 under a window with gated heads, and
+    chunked masks; a prompt that is walked whole and one that is continued, lengths off every tile. Three-term products: only the
+    attention differs, by 32-bit rounding (2^-21 of a score of a few units, halved on average over independent errors): 3e-5 of
+    the logits' size holds three layers of it."""
+    from tinyllama_cpp_amd import engine, synth
+    engine.init(0)
+    if family == "windows":
+        cfg = synth.stack_config(128, 90, [synth.stack_layer(4, 2, 64, 64, 40), synth.stack_layer(2, 1, 128, 128, None),
+                                           synth.stack_layer(6, 2, 128, 64, 33)])
+        tensors = synth.build_stack(cfg, 3)
+    elif family == "sink":
+        cfg = synth.sogalix_config(128, 90, [synth.sogalix_layer("attention", synth.sogalix_attention(6, 2, 64, 64, q_temp=(0.5, 20)), ff=64),
+                                             synth.sogalix_layer("attention", synth.sogalix_attention(1, 1, 128, 128), ff=64),
+                                             synth.sogalix_layer("latent_attention", synth.sogalix_latent(3, 64, 32, 64, 48, 40), ff=64)])
+        tensors = synth.build_sogalix(cfg, 3)
+    elif family == "latent":
+        cfg = synth.madudra_config(128, 90, [synth.madudra_layer("latent_attention", synth.madudra_latent(5, 64, 32, 64, 48, 40, w))
+                                             for w in (50, 0, 129)])
+        tensors = synth.build_madudra(cfg, 3)
+    else:
+        cfg = synth.ratuzen_config(128, 90, [synth.ratuzen_layer("parallel", synth.ratuzen_chunked(4, 1, 64, 64, c, 2, 16, 16, [0.5, 0.7]), ff=64)
+                                             for c in (48, 100)])
+        tensors = synth.build_ratuzen(cfg, 3)
+    toks = np.random.default_rng(5).integers(0, 90, 420).astype(np.int32)
+    m = engine.StackModel(cfg, 512, tensors).load(tensors)
+    m.set_prefill(3, 1)
+    got = []
+    for route in ("0", "1"):
+        monkeypatch.setenv("TL_HATTN", route)
+        m.reset_kv()
+        got.append(np.stack([np.array(m.prefill(toks[:a], 0) if a < 400 else m.prefill(toks[333:a], 333), np.float64) for a in (65, 333, 420)]))
+    m.free()
+    assert np.isfinite(got[1]).all() and not np.array_equal(got[0], got[1])
+    assert np.linalg.norm(got[1] - got[0]) <= 3e-5 * np.linalg.norm(got[0]), np.linalg.norm(got[1] - got[0]) / np.linalg.norm(got[0])

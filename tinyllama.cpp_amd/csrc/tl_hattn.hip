@@ -26,6 +26,7 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 namespace {
 
 constexpr int HA_ROWS = 128, HA_MAX_SPLIT = 16, HA_MAX_SLOTS = 2048;
+constexpr float LOG2E = 1.44269504088896340736f;
 constexpr float HA_P_BITS = 12.f;  // probabilities are held times 2^12: their second part stays normal down to 2^-15
 
 __device__ __forceinline__ int acc_row(int e, int h) { return (e & 3) + 8 * (e >> 2) + 4 * h; }
@@ -46,40 +47,50 @@ __device__ __forceinline__ void two_parts(const float (&x)[8], float f, half8& h
   }
 }
 
-// tile (blockIdx.x) of kv head (blockIdx.y): K then V fragments, 64 HD halves each, and the two exponents
-template <int HD>
-__global__ __launch_bounds__(256) void kv_planes_kernel(const float* __restrict__ kc, const float* __restrict__ vc, int len, int nkv,
-                                                        _Float16* __restrict__ planes, int* __restrict__ exps, int tiles) {
-  constexpr int PT = HD / 64;  // fragments of each operand per thread
+struct HPlanesArgs {
+  const float *kc, *vc;  // key rows kld floats apart, a head's part khs apart; value rows vld apart
+  int kld, khs, vld, lo, len, nkv, tile0, tiles;  // rows lo .. len - 1; tiles tile0 .. tile0 + tiles - 1 (others' rows: zeros)
+  _Float16* planes;      // [nkv][tiles][(KD + VD) * 64]: K then V fragments
+  int* exps;             // [nkv][tiles][2]
+};
+template <int KD, int VD>
+__global__ __launch_bounds__(256) void kv_planes_kernel(const HPlanesArgs a) {
+  constexpr int PK = (KD + 63) / 64, PV = (VD + 63) / 64;  // fragments of each operand per thread
   __shared__ float red[8];
-  const int tile = blockIdx.x, kvh = blockIdx.y, tid = threadIdx.x, p0 = tile * 32;
-  const size_t row = (size_t)nkv * HD;
-  const float *kp = kc + (size_t)kvh * HD, *vp = vc + (size_t)kvh * HD;
-  float k[PT][8], v[PT][8], mk = 0.f, mv = 0.f;
+  const int tile = blockIdx.x, kvh = blockIdx.y, tid = threadIdx.x, p0 = (a.tile0 + tile) * 32;
+  const float *kp = a.kc + (size_t)kvh * a.khs, *vp = a.vc + (size_t)kvh * VD;
+  float k[PK][8], v[PV][8], mk = 0.f, mv = 0.f;
 #pragma unroll
-  for (int t = 0; t < PT; ++t) {
+  for (int t = 0; t < PK; ++t) {
     const int f = tid + 256 * t, lane = f & 63, r = lane & 31, h = lane >> 5, g = f >> 6;
-    f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
-    if (p0 + r < len) {
-      const float* src = kp + (size_t)(p0 + r) * row + 16 * g + 8 * h;
-      a = *reinterpret_cast<const f32x4*>(src);
-      b = *reinterpret_cast<const f32x4*>(src + 4);
+    f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = x;
+    if (f < 4 * KD && p0 + r >= a.lo && p0 + r < a.len) {
+      const float* src = kp + (size_t)(p0 + r) * a.kld + 16 * g + 8 * h;
+      x = *reinterpret_cast<const f32x4*>(src);
+      y = *reinterpret_cast<const f32x4*>(src + 4);
     }
-    const int j = g / (HD / 32), d = 32 * (g % (HD / 32)) + r;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) k[t][i] = i < 4 ? x[i & 3] : y[i & 3];
+  }
+#pragma unroll
+  for (int t = 0; t < PV; ++t) {
+    const int f = tid + 256 * t, lane = f & 63, r = lane & 31, h = lane >> 5, g = f >> 6;
+    const int j = g / (VD / 32), d = 32 * (g % (VD / 32)) + r;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      k[t][i] = i < 4 ? a[i & 3] : b[i & 3];
       const int key = p0 + acc_row(8 * j + i, h);
-      v[t][i] = key < len ? vp[(size_t)key * row + d] : 0.f;
+      v[t][i] = f < 4 * VD && key >= a.lo && key < a.len ? vp[(size_t)key * a.vld + d] : 0.f;
     }
   }
 #pragma unroll
-  for (int t = 0; t < PT; ++t)
+  for (int i = 0; i < 8; ++i) {  // (an infinity or a NaN spoils its own key only)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {  // (an infinity or a NaN spoils its own key only)
+    for (int t = 0; t < PK; ++t)
       if (fabsf(k[t][i]) < INFINITY) mk = fmaxf(mk, fabsf(k[t][i]));
+#pragma unroll
+    for (int t = 0; t < PV; ++t)
       if (fabsf(v[t][i]) < INFINITY) mv = fmaxf(mv, fabsf(v[t][i]));
-    }
+  }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) {
     mk = fmaxf(mk, __shfl_xor(mk, o));
@@ -92,22 +103,29 @@ __global__ __launch_bounds__(256) void kv_planes_kernel(const float* __restrict_
   __syncthreads();
   const int ek = scale_exp(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
   const int ev = scale_exp(fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7])));
+  const size_t at = (size_t)kvh * a.tiles + tile;
   if (tid == 0) {
-    exps[2 * ((size_t)kvh * tiles + tile)] = ek;
-    exps[2 * ((size_t)kvh * tiles + tile) + 1] = ev;
+    a.exps[2 * at] = ek;
+    a.exps[2 * at + 1] = ev;
   }
-  _Float16* out = planes + ((size_t)kvh * tiles + tile) * (HD * 128);
+  _Float16* out = a.planes + at * ((KD + VD) * 64);
   const float fk = pow2i(ek), fv = pow2i(ev);
+  half8 hi, lo;
 #pragma unroll
-  for (int t = 0; t < PT; ++t) {
+  for (int t = 0; t < PK; ++t) {
     const int f = tid + 256 * t, lane = f & 63, g = f >> 6;
-    half8 hi, lo;
+    if (f >= 4 * KD) break;
     two_parts(k[t], fk, hi, lo);
     *reinterpret_cast<half8*>(out + ((size_t)(2 * g) * 64 + lane) * 8) = hi;
     *reinterpret_cast<half8*>(out + ((size_t)(2 * g + 1) * 64 + lane) * 8) = lo;
+  }
+#pragma unroll
+  for (int t = 0; t < PV; ++t) {
+    const int f = tid + 256 * t, lane = f & 63, g = f >> 6;
+    if (f >= 4 * VD) break;
     two_parts(v[t], fv, hi, lo);
-    *reinterpret_cast<half8*>(out + HD * 64 + ((size_t)(2 * g) * 64 + lane) * 8) = hi;
-    *reinterpret_cast<half8*>(out + HD * 64 + ((size_t)(2 * g + 1) * 64 + lane) * 8) = lo;
+    *reinterpret_cast<half8*>(out + KD * 64 + ((size_t)(2 * g) * 64 + lane) * 8) = hi;
+    *reinterpret_cast<half8*>(out + KD * 64 + ((size_t)(2 * g + 1) * 64 + lane) * 8) = lo;
   }
 }
 
@@ -118,40 +136,63 @@ __device__ __forceinline__ float half_max(float v) {
 }
 
 struct HAttnArgs {
-  const float* q;          // [T][nh][HD]
-  const _Float16* planes;  // [nkv][tiles][HD * 128]
-  const int* exps;         // [nkv][tiles][2]
-  float* out;              // [T][nh][HD]
-  float* part;             // [slot][HA_ROWS][HD]
+  TlHattn x;
+  const _Float16* planes;
+  const int* exps;
+  float* part;             // [slot][HA_ROWS][VD]
   float2* ml;              // [slot][HA_ROWS] (maximum in bits, sum)
-  int T, start_pos, nkv, group, tiles, splits, piece;
+  int group, tile0, tiles, splits, piece;
   float scale;             // times log2(e)
 };
-// key tiles of row tile rt (rows rt * 128 ..: row = query * group + head of the group)
-__host__ __device__ __forceinline__ int row_tiles(int T, int start_pos, int group, int rt) {
+// first position that position i sees
+__host__ __device__ __forceinline__ int first_key(const TlHattn& x, int i) {
+  int lo = x.window > 0 && i - x.window + 1 > 0 ? i - x.window + 1 : 0;
+  if (x.chunk > 0 && i - i % x.chunk > lo) lo = i - i % x.chunk;
+  return lo;
+}
+// key tiles [lo, hi) of row tile rt (rows rt * 128 ..: row = query * group + head of the group)
+struct TileRange {
+  int lo, hi;
+};
+__host__ __device__ __forceinline__ TileRange row_tiles(const TlHattn& x, int group, int rt) {
   const int last = (rt * HA_ROWS + HA_ROWS - 1) / group;
-  return (start_pos + (last < T ? last : T - 1)) / 32 + 1;
+  return {first_key(x, x.start_pos + rt * HA_ROWS / group) / 32, (x.start_pos + (last < x.T ? last : x.T - 1)) / 32 + 1};
 }
 
-template <int HD>
+// factor on a row's sum of values, whose weights are relative to 2^m and add up to l
+__device__ __forceinline__ float finish(const TlHattn& x, int t, int head, float m, float l) {
+  float f = 1.0f;
+  if (x.sink) {  // one more key without a value
+    const float sv = (x.sink_val ? x.sink_val[head] : 0.0f) * LOG2E, M = fmaxf(m, sv);
+    f = __builtin_amdgcn_exp2f(m - M);
+    l = l * f + __builtin_amdgcn_exp2f(sv - M);
+  }
+  f /= l + x.eps;
+  return x.gate ? f / (1.0f + expf(-x.gate[(size_t)t * x.gate_ld + head])) : f;
+}
+
+template <int KD, int VD>
 __global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs a) {
-  constexpr int DS = HD / 16, DB = HD / 32, TILE = HD * 128, NLD = TILE / 8 / 256;
+  constexpr int DS = KD / 16, DB = VD / 32, TILE = (KD + VD) * 64, NLD = TILE / 8 / 256;
   __shared__ __attribute__((aligned(16))) _Float16 win[2][TILE];
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5, wave = tid >> 6;
   // workgroup L runs on XCD L mod 8: with a multiple of eight kv heads every L2 holds the planes of its own ones; the row
   // tiles with the most keys first
-  const int kvh = blockIdx.x % a.nkv, slot = blockIdx.x / a.nkv, split = slot % a.splits;
-  const int nrt = (a.T * a.group + HA_ROWS - 1) / HA_ROWS, rt = nrt - 1 - slot / a.splits;
-  const int nt = row_tiles(a.T, a.start_pos, a.group, rt), ns = (nt + a.piece - 1) / a.piece;
+  const int nkv = a.x.kv_heads;
+  const int kvh = blockIdx.x % nkv, slot = blockIdx.x / nkv, split = slot % a.splits;
+  const int rows = a.x.T * a.group, nrt = (rows + HA_ROWS - 1) / HA_ROWS, rt = nrt - 1 - slot / a.splits;
+  const TileRange range = row_tiles(a.x, a.group, rt);
+  const int nt = range.hi - range.lo, ns = (nt + a.piece - 1) / a.piece;
   if (split >= ns) return;
-  const int t0 = (int)((long long)nt * split / ns), t1 = (int)((long long)nt * (split + 1) / ns);
-  const int row = rt * HA_ROWS + wave * 32 + r, rows = a.T * a.group;
-  const int rq = (row < rows ? row : rows - 1) / a.group, rg = (row < rows ? row : rows - 1) - rq * a.group;
-  const int qpos = a.start_pos + rq;
+  const int t0 = range.lo + (int)((long long)nt * split / ns), t1 = range.lo + (int)((long long)nt * (split + 1) / ns);
+  const int row = rt * HA_ROWS + wave * 32 + r;
+  const int rq = (row < rows ? row : rows - 1) / a.group, head = kvh * a.group + (row < rows ? row : rows - 1) - rq * a.group;
+  const int qpos = a.x.start_pos + rq, qlo = first_key(a.x, qpos);
   const int row0 = __builtin_amdgcn_readfirstlane(rt * HA_ROWS + wave * 32);
-  const int wave_last = a.start_pos + min(row0 + 31, rows - 1) / a.group, wave_first = a.start_pos + min(row0, rows - 1) / a.group;
-  const u32x4* src = reinterpret_cast<const u32x4*>(a.planes + (size_t)kvh * a.tiles * TILE);
-  const int2* ex = reinterpret_cast<const int2*>(a.exps) + (size_t)kvh * a.tiles;
+  const int wave_last = a.x.start_pos + min(row0 + 31, rows - 1) / a.group, wave_first = a.x.start_pos + min(row0, rows - 1) / a.group;
+  const int lo_first = first_key(a.x, wave_first), lo_last = first_key(a.x, wave_last);
+  const u32x4* src = reinterpret_cast<const u32x4*>(a.planes + ((long long)kvh * a.tiles - a.tile0) * TILE);
+  const int2* ex = reinterpret_cast<const int2*>(a.exps) + ((long long)kvh * a.tiles - a.tile0);
   u32x4 stage[NLD];
   int2 stage_ex;
   auto load = [&](int t) __attribute__((always_inline)) {
@@ -164,15 +205,15 @@ __global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs a) {
     for (int i = 0; i < NLD; ++i) *reinterpret_cast<u32x4*>(&win[buf][(i * 256 + tid) * 8]) = stage[i];
   };
   load(t0);
-  const size_t q_at = ((size_t)rq * a.nkv * a.group + (size_t)kvh * a.group + rg) * HD;
+  const float* qp = a.x.q + (size_t)rq * a.x.ldq + (size_t)head * a.x.qhs + 8 * h;
   half8 qh[DS], ql[DS];
   float cq;
   {
     float x[DS][8], mx = 0.f;
 #pragma unroll
     for (int s = 0; s < DS; ++s) {
-      const f32x4 u = *reinterpret_cast<const f32x4*>(a.q + q_at + 16 * s + 8 * h);
-      const f32x4 w = *reinterpret_cast<const f32x4*>(a.q + q_at + 16 * s + 8 * h + 4);
+      const f32x4 u = *reinterpret_cast<const f32x4*>(qp + 16 * s);
+      const f32x4 w = *reinterpret_cast<const f32x4*>(qp + 16 * s + 4);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         x[s][i] = i < 4 ? u[i & 3] : w[i & 3];
@@ -200,9 +241,9 @@ __global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs a) {
     const int buf = (t - t0) & 1, p0 = t * 32;
     load(t + 1 < t1 ? t + 1 : t);  // (the last one is not stored for anybody)
     __builtin_amdgcn_sched_barrier(0);
-    if (p0 <= wave_last) {
+    if (p0 <= wave_last && p0 + 31 >= lo_first) {
       const half8* kf = reinterpret_cast<const half8*>(&win[buf][0]) + lane;
-      const half8* vf = reinterpret_cast<const half8*>(&win[buf][HD * 64]) + lane;
+      const half8* vf = reinterpret_cast<const half8*>(&win[buf][KD * 64]) + lane;
       f32x16 s;
 #pragma unroll
       for (int e = 0; e < 16; ++e) s[e] = 0.f;
@@ -230,9 +271,12 @@ __global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs a) {
       }
       __builtin_amdgcn_sched_barrier(0);
       const float c = cq * pow2i(-ek);
-      if (p0 + 31 > wave_first) {  // some query of the wave does not see all of the tile
+      if (p0 + 31 > wave_first || p0 < lo_last) {  // some query of the wave does not see all of the tile
 #pragma unroll
-        for (int e = 0; e < 16; ++e) s[e] = p0 + acc_row(e, h) <= qpos ? s[e] : -INFINITY;
+        for (int e = 0; e < 16; ++e) {
+          const int p = p0 + acc_row(e, h);
+          s[e] = p <= qpos && p >= qlo ? s[e] : -INFINITY;
+        }
       }
       float tmax = fmaxf(s[0], s[1]);
 #pragma unroll
@@ -306,12 +350,12 @@ __global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs a) {
   float f = unit;
   if (ns == 1) {
     if (row >= rows) return;
-    f = unit * (1.0f / (l + 1e-9f));
-    dst = a.out + q_at;
+    f = unit * finish(a.x, rq, head, mrun, l);
+    dst = a.x.out + ((size_t)rq * nkv * a.group + head) * VD;
   } else {
     const size_t at = (size_t)blockIdx.x * HA_ROWS + wave * 32 + r;
     if (h == 0) a.ml[at] = make_float2(mrun, l);
-    dst = a.part + at * HD;
+    dst = a.part + at * VD;
   }
 #pragma unroll
   for (int b = 0; b < DB; ++b)
@@ -322,17 +366,19 @@ __global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs a) {
     }
 }
 
-// rows of the row tiles with several pieces: HD / 4 threads a row
-template <int HD>
+// rows of the row tiles with several pieces: VD / 4 threads a row
+template <int VD>
 __global__ __launch_bounds__(256) void hattn_combine_kernel(const HAttnArgs a) {
-  constexpr int TR = HD / 4, RPB = 256 / TR;  // threads a row, rows a workgroup
+  constexpr int TR = VD / 4, RPB = 256 / TR;  // threads a row, rows a workgroup
   const int kvh = blockIdx.y, row = blockIdx.x * RPB + threadIdx.x / TR, c = threadIdx.x % TR;
-  if (row >= a.T * a.group) return;
-  const int rt = row / HA_ROWS, nrt = (a.T * a.group + HA_ROWS - 1) / HA_ROWS;
-  const int nt = row_tiles(a.T, a.start_pos, a.group, rt), ns = (nt + a.piece - 1) / a.piece;
+  const int rows = a.x.T * a.group, nkv = a.x.kv_heads;
+  if (row >= rows) return;
+  const int rt = row / HA_ROWS, nrt = (rows + HA_ROWS - 1) / HA_ROWS;
+  const TileRange range = row_tiles(a.x, a.group, rt);
+  const int ns = (range.hi - range.lo + a.piece - 1) / a.piece;
   if (ns == 1) return;  // (written by the piece itself)
-  const size_t at = ((size_t)(nrt - 1 - rt) * a.splits * a.nkv + kvh) * HA_ROWS + row % HA_ROWS;
-  const size_t step = (size_t)a.nkv * HA_ROWS;
+  const size_t at = ((size_t)(nrt - 1 - rt) * a.splits * nkv + kvh) * HA_ROWS + row % HA_ROWS;
+  const size_t step = (size_t)nkv * HA_ROWS;
   float2 ml[HA_MAX_SPLIT];
   f32x4 v[HA_MAX_SPLIT];
 #pragma unroll
@@ -340,7 +386,7 @@ __global__ __launch_bounds__(256) void hattn_combine_kernel(const HAttnArgs a) {
     const size_t p = at + (s < ns ? s : 0) * step;
     ml[s] = a.ml[p];
     if (s >= ns) ml[s].x = -INFINITY;
-    if (s < ns) v[s] = *reinterpret_cast<const f32x4*>(a.part + p * HD + 4 * c);
+    if (s < ns) v[s] = *reinterpret_cast<const f32x4*>(a.part + p * VD + 4 * c);
   }
   float M = ml[0].x;
 #pragma unroll
@@ -356,84 +402,95 @@ __global__ __launch_bounds__(256) void hattn_combine_kernel(const HAttnArgs a) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) sum[i] += w * v[s][i];
     }
-  const float inv = 1.0f / (L + 1e-9f);
-  const int rq = row / a.group, rg = row - rq * a.group;
+  const int rq = row / a.group, head = kvh * a.group + row - rq * a.group;
+  const float f = finish(a.x, rq, head, M, L);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) sum[i] *= inv;
-  *reinterpret_cast<f32x4*>(a.out + ((size_t)rq * a.nkv * a.group + (size_t)kvh * a.group + rg) * HD + 4 * c) = sum;
+  for (int i = 0; i < 4; ++i) sum[i] *= f;
+  *reinterpret_cast<f32x4*>(a.x.out + ((size_t)rq * nkv * a.group + head) * VD + 4 * c) = sum;
 }
 
-size_t plane_bytes(int tiles, int nkv, int hd) { return (size_t)tiles * nkv * hd * 128 * sizeof(_Float16); }
+size_t plane_bytes(int tiles, int nkv, int kd, int vd) { return (size_t)tiles * nkv * (kd + vd) * 64 * sizeof(_Float16); }
 size_t exps_bytes(int tiles, int nkv) { return ((size_t)tiles * nkv * 2 * sizeof(int) + 255) & ~(size_t)255; }
 
 // Number of pieces: the least rounds of 2 workgroups a CU times tiles a piece, plus what a piece costs beside its tiles
 // (first tile, queries, output: about eight tiles of 2 us) and the pieces' way through memory.
-int plan_splits(int T, int start_pos, int nkv, int group, int* piece_out) {
-  const int nrt = (T * group + HA_ROWS - 1) / HA_ROWS, most = row_tiles(T, start_pos, group, nrt - 1);
+int plan_splits(const TlHattn& x, int group, int* piece_out) {
+  const int nrt = (x.T * group + HA_ROWS - 1) / HA_ROWS;
   const int slots = 2 * tl_num_cus();
+  int most = 1;
+  for (int rt = 0; rt < nrt; ++rt) {
+    const TileRange g = row_tiles(x, group, rt);
+    if (g.hi - g.lo > most) most = g.hi - g.lo;
+  }
   int best = 1, best_piece = most;
   double best_cost = 1e30;
   for (int S = 1; S <= HA_MAX_SPLIT && S <= most; ++S) {
-    if (S > 1 && (long long)nrt * S * nkv > HA_MAX_SLOTS) break;
+    if (S > 1 && (long long)nrt * S * x.kv_heads > HA_MAX_SLOTS) break;
     const int piece = (most + S - 1) / S;
     long long items = 0;
-    for (int rt = 0; rt < nrt; ++rt) items += (row_tiles(T, start_pos, group, rt) + piece - 1) / piece;
-    const double rounds = (double)((items * nkv + slots - 1) / slots);
-    const double cost = rounds * (piece + 8) + (S > 1 ? 2.0 + (double)items * nkv / slots * 2.0 : 0.0);
+    for (int rt = 0; rt < nrt; ++rt) {
+      const TileRange g = row_tiles(x, group, rt);
+      items += (g.hi - g.lo + piece - 1) / piece;
+    }
+    const double rounds = (double)((items * x.kv_heads + slots - 1) / slots);
+    const double cost = rounds * (piece + 8) + (S > 1 ? 2.0 + (double)items * x.kv_heads / slots * 2.0 : 0.0);
     if (cost < best_cost) best_cost = cost, best = S, best_piece = piece;
   }
   *piece_out = best_piece;
   return best;
 }
 
-}  // namespace
-
-bool tl_hattn_supported(int nh, int nkv, int hd) { return (hd == 64 || hd == 128) && nkv > 0 && nh > 0 && nh % nkv == 0; }
-
-size_t tl_hattn_bytes(int max_len, int nkv, int hd) {
-  const int tiles = (max_len + 31) / 32;
-  return plane_bytes(tiles, nkv, hd) + exps_bytes(tiles, nkv) + (size_t)HA_MAX_SLOTS * HA_ROWS * (sizeof(float) * hd + sizeof(float2));
+template <int KD, int VD>
+void launch(const HPlanesArgs& p, const HAttnArgs& a, hipStream_t s) {
+  const int rows = a.x.T * a.group, nrt = (rows + HA_ROWS - 1) / HA_ROWS, per = 256 / (VD / 4);
+  kv_planes_kernel<KD, VD><<<dim3(p.tiles, p.nkv), 256, 0, s>>>(p);
+  hattn_kernel<KD, VD><<<dim3(nrt * a.splits * a.x.kv_heads), 256, 0, s>>>(a);
+  if (a.splits > 1) hattn_combine_kernel<VD><<<dim3((rows + per - 1) / per, a.x.kv_heads), 256, 0, s>>>(a);
 }
 
-// q [T][nh][hd] (rotated), caches [.][nkv][hd] already holding positions 0 .. start_pos + T - 1, out [T][nh][hd];
-// ws: tl_hattn_bytes of at least start_pos + T positions
-int tl_launch_hattn(const float* q, const float* kc, const float* vc, float* out, int T, int start_pos, int nh, int nkv, int hd,
-                    float scale, void* ws, size_t ws_bytes, hipStream_t s) {
-  TL_REQUIRE(tl_hattn_supported(nh, nkv, hd), "tl_launch_hattn: unsupported head shape");
-  if (T == 0) return 0;
-  const int len = start_pos + T, tiles = (len + 31) / 32;
-  TL_REQUIRE(ws && ws_bytes >= tl_hattn_bytes(len, nkv, hd), "tl_launch_hattn: workspace too small");
-  HAttnArgs a = {};
+}  // namespace
+
+// head sizes that are whole matrix instructions, and rows and heads at 16 bytes: wide loads of queries and keys
+bool tl_hattn_supported(const TlHattn& x) {
+  const bool sizes = x.vdim == 64 ? x.dim == 64 || x.dim == 96 || x.dim == 128 : x.vdim == 128 && x.dim == 128;
+  return sizes && x.kv_heads > 0 && x.kv_heads <= 65535 && x.heads > 0 && x.heads % x.kv_heads == 0 &&
+         ((x.ldq | x.qhs | x.kld | x.khs) & 3) == 0 && (((size_t)x.q | (size_t)x.kc | (size_t)x.out) & 15) == 0;
+}
+
+// for launches over at most max_keys positions (those that T tokens see), any T
+size_t tl_hattn_bytes(int max_keys, int kv_heads, int dim, int vdim) {
+  const int tiles = max_keys / 32 + 2;  // (a range of keys starts and ends inside a tile)
+  return plane_bytes(tiles, kv_heads, dim, vdim) + exps_bytes(tiles, kv_heads) +
+         (size_t)HA_MAX_SLOTS * HA_ROWS * (sizeof(float) * vdim + sizeof(float2));
+}
+
+// ws: tl_hattn_bytes of at least the positions that the tokens see
+int tl_launch_hattn(const TlHattn& x, void* ws, size_t ws_bytes, hipStream_t s) {
+  if (x.T == 0) return 0;
+  TL_REQUIRE(tl_hattn_supported(x) && x.T > 0 && x.start_pos >= 0, "tl_launch_hattn: unsupported shapes");
+  const int len = x.start_pos + x.T, lo = first_key(x, x.start_pos), tile0 = lo / 32, tiles = (len + 31) / 32 - tile0;
+  TL_REQUIRE(ws && ws_bytes >= tl_hattn_bytes(len - lo, x.kv_heads, x.dim, x.vdim), "tl_launch_hattn: workspace too small");
   unsigned char* w = static_cast<unsigned char*>(ws);
-  _Float16* planes = reinterpret_cast<_Float16*>(w);
-  w += plane_bytes(tiles, nkv, hd);
-  int* exps = reinterpret_cast<int*>(w);
-  w += exps_bytes(tiles, nkv);
-  a.q = q;
-  a.planes = planes;
-  a.exps = exps;
-  a.out = out;
+  HPlanesArgs p = {x.kc, x.vc, x.kld, x.khs, x.vld, lo, len, x.kv_heads, tile0, tiles, reinterpret_cast<_Float16*>(w), nullptr};
+  w += plane_bytes(tiles, x.kv_heads, x.dim, x.vdim);
+  p.exps = reinterpret_cast<int*>(w);
+  w += exps_bytes(tiles, x.kv_heads);
+  HAttnArgs a = {};
+  a.x = x;
+  a.planes = p.planes;
+  a.exps = p.exps;
   a.part = reinterpret_cast<float*>(w);
-  a.ml = reinterpret_cast<float2*>(w + (size_t)HA_MAX_SLOTS * HA_ROWS * sizeof(float) * hd);
-  a.T = T;
-  a.start_pos = start_pos;
-  a.nkv = nkv;
-  a.group = nh / nkv;
+  a.ml = reinterpret_cast<float2*>(w + (size_t)HA_MAX_SLOTS * HA_ROWS * sizeof(float) * x.vdim);
+  a.group = x.heads / x.kv_heads;
+  a.tile0 = tile0;
   a.tiles = tiles;
-  a.scale = scale * 1.44269504088896340736f;
-  a.splits = plan_splits(T, start_pos, nkv, a.group, &a.piece);
-  const int rows = T * a.group, nrt = (rows + HA_ROWS - 1) / HA_ROWS, per = 256 / (hd / 4);
-  TL_REQUIRE((long long)nrt * a.splits * nkv <= 0x7fffffff && nkv <= 65535, "tl_launch_hattn: launch too large");
-  const dim3 grid(nrt * a.splits * nkv), cgrid((rows + per - 1) / per, nkv);
-  if (hd == 128) {
-    kv_planes_kernel<128><<<dim3(tiles, nkv), 256, 0, s>>>(kc, vc, len, nkv, planes, exps, tiles);
-    hattn_kernel<128><<<grid, 256, 0, s>>>(a);
-    if (a.splits > 1) hattn_combine_kernel<128><<<cgrid, 256, 0, s>>>(a);
-  } else {
-    kv_planes_kernel<64><<<dim3(tiles, nkv), 256, 0, s>>>(kc, vc, len, nkv, planes, exps, tiles);
-    hattn_kernel<64><<<grid, 256, 0, s>>>(a);
-    if (a.splits > 1) hattn_combine_kernel<64><<<cgrid, 256, 0, s>>>(a);
-  }
+  a.scale = x.scale * LOG2E;
+  a.splits = plan_splits(x, a.group, &a.piece);
+  TL_REQUIRE(((long long)x.T * a.group / HA_ROWS + 1) * a.splits * x.kv_heads <= 0x7fffffff, "tl_launch_hattn: launch too large");
+  if (x.vdim == 128) launch<128, 128>(p, a, s);
+  else if (x.dim == 128) launch<128, 64>(p, a, s);
+  else if (x.dim == 96) launch<96, 64>(p, a, s);
+  else launch<64, 64>(p, a, s);
   TL_HIP(hipGetLastError());
   return 0;
 }

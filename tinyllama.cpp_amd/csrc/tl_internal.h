@@ -281,11 +281,22 @@ int tl_launch_hsplit(int mode, const float* x, const float* aux, void* planes, s
 // y = (resid ? resid : 0) + the pending sums (what the GEMM launch would have run itself)
 int tl_launch_ksplit_reduce(const GemmParts& g, const float* resid, float* y, hipStream_t s);
 
-// causal prefill attention in two-part f16 over a workspace of converted K/V tiles (tl_hattn.hip)
-bool tl_hattn_supported(int nh, int nkv, int hd);
-size_t tl_hattn_bytes(int max_len, int nkv, int hd);
-int tl_launch_hattn(const float* q, const float* kc, const float* vc, float* out, int T, int start_pos, int nh, int nkv, int hd,
-                    float scale, void* ws, size_t ws_bytes, hipStream_t s);
+// causal attention of several tokens over one cache in two-part f16, over a workspace of converted K/V tiles (tl_hattn.hip)
+struct TlHattn {
+  const float *q, *kc, *vc;  // [T][ldq], a head's part qhs apart; key rows kld apart, a head's part khs apart; value rows vld apart
+  float* out;                // [T][heads * vdim]
+  int ldq, qhs, kld, khs, vld;
+  int T, start_pos, heads, kv_heads, dim, vdim;  // rows 0 .. start_pos + T - 1 (those that a token sees) are in the cache
+  float scale, eps;          // eps is added to the sum of the weights
+  int window, chunk;         // > 0: position i sees the last `window` positions, its own chunk of `chunk` positions
+  int sink;                  // one more key of score sink_val[head] (NULL: 0) without a value
+  const float* sink_val;
+  const float* gate;         // optional, [T][gate_ld]: head h's output times sigmoid(gate[h])
+  int gate_ld;
+};
+bool tl_hattn_supported(const TlHattn& x);
+size_t tl_hattn_bytes(int max_keys, int kv_heads, int dim, int vdim);
+int tl_launch_hattn(const TlHattn& x, void* ws, size_t ws_bytes, hipStream_t s);
 // causal prefill attention on the FP32 matrix instruction (tl_prefill.hip)
 bool tl_attn_prefill_mfma_supported(int nh, int nkv, int hd);
 // planes != NULL: the output as the attn_output GEMM's activation planes (tl_launch_split's layout) instead of `out`

@@ -1451,13 +1451,27 @@ static int prefill_attn_half(tl_model* m, int l, int T, int start_pos, hipStream
   // (no split launch; TL_ATTN_PLANES=0 keeps the launch, for A/B runs and the bit-identity test)
   const char* ap = getenv("TL_ATTN_PLANES");
   const char* ha = getenv("TL_HATTN");  // 0: the FP32 attention kernel everywhere (A/B runs and tests)
-  if (terms == TL_TERMS_HALF && tl_hattn_supported(m->nh_l, m->nkv_l, hd) && !(ha && atoi(ha) == 0)) {
+  TlHattn x = {};
+  x.q = p.qb;
+  x.kc = m->kc(l);
+  x.vc = m->vc(l);
+  x.out = p.ab;
+  x.ldq = m->qd_l;
+  x.kld = x.vld = m->nkv_l * hd;
+  x.qhs = x.khs = x.dim = x.vdim = hd;
+  x.T = T;
+  x.start_pos = start_pos;
+  x.heads = m->nh_l;
+  x.kv_heads = m->nkv_l;
+  x.scale = scale;
+  x.eps = 1e-9f;
+  if (terms == TL_TERMS_HALF && tl_hattn_supported(x) && !(ha && atoi(ha) == 0)) {
     if (!p.hattn) {
-      const size_t bytes = tl_hattn_bytes(c.max_position_embeddings, m->nkv_l, hd);
+      const size_t bytes = tl_hattn_bytes(c.max_position_embeddings, m->nkv_l, hd, hd);
       TL_HIP(hipMalloc(&p.hattn, bytes));
       p.hattn_bytes = bytes;
     }
-    TL_TRY(tl_launch_hattn(p.qb, m->kc(l), m->vc(l), p.ab, T, start_pos, m->nh_l, m->nkv_l, hd, scale, p.hattn, p.hattn_bytes, s));
+    TL_TRY(tl_launch_hattn(x, p.hattn, p.hattn_bytes, s));
     TL_TRY(tl_launch_split(0, p.ab, nullptr, p.planes, ps, T, m->qd_l, terms, 0.f, s));
   } else if (terms != TL_TERMS_HALF && tl_attn_prefill_mfma_supported(m->nh_l, m->nkv_l, hd) && !(ap && atoi(ap) == 0)) {
     TL_TRY(tl_launch_attn_prefill_mfma(p.qb, m->kc(l), m->vc(l), p.ab, T, start_pos, m->nh_l, m->nkv_l, hd, scale, s, p.planes,

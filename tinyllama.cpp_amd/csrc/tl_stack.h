@@ -127,6 +127,9 @@ struct SwaArgs {
   int chunk;
   const float* gate;  // optional, token t at gate + t * gate_ld (not with shared): head h's output is multiplied by sigmoid(gate[h])
   int gate_ld;
+  // optional: workspace of the two-part f16 kernel (tl_hattn.hip), tl_hattn_bytes of the keys that the tokens see
+  void* half_ws;
+  size_t half_ws_bytes;
 };
 int tl_launch_swa(const SwaArgs& a, hipStream_t s);
 int tl_swa_splits(int T, int window, int max_pos, int keep_first = 0);  // splits worth having for T tokens over a cache of max_pos rows

@@ -181,6 +181,8 @@ struct TlStack {
   int max_lq = 0, max_lqa = 0, max_gd = 0, gdelta_layers = 0;
   float *act_buf = nullptr, *eout = nullptr, *sact = nullptr, *sout = nullptr, *sgate = nullptr;
   float* wts = nullptr;
+  unsigned char* half_ws = nullptr;  // converted K/V tiles and partial outputs of a chunk's attention (tl_hattn.hip)
+  size_t half_bytes = 0;
   float* swa_ws = nullptr;  // partial results of split attention launches (few tokens, long windows)
   unsigned* swa_cnt = nullptr;  // their arrival counters (zero between launches)
   int *ids = nullptr, *off = nullptr, *slot_of = nullptr;
@@ -1209,6 +1211,15 @@ int tl_stack_finalize(TlStack* st, hipStream_t s) {
         ws = n > ws ? n : ws;
       }
     TL_TRY(dev_alloc(st, &st->swa_ws, ws));
+    for (const Layer* Lp : mixers) {  // chunks of 16 tokens on
+      const tl_layer_spec& sp = Lp->sp;
+      const bool lat = sp.mixer == TL_MIXER_LATENT && st->latent_expand > 0;
+      if (C < 16 || (sp.mixer != TL_MIXER_SWA && !lat) || (sp.vdim != 64 && sp.vdim != 128)) continue;
+      const int bound = swa_bound(sp), keys = bound > 0 && bound + (int)C < st->cfg.max_positions ? bound + (int)C : st->cfg.max_positions;
+      const size_t n = tl_hattn_bytes(keys, lat ? sp.heads : sp.kv_heads, lat ? sp.dim + sp.rot_dim : sp.dim, sp.vdim);
+      st->half_bytes = n > st->half_bytes ? n : st->half_bytes;
+    }
+    if (st->half_bytes) TL_TRY(dev_alloc(st, &st->half_ws, st->half_bytes));
     const size_t heads = st->max_heads > 0 ? st->max_heads : 1;
     TL_TRY(dev_alloc(st, &st->swa_cnt, 4 * heads));
     TL_HIP(hipMemsetAsync(st->swa_cnt, 0, sizeof(unsigned) * 4 * heads, s));
@@ -1670,6 +1681,8 @@ int swa_mixer(TlStack* st, Layer& L, const Layer& Wt, const float* in, int T, in
   a.nsplit = tl_swa_splits(T, swa_bound(sp), c.max_positions, sp.keep_first);
   a.ws = st->swa_ws;
   a.done_cnt = st->swa_cnt;
+  a.half_ws = st->half_ws;
+  a.half_ws_bytes = st->half_bytes;
   if (sp.score_maps == 2) {
     // two score maps per head over the same values: q and k rows hold [map 1 | map 2] per head, so each map is a launch over
     // every second block of dim; then o = (a1 - lambda a2) / rms (1 - diff_init) sigmoid(gate)
@@ -2000,6 +2013,8 @@ int latent_mixer(TlStack* st, Layer& L, const float* in, int T, int start_pos, c
     e.scale = sp.scale;
     e.start_pos = start_pos;
     e.nsplit = 1;
+    e.half_ws = st->half_ws;
+    e.half_ws_bytes = st->half_bytes;
     TL_TRY(tl_launch_swa(e, s));
     if (sp.head_gate) TL_TRY(tl_launch_head_gate(st->att, st->qkv + L.gate_off, ld, T, H, sp.vdim, s));
     if (sp.out_gate) TL_TRY(tl_launch_out_gate(st->att, st->qkv + L.gate_off, ld, T, L.od, s));

@@ -19,6 +19,7 @@
 #include <math.h>
 #include <stdlib.h>
 
+#include "tl_internal.h"
 #include "tl_stack.h"
 
 namespace {
@@ -728,6 +729,38 @@ static bool swa_mfma_wanted(const SwaArgs& a) {
   return on && a.T >= 16 && db <= 4 && sizeof(float) * swa_mfma_lds_floats(a.dim, db) <= 160 * 1024;
 }
 
+// ... and, where the caller has a workspace and the score is a plain one (window, chunk, sink and gate aside), to the two-part
+// f16 products of tl_hattn.hip (TL_HATTN=0: never): 1999 tokens, 32 heads of 64 over 8 kv heads or of 96 over their own, 110-140 us
+// against 571 in FP32; level with it from 16 tokens on
+static bool swa_half(const SwaArgs& a, TlHattn* x) {
+  const char* e = getenv("TL_HATTN");
+  if (!a.half_ws || a.pos_dev || a.sigmoid || a.softcap > 0.0f || a.dist_r1 || a.keep_first || (e && atoi(e) == 0)) return false;
+  x->q = a.q;
+  x->kc = a.kc;
+  x->vc = a.vc;
+  x->out = a.out;
+  x->ldq = a.ldq;
+  x->qhs = a.q_hstride > 0 ? a.q_hstride : a.dim;
+  x->khs = a.k_hstride > 0 ? a.k_hstride : a.dim;
+  x->kld = a.kld > 0 ? a.kld : a.kv_heads * x->khs;
+  x->vld = a.vld > 0 ? a.vld : a.kv_heads * a.vdim;
+  x->T = a.T;
+  x->start_pos = a.start_pos;
+  x->heads = a.heads;
+  x->kv_heads = a.kv_heads;
+  x->dim = a.dim;
+  x->vdim = a.vdim;
+  x->scale = a.scale;
+  x->eps = 0.0f;
+  x->window = a.window;
+  x->chunk = a.chunk;
+  x->sink = a.sink;
+  x->sink_val = a.sink_val;
+  x->gate = a.gate;
+  x->gate_ld = a.gate_ld;
+  return tl_hattn_supported(*x);
+}
+
 // splits of the shared-row kernel for tokens that see at most `window` of max_pos positions; 0: the shapes are not its own
 // (TL_SWA_SHARED=0: never)
 int tl_swa_shared_splits(const SwaArgs& a, int max_pos) {
@@ -768,6 +801,8 @@ int tl_launch_swa(const SwaArgs& a, hipStream_t s) {
     return a.vdim <= 256 ? launch_swa_shared<1>(a, s) : launch_swa_shared<2>(a, s);
   }
   if (swa_mfma_wanted(a)) {
+    TlHattn x = {};
+    if (swa_half(a, &x)) return tl_launch_hattn(x, a.half_ws, a.half_ws_bytes, s);
     switch ((a.vdim + 31) / 32) {
       case 1: return launch_swa_mfma<1>(a, s);
       case 2: return launch_swa_mfma<2>(a, s);
