@@ -422,3 +422,24 @@ def test_half_attention_routes(pkg, monkeypatch, family):
     m.free()
     assert np.isfinite(got[1]).all() and not np.array_equal(got[0], got[1])
     assert np.linalg.norm(got[1] - got[0]) <= 3e-5 * np.linalg.norm(got[0]), np.linalg.norm(got[1] - got[0]) / np.linalg.norm(got[0])
+
+
+@pytest.mark.parametrize("rows,cols,T,terms", [(64, 64, 64, 1), (65, 72, 63, 1), (130, 200, 65, 3), (33, 8, 16, 1), (70, 130, 40, 1),
+                                               (70, 131, 40, 3), (256, 192, 130, 1), (4096, 96, 1024, 1), (4100, 40, 1030, 1)])
+def test_dense_gemm_steps(pkg, rows, cols, T, terms):
+    """The pipelined steps of the dense GEMM: columns below, at and off one and two steps (zeros beyond the last), rows that are
+    not 16 bytes apart (narrow loads), both tiles with remainders. Against float64 over the operands that the terms keep: a bf16
+    activation exactly, three of them within 2^-24; a sum of cols products in FP32 is off by at most cols 2^-24 |w| . |x|."""
+    from tinyllama_cpp_amd import capi, engine, synth
+    engine.init(0)
+    rng = np.random.default_rng(rows + cols + T)
+    w = synth.to_bf16(rng.standard_normal((rows, cols)).astype(np.float32))
+    x = rng.standard_normal((T, cols)).astype(np.float32)
+    dev = engine.DeviceBuffer.from_numpy
+    wd, xd, yd = dev(w), dev(x), engine.DeviceBuffer(4 * T * rows)
+    capi.check(capi.lib().tl_dense_matmul(wd.ptr, rows, cols, xd.ptr, yd.ptr, T, terms, None), "tl_dense_matmul")
+    capi.check(capi.lib().tl_device_sync(), "sync")
+    W = synth.from_bf16(w).astype(np.float64)
+    X = (synth.from_bf16(synth.to_bf16(x)) if terms == 1 else x).astype(np.float64)
+    bound = (cols + 4) * 2.0 ** -24 * (np.abs(X) @ np.abs(W).T)
+    assert (np.abs(yd.to_numpy(np.float32, (T, rows)) - X @ W.T) <= bound).all()

@@ -2,14 +2,18 @@
 //
 //   GEMV (one token): a wave per output row, 16 B of weights per lane per step, widened exactly to FP32: FP32 arithmetic
 //   throughout, bound by the bytes of the matrix.
-//   GEMM (a chunk of tokens) on the matrix cores: v_mfma_f32_32x32x8_bf16 with the WEIGHTS as the A operand (M = output
+//   GEMM (a chunk of tokens) on the matrix cores: v_mfma_f32_32x32x16_bf16 with the WEIGHTS as the A operand (M = output
 //   features) and the tokens as B (N = tokens), so that a lane ends up holding 4 x 4 consecutive features of ONE token and
 //   stores them as 16-byte pieces of that token's output row. The FP32 activations are split while they are staged into
 //   LDS: terms = 1 keeps their bf16 rounding, terms = 3 keeps hi + mid + lo (3 x 8 mantissa bits = all 24 of an FP32
 //   value); the weights are bf16 to begin with, so three MFMAs per product reproduce the FP32 product exactly and only the
 //   order of the FP32 accumulation differs from a scalar loop.
-//   A workgroup of 4 waves owns a 64 x 64 or (enough rows and tokens) a 128 x 128 feature x token tile, BK = 32, with the
-//   next k-block's global loads in flight under the products of the block in LDS. Items may be gathered (x_rows), scattered (y_rows) and
+//   A workgroup of 4 waves owns a 64 x 64 or (enough rows and tokens) a 128 x 128 feature x token tile and walks 64 or 32
+//   columns a step. What bounds it is the way of the operands: a few workgroups a CU wait for the loads of a step, many of them
+//   for the 64 bytes a cycle that a CU's cache hands out (the activations are FP32 and every tile reads them). So two steps are
+//   in flight while a third is multiplied out of LDS, which needs loads without a branch around them: one kernel for wide
+//   loads, one for odd shapes. One step in flight behind a branch, products of eight columns: 2048 x 2048 times 64 / 512 / 1999
+//   tokens 30 / 39 / 63 us, now 17 / 19 / 47; 8192 x 2048 times 1999 182 -> 136 (495 TFLOP/s). Items may be gathered (x_rows), scattered (y_rows) and
 //   grouped (group_off: blockIdx.z = matrix of the group; tiles beyond a group's items leave at once), which is what the
 //   experts of a mixture need: the plan lives on the device, the grid is sized for the worst case.
 #include <math.h>
@@ -20,15 +24,10 @@
 
 namespace {
 
-typedef __attribute__((ext_vector_type(4))) short bf16x4;
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
-
-__device__ __forceinline__ unsigned short f2bf(float f) {  // round to nearest even
-  unsigned u = __float_as_uint(f);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (unsigned short)(u >> 16);
-}
-__device__ __forceinline__ float bf2f(unsigned short h) { return tl_bf2f(h); }
 
 // y = g * sigmoid(alpha * g) * (u + 1), g = min(gate, limit), u = clamp(up, -limit, limit)  (tl_moe.hip has the operator)
 __device__ __forceinline__ float dense_glu(float g, float u, float limit, float alpha, float up_add) {
@@ -37,19 +36,21 @@ __device__ __forceinline__ float dense_glu(float g, float u, float limit, float 
   return g / (1.0f + expf(-alpha * g)) * (u + up_add);
 }
 
-constexpr int BK = 32, LDK = 40;  // LDK: padded row of a tile in LDS (80 B, keeps 16 B / 8 B alignment)
-
-// A workgroup of 4 waves (2 x 2) owns a (64 WM)-feature x (64 WN)-token tile; a wave WM x WN products of 32 x 32. The next
-// k-block's weights and activations are asked for (into registers) before the products of the block in LDS start.
+// A workgroup of 4 waves (2 x 2) owns a (64 WM)-feature x (64 WN)-token tile; a wave WM x WN products of 32 x 32.
 // FIRST: the first 32 items are multiplied with two terms (terms == 1 otherwise): the second terms of those rows have a place of their
 // own in LDS, and the waves that own the 32 items add their products. (All three terms doubled those waves' products and cost 6 % of a
 // prompt of 2048 tokens at width 4096, since a launch of one round ends with its slowest workgroup; the second one alone costs 2 %.)
-template <int TERMS, int WM, int WN, bool FIRST = false>
+template <int TERMS, int WM, int WN, bool VEC, bool FIRST>
 __global__ __launch_bounds__(256) void dense_gemm_kernel(const DenseArgs a) {
   constexpr int BM = 64 * WM, BN = 64 * WN;
-  __shared__ __attribute__((aligned(16))) unsigned short Ws[BM][LDK];
-  __shared__ __attribute__((aligned(16))) unsigned short Xs[TERMS][BN][LDK];
-  __shared__ __attribute__((aligned(16))) unsigned short Xe[FIRST ? 32 : 1][LDK];
+  constexpr int BK = TERMS == 1 && WM == 1 ? 64 : 32;  // columns of a step
+  constexpr int LDK = BK + 8;                          // padded row of a tile in LDS: sixteen rows' 16-byte reads meet no bank twice
+  constexpr int NB = TERMS == 1 ? 2 : 1;               // steps in LDS (three terms in two would leave one workgroup a CU)
+  constexpr int KP = BK / 8, RP = 256 / KP;            // 16-byte pieces of a row, rows that the workgroup stages at a time
+  constexpr int PW = BM / RP, PX = BN / RP;            // pieces a thread stages
+  __shared__ __attribute__((aligned(16))) unsigned short Ws[NB][BM][LDK];
+  __shared__ __attribute__((aligned(16))) unsigned short Xs[NB][TERMS][BN][LDK];
+  __shared__ __attribute__((aligned(16))) unsigned short Xe[NB][FIRST ? 32 : 1][LDK];
   __shared__ int xrow[BN];
   const int tid = threadIdx.x, g = blockIdx.z;
   int lo = 0, hi = a.T;
@@ -72,54 +73,50 @@ __global__ __launch_bounds__(256) void dense_gemm_kernel(const DenseArgs a) {
   __syncthreads();
   const int wave = tid >> 6, lane = tid & 63, wm = wave & 1, wn = wave >> 1;
   const bool lead = FIRST && blockIdx.y == 0;
-  const int lr = tid >> 2, lk = (tid & 3) * 8;  // this thread stages 8 consecutive k of rows lr + 64 i of both tiles
+  const int lr = tid / KP, lk = (tid % KP) * 8;  // this thread stages 8 consecutive k of rows lr + RP i of both tiles
   const int K = a.cols;
-  const bool vec = (K & 7) == 0 && (a.ldx & 3) == 0 && ((size_t)X & 15) == 0 && ((size_t)W & 15) == 0;
-  const unsigned short* wp[WM];
-  const float* xp[WN];
-  bool wok[WM], xok[WN];
+  const unsigned short* wp[PW];
+  const float* xp[PX];
 #pragma unroll
-  for (int i = 0; i < WM; ++i) {
-    const int frow = f0 + lr + 64 * i;
-    wok[i] = frow < a.rows;
-    wp[i] = W + (size_t)(wok[i] ? frow : 0) * K;
+  for (int i = 0; i < PW; ++i) {  // (rows and items beyond the last: the first one's values, never stored)
+    const int frow = f0 + lr + RP * i;
+    wp[i] = W + (size_t)(frow < a.rows ? frow : 0) * K;
   }
 #pragma unroll
-  for (int j = 0; j < WN; ++j) {
-    const int xr = xrow[lr + 64 * j];
-    xok[j] = xr >= 0;
-    xp[j] = X + (size_t)(xok[j] ? xr : 0) * a.ldx;
+  for (int j = 0; j < PX; ++j) {
+    const int xr = xrow[lr + RP * j];
+    xp[j] = X + (size_t)(xr >= 0 ? xr : 0) * a.ldx;
   }
-  uint4 wreg[WM];
-  float xreg[WN][8];
-  auto fetch = [&](int k0) __attribute__((always_inline)) {
+  struct Step {
+    u32x4 w[PW];
+    f32x4 x[PX][2];
+  };
+  // a step's pieces; columns beyond K as zeros (a step beyond the last reads the last column's pieces again)
+  auto fetch = [&](Step& r, int k0) __attribute__((always_inline)) {
     const int k = k0 + lk;
-    if (vec && k + 8 <= K) {
+    if (VEC) {
+      const bool in = k < K;
+      const int kc = in ? k : 0;
 #pragma unroll
-      for (int i = 0; i < WM; ++i) wreg[i] = wok[i] ? *reinterpret_cast<const uint4*>(wp[i] + k) : make_uint4(0, 0, 0, 0);
+      for (int i = 0; i < PW; ++i) r.w[i] = *reinterpret_cast<const u32x4*>(wp[i] + kc);
 #pragma unroll
-      for (int j = 0; j < WN; ++j) {
-        float4 x0 = make_float4(0, 0, 0, 0), x1 = x0;
-        if (xok[j]) {
-          x0 = *reinterpret_cast<const float4*>(xp[j] + k);
-          x1 = *reinterpret_cast<const float4*>(xp[j] + k + 4);
-        }
-        xreg[j][0] = x0.x; xreg[j][1] = x0.y; xreg[j][2] = x0.z; xreg[j][3] = x0.w;
-        xreg[j][4] = x1.x; xreg[j][5] = x1.y; xreg[j][6] = x1.z; xreg[j][7] = x1.w;
+      for (int j = 0; j < PX; ++j) {
+        r.x[j][0] = *reinterpret_cast<const f32x4*>(xp[j] + kc);
+        r.x[j][1] = *reinterpret_cast<const f32x4*>(xp[j] + kc + 4);
       }
     } else {
 #pragma unroll
-      for (int i = 0; i < WM; ++i) {
+      for (int i = 0; i < PW; ++i) {
         unsigned short wv[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) wv[e] = (k + e < K && wok[i]) ? wp[i][k + e] : (unsigned short)0;
-        wreg[i].x = wv[0] | ((unsigned)wv[1] << 16); wreg[i].y = wv[2] | ((unsigned)wv[3] << 16);
-        wreg[i].z = wv[4] | ((unsigned)wv[5] << 16); wreg[i].w = wv[6] | ((unsigned)wv[7] << 16);
+        for (int e = 0; e < 8; ++e) wv[e] = k + e < K ? wp[i][k + e] : (unsigned short)0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r.w[i][e] = wv[2 * e] | ((unsigned)wv[2 * e + 1] << 16);
       }
 #pragma unroll
-      for (int j = 0; j < WN; ++j)
+      for (int j = 0; j < PX; ++j)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) xreg[j][e] = (k + e < K && xok[j]) ? xp[j][k + e] : 0.0f;
+        for (int e = 0; e < 8; ++e) r.x[j][e >> 2][e & 3] = k + e < K ? xp[j][k + e] : 0.0f;
     }
   };
   f32x16 acc[WM][WN];
@@ -129,65 +126,78 @@ __global__ __launch_bounds__(256) void dense_gemm_kernel(const DenseArgs a) {
     for (int j = 0; j < WN; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += BK) {
+  auto stage = [&](Step& r, int buf, int k0) __attribute__((always_inline)) {
+    const bool in = !VEC || k0 + lk < K;  // (VEC: a piece is inside or outside as a whole)
 #pragma unroll
-    for (int i = 0; i < WM; ++i) *reinterpret_cast<uint4*>(&Ws[lr + 64 * i][lk]) = wreg[i];
+    for (int i = 0; i < PW; ++i) *reinterpret_cast<u32x4*>(&Ws[buf][lr + RP * i][lk]) = in ? r.w[i] : u32x4{0, 0, 0, 0};
 #pragma unroll
-    for (int j = 0; j < WN; ++j) {
+    for (int j = 0; j < PX; ++j) {
+      float x[8];
 #pragma unroll
-      for (int t = 0; t < TERMS; ++t) {
-        unsigned short h[8];
+      for (int e = 0; e < 8; ++e) x[e] = in ? r.x[j][e >> 2][e & 3] : 0.0f;
+#pragma unroll
+      for (int t = 0; t < TERMS + (FIRST ? 1 : 0); ++t) {
+        if (t == TERMS && !(lead && lr + RP * j < 32)) break;
+        bf16x8 p;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          h[e] = f2bf(xreg[j][e]);
-          xreg[j][e] -= bf2f(h[e]);  // exact: the remainder of an FP32 value after its leading 8 bits
+          p[e] = (__bf16)x[e];
+          if (t + 1 < TERMS + (FIRST ? 1 : 0)) x[e] -= (float)p[e];  // exact: the remainder of an FP32 value after its leading 8 bits
         }
-        uint4 p;
-        p.x = h[0] | ((unsigned)h[1] << 16); p.y = h[2] | ((unsigned)h[3] << 16);
-        p.z = h[4] | ((unsigned)h[5] << 16); p.w = h[6] | ((unsigned)h[7] << 16);
-        *reinterpret_cast<uint4*>(&Xs[t][lr + 64 * j][lk]) = p;
-      }
-      if (FIRST && j == 0 && lead && lr < 32) {
-        unsigned short h[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) h[e] = f2bf(xreg[j][e]);
-        uint4 p;
-        p.x = h[0] | ((unsigned)h[1] << 16); p.y = h[2] | ((unsigned)h[3] << 16);
-        p.z = h[4] | ((unsigned)h[5] << 16); p.w = h[6] | ((unsigned)h[7] << 16);
-        *reinterpret_cast<uint4*>(&Xe[FIRST ? lr : 0][lk]) = p;
+        *reinterpret_cast<bf16x8*>(t < TERMS ? &Xs[buf][t < TERMS ? t : 0][lr + RP * j][lk] : &Xe[buf][FIRST ? (lr + RP * j) & 31 : 0][lk]) = p;
       }
     }
-    __syncthreads();
-    if (k0 + BK < K) fetch(k0 + BK);  // in flight while the products below run
+  };
+  auto multiply = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int ks = 0; ks < BK / 8; ++ks) {
-      const int kk = ks * 8 + (lane >> 5) * 4;
-      bf16x4 af[WM];
+    for (int ks = 0; ks < BK / 16; ++ks) {
+      const int kk = ks * 16 + (lane >> 5) * 8;
+      bf16x8 af[WM];
 #pragma unroll
-      for (int i = 0; i < WM; ++i) af[i] = *reinterpret_cast<const bf16x4*>(&Ws[(wm * WM + i) * 32 + (lane & 31)][kk]);
+      for (int i = 0; i < WM; ++i) af[i] = *reinterpret_cast<const bf16x8*>(&Ws[buf][(wm * WM + i) * 32 + (lane & 31)][kk]);
 #pragma unroll
       for (int t = TERMS - 1; t >= 0; --t) {  // small terms first
 #pragma unroll
         for (int j = 0; j < WN; ++j) {
-          const bf16x4 bfr = *reinterpret_cast<const bf16x4*>(&Xs[t][(wn * WN + j) * 32 + (lane & 31)][kk]);
+          const bf16x8 bfr = *reinterpret_cast<const bf16x8*>(&Xs[buf][t][(wn * WN + j) * 32 + (lane & 31)][kk]);
 #pragma unroll
-          for (int i = 0; i < WM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(af[i], bfr, acc[i][j], 0, 0, 0);
+          for (int i = 0; i < WM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i], bfr, acc[i][j], 0, 0, 0);
         }
       }
     }
     if (FIRST && lead && wn == 0) {  // (a loop of its own: the one above keeps its schedule)
 #pragma unroll
-      for (int ks = 0; ks < BK / 8; ++ks) {
-        const int kk = ks * 8 + (lane >> 5) * 4;
-        const bf16x4 bfr = *reinterpret_cast<const bf16x4*>(&Xe[FIRST ? lane & 31 : 0][kk]);
+      for (int ks = 0; ks < BK / 16; ++ks) {
+        const int kk = ks * 16 + (lane >> 5) * 8;
+        const bf16x8 bfr = *reinterpret_cast<const bf16x8*>(&Xe[buf][FIRST ? lane & 31 : 0][kk]);
 #pragma unroll
         for (int i = 0; i < WM; ++i)
-          acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(
-              *reinterpret_cast<const bf16x4*>(&Ws[(wm * WM + i) * 32 + (lane & 31)][kk]), bfr, acc[i][0], 0, 0, 0);
+          acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              *reinterpret_cast<const bf16x8*>(&Ws[buf][(wm * WM + i) * 32 + (lane & 31)][kk]), bfr, acc[i][0], 0, 0, 0);
       }
     }
-    __syncthreads();
+  };
+  // DEPTH steps' loads in flight: the one behind the step in LDS has arrived or is about to, the DEPTH-th after it is asked for
+  // now (four instead of two gain nothing)
+  constexpr int DEPTH = 2;
+  Step r[DEPTH];
+#pragma unroll
+  for (int u = 0; u < DEPTH; ++u) fetch(r[u], u * BK);
+  stage(r[0], 0, 0);
+  __syncthreads();
+  const int steps = (K + BK - 1) / BK;  // (rounded up to DEPTH: steps beyond the last multiply zeros)
+  for (int st = 0; st < steps; st += DEPTH) {
+#pragma unroll
+    for (int u = 0; u < DEPTH; ++u) {
+      const int k0 = (st + u) * BK, buf = u & (NB - 1);
+      fetch(r[u], k0 + DEPTH * BK);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(buf);
+      __builtin_amdgcn_sched_barrier(0);
+      if (NB == 1) __syncthreads();
+      stage(r[(u + 1) % DEPTH], buf ^ (NB - 1), k0 + BK);  // (NB == 2: its last readers are in front of the barrier of the step before)
+      __syncthreads();
+    }
   }
   // C layout: lane holds token (lane & 31) of a 32 x 32 product, features (e / 4) * 8 + (lane >> 5) * 4 + (e & 3)
   const bool v4 = (a.ldy & 3) == 0 && ((size_t)Y & 15) == 0;
@@ -279,26 +289,30 @@ int tl_launch_dense_gemm(const DenseArgs& a, hipStream_t s) {
   TL_REQUIRE(!a.bias || (!a.glu && groups == 1), "dense gemm: a bias with a gated unit or several matrices");
   // 128 x 128 tiles when there is enough of both sides to fill them (grouped launches: tokens per group on average)
   const long long per_group = a.group_off ? (long long)a.T / groups : a.T;
-  // Measured at width 4096, chunks of 512 tokens: a dense launch has too few 128 x 128 tiles to fill 256 CUs (6144 x 512:
-  // 192 tiles, 117 us against 109 us in 768 small ones); the experts' grouped launches, whose small tiles are mostly
+  // Measured: a dense launch needs a 128 x 128 tile a CU (192 tiles, 6144 rows, 4096 columns, 512 tokens: 80 us against 65 in
+  // small ones; 256 tiles, 4096 rows, 2048 columns, 1000 tokens: level; 256 tiles over 14336 columns: 265 against 333); the experts' grouped launches, whose small tiles are mostly
   // half-empty, gain from them with one term (221 -> 193 us) and lose with three (356 -> 413 us).
   const long long big_tiles = ((a.rows + 127) / 128) * ((per_group + 127) / 128) * groups;
   const char* force = getenv("TL_DENSE_TILE");  // 64 / 128: tests and A/B runs pick the tile themselves
   const bool big = force ? atoi(force) == 128
-                         : a.rows >= 256 && (a.group_off ? a.terms == 1 && per_group >= 96 : big_tiles >= 2 * tl_num_cus());
+                         : a.rows >= 256 && (a.group_off ? a.terms == 1 && per_group >= 96 : big_tiles >= tl_num_cus());
   const int BM = big ? 128 : 64, BN = big ? 128 : 64;
   dim3 grid((a.rows + BM - 1) / BM, (a.T + BN - 1) / BN, groups);
   TL_REQUIRE(grid.y <= 65535 && grid.z <= 65535, "dense gemm: launch too large");
   const bool first = a.exact_items > 0 && a.terms == 1;
+  // wide loads: every matrix, row and piece of eight columns at 16 bytes
+  const bool vec = (a.cols & 7) == 0 && (a.ldx & 3) == 0 && ((size_t)a.x & 15) == 0 && ((size_t)a.w & 15) == 0 && (a.x_gstride & 3) == 0;
+#define DENSE(T, W, F) (vec ? dense_gemm_kernel<T, W, W, true, F><<<grid, 256, 0, s>>>(a) : dense_gemm_kernel<T, W, W, false, F><<<grid, 256, 0, s>>>(a))
   if (big) {
-    if (first) dense_gemm_kernel<1, 2, 2, true><<<grid, 256, 0, s>>>(a);
-    else if (a.terms == 1) dense_gemm_kernel<1, 2, 2><<<grid, 256, 0, s>>>(a);
-    else dense_gemm_kernel<3, 2, 2><<<grid, 256, 0, s>>>(a);
+    if (first) DENSE(1, 2, true);
+    else if (a.terms == 1) DENSE(1, 2, false);
+    else DENSE(3, 2, false);
   } else {
-    if (first) dense_gemm_kernel<1, 1, 1, true><<<grid, 256, 0, s>>>(a);
-    else if (a.terms == 1) dense_gemm_kernel<1, 1, 1><<<grid, 256, 0, s>>>(a);
-    else dense_gemm_kernel<3, 1, 1><<<grid, 256, 0, s>>>(a);
+    if (first) DENSE(1, 1, true);
+    else if (a.terms == 1) DENSE(1, 1, false);
+    else DENSE(3, 1, false);
   }
+#undef DENSE
   TL_HIP(hipGetLastError());
   return 0;
 }
