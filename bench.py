@@ -924,11 +924,11 @@ def prefill_leg(model, S, cfg, mix, T, terms=6, reps=3, world=1):
         best = min(best, time.perf_counter() - t0)
     elems = sum(r * c for n, t, r, c in S.tensor_plan(cfg, mix) if n.startswith("blk.") and t != S.F32)
     flops = 2.0 * T * elems / world  # per GPU
-    # MFMAs per product: the integer-plane GEMM multiplies EXACT integer weights (one bf16 plane) with the activation in
-    # 3 / 2 / 1 bf16 planes (FP32-grade / 2^-17 / plain bf16); TL_GEMM_INT=0 (exact-dequantization kernel) spends 6 / 3 / 1
-    per_product = {6: 3, 3: 2, 1: 1}[terms] if os.environ.get("TL_GEMM_INT", "1") != "0" else terms
+    # matrix instructions per product: the f16 form multiplies exact weight operands with the activation's two f16 parts
+    # (32-bit grade, for 6 and 3 alike); 1: plain bf16
+    per_product = {6: 2, 3: 2, 1: 1}[terms]
     return {"prompt_tokens": T, "mfma_terms": terms, "mfma_per_product": per_product,
-            "precision": {6: "fp32-grade", 3: "2^-17 per product", 1: "bf16 activations"}[terms],
+            "precision": {6: "fp32-grade", 3: "fp32-grade", 1: "bf16 activations"}[terms],
             "ms": round(best * 1e3, 2), "tokens_per_s": round(T / best, 1),
             "gemm_tflops_algorithmic": round(flops / best / 1e12, 1),
             "bf16_mfma_tflops_executed": round(flops * per_product / best / 1e12, 1),

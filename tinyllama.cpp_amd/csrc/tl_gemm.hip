@@ -1717,8 +1717,9 @@ static int launch_gemm_dispatch(const QW& w, const __bf16* xp, size_t plane_stri
 
 // Up to three matrices over the same activation planes (q | k | v, gate | up) in one launch of the f16 kernel or of the
 // integer-plane kernel. Taken only when that changes no bit: all matrices of one format and width, and for every matrix the
-// number of K slices its own launch would use (the f16 kernel: one for the group). Outputs: with one slice y[i] directly; with more, the partial tiles go to defer[i] (required) for the consumer
-// to sum. *merged = false: nothing was launched, the caller runs the matrices one by one.
+// number of K slices its own launch would use (the f16 kernel: one for the group). Outputs: with one slice y[i] directly; with
+// more, the partial tiles go to defer[i] (required) for the consumer to sum. *merged = false: nothing was launched, the caller
+// runs the matrices one by one.
 int tl_launch_gemm_q_multi(const QW* w, int n, const void* planes, size_t plane_stride, float* const* y, int T, int terms,
                            hipStream_t s, GemmDefer* const* defer, bool* merged) {
   *merged = false;
