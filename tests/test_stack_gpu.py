@@ -443,3 +443,25 @@ def test_dense_gemm_steps(pkg, rows, cols, T, terms):
     X = (synth.from_bf16(synth.to_bf16(x)) if terms == 1 else x).astype(np.float64)
     bound = (cols + 4) * 2.0 ** -24 * (np.abs(X) @ np.abs(W).T)
     assert (np.abs(yd.to_numpy(np.float32, (T, rows)) - X @ W.T) <= bound).all()
+
+
+def test_causal_conv_output_behind_the_last_row(pkg):
+    """Channels at the end of wider rows, the output right behind the last row's: no overlap, whatever the row stride adds up to
+    (buffers that the allocator places back to back); one float earlier it is one, and refused."""
+    from tinyllama_cpp_amd import capi, engine, synth
+    engine.init(0)
+    rng = np.random.default_rng(2)
+    T, C, taps, ld, off = 9, 8, 3, 24, 16
+    x = rng.standard_normal(off + (T - 1) * ld + C + T * C).astype(np.float32)
+    w = synth.to_bf16(rng.standard_normal((C, taps)).astype(np.float32))
+    buf, wd = engine.DeviceBuffer.from_numpy(x), engine.DeviceBuffer.from_numpy(w)
+    end = buf.ptr + 4 * (off + (T - 1) * ld + C)
+    far, got = engine.DeviceBuffer(4 * T * C), []
+    for out in (far.ptr, end):
+        hist = engine.DeviceBuffer.from_numpy(np.zeros((taps - 1, C), np.float32))
+        capi.check(capi.lib().tl_causal_conv(buf.ptr + 4 * off, ld, C, taps, T, None, wd.ptr, hist.ptr, 0, 0, out, C, None), "conv")
+        capi.check(capi.lib().tl_device_sync(), "sync")
+        got.append(far.to_numpy(np.float32, (T, C)) if out == far.ptr else buf.to_numpy(np.float32, (x.size,))[-T * C:].reshape(T, C))
+    assert np.array_equal(got[0], got[1]) and np.abs(got[0]).max() > 0
+    hist = engine.DeviceBuffer.from_numpy(np.zeros((taps - 1, C), np.float32))
+    assert capi.lib().tl_causal_conv(buf.ptr + 4 * off, ld, C, taps, T, None, wd.ptr, hist.ptr, 0, 0, end - 4, C, None) != 0

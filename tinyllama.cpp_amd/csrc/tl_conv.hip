@@ -141,7 +141,8 @@ int tl_launch_causal_conv(const ConvArgs& a, hipStream_t s) {
   TL_REQUIRE(a.in && a.w && a.out && a.T > 0 && a.T <= 65535 && a.C > 0, "causal_conv: bad arguments");
   TL_REQUIRE(a.taps >= 1 && (a.taps == 1 || a.hist), "causal_conv: %d taps", a.taps);
   TL_REQUIRE(a.ldi >= a.C && a.ldo >= a.C, "causal_conv: row strides %d / %d below %d channels", a.ldi, a.ldo, a.C);
-  TL_REQUIRE(a.T == 1 || a.out + (size_t)a.T * a.ldo <= a.in || a.in + (size_t)a.T * a.ldi <= a.out,
+  // (the last row ends with its own C columns: what lies behind them may be the output)
+  TL_REQUIRE(a.T == 1 || a.out + (size_t)(a.T - 1) * a.ldo + a.C <= a.in || a.in + (size_t)(a.T - 1) * a.ldi + a.C <= a.out,
              "causal_conv: output over input with more than one token");
   TL_REQUIRE(a.act == 0 || a.act == 1, "causal_conv: activation %d", a.act);
   const bool al = a.T > 1 && (a.C & 3) == 0 && (a.ldi & 3) == 0 && (a.ldo & 3) == 0 && ((size_t)a.in & 15) == 0 &&
