@@ -229,3 +229,20 @@ def test_deferred_ksplit_reductions_are_bit_identical(pkg, monkeypatch):
         for other in ("10", "11"):
             for a, b in zip(got["01"], got[other]):
                 assert a.shape == b.shape and np.array_equal(a, b), (shape, other, np.abs(a.astype(np.float64) - b).max())
+
+
+def test_packed_prompts_longer_than_a_sequence(pkg):
+    """A packed batch of more tokens than a sequence has positions goes through as one chunk: every prompt's last logits are those
+    of its own prefill, up to the order of 32-bit sums (2^-22 a layer and product)."""
+    from tinyllama_cpp_amd import engine as E
+    E.init(0)
+    cfg, tensors = pkg.synth.build_model(dict(pkg.synth.SHAPES["tiny-gqa"], max_pos=96), "q4_k_m", seed=8)
+    m = E.Model(cfg).load(tensors)
+    m.batch_init(9)
+    rng = np.random.default_rng(8)
+    prompts = [rng.integers(0, cfg["vocab"], n).astype(np.int32) for n in (96, 95, 61, 96, 33, 96, 90, 17, 96)]  # 680 tokens
+    alone = np.stack([m.batch_prefill(i, p) for i, p in enumerate(prompts)])
+    packed, ids = m.batch_prefill_packed(prompts)
+    assert np.linalg.norm(packed - alone) <= 4e-6 * np.linalg.norm(alone)
+    assert np.array_equal(ids, packed.argmax(1))
+    m.free()

@@ -1285,7 +1285,7 @@ extern "C" int tl_model_generate_sampled(tl_model* m, int first_token, int start
 
 // ---- batched prefill (forward_device_batch_prefill model.cpp:1526-1862; math of CPUBatchProcessor::forward_cpu_batch,
 //      cpu_batch_processor.cpp:11-281) -----------------------------------------------------------------------------------
-// A chunk of up to kPrefillChunk tokens goes through every layer as a batch: RMSNorm -> bf16 planes, q/k/v GEMMs on
+// A chunk of up to kPrefillChunk tokens goes through every layer as a batch: RMSNorm -> activation planes, q/k/v GEMMs on
 // the matrix cores (tl_gemm.hip), batched RoPE + KV write, causal attention from the cache (tl_prefill.hip), O GEMM +
 // residual, RMSNorm -> planes, gate/up GEMMs, SwiGLU -> planes, down GEMM + residual. Longer prompts are walked chunk by
 // chunk over the growing cache. Short prompts (< prefill_min_batch) replay the decode graph token by token instead (same positions, KV contents and logits to ~1e-6).
@@ -1312,8 +1312,9 @@ static int ensure_prefill_ws(tl_model* m, bool all_logits) {
   const tl_model_config& c = m->cfg;
   tl_model::Prefill& p = m->pf;
   if (p.cap == 0) {
-    const int most = m->half_planes && m->tp == 1 ? kPrefillChunk : kChunkRows;
-    const int cap = c.max_position_embeddings < most ? c.max_position_embeddings : most;
+    // (a packed batch of prompts can hold more tokens than a sequence has positions: 1.1B Q4_K_M, 21 prompts of up to 150 tokens
+    // and 512 positions, 13.7 ms in chunks of 512, 10.1 whole)
+    const int cap = m->half_planes && m->tp == 1 ? kPrefillChunk : c.max_position_embeddings < kChunkRows ? c.max_position_embeddings : kChunkRows;
     const size_t H = c.hidden_size, maxk = H > (size_t)m->I_l ? H : (size_t)m->I_l;
     const size_t kmax = maxk > (size_t)m->qd_l ? maxk : (size_t)m->qd_l;
     p.plane_stride = tl_gemm_padded_tokens(cap) * kmax;

@@ -730,8 +730,8 @@ static bool swa_mfma_wanted(const SwaArgs& a) {
 }
 
 // ... and, where the caller has a workspace and the score is a plain one (window, chunk, sink and gate aside), to the two-part
-// f16 products of tl_hattn.hip (TL_HATTN=0: never): 1999 tokens, 32 heads of 64 over 8 kv heads or of 96 over their own, 110-140 us
-// against 571 in FP32; level with it from 16 tokens on
+// f16 products of tl_hattn.hip (TL_HATTN=0: never): 1999 tokens, 32 heads of 64 over 8 kv heads or of 96 over their own, 90 and
+// 110 us against 571 on average in FP32; at 16 tokens (Llama shapes) the two are level
 static bool swa_half(const SwaArgs& a, TlHattn* x) {
   const char* e = getenv("TL_HATTN");
   if (!a.half_ws || a.pos_dev || a.sigmoid || a.softcap > 0.0f || a.dist_r1 || a.keep_first || (e && atoi(e) == 0)) return false;
