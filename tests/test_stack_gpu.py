@@ -424,6 +424,26 @@ def test_half_attention_routes(pkg, monkeypatch, family):
     assert np.linalg.norm(got[1] - got[0]) <= 3e-5 * np.linalg.norm(got[0]), np.linalg.norm(got[1] - got[0]) / np.linalg.norm(got[0])
 
 
+@pytest.mark.parametrize("scale", [0.0, -0.125, 2.0 ** -140, 0.125])
+def test_attention_scale_of_any_sign_in_a_chunk(env, scale):
+    """A layer's factor on the scores is a plain number of its configuration: zero (every visible key alike), negative, or too small
+    for the powers of two of the two-part f16 kernel, which takes positive ones of ordinary size and leaves the rest to the FP32
+    kernel. Chunks of 16 tokens and more, whole and continued, against the oracle."""
+    L = env["synth"].stack_layer
+    cfg = env["synth"].stack_config(128, 90, [L(4, 2, 64, 64, 40, scale=scale), L(2, 1, 128, 128, None, scale=scale)])
+    m, _, oracle = make(env, cfg)
+    toks = np.random.default_rng(4).integers(0, 90, 150).astype(np.int32)
+    want = oracle.forward(toks)
+    for parts in ((150,), (70, 80)):
+        m.reset_kv()
+        at, got = 0, []
+        for n in parts:
+            got.append(m.prefill_rows(toks[at:at + n], at))
+            at += n
+        assert rel_rms(np.concatenate(got), want) < FP32_TOL, parts
+    m.free()
+
+
 @pytest.mark.parametrize("rows,cols,T,terms", [(64, 64, 64, 1), (65, 72, 63, 1), (130, 200, 65, 3), (33, 8, 16, 1), (70, 130, 40, 1),
                                                (70, 131, 40, 3), (256, 192, 130, 1), (4096, 96, 1024, 1), (4100, 40, 1030, 1)])
 def test_dense_gemm_steps(pkg, rows, cols, T, terms):

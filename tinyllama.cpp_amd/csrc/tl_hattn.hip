@@ -450,8 +450,11 @@ void launch(const HPlanesArgs& p, const HAttnArgs& a, hipStream_t s) {
 
 }  // namespace
 
-// head sizes that are whole matrix instructions, and rows and heads at 16 bytes: wide loads of queries and keys
+// head sizes that are whole matrix instructions, and rows and heads at 16 bytes: wide loads of queries and keys. The kernel takes
+// its maximum and its masks before the factor on the scores, so the factor has to be positive, and large enough to stay above
+// zero beside the powers of two of a query and a key tile of (almost) zeros, 2^-60 each; any other one is the FP32 kernels'
 bool tl_hattn_supported(const TlHattn& x) {
+  if (!(x.scale >= 0x1p-16f && x.scale <= 0x1p16f)) return false;
   const bool sizes = x.vdim == 64 ? x.dim == 64 || x.dim == 96 || x.dim == 128 : x.vdim == 128 && x.dim == 128;
   return sizes && x.kv_heads > 0 && x.kv_heads <= 65535 && x.heads > 0 && x.heads % x.kv_heads == 0 &&
          ((x.ldq | x.qhs | x.kld | x.khs) & 3) == 0 && (((size_t)x.q | (size_t)x.kc | (size_t)x.out) & 15) == 0;
