@@ -44,6 +44,12 @@ int tl_model_bench_kernel(tl_model* m, int kind, int iters, int warmup, float* a
  * in this process: lets a test prove which kernel formed a result. */
 int tl_debug_gemm_px_launches(long long* count_out);
 
+/* Test hook (no counterpart in the reference): tl_swa_attention's product through the two-part f16 kernels that prompt chunks
+ * take (tl_hattn.hip); head sizes 64, 96 or 128 over 64 and 128 over 128, a positive scale, 16-byte addresses. */
+int tl_debug_half_attention(const float* q_dev, const float* k_cache_dev, const float* v_cache_dev, float* out_dev,
+                            int num_tokens, int start_pos, int heads, int kv_heads, int dim, int vdim, int window, float scale,
+                            void* stream);
+
 /* Parity hook for layer-list models (no counterpart in the reference): cb(ctx, layer, x_dev, num_tokens, width) is called after
  * every layer of every forward pass, the stream synchronised, with the residual stream on the device. NULL switches it off.
  * With the hook set the decode step must run eagerly (TL_NO_GRAPH=1 at finalize): a captured step cannot call back. */

@@ -424,6 +424,42 @@ def test_half_attention_routes(pkg, monkeypatch, family):
     assert np.linalg.norm(got[1] - got[0]) <= 3e-5 * np.linalg.norm(got[0]), np.linalg.norm(got[1] - got[0]) / np.linalg.norm(got[0])
 
 
+@pytest.mark.parametrize("dim,vdim,spread", [(64, 64, "row"), (128, 128, "row"), (96, 64, "first row"), (128, 64, "tiles"),
+                                             (64, 64, "steps"), (128, 128, "steps"), (64, 64, "none")])
+def test_half_attention_value_range(env, dim, vdim, spread):
+    """The two-part f16 attention holds one power of two per tile of 32 value rows and one for its running sum. A row 2^18 times
+    the others' size, of negligible weight, must coarsen neither the tiles behind it nor those in front of it (its own tile's rows
+    are held to 2^-39 of it: 2^-21), nor may tiles of values 2^-60 .. 2^60 apart, at random or rising and falling. As many heads as
+    keep the keys of a row in one piece. Against float64, relative to the weights times the values' size: two parts hold 2^-23 of
+    each factor, and errors of many keys average out, so 2^-22 bounds the L2 distance (FP32 kernel: 7e-8, this one 5e-8 to 1.3e-7)."""
+    rng = np.random.default_rng(dim + vdim)
+    heads, n, T = 128, 600, 512
+    u = rng.standard_normal(dim)
+    u /= np.linalg.norm(u)
+    q = (rng.standard_normal((T, heads, dim)) + 8 * u).astype(np.float32)
+    k = rng.standard_normal((n, heads, dim)).astype(np.float32)
+    v = rng.standard_normal((n, heads, vdim)).astype(np.float32)
+    tiles = -(-n // 32)
+    if spread in ("row", "first row"):
+        at = 70 if spread == "row" else 0
+        k[at] = -5.0 * np.sqrt(dim) * u  # (a score of -40)
+        v[at] *= 2.0 ** 18
+    elif spread != "none":
+        e = rng.integers(-60, 61, tiles) if spread == "tiles" else np.abs(np.arange(tiles) * 13 - 120) - 60
+        v *= np.exp2(e).astype(np.float32).repeat(32)[:n, None, None]
+    scale = dim ** -0.5
+    f = lambda a: a.reshape(len(a), -1).astype(np.float64)
+    args = (heads, heads, dim, vdim, 0, scale, np.arange(n - T, n), np.arange(n))
+    want = env["oracle"].window_attention(f(q), f(k), f(v), *args)
+    size = env["oracle"].window_attention(f(q), f(k), np.abs(f(v)), *args)
+    qd, kd, vd, od = dev(env, q), dev(env, k), dev(env, v), env["engine"].DeviceBuffer(4 * T * heads * vdim)
+    capi = env["capi"]
+    capi.check(capi.lib().tl_debug_half_attention(qd.ptr, kd.ptr, vd.ptr, od.ptr, T, n - T, heads, heads, dim, vdim, 0, scale, None), "half attention")
+    capi.check(capi.lib().tl_device_sync(), "sync")
+    err = np.linalg.norm((od.to_numpy(np.float32, want.shape) - want) / size) / np.sqrt(want.size)
+    assert err <= 2.0 ** -22, err
+
+
 @pytest.mark.parametrize("scale", [0.0, -0.125, 2.0 ** -140, 0.125])
 def test_attention_scale_of_any_sign_in_a_chunk(env, scale):
     """A layer's factor on the scores is a plain number of its configuration: zero (every visible key alike), negative, or too small

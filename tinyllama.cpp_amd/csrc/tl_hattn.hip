@@ -9,7 +9,10 @@
 //   1. kv_planes_kernel cuts the cache rows of every kv head into 32-key tiles of two-part f16 in the order in which the
 //      lanes of a matrix instruction take them (K: eight columns of one key; V: eight keys of one column, the keys in the
 //      order in which the accumulator of K Q^T holds them, so that the probabilities never change lanes). One power of two
-//      per tile brings its largest finite value to 2^14: products of the tile's rows keep 22 bits over 2^18 of range.
+//      per tile brings its largest finite value to 2^14: a value is held to 2^-23 of itself and 2^-39 of its tile's largest.
+//      Against float64 the output's error is 5e-8 of its weights times its values' size, the FP32 kernel's 7e-8 (both sides
+//      lose what the order of the sums gives); a row of a tile that is 2^20 times the others' size brings it to 1e-7, 2^24 to
+//      1.3e-6.
 //   2. hattn_kernel: four waves, 128 rows (query, head of the kv head's group), tiles through a double-buffered LDS window
 //      that all four waves read: one wave's operands straight from memory would need 85 bytes a cycle and CU. Two workgroups
 //      a CU, so that one's softmax runs under the other's products. A row tile's keys are cut into up to 16 pieces.
@@ -28,6 +31,7 @@ namespace {
 constexpr int HA_ROWS = 128, HA_MAX_SPLIT = 16, HA_MAX_SLOTS = 2048;
 constexpr float LOG2E = 1.44269504088896340736f;
 constexpr float HA_P_BITS = 12.f;  // probabilities are held times 2^12: their second part stays normal down to 2^-15
+constexpr int HA_P_SPARE = 8;      // ... and to 2^-29 of a row's largest at worst: what they may give up for a tile of small values
 
 __device__ __forceinline__ int acc_row(int e, int h) { return (e & 3) + 8 * (e >> 2) + 4 * h; }
 
@@ -233,7 +237,10 @@ __global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs a) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) o[b][e] = 0.f;
   float mrun = -INFINITY, lrun = 0.f;
-  int krun = 60;  // smallest exponent of the V tiles so far: o is held times 2^krun
+  // o is held times 2^krun. A tile of larger values (a smaller exponent) has o follow at once, one of smaller values when its
+  // probabilities would lose more than HA_P_SPARE bits: a tile with one huge row does not coarsen the tiles behind it. low: the
+  // smallest exponent so far, o is below 2^(27 + krun - low) times the weights' sum, hence krun <= low + 60
+  int krun = 60, low = 60;
   store(0);
   int ek = __builtin_amdgcn_readfirstlane(stage_ex.x), ev = __builtin_amdgcn_readfirstlane(stage_ex.y);
   __syncthreads();
@@ -293,16 +300,20 @@ __global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs a) {
         psum += s[e];
       }
       lrun = lrun * corr + psum;
-      if (ev != krun) {  // (uniform) the smaller exponent rules: o takes the tile's unit, or the probabilities take o's
-        const int down = ev - krun;
-        if (down < 0) {
-          corr *= pow2i(down < -126 ? -126 : down);
-          krun = ev;
-        } else {
-          const float f = pow2i(-down < -126 ? -126 : -down);
+      if (ev != krun) {  // (uniform)
+        int over = ev - krun;
+        if (over < 0 || over > HA_P_SPARE) {  // o takes the tile's unit, as far as its size allows
+          const int to = ev < low + 60 ? ev : low + 60, by = to - krun, part = by < -126 ? -126 : by;
+          corr *= pow2i(part) * pow2i(by - part);
+          krun = to;
+          over = ev - to;
+        }
+        if (over > 0) {  // the probabilities take o's
+          const float f = pow2i(over < 126 ? -over : -126);
 #pragma unroll
           for (int e = 0; e < 16; ++e) s[e] *= f;
         }
+        low = ev < low ? ev : low;
       }
       if (__any(corr != 1.f)) {
 #pragma unroll
@@ -496,4 +507,32 @@ int tl_launch_hattn(const TlHattn& x, void* ws, size_t ws_bytes, hipStream_t s) 
   else launch<64, 64>(p, a, s);
   TL_HIP(hipGetLastError());
   return 0;
+}
+
+// Measurement and test hook: the kernels above as an operator (tlhip_debug.h)
+extern "C" int tl_debug_half_attention(const float* q_dev, const float* k_cache_dev, const float* v_cache_dev, float* out_dev, int num_tokens,
+                                       int start_pos, int heads, int kv_heads, int dim, int vdim, int window, float scale, void* stream) {
+  TL_REQUIRE(q_dev && k_cache_dev && v_cache_dev && out_dev && num_tokens > 0 && start_pos >= 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0,
+             "tl_debug_half_attention: bad argument");
+  TlHattn x = {};
+  x.q = q_dev;
+  x.kc = k_cache_dev;
+  x.vc = v_cache_dev;
+  x.out = out_dev;
+  x.ldq = heads * dim;
+  x.kld = kv_heads * dim;
+  x.vld = kv_heads * vdim;
+  x.qhs = x.khs = x.dim = dim;
+  x.vdim = vdim;
+  x.T = num_tokens;
+  x.start_pos = start_pos;
+  x.heads = heads;
+  x.kv_heads = kv_heads;
+  x.scale = scale;
+  x.window = window;
+  TL_REQUIRE(tl_hattn_supported(x), "tl_debug_half_attention: not shapes of the two-part f16 kernel");
+  const size_t bytes = tl_hattn_bytes(start_pos + num_tokens, kv_heads, dim, vdim);
+  void* ws = nullptr;
+  TL_TRY(tl_scratch(TL_SCRATCH_ATTN, bytes, &ws));
+  return tl_launch_hattn(x, ws, bytes, static_cast<hipStream_t>(stream));
 }
