@@ -349,6 +349,28 @@ def test_half_plane_gemm_edges(E, pkg, name, rows, cols, T):
     w.free()
 
 
+@pytest.mark.parametrize("name", ["q4_k", "q6_k", "q8_0", "q8_k"])
+@pytest.mark.parametrize("power", [125, 121, -112, -120])
+def test_half_plane_gemm_largest_and_smallest_activations(E, pkg, name, power):
+    """Activations at the ends of FP32's range (a row's largest just below 2^128, or far below 2^-100), another row at 1: the power
+    of two that brings a super-block into f16's range exists for all of them, and so do Q4_K's block sums. Finite products keep
+    their relative error (test_half_plane_gemm_edges' bound; below 2^-126 an output rounds to 2^-149)."""
+    t, S = TYPES[name], pkg.synth
+    rows, cols, T = 70, 512, 9
+    rng = np.random.default_rng(power + 200)
+    w = E.QWeight(t, S.random_blocks(t, rows * cols // S.BLOCK_ELEMS[t], rng, w_std=1.0 / np.sqrt(cols)), rows, cols)
+    x = rng.uniform(-4.0, 4.0, (T, cols)).astype(np.float32)
+    x[3:] = np.ldexp(x[3:], power)
+    W = w.dequantize().astype(np.float64)
+    want = x.astype(np.float64) @ W.T
+    scale = np.abs(x).astype(np.float64) @ (np.abs(W) + 4.0 * np.abs(W).max(axis=1, keepdims=True)).T
+    fits = np.abs(want) < 2.0 ** 127
+    assert fits.mean() > 0.5
+    y = _matmul(E, w, x)
+    assert (np.abs(y - want) <= (2.0 ** -22 + 50 * 2.0 ** -24) * scale + 2.0 ** -147)[fits].all()
+    w.free()
+
+
 @pytest.mark.parametrize("heads,kv,hd,start,T", [
     (4, 2, 64, 0, 8), (8, 1, 64, 33, 95), (16, 16, 64, 31, 33), (4, 1, 64, 900, 129), (6, 2, 128, 0, 129), (2, 2, 128, 63, 64),
     (6, 2, 128, 1000, 300), (8, 8, 128, 7, 150), (16, 2, 128, 2000, 9)])

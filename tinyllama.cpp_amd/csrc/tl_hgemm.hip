@@ -533,21 +533,23 @@ __device__ __forceinline__ void hsplit8(const float* v, _Float16* __restrict__ p
 #pragma unroll
   for (int o = 16; o >= 1; o >>= 1) top = fmaxf(top, __shfl_xor(top, o));
   if (i0 >= K) return;  // (whole quads of threads: K is a multiple of 32)
-  // top * 2^k in [512, 1024); zeros, and sub-normals or infinities, keep k in the normal range
+  // top * 2^k in [512, 1024); k of zeros and of sub-normals keeps 2^k and 2^-k normal
   int ex = (int)((__builtin_bit_cast(unsigned, top) >> 23) & 255u) - 127;
-  ex = top == 0.f ? 0 : ex < -110 ? -110 : ex > 120 ? 120 : ex;
+  ex = top == 0.f ? 0 : ex < -117 ? -117 : ex;
   const float scale = __builtin_bit_cast(float, (unsigned)(127 + 9 - ex) << 23);
   _Float16* bs = planes + 2 * ps;
   float* inv = reinterpret_cast<float*>(bs + ps / 16);
   const int sb = i0 >> 8;
   if ((i0 & 255) == 0) inv[(size_t)sb * tpad + t] = __builtin_bit_cast(float, (unsigned)(127 - 9 + ex) << 23);
-  float s = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+  float x[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = v[e] * scale;
+  float s = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));  // (scaled: below 2^15 whatever the row holds)
   s += __shfl_xor(s, 1);
   s += __shfl_xor(s, 2);
   if ((i0 & 31) == 0 && (K & 255) == 0) {  // sum of the 32-column block, at the place of its minimum in the operand
     const int j = (i0 >> 5) & 7, at = j < 4 ? 2 * j : 2 * (j - 4) + 1;
     _Float16* o = bs + ((size_t)sb * tpad + t) * 16 + at;
-    s *= scale;
     const _Float16 h = (_Float16)s;
     o[0] = h;
     o[8] = (_Float16)(s - (float)h);
@@ -556,9 +558,8 @@ __device__ __forceinline__ void hsplit8(const float* v, _Float16* __restrict__ p
   f16x8 hi, lo;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    const float xv = v[ORDER[e]] * scale;
-    hi[e] = (_Float16)xv;
-    lo[e] = (_Float16)(xv - (float)hi[e]);
+    hi[e] = (_Float16)x[ORDER[e]];
+    lo[e] = (_Float16)(x[ORDER[e]] - (float)hi[e]);
   }
   *reinterpret_cast<f16x8*>(planes + (size_t)t * K + i0) = hi;
   *reinterpret_cast<f16x8*>(planes + ps + (size_t)t * K + i0) = lo;
