@@ -231,6 +231,26 @@ def test_deferred_ksplit_reductions_are_bit_identical(pkg, monkeypatch):
                 assert a.shape == b.shape and np.array_equal(a, b), (shape, other, np.abs(a.astype(np.float64) - b).max())
 
 
+@pytest.mark.parametrize("mix,n", [("q4_k_m", 330), ("q6_k", 200), ("q8_0", 150)])
+def test_merged_and_separate_launches_round_alike(pkg, monkeypatch, mix, n):
+    """gate | up of 2 x 5632 rows and 330 tokens fill the chip in another workgroup shape than one of them does, and the shapes do
+    not round alike: launched one after another (TL_GEMM_MERGE=0) the matrices of a group keep the group's shape and slices, so
+    every logit is the same bit for bit."""
+    from tinyllama_cpp_amd import engine as E
+    E.init(0)
+    cfg, tensors = pkg.synth.build_model(dict(hidden=2048, inter=5632, n_heads=32, n_kv_heads=4, n_layers=1, vocab=64, max_pos=512, eps=1e-5,
+                                              rope_theta=10000.0), mix, seed=6)
+    m = E.Model(cfg).load(tensors)
+    toks = np.random.default_rng(6).integers(0, cfg["vocab"], n).astype(np.int32)
+    got = []
+    for merge in ("0", "1"):
+        monkeypatch.setenv("TL_GEMM_MERGE", merge)
+        m.reset_kv()
+        got.append(np.array(m.prefill(toks, 0, all_logits=True)[1]))
+    m.free()
+    assert np.array_equal(got[0], got[1]), np.abs(got[0].astype(np.float64) - got[1]).max()
+
+
 def test_packed_prompts_longer_than_a_sequence(pkg):
     """A packed batch of more tokens than a sequence has positions goes through as one chunk: every prompt's last logits are those
     of its own prefill, up to the order of 32-bit sums (2^-22 a layer and product)."""

@@ -1501,8 +1501,8 @@ int launch_gemm_qi(const QW& w, const __bf16* xp, size_t ps, float* y, const flo
 }
 
 // set by tl_launch_gemm_q_multi while it launches the matrices of a group one by one (no buffers for the partial tiles): the
-// slice count it chose for the group, so that the sums do not depend on the route
-static thread_local int t_group_slices = 0;
+// shape and slices it chose for the group, so that the sums do not depend on the route
+static thread_local HgemmPlan t_group_plan = {0, 0};
 // token counts up to which tl_matmul_q takes the f16 form (tl_hgemm.hip; TL_GEMM_DIRECT: 0 = never, at most 64; read at
 // every launch so that one process can compare the routes). Beyond, its integer-plane kernels (and tl_qweight_expand) hold
 static int gemm_direct_max() {
@@ -1671,15 +1671,20 @@ int tl_launch_split(int mode, const float* x, const float* aux, void* planes, si
 // describes them (the consumer adds `resid` itself); otherwise defer->got.S = 0 and y is complete as usual
 static int launch_gemm_dispatch(const QW& w, const __bf16* xp, size_t plane_stride, float* y, const float* resid, int T,
                                 int terms, hipStream_t s);
-// one matrix on the f16 form, K split as tl_hgemm_slices says (or as the group of tl_launch_gemm_q_multi does)
+// one matrix on the f16 form, as tl_hgemm_plan says for it (or for the group of tl_launch_gemm_q_multi)
+static HgemmPlan half_plan(const QW* w, int n, int T) {
+  HgemmPlan p = tl_hgemm_plan(w, n, T);
+  if (!ksplit_enabled()) p.S = 1;
+  return p;
+}
 static int launch_half(const QW& w, const void* planes, size_t plane_stride, float* y, const float* resid, int T, hipStream_t s) {
-  int S = t_group_slices > 0 ? t_group_slices : ksplit_enabled() ? tl_hgemm_slices(&w, 1, T) : 1;
+  HgemmPlan p = t_group_plan.S > 0 ? t_group_plan : half_plan(&w, 1, T);
   float* part = nullptr;
   bool deferred = false;
-  TL_TRY(ksplit_workspace(s, T, w.rows, &S, &part, &deferred));
-  float* out = S == 1 ? y : part;
-  TL_TRY(tl_launch_hgemm(&w, 1, planes, plane_stride, &out, S == 1 ? resid : nullptr, T, S, s));
-  if (S > 1) ksplit_finish(part, S, (size_t)T * w.rows, resid, y, deferred, s);
+  TL_TRY(ksplit_workspace(s, T, w.rows, &p.S, &part, &deferred));
+  float* out = p.S == 1 ? y : part;
+  TL_TRY(tl_launch_hgemm(&w, 1, planes, plane_stride, &out, p.S == 1 ? resid : nullptr, T, p, s));
+  if (p.S > 1) ksplit_finish(part, p.S, (size_t)T * w.rows, resid, y, deferred, s);
   TL_HIP(hipGetLastError());
   return 0;
 }
@@ -1716,10 +1721,11 @@ static int launch_gemm_dispatch(const QW& w, const __bf16* xp, size_t plane_stri
 }
 
 // Up to three matrices over the same activation planes (q | k | v, gate | up) in one launch of the f16 kernel or of the
-// integer-plane kernel. Taken only when that changes no bit: all matrices of one format and width, and for every matrix the
-// number of K slices its own launch would use (the f16 kernel: one for the group). Outputs: with one slice y[i] directly; with
-// more, the partial tiles go to defer[i] (required) for the consumer to sum. *merged = false: nothing was launched, the caller
-// runs the matrices one by one.
+// integer-plane kernel. All matrices of one format and width. The integer-plane kernel: taken only when that changes no bit, with
+// the number of K slices that each matrix's own launch would use. The f16 kernel: the shape and slices are the group's, also where
+// its matrices have to be launched one after another, so the sums do not depend on whether they could be merged. Outputs: with one
+// slice y[i] directly; with more, the partial tiles go to defer[i] (required) for the consumer to sum. *merged = false: nothing was
+// launched, the caller runs the matrices one by one.
 int tl_launch_gemm_q_multi(const QW* w, int n, const void* planes, size_t plane_stride, float* const* y, int T, int terms,
                            hipStream_t s, GemmDefer* const* defer, bool* merged) {
   *merged = false;
@@ -1736,8 +1742,10 @@ int tl_launch_gemm_q_multi(const QW* w, int n, const void* planes, size_t plane_
   const int BN = (T <= 64 || qi_narrow_always()) ? 64 : GB_N;
   const int ntiles = (T + BN - 1) / BN;
   int S[3] = {1, 1, 1};
-  if (half) {  // one slice count for the group, from the tiles of the whole launch
-    S[0] = S[1] = S[2] = ksplit_enabled() ? tl_hgemm_slices(w, n, T) : 1;
+  HgemmPlan plan = {0, 1};
+  if (half) {  // one shape and slice count for the group, from the tiles of the whole launch
+    plan = half_plan(w, n, T);
+    S[0] = S[1] = S[2] = plan.S;
   } else {     // K slices of every matrix as its own launch would choose them
     for (int i = 0; i < n; ++i) S[i] = qi_slices((w[i].rows + 127) / 128 * ntiles, w[i].cols / GB_K, T);
     if (px_own_slices() && px_ready(w, n))  // the expanded-plane kernel: one slice count from the launch's tiles
@@ -1757,11 +1765,11 @@ int tl_launch_gemm_q_multi(const QW* w, int n, const void* planes, size_t plane_
   }
   if (!can_merge) {
     if (!half) return 0;  // (integer-plane route: every matrix keeps its own slice count, the caller's launches are the same)
-    // the f16 form one matrix at a time, with the group's slice count: the same sums as the merged launch
+    // the f16 form one matrix at a time, with the group's shape and slices: the same sums as the merged launch
     for (int i = 0; i < n; ++i) {
-      t_group_slices = S[0];
+      t_group_plan = plan;
       const int rc1 = tl_launch_gemm_q(w[i], planes, plane_stride, y[i], nullptr, T, terms, s, defer ? defer[i] : nullptr);
-      t_group_slices = 0;
+      t_group_plan = {0, 0};
       if (rc1) return rc1;
     }
     *merged = true;
@@ -1770,7 +1778,7 @@ int tl_launch_gemm_q_multi(const QW* w, int n, const void* planes, size_t plane_
   const __bf16* xp = static_cast<const __bf16*>(planes);
   int rc = 0;
   if (half) {
-    TL_TRY(tl_launch_hgemm(w, n, planes, plane_stride, out, nullptr, T, S[0], s));
+    TL_TRY(tl_launch_hgemm(w, n, planes, plane_stride, out, nullptr, T, plan, s));
     for (int i = 0; i < n; ++i)
       if (defer && defer[i]) defer[i]->got = S[i] > 1 ? GemmParts{out[i], (size_t)T * w[i].rows, S[i]} : GemmParts{nullptr, 0, 0};
     *merged = true;

@@ -653,15 +653,12 @@ float hgemm_us(int type, int shape) {
   constexpr float US[] = {1.2f, 2.0f, 4.9f, 9.0f, 5.0f};
   return US[shape] * (type == TL_Q6_K ? 1.37f : 1.f);
 }
-struct HPlan {
-  int shape, bm, bn, S;
-};
 // The shape and the K slices with the least of: rounds over the chip x (a workgroup's super-blocks + its start and end) + the
 // partial sums written and read once at about 4 TB/s.
-HPlan hgemm_plan(const QW* w, int n, int T) {
+HgemmPlan hgemm_plan(const QW* w, int n, int T) {
   const int nsb = (w[0].cols + 255) / 256, type = w[0].type;
   const int lo = T <= 16 ? 0 : T <= 64 ? 1 : type == TL_Q8_0 ? 4 : 2, hi = T <= 64 ? lo : 4;
-  HPlan best = {lo, 0, 0, 1};
+  HgemmPlan best = {lo, 1};
   float least = -1.f;
   for (int v = lo; v <= hi; ++v) {
     if (v == 3 && type == TL_Q6_K) continue;  // (spills)
@@ -679,7 +676,7 @@ HPlan hgemm_plan(const QW* w, int n, int T) {
                          (S > 1 ? (float)S * (0.3f + (float)T * (float)rows * 2e-6f) : 0.f);
       if (least < 0.f || cost < least) {
         least = cost;
-        best = {v, bm, bn, S};
+        best = {v, S};
       }
     }
   }
@@ -700,14 +697,15 @@ int hgemm_go(const HSegs& g, int mt, const HAct& act, const float* resid, int T,
   return 0;
 }
 template <int TYPE>
-int hgemm_typed(const QW* w, int n, const HPlan& p, const HAct& act, float* const* out, const float* resid, int T, hipStream_t s) {
+int hgemm_typed(const QW* w, int n, const HgemmPlan& p, const HAct& act, float* const* out, const float* resid, int T, hipStream_t s) {
   HSegs g = {};
   int mt = 0;
+  const int bm = SHAPE[p.shape].tk * SHAPE[p.shape].mi * SHAPE[p.shape].nw;
   for (int i = 0; i < 3; ++i) {
     const int k = i < n ? i : n - 1;  // (unused slots repeat the last matrix; their tile range is empty)
     g.w[i] = w[k];
     g.y[i] = out[k];
-    if (i < n) mt += (w[i].rows + p.bm - 1) / p.bm;
+    if (i < n) mt += (w[i].rows + bm - 1) / bm;
     g.mt_end[i] = mt;
   }
   if (p.shape == 0) return hgemm_go<TYPE, 0>(g, mt, act, resid, T, p.S, s);
@@ -726,13 +724,16 @@ bool tl_hgemm_supported(const QW& w) {
   return (k256 || w.type == TL_Q8_0) && w.cols % (k256 ? 256 : 64) == 0 && w.cols <= HMAX_COLS && w.rows > 0 &&
          (size_t)w.rows * w.cols < ((size_t)1 << 32);  // (32-bit byte offsets)
 }
-int tl_hgemm_slices(const QW* w, int n, int T) { return hgemm_plan(w, n, T).S; }
-int tl_launch_hgemm(const QW* w, int n, const void* planes, size_t ps, float* const* out, const float* resid, int T, int S, hipStream_t s) {
+HgemmPlan tl_hgemm_plan(const QW* w, int n, int T) { return hgemm_plan(w, n, T); }
+int tl_launch_hgemm(const QW* w, int n, const void* planes, size_t ps, float* const* out, const float* resid, int T, const HgemmPlan& p,
+                    hipStream_t s) {
   for (int i = 0; i < n; ++i)
     TL_REQUIRE(tl_hgemm_supported(w[i]) && w[i].type == w[0].type && w[i].cols == w[0].cols, "half-plane GEMM: matrix %d does not fit", i);
-  TL_REQUIRE(n >= 1 && n <= 3 && T > 0 && S >= 1 && ps < ((size_t)1 << 31) && ps >= tl_gemm_padded_tokens(T) * (size_t)w[0].cols, "half-plane GEMM: bad argument");
-  HPlan p = hgemm_plan(w, n, T);
-  p.S = S;
+  const int nsb = (w[0].cols + 255) / 256;
+  TL_REQUIRE(p.S >= 1 && (p.S - 1) * ((nsb + p.S - 1) / p.S) < nsb && p.shape >= 0 && p.shape <= 4 && !(p.shape == 2 && w[0].type == TL_Q8_0) &&
+                 !(p.shape == 3 && w[0].type != TL_Q4_K && w[0].type != TL_Q8_K),
+             "half-plane GEMM: shape %d, %d K slices of %d super-blocks", p.shape, p.S, nsb);
+  TL_REQUIRE(n >= 1 && n <= 3 && T > 0 && ps < ((size_t)1 << 31) && ps >= tl_gemm_padded_tokens(T) * (size_t)w[0].cols, "half-plane GEMM: bad argument");
   const HAct act = hact(planes, ps, T);
   switch (w[0].type) {
     case TL_Q4_K: return hgemm_typed<TL_Q4_K>(w, n, p, act, out, resid, T, s);

@@ -273,9 +273,12 @@ int tl_launch_gemm_q_multi(const QW* w, int n, const void* planes, size_t plane_
 // TL_TERMS_HALF: activations as two f16 parts + a power of two per token, any supported format, 32-bit grade
 constexpr int TL_TERMS_HALF = 2;
 bool tl_hgemm_supported(const QW& w);
-int tl_hgemm_slices(const QW* w, int n, int T);
-int tl_launch_hgemm(const QW* w, int n, const void* planes, size_t plane_stride, float* const* out, const float* resid, int T, int S,
-                    hipStream_t s);
+struct HgemmPlan {
+  int shape, S;  // the workgroup's shape, the K slices
+};
+HgemmPlan tl_hgemm_plan(const QW* w, int n, int T);  // of one launch over w[0 .. n - 1]; fewer slices than its S only as S = 1
+int tl_launch_hgemm(const QW* w, int n, const void* planes, size_t plane_stride, float* const* out, const float* resid, int T,
+                    const HgemmPlan& plan, hipStream_t s);
 int tl_launch_hsplit(int mode, const float* x, const float* aux, void* planes, size_t plane_stride, int T, int K, float eps,
                      hipStream_t s, const GemmParts& a, const GemmParts& b, float* xout);
 // y = (resid ? resid : 0) + the pending sums (what the GEMM launch would have run itself)
