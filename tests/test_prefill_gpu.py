@@ -403,6 +403,34 @@ def test_half_attention_edges(E, pkg, monkeypatch, heads, kv, hd, start, T):
     assert np.linalg.norm(got[1] - got[0]) <= 1e-5 * np.linalg.norm(got[0]), np.linalg.norm(got[1] - got[0]) / np.linalg.norm(got[0])
 
 
+@pytest.mark.parametrize("mix", ["q4_k_m", "q6_k"])
+def test_split_products_of_long_chunks_stay_in_the_models_buffers(E, pkg, mix):
+    """ffn_down of 3072 x 8192 in Q6_K and 1400 tokens takes four K slices: 17.2 million partial sums. They have a place in the
+    model's own workspaces (summed by the next kernel), so once a first prompt has made those, prompts of other lengths allocate
+    nothing, in the model or process-wide (tl_shutdown drops what other tests left there)."""
+    import ctypes as C
+    from tinyllama_cpp_amd.capi import check, lib
+    hip = C.CDLL("libamdhip64.so")
+
+    def free_bytes():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    cfg = dict(hidden=3072, inter=8192, n_heads=24, n_kv_heads=8, n_layers=1, vocab=64, max_pos=2048, eps=1e-5, rope_theta=10000.0)
+    _, tensors = pkg.synth.build_model(cfg, mix, seed=1)
+    m = E.Model(cfg).load(tensors)
+    check(lib().tl_shutdown(), "tl_shutdown")
+    toks = np.random.default_rng(1).integers(0, cfg["vocab"], 2048).astype(np.int32)
+    m.prefill(toks, 0)
+    before = free_bytes()
+    for T in (1100, 1380, 1400, 1660, 600, 300, 100, 20):
+        m.reset_kv()
+        m.prefill(toks[:T], 0)
+        assert free_bytes() == before, T
+    m.free()
+
+
 @pytest.mark.parametrize("T", [2048, 2049, 2600])
 def test_prefill_chunks_of_2048(E, pkg, T):
     """Prompts around the largest chunk: the last logits of the whole prompt against the last row of an all-logits prefill, which

@@ -14,6 +14,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <vector>
 
 #include <rccl/rccl.h>
@@ -102,7 +103,7 @@ struct tl_model {
     // (folded into the next RMSNorm split, which writes the new residual stream to xb2; the two then swap)
     float* xb2 = nullptr;
     float* part[3] = {nullptr, nullptr, nullptr};
-    size_t part_cap = 0;
+    size_t part_cap[3] = {0, 0, 0};  // floats; 0 in all: no deferred sums
     GemmParts pend = {nullptr, 0, 0};
     GemmDefer dq = {}, dk = {}, dv = {};  // q / k / v of the layer in hand (qkv_deferred)
     void* planes = nullptr;    // bf16 [3][plane_stride]
@@ -1289,7 +1290,7 @@ extern "C" int tl_model_generate_sampled(tl_model* m, int first_token, int start
 // the matrix cores (tl_gemm.hip), batched RoPE + KV write, causal attention from the cache (tl_prefill.hip), O GEMM +
 // residual, RMSNorm -> planes, gate/up GEMMs, SwiGLU -> planes, down GEMM + residual. Longer prompts are walked chunk by
 // chunk over the growing cache. Short prompts (< prefill_min_batch) replay the decode graph token by token instead (same positions, KV contents and logits to ~1e-6).
-// Unsharded models whose products take the f16 form: 2048, where a projection has four times the tiles and no K slices, and the
+// Unsharded models whose products take the f16 form: 2048, where a projection has four times the tiles and fewer K slices, and the
 // attention converts the cache and sums its pieces a quarter as often (3B Q6_K, 3989 tokens: 98 ms in chunks of 512, 92 in these;
 // more would only grow the workspaces). The bf16 routes and tensor-parallel shards keep the 512 that they were tuned at, which
 // is also the most sequences of a step and the most logits rows of a chunk.
@@ -1308,6 +1309,53 @@ static int chunk_terms(const tl_model* m) {
 static int chunk_tokens(const tl_model* m) {
   return chunk_terms(m) == TL_TERMS_HALF ? m->pf.cap : m->pf.cap < kChunkRows ? m->pf.cap : kChunkRows;
 }
+// raises cap[0..2] to what the f16 form's K-split launches of chunks of up to `most` tokens leave in pf.part[0..2]
+static void half_part_floats(const tl_model* m, int most, size_t (&cap)[3]) {
+  struct Group {
+    QW w[3];
+    int n, at;  // matrices of one launch, the buffer of the first
+  };
+  std::vector<Group> groups;
+  auto add = [&](const LayerW& L, std::initializer_list<int> ts, int at) {
+    Group g = {{}, 0, at};
+    for (int t : ts) g.w[g.n++] = qw_view(L.q[t]);
+    for (const Group& o : groups) {  // (layers repeat)
+      bool same = o.n == g.n && o.at == g.at;
+      for (int i = 0; i < g.n && same; ++i) same = o.w[i].type == g.w[i].type && o.w[i].rows == g.w[i].rows && o.w[i].cols == g.w[i].cols;
+      if (same) return;
+    }
+    groups.push_back(g);
+  };
+  for (const LayerW& L : m->layers) {
+    // as qkv_deferred and prefill_mlp_half launch them: runs of equal formats together, the others alone
+    const int tq = L.q[TL_T_ATTN_Q]->type, tk = L.q[TL_T_ATTN_K]->type, tv = L.q[TL_T_ATTN_V]->type;
+    if (tq == tk && tq == tv) {
+      add(L, {TL_T_ATTN_Q, TL_T_ATTN_K, TL_T_ATTN_V}, 0);
+    } else {
+      if (tq == tk) {
+        add(L, {TL_T_ATTN_Q, TL_T_ATTN_K}, 0);
+      } else {
+        add(L, {TL_T_ATTN_Q}, 0);
+        add(L, {TL_T_ATTN_K}, 1);
+      }
+      add(L, {TL_T_ATTN_V}, 2);
+    }
+    add(L, {TL_T_ATTN_OUTPUT}, 0);
+    if (L.q[TL_T_FFN_GATE]->type == L.q[TL_T_FFN_UP]->type) {
+      add(L, {TL_T_FFN_GATE, TL_T_FFN_UP}, 0);
+    } else {
+      add(L, {TL_T_FFN_GATE}, 0);
+      add(L, {TL_T_FFN_UP}, 1);
+    }
+    add(L, {TL_T_FFN_DOWN}, 0);
+  }
+  // between multiples of 16 tokens a plan's tiles stay and only the price of its partial sums rises: S is largest at the first
+  for (const Group& g : groups)
+    for (int T = 1; T <= most; T += 16) {
+      const int S = tl_hgemm_plan(g.w, g.n, T).S;
+      for (int i = 0; i < g.n && S > 1; ++i) cap[g.at + i] = std::max(cap[g.at + i], (size_t)S * std::min(T + 15, most) * g.w[i].rows);
+    }
+}
 static int ensure_prefill_ws(tl_model* m, bool all_logits) {
   const tl_model_config& c = m->cfg;
   tl_model::Prefill& p = m->pf;
@@ -1322,13 +1370,15 @@ static int ensure_prefill_ws(tl_model* m, bool all_logits) {
     if (m->tp > 1) TL_HIP(hipMalloc(&p.xpart, sizeof(float) * cap * H));
     const char* dz = getenv("TL_GEMM_DEFER");  // 0: every K-split GEMM runs its own reduction launch (A/B runs)
     if (m->tp == 1 && !(dz && atoi(dz) == 0)) {
-      // a split launch has fewer than 4 * CUs (slice, tile) pairs of at most 128 x 128 outputs
+      // a split launch of the bf16 kernels has fewer than 4 * CUs (slice, tile) pairs of at most 128 x 128 outputs; the f16 form's
+      // plans are asked one by one (a product of 4096 x 14336 and 1537 tokens in Q6_K: 3 slices, 1.1 times that)
       const size_t rows_max = kmax > (size_t)c.vocab_size ? kmax : (size_t)c.vocab_size;
       size_t floats = (size_t)4 * tl_num_cus() * 128 * 128;
       if (floats > (size_t)8 * cap * rows_max) floats = (size_t)8 * cap * rows_max;
+      for (size_t& f : p.part_cap) f = floats;
+      if (m->half_planes) half_part_floats(m, cap, p.part_cap);
       TL_HIP(hipMalloc(&p.xb2, sizeof(float) * cap * H));
-      for (int i = 0; i < 3; ++i) TL_HIP(hipMalloc(&p.part[i], sizeof(float) * floats));
-      p.part_cap = floats;
+      for (int i = 0; i < 3; ++i) TL_HIP(hipMalloc(&p.part[i], sizeof(float) * p.part_cap[i]));
     }
     TL_HIP(hipMalloc(&p.qb, sizeof(float) * cap * (size_t)m->qd_l));
     TL_HIP(hipMalloc(&p.kb, sizeof(float) * cap * (size_t)m->kv_dim));
@@ -1381,10 +1431,10 @@ static int flush_residual(tl_model* m, hipStream_t s) {
 static int project_residual(tl_model* m, const tl_qweight* w, int T, hipStream_t s) {
   tl_model::Prefill& p = m->pf;
   const int terms = chunk_terms(m);
-  if (m->tp > 1 || !p.part_cap)
+  if (m->tp > 1 || !p.part_cap[0])
     return tl_launch_gemm_q(qw_view(w), p.planes, p.plane_stride, m->tp > 1 ? p.xpart : p.xb, m->rank == 0 ? p.xb : nullptr, T,
                             terms, s);
-  GemmDefer d = {p.part[0], p.part_cap, {nullptr, 0, 0}};
+  GemmDefer d = {p.part[0], p.part_cap[0], {nullptr, 0, 0}};
   TL_TRY(tl_launch_gemm_q(qw_view(w), p.planes, p.plane_stride, p.xb, p.xb, T, terms, s, &d));
   p.pend = d.got;
   return 0;
@@ -1395,10 +1445,10 @@ static int qkv_deferred(tl_model* m, LayerW& L, int T, hipStream_t s) {
   tl_model::Prefill& p = m->pf;
   const int terms = chunk_terms(m);
   const size_t ps = p.plane_stride;
-  p.dq = {p.part[0], p.part_cap, {nullptr, 0, 0}};
-  p.dk = {p.part[1], p.part_cap, {nullptr, 0, 0}};
-  p.dv = {p.part[2], p.part_cap, {nullptr, 0, 0}};
-  const bool defer = p.part_cap != 0;
+  p.dq = {p.part[0], p.part_cap[0], {nullptr, 0, 0}};
+  p.dk = {p.part[1], p.part_cap[1], {nullptr, 0, 0}};
+  p.dv = {p.part[2], p.part_cap[2], {nullptr, 0, 0}};
+  const bool defer = p.part_cap[0] != 0;
   // one launch where that changes no bit (runs of equal formats: Q4_K_M files hold v as Q6_K in some layers)
   bool merged = false;
   const QW w3[3] = {qw_view(L.q[TL_T_ATTN_Q]), qw_view(L.q[TL_T_ATTN_K]), qw_view(L.q[TL_T_ATTN_V])};
@@ -1430,7 +1480,7 @@ static int prefill_attn_half(tl_model* m, int l, int T, int start_pos, hipStream
   const float scale = 1.0f / sqrtf((float)hd);
   (void)H;
   TL_TRY(split_residual(m, L.attn_norm, T, s));
-  if (p.part_cap && m->tp == 1) {
+  if (p.part_cap[0] && m->tp == 1) {
     // q | k | v with their K-split sums left to ONE RoPE + cache-write kernel (instead of three reductions, the rotation
     // and two cache copies), merged into one launch where that changes no bit
     TL_TRY(qkv_deferred(m, L, T, s));
@@ -1492,8 +1542,8 @@ static int prefill_mlp_half(tl_model* m, int l, int T, hipStream_t s) {
   const size_t ps = p.plane_stride;
   (void)c;
   TL_TRY(split_residual(m, L.ffn_norm, T, s));
-  GemmDefer dg = {p.part[0], p.part_cap, {nullptr, 0, 0}}, du = {p.part[1], p.part_cap, {nullptr, 0, 0}};
-  const bool defer = p.part_cap != 0;
+  GemmDefer dg = {p.part[0], p.part_cap[0], {nullptr, 0, 0}}, du = {p.part[1], p.part_cap[1], {nullptr, 0, 0}};
+  const bool defer = p.part_cap[0] != 0;
   bool merged = false;  // gate | up in one launch where that changes no bit
   const QW w2[2] = {qw_view(L.q[TL_T_FFN_GATE]), qw_view(L.q[TL_T_FFN_UP])};
   float* const y2[2] = {p.gb, p.ub};
