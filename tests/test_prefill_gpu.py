@@ -349,6 +349,40 @@ def test_half_plane_gemm_edges(E, pkg, name, rows, cols, T):
     w.free()
 
 
+@pytest.mark.parametrize("shape", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("name,rows,cols,T,slices", [
+    ("q4_k", 1, 256, 65, 1), ("q4_k", 129, 768, 127, 2), ("q4_k", 257, 2304, 300, 5), ("q4_k", 300, 1280, 63, 5), ("q6_k", 1, 512, 129, 2),
+    ("q6_k", 257, 1792, 65, 4), ("q6_k", 129, 256, 300, 1), ("q8_0", 129, 64, 65, 1), ("q8_0", 257, 320, 127, 2), ("q8_0", 1, 1088, 300, 5),
+    ("q8_0", 255, 1984, 64, 3), ("q8_0", 70, 192, 129, 1), ("q8_k", 257, 1280, 127, 3), ("q8_k", 130, 256, 65, 1)])
+def test_half_plane_gemm_shapes(E, pkg, shape, name, rows, cols, T, slices):
+    """Every workgroup shape of tl_hgemm.hip by itself, those of long chunks (2, 3, 4: the ring of three 64-column steps, two row
+    tiles a wave, eight waves) at sizes off their tiles: one row, one more than a tile, tokens around 64 and 128, one super-block,
+    K slices with a short last one, Q8_0 rows that end inside a super-block. The bound of test_half_plane_gemm_edges."""
+    from tinyllama_cpp_amd.capi import check, lib
+    t, S = TYPES[name], pkg.synth
+    rng = np.random.default_rng(rows + 7 * cols + T)
+    w = E.QWeight(t, S.random_blocks(t, rows * cols // S.BLOCK_ELEMS[t], rng, w_std=1.0 / np.sqrt(cols)), rows, cols)
+    x = rng.standard_normal((T, cols)).astype(np.float32)
+    x *= np.exp2(rng.integers(-20, 21, (T, -(-cols // 256)))).astype(np.float32).repeat(256, axis=1)[:, :cols]
+    x[T // 2] = 0.0
+    xb, yb = E.DeviceBuffer.from_numpy(x), E.DeviceBuffer(4 * T * rows)
+    check(lib().tl_memset(yb.ptr, 0xff, yb.nbytes, None))
+    rc = lib().tl_debug_half_gemm(w.h, xb.ptr, yb.ptr, T, shape, slices, None)
+    if (shape == 2 and name == "q8_0") or (shape == 3 and name in ("q6_k", "q8_0")):
+        assert rc != 0  # (not instantiated)
+        w.free()
+        return
+    check(rc)
+    y = yb.to_numpy(np.float32, (T, rows))
+    W = w.dequantize().astype(np.float64)
+    want = x.astype(np.float64) @ W.T
+    scale = np.abs(x).astype(np.float64) @ (np.abs(W) + 4.0 * np.abs(W).max(axis=1, keepdims=True)).T
+    assert (np.abs(y - want) <= (2.0 ** -22 + 48 * 2.0 ** -24 + cols / 256 * 2.0 ** -24) * scale).all(), (np.abs(y - want) / np.maximum(scale, 1e-30)).max()
+    assert not y[T // 2].any()
+    assert lib().tl_debug_half_gemm(w.h, xb.ptr, yb.ptr, T, shape, 8 if cols <= 1792 else 7, None) != 0  # an empty slice: refused
+    w.free()
+
+
 @pytest.mark.parametrize("name", ["q4_k", "q6_k", "q8_0", "q8_k"])
 @pytest.mark.parametrize("power", [125, 121, -112, -120])
 def test_half_plane_gemm_largest_and_smallest_activations(E, pkg, name, power):

@@ -1866,3 +1866,17 @@ extern "C" int tl_matmul_q(const tl_qweight* w, const float* x_dev, float* y_dev
   TL_TRY(tl_launch_split(SPLIT_PLAIN, x_dev, nullptr, ws, ps, num_tokens, w->cols, terms, 0.f, s));
   return tl_launch_gemm_q(qw_view(w), ws, ps, y_dev, nullptr, num_tokens, terms, s);
 }
+
+// Measurement and test hook (include/tlhip_debug.h): the f16 form of one matrix in a workgroup shape and K slices of the caller's
+extern "C" int tl_debug_half_gemm(const tl_qweight* w, const float* x_dev, float* y_dev, int num_tokens, int shape, int slices, void* stream) {
+  TL_REQUIRE(w && x_dev && y_dev && num_tokens >= 1 && slices >= 1 && slices <= 8 && tl_hgemm_supported(qw_view(w)), "tl_debug_half_gemm: bad argument");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const size_t ps = tl_gemm_padded_tokens(num_tokens) * (size_t)w->cols;
+  void* ws = nullptr;
+  TL_TRY(tl_scratch(TL_SCRATCH_GEMM_PLANES, tl_gemm_planes_bytes(ps), &ws));
+  TL_TRY(tl_launch_split(SPLIT_PLAIN, x_dev, nullptr, ws, ps, num_tokens, w->cols, TL_TERMS_HALF, 0.f, s));
+  t_group_plan = {shape, slices};
+  const int rc = tl_launch_gemm_q(qw_view(w), ws, ps, y_dev, nullptr, num_tokens, TL_TERMS_HALF, s);
+  t_group_plan = {0, 0};
+  return rc;
+}
