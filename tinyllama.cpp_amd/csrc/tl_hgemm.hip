@@ -648,22 +648,40 @@ struct HShape {
   int tk, ni, mi, nw, wpe, percu;
 };
 constexpr HShape SHAPE[] = {{16, 1, 1, 4, 4, 4}, {32, 1, 1, 4, 2, 2}, {32, 2, 1, 8, 2, 1}, {32, 2, 2, 4, 2, 2}, {32, 2, 1, 4, 2, 2}};
-// us of a super-block of a workgroup on a full chip (measured; Q6_K's third product and longer unpacking)
-float hgemm_us(int type, int shape) {
-  constexpr float US[] = {1.2f, 2.0f, 4.9f, 9.0f, 5.0f};
-  return US[shape] * (type == TL_Q6_K ? 1.37f : 1.f);
+// us of a super-block of a workgroup on a full chip (measured)
+constexpr float HGEMM_US[] = {1.2f, 2.0f, 4.9f, 9.0f, 5.0f};
+// Price of a launch of n workgroups of `per` super-blocks, and of S slices' partial sums of `outputs` numbers.
+// Q4_K and Q8_K, and all formats up to 64 tokens: rounds over the chip x (super-blocks + start and end) + the partial sums written
+// and read once at about 4 TB/s. Q6_K (a third product, longer unpacking) and Q8_0 (16 additions and FMAs a block) beyond: the
+// time of the fullest CU, whose last workgroup takes 0.6 of a pair's time where two share it, and 0.16 of the way to what an even
+// share would take (clocks rise where CUs run dry). Over the projections of the 1B, 3B and 8B shapes and 100 to 2048 tokens that
+// picks within 0.5 % of the best shape and slices on average and 6 % at worst; rounds, which priced Q8_0 like Q4_K and left it one
+// shape, within 3 % and 20: 11264 x 2048 times 512 tokens in Q6_K 108 us, now 96; 3072 x 8192 in Q8_0 109, now 103. (For Q4_K it
+// would choose shape 3 more often, whose single chain of sums rounds more.)
+float hgemm_price(int type, int shape, long n, int per, int S, float outputs) {
+  const HShape& q = SHAPE[shape];
+  const float cus = (float)tl_num_cus();
+  if (shape >= 2 && (type == TL_Q6_K || type == TL_Q8_0)) {
+    const float us = type == TL_Q6_K ? (shape == 2 ? 6.4f : 6.85f) : (shape == 2 ? 5.6f : 6.0f), alone = q.percu == 2 ? 0.6f : 1.f;
+    const long most = (n + tl_num_cus() - 1) / tl_num_cus();
+    const float fullest = q.percu == 2 ? (float)(most / 2) + (most & 1 ? alone : 0.f) : (float)most;
+    const float even = (float)n / cus / (float)q.percu;
+    return (0.84f * fullest + 0.16f * (even > alone ? even : alone)) * ((float)per + 0.6f) * us + (S > 1 ? (float)S * (0.3f + outputs * 1.4e-6f) : 0.f);
+  }
+  const long slots = (long)tl_num_cus() * q.percu;
+  return (float)((n + slots - 1) / slots) * (float)(per + (shape < 2 ? 2 : 1)) * HGEMM_US[shape] * (type == TL_Q6_K ? 1.37f : 1.f) +
+         (S > 1 ? (float)S * (0.3f + outputs * 2e-6f) : 0.f);
 }
-// The shape and the K slices with the least of: rounds over the chip x (a workgroup's super-blocks + its start and end) + the
-// partial sums written and read once at about 4 TB/s.
+// the shape and the K slices of the least price
 HgemmPlan hgemm_plan(const QW* w, int n, int T) {
   const int nsb = (w[0].cols + 255) / 256, type = w[0].type;
-  const int lo = T <= 16 ? 0 : T <= 64 ? 1 : type == TL_Q8_0 ? 4 : 2, hi = T <= 64 ? lo : 4;
+  const int lo = T <= 16 ? 0 : T <= 64 ? 1 : 2, hi = T <= 64 ? lo : 4;
   HgemmPlan best = {lo, 1};
   float least = -1.f;
   for (int v = lo; v <= hi; ++v) {
-    if (v == 3 && type == TL_Q6_K) continue;  // (spills)
+    if (v == 3 && (type == TL_Q6_K || type == TL_Q8_0)) continue;  // (spills)
     const HShape& q = SHAPE[v];
-    const int bm = q.tk * q.mi * q.nw, bn = q.tk * q.ni, ntiles = (T + bn - 1) / bn, slots = tl_num_cus() * q.percu;
+    const int bm = q.tk * q.mi * q.nw, bn = q.tk * q.ni, ntiles = (T + bn - 1) / bn;
     long tiles = 0, rows = 0;
     for (int i = 0; i < n; ++i) {
       tiles += (long)((w[i].rows + bm - 1) / bm) * ntiles;
@@ -672,10 +690,9 @@ HgemmPlan hgemm_plan(const QW* w, int n, int T) {
     for (int S = 1; S <= 8 && S <= nsb; ++S) {
       const int per = (nsb + S - 1) / S;
       if ((nsb + per - 1) / per != S) continue;  // (no empty slice)
-      const float cost = (float)((tiles * S + slots - 1) / slots) * (float)(per + (v < 2 ? 2 : 1)) * hgemm_us(type, v) +
-                         (S > 1 ? (float)S * (0.3f + (float)T * (float)rows * 2e-6f) : 0.f);
-      if (least < 0.f || cost < least) {
-        least = cost;
+      const float price = hgemm_price(type, v, tiles * S, per, S, (float)T * (float)rows);
+      if (least < 0.f || price < least) {
+        least = price;
         best = {v, S};
       }
     }
@@ -710,8 +727,7 @@ int hgemm_typed(const QW* w, int n, const HgemmPlan& p, const HAct& act, float* 
   }
   if (p.shape == 0) return hgemm_go<TYPE, 0>(g, mt, act, resid, T, p.S, s);
   if (p.shape == 1) return hgemm_go<TYPE, 1>(g, mt, act, resid, T, p.S, s);
-  if constexpr (TYPE != TL_Q8_0)
-    if (p.shape == 2) return hgemm_go<TYPE, 2>(g, mt, act, resid, T, p.S, s);
+  if (p.shape == 2) return hgemm_go<TYPE, 2>(g, mt, act, resid, T, p.S, s);
   if constexpr (TYPE == TL_Q4_K || TYPE == TL_Q8_K)
     if (p.shape == 3) return hgemm_go<TYPE, 3>(g, mt, act, resid, T, p.S, s);
   return hgemm_go<TYPE, 4>(g, mt, act, resid, T, p.S, s);
@@ -730,7 +746,7 @@ int tl_launch_hgemm(const QW* w, int n, const void* planes, size_t ps, float* co
   for (int i = 0; i < n; ++i)
     TL_REQUIRE(tl_hgemm_supported(w[i]) && w[i].type == w[0].type && w[i].cols == w[0].cols, "half-plane GEMM: matrix %d does not fit", i);
   const int nsb = (w[0].cols + 255) / 256;
-  TL_REQUIRE(p.S >= 1 && (p.S - 1) * ((nsb + p.S - 1) / p.S) < nsb && p.shape >= 0 && p.shape <= 4 && !(p.shape == 2 && w[0].type == TL_Q8_0) &&
+  TL_REQUIRE(p.S >= 1 && (p.S - 1) * ((nsb + p.S - 1) / p.S) < nsb && p.shape >= 0 && p.shape <= 4 &&
                  !(p.shape == 3 && w[0].type != TL_Q4_K && w[0].type != TL_Q8_K),
              "half-plane GEMM: shape %d, %d K slices of %d super-blocks", p.shape, p.S, nsb);
   TL_REQUIRE(n >= 1 && n <= 3 && T > 0 && ps < ((size_t)1 << 31) && ps >= tl_gemm_padded_tokens(T) * (size_t)w[0].cols, "half-plane GEMM: bad argument");
