@@ -323,6 +323,45 @@ def test_prefill_attention_writes_the_gemm_planes_bit_identically(E, pkg, monkey
             assert a.shape == b.shape and np.array_equal(a, b), (shape, np.abs(a - b).max())
 
 
+# a model without the f16 form of the chunk products: Q8_0 rows (352 columns) that are not whole pairs of blocks
+ODD_Q8 = dict(hidden=256, inter=352, n_heads=4, n_kv_heads=2, n_layers=2, vocab=64, max_pos=160, eps=1e-5, rope_theta=10000.0)
+
+
+def _count(name):
+    import ctypes as C
+    from tinyllama_cpp_amd.capi import check, lib
+    n = C.c_longlong()
+    check(getattr(lib(), name)(C.byref(n)))
+    return n.value
+
+
+def test_expanded_planes_of_models(E, pkg, oracle, monkeypatch):
+    """A model whose matrices all have the f16 form keeps no expanded planes, whatever TL_PREFILL_PLANES says: no chunk of it reads
+    them. One with a matrix that has none does (unless 0), and its chunks go through them: the logits of the oracle, and bit for bit
+    those of the kernel that unpacks the quantized planes."""
+    cfg, tensors = pkg.synth.build_model("tiny-gqa", "q8_0", seed=4)
+    monkeypatch.setenv("TL_PREFILL_PLANES", "1")
+    m = E.Model(cfg).load(tensors)
+    assert m.prefill_planes_bytes() == 0
+    m.free()
+    cfg, tensors = pkg.synth.build_model(ODD_Q8, "q8_0", seed=4)
+    toks = np.random.default_rng(3).integers(0, cfg["vocab"], 100).astype(np.int32)
+    monkeypatch.setenv("TL_GEMM_PX_SLICES", "0")  # the unpacking kernel's K slices
+    got = []
+    for planes in ("1", "0"):
+        monkeypatch.setenv("TL_PREFILL_PLANES", planes)
+        m = E.Model(cfg).load(tensors)
+        assert (m.prefill_planes_bytes() > 0) == (planes == "1")
+        before = _count("tl_debug_gemm_px_launches")
+        got.append(np.array(m.prefill(toks, 0, all_logits=True)[1]))
+        assert (_count("tl_debug_gemm_px_launches") > before) == (planes == "1")
+        m.free()
+    assert np.array_equal(got[0], got[1])
+    om = OracleModel(oracle, cfg, tensors)
+    _, want = om.forward_batch(np.stack([om.lookup_embedding(t) for t in toks]), 0)
+    assert close(got[0], want, TOL[6]).all()
+
+
 @pytest.mark.parametrize("name,rows,cols,T", [
     ("q4_k", 1, 256, 8), ("q4_k", 65, 512, 16), ("q4_k", 129, 4096, 17), ("q4_k", 300, 14336, 32), ("q6_k", 63, 256, 9),
     ("q6_k", 130, 2304, 16), ("q6_k", 97, 768, 31), ("q8_0", 31, 64, 8), ("q8_0", 70, 320, 13), ("q8_0", 129, 448, 27),

@@ -752,12 +752,12 @@ static int plan_chain(tl_model* m) {
   return 0;
 }
 // Expanded prefill planes for every quantized matrix of a model whose chunks go through bf16 parts (tl_gemm.hip,
-// gemm_px_kernel), when they are affordable: at most a quarter of the device's memory and what is free now less 4 GiB
-// (TL_PREFILL_PLANES=0 / 1: never / always).
+// gemm_px_kernel: some matrix has no f16 form, as a Q8_0 one whose rows are not whole pairs of blocks), when they are affordable:
+// at most a quarter of the device's memory and what is free now less 4 GiB (TL_PREFILL_PLANES=0 / 1: never / whatever they cost).
 static int expand_prefill_planes(tl_model* m) {
   const char* e = getenv("TL_PREFILL_PLANES");
   const int mode = e ? (atoi(e) != 0 ? 1 : 0) : -1;
-  if (mode == 0 || (mode < 0 && m->half_planes)) return 0;  // (the f16 form reads the quantized planes themselves)
+  if (mode == 0 || m->half_planes) return 0;  // (the f16 form reads the quantized planes themselves, plain bf16 chunks do too)
   std::vector<const tl_qweight*> ws;
   for (auto& l : m->layers)
     for (auto* w : l.q)
