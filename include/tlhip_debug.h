@@ -43,6 +43,8 @@ int tl_model_bench_kernel(tl_model* m, int kind, int iters, int warmup, float* a
 /* Diagnostic hook (no counterpart in the reference): launches of the expanded-plane GEMM kernel (tl_qweight_expand) so far
  * in this process: lets a test prove which kernel formed a result. */
 int tl_debug_gemm_px_launches(long long* count_out);
+/* ... and launches that split activations into a chunk product's planes (those that attention writes itself are none) */
+int tl_debug_split_launches(long long* count_out);
 
 /* Test hook (no counterpart in the reference): tl_matmul_q through the f16 form that a model's chunks and multi-sequence steps
  * take (tl_hgemm.hip), any number of tokens, in a workgroup shape (0: 64 rows x 16 tokens, 1: 128 x 32, 2: 256 x 64, 3: 256 x 64 in
@@ -62,7 +64,7 @@ typedef void (*tl_layer_hook_fn)(void* ctx, int layer, const float* x_dev, int n
 int tl_model_debug_layer_hook(tl_model* m, tl_layer_hook_fn cb, void* ctx);
 
 /* ---- libtlhip_tools.so (csrc/tl_stream.hip; built beside libtlhip.so, not part of it): a measured negative result kept
- * for the record -- the persistent ring-loader engine of round 2. */
+ * for the record -- a persistent ring-loader engine. */
 /* Measurement / parity hook (no counterpart in the reference): y_i = W_i x through the ring-loader engine (tl_stream.hip),
  * the nw equally shaped matrices as nw phases of ONE persistent launch (ys_dev: [nw][rows]); avg_us_out (may be NULL) =
  * microseconds per matrix over `reps` launches. */

@@ -203,29 +203,38 @@ def test_deferred_ksplit_reductions_are_bit_identical(pkg, monkeypatch):
     """Skinny GEMMs split K; their partial tiles are summed by the NEXT kernel (RMSNorm split, SwiGLU split, RoPE + cache
     write) instead of a reduction launch of their own. Same sums in the same order: logits of a batched step, a packed
     prefill and an all-logits prefill are bit-for-bit those of TL_GEMM_DEFER=0 (one ksplit_reduce launch per GEMM), with
-    and without q | k | v and gate | up merged into one launch each."""
+    and without q | k | v and gate | up merged into one launch each. The last model's products are in bf16 parts (Q8_0 rows that
+    are not whole pairs of blocks): its batched attention writes the attn_output GEMM's planes itself (TL_ATTN_PLANES)."""
+    import ctypes as C
     from tinyllama_cpp_amd import engine as E
+    from tinyllama_cpp_amd.capi import lib
     monkeypatch.setenv("TL_BATCH_GEMV_MAX", "0")
     E.init(0)
     rng = np.random.default_rng(8)
-    for shape, mix in (("tiny-tp", "q4_k_m"), ("tiny-gqa", "q6_k")):
+    odd = dict(hidden=512, inter=1056, n_heads=8, n_kv_heads=2, n_layers=2, vocab=128, max_pos=128, eps=1e-5, rope_theta=10000.0)
+    for shape, mix in (("tiny-tp", "q4_k_m"), ("tiny-gqa", "q6_k"), (odd, "q8_0")):
         cfg, tensors = pkg.synth.build_model(shape, mix, seed=5)
         prompts = [rng.integers(0, cfg["vocab"], n).astype(np.int32) for n in [9, 3, 14, 6, 11, 2, 8, 5, 7, 10, 4, 12]]
         long_prompt = rng.integers(0, cfg["vocab"], 100).astype(np.int32)
-        got = {}
+        got, splits = {}, {}
         for defer, merge in (("0", "1"), ("1", "0"), ("1", "1")):
             monkeypatch.setenv("TL_GEMM_DEFER", defer)  # read when the model's prefill workspaces are made
             monkeypatch.setenv("TL_GEMM_MERGE", merge)  # q | k | v and gate | up in one launch each (needs DEFER)
-            monkeypatch.setenv("TL_ATTN_PLANES", defer)  # batched attention writes the attn_output GEMM's planes itself
+            monkeypatch.setenv("TL_ATTN_PLANES", defer)
             m = E.Model(cfg).load(tensors)
             m.batch_init(12)
+            n0, n1 = C.c_longlong(), C.c_longlong()
+            assert lib().tl_debug_split_launches(C.byref(n0)) == 0
             logits, ids = m.batch_prefill_packed(prompts)
+            assert lib().tl_debug_split_launches(C.byref(n1)) == 0
+            splits[defer] = n1.value - n0.value
             step, nxt = m.batch_decode(list(ids), [len(p) for p in prompts], list(range(12)))
             more = m.batch_generate_greedy(list(nxt), [len(p) + 1 for p in prompts], list(range(12)), 3)
-            _, all_logits = m.prefill(long_prompt, all_logits=True)       # 100 tokens: integer-plane kernel, 128-token tiles
-            _, all_logits40 = m.prefill(long_prompt[:40], all_logits=True)  # 40 tokens: its 64-token tiles
+            _, all_logits = m.prefill(long_prompt, all_logits=True)       # 64-token tiles of the f16 form, 128-token ones of the other
+            _, all_logits40 = m.prefill(long_prompt[:40], all_logits=True)  # 32- and 64-token tiles
             got[defer + merge] = [np.array(x) for x in (logits, ids, step, nxt, more, all_logits, all_logits40)]
             m.free()
+        assert splits["0"] - splits["1"] == (cfg["n_layers"] if mix == "q8_0" else 0), (shape, splits)
         for other in ("10", "11"):
             for a, b in zip(got["01"], got[other]):
                 assert a.shape == b.shape and np.array_equal(a, b), (shape, other, np.abs(a.astype(np.float64) - b).max())

@@ -72,10 +72,10 @@ def test_gemm_vs_oracle(E, pkg, oracle, name, rows, cols, T):
     ("q4_k", 333, 4096, 9), ("q4_k", 1024, 14336, 12), ("q6_k", 257, 1024, 32), ("q6_k", 4100, 4096, 40),
     ("q8_0", 100, 192, 17), ("q8_k", 130, 768, 20), ("q4_k", 96, 256, 64), ("q8_0", 2048, 2048, 50)])
 def test_direct_small_token_gemm(E, pkg, oracle, monkeypatch, name, rows, cols, T):
-    """gemm_qd_kernel (weights from global memory straight into the MFMA operand; launches of at most 32 tokens by
-    default, 64 with TL_GEMM_DIRECT=64): every format, row counts off the 32-row fragments, K splits with many and with
-    a single 64-column step, 32- and 64-token tiles -- against the oracle at the GEMM bars, and against the
-    integer-plane kernel it stands in for (TL_GEMM_DIRECT=0): same factorisation, so FP32 rounding apart."""
+    """The f16 form in tl_matmul_q (weights from global memory straight into the operands; launches of at most 32 tokens by
+    default, 64 with TL_GEMM_DIRECT=64): every format, row counts off the 64- and 128-row tiles, K splits and a single
+    super-block -- against the oracle at the GEMM bars, and against the integer-plane kernel it stands in for
+    (TL_GEMM_DIRECT=0): both of the 32-bit grade, so FP32 rounding apart."""
     from tinyllama_cpp_amd.capi import lib, check
     t, S = TYPES[name], pkg.synth
     rng = np.random.default_rng(7 * rows + cols + T)
@@ -298,31 +298,6 @@ def test_model_prefill_continues_cache_and_reduced_terms(E, pkg, oracle):
     om.close()
 
 
-def test_prefill_attention_writes_the_gemm_planes_bit_identically(E, pkg, monkeypatch):
-    """The prefill attention kernel writes the attn_output GEMM's activation planes itself (no split launch); every logit of
-    an all-logits prefill -- one call, and a second call appending to the cache, with 6 and 3 MFMA terms -- is bit for bit
-    what TL_ATTN_PLANES=0 (attention -> float rows -> split launch) gives."""
-    rng = np.random.default_rng(12)
-    for shape, mix, n in (("tiny-gqa", "q4_k_m", 150), ("tiny-tp", "q6_k", 77)):
-        cfg, tensors = pkg.synth.build_model(shape, mix, seed=4)
-        toks = rng.integers(0, cfg["vocab"], n).astype(np.int32)
-        got = {}
-        for ap in ("0", "1"):
-            monkeypatch.setenv("TL_ATTN_PLANES", ap)
-            m = E.Model(cfg).load(tensors)
-            out = []
-            for terms in (6, 3):
-                m.reset_kv()
-                m.set_prefill(terms=terms, min_batch=8)
-                _, a = m.prefill(toks[:n - 40], 0, all_logits=True)
-                _, b = m.prefill(toks[n - 40:], n - 40, all_logits=True)
-                out += [np.array(a), np.array(b)]
-            got[ap] = out
-            m.free()
-        for a, b in zip(got["0"], got["1"]):
-            assert a.shape == b.shape and np.array_equal(a, b), (shape, np.abs(a - b).max())
-
-
 # a model without the f16 form of the chunk products: Q8_0 rows (352 columns) that are not whole pairs of blocks
 ODD_Q8 = dict(hidden=256, inter=352, n_heads=4, n_kv_heads=2, n_layers=2, vocab=64, max_pos=160, eps=1e-5, rope_theta=10000.0)
 
@@ -333,6 +308,32 @@ def _count(name):
     n = C.c_longlong()
     check(getattr(lib(), name)(C.byref(n)))
     return n.value
+
+
+@pytest.mark.parametrize("shape,mix,n,every", [("tiny-gqa", "q4_k_m", 150, (1,)), ("tiny-tp", "q6_k", 77, (1,)), (ODD_Q8, "q8_0", 150, (6, 3, 1))])
+def test_prefill_attention_writes_the_gemm_planes_bit_identically(E, pkg, monkeypatch, shape, mix, n, every):
+    """The prefill attention kernel writes the bf16 planes of the attn_output GEMM itself (no split launch): every logit of an
+    all-logits prefill -- one call, and a second call appending to the cache -- is bit for bit what TL_ATTN_PLANES=0 (attention ->
+    float rows -> split launch) gives. With plain bf16 chunks, and, for a model whose matrices have no f16 form, with 6 and 3 MFMA
+    terms. The split launches are counted: a layer of a chunk has three, and one more with TL_ATTN_PLANES=0."""
+    rng = np.random.default_rng(12)
+    cfg, tensors = pkg.synth.build_model(shape, mix, seed=4)
+    toks = rng.integers(0, cfg["vocab"], n).astype(np.int32)
+    m = E.Model(cfg).load(tensors)
+    for terms in every:
+        m.set_prefill(terms=terms, min_batch=8)
+        got, splits = {}, {}
+        for ap in ("0", "1"):
+            monkeypatch.setenv("TL_ATTN_PLANES", ap)
+            m.reset_kv()
+            before = _count("tl_debug_split_launches")
+            _, a = m.prefill(toks[:n - 40], 0, all_logits=True)
+            _, b = m.prefill(toks[n - 40:], n - 40, all_logits=True)
+            got[ap], splits[ap] = [np.array(a), np.array(b)], _count("tl_debug_split_launches") - before
+        assert splits["0"] - splits["1"] == 2 * cfg["n_layers"], (terms, splits)
+        for a, b in zip(got["0"], got["1"]):
+            assert a.shape == b.shape and np.array_equal(a, b), (terms, np.abs(a - b).max())
+    m.free()
 
 
 def test_expanded_planes_of_models(E, pkg, oracle, monkeypatch):

@@ -194,6 +194,7 @@ DEBUG_SIGNATURES = {
     "tl_model_bench_kernel": [_vp, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_float), C.POINTER(C.c_double)],
     "tl_chain_set_stamps": [_vp, _sz],
     "tl_debug_gemm_px_launches": [C.POINTER(C.c_longlong)],
+    "tl_debug_split_launches": [C.POINTER(C.c_longlong)],
     "tl_debug_half_gemm": [_vp, _fp, _fp, C.c_int, C.c_int, C.c_int, _vp],
     "tl_debug_half_attention": [_fp, _fp, _fp, _fp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_float, _vp],
     "tl_model_debug_layer_hook": [_vp, LAYER_HOOK, _vp],

@@ -1624,9 +1624,11 @@ size_t tl_gemm_padded_tokens(int T) { return (size_t)((T + GB_N - 1) / GB_N) * G
 // every 32-column block
 size_t tl_gemm_planes_bytes(size_t plane_stride) { return 3 * plane_stride * sizeof(__bf16) + plane_stride / 32 * sizeof(float); }
 
+static std::atomic<long long> g_splits{0};
 int tl_launch_split(int mode, const float* x, const float* aux, void* planes, size_t plane_stride, int T, int K,
                     int terms, float eps, hipStream_t s, const GemmParts* pa, const GemmParts* pb, float* xout) {
   if (T == 0) return 0;
+  g_splits.fetch_add(1, std::memory_order_relaxed);
   if (terms == TL_TERMS_HALF) {
     const GemmParts none = {nullptr, 0, 0}, a = pa ? *pa : none, b = pb ? *pb : none;
     const size_t n = (size_t)T * K;
@@ -1827,6 +1829,12 @@ extern "C" int tl_debug_px_stamps(unsigned long long* host_out, int clear) {
 extern "C" int tl_debug_gemm_px_launches(long long* count_out) {
   TL_REQUIRE(count_out, "tl_debug_gemm_px_launches: null argument");
   *count_out = g_px_launches.load();
+  return 0;
+}
+
+extern "C" int tl_debug_split_launches(long long* count_out) {
+  TL_REQUIRE(count_out, "tl_debug_split_launches: null argument");
+  *count_out = g_splits.load();
   return 0;
 }
 
