@@ -501,6 +501,29 @@ def test_dense_gemm_steps(pkg, rows, cols, T, terms):
     assert (np.abs(yd.to_numpy(np.float32, (T, rows)) - X @ W.T) <= bound).all()
 
 
+@pytest.mark.parametrize("rows,cols,T", [(257, 96, 129), (4096, 96, 1024), (4100, 40, 1030), (260, 130, 70)])
+@pytest.mark.parametrize("terms", [1, 3])
+def test_dense_gemm_tiles_give_the_same_bits(pkg, monkeypatch, rows, cols, T, terms):
+    """The rule between small and large tiles looks at their number and at the columns only: each output is the same sum in the same
+    order in either, with one row and one token beyond a tile too, so the choice changes no bit. Bound as above."""
+    from tinyllama_cpp_amd import capi, engine, synth
+    engine.init(0)
+    rng = np.random.default_rng(rows + cols + T)
+    w = synth.to_bf16(rng.standard_normal((rows, cols)).astype(np.float32))
+    x = rng.standard_normal((T, cols)).astype(np.float32)
+    dev, got = engine.DeviceBuffer.from_numpy, []
+    wd, xd, yd = dev(w), dev(x), engine.DeviceBuffer(4 * T * rows)
+    for tile in ("64", "128", None):
+        monkeypatch.setenv("TL_DENSE_TILE", tile) if tile else monkeypatch.delenv("TL_DENSE_TILE")
+        capi.check(capi.lib().tl_dense_matmul(wd.ptr, rows, cols, xd.ptr, yd.ptr, T, terms, None), "tl_dense_matmul")
+        capi.check(capi.lib().tl_device_sync(), "sync")
+        got.append(yd.to_numpy(np.float32, (T, rows)))
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    W = synth.from_bf16(w).astype(np.float64)
+    X = (synth.from_bf16(synth.to_bf16(x)) if terms == 1 else x).astype(np.float64)
+    assert (np.abs(got[0] - X @ W.T) <= (cols + 4) * 2.0 ** -24 * (np.abs(X) @ np.abs(W).T)).all()
+
+
 def test_causal_conv_output_behind_the_last_row(pkg):
     """Channels at the end of wider rows, the output right behind the last row's: no overlap, whatever the row stride adds up to
     (buffers that the allocator places back to back); one float earlier it is one, and refused."""

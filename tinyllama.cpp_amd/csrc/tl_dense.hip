@@ -13,7 +13,7 @@
 //   for the 64 bytes a cycle that a CU's cache hands out (the activations are FP32 and every tile reads them). So two steps are
 //   in flight while a third is multiplied out of LDS, which needs loads without a branch around them: one kernel for wide
 //   loads, one for odd shapes. One step in flight behind a branch, products of eight columns: 2048 x 2048 times 64 / 512 / 1999
-//   tokens 30 / 39 / 63 us, now 17 / 19 / 47; 8192 x 2048 times 1999 182 -> 136 (495 TFLOP/s). Items may be gathered (x_rows), scattered (y_rows) and
+//   tokens 30 / 39 / 63 us, now 17 / 19 / 47; 8192 x 2048 times 1999 148 -> 113 (594 TFLOP/s; among a prompt's other launches 182 -> 140). Items may be gathered (x_rows), scattered (y_rows) and
 //   grouped (group_off: blockIdx.z = matrix of the group; tiles beyond a group's items leave at once), which is what the
 //   experts of a mixture need: the plan lives on the device, the grid is sized for the worst case.
 #include <math.h>
@@ -91,7 +91,7 @@ __global__ __launch_bounds__(256) void dense_gemm_kernel(const DenseArgs a) {
     u32x4 w[PW];
     f32x4 x[PX][2];
   };
-  // a step's pieces; columns beyond K as zeros (a step beyond the last reads the last column's pieces again)
+  // a step's pieces; columns beyond K as zeros (a step beyond the last reads the first column's pieces)
   auto fetch = [&](Step& r, int k0) __attribute__((always_inline)) {
     const int k = k0 + lk;
     if (VEC) {
@@ -289,13 +289,20 @@ int tl_launch_dense_gemm(const DenseArgs& a, hipStream_t s) {
   TL_REQUIRE(!a.bias || (!a.glu && groups == 1), "dense gemm: a bias with a gated unit or several matrices");
   // 128 x 128 tiles when there is enough of both sides to fill them (grouped launches: tokens per group on average)
   const long long per_group = a.group_off ? (long long)a.T / groups : a.T;
-  // Measured: a dense launch needs a 128 x 128 tile a CU (192 tiles, 6144 rows, 4096 columns, 512 tokens: 80 us against 65 in
-  // small ones; 256 tiles, 4096 rows, 2048 columns, 1000 tokens: level; 256 tiles over 14336 columns: 265 against 333); the experts' grouped launches, whose small tiles are mostly
-  // half-empty, gain from them with one term (221 -> 193 us) and lose with three (356 -> 413 us).
+  // Measured: a dense launch needs a 128 x 128 tile a CU (192 tiles, 6144 rows, 4096 columns, 512 tokens: 78 us against 75 in
+  // small ones with one term, 153 against 126 with three). Where its small tiles are four a CU, one round, large ones need long
+  // rows too, so that a tile's way in and out is short beside its products: 256 tiles, large / small, 512 columns 22.1 / 16.4 us
+  // with one term and 32.2 / 23.7 with three, 1024 29.3 / 25.9 and 48.4 / 41.7, 2048 43.7 / 42.1 and 82.9 / 77.5, 4096 74 / 78 and
+  // 148 / 149, 14336 224 / 345 and 483 / 511. Beyond, small tiles start a second round: 264 tiles of 2048 columns 56 / 63 and
+  // 87 / 91, 384 of 1024 32 / 36 and 53 / 59, 448 of 4096 107 / 154 and 200 / 265. Either tile gives the same bits. The experts'
+  // grouped launches, whose small tiles are mostly half-empty, gain from large ones with one term (221 -> 193 us) and lose with
+  // three (356 -> 413 us).
+  const long long small_tiles = ((a.rows + 63) / 64) * ((per_group + 63) / 64) * groups;
   const long long big_tiles = ((a.rows + 127) / 128) * ((per_group + 127) / 128) * groups;
   const char* force = getenv("TL_DENSE_TILE");  // 64 / 128: tests and A/B runs pick the tile themselves
   const bool big = force ? atoi(force) == 128
-                         : a.rows >= 256 && (a.group_off ? a.terms == 1 && per_group >= 96 : big_tiles >= tl_num_cus());
+                         : a.rows >= 256 && (a.group_off ? a.terms == 1 && per_group >= 96
+                                                         : big_tiles >= tl_num_cus() && (small_tiles > 4 * tl_num_cus() || a.cols >= 4096));
   const int BM = big ? 128 : 64, BN = big ? 128 : 64;
   dim3 grid((a.rows + BM - 1) / BM, (a.T + BN - 1) / BN, groups);
   TL_REQUIRE(grid.y <= 65535 && grid.z <= 65535, "dense gemm: launch too large");
