@@ -658,23 +658,22 @@ constexpr float HGEMM_US[] = {1.2f, 2.0f, 4.9f, 9.0f, 5.0f};
 // picks within 0.5 % of the best shape and slices on average and 6 % at worst; rounds, which priced Q8_0 like Q4_K and left it one
 // shape, within 3 % and 20: 11264 x 2048 times 512 tokens in Q6_K 108 us, now 96; 3072 x 8192 in Q8_0 109, now 103. (For Q4_K it
 // would choose shape 3 more often, whose single chain of sums rounds more.)
-float hgemm_price(int type, int shape, long n, int per, int S, float outputs) {
+float hgemm_price(int cus, int type, int shape, long n, int per, int S, float outputs) {
   const HShape& q = SHAPE[shape];
-  const float cus = (float)tl_num_cus();
   if (shape >= 2 && (type == TL_Q6_K || type == TL_Q8_0)) {
     const float us = type == TL_Q6_K ? (shape == 2 ? 6.4f : 6.85f) : (shape == 2 ? 5.6f : 6.0f), alone = q.percu == 2 ? 0.6f : 1.f;
-    const long most = (n + tl_num_cus() - 1) / tl_num_cus();
+    const long most = (n + cus - 1) / cus;
     const float fullest = q.percu == 2 ? (float)(most / 2) + (most & 1 ? alone : 0.f) : (float)most;
-    const float even = (float)n / cus / (float)q.percu;
+    const float even = (float)n / (float)cus / (float)q.percu;
     return (0.84f * fullest + 0.16f * (even > alone ? even : alone)) * ((float)per + 0.6f) * us + (S > 1 ? (float)S * (0.3f + outputs * 1.4e-6f) : 0.f);
   }
-  const long slots = (long)tl_num_cus() * q.percu;
+  const long slots = (long)cus * q.percu;
   return (float)((n + slots - 1) / slots) * (float)(per + (shape < 2 ? 2 : 1)) * HGEMM_US[shape] * (type == TL_Q6_K ? 1.37f : 1.f) +
          (S > 1 ? (float)S * (0.3f + outputs * 2e-6f) : 0.f);
 }
 // the shape and the K slices of the least price
 HgemmPlan hgemm_plan(const QW* w, int n, int T) {
-  const int nsb = (w[0].cols + 255) / 256, type = w[0].type;
+  const int nsb = (w[0].cols + 255) / 256, type = w[0].type, cus = tl_num_cus();  // (the call asks the runtime: once a plan)
   const int lo = T <= 16 ? 0 : T <= 64 ? 1 : 2, hi = T <= 64 ? lo : 4;
   HgemmPlan best = {lo, 1};
   float least = -1.f;
@@ -690,7 +689,7 @@ HgemmPlan hgemm_plan(const QW* w, int n, int T) {
     for (int S = 1; S <= 8 && S <= nsb; ++S) {
       const int per = (nsb + S - 1) / S;
       if ((nsb + per - 1) / per != S) continue;  // (no empty slice)
-      const float price = hgemm_price(type, v, tiles * S, per, S, (float)T * (float)rows);
+      const float price = hgemm_price(cus, type, v, tiles * S, per, S, (float)T * (float)rows);
       if (least < 0.f || price < least) {
         least = price;
         best = {v, S};
