@@ -925,8 +925,10 @@ def prefill_leg(model, S, cfg, mix, T, terms=6, reps=3, world=1):
     elems = sum(r * c for n, t, r, c in S.tensor_plan(cfg, mix) if n.startswith("blk.") and t != S.F32)
     flops = 2.0 * T * elems / world  # per GPU
     # matrix instructions per product: the f16 form multiplies exact weight operands with the activation's two f16 parts
-    # (32-bit grade, for 6 and 3 alike); 1: plain bf16
-    per_product = {6: 2, 3: 2, 1: 1}[terms]
+    # (32-bit grade, for 6 and 3 alike; three for Q6_K, whose operands are a rounded product and its remainder: the mean
+    # over the matrices' elements); 1: plain bf16
+    per_product = 1 if terms == 1 else round(sum(r * c * (3 if t == S.Q6_K else 2) for n, t, r, c in S.tensor_plan(cfg, mix)
+                                                 if n.startswith("blk.") and t != S.F32) / elems, 3)
     return {"prompt_tokens": T, "mfma_terms": terms, "mfma_per_product": per_product,
             "precision": {6: "fp32-grade", 3: "fp32-grade", 1: "bf16 activations"}[terms],
             "ms": round(best * 1e3, 2), "tokens_per_s": round(T / best, 1),

@@ -65,13 +65,15 @@ int tl_device_sync(void);
 int tl_qweight_upload(int type, const void* host_blocks, int rows, int cols, tl_qweight** out, void* stream);
 int tl_qweight_free(tl_qweight* w);
 int tl_qweight_info(const tl_qweight* w, int* type, int* rows, int* cols, size_t* device_bytes);
-/* Optional: keeps an expanded copy of the matrix for the batched products in bf16 parts (tl_matmul_q with more than 64
- * tokens, chunks of a model with tl_model_set_prefill(1)): the integers as one bf16 plane + FP32 scale words, 2.375 bytes per weight, from which the
- * matrix cores are fed by LDS-DMA instead of unpacking the quantized planes in every workgroup. Results do not change by
- * a bit. The counterpart of the reference's FP32 expansion, ensure_f32_concatenated_weights_loaded
- * (weight_management.cpp:199-435; 4 bytes per weight there). A model whose matrices all have the f16 form (Q4_K, Q6_K, Q8_0) needs
- * none; for the others tl_model_finalize does this when the copy is at most a quarter of the device's memory
- * (TL_PREFILL_PLANES=0 / 1: never / always, for every model). tl_qweight_free drops it.
+/* Optional: keeps an expanded copy of the matrix for the batched products in bf16 parts at 3 or 6 terms (tl_matmul_q with more than
+ * 64 tokens; chunks of a model that has some matrix without the f16 form): the integers as one bf16 plane + FP32 scale words,
+ * 2.375 bytes per weight, from which the matrix cores are fed by LDS-DMA instead of unpacking the quantized planes in every
+ * workgroup. Plain bf16 products (1 term) never read it. The sums are the unpacking kernel's, FP32 rounding apart (bit for bit with
+ * TL_GEMM_PX_SLICES=0). The counterpart of the reference's FP32 expansion, ensure_f32_concatenated_weights_loaded
+ * (weight_management.cpp:199-435; 4 bytes per weight there). A model whose matrices all have the f16 form (Q4_K, Q6_K and Q8_K; Q8_0
+ * whose rows are whole pairs of 32-column blocks; rows of up to 32768 columns) needs none; for the others tl_model_finalize does
+ * this when the copy is at most a quarter of the device's memory (TL_PREFILL_PLANES=0 / 1: never / whatever it costs).
+ * tl_qweight_free drops it.
  * *expanded_bytes (may be NULL): device bytes of the copy (0: this format has none -- F32 / BF16 matrices). */
 int tl_qweight_expand(tl_qweight* w, size_t* expanded_bytes, void* stream);
 
@@ -91,7 +93,8 @@ int tl_matvec_q(const tl_qweight* w, const float* x_dev, float* y_dev, void* str
  * smart_gemm_batch_cuda (model.cpp:2141-2249) for batched prefill. */
 int tl_matmul_q(const tl_qweight* w, const float* x_dev, float* y_dev, int num_tokens, void* stream);
 /* bf16 MFMAs per FP32 product in tl_matmul_q (num_tokens >= 8) and, by default, in tl_model_prefill: both operands
- * are split into bf16 planes and a product is assembled from 1 (plain bf16), 3 or 6 (default; FP32-grade) MFMAs. */
+ * are split into bf16 planes and a product is assembled from 1 (plain bf16), 3 or 6 (default; FP32-grade) MFMAs. For 3 and 6
+ * launches of up to 32 tokens, and the chunks of models whose matrices all have it, take the f16 form at the grade of 6. */
 int tl_gemm_set_terms(int terms);
 
 /* ---- glue operators (same argument meaning as the cuda_kernels.h wrappers they replace) ------- */
@@ -201,7 +204,8 @@ int tl_model_prefill(tl_model* m, const int* tokens_host, int num_tokens, int st
 /* Batched-prefill numerics / routing of this model (no counterpart in the reference, whose GPU prefill is FP32
  * cublasSgemm or BF16 cublasGemmEx by a T >= 4 rule, model.cpp:2152-2153): terms = grade of a product in the prefill
  * GEMMs: 6 (default, FP32-grade, logits within the decode tolerance), 3 (~2^-17 per product), 1 (plain bf16); a model
- * whose matrices all have the f16 form takes it, at the grade of 6, for 3 as well (two MFMAs a product). 0 = the process-wide value of tl_gemm_set_terms; prompts shorter than min_batch (default 8) and tensor-parallel
+ * whose matrices all have the f16 form takes it, at the grade of 6, for 3 as well (two MFMAs a product, Q6_K three).
+ * 0 = the process-wide value of tl_gemm_set_terms; prompts shorter than min_batch (default 8) and tensor-parallel
  * shards replay the decode graph token by token. */
 int tl_model_set_prefill(tl_model* m, int terms, int min_batch);
 /* device pointers into the model's state, for parity tests and for hosts that keep using the operator-level
@@ -210,8 +214,8 @@ int tl_model_device_ptr(tl_model* m, int which, int layer, void** dev_out);
 /* algorithmic bytes one decode step at position pos must move on this rank (SURVEY §8d B_tok) */
 int tl_model_bytes_per_token(const tl_model* m, int pos, double* weight_bytes, double* kv_bytes);
 /* device bytes of the expanded prefill planes that tl_model_finalize keeps for this model's matrices (tl_qweight_expand;
- * 0: none -- not needed by the f16 form, switched off, or not affordable on this device). They serve the batched paths only: a decode step never
- * reads them. */
+ * 0: none -- not needed by the f16 form, switched off, or not affordable on this device). They serve the batched paths only: a
+ * decode step never reads them. */
 int tl_model_prefill_planes_bytes(const tl_model* m, size_t* bytes_out);
 /* Multi-sequence decode (generate_batch api.cpp:836-1142; batch_prefill_parallel :1144, batch_generation_parallel :1423;
  * forward_cpu_batch_generation model.cpp:1158-1523 / forward_device_batch_generation :1863-2114): up to max_batch

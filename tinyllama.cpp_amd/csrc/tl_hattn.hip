@@ -4,8 +4,8 @@
 // The FP32 matrix instructions do 64 multiply-adds a cycle and SIMD, the f16 ones 512: a product of two-part numbers
 // (x 2^k = hi + lo, 22 bits, lo lo left out) costs three of the latter and still leaves a factor of five. The FP32 kernel
 // (tl_prefill.hip) was bound by its matrix cores: 3989 tokens of 24 heads of 128 in chunks of 512, 28 layers, took it 44 ms;
-// the three kernels here take 16 ms (of which the conversion 2.2, the sums 1.9), and the whole prompt 136 -> 105 ms. Now the
-// matrix cores are half busy (a 32 x 32 tile pair of 2 us holds 1.5 us of products at the clock they leave).
+// the three kernels here take 16 ms of such chunks (of which the conversion 2.2, the sums 1.9; the whole prompt 136 -> 105 ms)
+// and 12 of chunks of 2048 (0.7 and 1.0).
 //   1. kv_planes_kernel cuts the cache rows of every kv head into 32-key tiles of two-part f16 in the order in which the
 //      lanes of a matrix instruction take them (K: eight columns of one key; V: eight keys of one column, the keys in the
 //      order in which the accumulator of K Q^T holds them, so that the probabilities never change lanes). One power of two

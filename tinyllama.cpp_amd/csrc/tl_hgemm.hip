@@ -639,9 +639,11 @@ __global__ __launch_bounds__(256) void hsplit_kernel(const float* __restrict__ x
 // The shapes of a workgroup. Up to 16 tokens: 64 rows, four workgroups (sixteen waves) on a CU, which keeps the most weight
 // bytes in flight: a step of 16 sequences of the 8B shape (8 layers) 0.96 ms against 0.98 with the 32-token shape (Q8_0 of
 // 1.1B 0.58 against 0.63). Up to 64: 128 rows x 32 tokens, two on a CU (32 sequences 1.04 ms; 64: 1.46 against 1.49 with
-// 64-token tiles). More: 64-token tiles, each operand unpacked once for two token fragments. There the matrix cores set the
-// pace: without unpacking, fragment reads and scale FMAs a 512-token chunk is 20 % shorter, no more, and the clock falls to
-// 1.9 GHz under them; which of the three shapes is taken is a matter of filling the chip, so the plan below weighs them.
+// 64-token tiles). More: 64-token tiles, each operand unpacked once for two token fragments. No one unit is full there: in shape 2
+// the matrix cores are busy in 36 % (28672 x 4096 in Q4_K, 128 tokens, 224 workgroups on 256 CUs), 42 % (512 tokens) and 50 %
+// (16384 x 3072 in Q6_K, 2048 tokens) of the cycles, at 2.1, 1.9 and 1.8 GHz, the two waves of a SIMD wait in 29 % of theirs for
+// data and barriers and in 37 % for their turn to issue. Without unpacking, fragment reads and scale FMAs a 512-token chunk is 20 %
+// shorter. Which of the three shapes is taken is a matter of filling the chip, so the plan below weighs them.
 // (8 layers of the 8B shape in ms, this kernel / the bf16 kernels it replaced: 8 sequences 0.86 / 1.56, 32: 1.05 / 1.62,
 // 64: 1.52 / 2.03, 128: 2.2 / 2.7; a prompt of 512: 5.3 / 7.0.)
 struct HShape {

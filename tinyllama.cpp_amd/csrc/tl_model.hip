@@ -1299,7 +1299,7 @@ constexpr int kPrefillChunk = 2048, kChunkRows = 512;
 __global__ void set_token_kernel(int* state, const int* tokens, int i) { state[0] = tokens[i]; }
 
 // how a chunk's products are formed: 1 = plain bf16; 3 and 6 both as the f16 form of the 32-bit grade where every matrix has
-// it (tl_hgemm.hip: two matrix instructions a product, what 3 terms of bf16 parts cost, at the grade of 6), else bf16 parts
+// it (tl_hgemm.hip: two matrix instructions a product, three for Q6_K, at the grade of 6), else bf16 parts
 static int chunk_terms(const tl_model* m) {
   const int terms = m->prefill_terms ? m->prefill_terms : tl_gemm_default_terms();
   return terms != 1 && m->half_planes ? TL_TERMS_HALF : terms;
@@ -1450,7 +1450,7 @@ static int qkv_deferred(tl_model* m, LayerW& L, int T, hipStream_t s) {
   p.dk = {p.part[1], p.part_cap[1], {nullptr, 0, 0}};
   p.dv = {p.part[2], p.part_cap[2], {nullptr, 0, 0}};
   const bool defer = p.part_cap[0] != 0;
-  // one launch where that changes no bit (runs of equal formats: Q4_K_M files hold v as Q6_K in some layers)
+  // one launch where the formats are equal (Q4_K_M files hold v as Q6_K in some layers)
   bool merged = false;
   const QW w3[3] = {qw_view(L.q[TL_T_ATTN_Q]), qw_view(L.q[TL_T_ATTN_K]), qw_view(L.q[TL_T_ATTN_V])};
   float* const y3[3] = {p.qb, p.kb, p.vb};
@@ -1483,7 +1483,7 @@ static int prefill_attn_half(tl_model* m, int l, int T, int start_pos, hipStream
   TL_TRY(split_residual(m, L.attn_norm, T, s));
   if (p.part_cap[0] && m->tp == 1) {
     // q | k | v with their K-split sums left to ONE RoPE + cache-write kernel (instead of three reductions, the rotation
-    // and two cache copies), merged into one launch where that changes no bit
+    // and two cache copies), merged into one launch where formats allow
     TL_TRY(qkv_deferred(m, L, T, s));
     TL_TRY(tl_launch_batch_rope_kv(p.qb, p.kb, p.vb, m->kc(l), m->vc(l), 0, m->rope, nullptr, nullptr, T, m->nh_l, m->nkv_l, hd,
                                    c.max_position_embeddings, 1, s, &p.dq.got, &p.dk.got, &p.dv.got, start_pos));
@@ -1545,7 +1545,7 @@ static int prefill_mlp_half(tl_model* m, int l, int T, hipStream_t s) {
   TL_TRY(split_residual(m, L.ffn_norm, T, s));
   GemmDefer dg = {p.part[0], p.part_cap[0], {nullptr, 0, 0}}, du = {p.part[1], p.part_cap[1], {nullptr, 0, 0}};
   const bool defer = p.part_cap[0] != 0;
-  bool merged = false;  // gate | up in one launch where that changes no bit
+  bool merged = false;  // gate | up in one launch where their formats are equal
   const QW w2[2] = {qw_view(L.q[TL_T_FFN_GATE]), qw_view(L.q[TL_T_FFN_UP])};
   float* const y2[2] = {p.gb, p.ub};
   GemmDefer* const d2[2] = {&dg, &du};

@@ -1,5 +1,5 @@
 #!/bin/bash
-# SQ stall breakdown of the direct small-token GEMM (gemm_qd_kernel) of the 32-sequence decode step.
+# SQ stall breakdown of the f16 GEMM (hgemm_kernel) of the 32-sequence decode step.
 # Round 1 ran the whole batch bench under ONE --pmc pass of 8 SQ counters and rocprofv3 died with SIGSEGV. Round 2 found
 # the same fault with FOUR counters: it is raised inside a kernel launch of the eager decode step (stack: memmove under
 # the profiler's dispatch callback under gemv_launch_pair, profiles/r02_f_pmc_qd_abort.txt), so it is not the counter
@@ -18,8 +18,8 @@ if not fs:
 agg = {}
 for r in csv.DictReader(open(fs[0])):
     k = r["Kernel_Name"]
-    if "gemm_qd_kernel" not in k: continue
-    key = k[k.index("gemm_qd"):][:32] + " grid=" + r.get("Grid_Size", "?")
+    if "hgemm_kernel" not in k: continue
+    key = k[k.index("hgemm_kernel"):][:36] + " grid=" + r.get("Grid_Size", "?")
     c = agg.setdefault(key, {}).setdefault(r["Counter_Name"], [0, 0.0]); c[0] += 1; c[1] += float(r["Counter_Value"])
 for k, a in sorted(agg.items()):
     row = {n: round(v / c) for n, (c, v) in a.items()}

@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""The smallest program that launches the direct small-token GEMM (gemm_qd_kernel) of the 32-sequence decode step:
+"""The smallest program that launches the f16 GEMM (hgemm_kernel) of the 32-sequence decode step:
 tl_matmul_q with 32 tokens on the two Llama-3-8B FFN shapes, three launches each and nothing else (no model, no decode
 step). For rocprofv3 --pmc passes: with a whole model in the process the profiler's counter collection faulted inside a
 launch of the eager decode step (profiles/r02_f_pmc_qd_abort.txt), whatever the counter set."""
