@@ -423,6 +423,29 @@ def test_half_plane_gemm_shapes(E, pkg, shape, name, rows, cols, T, slices):
     w.free()
 
 
+@pytest.mark.parametrize("shape", [2, 3, 4])
+@pytest.mark.parametrize("T", [512, 513, 1050])
+def test_half_plane_gemm_panels_of_token_tiles(E, pkg, shape, T):
+    """Workgroups walk panels of eight 64-token tiles: whole panels, a last panel of one tile, several row tiles and K slices. Every
+    token's row equals, to the bit, that of a launch of 64 tokens."""
+    from tinyllama_cpp_amd.capi import check, lib
+    S, rows, cols = pkg.synth, 520, 512
+    rng = np.random.default_rng(T)
+    w = E.QWeight(Q4_K, S.random_blocks(Q4_K, rows * cols // 256, rng, w_std=1.0 / np.sqrt(cols)), rows, cols)
+    x = rng.standard_normal((T, cols)).astype(np.float32)
+
+    def run(a, slices):
+        xb, yb = E.DeviceBuffer.from_numpy(np.ascontiguousarray(a)), E.DeviceBuffer(4 * a.shape[0] * rows)
+        check(lib().tl_memset(yb.ptr, 0xff, yb.nbytes, None))
+        check(lib().tl_debug_half_gemm(w.h, xb.ptr, yb.ptr, a.shape[0], shape, slices, None))
+        return yb.to_numpy(np.float32, (a.shape[0], rows))
+
+    for slices in (1, 2):
+        want = np.concatenate([run(x[i:i + 64], slices) for i in range(0, T, 64)])
+        assert np.array_equal(run(x, slices).view(np.uint32), want.view(np.uint32))
+    w.free()
+
+
 @pytest.mark.parametrize("name", ["q4_k", "q6_k", "q8_0", "q8_k"])
 @pytest.mark.parametrize("power", [125, 121, -112, -120])
 def test_half_plane_gemm_largest_and_smallest_activations(E, pkg, name, power):
