@@ -51,6 +51,12 @@ int tl_debug_split_launches(long long* count_out);
  * waves of 64 rows, Q4_K and Q8_K, 4: 128 x 64) and a number of K slices, none of them empty. */
 int tl_debug_half_gemm(const tl_qweight* w, const float* x_dev, float* y_dev, int num_tokens, int shape, int slices, void* stream);
 
+/* Test hook (no counterpart in the reference): tl_dense_matmul's product with one term through the kernel that takes the items from a
+ * bf16 plane (tl_dense.hip): rows ldx floats apart, whole steps of 64 columns, the first `exact_items` (at most 32) items with two
+ * terms, `waves` 4 (two workgroups a CU) or 8 (one), plane_dev room for [num_tokens + 32][cols] bf16. */
+int tl_debug_dense_plane(const void* w_bf16_dev, int rows, int cols, const float* x_dev, int ldx, float* y_dev, int num_tokens,
+                         int exact_items, int waves, void* plane_dev, void* stream);
+
 /* Test hook (no counterpart in the reference): tl_swa_attention's product through the two-part f16 kernels that prompt chunks
  * take (tl_hattn.hip); head sizes 64, 96 or 128 over 64 and 128 over 128, a positive scale, 16-byte addresses. */
 int tl_debug_half_attention(const float* q_dev, const float* k_cache_dev, const float* v_cache_dev, float* out_dev,

@@ -13,7 +13,11 @@
 //   for the 64 bytes a cycle that a CU's cache hands out (the activations are FP32 and every tile reads them). So two steps are
 //   in flight while a third is multiplied out of LDS, which needs loads without a branch around them: one kernel for wide
 //   loads, one for odd shapes. One step in flight behind a branch, products of eight columns: 2048 x 2048 times 64 / 512 / 1999
-//   tokens 30 / 39 / 63 us, now 17 / 19 / 47; 8192 x 2048 times 1999 148 -> 113 (594 TFLOP/s; among a prompt's other launches 182 -> 140). Items may be gathered (x_rows), scattered (y_rows) and
+//   tokens 30 / 39 / 63 us, now 17 / 19 / 47; 8192 x 2048 times 1999 148 -> 113 (594 TFLOP/s; among a prompt's other launches 182 -> 140).
+//   Large products of one term do without the conversion in every tile: the items are rounded to a bf16 plane once, and both sides go
+//   from memory to LDS without registers in between (dense_plane_kernel: 10304 x 2048 times 1999 tokens 174 -> 114 us with the
+//   conversion of 8, that is 740 and 800 TFLOP/s; staged through registers from the same plane 133). What bounds it now: barriers
+//   and fragment reads between the products of a step, and at these sizes the last of 2.5 rounds of tiles. Items may be gathered (x_rows), scattered (y_rows) and
 //   grouped (group_off: blockIdx.z = matrix of the group; tiles beyond a group's items leave at once), which is what the
 //   experts of a mixture need: the plan lives on the device, the grid is sized for the worst case.
 #include <math.h>
@@ -34,6 +38,57 @@ __device__ __forceinline__ float dense_glu(float g, float u, float limit, float 
   g = fminf(g, limit);
   u = fminf(fmaxf(u, -limit), limit);
   return g / (1.0f + expf(-alpha * g)) * (u + up_add);
+}
+
+// The epilogue of a wave: WM x WN products of 32 x 32, features from f0 on, items from i0 on (items below hi are stored).
+template <int WM, int WN>
+__device__ __forceinline__ void dense_store(const DenseArgs& a, f32x16 (&acc)[WM][WN], float* Y, int f0, int i0, int hi, int lane) {
+  // C layout: lane holds token (lane & 31) of a 32 x 32 product, features (e / 4) * 8 + (lane >> 5) * 4 + (e & 3)
+  const bool v4 = (a.ldy & 3) == 0 && ((size_t)Y & 15) == 0;
+  const int act_to = a.act_to > 0 ? a.act_to : a.rows;
+#pragma unroll
+  for (int j = 0; j < WN; ++j) {
+    const int it = i0 + j * 32 + (lane & 31);
+    if (it >= hi) continue;
+    const int orow = a.y_rows ? a.y_rows[it] : it;
+    float* yr = Y + (size_t)orow * a.ldy;
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+#pragma unroll
+      for (int gq = 0; gq < 4; ++gq) {
+        const int f = f0 + i * 32 + gq * 8 + (lane >> 5) * 4;
+        if (a.glu) {  // (gate, up) pairs: features f, f + 1 -> unit f / 2; f + 2, f + 3 -> the next one
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+            if (f + 2 * e + 1 < a.rows)
+              yr[(f >> 1) + e] = tl_glu_apply(a.glu_kind, acc[i][j][gq * 4 + 2 * e], acc[i][j][gq * 4 + 2 * e + 1], a.glu_limit, a.glu_alpha, a.glu_up_add);
+          continue;
+        }
+        if (a.bias) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (f + e < a.rows) acc[i][j][gq * 4 + e] += a.bias[f + e];
+        }
+        if (a.softcap > 0.0f) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][j][gq * 4 + e] = a.softcap * tanhf(acc[i][j][gq * 4 + e] / a.softcap);
+        }
+        if (a.act) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (f + e >= a.act_from && f + e < act_to) acc[i][j][gq * 4 + e] = tl_act_apply(a.act, acc[i][j][gq * 4 + e], a.act_p, a.act_q);
+        }
+        if (v4 && f + 4 <= a.rows) {
+          *reinterpret_cast<float4*>(yr + f) =
+              make_float4(acc[i][j][gq * 4], acc[i][j][gq * 4 + 1], acc[i][j][gq * 4 + 2], acc[i][j][gq * 4 + 3]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (f + e < a.rows) yr[f + e] = acc[i][j][gq * 4 + e];
+        }
+      }
+    }
+  }
 }
 
 // A workgroup of 4 waves (2 x 2) owns a (64 WM)-feature x (64 WN)-token tile; a wave WM x WN products of 32 x 32.
@@ -199,52 +254,127 @@ __global__ __launch_bounds__(256) void dense_gemm_kernel(const DenseArgs a) {
       __syncthreads();
     }
   }
-  // C layout: lane holds token (lane & 31) of a 32 x 32 product, features (e / 4) * 8 + (lane >> 5) * 4 + (e & 3)
-  const bool v4 = (a.ldy & 3) == 0 && ((size_t)Y & 15) == 0;
-  const int act_to = a.act_to > 0 ? a.act_to : a.rows;
+  dense_store<WM, WN>(a, acc, Y, f0 + wm * WM * 32, t0 + wn * WN * 32, hi, lane);
+}
+
+// 16 bytes a lane from base + off to LDS bytes at .. at + 1023, no registers in between (at, base: the same in all lanes). M0 holds the
+// LDS address and belongs to the compiler: saved and restored in the same statement
+__device__ __forceinline__ void dma16(unsigned at, unsigned off, const void* base) {
+  unsigned keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep) : "s"(at), "v"(off), "s"(base) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void dma_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// One matrix, one term, items whose bf16 values lie in a plane [items][cols] already (dense_rows_kernel), whole steps of 64 columns.
+// NWM x NWN waves, 32 WM features x 32 WN items each. Workgroups walk panels of eight item tiles, a contiguous range of tiles per XCD
+// (as in the f16 GEMM of quantized matrices). Both sides go from memory to LDS directly, NS - 1 steps ahead;
+// the loop has no other loads, so that waiting for all but the last NS - 2 steps' pieces is waiting for the step in hand.
+template <int NWM, int NWN, int WM, int WN, int NS, bool FIRST>
+__global__ __launch_bounds__(64 * NWM * NWN, 2) void dense_plane_kernel(const DenseArgs a, int mtiles, int ntiles) {
+  constexpr int NW = NWM * NWN, BM = 32 * WM * NWM, BN = 32 * WN * NWN, ROWS = BM + BN + (FIRST ? 32 : 0), STAGE = ROWS * 128;
+  constexpr int IW = BM / 8 / NW, IX = BN / 8 / NW;  // pieces of 8 rows x 64 columns that a wave fetches
+  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "");
+  extern __shared__ __attribute__((aligned(16))) unsigned char dlds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave % NWM, wn = wave / NWM;
+  constexpr int PANEL = 8;
+  const int total = mtiles * ntiles, per8 = total >> 3, rem8 = total & 7, xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+  const int v = xcd * per8 + (xcd < rem8 ? xcd : rem8) + at;
+  const int panel = v / (PANEL * mtiles), in_panel = v - panel * PANEL * mtiles;
+  const int width = ntiles - PANEL * panel < PANEL ? ntiles - PANEL * panel : PANEL;
+  const int t0 = (PANEL * panel + in_panel % width) * BN, f0 = in_panel / width * BM;
+  const int K = a.cols, hi = a.T;
+  const bool lead = FIRST && t0 == 0;
+  // row r of a stage lies at 128 r, its 16-byte piece q at q ^ (r / 2 & 7): the 16 rows of a fragment read cover the 64 banks once
+  const int lr = lane >> 3;
+  unsigned wo[IW], xo[IX], eo = 0;
 #pragma unroll
-  for (int j = 0; j < WN; ++j) {
-    const int it = t0 + (wn * WN + j) * 32 + (lane & 31);
-    if (it >= hi) continue;
-    const int orow = a.y_rows ? a.y_rows[it] : it;
-    float* yr = Y + (size_t)orow * a.ldy;
+  for (int i = 0; i < IW; ++i) {  // (rows and items beyond the last: the first one's values, never stored)
+    const int row = (wave * IW + i) * 8 + lr, r = f0 + row;
+    wo[i] = ((unsigned)(r < a.rows ? r : 0) * (unsigned)K + (((lane & 7) ^ ((row >> 1) & 7)) << 3)) * 2u;
+  }
 #pragma unroll
-    for (int i = 0; i < WM; ++i) {
+  for (int j = 0; j < IX; ++j) {
+    const int row = (wave * IX + j) * 8 + lr, r = t0 + row;
+    xo[j] = ((unsigned)(r < hi ? r : 0) * (unsigned)K + (((lane & 7) ^ ((row >> 1) & 7)) << 3)) * 2u;
+  }
+  if (FIRST) {
+    const int row = (wave & 3) * 8 + lr;
+    eo = ((unsigned)(row < a.T ? row : 0) * (unsigned)K + (((lane & 7) ^ ((row >> 1) & 7)) << 3)) * 2u;
+  }
+  const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)dlds;
+  const int steps = K / 64;
+  auto fetch = [&](int st, int slot) __attribute__((always_inline)) {  // (a step beyond the last: the last one again, never read)
+    const size_t k = (size_t)(st < steps ? st : steps - 1) * 128;
+    const unsigned b = lds0 + slot * STAGE;
+    const char* wb = reinterpret_cast<const char*>(a.w) + k;
+    const char* xb = reinterpret_cast<const char*>(a.plane) + k;
 #pragma unroll
-      for (int gq = 0; gq < 4; ++gq) {
-        const int f = f0 + (wm * WM + i) * 32 + gq * 8 + (lane >> 5) * 4;
-        if (a.glu) {  // (gate, up) pairs: features f, f + 1 -> unit f / 2; f + 2, f + 3 -> the next one
+    for (int i = 0; i < IW; ++i) dma16(b + (wave * IW + i) * 1024, wo[i], wb);
 #pragma unroll
-          for (int e = 0; e < 2; ++e)
-            if (f + 2 * e + 1 < a.rows)
-              yr[(f >> 1) + e] = tl_glu_apply(a.glu_kind, acc[i][j][gq * 4 + 2 * e], acc[i][j][gq * 4 + 2 * e + 1], a.glu_limit, a.glu_alpha, a.glu_up_add);
-          continue;
-        }
-        if (a.bias) {
+    for (int j = 0; j < IX; ++j) dma16(b + BM * 128 + (wave * IX + j) * 1024, xo[j], xb);
+    if (FIRST && lead) dma16(b + (BM + BN) * 128 + (wave & 3) * 1024, eo, xb + (size_t)a.T * K * 2);
+  };
+  f32x16 acc[WM][WN];
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (f + e < a.rows) acc[i][j][gq * 4 + e] += a.bias[f + e];
-        }
-        if (a.softcap > 0.0f) {
+  for (int i = 0; i < WM; ++i)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[i][j][gq * 4 + e] = a.softcap * tanhf(acc[i][j][gq * 4 + e] / a.softcap);
-        }
-        if (a.act) {
+    for (int j = 0; j < WN; ++j)
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (f + e >= a.act_from && f + e < act_to) acc[i][j][gq * 4 + e] = tl_act_apply(a.act, acc[i][j][gq * 4 + e], a.act_p, a.act_q);
-        }
-        if (v4 && f + 4 <= a.rows) {
-          *reinterpret_cast<float4*>(yr + f) =
-              make_float4(acc[i][j][gq * 4], acc[i][j][gq * 4 + 1], acc[i][j][gq * 4 + 2], acc[i][j][gq * 4 + 3]);
-        } else {
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+  const int fr = lane & 31, sw = (fr >> 1) & 7;
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (f + e < a.rows) yr[f + e] = acc[i][j][gq * 4 + e];
-        }
+  for (int st = 0; st < NS - 1; ++st) fetch(st, st);
+  int slot = 0;
+  for (int st = 0; st < steps; ++st) {
+    if (FIRST && lead) dma_wait<(IW + IX + 1) * (NS - 2)>();
+    else dma_wait<(IW + IX) * (NS - 2)>();
+    __syncthreads();  // the step has arrived for all waves, and all have left the slot of the step before
+    fetch(st + NS - 1, slot == 0 ? NS - 1 : slot - 1);
+    const unsigned char* b = dlds + slot * STAGE;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const int q = ((2 * ks + (lane >> 5)) ^ sw) << 4;
+      bf16x8 af[WM], bf[WN];
+#pragma unroll
+      for (int i = 0; i < WM; ++i) af[i] = *reinterpret_cast<const bf16x8*>(b + ((wm * WM + i) * 32 + fr) * 128 + q);
+#pragma unroll
+      for (int j = 0; j < WN; ++j) bf[j] = *reinterpret_cast<const bf16x8*>(b + (BM + (wn * WN + j) * 32 + fr) * 128 + q);
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int i = 0; i < WM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i], bf[j], acc[i][j], 0, 0, 0);
+      if (FIRST && lead && wn == 0) {
+        const bf16x8 x = *reinterpret_cast<const bf16x8*>(b + (BM + BN + fr) * 128 + q);
+#pragma unroll
+        for (int i = 0; i < WM; ++i) acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i], x, acc[i][0], 0, 0, 0);
       }
     }
+    slot = slot == NS - 1 ? 0 : slot + 1;
   }
+  dma_wait<0>();
+  dense_store<WM, WN>(a, acc, a.y, f0 + wm * WM * 32, t0 + wn * WN * 32, hi, lane);
+}
+
+// x[T][ldx] -> bf16 [T][cols], and behind it the second terms of the first `exact` rows; eight columns a thread
+__global__ __launch_bounds__(256) void dense_rows_kernel(const float* __restrict__ x, int ldx, int T, int cols, int exact,
+                                                         unsigned short* __restrict__ plane) {
+  const long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 8;
+  if (i >= (long long)T * cols) return;
+  const int t = (int)(i / cols), c = (int)(i - (long long)t * cols);
+  const f32x4 a = *reinterpret_cast<const f32x4*>(x + (size_t)t * ldx + c), b = *reinterpret_cast<const f32x4*>(x + (size_t)t * ldx + c + 4);
+  bf16x8 hi, lo;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float f = e < 4 ? a[e] : b[e - 4];
+    hi[e] = (__bf16)f;
+    lo[e] = (__bf16)(f - (float)hi[e]);
+  }
+  *reinterpret_cast<bf16x8*>(plane + i) = hi;
+  if (t < exact) *reinterpret_cast<bf16x8*>(plane + (size_t)T * cols + i) = lo;
 }
 
 // RW rows per wave, 4 waves per workgroup: 2 x RW sixteen-byte weight loads in flight per lane (tl_bf16.h)
@@ -273,6 +403,31 @@ __global__ __launch_bounds__(256) void dense_gemv_kernel(const unsigned short* _
   }
 }
 
+template <int NWM, int NWN, int WM, int WN, int NS, bool FIRST>
+int dense_plane_go(const DenseArgs& a, hipStream_t s) {
+  constexpr int BM = 32 * WM * NWM, BN = 32 * WN * NWN, LDS = NS * 128 * (BM + BN + (FIRST ? 32 : 0));
+  static TlDeviceOnce lds_raised;
+  auto kernel = dense_plane_kernel<NWM, NWN, WM, WN, NS, FIRST>;
+  TL_TRY(tl_raise_lds_limit(kernel, LDS, lds_raised));
+  const int mt = (a.rows + BM - 1) / BM, nt = (a.T + BN - 1) / BN;
+  kernel<<<mt * nt, 64 * NWM * NWN, LDS, s>>>(a, mt, nt);
+  TL_HIP(hipGetLastError());
+  return 0;
+}
+
+int dense_plane_run(const DenseArgs& a, int waves, hipStream_t s) {
+  const bool first = a.exact_items > 0;
+  const long long pieces = (long long)a.T * a.cols / 8;
+  dense_rows_kernel<<<dim3((unsigned)((pieces + 255) / 256)), 256, 0, s>>>(a.x, a.ldx, a.T, a.cols, first ? a.exact_items : 0, a.plane);
+  TL_HIP(hipGetLastError());
+  if (waves == 8) return first ? dense_plane_go<4, 2, 1, 2, 4, true>(a, s) : dense_plane_go<4, 2, 1, 2, 4, false>(a, s);
+  return first ? dense_plane_go<2, 2, 2, 2, 2, true>(a, s) : dense_plane_go<2, 2, 2, 2, 2, false>(a, s);
+}
+// (32-bit byte offsets inside the matrix and the plane)
+bool dense_plane_fits(const DenseArgs& a) {
+  return a.cols % 64 == 0 && (size_t)a.rows * a.cols < ((size_t)1 << 31) && ((size_t)a.T + 32) * a.cols < ((size_t)1 << 31);
+}
+
 }  // namespace
 
 int tl_launch_dense_gemm(const DenseArgs& a, hipStream_t s) {
@@ -294,7 +449,8 @@ int tl_launch_dense_gemm(const DenseArgs& a, hipStream_t s) {
   // rows too, so that a tile's way in and out is short beside its products: 256 tiles, large / small, 512 columns 22.1 / 16.4 us
   // with one term and 32.2 / 23.7 with three, 1024 29.3 / 25.9 and 48.4 / 41.7, 2048 43.7 / 42.1 and 82.9 / 77.5, 4096 74 / 78 and
   // 148 / 149, 14336 224 / 345 and 483 / 511. Beyond, small tiles start a second round: 264 tiles of 2048 columns 56 / 63 and
-  // 87 / 91, 384 of 1024 32 / 36 and 53 / 59, 448 of 4096 107 / 154 and 200 / 265. Either tile gives the same bits. The experts'
+  // 87 / 91, 384 of 1024 32 / 36 and 53 / 59, 448 of 4096 107 / 154 and 200 / 265. Either tile gives the same bits (but
+  // for exact_items, whose second terms join after each step's products). The experts'
   // grouped launches, whose small tiles are mostly half-empty, gain from large ones with one term (221 -> 193 us) and lose with
   // three (356 -> 413 us).
   const long long small_tiles = ((a.rows + 63) / 64) * ((per_group + 63) / 64) * groups;
@@ -303,12 +459,22 @@ int tl_launch_dense_gemm(const DenseArgs& a, hipStream_t s) {
   const bool big = force ? atoi(force) == 128
                          : a.rows >= 256 && (a.group_off ? a.terms == 1 && per_group >= 96
                                                          : big_tiles >= tl_num_cus() && (small_tiles > 4 * tl_num_cus() || a.cols >= 4096));
-  const int BM = big ? 128 : 64, BN = big ? 128 : 64;
-  dim3 grid((a.rows + BM - 1) / BM, (a.T + BN - 1) / BN, groups);
-  TL_REQUIRE(grid.y <= 65535 && grid.z <= 65535, "dense gemm: launch too large");
   const bool first = a.exact_items > 0 && a.terms == 1;
   // wide loads: every matrix, row and piece of eight columns at 16 bytes
   const bool vec = (a.cols & 7) == 0 && (a.ldx & 3) == 0 && ((size_t)a.x & 15) == 0 && ((size_t)a.w & 15) == 0 && (a.x_gstride & 3) == 0;
+  // The plane kernel takes the launches whose 128 x 128 tiles occupy half of the CUs or more and are long enough to pay for the
+  // conversion (rows x columns x items, without / with it, conversion included: 10304 x 2048 x 1999 174 / 114 us, x 512 56 / 36,
+  // x 200 36 / 24; 4096 x 2048 x 1999 66 / 45, x 1024 46 / 30; 2048 x 4096 x 1999 80 / 51, x 1024 47 / 43; 4096 x 1024 x 1024 26 / 20;
+  // on the line 4096 x 2048 x 512 26.3 / 25.8 and 2048 x 2048 x 1024 26.4 / 26.5; below 1024 x 1024 x 1999 16 / 18, 2048 x 4096 x 512
+  // 33 / 39). One tile a CU: eight waves and three steps ahead; more: two workgroups of four waves, which fill each other's waits
+  // (256 tiles 30.3 / 32.5 us, 324 tiles 44.8 / 36.4). TL_DENSE_TILE=64, 128: the kernel above.
+  if (a.plane && a.terms == 1 && groups == 1 && !a.group_off && !a.x_rows && vec && dense_plane_fits(a) && !force &&
+      2 * big_tiles >= tl_num_cus() && big_tiles * a.cols > 1024ll * tl_num_cus()) {
+    return dense_plane_run(a, big_tiles <= tl_num_cus() ? 8 : 4, s);
+  }
+  const int BM = big ? 128 : 64, BN = big ? 128 : 64;
+  dim3 grid((a.rows + BM - 1) / BM, (a.T + BN - 1) / BN, groups);
+  TL_REQUIRE(grid.y <= 65535 && grid.z <= 65535, "dense gemm: launch too large");
 #define DENSE(T, W, F) (vec ? dense_gemm_kernel<T, W, W, true, F><<<grid, 256, 0, s>>>(a) : dense_gemm_kernel<T, W, W, false, F><<<grid, 256, 0, s>>>(a))
   if (big) {
     if (first) DENSE(1, 2, true);
@@ -450,4 +616,25 @@ extern "C" int tl_dense_matmul_heads(const void* w_bf16_dev, int groups, int row
   a.x_gstride = x_stride;
   a.y_gstride = y_stride;
   return tl_launch_dense_gemm(a, s);
+}
+
+extern "C" int tl_debug_dense_plane(const void* w_bf16_dev, int rows, int cols, const float* x_dev, int ldx, float* y_dev, int num_tokens,
+                                    int exact_items, int waves, void* plane_dev, void* stream) {
+  DenseArgs a = {};
+  a.w = static_cast<const uint16_t*>(w_bf16_dev);
+  a.rows = rows;
+  a.cols = cols;
+  a.x = x_dev;
+  a.ldx = ldx;
+  a.y = y_dev;
+  a.ldy = rows;
+  a.T = num_tokens;
+  a.terms = 1;
+  a.exact_items = exact_items;
+  a.plane = static_cast<uint16_t*>(plane_dev);
+  TL_REQUIRE(a.w && x_dev && y_dev && plane_dev && rows > 0 && cols > 0 && num_tokens > 0 && ldx >= cols && ldx % 4 == 0 &&
+                 exact_items >= 0 && exact_items <= 32 && (waves == 4 || waves == 8) && dense_plane_fits(a) &&
+                 (((size_t)w_bf16_dev | (size_t)x_dev | (size_t)plane_dev) & 15) == 0,
+             "tl_debug_dense_plane: bad argument");
+  return dense_plane_run(a, waves, static_cast<hipStream_t>(stream));
 }
