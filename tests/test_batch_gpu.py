@@ -275,3 +275,40 @@ def test_packed_prompts_longer_than_a_sequence(pkg):
     assert np.linalg.norm(packed - alone) <= 4e-6 * np.linalg.norm(alone)
     assert np.array_equal(ids, packed.argmax(1))
     m.free()
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd", [(8, 1, 64), (6, 2, 128), (4, 4, 64)])
+def test_packed_attention_by_row_tiles(pkg, monkeypatch, heads, kv_heads, hd):
+    """A packed batch large enough for the matrix-core attention: runs of 1, 31, 32, 33, 127, 129 tokens, slots out of order, a
+    second batch that goes on behind the first one's rows and two runs of one sequence in a batch. Against the per-token FP32
+    kernel: both are within 2^-22 of the exact sums a layer and product (two layers, a handful of products each)."""
+    from tinyllama_cpp_amd import engine as E
+    E.init(0)
+    cfg = dict(pkg.synth.SHAPES["tiny-gqa"], hidden=heads * hd, n_heads=heads, n_kv_heads=kv_heads, n_layers=2, max_pos=640)
+    cfg, tensors = pkg.synth.build_model(cfg, "q4_k_m", seed=4)
+    m = E.Model(cfg).load(tensors)
+    m.batch_init(9)
+    rng = np.random.default_rng(9)
+    lens, slots = (33, 1, 129, 320, 31, 127, 32, 300), [8, 3, 0, 5, 2, 7, 1, 4]
+    runs = [(s, 0, rng.integers(0, cfg["vocab"], n)) for s, n in zip(slots, lens)]
+    more = [(s, n, rng.integers(0, cfg["vocab"], k)) for s, n, k in zip(slots, lens, (40, 300, 1, 200, 65, 5, 96, 7))]
+    more.append((more[3][0], more[3][1] + 200, rng.integers(0, cfg["vocab"], 90)))  # goes on behind other sequences' tokens
+    want = {}
+    for switch in ("0", "1"):
+        monkeypatch.setenv("TL_HATTN", switch)
+        m.reset_kv()
+        for k, part in enumerate((runs, more)):
+            toks = np.concatenate([t for _, _, t in part]).astype(np.int32)
+            pos = np.concatenate([np.arange(p, p + len(t)) for _, p, t in part]).astype(np.int32)
+            seq = np.concatenate([np.full(len(t), s) for s, _, t in part]).astype(np.int32)
+            last = np.cumsum([len(t) for _, _, t in part]).astype(np.int32) - 1
+            logits, ids = np.zeros((len(last), cfg["vocab"]), np.float32), np.zeros(len(last), np.int32)
+            from tinyllama_cpp_amd.capi import check, lib
+            check(lib().tl_model_batch_prefill_packed(m.h, toks.size, toks.ctypes.data, pos.ctypes.data, seq.ctypes.data, last.size,
+                                                      last.ctypes.data, logits.ctypes.data, ids.ctypes.data), "packed")
+            if switch == "0":
+                want[k] = logits
+            else:
+                assert not np.array_equal(logits, want[k])  # (the other kernel ran)
+                assert np.linalg.norm(logits - want[k]) <= 4e-6 * np.linalg.norm(want[k])
+    m.free()

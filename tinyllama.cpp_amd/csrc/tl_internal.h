@@ -4,6 +4,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <vector>
+
 #include "tlhip.h"
 #include "tlhip_debug.h"
 
@@ -300,6 +302,19 @@ struct TlHattn {
 bool tl_hattn_supported(const TlHattn& x);
 size_t tl_hattn_bytes(int max_keys, int kv_heads, int dim, int vdim);
 int tl_launch_hattn(const TlHattn& x, void* ws, size_t ws_bytes, hipStream_t s);
+// the same for a packed batch of several sequences' tokens, whose caches lie seq_stride floats apart
+struct TlHattnTile {  // 32 positions from pos on of a sequence of len rows
+  int pos, len, seq, pad;
+};
+struct TlHattnItem {  // 128 rows (token, head) of the run of T tokens tok0 .. at positions start_pos ..; tile: its first key tile in the list
+  int tok0, T, start_pos, row_tile, tile, pad[3];
+};
+constexpr int TL_HATTN_PACK_MAX = 4096;  // tiles, and row tiles, of a launch
+// false: the per-token kernel serves this batch better, or the tiles do not fit the workspace
+bool tl_hattn_pack(const int* pos, const int* seq, int T, int group, int kv_heads, int dim, size_t ws_bytes, std::vector<TlHattnTile>* tiles,
+                   std::vector<TlHattnItem>* items);
+int tl_launch_hattn_packed(const TlHattn& x, size_t seq_stride, const TlHattnTile* tiles_dev, int tiles, const TlHattnItem* items_dev, int items,
+                           void* ws, size_t ws_bytes, hipStream_t s);
 // causal prefill attention on the FP32 matrix instruction (tl_prefill.hip)
 bool tl_attn_prefill_mfma_supported(int nh, int nkv, int hd);
 // planes != NULL: the output as the attn_output GEMM's activation planes (tl_launch_split's layout) instead of `out`

@@ -127,6 +127,7 @@ struct tl_model {
     int max_batch = 0;
     float* kv = nullptr;
     int *toks = nullptr, *pos = nullptr, *seq = nullptr;  // [max_batch]
+    void* pack = nullptr;                                 // [TL_HATTN_PACK_MAX] key tiles, then row tiles of a packed chunk's attention
     float* last_h = nullptr;                              // [max_batch][hidden]: hidden rows whose logits a packed prefill returns
     int* ids = nullptr;                                   // generated ids [step][n]
     size_t ids_cap = 0;
@@ -270,6 +271,7 @@ extern "C" int tl_model_free(tl_model* m) {
   hipFree(m->bt.seq);
   hipFree(m->bt.ids);
   hipFree(m->bt.last_h);
+  hipFree(m->bt.pack);
   if (m->pf.fork) hipEventDestroy(m->pf.fork);
   if (m->pf.join) hipEventDestroy(m->pf.join);
   if (m->pf.side) hipStreamDestroy(m->pf.side);
@@ -1471,6 +1473,36 @@ static int qkv_deferred(tl_model* m, LayerW& L, int T, hipStream_t s) {
   TL_HIP(hipStreamWaitEvent(s, p.join, 0));
   return 0;
 }
+// the f16 attention over layer l's rows at kc / vc, and its workspace (made at the first use)
+static TlHattn half_attn(tl_model* m, const float* kc, const float* vc, int T, int start_pos) {
+  TlHattn x = {};
+  x.q = m->pf.qb;
+  x.kc = kc;
+  x.vc = vc;
+  x.out = m->pf.ab;
+  x.ldq = m->qd_l;
+  x.qhs = x.khs = x.dim = x.vdim = m->head_dim;
+  x.kld = x.vld = m->nkv_l * m->head_dim;
+  x.T = T;
+  x.start_pos = start_pos;
+  x.heads = m->nh_l;
+  x.kv_heads = m->nkv_l;
+  x.scale = 1.0f / sqrtf((float)m->head_dim);
+  x.eps = 1e-9f;
+  return x;
+}
+static bool half_attn_on() {  // TL_HATTN=0: the FP32 attention kernels everywhere (A/B runs and tests)
+  const char* ha = getenv("TL_HATTN");
+  return !(ha && atoi(ha) == 0);
+}
+static int half_attn_ws(tl_model* m) {
+  tl_model::Prefill& p = m->pf;
+  if (p.hattn) return 0;
+  const size_t bytes = tl_hattn_bytes(m->cfg.max_position_embeddings, m->nkv_l, m->head_dim, m->head_dim);
+  TL_HIP(hipMalloc(&p.hattn, bytes));
+  p.hattn_bytes = bytes;
+  return 0;
+}
 static int prefill_attn_half(tl_model* m, int l, int T, int start_pos, hipStream_t s) {
   const tl_model_config& c = m->cfg;
   tl_model::Prefill& p = m->pf;
@@ -1502,27 +1534,9 @@ static int prefill_attn_half(tl_model* m, int l, int T, int start_pos, hipStream
   // the attention output goes straight into the planes of the attn_output GEMM where the MFMA kernel serves the head shape
   // (no split launch; TL_ATTN_PLANES=0 keeps the launch, for A/B runs and the bit-identity test)
   const char* ap = getenv("TL_ATTN_PLANES");
-  const char* ha = getenv("TL_HATTN");  // 0: the FP32 attention kernel everywhere (A/B runs and tests)
-  TlHattn x = {};
-  x.q = p.qb;
-  x.kc = m->kc(l);
-  x.vc = m->vc(l);
-  x.out = p.ab;
-  x.ldq = m->qd_l;
-  x.kld = x.vld = m->nkv_l * hd;
-  x.qhs = x.khs = x.dim = x.vdim = hd;
-  x.T = T;
-  x.start_pos = start_pos;
-  x.heads = m->nh_l;
-  x.kv_heads = m->nkv_l;
-  x.scale = scale;
-  x.eps = 1e-9f;
-  if (terms == TL_TERMS_HALF && tl_hattn_supported(x) && !(ha && atoi(ha) == 0)) {
-    if (!p.hattn) {
-      const size_t bytes = tl_hattn_bytes(c.max_position_embeddings, m->nkv_l, hd, hd);
-      TL_HIP(hipMalloc(&p.hattn, bytes));
-      p.hattn_bytes = bytes;
-    }
+  const TlHattn x = half_attn(m, m->kc(l), m->vc(l), T, start_pos);
+  if (terms == TL_TERMS_HALF && tl_hattn_supported(x) && half_attn_on()) {
+    TL_TRY(half_attn_ws(m));
     TL_TRY(tl_launch_hattn(x, p.hattn, p.hattn_bytes, s));
     TL_TRY(tl_launch_split(0, p.ab, nullptr, p.planes, ps, T, m->qd_l, terms, 0.f, s));
   } else if (terms != TL_TERMS_HALF && tl_attn_prefill_mfma_supported(m->nh_l, m->nkv_l, hd) && !(ap && atoi(ap) == 0)) {
@@ -1711,7 +1725,11 @@ extern "C" int tl_tp_local_group_prefill(tl_model* const* ms, int n, const int* 
 // more GEMM, and a per-row arg-max writes the next token ids and advances the positions on the device, so that a greedy
 // generation loop needs no host round trip per step. Every sequence decodes exactly as it would alone (see tl_batch.hip
 // on the reference's history_len quirk). tp_size 1 only.
-static int batch_attn_half(tl_model* m, int l, int T, hipStream_t s) {
+struct BatchPack {  // a packed chunk's attention by row tiles (tl_hattn.hip); no tiles: token by token
+  std::vector<TlHattnTile> tiles;
+  std::vector<TlHattnItem> items;
+};
+static int batch_attn_half(tl_model* m, int l, int T, const BatchPack* pack, hipStream_t s) {
   const tl_model_config& c = m->cfg;
   tl_model::Prefill& p = m->pf;
   LayerW& L = m->layers[l];
@@ -1728,7 +1746,12 @@ static int batch_attn_half(tl_model* m, int l, int T, hipStream_t s) {
   // the attention output goes straight into the planes of the attn_output GEMM (no split launch; TL_ATTN_PLANES=0 keeps
   // the launch, for A/B runs and the bit-identity test)
   const char* ap = getenv("TL_ATTN_PLANES");
-  if (terms == TL_TERMS_HALF || (ap && atoi(ap) == 0)) {
+  if (pack && !pack->items.empty()) {
+    const TlHattnTile* tiles = static_cast<const TlHattnTile*>(m->bt.pack);
+    TL_TRY(tl_launch_hattn_packed(half_attn(m, m->bkc(l), m->bvc(l), T, 0), m->kv_layer_elems, tiles, (int)pack->tiles.size(),
+                                  reinterpret_cast<const TlHattnItem*>(tiles + TL_HATTN_PACK_MAX), (int)pack->items.size(), p.hattn, p.hattn_bytes, s));
+    TL_TRY(tl_launch_split(0, p.ab, nullptr, p.planes, ps, T, m->qd_l, terms, 0.f, s));
+  } else if (terms == TL_TERMS_HALF || (ap && atoi(ap) == 0)) {
     TL_TRY(tl_launch_batch_attn(p.qb, m->bkc(l), m->bvc(l), m->kv_layer_elems, p.ab, m->bt.pos, m->bt.seq, T, m->nh_l,
                                 m->nkv_l, hd, c.max_position_embeddings, m->bt.max_batch, scale, s));
     TL_TRY(tl_launch_split(0, p.ab, nullptr, p.planes, ps, T, m->qd_l, terms, 0.f, s));
@@ -1826,12 +1849,12 @@ static int batch_layers_gemv(tl_model* m, int T, hipStream_t s) {
 // one step for the T tokens in bt.toks / bt.pos / bt.seq; ids_dev: [T] next ids (first maximum of each logits row);
 // advance: the ids become the next tokens and the positions move on (device-resident loop)
 // all layers for the T tokens in bt.toks / bt.pos / bt.seq: the residual stream ends up in pf.xb [T][hidden]
-static int batch_layers(tl_model* m, int T, hipStream_t s) {
+static int batch_layers(tl_model* m, int T, hipStream_t s, const BatchPack* pack = nullptr) {
   TL_REQUIRE(T >= 1 && T <= m->pf.cap, "tl_model: a batched step of %d tokens exceeds the chunk workspaces (%d)", T, m->pf.cap);
   if (T <= m->bt.gemv_max) return batch_layers_gemv(m, T, s);
   TL_TRY(prefill_embed(m, m->bt.toks, T, s));
   for (int l = 0; l < m->cfg.num_hidden_layers; ++l) {
-    TL_TRY(batch_attn_half(m, l, T, s));
+    TL_TRY(batch_attn_half(m, l, T, pack, s));
     TL_TRY(prefill_mlp_half(m, l, T, s));
   }
   return flush_residual(m, s);
@@ -1890,6 +1913,7 @@ extern "C" int tl_model_batch_init(tl_model* m, int max_batch) {
     TL_HIP(hipFree(b.pos));
     TL_HIP(hipFree(b.seq));
     TL_HIP(hipFree(b.last_h));
+    TL_HIP(hipFree(b.pack));
     if (b.ids) TL_HIP(hipFree(b.ids));
     b = tl_model::Batch();
   }
@@ -1899,6 +1923,7 @@ extern "C" int tl_model_batch_init(tl_model* m, int max_batch) {
   TL_HIP(hipMalloc(&b.toks, sizeof(int) * kPrefillChunk));  // a packed prompt chunk carries up to kPrefillChunk tokens
   TL_HIP(hipMalloc(&b.pos, sizeof(int) * kPrefillChunk));
   TL_HIP(hipMalloc(&b.seq, sizeof(int) * kPrefillChunk));
+  TL_HIP(hipMalloc(&b.pack, (sizeof(TlHattnTile) + sizeof(TlHattnItem)) * TL_HATTN_PACK_MAX));
   TL_HIP(hipMalloc(&b.last_h, sizeof(float) * (size_t)max_batch * m->cfg.hidden_size));
   b.max_batch = max_batch;
   b.gemv_max = batch_gemv_ok(m) ? 4 : 0;  // one pass of up to four vectors: 2.5 / 4.0 / 4.1 ms per step for 2 / 3 / 4 sequences; the
@@ -1983,12 +2008,22 @@ extern "C" int tl_model_batch_prefill_packed(tl_model* m, int n_tokens, const in
   const size_t H = c.hidden_size;
   const int chunk = chunk_tokens(m);
   TL_REQUIRE(chunk >= 1 && chunk <= kPrefillChunk, "tl_model_batch_prefill_packed: workspaces are missing");
+  const bool half = chunk_terms(m) == TL_TERMS_HALF && half_attn_on() && tl_hattn_supported(half_attn(m, m->bkc(0), m->bvc(0), 1, 0));
+  if (half) TL_TRY(half_attn_ws(m));
+  std::vector<BatchPack> packs((n_tokens + chunk - 1) / chunk);  // (live until the stream has been waited for)
   for (int c0 = 0; c0 < n_tokens; c0 += chunk) {
     const int T = n_tokens - c0 < chunk ? n_tokens - c0 : chunk;
+    BatchPack& pack = packs[c0 / chunk];
+    if (half && T > m->bt.gemv_max &&
+        tl_hattn_pack(positions_host + c0, seq_idx_host + c0, T, m->nh_l / m->nkv_l, m->nkv_l, m->head_dim, m->pf.hattn_bytes, &pack.tiles, &pack.items)) {
+      TlHattnTile* tiles = static_cast<TlHattnTile*>(m->bt.pack);
+      TL_HIP(hipMemcpyAsync(tiles, pack.tiles.data(), sizeof(TlHattnTile) * pack.tiles.size(), hipMemcpyHostToDevice, s));
+      TL_HIP(hipMemcpyAsync(tiles + TL_HATTN_PACK_MAX, pack.items.data(), sizeof(TlHattnItem) * pack.items.size(), hipMemcpyHostToDevice, s));
+    } else pack.items.clear();
     TL_HIP(hipMemcpyAsync(m->bt.toks, tokens_host + c0, sizeof(int) * T, hipMemcpyHostToDevice, s));
     TL_HIP(hipMemcpyAsync(m->bt.pos, positions_host + c0, sizeof(int) * T, hipMemcpyHostToDevice, s));
     TL_HIP(hipMemcpyAsync(m->bt.seq, seq_idx_host + c0, sizeof(int) * T, hipMemcpyHostToDevice, s));
-    TL_TRY(batch_layers(m, T, s));
+    TL_TRY(batch_layers(m, T, s, &pack));
     for (int j = 0; j < n_last; ++j) {
       const int r = last_rows_host[j] - c0;
       if (r >= 0 && r < T)
