@@ -570,3 +570,29 @@ def test_causal_conv_output_behind_the_last_row(pkg):
     assert np.array_equal(got[0], got[1]) and np.abs(got[0]).max() > 0
     hist = engine.DeviceBuffer.from_numpy(np.zeros((taps - 1, C), np.float32))
     assert capi.lib().tl_causal_conv(buf.ptr + 4 * off, ld, C, taps, T, None, wd.ptr, hist.ptr, 0, 0, end - 4, C, None) != 0
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,window", [(8, 2, 64, 300), (3, 3, 64, 0), (4, 1, 128, 259), (2, 2, 128, 64)])
+def test_window_attention_over_wide_rows(env, heads, kv_heads, dim, window):
+    """Rows of 64 and 128 numbers for keys and values: sixteen lanes a key, records merged in a second launch."""
+    test_window_attention_prompt_and_decode(env, heads, kv_heads, dim, dim, window)
+
+
+@pytest.mark.parametrize("dim,top,ff,shared_ff", [(64, 6, 1032, 40), (128, 4, 24, 0), (64, 10, 16, 1544)])
+def test_decode_step_with_wide_rows_and_many_slots(env, dim, top, ff, shared_ff):
+    """The captured decode step over heads of 64 and 128: positions across 256, 512 and the window (one split, several, the last of
+    which merges), seven to eleven expert slots of rows below, at and above 1024 columns, and a norm row of two numbers a thread."""
+    S = env["synth"]
+    L = S.stack_layer
+    cfg = S.stack_config(1040, 211, [L(4, 2, dim, dim, 600, v_mix=True, experts=12, top=top, ff=ff, shared_ff=shared_ff),
+                                     L(2, 2, dim, dim, None, v_mix=True, experts=12, top=top, ff=ff, shared_ff=shared_ff)])
+    m, _, orc = make(env, cfg, seed=5, max_pos=1024)
+    toks = np.random.default_rng(dim).integers(0, cfg["vocab"], 640).astype(np.int32)
+    want = orc.forward(list(toks))
+    for lo, hi in ((0, 3), (252, 260), (508, 516), (596, 604), (636, 640)):
+        m.reset_kv()
+        if lo:
+            m.prefill_rows(toks[:lo], 0, np.array([lo - 1], np.int32))
+        got = np.stack([m.decode(int(toks[i]), i)[0] for i in range(lo, hi)])
+        assert rel_rms(got, want[lo:hi]) < FP32_TOL, (lo, hi)
+    m.free()

@@ -19,6 +19,8 @@
 #include <math.h>
 #include <stdlib.h>
 
+#include <type_traits>
+
 #include "tl_internal.h"
 #include "tl_stack.h"
 
@@ -62,12 +64,15 @@ __device__ __forceinline__ float swa_ld_agent(const float* p) {  // past this CU
 }
 
 // out = sum_z o_z e^(m_z - M) / sum_z l_z e^(m_z - M) over the nsplit records of a (token, head), in split order; one wave
-__device__ __forceinline__ void swa_merge_records(const SwaArgs& a, int t, int h, int lane) {
+__device__ __forceinline__ void swa_merge_records(const SwaArgs& a, int nsplit, int t, int h, int lane) {
   const int rs = a.vdim + 2;
   const float* rec = a.ws + ((size_t)t * a.heads + h) * a.nsplit * rs;
   // lane z holds record z's max and sum (nsplit <= 64): one round trip, then everything is in registers
-  const float mz = lane < a.nsplit ? swa_ld_agent(rec + (size_t)lane * rs) : -INFINITY;
-  const float lz = lane < a.nsplit ? swa_ld_agent(rec + (size_t)lane * rs + 1) : 0.0f;
+  const float mz = lane < nsplit ? swa_ld_agent(rec + (size_t)lane * rs) : -INFINITY;
+  const float lz = lane < nsplit ? swa_ld_agent(rec + (size_t)lane * rs + 1) : 0.0f;
+  float first[8];  // ... with the first eight records' values behind them
+#pragma unroll
+  for (int u = 0; u < 8; ++u) first[u] = lane < a.vdim ? swa_ld_agent(rec + (size_t)(u < nsplit ? u : nsplit - 1) * rs + 2 + lane) : 0.0f;
   float M = mz;
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
@@ -75,28 +80,95 @@ __device__ __forceinline__ void swa_merge_records(const SwaArgs& a, int t, int h
   if (a.sink) M = fmaxf(M, sv);
   const float fz = mz == -INFINITY ? 0.0f : expf(mz - M);
   float L = a.sink ? expf(sv - M) : 0.0f;
-  for (int z = 0; z < a.nsplit; ++z) L += __shfl(lz * fz, z);  // in split order
+  for (int z = 0; z < nsplit; ++z) L += __shfl(lz * fz, z);  // in split order
   float* op = a.out + (size_t)t * a.heads * a.vdim + (size_t)h * a.vdim;
   const float of = swa_out_factor(a, t, h);
   for (int d0 = 0; d0 < a.vdim; d0 += 64) {  // every lane stays in the loop: a shuffle reads nothing from a lane that has left
     const int d = d0 + lane;
     float acc = 0.0f;
-    for (int z0 = 0; z0 < a.nsplit; z0 += 8) {  // eight records' values in flight together (clamped index, weight 0 beyond)
+    for (int z0 = 0; z0 < nsplit; z0 += 8) {  // eight records' values in flight together (clamped index, weight 0 beyond)
       float v[8], f[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        const int z = z0 + u < a.nsplit ? z0 + u : a.nsplit - 1;
-        v[u] = d < a.vdim ? swa_ld_agent(rec + (size_t)z * rs + 2 + d) : 0.0f;
+        const int z = z0 + u < nsplit ? z0 + u : nsplit - 1;
+        v[u] = d0 + z0 == 0 ? first[u] : d < a.vdim ? swa_ld_agent(rec + (size_t)z * rs + 2 + d) : 0.0f;
       }
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        const float fu = __shfl(fz, z0 + u < a.nsplit ? z0 + u : 0);
-        f[u] = z0 + u < a.nsplit ? fu : 0.0f;
+        const float fu = __shfl(fz, z0 + u < nsplit ? z0 + u : 0);
+        f[u] = z0 + u < nsplit ? fu : 0.0f;
       }
 #pragma unroll
       for (int u = 0; u < 8; ++u) acc += v[u] * f[u];  // in split order
     }
     if (d < a.vdim) op[d] = (a.sigmoid ? acc : acc / L) * of;
+  }
+}
+
+// The waves' partial (max, sum) in ml[waves][2] and outputs in ow (NSUB rows of vdim a wave, to be added up) -> the output of
+// (token, head), or the record of this split and, from the last split to arrive, the output.
+template <int NSUB>
+__device__ __forceinline__ float swa_wave_out(const float* ow, int vdim, int w, int d) {
+  float v = ow[(size_t)w * NSUB * vdim + d];
+#pragma unroll
+  for (int u = 1; u < NSUB; ++u) v += ow[(size_t)(w * NSUB + u) * vdim + d];
+  return v;
+}
+// nsplit: the splits that leave a record.
+template <int NSUB, int WAVES>
+__device__ __forceinline__ void swa_finish(const SwaArgs& a, const float* ml, const float* ow, int nsplit, int t, int h) {
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  __syncthreads();
+  float M = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) M = fmaxf(M, ml[w * 2]);
+  // the sink joins where the LAST merge happens: here without splits, in swa_merge_records with them
+  const bool sink_here = a.sink && nsplit == 1;
+  const float sv = a.sink && a.sink_val ? a.sink_val[h] : 0.0f;
+  if (sink_here) M = fmaxf(M, sv);
+  float f[WAVES], L = sink_here ? expf(sv - M) : 0.0f;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    f[w] = ml[w * 2] == -INFINITY ? 0.0f : expf(ml[w * 2] - M);  // a wave without a piece counts nothing
+    L += ml[w * 2 + 1] * f[w];
+  }
+  if (nsplit > 1) {
+    float* rec = a.ws + (((size_t)t * a.heads + h) * a.nsplit + blockIdx.z) * (a.vdim + 2);
+    // (agent-scope stores: with the merge in this launch the reader may sit on another XCD, behind another L2)
+    if (tid == 0) {
+      swa_st_agent(rec, M);  // -inf and sum 0 when this split had no piece
+      swa_st_agent(rec + 1, M == -INFINITY ? 0.0f : L);
+    }
+    for (int d = tid; d < a.vdim; d += 64 * WAVES) {
+      float acc = 0.0f;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) acc += f[w] == 0.0f ? 0.0f : swa_wave_out<NSUB>(ow, a.vdim, w, d) * f[w];
+      swa_st_agent(rec + 2 + d, M == -INFINITY ? 0.0f : acc);
+    }
+    if (!a.done_cnt) return;  // swa_combine_kernel follows
+    // The last workgroup of this (token, head) to arrive merges the records itself (no second launch): the record stores
+    // are acknowledged, then one arrival per workgroup is counted; the counter goes back to zero for the next launch.
+    __shared__ int is_last;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+      unsigned* c = a.done_cnt + (size_t)t * a.heads + h;
+      const unsigned before = __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      is_last = before + 1u == (unsigned)nsplit;
+      if (is_last) __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!is_last || wave != 0) return;
+    swa_merge_records(a, nsplit, t, h, lane);
+    return;
+  }
+  float* op = a.out + (size_t)t * a.heads * a.vdim + (size_t)h * a.vdim;
+  const float of = swa_out_factor(a, t, h);
+  for (int d = tid; d < a.vdim; d += 64 * WAVES) {
+    float acc = 0.0f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) acc += f[w] == 0.0f ? 0.0f : swa_wave_out<NSUB>(ow, a.vdim, w, d) * f[w];
+    op[d] = (a.sigmoid ? acc : acc / L) * of;
   }
 }
 
@@ -219,61 +291,124 @@ __global__ __launch_bounds__(256) void swa_kernel(const SwaArgs a) {
     const int d = lane + 64 * r;
     if (d < a.vdim) ow[wave * a.vdim + d] = o[r];
   }
-  __syncthreads();
-  float M = -INFINITY;
-#pragma unroll
-  for (int w = 0; w < SWA_WAVES; ++w) M = fmaxf(M, ml[w * 2]);
-  // the sink joins where the LAST merge happens: here without splits, in swa_merge_records with them
-  const bool sink_here = a.sink && nsplit == 1;
-  const float sv = a.sink && a.sink_val ? a.sink_val[h] : 0.0f;
-  if (sink_here) M = fmaxf(M, sv);
-  float f[SWA_WAVES], L = sink_here ? expf(sv - M) : 0.0f;
-#pragma unroll
-  for (int w = 0; w < SWA_WAVES; ++w) {
-    f[w] = ml[w * 2] == -INFINITY ? 0.0f : expf(ml[w * 2] - M);  // a wave without a piece counts nothing
-    L += ml[w * 2 + 1] * f[w];
-  }
-  if (nsplit > 1) {
-    float* rec = a.ws + (((size_t)t * a.heads + h) * nsplit + blockIdx.z) * (a.vdim + 2);
-    // (agent-scope stores: with the merge in this launch the reader may sit on another XCD, behind another L2)
-    if (tid == 0) {
-      swa_st_agent(rec, M);  // -inf and sum 0 when this split had no piece
-      swa_st_agent(rec + 1, M == -INFINITY ? 0.0f : L);
-    }
-    for (int d = tid; d < a.vdim; d += 256) {
-      float acc = 0.0f;
-#pragma unroll
-      for (int w = 0; w < SWA_WAVES; ++w) acc += f[w] == 0.0f ? 0.0f : ow[w * a.vdim + d] * f[w];
-      swa_st_agent(rec + 2 + d, M == -INFINITY ? 0.0f : acc);
-    }
-    if (!a.done_cnt) return;  // swa_combine_kernel follows
-    // The last workgroup of this (token, head) to arrive merges the records itself (no second launch): the record stores
-    // are acknowledged, then one arrival per workgroup is counted; the counter goes back to zero for the next launch.
-    __shared__ int is_last;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (tid == 0) {
-      unsigned* c = a.done_cnt + (size_t)t * a.heads + h;
-      const unsigned before = __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      is_last = before + 1u == (unsigned)nsplit;
-      if (is_last) __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();
-    if (!is_last || wave != 0) return;
-    swa_merge_records(a, t, h, lane);
-    return;
-  }
-  float* op = a.out + (size_t)t * a.heads * a.vdim + (size_t)h * a.vdim;
-  const float of = swa_out_factor(a, t, h);
-  for (int d = tid; d < a.vdim; d += 256) {
-    float acc = 0.0f;
-#pragma unroll
-    for (int w = 0; w < SWA_WAVES; ++w) acc += f[w] == 0.0f ? 0.0f : ow[w * a.vdim + d] * f[w];
-    op[d] = (a.sigmoid ? acc : acc / L) * of;
-  }
+  swa_finish<1, SWA_WAVES>(a, ml, ow, nsplit, t, h);
 }
 
-__global__ __launch_bounds__(64) void swa_combine_kernel(const SwaArgs a) { swa_merge_records(a, blockIdx.x, blockIdx.y, threadIdx.x); }
+// The same work split and tail for key and value rows of 64 NV numbers at 16 bytes: sixteen lanes own a key (its dot product is four
+// DPP additions), four keys a load, and all the loads of a step -- 64 / NV keys, their values and the query -- are in flight together.
+// With a lane per key, the values' eight rows a step are eight round trips one after another, which is what that kernel's time is:
+// 32 heads of 64 over 700 keys, one token, 14.1 us, here 10.3 (a launch without work takes 3; what is left is the position, the rows and, from
+// 257 keys on, the records, one after another). Eight waves a workgroup and half the splits: 11.9; 1024 keys without records: 12.4.
+__device__ __forceinline__ float swa_sum16(float v) {
+  auto add = [](float x, auto ctrl_c) {
+    constexpr int CTRL = decltype(ctrl_c)::value;
+    return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, false));
+  };
+  v = add(v, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
+  v = add(v, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+  v = add(v, std::integral_constant<int, 0x141>{});  // row_half_mirror
+  return add(v, std::integral_constant<int, 0x140>{});  // row_mirror
+}
+template <int NV>
+__global__ __launch_bounds__(256) void swa_rows_kernel(const SwaArgs a) {
+  constexpr int W = SWA_WAVES, D = 64 * NV, U = 16 / NV;  // keys a lane group takes in a step
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  __shared__ __attribute__((aligned(16))) float ow[W * 4 * D];
+  __shared__ float ml[W * 2];
+  // neighbouring workgroups go to the 8 XCDs in turn: with kv heads fastest, the query heads of a kv head share an L2
+  const int G = a.heads / a.kv_heads, g = blockIdx.y % a.kv_heads, h = g * G + blockIdx.y / a.kv_heads;
+  const int t = blockIdx.x, lane = threadIdx.x & 63, sub = lane >> 4, ln = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = (a.pos_dev ? *a.pos_dev : a.start_pos) + t;
+  const int qhs = a.q_hstride > 0 ? a.q_hstride : D, khs = a.k_hstride > 0 ? a.k_hstride : D;
+  const int kld = a.kld > 0 ? a.kld : a.kv_heads * khs, vld = a.vld > 0 ? a.vld : a.kv_heads * D;
+  const float* qp = a.q + (size_t)t * a.ldq + (size_t)h * qhs + 4 * ln;
+  f32x4 q[NV], o[NV];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    q[v] = *reinterpret_cast<const f32x4*>(qp + 64 * v);
+    o[v] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  const int jlo = swa_first_key(a, i), n = i - jlo + 1;
+  const int nf = a.keep_first > 0 ? (a.keep_first < jlo ? a.keep_first : jlo) : 0, pf = (nf + 63) >> 6;  // (as in swa_kernel)
+  const float hb = a.sigmoid && a.head_bias ? a.head_bias[h] : 0.0f;
+  const float r1 = a.dist_r1 ? a.dist_r1[h] : 0.0f, r2 = a.dist_r1 ? a.dist_r2[h] : 0.0f;
+  const int pieces = pf + ((n + 63) >> 6);
+  // no more splits than a piece a wave fills: 256 keys need no records and no last arrival (the launch is sized for the whole window)
+  int nsplit = a.nsplit > 1 ? a.nsplit : 1;
+  if (a.done_cnt && nsplit > (pieces + W - 1) / W) nsplit = (pieces + W - 1) / W;
+  if ((int)blockIdx.z >= nsplit) return;
+  const int per = (pieces + nsplit - 1) / nsplit;
+  const int c_lo = blockIdx.z * per, c_hi = c_lo + per < pieces ? c_lo + per : pieces;
+  const float* kb = a.kc + (size_t)g * khs + 4 * ln;
+  const float* vb = a.vc + (size_t)g * D + 4 * ln;
+  float m = -INFINITY, l = 0.0f;
+  for (int c = c_lo + wave; c < c_hi; c += W) {
+    const int jend = c < pf ? nf - 1 : i;
+    for (int j0 = c < pf ? c * 64 : jlo + (c - pf) * 64, part = 0; part < NV && j0 <= jend; ++part, j0 += 4 * U) {
+      f32x4 kk[U][NV], vv[U][NV];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int j = j0 + 4 * u + sub, jc = j <= jend ? j : jend;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) kk[u][v] = *reinterpret_cast<const f32x4*>(kb + (size_t)jc * kld + 64 * v);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int j = j0 + 4 * u + sub, jc = j <= jend ? j : jend;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) vv[u][v] = *reinterpret_cast<const f32x4*>(vb + (size_t)jc * vld + 64 * v);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // (all of them asked for before the first product)
+      float s[U], mx = -INFINITY;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int j = j0 + 4 * u + sub;
+        float d = 0.0f;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) d += (q[v][0] * kk[u][v][0] + q[v][1] * kk[u][v][1]) + (q[v][2] * kk[u][v][2] + q[v][3] * kk[u][v][3]);
+        d = swa_sum16(d) * a.scale;
+        if (a.softcap > 0.0f) d = swa_cap(d, a.softcap, 1.0f / a.softcap);
+        if (a.dist_r1) d -= swa_dist(r1, r2, i - j);
+        s[u] = j <= jend ? d : -INFINITY;
+        mx = fmaxf(mx, s[u]);
+      }
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      const float mn = a.sigmoid ? 0.0f : fmaxf(m, mx);  // finite: the first key of a piece is a visible one
+      const float corr = expf(m - mn);                   // m = -inf at the first piece: 0
+      m = mn;
+      l *= corr;
+#pragma unroll
+      for (int v = 0; v < NV; ++v) o[v] *= corr;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float p = j0 + 4 * u + sub > jend ? 0.0f : a.sigmoid ? 1.0f / (1.0f + expf(-(s[u] + hb))) : expf(s[u] - mn);
+        l += p;
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[v][e] = fmaf(p, vv[u][v][e], o[v][e]);
+      }
+    }
+  }
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+  if (lane == 0) {
+    ml[wave * 2] = m;
+    ml[wave * 2 + 1] = l;
+  }
+#pragma unroll
+  for (int v = 0; v < NV; ++v) *reinterpret_cast<f32x4*>(ow + (wave * 4 + sub) * D + 64 * v + 4 * ln) = o[v];
+  swa_finish<4, W>(a, ml, ow, nsplit, t, h);
+}
+// rows of 64 or 128 numbers for keys and values alike, rows and heads at 16 bytes
+bool swa_rows_fit(const SwaArgs& a) {
+  return a.dim == a.vdim && (a.dim == 64 || a.dim == 128) && ((a.ldq | a.q_hstride | a.k_hstride | a.kld | a.vld) & 3) == 0 &&
+         (((size_t)a.q | (size_t)a.kc | (size_t)a.vc) & 15) == 0;
+}
+
+__global__ __launch_bounds__(64) void swa_combine_kernel(const SwaArgs a) { swa_merge_records(a, a.nsplit, blockIdx.x, blockIdx.y, threadIdx.x); }
 
 // ---- few tokens, many query heads over ONE head of keys whose rows are the values as well (a latent cache) ------------------
 // All heads read the same rows, so a workgroup takes a tile of 32 keys for 32 heads at once: the rows go into LDS once, and both
@@ -816,7 +951,10 @@ int tl_launch_swa(const SwaArgs& a, hipStream_t s) {
   const int nsplit = a.nsplit > 1 ? a.nsplit : 1;
   TL_REQUIRE(nsplit == 1 || a.ws, "swa: split launch without a workspace");
   TL_REQUIRE(nsplit <= 64, "swa: %d splits", nsplit);
-  swa_kernel<<<dim3(a.T, a.heads, nsplit), 256, lds, s>>>(a);
+  const dim3 grid(a.T, a.heads, nsplit);
+  if (!swa_rows_fit(a)) swa_kernel<<<grid, 256, lds, s>>>(a);
+  else if (a.dim == 64) swa_rows_kernel<1><<<grid, 256, 0, s>>>(a);
+  else swa_rows_kernel<2><<<grid, 256, 0, s>>>(a);
   if (nsplit > 1 && !a.done_cnt) swa_combine_kernel<<<dim3(a.T, a.heads), 64, 0, s>>>(a);
   TL_HIP(hipGetLastError());
   return 0;
