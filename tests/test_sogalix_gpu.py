@@ -629,3 +629,36 @@ def test_configurations_drawn_at_random(env, seed, tmp_path):
         got += [s.forward(toks[i:i + 1], i, [0]) for i in range(p, n)]
         assert rel_rms(np.concatenate(got), want) < FP32_TOL, json.dumps(cfg)
     s.close()
+
+
+@pytest.mark.parametrize("heads,dim", [(3, 64), (2, 128)])
+def test_generalized_delta_rule_of_aligned_rows(env, heads, dim):
+    """Rows at 16 bytes take the unrolled scan: portions below, at and above its stages of 16 and 8 tokens, against the recurrence
+    in 64 bits (a few 32-bit roundings a token, decayed by w >= 0.54: some 1e-6 of the outputs' size)."""
+    capi, orc = env["capi"], env["oracle"]
+    rng = np.random.default_rng(dim + 1)
+    portions = (1, 7, 8, 9, 15, 16, 17, 64, 2, 33)
+    n, hd = sum(portions), heads * dim
+    ld, scale = 5 * hd + 4, math.exp(-0.5)
+    p = rng.standard_normal((n, ld)).astype(np.float32)
+    dw = (2.0 * rng.standard_normal((n, hd))).astype(np.float32)
+    w0, ab = rng.standard_normal(hd).astype(np.float32), rng.standard_normal(hd).astype(np.float32)
+    r, k, v = (p[:, i * hd:(i + 1) * hd].astype(np.float64).reshape(n, heads, dim) for i in range(3))
+    a = orc.sigmoid(p[:, 4 * hd:5 * hd].astype(np.float64) + ab).reshape(n, heads, dim)
+    w = np.exp(-scale * orc.sigmoid(dw.astype(np.float64) + w0)).reshape(n, heads, dim)
+    S = np.zeros((heads, dim, dim))
+    want = np.stack([orc.generalized_delta(r[:, h], k[:, h], v[:, h], w[:, h], a[:, h], S[h]) for h in range(heads)], 1)
+    sd, w0d, abd = dev(env, np.zeros((heads, dim, dim), np.float32)), dev(env, w0), dev(env, ab)
+    got, t0 = [], 0
+    for T in portions:
+        pd, dwd = dev(env, p[t0:t0 + T]), dev(env, dw[t0:t0 + T])
+        od = env["engine"].DeviceBuffer(4 * T * hd)
+        scratch = env["engine"].DeviceBuffer(4 * (3 * T * hd + 2 * T * heads))
+        capi.check(capi.lib().tl_general_delta(pd.ptr, ld, dwd.ptr, w0d.ptr, abd.ptr, scale, sd.ptr, od.ptr, scratch.ptr, T, heads,
+                                               dim, None), "tl_general_delta")
+        sync(env)
+        got.append(od.to_numpy(np.float32, (T, heads, dim)))
+        t0 += T
+    err = np.linalg.norm(np.concatenate(got) - want) / np.linalg.norm(want)
+    state = np.linalg.norm(sd.to_numpy(np.float32, (heads, dim, dim)) - S.transpose(0, 2, 1)) / np.linalg.norm(S)
+    assert err < 4e-6 and state < 4e-6, (err, state)
