@@ -312,3 +312,21 @@ def test_packed_attention_by_row_tiles(pkg, monkeypatch, heads, kv_heads, hd):
                 assert not np.array_equal(logits, want[k])  # (the other kernel ran)
                 assert np.linalg.norm(logits - want[k]) <= 4e-6 * np.linalg.norm(want[k])
     m.free()
+
+
+def test_many_logits_reach_the_caller(pkg):
+    """Logits of 4 MB and more come through four threads' stripes: every row where it belongs, whole pages and not, one buffer after
+    another. Against steps of a few sequences (the runtime's own copy): the same products in another order of sums."""
+    from tinyllama_cpp_amd import engine as E
+    E.init(0)
+    cfg, tensors = pkg.synth.build_model(dict(pkg.synth.SHAPES["tiny-gqa"], vocab=50003, n_layers=1), "q4_k_m", seed=6)
+    m = E.Model(cfg).load(tensors)
+    m.batch_init(101)
+    toks = np.random.default_rng(1).integers(0, cfg["vocab"], 101).astype(np.int32)
+    at = lambda lo, hi: m.batch_decode(toks[lo:hi], np.zeros(hi - lo, np.int32), np.arange(lo, hi))
+    want = np.concatenate([at(lo, min(lo + 15, 101))[0] for lo in range(0, 101, 15)])
+    for n in (20, 21, 22, 50, 101):
+        logits, ids = at(0, n)
+        assert np.linalg.norm(logits - want[:n]) <= 4e-6 * np.linalg.norm(want[:n]) and np.array_equal(ids, logits.argmax(1)), n
+        assert np.abs(logits - want[:n]).max() <= 1e-4 * np.abs(want).max(), n
+    m.free()

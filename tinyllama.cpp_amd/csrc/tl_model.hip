@@ -15,6 +15,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <thread>
 #include <vector>
 
 #include <rccl/rccl.h>
@@ -131,6 +132,8 @@ struct tl_model {
     float* last_h = nullptr;                              // [max_batch][hidden]: hidden rows whose logits a packed prefill returns
     int* ids = nullptr;                                   // generated ids [step][n]
     size_t ids_cap = 0;
+    unsigned char* stage = nullptr;  // pinned, kCopyThreads x 2 pieces: many logits on their way to the caller (copy_to_caller)
+    hipEvent_t staged[8] = {};
     int gemv_max = 0;  // steps with at most this many sequences take the multi-vector GEMV route (0: never)
   } bt;
   // Chain launches (tl_gemv.hip): the step's GEMVs between two attention launches -- attn_output, gate/up, ffn_down and the
@@ -229,6 +232,13 @@ extern "C" int tl_model_create(const tl_model_config* cfg, tl_model** out) {
   return 0;
 }
 
+static void batch_unstage(tl_model::Batch& b) {
+  if (!b.stage) return;
+  hipHostFree(b.stage);
+  for (hipEvent_t e : b.staged)
+    if (e) hipEventDestroy(e);
+  b.stage = nullptr;
+}
 extern "C" int tl_model_free(tl_model* m) {
   if (!m) return 0;
   if (m->stream) hipStreamSynchronize(m->stream);
@@ -272,6 +282,7 @@ extern "C" int tl_model_free(tl_model* m) {
   hipFree(m->bt.ids);
   hipFree(m->bt.last_h);
   hipFree(m->bt.pack);
+  batch_unstage(m->bt);
   if (m->pf.fork) hipEventDestroy(m->pf.fork);
   if (m->pf.join) hipEventDestroy(m->pf.join);
   if (m->pf.side) hipStreamDestroy(m->pf.side);
@@ -1297,6 +1308,8 @@ extern "C" int tl_model_generate_sampled(tl_model* m, int first_token, int start
 // more would only grow the workspaces). The bf16 routes and tensor-parallel shards keep the 512 that they were tuned at, which
 // is also the most sequences of a step and the most logits rows of a chunk.
 constexpr int kPrefillChunk = 2048, kChunkRows = 512;
+constexpr int kCopyThreads = 4;  // copy_to_caller
+constexpr size_t kCopyPiece = (size_t)2 << 20, kCopySpread = (size_t)4 << 20;
 
 __global__ void set_token_kernel(int* state, const int* tokens, int i) { state[0] = tokens[i]; }
 
@@ -1880,16 +1893,62 @@ static int batch_head(tl_model* m, const float* hidden, int R, hipStream_t s) {
   return tl_launch_gemm_q(qw_view(m->out), p.planes, p.plane_stride, p.logits_all, nullptr, R, terms, s);
 }
 
+// Many logits to the caller's memory, behind what the stream holds. The runtime takes pageable memory through one thread's copies (and its
+// page faults): 128 rows of 128256 (66 MB) 6.2 ms, here 1.9; 64 rows 1.8 and 0.9, 16 rows 0.47 and 0.31, 8 rows level. Four threads take a stripe each through two pinned pieces, one on its way from the
+// device while the other is copied out. Up to kCopySpread bytes: the runtime's own copy, complete when the stream is waited for.
+static int copy_to_caller(tl_model* m, float* dst, const float* src, size_t bytes, hipStream_t s) {
+  tl_model::Batch& b = m->bt;
+  if (!b.stage || bytes < kCopySpread) {
+    TL_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
+    return 0;
+  }
+  int device = 0;
+  TL_HIP(hipGetDevice(&device));
+  hipError_t err[kCopyThreads] = {};
+  auto stripe = [&](int t) {
+    const size_t pages = (bytes + 4095) / 4096, lo = pages * t / kCopyThreads * 4096;
+    const size_t end = std::min(bytes, pages * (t + 1) / kCopyThreads * 4096), n = (end - lo + kCopyPiece - 1) / kCopyPiece;
+    unsigned char* pin = b.stage + (size_t)t * 2 * kCopyPiece;
+    hipError_t e = hipSetDevice(device);
+    for (size_t k = 0; k <= n && e == hipSuccess; ++k) {
+      if (k < n) {
+        const size_t at = lo + k * kCopyPiece, len = std::min(kCopyPiece, end - at);
+        e = hipMemcpyAsync(pin + (k & 1) * kCopyPiece, reinterpret_cast<const unsigned char*>(src) + at, len, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipEventRecord(b.staged[2 * t + (k & 1)], s);
+      }
+      if (k > 0 && e == hipSuccess) {
+        const size_t at = lo + (k - 1) * kCopyPiece, len = std::min(kCopyPiece, end - at);
+        e = hipEventSynchronize(b.staged[2 * t + ((k - 1) & 1)]);
+        if (e == hipSuccess) memcpy(reinterpret_cast<unsigned char*>(dst) + at, pin + ((k - 1) & 1) * kCopyPiece, len);
+      }
+    }
+    err[t] = e;
+  };
+  std::thread others[kCopyThreads];
+  bool here[kCopyThreads] = {true};
+  for (int t = 1; t < kCopyThreads; ++t) {
+    try {
+      others[t] = std::thread(stripe, t);
+    } catch (...) {  // (no thread to be had)
+      here[t] = true;
+    }
+  }
+  for (int t = 0; t < kCopyThreads; ++t)
+    if (here[t]) stripe(t);
+  for (std::thread& t : others)
+    if (t.joinable()) t.join();
+  for (hipError_t e : err) TL_HIP(e);
+  return 0;
+}
+
 static int batch_step(tl_model* m, int T, int* ids_dev, bool advance, float* logits_host) {
   const tl_model_config& c = m->cfg;
   tl_model::Prefill& p = m->pf;
   hipStream_t s = m->stream;
   TL_TRY(batch_layers(m, T, s));
   TL_TRY(batch_head(m, p.xb, T, s));
-  if (logits_host)
-    TL_HIP(hipMemcpyAsync(logits_host, p.logits_all, sizeof(float) * (size_t)T * c.vocab_size, hipMemcpyDeviceToHost, s));
-  return tl_launch_batch_argmax_advance(p.logits_all, T, c.vocab_size, advance ? m->bt.toks : nullptr,
-                                        advance ? m->bt.pos : nullptr, ids_dev, s);
+  TL_TRY(tl_launch_batch_argmax_advance(p.logits_all, T, c.vocab_size, advance ? m->bt.toks : nullptr, advance ? m->bt.pos : nullptr, ids_dev, s));
+  return logits_host ? copy_to_caller(m, logits_host, p.logits_all, sizeof(float) * (size_t)T * c.vocab_size, s) : 0;
 }
 
 extern "C" int tl_model_batch_init(tl_model* m, int max_batch) {
@@ -1914,6 +1973,7 @@ extern "C" int tl_model_batch_init(tl_model* m, int max_batch) {
     TL_HIP(hipFree(b.seq));
     TL_HIP(hipFree(b.last_h));
     TL_HIP(hipFree(b.pack));
+    batch_unstage(b);
     if (b.ids) TL_HIP(hipFree(b.ids));
     b = tl_model::Batch();
   }
@@ -1925,6 +1985,10 @@ extern "C" int tl_model_batch_init(tl_model* m, int max_batch) {
   TL_HIP(hipMalloc(&b.seq, sizeof(int) * kPrefillChunk));
   TL_HIP(hipMalloc(&b.pack, (sizeof(TlHattnTile) + sizeof(TlHattnItem)) * TL_HATTN_PACK_MAX));
   TL_HIP(hipMalloc(&b.last_h, sizeof(float) * (size_t)max_batch * m->cfg.hidden_size));
+  if (sizeof(float) * (size_t)max_batch * m->cfg.vocab_size >= kCopySpread) {
+    TL_HIP(hipHostMalloc(reinterpret_cast<void**>(&b.stage), 2 * kCopyThreads * kCopyPiece, hipHostMallocDefault));
+    for (hipEvent_t& e : b.staged) TL_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  }
   b.max_batch = max_batch;
   b.gemv_max = batch_gemv_ok(m) ? 4 : 0;  // one pass of up to four vectors: 2.5 / 4.0 / 4.1 ms per step for 2 / 3 / 4 sequences; the
                                           // direct small-token GEMM route costs 5.3 ms whatever the count (two GEMV passes: 6.1 - 7.8)
@@ -2033,10 +2097,8 @@ extern "C" int tl_model_batch_prefill_packed(tl_model* m, int n_tokens, const in
   if (n_last > 0) {
     TL_TRY(batch_ids(m, (size_t)n_last));
     TL_TRY(batch_head(m, m->bt.last_h, n_last, s));
-    if (last_logits_host)
-      TL_HIP(hipMemcpyAsync(last_logits_host, m->pf.logits_all, sizeof(float) * (size_t)n_last * c.vocab_size,
-                            hipMemcpyDeviceToHost, s));
     TL_TRY(tl_launch_batch_argmax_advance(m->pf.logits_all, n_last, c.vocab_size, nullptr, nullptr, m->bt.ids, s));
+    if (last_logits_host) TL_TRY(copy_to_caller(m, last_logits_host, m->pf.logits_all, sizeof(float) * (size_t)n_last * c.vocab_size, s));
     if (last_ids_host)
       TL_HIP(hipMemcpyAsync(last_ids_host, m->bt.ids, sizeof(int) * n_last, hipMemcpyDeviceToHost, s));
   }
