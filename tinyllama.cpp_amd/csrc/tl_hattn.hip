@@ -190,6 +190,13 @@ __device__ __forceinline__ float finish(const TlHattn& x, int t, int head, float
   return x.gate ? f / (1.0f + expf(-x.gate[(size_t)t * x.gate_ld + head])) : f;
 }
 
+// 16 bytes a lane from base + off to LDS bytes at .. at + 1023 (at, base: the same in all lanes). M0 belongs to the compiler: saved and
+// restored in the same statement
+__device__ __forceinline__ void lds_load16(unsigned at, unsigned off, const void* base) {
+  unsigned keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep) : "s"(at), "v"(off), "s"(base) : "memory");
+}
 // PACKED: a row tile's sequence, tokens and key tiles come from a list, the one with the most keys first (one piece each)
 template <int KD, int VD, bool PACKED>
 __global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs arg) {
@@ -223,18 +230,18 @@ __global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs arg) {
   const int lo_first = first_key(a.x, wave_first), lo_last = first_key(a.x, wave_last);
   const u32x4* src = reinterpret_cast<const u32x4*>(a.planes + ((long long)kvh * a.tiles - a.tile0) * TILE);
   const int2* ex = reinterpret_cast<const int2*>(a.exps) + ((long long)kvh * a.tiles - a.tile0);
-  u32x4 stage[NLD];
+  // a tile goes straight into the window (32 registers fewer than through them, which is what keeps heads of 128 from spilling)
+  const int first = __builtin_amdgcn_readfirstlane(wave * 64);
+  const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) _Float16*)&win[0][0];
   int2 stage_ex;
-  auto load = [&](int t) __attribute__((always_inline)) {
+  auto load = [&](int t, int buf) __attribute__((always_inline)) {
     stage_ex = ex[t];
 #pragma unroll
-    for (int i = 0; i < NLD; ++i) stage[i] = src[(size_t)t * (TILE / 8) + i * 256 + tid];
+    for (int i = 0; i < NLD; ++i)
+      lds_load16(lds0 + (unsigned)(buf * TILE * 2 + (i * 256 + first) * 16), lane * 16, src + (size_t)t * (TILE / 8) + i * 256 + first);
   };
-  auto store = [&](int buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < NLD; ++i) *reinterpret_cast<u32x4*>(&win[buf][(i * 256 + tid) * 8]) = stage[i];
-  };
-  load(t0);
+  auto arrived = [] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };  // of this wave's pieces; the barrier behind it: of all
+  load(t0, 0);
   const float* qp = a.x.q + (size_t)rq * a.x.ldq + (size_t)head * a.x.qhs + 8 * h;
   half8 qh[DS], ql[DS];
   float cq;
@@ -267,12 +274,12 @@ __global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs arg) {
   // probabilities would lose more than HA_P_SPARE bits: a tile with one huge row does not coarsen the tiles behind it. low: the
   // smallest exponent so far, o is below 2^(27 + krun - low) times the weights' sum, hence krun <= low + 60
   int krun = 60, low = 60;
-  store(0);
+  arrived();
   int ek = __builtin_amdgcn_readfirstlane(stage_ex.x), ev = __builtin_amdgcn_readfirstlane(stage_ex.y);
   __syncthreads();
   for (int t = t0; t < t1; ++t) {
     const int buf = (t - t0) & 1, p0 = t * 32;
-    load(t + 1 < t1 ? t + 1 : t);  // (the last one is not stored for anybody)
+    if (t + 1 < t1) load(t + 1, buf ^ 1);  // (last read a tile ago, in front of the barrier below)
     __builtin_amdgcn_sched_barrier(0);
     if (p0 <= wave_last && p0 + 31 >= lo_first) {
       const half8* kf = reinterpret_cast<const half8*>(&win[buf][0]) + lane;
@@ -380,7 +387,7 @@ __global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs arg) {
       __builtin_amdgcn_sched_group_barrier(0x8, 6, 1);
     }
     __builtin_amdgcn_sched_barrier(0);
-    store(buf ^ 1);  // (last read a tile ago, in front of the barrier below)
+    arrived();
     ek = __builtin_amdgcn_readfirstlane(stage_ex.x);
     ev = __builtin_amdgcn_readfirstlane(stage_ex.y);
     __syncthreads();
