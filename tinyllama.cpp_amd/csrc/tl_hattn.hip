@@ -10,9 +10,11 @@
 //      lanes of a matrix instruction take them (K: eight columns of one key; V: eight keys of one column, the keys in the
 //      order in which the accumulator of K Q^T holds them, so that the probabilities never change lanes). One power of two
 //      per tile brings its largest finite value to 2^14: a value is held to 2^-23 of itself and 2^-39 of its tile's largest.
-//      Against float64 the output's error is 5e-8 of its weights times its values' size, the FP32 kernel's 7e-8 (both sides
+//      Against float64 the output's error is at most 5e-8 of its weights times its values' size, the FP32 kernel's 7e-8 (both sides
 //      lose what the order of the sums gives); a row of a tile that is 2^20 times the others' size brings it to 1e-7, 2^24 to
 //      1.3e-6.
+//      The sums of a tile and of the small products are kept apart, and the weights' 2^12 stands outside the exponential: packed
+//      prompts' logits are as far from float64 as with the per-token FP32 kernel (20 batches: within 1 %; before, 2 to 5 % further).
 //   2. hattn_kernel: four waves, 128 rows (query, head of the kv head's group), tiles through a double-buffered LDS window
 //      that all four waves read: one wave's operands straight from memory would need 85 bytes a cycle and CU. Two workgroups
 //      a CU, so that one's softmax runs under the other's products. A row tile's keys are cut into up to 16 pieces.
