@@ -545,3 +545,22 @@ def test_prefill_chunks_of_2048(E, pkg, T):
     for got in (last, packed):
         assert np.linalg.norm(got - rows[-1]) <= 4e-6 * np.linalg.norm(rows[-1])
     m.free()
+
+
+@pytest.mark.parametrize("heads,kv,hd", [(3, 1, 64), (8, 8, 32), (2, 2, 128), (9, 3, 64)])
+def test_prompt_rotation_and_cache_rows(E, pkg, heads, kv, hd):
+    """A prompt in two portions (q, k and v below, at and above a block of the rotation kernel, positions from the second portion's
+    start on), then decoding over its cache rows, against the same tokens decoded one by one: 32-bit rounding on both sides, the
+    decode tests' tolerance."""
+    cfg = dict(hidden=heads * hd if heads * hd % 64 == 0 else 64, inter=512, n_heads=heads, n_kv_heads=kv, n_layers=2, vocab=96, max_pos=64,
+               eps=1e-5, rope_theta=10000.0)
+    cfg, tensors = pkg.synth.build_model(cfg, "q8_0", seed=heads)
+    m = E.Model(cfg).load(tensors)
+    toks = np.random.default_rng(heads).integers(0, 96, 40).astype(np.int32)
+    want = [np.array(m.decode(int(t), i)[0], np.float64) for i, t in enumerate(toks)]
+    m.reset_kv()
+    got = {16: np.array(m.prefill(toks[:17], 0)), 36: np.array(m.prefill(toks[17:37], 17))}
+    got.update({i: np.array(m.decode(int(toks[i]), i)[0]) for i in (37, 38, 39)})
+    for i, g in got.items():
+        assert (np.abs(g - want[i]) <= 1e-4 * np.maximum(1.0, np.abs(want[i]))).all(), (i, np.abs(g - want[i]).max())
+    m.free()
