@@ -221,10 +221,13 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
   const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
   const int v = xcd * per8 + (xcd < rem8 ? xcd : rem8) + at;
   const int slice = v / (mtiles * ntiles), in_slice = v - slice * mtiles * ntiles;
-  const int panel = in_slice / (PANEL * mtiles), in_panel = in_slice - panel * PANEL * mtiles;
-  const int width = ntiles - PANEL * panel < PANEL ? ntiles - PANEL * panel : PANEL;
-  const int nt = PANEL * panel + in_panel % width;
-  int mt = in_panel / width;
+  int nt = 0, mt = in_slice;
+  if (ntiles > 1) {  // (one tile of tokens: launches of 6 us, which need none of these divisions)
+    const int panel = in_slice / (PANEL * mtiles), in_panel = in_slice - panel * PANEL * mtiles;
+    const int width = ntiles - PANEL * panel < PANEL ? ntiles - PANEL * panel : PANEL;
+    mt = in_panel / width;
+    nt = PANEL * panel + in_panel - mt * width;
+  }
   const int seg = (mt >= segs.mt_end[0]) + (mt >= segs.mt_end[1]);
   if (seg) mt -= segs.mt_end[seg - 1];
   const QW w = segs.w[seg];
