@@ -237,6 +237,7 @@ static void batch_unstage(tl_model::Batch& b) {
   hipHostFree(b.stage);
   for (hipEvent_t e : b.staged)
     if (e) hipEventDestroy(e);
+  std::fill(std::begin(b.staged), std::end(b.staged), nullptr);
   b.stage = nullptr;
 }
 extern "C" int tl_model_free(tl_model* m) {
@@ -1986,8 +1987,14 @@ extern "C" int tl_model_batch_init(tl_model* m, int max_batch) {
   TL_HIP(hipMalloc(&b.pack, (sizeof(TlHattnTile) + sizeof(TlHattnItem)) * TL_HATTN_PACK_MAX));
   TL_HIP(hipMalloc(&b.last_h, sizeof(float) * (size_t)max_batch * m->cfg.hidden_size));
   if (sizeof(float) * (size_t)max_batch * m->cfg.vocab_size >= kCopySpread) {
-    TL_HIP(hipHostMalloc(reinterpret_cast<void**>(&b.stage), 2 * kCopyThreads * kCopyPiece, hipHostMallocDefault));
-    for (hipEvent_t& e : b.staged) TL_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&b.stage), 2 * kCopyThreads * kCopyPiece, hipHostMallocDefault);
+    if (e != hipSuccess) b.stage = nullptr;
+    for (hipEvent_t& ev : b.staged)
+      if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    if (e != hipSuccess) {  // (no pinned memory to be had: the runtime's own copies)
+      batch_unstage(b);
+      (void)hipGetLastError();
+    }
   }
   b.max_batch = max_batch;
   b.gemv_max = batch_gemv_ok(m) ? 4 : 0;  // one pass of up to four vectors: 2.5 / 4.0 / 4.1 ms per step for 2 / 3 / 4 sequences; the
