@@ -53,7 +53,8 @@ int tl_debug_half_gemm(const tl_qweight* w, const float* x_dev, float* y_dev, in
 
 /* Test hook (no counterpart in the reference): tl_dense_matmul's product with one term through the kernel that takes the items from a
  * bf16 plane (tl_dense.hip): rows ldx floats apart, whole steps of 64 columns, the first `exact_items` (at most 32) items with two
- * terms, `waves` 4 (two workgroups a CU) or 8 (one), plane_dev room for [num_tokens + 32][cols] bf16. */
+ * terms, `waves` 4 (two workgroups a CU) or 8 (one), plane_dev room for [num_tokens + 32][cols] bf16 (NULL: the kernel that converts
+ * them itself, in the tile of TL_DENSE_TILE, whose order of sums the first items have in either). */
 int tl_debug_dense_plane(const void* w_bf16_dev, int rows, int cols, const float* x_dev, int ldx, float* y_dev, int num_tokens,
                          int exact_items, int waves, void* plane_dev, void* stream);
 

@@ -440,6 +440,31 @@ def test_first_token_of_a_long_prompt_keeps_more_bits_in_bf16_mode(env):
     loose.free()
 
 
+def test_wide_model_through_the_large_products(env, monkeypatch):
+    """2048 wide, 1100 tokens in bf16 mode: the products of both layers take the kernel that reads its items from a bf16 plane, which
+    every product of the model writes in turn. With the first token's second terms every row against the float64 oracle; without them
+    (either tile gives the same bits) the rows of the kernel that converts its items itself, to the bit."""
+    K, C, D, L = env["synth"].ratuzen_chunked, env["synth"].ratuzen_causal, env["synth"].ratuzen_delta, env["synth"].ratuzen_layer
+    cfg = env["synth"].ratuzen_config(2048, 300, [L("parallel_2", C(16, 4, 64, 64, 16, 64, 64), 4096), L("delta", D(16, 4, 64, 64), 4096),
+                                                  L("parallel", K(16, 4, 64, 64, 300, 16, 64, 64, np.linspace(0.9, 0.99, 16)), 4096)])
+    m, tensors, orc = make(env, cfg, seed=21, max_pos=1100, exact=False)
+    toks = np.random.default_rng(7).integers(0, cfg["vocab"], 1100).astype(np.int32)
+    got, want = f64(m.prefill_rows(toks, 0)), orc.forward(list(toks))
+    err = np.sqrt(((got - want) ** 2).mean(-1)) / np.sqrt((want * want).mean())
+    assert err.max() < BF16_TOL, (err[:33], err.max())  # (1.3e-2 seen; stale second terms: 0.9 in rows 1 to 31)
+    monkeypatch.setenv("TL_DENSE_TILE", "128")
+    m.reset_kv()
+    assert not np.array_equal(got, m.prefill_rows(toks, 0))  # (the other kernel ran: its order of the second terms is one tile's)
+    m.free()
+    monkeypatch.delenv("TL_DENSE_TILE")
+    loose, _, _ = make(env, cfg, tensors=tensors, max_pos=1100, exact=False, TL_STACK_EXACT_FIRST=0)
+    plane = loose.prefill_rows(toks, 0)
+    monkeypatch.setenv("TL_DENSE_TILE", "128")
+    loose.reset_kv()
+    assert np.array_equal(plane, loose.prefill_rows(toks, 0))
+    loose.free()
+
+
 @pytest.mark.parametrize("variant", VARIANTS)
 def test_prompt_against_token_by_token_decoding(env, variant):
     """The whole prompt in one pass, and the same tokens one by one through the captured decode step (from the very first

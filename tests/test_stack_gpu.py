@@ -526,11 +526,12 @@ def test_dense_gemm_tiles_give_the_same_bits(pkg, monkeypatch, rows, cols, T, te
 
 @pytest.mark.parametrize("rows,cols,T,ld", [(1, 64, 1, 64), (257, 192, 129, 200), (130, 1088, 1050, 1088), (128, 128, 31, 132), (900, 64, 33, 64)])
 @pytest.mark.parametrize("waves", [4, 8])
-@pytest.mark.parametrize("exact", [0, 32])
+@pytest.mark.parametrize("exact", [0, 1, 5, 31, 32])
 def test_dense_plane_gemm_gives_the_same_bits(pkg, monkeypatch, rows, cols, T, ld, waves, exact):
     """The kernel that takes its items from a bf16 plane against the one that converts them itself: tiles with one row and one token
-    more, fewer steps than it fetches ahead, item tiles beyond a panel of eight, rows apart. One term: the same sums in the same order.
-    The first items' second terms are added in another place: float64 bounds them (16 of 24 bits are kept: 2^-16 of each product)."""
+    more, fewer steps than it fetches ahead, item tiles beyond a panel of eight, rows apart, a plane that holds NaN before. The same
+    sums in the same order, also where the first items have two terms (as the tile that is chosen has them). Against float64: with two
+    terms 16 of 24 bits are kept (2^-16 of each product), for all of the first 32 items."""
     from tinyllama_cpp_amd import capi, engine, synth
     engine.init(0)
     rng = np.random.default_rng(rows + cols + T + waves)
@@ -538,16 +539,23 @@ def test_dense_plane_gemm_gives_the_same_bits(pkg, monkeypatch, rows, cols, T, l
     x = np.full((T, ld), np.nan, np.float32)
     x[:, :cols] = rng.standard_normal((T, cols))
     dev = engine.DeviceBuffer.from_numpy
-    wd, xd, xc, yd, zd = dev(w), dev(x), dev(np.ascontiguousarray(x[:, :cols])), engine.DeviceBuffer(4 * T * rows), engine.DeviceBuffer(4 * T * rows)
+    wd, xd, yd = dev(w), dev(x), engine.DeviceBuffer(4 * T * rows)
     plane = engine.DeviceBuffer(2 * (T + 32) * cols)
-    capi.check(capi.lib().tl_memset(yd.ptr, 0xff, yd.nbytes, None))
-    capi.check(capi.lib().tl_debug_dense_plane(wd.ptr, rows, cols, xd.ptr, ld, yd.ptr, T, exact, waves, plane.ptr, None), "tl_debug_dense_plane")
-    capi.check(capi.lib().tl_dense_matmul(wd.ptr, rows, cols, xc.ptr, zd.ptr, T, 1, None), "tl_dense_matmul")
-    capi.check(capi.lib().tl_device_sync(), "sync")
-    got, want = yd.to_numpy(np.float32, (T, rows)), zd.to_numpy(np.float32, (T, rows))
-    assert np.array_equal(got[exact:], want[exact:])
-    X, W = x[:exact, :cols].astype(np.float64), synth.from_bf16(w).astype(np.float64)
-    assert (np.abs(got[:exact] - X @ W.T) <= (2.0 ** -16 + (cols + 4) * 2.0 ** -24) * (np.abs(X) @ np.abs(W).T)).all()
+
+    def run(at):
+        capi.check(capi.lib().tl_memset(yd.ptr, 0xff, yd.nbytes, None))
+        capi.check(capi.lib().tl_memset(plane.ptr, 0xff, plane.nbytes, None))
+        capi.check(capi.lib().tl_debug_dense_plane(wd.ptr, rows, cols, xd.ptr, ld, yd.ptr, T, exact, waves, at, None), "tl_debug_dense_plane")
+        capi.check(capi.lib().tl_device_sync(), "sync")
+        return yd.to_numpy(np.float32, (T, rows))
+
+    X, W = x[:32, :cols].astype(np.float64), synth.from_bf16(w).astype(np.float64)
+    for tile in ("64", "128"):
+        monkeypatch.setenv("TL_DENSE_TILE", tile)
+        got = run(plane.ptr)
+        if exact:
+            assert (np.abs(got[:32] - X @ W.T) <= (2.0 ** -16 + (cols + 4) * 2.0 ** -24) * (np.abs(X) @ np.abs(W).T)).all()
+        assert np.array_equal(got, run(None)), tile
 
 
 def test_causal_conv_output_behind_the_last_row(pkg):

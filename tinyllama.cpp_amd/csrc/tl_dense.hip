@@ -273,8 +273,10 @@ __device__ __forceinline__ void dma_wait() {
 // NWM x NWN waves, 32 WM features x 32 WN items each. Workgroups walk panels of eight item tiles, a contiguous range of tiles per XCD
 // (as in the f16 GEMM of quantized matrices). Both sides go from memory to LDS directly, NS - 1 steps ahead;
 // the loop has no other loads, so that waiting for all but the last NS - 2 steps' pieces is waiting for the step in hand.
+// FIRST: the first 32 items' second terms join after every `join` products of 16 columns, where the tile of the kernel above that this
+// launch would have taken has them: the same bits.
 template <int NWM, int NWN, int WM, int WN, int NS, bool FIRST>
-__global__ __launch_bounds__(64 * NWM * NWN, 2) void dense_plane_kernel(const DenseArgs a, int mtiles, int ntiles) {
+__global__ __launch_bounds__(64 * NWM * NWN, 2) void dense_plane_kernel(const DenseArgs a, int mtiles, int ntiles, int join) {
   constexpr int NW = NWM * NWN, BM = 32 * WM * NWM, BN = 32 * WN * NWN, ROWS = BM + BN + (FIRST ? 32 : 0), STAGE = ROWS * 128;
   constexpr int IW = BM / 8 / NW, IX = BN / 8 / NW;  // pieces of 8 rows x 64 columns that a wave fetches
   static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "");
@@ -326,6 +328,15 @@ __global__ __launch_bounds__(64 * NWM * NWN, 2) void dense_plane_kernel(const De
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
   const int fr = lane & 31, sw = (fr >> 1) & 7;
+  auto second = [&](const unsigned char* b, int from, int to) __attribute__((always_inline)) {
+    for (int ks = from; ks < to; ++ks) {
+      const int q = ((2 * ks + (lane >> 5)) ^ sw) << 4;
+      const bf16x8 x = *reinterpret_cast<const bf16x8*>(b + (BM + BN + fr) * 128 + q);
+#pragma unroll
+      for (int i = 0; i < WM; ++i)
+        acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(b + ((wm * WM + i) * 32 + fr) * 128 + q), x, acc[i][0], 0, 0, 0);
+    }
+  };
 #pragma unroll
   for (int st = 0; st < NS - 1; ++st) fetch(st, st);
   int slot = 0;
@@ -347,10 +358,9 @@ __global__ __launch_bounds__(64 * NWM * NWN, 2) void dense_plane_kernel(const De
       for (int j = 0; j < WN; ++j)
 #pragma unroll
         for (int i = 0; i < WM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i], bf[j], acc[i][j], 0, 0, 0);
-      if (FIRST && lead && wn == 0) {
-        const bf16x8 x = *reinterpret_cast<const bf16x8*>(b + (BM + BN + fr) * 128 + q);
-#pragma unroll
-        for (int i = 0; i < WM; ++i) acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i], x, acc[i][0], 0, 0, 0);
+      if (FIRST && lead && wn == 0 && (ks & 1)) {  // (behind the products that the kernel above has in a step)
+        if (join == 2) second(b, ks - 1, ks + 1);
+        else if (ks == 3) second(b, 0, 4);
       }
     }
     slot = slot == NS - 1 ? 0 : slot + 1;
@@ -359,8 +369,8 @@ __global__ __launch_bounds__(64 * NWM * NWN, 2) void dense_plane_kernel(const De
   dense_store<WM, WN>(a, acc, a.y, f0 + wm * WM * 32, t0 + wn * WN * 32, hi, lane);
 }
 
-// x[T][ldx] -> bf16 [T][cols], and behind it the second terms of the first `exact` rows; eight columns a thread
-__global__ __launch_bounds__(256) void dense_rows_kernel(const float* __restrict__ x, int ldx, int T, int cols, int exact,
+// x[T][ldx] -> bf16 [T][cols], and behind it the second terms of the first `second` rows; eight columns a thread
+__global__ __launch_bounds__(256) void dense_rows_kernel(const float* __restrict__ x, int ldx, int T, int cols, int second,
                                                          unsigned short* __restrict__ plane) {
   const long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 8;
   if (i >= (long long)T * cols) return;
@@ -374,7 +384,7 @@ __global__ __launch_bounds__(256) void dense_rows_kernel(const float* __restrict
     lo[e] = (__bf16)(f - (float)hi[e]);
   }
   *reinterpret_cast<bf16x8*>(plane + i) = hi;
-  if (t < exact) *reinterpret_cast<bf16x8*>(plane + (size_t)T * cols + i) = lo;
+  if (t < second) *reinterpret_cast<bf16x8*>(plane + (size_t)T * cols + i) = lo;
 }
 
 // RW rows per wave, 4 waves per workgroup: 2 x RW sixteen-byte weight loads in flight per lane (tl_bf16.h)
@@ -404,24 +414,25 @@ __global__ __launch_bounds__(256) void dense_gemv_kernel(const unsigned short* _
 }
 
 template <int NWM, int NWN, int WM, int WN, int NS, bool FIRST>
-int dense_plane_go(const DenseArgs& a, hipStream_t s) {
+int dense_plane_go(const DenseArgs& a, int join, hipStream_t s) {
   constexpr int BM = 32 * WM * NWM, BN = 32 * WN * NWN, LDS = NS * 128 * (BM + BN + (FIRST ? 32 : 0));
   static TlDeviceOnce lds_raised;
   auto kernel = dense_plane_kernel<NWM, NWN, WM, WN, NS, FIRST>;
   TL_TRY(tl_raise_lds_limit(kernel, LDS, lds_raised));
   const int mt = (a.rows + BM - 1) / BM, nt = (a.T + BN - 1) / BN;
-  kernel<<<mt * nt, 64 * NWM * NWN, LDS, s>>>(a, mt, nt);
+  kernel<<<mt * nt, 64 * NWM * NWN, LDS, s>>>(a, mt, nt, join);
   TL_HIP(hipGetLastError());
   return 0;
 }
 
-int dense_plane_run(const DenseArgs& a, int waves, hipStream_t s) {
-  const bool first = a.exact_items > 0;
+int dense_plane_run(const DenseArgs& a, int waves, bool big, hipStream_t s) {
+  const bool first = a.exact_items > 0;  // (the kernels multiply the second terms of 32 items whatever their number)
+  const int join = big ? 2 : 4;
   const long long pieces = (long long)a.T * a.cols / 8;
-  dense_rows_kernel<<<dim3((unsigned)((pieces + 255) / 256)), 256, 0, s>>>(a.x, a.ldx, a.T, a.cols, first ? a.exact_items : 0, a.plane);
+  dense_rows_kernel<<<dim3((unsigned)((pieces + 255) / 256)), 256, 0, s>>>(a.x, a.ldx, a.T, a.cols, first ? 32 : 0, a.plane);
   TL_HIP(hipGetLastError());
-  if (waves == 8) return first ? dense_plane_go<4, 2, 1, 2, 4, true>(a, s) : dense_plane_go<4, 2, 1, 2, 4, false>(a, s);
-  return first ? dense_plane_go<2, 2, 2, 2, 2, true>(a, s) : dense_plane_go<2, 2, 2, 2, 2, false>(a, s);
+  if (waves == 8) return first ? dense_plane_go<4, 2, 1, 2, 4, true>(a, join, s) : dense_plane_go<4, 2, 1, 2, 4, false>(a, join, s);
+  return first ? dense_plane_go<2, 2, 2, 2, 2, true>(a, join, s) : dense_plane_go<2, 2, 2, 2, 2, false>(a, join, s);
 }
 // (32-bit byte offsets inside the matrix and the plane)
 bool dense_plane_fits(const DenseArgs& a) {
@@ -470,7 +481,7 @@ int tl_launch_dense_gemm(const DenseArgs& a, hipStream_t s) {
   // (256 tiles 30.3 / 32.5 us, 324 tiles 44.8 / 36.4). TL_DENSE_TILE=64, 128: the kernel above.
   if (a.plane && a.terms == 1 && groups == 1 && !a.group_off && !a.x_rows && vec && dense_plane_fits(a) && !force &&
       2 * big_tiles >= tl_num_cus() && big_tiles * a.cols > 1024ll * tl_num_cus()) {
-    return dense_plane_run(a, big_tiles <= tl_num_cus() ? 8 : 4, s);
+    return dense_plane_run(a, big_tiles <= tl_num_cus() ? 8 : 4, big, s);
   }
   const int BM = big ? 128 : 64, BN = big ? 128 : 64;
   dim3 grid((a.rows + BM - 1) / BM, (a.T + BN - 1) / BN, groups);
@@ -631,10 +642,12 @@ extern "C" int tl_debug_dense_plane(const void* w_bf16_dev, int rows, int cols, 
   a.T = num_tokens;
   a.terms = 1;
   a.exact_items = exact_items;
-  a.plane = static_cast<uint16_t*>(plane_dev);
-  TL_REQUIRE(a.w && x_dev && y_dev && plane_dev && rows > 0 && cols > 0 && num_tokens > 0 && ldx >= cols && ldx % 4 == 0 &&
+  TL_REQUIRE(a.w && x_dev && y_dev && rows > 0 && cols > 0 && num_tokens > 0 && ldx >= cols && ldx % 4 == 0 &&
                  exact_items >= 0 && exact_items <= 32 && (waves == 4 || waves == 8) && dense_plane_fits(a) &&
                  (((size_t)w_bf16_dev | (size_t)x_dev | (size_t)plane_dev) & 15) == 0,
              "tl_debug_dense_plane: bad argument");
-  return dense_plane_run(a, waves, static_cast<hipStream_t>(stream));
+  if (!plane_dev) return tl_launch_dense_gemm(a, static_cast<hipStream_t>(stream));
+  a.plane = static_cast<uint16_t*>(plane_dev);
+  const char* tile = getenv("TL_DENSE_TILE");
+  return dense_plane_run(a, waves, tile && atoi(tile) == 128, static_cast<hipStream_t>(stream));
 }
