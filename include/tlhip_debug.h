@@ -57,6 +57,9 @@ int tl_debug_half_gemm(const tl_qweight* w, const float* x_dev, float* y_dev, in
  * them itself, in the tile of TL_DENSE_TILE, whose order of sums the first items have in either). */
 int tl_debug_dense_plane(const void* w_bf16_dev, int rows, int cols, const float* x_dev, int ldx, float* y_dev, int num_tokens,
                          int exact_items, int waves, void* plane_dev, void* stream);
+/* ... and whether a model's product of these sizes takes that kernel, with room for `room` bf16 numbers, on `cus` compute units (a rule
+ * on the host: no device) */
+int tl_debug_dense_plane_taken(int rows, int cols, int num_tokens, long long room, int cus);
 
 /* Test hook (no counterpart in the reference): tl_swa_attention's product through the two-part f16 kernels that prompt chunks
  * take (tl_hattn.hip); head sizes 64, 96 or 128 over 64 and 128 over 128, a positive scale, 16-byte addresses. */

@@ -662,3 +662,20 @@ def test_generalized_delta_rule_of_aligned_rows(env, heads, dim):
     err = np.linalg.norm(np.concatenate(got) - want) / np.linalg.norm(want)
     state = np.linalg.norm(sd.to_numpy(np.float32, (heads, dim, dim)) - S.transpose(0, 2, 1)) / np.linalg.norm(S)
     assert err < 4e-6 and state < 4e-6, (err, state)
+
+
+def test_latent_rows_beyond_a_chunk(env, monkeypatch):
+    """Chunks of 64 tokens over a latent cache of up to 2240 rows: the values of all rows that a chunk sees are one product, large enough
+    for the kernel that reads its items from a plane, and more items than the plane of a 64-token chunk holds. The same bits as with
+    the kernel that has no plane."""
+    S = env["synth"]
+    cfg = S.sogalix_config(512, 200, [S.sogalix_layer("latent_attention", S.sogalix_latent(64, 64, 32, 64, 128, 512), ff=512)])
+    toks = np.random.default_rng(3).integers(0, cfg["vocab"], 2240).astype(np.int32)
+    got, tensors = [], None
+    for tile in (None, "128"):
+        if tile:
+            monkeypatch.setenv("TL_DENSE_TILE", tile)
+        m, tensors, _ = make(env, cfg, seed=5, max_pos=2240, exact=False, tensors=tensors, TL_STACK_CHUNK=64, TL_STACK_LEAD=0)
+        got.append(m.prefill_rows(toks, 0, np.array([0, 700, 2100, 2239], np.int32)))
+        m.free()
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1])

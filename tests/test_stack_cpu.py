@@ -117,3 +117,17 @@ def test_trace_program_arguments(tmp_path):
     r = subprocess.run([exe, "--model", str(tmp_path / "nothing"), "--dtype", "float32", "--out", str(tmp_path)],
                        capture_output=True, text=True, stdin=subprocess.DEVNULL)
     assert r.returncode == 1 and "cannot open" in r.stderr
+
+
+def test_items_go_to_the_bf16_plane_only_where_they_fit(pkg):
+    """A chunk's plane holds [chunk + 32][widest input]. A latent layer also multiplies every cache row that a chunk sees, more rows than
+    a chunk has: 8 heads of 512 over a rank of 512, chunks of 2048, 4096 wide: from position 16609 on they do not fit."""
+    from tinyllama_cpp_amd import capi
+    taken, room = capi.lib().tl_debug_dense_plane_taken, (2048 + 32) * 4096
+    assert taken(4096, 512, 16608, room, 256) == 1 and (16608 + 32) * 512 == room
+    for rows_seen in (16609, 20000, 131072):
+        assert taken(4096, 512, rows_seen, room, 256) == 0
+    assert taken(4096, 4096, 2048, room, 256) == 1 and taken(4096, 4096, 2049, room, 256) == 0
+    assert taken(4096, 4096, 1024, (1024 + 32) * 4096, 256) == 1 and taken(4096, 4096, 1024, (1024 + 32) * 4096 - 1, 256) == 0
+    assert taken(4096, 4096, 1024, 0, 256) == 0
+    assert taken(4096, 4064, 1024, room, 256) == 0 and taken(1024, 1024, 1999, room, 256) == 0  # (no whole steps; too little work)

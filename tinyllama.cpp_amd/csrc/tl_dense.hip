@@ -434,9 +434,21 @@ int dense_plane_run(const DenseArgs& a, int waves, bool big, hipStream_t s) {
   if (waves == 8) return first ? dense_plane_go<4, 2, 1, 2, 4, true>(a, join, s) : dense_plane_go<4, 2, 1, 2, 4, false>(a, join, s);
   return first ? dense_plane_go<2, 2, 2, 2, 2, true>(a, join, s) : dense_plane_go<2, 2, 2, 2, 2, false>(a, join, s);
 }
-// (32-bit byte offsets inside the matrix and the plane)
+// whole steps, the items and 32 second terms inside the plane, 32-bit byte offsets in it and in the matrix
 bool dense_plane_fits(const DenseArgs& a) {
-  return a.cols % 64 == 0 && (size_t)a.rows * a.cols < ((size_t)1 << 31) && ((size_t)a.T + 32) * a.cols < ((size_t)1 << 31);
+  return a.cols % 64 == 0 && (size_t)a.rows * a.cols < ((size_t)1 << 31) && ((size_t)a.T + 32) * a.cols < ((size_t)1 << 31) &&
+         ((size_t)a.T + 32) * a.cols <= a.plane_room;
+}
+long long dense_big_tiles(int rows, long long items) { return ((rows + 127) / 128) * ((items + 127) / 128); }
+// The plane kernel takes the launches whose 128 x 128 tiles occupy half of the CUs or more and are long enough to pay for the
+// conversion (rows x columns x items, without / with it, conversion included: 10304 x 2048 x 1999 174 / 114 us, x 512 56 / 36,
+// x 200 36 / 25; 4096 x 2048 x 1999 66 / 45, x 1024 46 / 30; 2048 x 4096 x 1999 80 / 51, x 1024 47 / 43; 4096 x 1024 x 1024 26 / 20;
+// many rows and a tile of items that is half full 32000 x 2048 x 64 26.5 / 26.1, 65536 x 1024 x 64 29.7 / 27.1, 128256 x 4096 x 100
+// 290 / 240; on the line 4096 x 2048 x 512 26.3 / 25.8 and 2048 x 2048 x 1024 26.4 / 26.5; below 1024 x 1024 x 1999 16 / 18,
+// 2048 x 4096 x 512 33 / 39).
+bool dense_plane_pays(const DenseArgs& a, int cus) {
+  const long long tiles = dense_big_tiles(a.rows, a.T);
+  return dense_plane_fits(a) && 2 * tiles >= cus && tiles * a.cols > 1024ll * cus;
 }
 
 }  // namespace
@@ -465,7 +477,7 @@ int tl_launch_dense_gemm(const DenseArgs& a, hipStream_t s) {
   // grouped launches, whose small tiles are mostly half-empty, gain from large ones with one term (221 -> 193 us) and lose with
   // three (356 -> 413 us).
   const long long small_tiles = ((a.rows + 63) / 64) * ((per_group + 63) / 64) * groups;
-  const long long big_tiles = ((a.rows + 127) / 128) * ((per_group + 127) / 128) * groups;
+  const long long big_tiles = dense_big_tiles(a.rows, per_group) * groups;
   const char* force = getenv("TL_DENSE_TILE");  // 64 / 128: tests and A/B runs pick the tile themselves
   const bool big = force ? atoi(force) == 128
                          : a.rows >= 256 && (a.group_off ? a.terms == 1 && per_group >= 96
@@ -473,16 +485,10 @@ int tl_launch_dense_gemm(const DenseArgs& a, hipStream_t s) {
   const bool first = a.exact_items > 0 && a.terms == 1;
   // wide loads: every matrix, row and piece of eight columns at 16 bytes
   const bool vec = (a.cols & 7) == 0 && (a.ldx & 3) == 0 && ((size_t)a.x & 15) == 0 && ((size_t)a.w & 15) == 0 && (a.x_gstride & 3) == 0;
-  // The plane kernel takes the launches whose 128 x 128 tiles occupy half of the CUs or more and are long enough to pay for the
-  // conversion (rows x columns x items, without / with it, conversion included: 10304 x 2048 x 1999 174 / 114 us, x 512 56 / 36,
-  // x 200 36 / 24; 4096 x 2048 x 1999 66 / 45, x 1024 46 / 30; 2048 x 4096 x 1999 80 / 51, x 1024 47 / 43; 4096 x 1024 x 1024 26 / 20;
-  // on the line 4096 x 2048 x 512 26.3 / 25.8 and 2048 x 2048 x 1024 26.4 / 26.5; below 1024 x 1024 x 1999 16 / 18, 2048 x 4096 x 512
-  // 33 / 39). One tile a CU: eight waves and three steps ahead; more: two workgroups of four waves, which fill each other's waits
-  // (256 tiles 30.3 / 32.5 us, 324 tiles 44.8 / 36.4). TL_DENSE_TILE=64, 128: the kernel above.
-  if (a.plane && a.terms == 1 && groups == 1 && !a.group_off && !a.x_rows && vec && dense_plane_fits(a) && !force &&
-      2 * big_tiles >= tl_num_cus() && big_tiles * a.cols > 1024ll * tl_num_cus()) {
+  // the plane kernel: one tile a CU: eight waves and three steps ahead; more: two workgroups of four waves, which fill each other's
+  // waits (256 tiles 30.3 / 32.5 us, 324 tiles 44.8 / 36.4). TL_DENSE_TILE=64, 128: the kernel above.
+  if (a.plane && a.terms == 1 && groups == 1 && !a.group_off && !a.x_rows && vec && !force && dense_plane_pays(a, tl_num_cus()))
     return dense_plane_run(a, big_tiles <= tl_num_cus() ? 8 : 4, big, s);
-  }
   const int BM = big ? 128 : 64, BN = big ? 128 : 64;
   dim3 grid((a.rows + BM - 1) / BM, (a.T + BN - 1) / BN, groups);
   TL_REQUIRE(grid.y <= 65535 && grid.z <= 65535, "dense gemm: launch too large");
@@ -642,6 +648,7 @@ extern "C" int tl_debug_dense_plane(const void* w_bf16_dev, int rows, int cols, 
   a.T = num_tokens;
   a.terms = 1;
   a.exact_items = exact_items;
+  a.plane_room = ((size_t)num_tokens + 32) * cols;
   TL_REQUIRE(a.w && x_dev && y_dev && rows > 0 && cols > 0 && num_tokens > 0 && ldx >= cols && ldx % 4 == 0 &&
                  exact_items >= 0 && exact_items <= 32 && (waves == 4 || waves == 8) && dense_plane_fits(a) &&
                  (((size_t)w_bf16_dev | (size_t)x_dev | (size_t)plane_dev) & 15) == 0,
@@ -650,4 +657,13 @@ extern "C" int tl_debug_dense_plane(const void* w_bf16_dev, int rows, int cols, 
   a.plane = static_cast<uint16_t*>(plane_dev);
   const char* tile = getenv("TL_DENSE_TILE");
   return dense_plane_run(a, waves, tile && atoi(tile) == 128, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int tl_debug_dense_plane_taken(int rows, int cols, int num_tokens, long long room, int cus) {
+  DenseArgs a = {};
+  a.rows = rows;
+  a.cols = cols;
+  a.T = num_tokens;
+  a.plane_room = (size_t)room;
+  return dense_plane_pays(a, cus);
 }

@@ -51,8 +51,10 @@ struct DenseArgs {
   // groups > 1 without group_off: one product per head over ALL items -- group g multiplies matrix g with the columns
   // x[.][g * x_gstride ..] (0: every head reads the same columns) and writes y[.][g * y_gstride ..]
   int x_gstride, y_gstride;
-  // optional: room for the items as bf16, [T + 32][cols]: large products of one matrix and one term convert them there first
+  // optional: room for plane_room bf16 numbers: large products of one matrix and one term convert their items there first, if
+  // [T + 32][cols] fit
   uint16_t* plane;
+  size_t plane_room;
 };
 int tl_launch_dense_gemm(const DenseArgs& a, hipStream_t s);
 // y[rows] = W x for one token, FP32 throughout (weights widened exactly)

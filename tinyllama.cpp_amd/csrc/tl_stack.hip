@@ -179,8 +179,8 @@ struct TlStack {
   int latent_expand = 64;                   // chunks of at least this many tokens expand (TL_STACK_LATENT_EXPAND; 0: never)
   float *gw = nullptr, *gu = nullptr, *gau = nullptr, *grau = nullptr, *grk = nullptr;  // generalized delta rule (gdelta_pre)
   int max_lq = 0, max_lqa = 0, max_gd = 0, gdelta_layers = 0;
-  uint16_t* plane = nullptr;  // items of one product as bf16, up to plane_cols columns (DenseArgs)
-  int plane_cols = 0;
+  uint16_t* plane = nullptr;  // items of one product as bf16 (DenseArgs)
+  size_t plane_room = 0;      // ... numbers: a chunk's tokens times the widest input of a product over them
   float *act_buf = nullptr, *eout = nullptr, *sact = nullptr, *sout = nullptr, *sgate = nullptr;
   float* wts = nullptr;
   unsigned char* half_ws = nullptr;  // converted K/V tiles and partial outputs of a chunk's attention (tl_hattn.hip)
@@ -1241,8 +1241,8 @@ int tl_stack_finalize(TlStack* st, hipStream_t s) {
     if (st->max_sff) TL_TRY(dev_alloc(st, &st->sact, C * st->max_sff));
   }
   if (C >= 64) {
-    st->plane_cols = std::max({(int)W, (int)st->max_od, (int)st->max_sff});
-    TL_TRY(dev_alloc(st, &st->plane, (C + 32) * st->plane_cols));
+    st->plane_room = (C + 32) * std::max({(size_t)W, (size_t)st->max_od, (size_t)st->max_sff});
+    TL_TRY(dev_alloc(st, &st->plane, st->plane_room));
   }
   bool any_parallel = false;
   for (const Layer& L : st->layers)
@@ -1374,8 +1374,12 @@ namespace {
 // one by one to FP32 accuracy instead of bf16's.
 inline int terms_for(const TlStack* st, int T) { return T < st->exact_below ? 3 : st->terms; }
 
-// where a chunk's product may put its items as bf16 (one after another on the chunk's stream: forks are for single tokens)
-inline uint16_t* plane_for(const TlStack* st, int cols) { return cols <= st->plane_cols ? st->plane : nullptr; }
+// where a chunk's product may put its items as bf16 (one after another on the chunk's stream: forks are for single tokens; a latent
+// cache's rows can be more than a chunk's, and than fit)
+inline void give_plane(const TlStack* st, DenseArgs* d) {
+  d->plane = st->plane;
+  d->plane_room = st->plane_room;
+}
 
 // y[T][rows] = x[T][cols] W^T for a chunk, or the GEMV for the one token of a decode step
 int project(TlStack* st, const uint16_t* w, int rows, int cols, const float* x, int ldx, float* y, int ldy, int T,
@@ -1393,7 +1397,7 @@ int project(TlStack* st, const uint16_t* w, int rows, int cols, const float* x, 
   d.terms = terms_for(st, T);
   d.exact_items = st->exact_items;
   d.softcap = softcap;
-  d.plane = plane_for(st, cols);
+  give_plane(st, &d);
   return tl_launch_dense_gemm(d, s);
 }
 
@@ -1418,7 +1422,7 @@ int project_act(TlStack* st, const uint16_t* w, int rows, int cols, const float*
   d.act_p = act.act_p;
   d.act_q = act.act_q;
   d.bias = act.bias;
-  d.plane = plane_for(st, cols);
+  give_plane(st, &d);
   return tl_launch_dense_gemm(d, s);
 }
 
@@ -1523,7 +1527,7 @@ int moe_experts(TlStack* st, const Layer& L, const Layer& Wt, const float* in, i
     u.glu_alpha = sp.act_alpha;
     u.glu_up_add = sp.glu_up_add;
     u.glu_kind = sp.glu;
-    u.plane = plane_for(st, W);
+    give_plane(st, &u);
     TL_TRY(tl_launch_dense_gemm(u, s));
     TL_TRY(project(st, Wt.sdown, W, sff, st->sact, sff, st->sout, W, T, s));
   }
@@ -2362,7 +2366,7 @@ int dense_unit(TlStack* st, const Layer& L, const Layer& Wt, const float* in, in
   u.glu_alpha = sp.act_alpha;
   u.glu_up_add = sp.glu_up_add;
   u.glu_kind = sp.glu;
-  u.plane = plane_for(st, W);
+  give_plane(st, &u);
   TL_TRY(tl_launch_dense_gemm(u, s));
   return project(st, Wt.sdown, W, ff, st->sact, ff, st->sout, W, T, s);
 }
