@@ -604,3 +604,21 @@ def test_decode_step_with_wide_rows_and_many_slots(env, dim, top, ff, shared_ff)
         got = np.stack([m.decode(int(toks[i]), i)[0] for i in range(lo, hi)])
         assert rel_rms(got, want[lo:hi]) < FP32_TOL, (lo, hi)
     m.free()
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,n,window", [(4, 2, 64, 70, 0), (2, 2, 128, 300, 0), (2, 1, 64, 290, 130), (3, 3, 128, 9, 5)])
+@pytest.mark.parametrize("T", [1, 3])
+def test_an_infinite_value_stays_one(env, heads, kv_heads, dim, n, window, T):
+    """The last key's value row has an infinity: that column is infinite for the token that sees it, not NaN, and all others are what
+    they are without it (loads beyond the last key read its row again)."""
+    rng = np.random.default_rng(n)
+    k, v = (rng.standard_normal((n, kv_heads * dim)).astype(np.float32) for _ in range(2))
+    q = rng.standard_normal((T, heads * dim)).astype(np.float32)
+    col = (kv_heads - 1) * dim + 5
+    v[-1, col] = np.inf
+    got = run_swa(env, q, k, v, n - T, heads, kv_heads, dim, dim, window, 0.1).reshape(T, heads, dim)
+    v[-1, col] = 0.0
+    want = run_swa(env, q, k, v, n - T, heads, kv_heads, dim, dim, window, 0.1).reshape(T, heads, dim)
+    sees = np.zeros((T, heads, dim), bool)
+    sees[-1, heads - heads // kv_heads:, 5] = True
+    assert (got[sees] == np.inf).all() and np.array_equal(got[~sees], want[~sees])

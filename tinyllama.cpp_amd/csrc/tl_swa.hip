@@ -86,7 +86,7 @@ __device__ __forceinline__ void swa_merge_records(const SwaArgs& a, int nsplit, 
   for (int d0 = 0; d0 < a.vdim; d0 += 64) {  // every lane stays in the loop: a shuffle reads nothing from a lane that has left
     const int d = d0 + lane;
     float acc = 0.0f;
-    for (int z0 = 0; z0 < nsplit; z0 += 8) {  // eight records' values in flight together (clamped index, weight 0 beyond)
+    for (int z0 = 0; z0 < nsplit; z0 += 8) {  // eight records' values in flight together (clamped index, left out beyond)
       float v[8], f[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
@@ -95,11 +95,10 @@ __device__ __forceinline__ void swa_merge_records(const SwaArgs& a, int nsplit, 
       }
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        const float fu = __shfl(fz, z0 + u < nsplit ? z0 + u : 0);
-        f[u] = z0 + u < nsplit ? fu : 0.0f;
+        f[u] = __shfl(fz, z0 + u < nsplit ? z0 + u : 0);
       }
 #pragma unroll
-      for (int u = 0; u < 8; ++u) acc += v[u] * f[u];  // in split order
+      for (int u = 0; u < 8; ++u) acc += z0 + u < nsplit ? v[u] * f[u] : 0.0f;  // in split order (0 times an infinity is none)
     }
     if (d < a.vdim) op[d] = (a.sigmoid ? acc : acc / L) * of;
   }
@@ -381,15 +380,24 @@ __global__ __launch_bounds__(256) void swa_rows_kernel(const SwaArgs a) {
       l *= corr;
 #pragma unroll
       for (int v = 0; v < NV; ++v) o[v] *= corr;
+      // FULL: all of the step's keys are visible. Otherwise a lane beyond the last key holds that key's row again, which has to be
+      // left out: zero times an infinity is none
+      auto add = [&](auto full_c) __attribute__((always_inline)) {
+        constexpr bool FULL = decltype(full_c)::value;
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const float p = j0 + 4 * u + sub > jend ? 0.0f : a.sigmoid ? 1.0f / (1.0f + expf(-(s[u] + hb))) : expf(s[u] - mn);
-        l += p;
+        for (int u = 0; u < U; ++u) {
+          if (!FULL && j0 + 4 * u > jend) break;
+          const bool out = !FULL && j0 + 4 * u + sub > jend;
+          const float p = out ? 0.0f : a.sigmoid ? 1.0f / (1.0f + expf(-(s[u] + hb))) : expf(s[u] - mn);
+          l += p;
 #pragma unroll
-        for (int v = 0; v < NV; ++v)
+          for (int v = 0; v < NV; ++v)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) o[v][e] = fmaf(p, vv[u][v][e], o[v][e]);
-      }
+            for (int e = 0; e < 4; ++e) o[v][e] = fmaf(p, out ? 0.0f : vv[u][v][e], o[v][e]);
+        }
+      };
+      if (j0 + 4 * U - 1 <= jend) add(std::true_type{});
+      else add(std::false_type{});
     }
   }
   l += __shfl_xor(l, 16);
