@@ -586,10 +586,10 @@ def test_window_attention_over_wide_rows(env, heads, kv_heads, dim, window):
     test_window_attention_prompt_and_decode(env, heads, kv_heads, dim, dim, window)
 
 
-@pytest.mark.parametrize("dim,top,ff,shared_ff", [(64, 6, 1032, 40), (128, 4, 24, 0), (64, 10, 16, 1544)])
+@pytest.mark.parametrize("dim,top,ff,shared_ff", [(64, 6, 1032, 40), (128, 4, 24, 0), (64, 10, 16, 1544), (128, 2, 776, 1536), (64, 1, 2048, 514)])
 def test_decode_step_with_wide_rows_and_many_slots(env, dim, top, ff, shared_ff):
     """The captured decode step over heads of 64 and 128: positions across 256, 512 and the window (one split, several, the last of
-    which merges), seven to eleven expert slots of rows below, at and above 1024 columns, and a norm row of two numbers a thread."""
+    which merges), two to eleven expert slots of rows below, at and above 512 and 1024 columns, 16-byte pieces or not, and a norm row of two numbers a thread."""
     S = env["synth"]
     L = S.stack_layer
     cfg = S.stack_config(1040, 211, [L(4, 2, dim, dim, 600, v_mix=True, experts=12, top=top, ff=ff, shared_ff=shared_ff),

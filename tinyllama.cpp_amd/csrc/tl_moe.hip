@@ -106,73 +106,50 @@ __global__ __launch_bounds__(256) void moe_decode_up_kernel(const MoeDecodeArgs 
   if (lane < 2 && r + lane < a.ff) a.act[(size_t)j * a.ff + r + lane] = tl_act_apply(a.unit_act, lane ? u2[1] : u2[0], 0.0f, 0.0f);
 }
 
-// The same for 16-byte pieces throughout: the rows of up to five slots (four chosen experts and the shared one) are in flight together,
-// 1024 columns at a time, and their weighted products meet in one sum over the lanes. One expert after another is a round trip and a
-// sum each: 2048 rows of 4 x 768 + 1024 columns 9.7 us, here 8.3 (16.8 MB; two rows a wave: 12).
-__global__ __launch_bounds__(256) void moe_decode_down_all_kernel(const MoeDecodeArgs a) {
-  constexpr int NS = 5;
-  const int lane = threadIdx.x & 63, r = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
-  if (r >= a.width) return;
-  const int slots = a.top + (a.sdown ? 1 : 0);
-  const float sg = a.sdown && a.sgate ? *a.sgate : 1.0f;
-  float y = 0.0f;
-  for (int j0 = 0; j0 < slots; j0 += NS) {
-    const unsigned short* w[NS];
-    const float* x[NS];
-    float f[NS], acc[NS];
-    int n[NS], most = 0;
-#pragma unroll
-    for (int u = 0; u < NS; ++u) {
-      const int j = j0 + u;
-      const bool live = j < slots, shared = j >= a.top;
-      n[u] = !live ? 0 : shared ? a.sff : a.ff;
-      w[u] = !live || shared ? a.sdown + (size_t)r * a.sff : a.down + ((size_t)a.ids[j] * a.width + r) * a.ff;
-      if (!live && !a.sdown) w[u] = a.down;  // (read at its first piece, for nothing)
-      x[u] = a.act + (size_t)(live ? j : 0) * a.ff;
-      f[u] = !live ? 0.0f : shared ? sg : a.wts[j];
-      acc[u] = 0.0f;
-      most = n[u] > most ? n[u] : most;
-    }
-    for (int k0 = 0; k0 < most; k0 += 1024) {
-      uint4 wv[NS][2];
-      float4 xv[NS][2][2];
-#pragma unroll
-      for (int u = 0; u < NS; ++u)
-#pragma unroll
-        for (int p = 0; p < 2; ++p) {
-          const int k = k0 + 512 * p + lane * 8, kc = k < n[u] ? k : 0;
-          wv[u][p] = tl_ldw(w[u] + kc);
-          xv[u][p][0] = *reinterpret_cast<const float4*>(x[u] + kc);
-          xv[u][p][1] = *reinterpret_cast<const float4*>(x[u] + kc + 4);
-        }
-#pragma unroll
-      for (int u = 0; u < NS; ++u)
-#pragma unroll
-        for (int p = 0; p < 2; ++p) {
-          const float s = tl_dot8(wv[u][p], xv[u][p][0], xv[u][p][1], acc[u]);
-          acc[u] = k0 + 512 * p + lane * 8 < n[u] ? s : acc[u];
-        }
-    }
-#pragma unroll
-    for (int u = 0; u < NS; ++u)
-      if (j0 + u < slots) y += f[u] * acc[u];
+// a lane's part of a bf16 row times x: 1024 columns in flight at a time, also the last 513 to 1023 (one loop: a loop for whole steps
+// and a tail of its own took 1.3 times as long over rows of 768)
+__device__ __forceinline__ float lane_dot(const unsigned short* __restrict__ w, const float* __restrict__ x, int n, bool vec, int lane) {
+  auto dot = [&](const uint4& wv, int k, float acc) __attribute__((always_inline)) {
+    return tl_dot8(wv, *reinterpret_cast<const float4*>(x + k), *reinterpret_cast<const float4*>(x + k + 4), acc);
+  };
+  float acc = 0.0f;
+  if (!vec) {
+    for (int k = lane; k < n; k += 64) acc += tl_bf2f(w[k]) * x[k];
+    return acc;
   }
-  y = tl_wave_sum(y);
-  if (lane == 0) a.y[r] = y;
+  int k0 = 0;
+  for (; k0 + 512 < n; k0 += 1024) {  // (lanes beyond the row read its first columns and count nothing)
+    const int k = k0 + lane * 8;
+    const bool in = k + 512 < n;
+    const int k2 = in ? k + 512 : 0;
+    const uint4 wa = tl_ldw(w + k), wb = tl_ldw(w + k2);
+    acc = dot(wa, k, acc);
+    const float s = dot(wb, k2, acc);
+    acc = in ? s : acc;
+  }
+  if (k0 < n) {
+    const int k = k0 + lane * 8, k1 = k < n ? k : 0;
+    const float s = dot(tl_ldw(w + k1), k1, acc);
+    acc = k < n ? s : acc;
+  }
+  return acc;
 }
 
+// A wave owns a row: the chosen experts one after another, then the shared one, and one sum over the lanes at the end. With a sum per
+// expert, and a row's last 513 to 1023 columns in two goes: 2048 rows of 4 x 768 + 1024 columns 9.0 us, here 6.5 (16.8 MB); of 2 x 1024
+// 4.4 and 4.1, of 8 x 512 9.0 and 7.7, of 8 x 1536 + 2048 16.4 and 15.1; of one unit of 4096 or 11264 5.4 and 10.3, 5.4 and 10.4. With five
+// slots' loads in flight together, there or not: 8.1, 6.1, 10.8, 23 and, for one unit, 13 and 34.
 __global__ __launch_bounds__(256) void moe_decode_down_kernel(const MoeDecodeArgs a, int vec_e, int vec_s) {
-  const int lane = threadIdx.x & 63, r = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, r = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
   if (r >= a.width) return;
   float y = 0.0f;
-  for (int j = 0; j < a.top; ++j) {
-    const unsigned short* d = a.down + ((size_t)a.ids[j] * a.width + r) * a.ff;
-    y += a.wts[j] * wave_dot(d, a.act + (size_t)j * a.ff, a.ff, vec_e != 0, lane);
-  }
+  for (int j = 0; j < a.top; ++j)
+    y += a.wts[j] * lane_dot(a.down + ((size_t)a.ids[j] * a.width + r) * a.ff, a.act + (size_t)j * a.ff, a.ff, vec_e != 0, lane);
   if (a.sdown) {
-    const float sh = wave_dot(a.sdown + (size_t)r * a.sff, a.act + (size_t)a.top * a.ff, a.sff, vec_s != 0, lane);
+    const float sh = lane_dot(a.sdown + (size_t)r * a.sff, a.act + (size_t)a.top * a.ff, a.sff, vec_s != 0, lane);
     y += a.sgate ? *a.sgate * sh : sh;
   }
+  y = tl_wave_sum(y);
   if (lane == 0) a.y[r] = y;
 }
 
@@ -235,8 +212,7 @@ int tl_launch_moe_decode(const MoeDecodeArgs& a, hipStream_t s) {
   } else {
     moe_decode_gu_kernel<<<dim3((ffmax + 3) / 4, a.top + (a.sgu ? 1 : 0)), 256, 0, s>>>(a, vec_x);
   }
-  if (vec_e && (vec_s || !a.sdown)) moe_decode_down_all_kernel<<<(a.width + 3) / 4, 256, 0, s>>>(a);
-  else moe_decode_down_kernel<<<(a.width + 3) / 4, 256, 0, s>>>(a, vec_e, vec_s);
+  moe_decode_down_kernel<<<(a.width + 3) / 4, 256, 0, s>>>(a, vec_e, vec_s);
   TL_HIP(hipGetLastError());
   return 0;
 }
