@@ -622,3 +622,32 @@ def test_an_infinite_value_stays_one(env, heads, kv_heads, dim, n, window, T):
     sees = np.zeros((T, heads, dim), bool)
     sees[-1, heads - heads // kv_heads:, 5] = True
     assert (got[sees] == np.inf).all() and np.array_equal(got[~sees], want[~sees])
+
+
+@pytest.mark.parametrize("T,width", [(1, 513), (8, 1024), (3, 1025), (1, 2048), (5, 4095), (2, 4097), (1, 8192), (9, 512), (20, 513), (9, 1024), (1025, 1023),
+                                     (9, 2047), (1030, 2048), (10, 2049)])
+def test_residual_output_norm_of_every_row_length(env, T, width):
+    """One, two, four and eight numbers a thread and the loop, in workgroups of 1024 (up to 8 rows) and 256 threads."""
+    rng = np.random.default_rng(width)
+    x, y = (rng.standard_normal((T, width)).astype(np.float32) for _ in range(2))
+    w = (0.1 * rng.standard_normal(width)).astype(np.float32)
+    xd, yd, wd = dev(env, x), dev(env, y), dev(env, w)
+    env["capi"].check(env["capi"].lib().tl_resid_rmsnorm(xd.ptr, yd.ptr, wd.ptr, T, width, 1e-6, None), "tl_resid_rmsnorm")
+    env["capi"].check(env["capi"].lib().tl_device_sync(), "sync")
+    want = x + env["oracle"].rms_norm(y.astype(np.float64), w.astype(np.float64), 1e-6, True)
+    assert np.allclose(xd.to_numpy(np.float32, (T, width)), want, rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("heads,dim,width", [(16, 64, 1024), (16, 128, 1000), (32, 128, 2048), (36, 128, 520)])
+def test_projections_and_router_rows_of_every_length(env, heads, dim, width):
+    """Queries of 1024, 2048, 4096 and more numbers, routers over rows of one to four pieces a lane: a short portion, a longer one and
+    single tokens against the float64 oracle."""
+    S = env["synth"]
+    L = S.stack_layer
+    cfg = S.stack_config(width, 211, [L(heads, 4, dim, dim, 50, v_mix=True, experts=20, top=3, ff=64, shared_ff=32) for _ in range(2)])
+    m, _, orc = make(env, cfg, seed=9, max_pos=64)
+    toks = np.random.default_rng(width).integers(0, cfg["vocab"], 40).astype(np.int32)
+    want = orc.forward(list(toks))
+    got = np.concatenate([m.prefill_rows(toks[:5], 0), m.prefill_rows(toks[5:37], 5), np.stack([m.decode(int(toks[i]), i)[0] for i in (37, 38, 39)])])
+    assert rel_rms(got, want) < FP32_TOL
+    m.free()

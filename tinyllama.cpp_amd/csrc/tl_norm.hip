@@ -168,10 +168,10 @@ __global__ __launch_bounds__(1024) void resid_norm_kernel(const ResidNormArgs a)
     }
     return y;
   };
-  constexpr int EARLY = 2048;  // columns of a router row that a wave holds: 32 a lane
+  constexpr int RP = NP == 1 || NP == 4 ? 2 : 4, EARLY = 512 * RP;  // pieces and columns of a router row that a wave holds, if a row is no longer
   const bool vec = (a.width & 7) == 0 && ((size_t)a.route.w & 15) == 0;
   const bool early = NP > 0 && a.route.w && vec && a.width <= EARLY && wave < a.route.experts;
-  uint4 rw[4];
+  uint4 rw[RP];
   float ss = 0.0f;
   if constexpr (NP > 0) {
     float y[NP], xv[NP], wv[NP];
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(1024) void resid_norm_kernel(const ResidNormArgs a)
     }
     if (early) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
+      for (int k = 0; k < RP; ++k) {
         const int c = lane * 8 + 512 * k;
         rw[k] = tl_ldw(a.route.w + (size_t)wave * a.width + (c < a.width ? c : 0));
       }
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(1024) void resid_norm_kernel(const ResidNormArgs a)
     float sdot = 0.0f;
     if (early && e == wave) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
+      for (int k = 0; k < RP; ++k) {
         const int c = lane * 8 + 512 * k;
         if (c < a.width) sdot = tl_dot8(rw[k], *reinterpret_cast<const float4*>(row + c), *reinterpret_cast<const float4*>(row + c + 4), sdot);
       }
@@ -753,7 +753,9 @@ int tl_launch_qkv_post(const QkvPostArgs& a, hipStream_t s) {
                                  a.vmix == 0 && a.q_temp_every == 0),
              "qkv_post: a norm per block of %d over %d / %d", a.head_dim, a.qd, a.kd);
   const int threads = row_threads(a.T), most = a.qd > a.kd ? (a.qd > a.vd ? a.qd : a.vd) : a.kd > a.vd ? a.kd : a.vd;
-  if (most <= 4 * threads) qkv_post_kernel<4><<<a.T, threads, 0, s>>>(a);
+  if (most <= threads) qkv_post_kernel<1><<<a.T, threads, 0, s>>>(a);
+  else if (most <= 2 * threads) qkv_post_kernel<2><<<a.T, threads, 0, s>>>(a);
+  else if (most <= 4 * threads) qkv_post_kernel<4><<<a.T, threads, 0, s>>>(a);
   else qkv_post_kernel<0><<<a.T, threads, 0, s>>>(a);
   TL_HIP(hipGetLastError());
   return 0;
@@ -770,9 +772,16 @@ int tl_launch_resid_norm(const ResidNormArgs& a, hipStream_t s) {
     lds = sizeof(float) * (((a.width + 3) & ~3) + a.route.experts);
     TL_REQUIRE(lds <= 64 * 1024, "resid_norm: width %d + %d experts do not fit the staged row", a.width, a.route.experts);
   }
+  // Few rows: 512 wide the loop is as fast (one token 2.5 us, 2.8 with early loads), from there on as many numbers a thread as the row
+  // has (4096 wide with four experts' slots 7.4 us in a loop, 6.7 with four, 8.3 with room for eight; 8192 wide 6.6 and 3.7). Many rows:
+  // only as long as a round of workgroups takes them all (512 rows of 1024 3.5 and 3.2, 2000 rows 5.1 and 5.3; 2000 rows of 2048 with four
+  // slots 19.5 and 25.3: registers in place of workgroups); rows of 2048 without slots or router always (2000 rows 8.3 and 6.7).
   const int threads = row_threads(a.T), per = (a.width + threads - 1) / threads;
-  if (per <= 2) resid_norm_kernel<2><<<a.T, threads, lds, s>>>(a);
-  else if (per <= 8) resid_norm_kernel<8><<<a.T, threads, lds, s>>>(a);
+  const bool few = a.T <= 8, round = few || a.T <= 4 * tl_num_cus();
+  if (few && a.width > 512 && per <= 1) resid_norm_kernel<1><<<a.T, threads, lds, s>>>(a);
+  else if (few && a.width > 512 && per <= 2) resid_norm_kernel<2><<<a.T, threads, lds, s>>>(a);
+  else if (per > 2 && per <= 4 && round && (few || !a.route.w)) resid_norm_kernel<4><<<a.T, threads, lds, s>>>(a);
+  else if (per > 4 && per <= 8 && (round || (!a.slots && !a.route.w))) resid_norm_kernel<8><<<a.T, threads, lds, s>>>(a);
   else resid_norm_kernel<0><<<a.T, threads, lds, s>>>(a);
   TL_HIP(hipGetLastError());
   return 0;
