@@ -67,6 +67,12 @@ int tl_debug_half_attention(const float* q_dev, const float* k_cache_dev, const 
                             int num_tokens, int start_pos, int heads, int kv_heads, int dim, int vdim, int window, float scale,
                             void* stream);
 
+/* Test hook (no counterpart in the reference): the row-tile attention of packed prompts (tl_prefill.hip) over q [T][heads][dim], token i
+ * at positions_host[i] of sequence seq_idx_host[i], whose caches [*][kv_heads][dim] lie seq_stride floats apart; dim 64 or 128. */
+int tl_debug_packed_attention(const float* q_dev, const float* k_cache_dev, const float* v_cache_dev, float* out_dev, long long seq_stride,
+                              const int* positions_host, const int* seq_idx_host, int num_tokens, int heads, int kv_heads, int dim,
+                              float scale, void* stream);
+
 /* Parity hook for layer-list models (no counterpart in the reference): cb(ctx, layer, x_dev, num_tokens, width) is called after
  * every layer of every forward pass, the stream synchronised, with the residual stream on the device. NULL switches it off.
  * With the hook set the decode step must run eagerly (TL_NO_GRAPH=1 at finalize): a captured step cannot call back. */

@@ -330,3 +330,128 @@ def test_many_logits_reach_the_caller(pkg):
         assert np.linalg.norm(logits - want[:n]) <= 4e-6 * np.linalg.norm(want[:n]) and np.array_equal(ids, logits.argmax(1)), n
         assert np.abs(logits - want[:n]).max() <= 1e-4 * np.abs(want).max(), n
     m.free()
+
+@pytest.mark.parametrize("heads,kv_heads,hd,lens", [(4, 4, 64, (320, 40)), (6, 2, 128, (500, 300))])
+@pytest.mark.parametrize("bad", ["nan", "huge"])
+def test_packed_attention_before_a_row_out_of_range(pkg, monkeypatch, heads, kv_heads, hd, lens, bad):
+    """A token whose key and value rows are NaN, or 2^30 times and more as large as its neighbours', in the middle of a key tile: the tokens in
+    front of it give what the per-token FP32 kernel gives, to the tolerance of finite batches; those behind it are NaN in both."""
+    from tinyllama_cpp_amd import engine as E
+    from tinyllama_cpp_amd.capi import check, lib
+    E.init(0)
+    cfg = dict(pkg.synth.SHAPES["tiny-gqa"], hidden=heads * hd, n_heads=heads, n_kv_heads=kv_heads, n_layers=1, max_pos=640)
+    cfg, tensors = pkg.synth.build_model(cfg, "q4_k_m", seed=8)
+    typ, emb, rows, cols = tensors["token_embd.weight"]
+    blocks = emb.copy().reshape(rows, cols // 256, 144)
+    half = blocks[7, :, :4].copy().view(np.float16)  # a block's scale and minimum
+    half[:] = np.nan if bad == "nan" else 6e4
+    blocks[7, :, :4] = half.view(np.uint8)
+    if bad == "huge":  # norms that keep a row's size (eps over its mean square), and everybody else small
+        others = np.arange(rows) != 7
+        small = blocks[others, :, :4].copy().view(np.float16) * np.float16(2.0 ** -10)
+        blocks[others, :, :4] = small.view(np.uint8)
+        cfg["eps"] = 1e24
+        for name in ("blk.0.attn_norm.weight", "blk.0.ffn_norm.weight", "output_norm.weight"):
+            t, w, r, c = tensors[name]
+            tensors[name] = (t, (w * np.float32(0.0 if "ffn" in name else 1e12)).astype(w.dtype), r, c)
+    tensors["token_embd.weight"] = (typ, blocks.reshape(emb.shape), rows, cols)
+    m = E.Model(cfg).load(tensors)
+    m.batch_init(8)
+    rng = np.random.default_rng(2)
+    toks = rng.integers(8, cfg["vocab"], sum(lens)).astype(np.int32)
+    at = 290
+    toks[at] = 7
+    pos = np.concatenate([np.arange(n) for n in lens]).astype(np.int32)
+    seq = np.concatenate([np.full(n, s) for s, n in zip((3, 1), lens)]).astype(np.int32)
+    last = np.array([5, 200, 287, 288, at - 1, at, lens[0] - 1, sum(lens) - 1], np.int32)
+    got = []
+    for switch in ("0", "1"):
+        monkeypatch.setenv("TL_HATTN", switch)
+        m.reset_kv()
+        logits, ids = np.zeros((last.size, cfg["vocab"]), np.float32), np.zeros(last.size, np.int32)
+        check(lib().tl_model_batch_prefill_packed(m.h, toks.size, toks.ctypes.data, pos.ctypes.data, seq.ctypes.data, last.size,
+                                                  last.ctypes.data, logits.ctypes.data, ids.ctypes.data), "packed")
+        got.append(logits)
+    assert not np.array_equal(got[0], got[1])  # (the other kernel ran)
+    for j, r in enumerate(last):
+        if bad == "nan" and at <= r < lens[0]:
+            assert np.isnan(got[0][j]).all() and np.isnan(got[1][j]).all(), r
+        else:
+            assert np.isfinite(got[0][j]).all() and np.linalg.norm(got[1][j] - got[0][j]) <= 4e-6 * np.linalg.norm(got[0][j]), r
+    m.free()
+
+
+def test_packed_prompts_need_no_memory_of_their_own(pkg):
+    """What the attention of packed prompts converts its rows into is laid out with the sequences' caches: neither a small batch (the
+    per-token kernel) nor a large one takes device memory when the first one comes."""
+    import ctypes as C
+    from tinyllama_cpp_amd import engine as E
+    E.init(0)
+    hip = C.CDLL("libamdhip64.so")
+
+    def free_bytes():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    cfg = dict(pkg.synth.SHAPES["tiny-gqa"], hidden=256, n_heads=4, n_kv_heads=4, n_layers=1, max_pos=640)
+    cfg, tensors = pkg.synth.build_model(cfg, "q4_k_m", seed=8)
+    rng = np.random.default_rng(3)
+    prompts = [rng.integers(0, cfg["vocab"], n).astype(np.int32) for n in (320, 40, 9)]
+    for warm in (True, False):  # (the first model's calls make what the process keeps: loaded kernels, scratch)
+        m = E.Model(cfg).load(tensors)
+        m.batch_init(4)
+        m.batch_decode(np.array([1]), np.array([0]), np.array([3]))
+        before = free_bytes()
+        m.batch_prefill_packed(prompts[2:])
+        m.batch_prefill_packed(prompts)
+        if not warm:
+            assert free_bytes() == before
+        m.free()
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd", [(8, 1, 64), (6, 2, 64), (3, 3, 64), (4, 2, 128), (8, 1, 128), (3, 1, 128)])
+def test_packed_attention_kernel(pkg, heads, kv_heads, hd):
+    """Row tiles of one to 32 rows and tiles of one to 32 keys, at the edges of both, one key and many; NaN behind every sequence's last
+    position. Against float64: half a dozen roundings on the way to a score (a sum of eight, met in a tree; sizes up to 8 in here), as many on
+    the way of the values."""
+    from tinyllama_cpp_amd import engine as E
+    from tinyllama_cpp_amd.capi import check, lib
+    E.init(0)
+    rng = np.random.default_rng(heads * hd + kv_heads)
+    runs = [(3, 0, 1), (0, 0, 33), (4, 31, 1), (1, 30, 5), (2, 0, 64), (6, 97, 31), (5, 200, 40), (7, 0, 2)]
+    S, group = 256, heads // kv_heads
+    pos = np.concatenate([np.arange(p, p + n) for _, p, n in runs]).astype(np.int32)
+    seq = np.concatenate([np.full(n, s) for s, _, n in runs]).astype(np.int32)
+    q = rng.standard_normal((pos.size, heads, hd)).astype(np.float32)
+    k, v = (rng.standard_normal((8, S, kv_heads, hd)).astype(np.float32) for _ in range(2))
+    for s, p, n in runs:
+        k[s, p + n:], v[s, p + n:] = np.nan, np.nan
+    scale = float(np.float32(2.0 / np.sqrt(hd)))
+
+    def run(v):
+        dev = [E.DeviceBuffer.from_numpy(a) for a in (q, k, v)]
+        out = E.DeviceBuffer(4 * q.size)
+        check(lib().tl_memset(out.ptr, 0xff, out.nbytes, None))
+        check(lib().tl_debug_packed_attention(*(d.ptr for d in dev), out.ptr, S * kv_heads * hd, pos.ctypes.data, seq.ctypes.data, pos.size, heads,
+                                              kv_heads, hd, scale, None), "tl_debug_packed_attention")
+        return out.to_numpy(np.float32, q.shape)
+
+    got = run(v)
+    for i, (p, s) in enumerate(zip(pos, seq)):
+        K, V = (np.repeat(a[s, :p + 1].astype(np.float64), group, 1) for a in (k, v))
+        sc = np.einsum("hd,jhd->hj", q[i].astype(np.float64), K) * scale
+        w = np.exp(sc - sc.max(1, keepdims=True))
+        w /= w.sum(1, keepdims=True)
+        want = np.einsum("hj,jhd->hd", w, V)
+        bound = 2.0 ** -24 * np.einsum("hj,jhd->hd", w * (12 + 8 * np.abs(sc).max()), np.abs(V))
+        assert (np.abs(got[i] - want) <= bound).all(), (i, p, s, float((np.abs(got[i] - want) / bound).max()))
+    # an infinity and a NaN in two columns of one position: seen from there on, and nowhere else
+    s, p, n = runs[1]
+    v[s, 20, 0, 3], v[s, 20, kv_heads - 1, hd - 2] = np.inf, np.nan
+    odd = run(v)
+    sees = (seq == s) & (pos >= 20)
+    assert (odd[sees][:, :group, 3] == np.inf).all() and np.isnan(odd[sees][:, heads - group:, hd - 2]).all()
+    odd[np.ix_(sees, np.arange(group), [3])] = got[np.ix_(sees, np.arange(group), [3])]
+    odd[np.ix_(sees, np.arange(heads - group, heads), [hd - 2])] = got[np.ix_(sees, np.arange(heads - group, heads), [hd - 2])]
+    assert np.array_equal(odd, got)

@@ -10,19 +10,16 @@
 //      lanes of a matrix instruction take them (K: eight columns of one key; V: eight keys of one column, the keys in the
 //      order in which the accumulator of K Q^T holds them, so that the probabilities never change lanes). One power of two
 //      per tile brings its largest finite value to 2^14: a value is held to 2^-23 of itself and 2^-39 of its tile's largest.
-//      Against float64 the output's error is at most 5e-8 of its weights times its values' size, the FP32 kernel's 7e-8 (both sides
+//      Against float64 the output's error is 5e-8 of its weights times its values' size, the FP32 matrix kernel's 7e-8 (both sides
 //      lose what the order of the sums gives); a row of a tile that is 2^20 times the others' size brings it to 1e-7, 2^24 to
-//      1.3e-6.
-//      The sums of a tile and of the small products are kept apart, and the weights' 2^12 stands outside the exponential: packed
-//      prompts' logits are as far from float64 as with the per-token FP32 kernel (20 batches: within 1 %; before, 2 to 5 % further).
+//      1.3e-6. The sums of a tile and of the small products are kept apart, and the weights' 2^12 stands outside the
+//      exponential: 8B prompts' logits 2.65e-6 -> 2.21e-6 off float64, for 1.7 % of the kernel's time (0 to 7 % over 70 shapes: 8 heads of
+//      128 over 64, 64 tokens, 12.0 -> 12.9 us; two blocks of 32 columns in turn gain nothing back).
 //   2. hattn_kernel: four waves, 128 rows (query, head of the kv head's group), tiles through a double-buffered LDS window
 //      that all four waves read: one wave's operands straight from memory would need 85 bytes a cycle and CU. Two workgroups
 //      a CU, so that one's softmax runs under the other's products. A row tile's keys are cut into up to 16 pieces.
 //   3. hattn_combine_kernel sums the pieces of a row tile that has more than one, in order.
 #include <math.h>
-
-#include <algorithm>
-#include <vector>
 
 #include "tl_internal.h"
 
@@ -61,30 +58,19 @@ struct HPlanesArgs {
   int kld, khs, vld, lo, len, nkv, tile0, tiles;  // rows lo .. len - 1; tiles tile0 .. tile0 + tiles - 1 (others' rows: zeros)
   _Float16* planes;      // [nkv][tiles][(KD + VD) * 64]: K then V fragments
   int* exps;             // [nkv][tiles][2]
-  const TlHattnTile* pack;  // PACKED: the tiles of several sequences, seq_stride floats apart
-  size_t seq_stride;
 };
-template <int KD, int VD, bool PACKED>
+template <int KD, int VD>
 __global__ __launch_bounds__(256) void kv_planes_kernel(const HPlanesArgs a) {
   constexpr int PK = (KD + 63) / 64, PV = (VD + 63) / 64;  // fragments of each operand per thread
   __shared__ float red[8];
-  const int tile = blockIdx.x, kvh = blockIdx.y, tid = threadIdx.x;
-  int p0 = (a.tile0 + tile) * 32, lo_key = a.lo, len = a.len;
+  const int tile = blockIdx.x, kvh = blockIdx.y, tid = threadIdx.x, p0 = (a.tile0 + tile) * 32;
   const float *kp = a.kc + (size_t)kvh * a.khs, *vp = a.vc + (size_t)kvh * VD;
-  if (PACKED) {
-    const TlHattnTile it = a.pack[tile];
-    p0 = it.pos;
-    lo_key = 0;
-    len = it.len;
-    kp += (size_t)it.seq * a.seq_stride;
-    vp += (size_t)it.seq * a.seq_stride;
-  }
   float k[PK][8], v[PV][8], mk = 0.f, mv = 0.f;
 #pragma unroll
   for (int t = 0; t < PK; ++t) {
     const int f = tid + 256 * t, lane = f & 63, r = lane & 31, h = lane >> 5, g = f >> 6;
     f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = x;
-    if (f < 4 * KD && p0 + r >= lo_key && p0 + r < len) {
+    if (f < 4 * KD && p0 + r >= a.lo && p0 + r < a.len) {
       const float* src = kp + (size_t)(p0 + r) * a.kld + 16 * g + 8 * h;
       x = *reinterpret_cast<const f32x4*>(src);
       y = *reinterpret_cast<const f32x4*>(src + 4);
@@ -99,7 +85,7 @@ __global__ __launch_bounds__(256) void kv_planes_kernel(const HPlanesArgs a) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int key = p0 + acc_row(8 * j + i, h);
-      v[t][i] = f < 4 * VD && key >= lo_key && key < len ? vp[(size_t)key * a.vld + d] : 0.f;
+      v[t][i] = f < 4 * VD && key >= a.lo && key < a.len ? vp[(size_t)key * a.vld + d] : 0.f;
     }
   }
 #pragma unroll
@@ -163,7 +149,6 @@ struct HAttnArgs {
   float2* ml;              // [slot][HA_ROWS] (maximum in bits, sum)
   int group, tile0, tiles, splits, piece;
   float scale;             // times log2(e)
-  const TlHattnItem* pack; // PACKED: the row tiles of several sequences' tokens, each over tiles of its own
 };
 // first position that position i sees
 __host__ __device__ __forceinline__ int first_key(const TlHattn& x, int i) {
@@ -199,29 +184,18 @@ __device__ __forceinline__ void lds_load16(unsigned at, unsigned off, const void
   asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
                : "=&s"(keep) : "s"(at), "v"(off), "s"(base) : "memory");
 }
-// PACKED: a row tile's sequence, tokens and key tiles come from a list, the one with the most keys first (one piece each)
-template <int KD, int VD, bool PACKED>
-__global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs arg) {
+template <int KD, int VD>
+__global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs a) {
   constexpr int DS = KD / 16, DB = VD / 32, TILE = (KD + VD) * 64, NLD = TILE / 8 / 256;
   __shared__ __attribute__((aligned(16))) _Float16 win[2][TILE];
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5, wave = tid >> 6;
   // workgroup L runs on XCD L mod 8: with a multiple of eight kv heads every L2 holds the planes of its own ones; the row
   // tiles with the most keys first
-  HAttnArgs a = arg;
   const int nkv = a.x.kv_heads;
-  const int kvh = blockIdx.x % nkv, slot = blockIdx.x / nkv, split = PACKED ? 0 : slot % a.splits;
-  if (PACKED) {
-    const TlHattnItem it = a.pack[slot];
-    a.x.T = it.T;
-    a.x.start_pos = it.start_pos;
-    a.x.q += (size_t)it.tok0 * a.x.ldq;
-    a.x.out += (size_t)it.tok0 * nkv * a.group * VD;
-    a.tile0 = -it.tile;  // (tile t of the sequence is tile it.tile + t of the list)
-  }
-  const int rows = a.x.T * a.group, nrt = (rows + HA_ROWS - 1) / HA_ROWS;
-  const int rt = PACKED ? a.pack[slot].row_tile : nrt - 1 - slot / a.splits;
+  const int kvh = blockIdx.x % nkv, slot = blockIdx.x / nkv, split = slot % a.splits;
+  const int rows = a.x.T * a.group, nrt = (rows + HA_ROWS - 1) / HA_ROWS, rt = nrt - 1 - slot / a.splits;
   const TileRange range = row_tiles(a.x, a.group, rt);
-  const int nt = range.hi - range.lo, ns = PACKED ? 1 : (nt + a.piece - 1) / a.piece;
+  const int nt = range.hi - range.lo, ns = (nt + a.piece - 1) / a.piece;
   if (split >= ns) return;
   const int t0 = range.lo + (int)((long long)nt * split / ns), t1 = range.lo + (int)((long long)nt * (split + 1) / ns);
   const int row = rt * HA_ROWS + wave * 32 + r;
@@ -493,15 +467,9 @@ int plan_splits(const TlHattn& x, int group, int* piece_out) {
 template <int KD, int VD>
 void launch(const HPlanesArgs& p, const HAttnArgs& a, hipStream_t s) {
   const int rows = a.x.T * a.group, nrt = (rows + HA_ROWS - 1) / HA_ROWS, per = 256 / (VD / 4);
-  kv_planes_kernel<KD, VD, false><<<dim3(p.tiles, p.nkv), 256, 0, s>>>(p);
-  hattn_kernel<KD, VD, false><<<dim3(nrt * a.splits * a.x.kv_heads), 256, 0, s>>>(a);
+  kv_planes_kernel<KD, VD><<<dim3(p.tiles, p.nkv), 256, 0, s>>>(p);
+  hattn_kernel<KD, VD><<<dim3(nrt * a.splits * a.x.kv_heads), 256, 0, s>>>(a);
   if (a.splits > 1) hattn_combine_kernel<VD><<<dim3((rows + per - 1) / per, a.x.kv_heads), 256, 0, s>>>(a);
-}
-
-template <int D>
-void launch_packed(const HPlanesArgs& p, const HAttnArgs& a, int items, hipStream_t s) {
-  kv_planes_kernel<D, D, true><<<dim3(p.tiles, p.nkv), 256, 0, s>>>(p);
-  hattn_kernel<D, D, true><<<dim3(items * a.x.kv_heads), 256, 0, s>>>(a);
 }
 
 }  // namespace
@@ -550,63 +518,6 @@ int tl_launch_hattn(const TlHattn& x, void* ws, size_t ws_bytes, hipStream_t s) 
   else if (x.dim == 128) launch<128, 64>(p, a, s);
   else if (x.dim == 96) launch<96, 64>(p, a, s);
   else launch<64, 64>(p, a, s);
-  TL_HIP(hipGetLastError());
-  return 0;
-}
-
-// The row tiles of a packed batch: runs of consecutive tokens of one sequence at consecutive positions, every one over the keys that
-// its last token sees. Per token (tl_batch.hip) a workgroup reads its sequence's rows again for every token and does its products
-// on the vector units: 77 us a layer for 21 prompts of up to 150 tokens (1650) of the 1.1B shape. Converting every sequence's rows once and
-// walking them 128 (token, head) rows at a time is the same prompt kernel with one more indirection; the whole call 9.8 -> 8.5 ms,
-// 2 prompts of 200 and 400 tokens 6.3 -> 5.2. What a launch costs whatever it does (5 to 8 us a layer, twice the launches) sets the
-// line: with w = workgroups of the per-token kernel for a token, it wins from w / 8 (tokens + keys read / 64) = 170 on with heads of 64
-// and 340 to 440 with heads of 128 (24 prompts of up to 25 tokens 1.05 and 1.00 times as fast, of up to 13 tokens 1.00 and 0.99, of up to 60
-// 1.11 and 1.01 to 1.03). A row tile walks its keys alone, 2 us a tile, so that few tokens over many keys stay with the per-token kernel.
-bool tl_hattn_pack(const int* pos, const int* seq, int T, int group, int kv_heads, int dim, size_t ws_bytes, std::vector<TlHattnTile>* tiles,
-                   std::vector<TlHattnItem>* items) {
-  tiles->clear();
-  items->clear();
-  long long per_token = 0;
-  int most = 0;
-  for (int t0 = 0, t1; t0 < T; t0 = t1) {
-    for (t1 = t0 + 1; t1 < T && seq[t1] == seq[t0] && pos[t1] == pos[t1 - 1] + 1;) ++t1;
-    const int n = t1 - t0, len = pos[t0] + n, kt = (len + 31) / 32, rts = (n * group + HA_ROWS - 1) / HA_ROWS;
-    if (tiles->size() + kt > TL_HATTN_PACK_MAX || items->size() + rts > TL_HATTN_PACK_MAX) return false;
-    for (int rt = 0; rt < rts; ++rt) items->push_back({t0, n, pos[t0], rt, (int)tiles->size(), {0, 0, 0}});
-    for (int k = 0; k < kt; ++k) tiles->push_back({32 * k, len, seq[t0], 0});
-    per_token += (long long)n * (len + pos[t0]) / 2;
-    if (kt > most) most = kt;
-  }
-  const size_t nt = tiles->size();
-  if (plane_bytes((int)nt, kv_heads, dim, dim) + exps_bytes((int)nt, kv_heads) > ws_bytes) return false;
-    const double units = kv_heads * (group == 8 ? 2 : 1) / 8.0;
-  if (units * ((double)T + (double)per_token / 64) < 3.0 * dim || 2.0 * most > 8.0 + 7e-4 * units * (double)per_token) return false;
-  auto keys = [&](const TlHattnItem& i) { return i.start_pos + std::min((i.row_tile * HA_ROWS + HA_ROWS - 1) / group, i.T - 1); };
-  std::stable_sort(items->begin(), items->end(), [&](const TlHattnItem& a, const TlHattnItem& b) { return keys(a) > keys(b); });
-  return true;
-}
-// x: T, start_pos and the caches' first sequence; x.q and x.out hold the whole batch. tiles, items: tl_hattn_pack's, on the device
-int tl_launch_hattn_packed(const TlHattn& x, size_t seq_stride, const TlHattnTile* tiles_dev, int tiles, const TlHattnItem* items_dev, int items,
-                           void* ws, size_t ws_bytes, hipStream_t s) {
-  TL_REQUIRE(tl_hattn_supported(x) && x.dim == x.vdim && tiles > 0 && items > 0 && tiles <= TL_HATTN_PACK_MAX && items <= TL_HATTN_PACK_MAX &&
-                 x.window == 0 && x.chunk == 0 && !x.sink && !x.gate && (seq_stride & 3) == 0, "tl_launch_hattn_packed: unsupported shapes");
-  const size_t planes = plane_bytes(tiles, x.kv_heads, x.dim, x.vdim);
-  TL_REQUIRE(ws && ws_bytes >= planes + exps_bytes(tiles, x.kv_heads), "tl_launch_hattn_packed: workspace too small");
-  unsigned char* w = static_cast<unsigned char*>(ws);
-  HPlanesArgs p = {x.kc, x.vc, x.kld, x.khs, x.vld, 0, 0, x.kv_heads, 0, tiles, reinterpret_cast<_Float16*>(w), reinterpret_cast<int*>(w + planes)};
-  p.pack = tiles_dev;
-  p.seq_stride = seq_stride;
-  HAttnArgs a = {};
-  a.x = x;
-  a.planes = p.planes;
-  a.exps = p.exps;
-  a.group = x.heads / x.kv_heads;
-  a.tiles = tiles;
-  a.splits = 1;
-  a.scale = x.scale * LOG2E;
-  a.pack = items_dev;
-  if (x.dim == 128) launch_packed<128>(p, a, items, s);
-  else launch_packed<64>(p, a, items, s);
   TL_HIP(hipGetLastError());
   return 0;
 }

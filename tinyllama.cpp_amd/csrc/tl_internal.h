@@ -302,21 +302,17 @@ struct TlHattn {
 bool tl_hattn_supported(const TlHattn& x);
 size_t tl_hattn_bytes(int max_keys, int kv_heads, int dim, int vdim);
 int tl_launch_hattn(const TlHattn& x, void* ws, size_t ws_bytes, hipStream_t s);
-// the same for a packed batch of several sequences' tokens, whose caches lie seq_stride floats apart
-struct TlHattnTile {  // 32 positions from pos on of a sequence of len rows
-  int pos, len, seq, pad;
-};
-struct TlHattnItem {  // 128 rows (token, head) of the run of T tokens tok0 .. at positions start_pos ..; tile: its first key tile in the list
-  int tok0, T, start_pos, row_tile, tile, pad[3];
-};
-constexpr int TL_HATTN_PACK_MAX = 4096;  // tiles, and row tiles, of a launch
-// false: the per-token kernel serves this batch better, or the tiles do not fit the workspace
-bool tl_hattn_pack(const int* pos, const int* seq, int T, int group, int kv_heads, int dim, size_t ws_bytes, std::vector<TlHattnTile>* tiles,
-                   std::vector<TlHattnItem>* items);
-int tl_launch_hattn_packed(const TlHattn& x, size_t seq_stride, const TlHattnTile* tiles_dev, int tiles, const TlHattnItem* items_dev, int items,
-                           void* ws, size_t ws_bytes, hipStream_t s);
 // causal prefill attention on the FP32 matrix instruction (tl_prefill.hip)
 bool tl_attn_prefill_mfma_supported(int nh, int nkv, int hd);
+// ... of a packed batch of several sequences' tokens, whose caches lie seq_stride floats apart
+struct TlAttnItem {  // 32 rows (token, head of a kv head) of the run of T tokens tok0 .. of sequence seq at positions start_pos ..
+  int tok0, T, start_pos, seq, row_tile, pad[3];
+};
+constexpr int TL_ATTN_PACK_MAX = 4096;  // items of a launch
+// false: too many, or (unless `always`) the per-token kernel serves this batch better
+bool tl_attn_pack(const int* pos, const int* seq, int T, int nh, int nkv, int hd, bool always, std::vector<TlAttnItem>* items);
+int tl_launch_attn_packed(const float* q, const float* kc, const float* vc, float* out, size_t seq_stride, const TlAttnItem* items_dev, int items,
+                          int nh, int nkv, int hd, float scale, hipStream_t s);
 // planes != NULL: the output as the attn_output GEMM's activation planes (tl_launch_split's layout) instead of `out`
 int tl_launch_attn_prefill_mfma(const float* q, const float* kc, const float* vc, float* out, int T, int start_pos,
                                 int nh, int nkv, int hd, float scale, hipStream_t s, void* planes = nullptr,

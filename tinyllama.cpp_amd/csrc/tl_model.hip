@@ -128,7 +128,8 @@ struct tl_model {
     int max_batch = 0;
     float* kv = nullptr;
     int *toks = nullptr, *pos = nullptr, *seq = nullptr;  // [max_batch]
-    void* pack = nullptr;                                 // [TL_HATTN_PACK_MAX] key tiles, then row tiles of a packed chunk's attention
+    TlAttnItem* pack = nullptr;                           // [TL_ATTN_PACK_MAX] row tiles of a packed chunk's attention
+    std::vector<std::vector<TlAttnItem>> packs;           // ... of a call's chunks, on the host until their copies are through
     float* last_h = nullptr;                              // [max_batch][hidden]: hidden rows whose logits a packed prefill returns
     int* ids = nullptr;                                   // generated ids [step][n]
     size_t ids_cap = 0;
@@ -1739,11 +1740,8 @@ extern "C" int tl_tp_local_group_prefill(tl_model* const* ms, int n, const int* 
 // more GEMM, and a per-row arg-max writes the next token ids and advances the positions on the device, so that a greedy
 // generation loop needs no host round trip per step. Every sequence decodes exactly as it would alone (see tl_batch.hip
 // on the reference's history_len quirk). tp_size 1 only.
-struct BatchPack {  // a packed chunk's attention by row tiles (tl_hattn.hip); no tiles: token by token
-  std::vector<TlHattnTile> tiles;
-  std::vector<TlHattnItem> items;
-};
-static int batch_attn_half(tl_model* m, int l, int T, const BatchPack* pack, hipStream_t s) {
+// packed: that many row tiles of a packed chunk in bt.pack (0: token by token)
+static int batch_attn_half(tl_model* m, int l, int T, int packed, hipStream_t s) {
   const tl_model_config& c = m->cfg;
   tl_model::Prefill& p = m->pf;
   LayerW& L = m->layers[l];
@@ -1760,10 +1758,8 @@ static int batch_attn_half(tl_model* m, int l, int T, const BatchPack* pack, hip
   // the attention output goes straight into the planes of the attn_output GEMM (no split launch; TL_ATTN_PLANES=0 keeps
   // the launch, for A/B runs and the bit-identity test)
   const char* ap = getenv("TL_ATTN_PLANES");
-  if (pack && !pack->items.empty()) {
-    const TlHattnTile* tiles = static_cast<const TlHattnTile*>(m->bt.pack);
-    TL_TRY(tl_launch_hattn_packed(half_attn(m, m->bkc(l), m->bvc(l), T, 0), m->kv_layer_elems, tiles, (int)pack->tiles.size(),
-                                  reinterpret_cast<const TlHattnItem*>(tiles + TL_HATTN_PACK_MAX), (int)pack->items.size(), p.hattn, p.hattn_bytes, s));
+  if (packed) {
+    TL_TRY(tl_launch_attn_packed(p.qb, m->bkc(l), m->bvc(l), p.ab, m->kv_layer_elems, m->bt.pack, packed, m->nh_l, m->nkv_l, hd, scale, s));
     TL_TRY(tl_launch_split(0, p.ab, nullptr, p.planes, ps, T, m->qd_l, terms, 0.f, s));
   } else if (terms == TL_TERMS_HALF || (ap && atoi(ap) == 0)) {
     TL_TRY(tl_launch_batch_attn(p.qb, m->bkc(l), m->bvc(l), m->kv_layer_elems, p.ab, m->bt.pos, m->bt.seq, T, m->nh_l,
@@ -1863,12 +1859,12 @@ static int batch_layers_gemv(tl_model* m, int T, hipStream_t s) {
 // one step for the T tokens in bt.toks / bt.pos / bt.seq; ids_dev: [T] next ids (first maximum of each logits row);
 // advance: the ids become the next tokens and the positions move on (device-resident loop)
 // all layers for the T tokens in bt.toks / bt.pos / bt.seq: the residual stream ends up in pf.xb [T][hidden]
-static int batch_layers(tl_model* m, int T, hipStream_t s, const BatchPack* pack = nullptr) {
+static int batch_layers(tl_model* m, int T, hipStream_t s, int packed = 0) {
   TL_REQUIRE(T >= 1 && T <= m->pf.cap, "tl_model: a batched step of %d tokens exceeds the chunk workspaces (%d)", T, m->pf.cap);
   if (T <= m->bt.gemv_max) return batch_layers_gemv(m, T, s);
   TL_TRY(prefill_embed(m, m->bt.toks, T, s));
   for (int l = 0; l < m->cfg.num_hidden_layers; ++l) {
-    TL_TRY(batch_attn_half(m, l, T, pack, s));
+    TL_TRY(batch_attn_half(m, l, T, packed, s));
     TL_TRY(prefill_mlp_half(m, l, T, s));
   }
   return flush_residual(m, s);
@@ -1984,7 +1980,7 @@ extern "C" int tl_model_batch_init(tl_model* m, int max_batch) {
   TL_HIP(hipMalloc(&b.toks, sizeof(int) * kPrefillChunk));  // a packed prompt chunk carries up to kPrefillChunk tokens
   TL_HIP(hipMalloc(&b.pos, sizeof(int) * kPrefillChunk));
   TL_HIP(hipMalloc(&b.seq, sizeof(int) * kPrefillChunk));
-  TL_HIP(hipMalloc(&b.pack, (sizeof(TlHattnTile) + sizeof(TlHattnItem)) * TL_HATTN_PACK_MAX));
+  TL_HIP(hipMalloc(&b.pack, sizeof(TlAttnItem) * TL_ATTN_PACK_MAX));
   TL_HIP(hipMalloc(&b.last_h, sizeof(float) * (size_t)max_batch * m->cfg.hidden_size));
   if (sizeof(float) * (size_t)max_batch * m->cfg.vocab_size >= kCopySpread) {
     hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&b.stage), 2 * kCopyThreads * kCopyPiece, hipHostMallocDefault);
@@ -2079,22 +2075,25 @@ extern "C" int tl_model_batch_prefill_packed(tl_model* m, int n_tokens, const in
   const size_t H = c.hidden_size;
   const int chunk = chunk_tokens(m);
   TL_REQUIRE(chunk >= 1 && chunk <= kPrefillChunk, "tl_model_batch_prefill_packed: workspaces are missing");
-  const bool half = chunk_terms(m) == TL_TERMS_HALF && half_attn_on() && tl_hattn_supported(half_attn(m, m->bkc(0), m->bvc(0), 1, 0));
-  if (half) TL_TRY(half_attn_ws(m));
-  std::vector<BatchPack> packs((n_tokens + chunk - 1) / chunk);  // (live until the stream has been waited for)
+  const char* ha = getenv("TL_HATTN");  // 0: every chunk token by token, any other number: by row tiles (A/B runs and tests)
+  const bool always = ha && atoi(ha) != 0;
+  const bool tiles = chunk_terms(m) == TL_TERMS_HALF && tl_attn_prefill_mfma_supported(m->nh_l, m->nkv_l, m->head_dim) && (always || !ha);
   for (int c0 = 0; c0 < n_tokens; c0 += chunk) {
     const int T = n_tokens - c0 < chunk ? n_tokens - c0 : chunk;
-    BatchPack& pack = packs[c0 / chunk];
-    if (half && T > m->bt.gemv_max &&
-        tl_hattn_pack(positions_host + c0, seq_idx_host + c0, T, m->nh_l / m->nkv_l, m->nkv_l, m->head_dim, m->pf.hattn_bytes, &pack.tiles, &pack.items)) {
-      TlHattnTile* tiles = static_cast<TlHattnTile*>(m->bt.pack);
-      TL_HIP(hipMemcpyAsync(tiles, pack.tiles.data(), sizeof(TlHattnTile) * pack.tiles.size(), hipMemcpyHostToDevice, s));
-      TL_HIP(hipMemcpyAsync(tiles + TL_HATTN_PACK_MAX, pack.items.data(), sizeof(TlHattnItem) * pack.items.size(), hipMemcpyHostToDevice, s));
-    } else pack.items.clear();
+    int packed = 0;
+    if (tiles && T > m->bt.gemv_max) {
+      try {
+        if (m->bt.packs.size() <= (size_t)(c0 / chunk)) m->bt.packs.resize(c0 / chunk + 1);
+        std::vector<TlAttnItem>& items = m->bt.packs[c0 / chunk];
+        if (tl_attn_pack(positions_host + c0, seq_idx_host + c0, T, m->nh_l, m->nkv_l, m->head_dim, always, &items)) packed = (int)items.size();
+      } catch (const std::bad_alloc&) {  // (no memory for the list: token by token)
+      }
+      if (packed) TL_HIP(hipMemcpyAsync(m->bt.pack, m->bt.packs[c0 / chunk].data(), sizeof(TlAttnItem) * packed, hipMemcpyHostToDevice, s));
+    }
     TL_HIP(hipMemcpyAsync(m->bt.toks, tokens_host + c0, sizeof(int) * T, hipMemcpyHostToDevice, s));
     TL_HIP(hipMemcpyAsync(m->bt.pos, positions_host + c0, sizeof(int) * T, hipMemcpyHostToDevice, s));
     TL_HIP(hipMemcpyAsync(m->bt.seq, seq_idx_host + c0, sizeof(int) * T, hipMemcpyHostToDevice, s));
-    TL_TRY(batch_layers(m, T, s, &pack));
+    TL_TRY(batch_layers(m, T, s, packed));
     for (int j = 0; j < n_last; ++j) {
       const int r = last_rows_host[j] - c0;
       if (r >= 0 && r < T)

@@ -25,6 +25,9 @@
 // merge with four exps per output element.
 #include <math.h>
 
+#include <algorithm>
+#include <vector>
+
 #include "tl_internal.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -341,6 +344,165 @@ __global__ __launch_bounds__(64 * PF_NW) void attn_prefill_mfma_kernel(const flo
   }
 }
 
+struct PackArgs {
+  const float *q, *kc, *vc;  // q, out: [T][nh][64 NW], caches: sequence 0's
+  float* out;
+  size_t seq_stride;
+  const TlAttnItem* items;   // the ones with the most keys first
+  int group, nkv;
+  float scale;
+};
+// Runs of a packed batch: 32 rows (token, head of a kv head) a workgroup, one wave for 64 columns of the heads: of the queries and keys,
+// whose parts of the scores meet in LDS, and of the values and outputs. Per token (tl_batch.hip) a workgroup reads its sequence's rows again
+// for every token and multiplies on the vector units: 21 runs of 78 tokens, 32 heads of 64 over 4 96 us, here 21; 24 of 128 over 8 85 and 32,
+// 64 runs of 16 tokens 60 and 9. A tile of 32 keys is 64 products of 64 cycles in 3.7 us: the chain of a wave (keys, softmax, values).
+// No bit is given up for it: the products are FP32's, scores are sums of eight columns met in a tree (one chain over the columns is
+// 1.3 to 1.7 times as far off 64 bits as the per-token kernel, this 0.93 to 1.02 times), a tile's values have sums of their own.
+// A value that is not finite counts where it is visible, behind the sums: in them a weight of zero would not undo it.
+template <int NW>
+__global__ __launch_bounds__(64 * NW, 2) void attn_pack_kernel(const PackArgs a) {
+  constexpr int HD = 64 * NW, LDQ = 68;
+  __shared__ __attribute__((aligned(16))) float sm_q[NW][32 * LDQ];
+  __shared__ __attribute__((aligned(16))) float sm_s[2][NW][NW > 1 ? 4 : 1][64][4];
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kvh = blockIdx.x % a.nkv;
+  const TlAttnItem it = a.items[blockIdx.x / a.nkv];
+  const int rows = it.T * a.group, nh = a.nkv * a.group, kv_dim = a.nkv * HD, row0 = it.row_tile * 32;
+  const int row = row0 + r < rows ? row0 + r : rows - 1, rq = row / a.group;
+  const int qpos = it.start_pos + rq, off = ((it.tok0 + rq) * nh + kvh * a.group + row - rq * a.group) * HD + 64 * wave;
+  const int first = it.start_pos + row0 / a.group, last = it.start_pos + min(row0 + 31, rows - 1) / a.group;
+  const int ntile = last / 32 + 1;
+  const float* kb = a.kc + (size_t)it.seq * a.seq_stride + (size_t)kvh * HD + 64 * wave + 4 * h;
+  const float* vb = a.vc + (size_t)it.seq * a.seq_stride + (size_t)kvh * HD + 64 * wave + r;
+  float* qs = sm_q[wave] + r * LDQ + 4 * h;  // (a lane reads what it writes)
+#pragma unroll
+  for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(qs + 8 * i) = *reinterpret_cast<const f32x4*>(a.q + off + 4 * h + 8 * i);
+  f32x4 kreg[8];
+  auto load_k = [&](int tile) __attribute__((always_inline)) {
+    const int p = tile * 32 + r;
+    const float* kp = kb + (size_t)(p < last ? p : last) * kv_dim;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) kreg[i] = *reinterpret_cast<const f32x4*>(kp + 8 * i);
+  };
+  load_k(0);
+  f32x16 o[2];
+  float bad[2] = {0.f, 0.f};  // what a column's values hold that is not finite, and from which position on
+  int bad_at[2] = {0x7fffffff, 0x7fffffff};
+#pragma unroll
+  for (int e = 0; e < 16; ++e) o[0][e] = o[1][e] = 0.f;
+  float mrun = -INFINITY, lrun = 0.f;
+  for (int t = 0; t < ntile; ++t) {
+    const int p0 = t * 32;
+    f32x16 s;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      f32x16 c[4];
+      f32x4 qv[4];
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        qv[n] = *reinterpret_cast<const f32x4*>(qs + 8 * (4 * j + n));
+#pragma unroll
+        for (int e = 0; e < 16; ++e) c[n][e] = 0.f;
+      }
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int n = 0; n < 4; ++n) c[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(kreg[4 * j + n][m], qv[n][m], c[n], 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float x = (c[0][e] + c[1][e]) + (c[2][e] + c[3][e]);
+        s[e] = j ? s[e] + x : x;
+      }
+    }
+    if (t + 1 < ntile) load_k(t + 1);
+    float v[16];
+    auto load_v = [&](int e, int b) __attribute__((always_inline)) {
+      const int p = p0 + acc_row(e, h);
+      v[e] = vb[(size_t)(p < last ? p : last) * kv_dim + 32 * b];
+    };
+#pragma unroll
+    for (int e = 0; e < 16; ++e) load_v(e, 0);
+    if (NW > 1) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) *reinterpret_cast<f32x4*>(sm_s[t & 1][wave][i][lane]) = f32x4{s[4 * i], s[4 * i + 1], s[4 * i + 2], s[4 * i + 3]};
+      __syncthreads();  // (a wave is at most a tile ahead: the other buffer)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(sm_s[t & 1][NW - 1 - wave][i][lane]);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) s[4 * i + c] += x[c];
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float tmax = -INFINITY;
+    if (p0 + 31 > first) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s[e] = p0 + acc_row(e, h) <= qpos ? s[e] * a.scale : -INFINITY;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s[e] *= a.scale;
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) tmax = fmaxf(tmax, s[e]);
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+    const float mnew = fmaxf(mrun, tmax);
+    const float corr = mrun == -INFINITY ? 0.f : expf(mrun - mnew);
+    mrun = mnew;
+    float ps[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      s[e] = s[e] == -INFINITY ? 0.f : expf(s[e] - mnew);
+      ps[e & 3] += s[e];
+    }
+    lrun = lrun * corr + ((ps[0] + ps[1]) + (ps[2] + ps[3]));
+    float cr[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) cr[e] = __shfl(corr, acc_row(e, h));
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      f32x16 u[2];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) u[0][e] = u[1][e] = 0.f;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        float x = v[e];
+        if (!(fabsf(x) < INFINITY)) {
+          const int p = p0 + acc_row(e, h);
+          bad[b] += x;
+          bad_at[b] = min(bad_at[b], min(p, last));
+          x = 0.f;
+        }
+        u[e & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(s[e], x, u[e & 1], 0, 0, 0);
+        if (b == 0) load_v(e, 1);
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) o[b][e] = fmaf(o[b][e], cr[e], u[0][e] + u[1][e]);
+    }
+  }
+  const float inv = 1.0f / (lrun + __shfl_xor(lrun, 32) + 1e-9f);
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const int at = min(bad_at[b], __shfl_xor(bad_at[b], 32));
+    if (__any(at != 0x7fffffff)) {
+      const float x = bad[b] + __shfl_xor(bad[b], 32);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int seen = it.start_pos + min(row0 + acc_row(e, h), rows - 1) / a.group;
+        o[b][e] += at <= seen ? x : 0.f;
+      }
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const int rr = acc_row(e, h), to = __shfl(off, rr);
+    const float f = __shfl(inv, rr);
+    if (row0 + rr < rows) {
+      a.out[(size_t)to + r] = o[0][e] * f;
+      a.out[(size_t)to + 32 + r] = o[1][e] * f;
+    }
+  }
+}
+
 }  // namespace
 
 #ifdef TL_PF_STAMP
@@ -382,4 +544,69 @@ int tl_launch_attn_prefill_mfma(const float* q, const float* kc, const float* vc
   }
   TL_HIP(hipGetLastError());
   return 0;
+}
+
+// Runs of consecutive tokens of one sequence at consecutive positions, cut into row tiles. The rule compares what both kernels take,
+// in us, fitted to 34 batches of 1 to 64 runs of 1 to 2000 tokens behind 0 to 2000 others, for six head shapes (32/4 and 16/2 and 16/16 heads
+// of 64, 24/8, 32/8 and 8/1 of 128), within 0.6 to 1.4 of the measured times: per token, every head pays for a token and for a key; by tiles,
+// the longest chain of one workgroup or the chip's products, whichever is longer (two waves a workgroup: beyond one workgroup a
+// CU the chain is 1.6 times as long). Taken where it promises a tenth: none of the 204 cases lost (8 x 40 tokens 21.1 / 10.8 us, 30 x 3
+// behind 700 40 / 84, one run of 500 75 / 61).
+bool tl_attn_pack(const int* pos, const int* seq, int T, int nh, int nkv, int hd, bool always, std::vector<TlAttnItem>* items) {
+  const int group = nh / nkv;
+  items->clear();
+  double keys = 0.0, walk = 0.0;
+  int most = 0;
+  auto tiles = [&](const TlAttnItem& i) { return (i.start_pos + std::min(i.row_tile * 32 + 31, i.T * group - 1) / group) / 32 + 1; };
+  for (int t0 = 0, t1; t0 < T; t0 = t1) {
+    for (t1 = t0 + 1; t1 < T && seq[t1] == seq[t0] && pos[t1] == pos[t1 - 1] + 1;) ++t1;
+    const int n = t1 - t0, row_tiles = (n * group + 31) / 32;
+    if (items->size() + row_tiles > (size_t)TL_ATTN_PACK_MAX) return false;
+    for (int rt = 0; rt < row_tiles; ++rt) {
+      items->push_back({t0, n, pos[t0], seq[t0], rt, {0, 0, 0}});
+      const int kt = tiles(items->back());
+      walk += kt;
+      most = std::max(most, kt);
+    }
+    keys += n * (pos[t0] + 0.5 * (n + 1));
+  }
+  if (!always) {
+    const double per_token = 3.5 + nh * (0.0014 * T + (hd == 64 ? 1.3e-5 : 1.8e-5) * keys);
+    const double chain = most * (hd == 64 ? 3.7 : 4.0 * ((double)items->size() * nkv > tl_num_cus() ? 1.6 : 1.0));
+    const double by_tiles = 4.0 + std::max(chain, (0.0042 * walk + 0.003 * items->size()) * nkv * hd / 64);
+    if (by_tiles > 0.9 * per_token) return false;
+  }
+  std::stable_sort(items->begin(), items->end(), [&](const TlAttnItem& a, const TlAttnItem& b) { return tiles(a) > tiles(b); });
+  return true;
+}
+// q, out [T][nh][hd], kc, vc: sequence 0's caches [max_seq][nkv][hd] of the layer, which hold every position of the items; items_dev:
+// tl_attn_pack's, on the device
+int tl_launch_attn_packed(const float* q, const float* kc, const float* vc, float* out, size_t seq_stride, const TlAttnItem* items_dev, int items,
+                          int nh, int nkv, int hd, float scale, hipStream_t s) {
+  TL_REQUIRE(tl_attn_prefill_mfma_supported(nh, nkv, hd) && q && kc && vc && out && items_dev && items > 0 && items <= TL_ATTN_PACK_MAX &&
+                 (seq_stride & 3) == 0 && (((size_t)q | (size_t)kc | (size_t)vc | (size_t)out) & 15) == 0,
+             "tl_launch_attn_packed: unsupported shapes");
+  const PackArgs a = {q, kc, vc, out, seq_stride, items_dev, nh / nkv, nkv, scale};
+  if (hd == 64) attn_pack_kernel<1><<<items * nkv, 64, 0, s>>>(a);
+  else attn_pack_kernel<2><<<items * nkv, 128, 0, s>>>(a);
+  TL_HIP(hipGetLastError());
+  return 0;
+}
+
+// Test hook (tlhip_debug.h): the kernel above over a batch, whatever the rule says of it
+extern "C" int tl_debug_packed_attention(const float* q_dev, const float* k_cache_dev, const float* v_cache_dev, float* out_dev, long long seq_stride,
+                                         const int* positions_host, const int* seq_idx_host, int num_tokens, int heads, int kv_heads, int dim,
+                                         float scale, void* stream) {
+  TL_REQUIRE(positions_host && seq_idx_host && num_tokens > 0 && seq_stride > 0 && tl_attn_prefill_mfma_supported(heads, kv_heads, dim),
+             "tl_debug_packed_attention: bad argument");
+  std::vector<TlAttnItem> items;
+  TL_REQUIRE(tl_attn_pack(positions_host, seq_idx_host, num_tokens, heads, kv_heads, dim, true, &items), "tl_debug_packed_attention: too many row tiles");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  TlAttnItem* dev = nullptr;
+  TL_HIP(hipMalloc(&dev, sizeof(TlAttnItem) * items.size()));
+  TL_HIP(hipMemcpyAsync(dev, items.data(), sizeof(TlAttnItem) * items.size(), hipMemcpyHostToDevice, s));
+  const int rc = tl_launch_attn_packed(q_dev, k_cache_dev, v_cache_dev, out_dev, (size_t)seq_stride, dev, (int)items.size(), heads, kv_heads, dim, scale, s);
+  TL_HIP(hipStreamSynchronize(s));
+  TL_HIP(hipFree(dev));
+  return rc;
 }
