@@ -455,3 +455,36 @@ def test_packed_attention_kernel(pkg, heads, kv_heads, hd):
     odd[np.ix_(sees, np.arange(group), [3])] = got[np.ix_(sees, np.arange(group), [3])]
     odd[np.ix_(sees, np.arange(heads - group, heads), [hd - 2])] = got[np.ix_(sees, np.arange(heads - group, heads), [hd - 2])]
     assert np.array_equal(odd, got)
+
+
+def test_many_logits_into_memory_that_the_runtime_knows(pkg):
+    """Logits of 4 MB and more into pinned memory, a device's memory and ordinary memory: what the runtime knows it copies to itself (no
+    thread of the host could write a device's), and every destination holds the same."""
+    import ctypes as C
+    from tinyllama_cpp_amd import engine as E
+    from tinyllama_cpp_amd.capi import check, lib
+    E.init(0)
+    cfg, tensors = pkg.synth.build_model(dict(pkg.synth.SHAPES["tiny-gqa"], vocab=50003, n_layers=1), "q4_k_m", seed=6)
+    m = E.Model(cfg).load(tensors)
+    m.batch_init(24)
+    n = 24
+    toks = np.random.default_rng(1).integers(0, cfg["vocab"], n).astype(np.int32)
+    pos, seq, nxt = np.zeros(n, np.int32), np.arange(n, dtype=np.int32), np.zeros(n, np.int32)
+    want, ids = m.batch_decode(toks, pos, seq)
+    hip = C.CDLL("libamdhip64.so")
+    pinned = C.c_void_p()
+    assert hip.hipHostMalloc(C.byref(pinned), C.c_size_t(want.nbytes), 0) == 0
+    on_device = E.DeviceBuffer(want.nbytes)
+
+    def step(dst):
+        nxt[:] = -1
+        check(lib().tl_model_batch_decode(m.h, n, toks.ctypes.data, pos.ctypes.data, seq.ctypes.data, dst, nxt.ctypes.data), "tl_model_batch_decode")
+        assert np.array_equal(nxt, ids)
+
+    C.memset(pinned.value, 0xff, want.nbytes)
+    step(pinned.value)
+    assert np.array_equal(np.ctypeslib.as_array(C.cast(pinned, C.POINTER(C.c_float)), want.shape), want)
+    step(on_device.ptr)
+    assert np.array_equal(on_device.to_numpy(np.float32, want.shape), want)
+    assert hip.hipHostFree(pinned) == 0
+    m.free()

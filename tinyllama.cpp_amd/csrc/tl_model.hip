@@ -1895,7 +1895,10 @@ static int batch_head(tl_model* m, const float* hidden, int R, hipStream_t s) {
 // device while the other is copied out. Up to kCopySpread bytes: the runtime's own copy, complete when the stream is waited for.
 static int copy_to_caller(tl_model* m, float* dst, const float* src, size_t bytes, hipStream_t s) {
   tl_model::Batch& b = m->bt;
-  if (!b.stage || bytes < kCopySpread) {
+  hipPointerAttribute_t at = {};  // memory that the runtime knows (pinned, managed, a device's) it copies to directly
+  const bool known = hipPointerGetAttributes(&at, dst) == hipSuccess && at.type != hipMemoryTypeUnregistered;
+  if (!known) (void)hipGetLastError();
+  if (!b.stage || bytes < kCopySpread || known) {
     TL_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
     return 0;
   }
@@ -1987,6 +1990,9 @@ extern "C" int tl_model_batch_init(tl_model* m, int max_batch) {
     if (e != hipSuccess) b.stage = nullptr;
     for (hipEvent_t& ev : b.staged)
       if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    for (hipEvent_t& ev : b.staged)  // (pages and events in use once: the first step's copy is as fast as any)
+      if (e == hipSuccess) e = hipEventRecord(ev, m->stream);
+    if (e == hipSuccess) memset(b.stage, 0, 2 * kCopyThreads * kCopyPiece);
     if (e != hipSuccess) {  // (no pinned memory to be had: the runtime's own copies)
       batch_unstage(b);
       (void)hipGetLastError();
