@@ -424,9 +424,10 @@ def test_half_plane_gemm_shapes(E, pkg, shape, name, rows, cols, T, slices):
 
 
 @pytest.mark.parametrize("shape", [2, 3, 4])
-@pytest.mark.parametrize("T", [512, 513, 1050])
+@pytest.mark.parametrize("T", [512, 513, 1024, 1050, 1500])
 def test_half_plane_gemm_panels_of_token_tiles(E, pkg, shape, T):
-    """Workgroups walk panels of eight 64-token tiles: whole panels, a last panel of one tile, several row tiles and K slices. Every
+    """Workgroups walk panels of 64-token tiles: one panel (8 and 9 tiles), equal ones (16), a last one that is narrower, several row
+    tiles and K slices. Every
     token's row equals, to the bit, that of a launch of 64 tokens."""
     from tinyllama_cpp_amd.capi import check, lib
     S, rows, cols = pkg.synth, 520, 512

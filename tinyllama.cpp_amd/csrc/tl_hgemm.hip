@@ -200,7 +200,7 @@ struct HSegs {  // up to three matrices over the same activations (q | k | v, ga
 // super-block's block sums and powers of two.
 template <int TYPE, int TK, int NI, int MI, int NW, int WPE>
 __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct act, const float* __restrict__ resid, int T, int mtiles,
-                                                           int ntiles, int nslices) {
+                                                           int ntiles, int nslices, int panel) {
   typedef Tile<TK> TL;
   typedef typename TL::Acc Acc;
   constexpr int NG = 64 / TK, US = 8 / NG;                        // lane groups, steps of a super-block
@@ -211,22 +211,21 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
   constexpr bool CHUNKED = TYPE == TL_Q4_K || TYPE == TL_Q6_K;
   constexpr bool RINGED = BN > 32;                                // the tile goes through a ring of three 64-column steps
   extern __shared__ __attribute__((aligned(16))) _Float16 hlds[];
-  // consecutive workgroups go to the 8 XCDs in turn: each XCD walks a contiguous range, panels of 8 token tiles one after another
+  // consecutive workgroups go to the 8 XCDs in turn: each XCD walks a contiguous range, panels of `panel` token tiles one after another
   // and inside a panel token tiles fastest. The workgroups that read the same weights thereby share an L2, and the 32 or 64 that an
   // XCD runs at a time read 8 token tiles' activations and 4 or 8 row tiles' weights; with all token tiles side by side, 2048 tokens
   // (32 tiles, 32 MB of activations a round) fetched three times as much through the fabric, which costs time and clock: 28672 x 4096
   // in Q4_K times 2048 tokens 986 -> 967 us in shape 3 and 1200 -> 1116 in shape 4, 16384 x 3072 in Q6_K 682 -> 648.
-  constexpr int PANEL = 8;
   const int total = mtiles * ntiles * nslices, per8 = total >> 3, rem8 = total & 7;
   const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
   const int v = xcd * per8 + (xcd < rem8 ? xcd : rem8) + at;
   const int slice = v / (mtiles * ntiles), in_slice = v - slice * mtiles * ntiles;
   int nt = 0, mt = in_slice;
   if (ntiles > 1) {  // (one tile of tokens: launches of 6 us, which need none of these divisions)
-    const int panel = in_slice / (PANEL * mtiles), in_panel = in_slice - panel * PANEL * mtiles;
-    const int width = ntiles - PANEL * panel < PANEL ? ntiles - PANEL * panel : PANEL;
+    const int pi = in_slice / (panel * mtiles), in_panel = in_slice - pi * panel * mtiles;
+    const int width = ntiles - panel * pi < panel ? ntiles - panel * pi : panel;
     mt = in_panel / width;
-    nt = PANEL * panel + in_panel - mt * width;
+    nt = panel * pi + in_panel - mt * width;
   }
   const int seg = (mt >= segs.mt_end[0]) + (mt >= segs.mt_end[1]);
   if (seg) mt -= segs.mt_end[seg - 1];
@@ -659,7 +658,7 @@ struct HShape {
   int tk, ni, mi, nw, wpe, percu;
 };
 constexpr HShape SHAPE[] = {{16, 1, 1, 4, 4, 4}, {32, 1, 1, 4, 2, 2}, {32, 2, 1, 8, 2, 1}, {32, 2, 2, 4, 2, 2}, {32, 2, 1, 4, 2, 2}};
-// us of a super-block of a workgroup on a full chip (measured)
+// us of a super-block of a workgroup on a full chip (measured before the panels, which made long prompts 2 to 7 % cheaper)
 constexpr float HGEMM_US[] = {1.2f, 2.0f, 4.9f, 9.0f, 5.0f};
 // Price of a launch of n workgroups of `per` super-blocks, and of S slices' partial sums of `outputs` numbers.
 // Q4_K and Q8_K, and all formats up to 64 tokens: rounds over the chip x (super-blocks + start and end) + the partial sums written
@@ -718,8 +717,10 @@ int hgemm_go(const HSegs& g, int mt, const HAct& act, const float* resid, int T,
   static TlDeviceOnce lds_raised;
   auto kernel = hgemm_kernel<TYPE, q.tk, q.ni, q.mi, q.nw, q.wpe>;
   TL_TRY(tl_raise_lds_limit(kernel, (int)lds, lds_raised));
-  const int ntiles = (T + BN - 1) / BN;
-  kernel<<<dim3((unsigned)(mt * ntiles * S)), dim3(64 * q.nw), lds, s>>>(g, act, resid, T, mt, ntiles, S);
+  // panels of eight token tiles and more, all alike: a panel of the one tile that is left over reads all weights again for it (28672 x
+  // 4096 in Q4_K times 513 tokens, nine tiles, 274 us in one panel of shape 3, 281 in eight and one)
+  const int ntiles = (T + BN - 1) / BN, panels = ntiles < 16 ? 1 : ntiles / 8, panel = (ntiles + panels - 1) / panels;
+  kernel<<<dim3((unsigned)(mt * ntiles * S)), dim3(64 * q.nw), lds, s>>>(g, act, resid, T, mt, ntiles, S, panel);
   TL_HIP(hipGetLastError());
   return 0;
 }
