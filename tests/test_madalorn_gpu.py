@@ -612,3 +612,21 @@ def test_configurations_drawn_at_random(env, seed, tmp_path):
 def json_of(cfg):
     import json
     return json.dumps(cfg)
+
+
+def test_large_products_give_the_same_bits_from_a_plane(env, monkeypatch):
+    """1024 wide, 1100 tokens in bf16 mode: gated units, shared experts, activated first products and the soft-capped head take the kernel
+    that reads its items from a bf16 plane; with the kernel that converts them itself every logit is the same to the bit."""
+    S = env["synth"]
+    A, D, M, L = S.madalorn_attention, S.madalorn_delta, S.madalorn_moe, S.madalorn_layer
+    cfg = S.madalorn_config(1024, 5000, [L("attention", A(16, 4, 64, window=300, keep_first=4, rot_dims=64), {"kind": "dense", "ff": 4096}),
+                                         L("channel_delta", D(16, 16, 64, 64, conv=4), M(8, 2, 64, shared_ff=4096, groups=2, keep=1))], softcap=7.0)
+    m, _, _ = make(env, cfg, seed=4, max_pos=1100, exact=False)
+    toks = np.random.default_rng(8).integers(0, cfg["vocab"], 1100).astype(np.int32)
+    taken = env["capi"].lib().tl_debug_dense_plane_taken  # (256 compute units; the plane holds 2048 tokens)
+    assert all(taken(rows, 1024, 1100, 2080 * 4096, 256) == 1 for rows in (8192, 5000))
+    got = m.prefill_rows(toks, 0)
+    monkeypatch.setenv("TL_DENSE_TILE", "128")
+    m.reset_kv()
+    assert np.isfinite(got).all() and np.array_equal(got, m.prefill_rows(toks, 0))
+    m.free()

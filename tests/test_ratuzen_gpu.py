@@ -449,6 +449,7 @@ def test_wide_model_through_the_large_products(env, monkeypatch):
                                                   L("parallel", K(16, 4, 64, 64, 300, 16, 64, 64, np.linspace(0.9, 0.99, 16)), 4096)])
     m, tensors, orc = make(env, cfg, seed=21, max_pos=1100, exact=False)
     toks = np.random.default_rng(7).integers(0, cfg["vocab"], 1100).astype(np.int32)
+    assert all(env["capi"].lib().tl_debug_dense_plane_taken(rows, 2048, 1100, 2080 * 4096, 256) == 1 for rows in (4096, 8192))
     got, want = f64(m.prefill_rows(toks, 0)), orc.forward(list(toks))
     err = np.sqrt(((got - want) ** 2).mean(-1)) / np.sqrt((want * want).mean())
     assert err.max() < BF16_TOL, (err[:33], err.max())  # (1.3e-2 seen; stale second terms: 0.9 in rows 1 to 31)

@@ -679,3 +679,21 @@ def test_latent_rows_beyond_a_chunk(env, monkeypatch):
         got.append(m.prefill_rows(toks, 0, np.array([0, 700, 2100, 2239], np.int32)))
         m.free()
     assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1])
+
+
+def test_large_products_give_the_same_bits_from_a_plane(env, monkeypatch):
+    """1024 wide, 1100 tokens in bf16 mode: first products and feed-forwards with activations of their own take the kernel that reads its
+    items from a bf16 plane; with the kernel that converts them itself every logit is the same to the bit."""
+    S = env["synth"]
+    A, M, D, L = S.sogalix_attention, S.sogalix_latent, S.sogalix_delta, S.sogalix_layer
+    cfg = S.sogalix_config(1024, 300, [L("general_delta", D(16, 64), ff=4096), L("latent_attention", M(16, 64, 32, 64, 512, 256), ff=4096),
+                                       L("attention", A(32, 8, 64, 64, q_temp=(0.1, 512)), ff=4096)])
+    m, _, _ = make(env, cfg, seed=6, max_pos=1100, exact=False)
+    toks = np.random.default_rng(9).integers(0, cfg["vocab"], 1100).astype(np.int32)
+    taken = env["capi"].lib().tl_debug_dense_plane_taken  # (256 compute units; the plane holds 2048 tokens)
+    assert all(taken(rows, 1024, 1100, 2080 * 4096, 256) == 1 for rows in (5184, 4096))
+    got = m.prefill_rows(toks, 0)
+    monkeypatch.setenv("TL_DENSE_TILE", "128")
+    m.reset_kv()
+    assert np.isfinite(got).all() and np.array_equal(got, m.prefill_rows(toks, 0))
+    m.free()
