@@ -1,5 +1,5 @@
-// tl_bf16.h — device helpers shared by the bf16-weight kernels (tl_dense.hip, tl_moe.hip): exact widening of bf16 pairs and
-// the dot product of bf16 weight rows with an FP32 vector over the lanes of a wave.
+// tl_bf16.h — device helpers shared by the layer-list kernels (tl_dense.hip, tl_moe.hip, tl_norm.hip, tl_swa.hip, tl_delta.hip): exact
+// widening of bf16 pairs, the dot product of bf16 weight rows with an FP32 vector over the lanes of a wave, sums over lanes.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -22,6 +22,15 @@ __device__ __forceinline__ uint4 tl_ldw(const unsigned short* p) {  // weights a
   typedef unsigned tl_u32x4 __attribute__((ext_vector_type(4)));
   const tl_u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const tl_u32x4*>(p));
   return make_uint4(v[0], v[1], v[2], v[3]);
+}
+
+// sum over the 16 lanes of a row, result in all of them: lane swaps inside quads, then mirrored halves (no LDS round trip)
+__device__ __forceinline__ float tl_row16_sum(float x) {
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0xB1, 0xf, 0xf, false));   // quad_perm [1,0,3,2]
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x4E, 0xf, 0xf, false));   // quad_perm [2,3,0,1]
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x141, 0xf, 0xf, false));  // row_half_mirror
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x140, 0xf, 0xf, false));  // row_mirror
+  return x;
 }
 
 __device__ __forceinline__ float tl_wave_sum(float s) {

@@ -115,15 +115,6 @@ __global__ __launch_bounds__(256) void conv_history_kernel(const DeltaPreArgs a)
   }
 }
 
-// sum over the 16 lanes of a row, result in all of them: lane swaps inside quads, then mirrored halves (no LDS round trip)
-__device__ __forceinline__ float row16_sum(float x) {
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0xB1, 0xf, 0xf, false));   // quad_perm [1,0,3,2]
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x4E, 0xf, 0xf, false));   // quad_perm [2,3,0,1]
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x141, 0xf, 0xf, false));  // row_half_mirror
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x140, 0xf, 0xf, false));  // row_mirror
-  return x;
-}
-
 // E key channels per lane: dim <= 16 E. grid (vdim / 16 rounded up, heads), 256 threads.
 // The operands of 16 (8 for the largest key size) tokens at a time (k, q, g of the head; v of the workgroup's 16 columns; beta) are staged in LDS by
 // all threads together, the next stage's global loads in flight while the tokens of the stage in hand are walked: a token
@@ -201,7 +192,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const DeltaScanArgs a) 
           s[e] = s[e] * gc[e] + kc[e] * u;
           sq += s[e] * qc[e];
         }
-        sq = row16_sum(sq);
+        sq = tl_row16_sum(sq);
         if (live && sub == 0) a.o[(size_t)(t0 + tt) * a.heads * a.vdim + (size_t)h * a.vdim + col] = sq * oscale;
         continue;
       }
@@ -212,9 +203,9 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const DeltaScanArgs a) 
         sq += s[e] * qc[e];
         kq += kc[e] * qc[e];
       }
-      sk = row16_sum(sk);
-      sq = row16_sum(sq);
-      kq = row16_sum(kq);
+      sk = tl_row16_sum(sk);
+      sq = tl_row16_sum(sq);
+      kq = tl_row16_sum(kq);
       const float u = bc * (vc - sk);
 #pragma unroll
       for (int e = 0; e < E; ++e) s[e] += kc[e] * u;
@@ -296,7 +287,7 @@ __global__ __launch_bounds__(1024) void gla_step_kernel(const GlaStepArgs a, int
         s[i][e] = ac[e] * s[i][e] + kc[e] * v;
         o += s[i][e] * qc[e];
       }
-      o = row16_sum(o);
+      o = tl_row16_sum(o);
       if (!live) continue;
       if (sub == 0) so[col] = o * a.q_scale;
       float* p = S + (size_t)col * a.dim + d0;
@@ -490,8 +481,8 @@ __global__ __launch_bounds__(256) void gdelta_scan_kernel(const GDeltaScanArgs a
         s[e] *= wc[e];
         y += rc_[e] * s[e];
       }
-      x = row16_sum(x);
-      y = row16_sum(y);
+      x = tl_row16_sum(x);
+      y = tl_row16_sum(y);
 #pragma unroll
       for (int e = 0; e < E; ++e) s[e] += kc[e] * vc - ac[e] * x;
       if (live && sub == 0) a.o[(size_t)(t0 + tt) * a.heads * a.vdim + (size_t)h * a.vdim + col] = y - rau * x + rkk * vc;
@@ -509,8 +500,8 @@ __global__ __launch_bounds__(256) void gdelta_scan_kernel(const GDeltaScanArgs a
 // The same for key sizes of exactly 16 E and rows at 16 bytes. One wave a SIMD walks the tokens, so what a token costs is the number of
 // its instructions: here five 16-byte LDS reads at constant offsets (a stage is unrolled), 5 E products and sums, and two row sums. (r w)
 // is formed once in staging; the lane whose number is the token's keeps x and y, and a stage's outputs are finished and stored together.
-// The new column is one rounding of w s + (k v - a u x). 32 heads of 64 times 1999 tokens: 239 us with a stage that is not unrolled and an output stored per token; a layer-list
-// prompt of eight such layers 8.5 -> 7.4 ms, about 100 us a launch.
+// The new column is one rounding of w s + (k v - a u x). 32 heads of 64 times 1999 tokens: 239 us with a stage that is not unrolled and
+// an output stored per token; a layer-list prompt of eight such layers 8.5 -> 7.4 ms, about 100 us a launch.
 template <int E>
 __global__ __launch_bounds__(256) void gdelta_scan_wide_kernel(const GDeltaScanArgs a) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -566,8 +557,8 @@ __global__ __launch_bounds__(256) void gdelta_scan_wide_kernel(const GDeltaScanA
       x += fmaf(q[U][e][0], s[e][0], q[U][e][1] * s[e][1]) + fmaf(q[U][e][2], s[e][2], q[U][e][3] * s[e][3]);
       y += fmaf(q[RW][e][0], s[e][0], q[RW][e][1] * s[e][1]) + fmaf(q[RW][e][2], s[e][2], q[RW][e][3] * s[e][3]);
     }
-    x = row16_sum(x);
-    y = row16_sum(y);
+    x = tl_row16_sum(x);
+    y = tl_row16_sum(y);
 #pragma unroll
     for (int e = 0; e < E / 4; ++e)
 #pragma unroll

@@ -17,13 +17,15 @@
 //   Large products of one term do without the conversion in every tile: the items are rounded to a bf16 plane once, and both sides go
 //   from memory to LDS without registers in between (dense_plane_kernel: 10304 x 2048 times 1999 tokens 174 -> 114 us with the
 //   conversion of 8, that is 740 and 800 TFLOP/s; staged through registers from the same plane 133). What bounds it now: barriers
-//   and fragment reads between the products of a step, and at these sizes the last of 2.5 rounds of tiles. Items may be gathered (x_rows), scattered (y_rows) and
-//   grouped (group_off: blockIdx.z = matrix of the group; tiles beyond a group's items leave at once), which is what the
-//   experts of a mixture need: the plan lives on the device, the grid is sized for the worst case.
+//   and fragment reads between the products of a step, and at these sizes the last of 2.5 rounds of tiles.
+//   Items may be gathered (x_rows), scattered (y_rows) and grouped (group_off: blockIdx.z = matrix of the group; tiles beyond a
+//   group's items leave at once), which is what the experts of a mixture need: the plan lives on the device, the grid is sized for
+//   the worst case.
 #include <math.h>
 #include <stdlib.h>
 
 #include "tl_bf16.h"
+#include "tl_lds.h"
 #include "tl_stack.h"
 
 namespace {
@@ -257,13 +259,6 @@ __global__ __launch_bounds__(256) void dense_gemm_kernel(const DenseArgs a) {
   dense_store<WM, WN>(a, acc, Y, f0 + wm * WM * 32, t0 + wn * WN * 32, hi, lane);
 }
 
-// 16 bytes a lane from base + off to LDS bytes at .. at + 1023, no registers in between (at, base: the same in all lanes). M0 holds the
-// LDS address and belongs to the compiler: saved and restored in the same statement
-__device__ __forceinline__ void dma16(unsigned at, unsigned off, const void* base) {
-  unsigned keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
-               : "=&s"(keep) : "s"(at), "v"(off), "s"(base) : "memory");
-}
 template <int N>
 __device__ __forceinline__ void dma_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
@@ -315,10 +310,10 @@ __global__ __launch_bounds__(64 * NWM * NWN, 2) void dense_plane_kernel(const De
     const char* wb = reinterpret_cast<const char*>(a.w) + k;
     const char* xb = reinterpret_cast<const char*>(a.plane) + k;
 #pragma unroll
-    for (int i = 0; i < IW; ++i) dma16(b + (wave * IW + i) * 1024, wo[i], wb);
+    for (int i = 0; i < IW; ++i) tl_lds_load16(b + (wave * IW + i) * 1024, wo[i], wb);
 #pragma unroll
-    for (int j = 0; j < IX; ++j) dma16(b + BM * 128 + (wave * IX + j) * 1024, xo[j], xb);
-    if (FIRST && lead) dma16(b + (BM + BN) * 128 + (wave & 3) * 1024, eo, xb + (size_t)a.T * K * 2);
+    for (int j = 0; j < IX; ++j) tl_lds_load16(b + BM * 128 + (wave * IX + j) * 1024, xo[j], xb);
+    if (FIRST && lead) tl_lds_load16(b + (BM + BN) * 128 + (wave & 3) * 1024, eo, xb + (size_t)a.T * K * 2);
   };
   f32x16 acc[WM][WN];
 #pragma unroll

@@ -22,6 +22,7 @@
 #include <math.h>
 
 #include "tl_internal.h"
+#include "tl_lds.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -177,13 +178,6 @@ __device__ __forceinline__ float finish(const TlHattn& x, int t, int head, float
   return x.gate ? f / (1.0f + expf(-x.gate[(size_t)t * x.gate_ld + head])) : f;
 }
 
-// 16 bytes a lane from base + off to LDS bytes at .. at + 1023 (at, base: the same in all lanes). M0 belongs to the compiler: saved and
-// restored in the same statement
-__device__ __forceinline__ void lds_load16(unsigned at, unsigned off, const void* base) {
-  unsigned keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
-               : "=&s"(keep) : "s"(at), "v"(off), "s"(base) : "memory");
-}
 template <int KD, int VD>
 __global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs a) {
   constexpr int DS = KD / 16, DB = VD / 32, TILE = (KD + VD) * 64, NLD = TILE / 8 / 256;
@@ -214,7 +208,7 @@ __global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs a) {
     stage_ex = ex[t];
 #pragma unroll
     for (int i = 0; i < NLD; ++i)
-      lds_load16(lds0 + (unsigned)(buf * TILE * 2 + (i * 256 + first) * 16), lane * 16, src + (size_t)t * (TILE / 8) + i * 256 + first);
+      tl_lds_load16(lds0 + (unsigned)(buf * TILE * 2 + (i * 256 + first) * 16), lane * 16, src + (size_t)t * (TILE / 8) + i * 256 + first);
   };
   auto arrived = [] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };  // of this wave's pieces; the barrier behind it: of all
   load(t0, 0);

@@ -1304,7 +1304,8 @@ extern "C" int tl_model_generate_sampled(tl_model* m, int first_token, int start
 // A chunk of up to kPrefillChunk tokens goes through every layer as a batch: RMSNorm -> activation planes, q/k/v GEMMs on
 // the matrix cores (tl_gemm.hip), batched RoPE + KV write, causal attention from the cache (tl_prefill.hip), O GEMM +
 // residual, RMSNorm -> planes, gate/up GEMMs, SwiGLU -> planes, down GEMM + residual. Longer prompts are walked chunk by
-// chunk over the growing cache. Short prompts (< prefill_min_batch) replay the decode graph token by token instead (same positions, KV contents and logits to ~1e-6).
+// chunk over the growing cache. Short prompts (< prefill_min_batch) replay the decode graph token by token instead (same positions, KV
+// contents and logits to ~1e-6).
 // Unsharded models whose products take the f16 form: 2048, where a projection has four times the tiles and fewer K slices, and the
 // attention converts the cache and sums its pieces a quarter as often (3B Q6_K, 3989 tokens: 98 ms in chunks of 512, 92 in these;
 // more would only grow the workspaces). The bf16 routes and tensor-parallel shards keep the 512 that they were tuned at, which
@@ -1891,8 +1892,9 @@ static int batch_head(tl_model* m, const float* hidden, int R, hipStream_t s) {
 }
 
 // Many logits to the caller's memory, behind what the stream holds. The runtime takes pageable memory through one thread's copies (and its
-// page faults): 128 rows of 128256 (66 MB) 6.2 ms, here 1.9; 64 rows 1.8 and 0.9, 16 rows 0.47 and 0.31, 8 rows level. Four threads take a stripe each through two pinned pieces, one on its way from the
-// device while the other is copied out. Up to kCopySpread bytes: the runtime's own copy, complete when the stream is waited for.
+// page faults): 128 rows of 128256 (66 MB) 6.2 ms, here 1.9; 64 rows 1.8 and 0.9, 16 rows 0.47 and 0.31, 8 rows level. Four threads take
+// a stripe each through two pinned pieces, one on its way from the device while the other is copied out. Up to kCopySpread bytes: the
+// runtime's own copy, complete when the stream is waited for.
 static int copy_to_caller(tl_model* m, float* dst, const float* src, size_t bytes, hipStream_t s) {
   tl_model::Batch& b = m->bt;
   hipPointerAttribute_t at = {};  // memory that the runtime knows (pinned, managed, a device's) it copies to directly

@@ -1,8 +1,9 @@
 // tl_norm.hip — the row-wise FP32 steps between the matrix products of a layer-list model. An RMS norm here is
 // y = x / sqrt(mean(x^2) + eps) * weight, eps inside the root; "one-plus" weights are stored around zero and applied as
 // (1 + w). Norm-first blocks with the Dynamic Tanh norm (tanh(alpha x) * w + b: elementwise, no statistics) need no staged
-// row: embedding gather, residual sum and row gather carry the norm of the block that follows in the same pass. One workgroup per token row (256 threads for the rows of a prompt chunk, 1024 for the few rows of a decode step,
-// whose launches are nothing but a chain of memory round trips); a row is staged in LDS, so that it is read from memory once.
+// row: embedding gather, residual sum and row gather carry the norm of the block that follows in the same pass. One workgroup per
+// token row (256 threads for the rows of a prompt chunk, 1024 for the few rows of a decode step, whose launches are nothing but a chain of
+// memory round trips); a row is staged in LDS, so that it is read from memory once.
 #include <math.h>
 
 #include "tl_bf16.h"

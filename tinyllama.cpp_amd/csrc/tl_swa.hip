@@ -21,6 +21,7 @@
 
 #include <type_traits>
 
+#include "tl_bf16.h"
 #include "tl_internal.h"
 #include "tl_stack.h"
 
@@ -296,18 +297,8 @@ __global__ __launch_bounds__(256) void swa_kernel(const SwaArgs a) {
 // The same work split and tail for key and value rows of 64 NV numbers at 16 bytes: sixteen lanes own a key (its dot product is four
 // DPP additions), four keys a load, and all the loads of a step -- 64 / NV keys, their values and the query -- are in flight together.
 // With a lane per key, the values' eight rows a step are eight round trips one after another, which is what that kernel's time is:
-// 32 heads of 64 over 700 keys, one token, 14.1 us, here 10.3 (a launch without work takes 3; what is left is the position, the rows and, from
-// 257 keys on, the records, one after another). Eight waves a workgroup and half the splits: 11.9; 1024 keys without records: 12.4.
-__device__ __forceinline__ float swa_sum16(float v) {
-  auto add = [](float x, auto ctrl_c) {
-    constexpr int CTRL = decltype(ctrl_c)::value;
-    return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, false));
-  };
-  v = add(v, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
-  v = add(v, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
-  v = add(v, std::integral_constant<int, 0x141>{});  // row_half_mirror
-  return add(v, std::integral_constant<int, 0x140>{});  // row_mirror
-}
+// 32 heads of 64 over 700 keys, one token, 14.1 us, here 10.3 (a launch without work takes 3; what is left is the position, the rows and,
+// from 257 keys on, the records, one after another). Eight waves a workgroup and half the splits: 11.9; 1024 keys without records: 12.4.
 template <int NV>
 __global__ __launch_bounds__(256) void swa_rows_kernel(const SwaArgs a) {
   constexpr int W = SWA_WAVES, D = 64 * NV, U = 16 / NV;  // keys a lane group takes in a step
@@ -366,7 +357,7 @@ __global__ __launch_bounds__(256) void swa_rows_kernel(const SwaArgs a) {
         float d = 0.0f;
 #pragma unroll
         for (int v = 0; v < NV; ++v) d += (q[v][0] * kk[u][v][0] + q[v][1] * kk[u][v][1]) + (q[v][2] * kk[u][v][2] + q[v][3] * kk[u][v][3]);
-        d = swa_sum16(d) * a.scale;
+        d = tl_row16_sum(d) * a.scale;
         if (a.softcap > 0.0f) d = swa_cap(d, a.softcap, 1.0f / a.softcap);
         if (a.dist_r1) d -= swa_dist(r1, r2, i - j);
         s[u] = j <= jend ? d : -INFINITY;
