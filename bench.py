@@ -1,10 +1,10 @@
 #!/usr/bin/env python3
-"""bench.py — greedy decode throughput of the quantized forward pass on MI355X (BASELINE.json metric).
+"""bench.py — greedy decode throughput of the quantized forward pass on MI355X.
 
 A "step" is one decoded token: one pass of the hot path (embedding lookup, L transformer layers over the
 device-resident KV cache, lm_head, on-device greedy sampling) for one sequence. The default workload is the one
 the north star's target is quoted on and that fits one GPU: Llama-3-8B-shaped synthetic random-init Q4_K_M
-(SURVEY §8d tensor mix; 4.62 GB of quantized weights per token), weights resident in HBM before the timed region.
+(the Q4_K_M tensor mix; 4.62 GB of quantized weights per token), weights resident in HBM before the timed region.
 
     python bench.py --gpus 1 --steps 128 --warmup 16 [--workload llama-3-8b|tinyllama-1.1b|llama-3.2-3b|tiny]
 
@@ -595,7 +595,7 @@ def main():
     try:
         pkg_tp = __import__("tinyllama_cpp_amd.tp", fromlist=["check"])
         pkg_tp.check(cfg, world)
-    except ValueError as e:  # this shape does not split `world` ways (SURVEY 8e): say so and stop, on every rank
+    except ValueError as e:  # this shape does not split `world` ways: say so and stop, on every rank
         tp_err = str(e)
     if tp_err:
         if rank == 0:
@@ -762,7 +762,7 @@ def main():
 
     # ---- the dominant kernel (fused RMSNorm + ffn_gate/ffn_up GEMV + SwiGLU): average launch duration with HIP events
     #      on the engine's stream, back-to-back launches cycling through the layers (every launch streams from HBM);
-    #      algorithmic bytes = GGUF bytes of the two matrices one launch reads (SURVEY 8d) --------------------------
+    #      algorithmic bytes = GGUF bytes of the two matrices one launch reads --------------------------
     gu_us, gu_bytes = model.bench_kernel("gate_up_gemv", iters=8 * cfg["n_layers"], warmup=8 * cfg["n_layers"])  # (the clocks settle during the warm-up)
     achieved = gu_bytes / (gu_us * 1e-6) / 1e9 if gu_us > 0 else 0.0
     kern = {}
@@ -862,7 +862,7 @@ def main():
         except Exception as e:  # the decode numbers above stay valid
             out["prefill"] = {"error": str(e)[:300]}
 
-    # ---- multi-sequence decode (generate_batch's engine, SURVEY f4; outside the timed single-sequence region): B
+    # ---- multi-sequence decode (generate_batch's engine; outside the timed single-sequence region): B
     # sequences share every step's weight stream (skinny GEMMs on the matrix cores), FP32-grade 6-term products
     if tp_world == 1 and world == 1 and not args.no_batch_leg and cfg["max_pos"] >= 64:
         try:
@@ -911,7 +911,7 @@ def batch_leg(model, cfg, B, plen=16, steps=16, terms=6):
 
 def prefill_leg(model, S, cfg, mix, T, terms=6, reps=3, world=1):
     """tokens/s of tl_model_prefill (MFMA GEMMs over the quantized weights, FP32-MFMA attention) for a T-token prompt;
-    executed bf16 MFMA flops = (MFMAs per product) x the algorithmic GEMM flops 2*T*(layer weight elements) (SURVEY 8d)."""
+    executed bf16 MFMA flops = (MFMAs per product) x the algorithmic GEMM flops 2*T*(layer weight elements)."""
     toks = np.random.default_rng(1).integers(0, cfg["vocab"], T).astype(np.int32)
     model.set_prefill(terms=terms, min_batch=8)
     model.reset_kv()

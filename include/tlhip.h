@@ -12,7 +12,7 @@
  *     error instead of the reference's log-and-return-silently (cuda_kernels.cu:1335-1351).
  *   - `*_dev` pointers are device pointers BORROWED from the caller; `*_host` are host pointers borrowed
  *     for the duration of the call. tl_qweight / tl_model handles own their device memory.
- *   - one host thread per handle, no re-entrancy (the reference's threading model, SURVEY §8b.3).
+ *   - one host thread per handle, no re-entrancy (the reference's threading model).
  *
  * The big difference from the reference backend: weights stay QUANTIZED on the device. The reference
  * dequantizes every GPU layer to FP32 on the host and calls cublasSgemm with N=1
@@ -37,7 +37,7 @@ typedef struct tl_qweight tl_qweight; /* one quantized [rows x cols] matrix resi
 typedef struct tl_model tl_model;     /* a whole model + KV cache + workspaces + decode graph */
 
 /* ---- runtime: replaces the inline cudaSetDevice/cudaMalloc/cudaMemcpy/cudaFree/cudaStream*/
-/*      cublasCreate sites (215 of them, SURVEY §2.1) ---------------------------------------- */
+/*      cublasCreate sites (215 of them) ---------------------------------------- */
 const char* tl_last_error(void);
 /* hipSetDevice + sanity (gfx950 expected) + this device's address of the static no-allocation workspace
  * (tl_attention_noalloc); call once per device the process uses, with that device's ordinal */
@@ -211,7 +211,7 @@ int tl_model_set_prefill(tl_model* m, int terms, int min_batch);
 /* device pointers into the model's state, for parity tests and for hosts that keep using the operator-level
  * calls: which = 0 K cache, 1 V cache of `layer` ([max_pos][n_kv_heads_local][head_dim] f32), 2 = x (hidden) */
 int tl_model_device_ptr(tl_model* m, int which, int layer, void** dev_out);
-/* algorithmic bytes one decode step at position pos must move on this rank (SURVEY §8d B_tok) */
+/* algorithmic bytes one decode step at position pos must move on this rank */
 int tl_model_bytes_per_token(const tl_model* m, int pos, double* weight_bytes, double* kv_bytes);
 /* device bytes of the expanded prefill planes that tl_model_finalize keeps for this model's matrices (tl_qweight_expand;
  * 0: none -- not needed by the f16 form, switched off, or not affordable on this device). They serve the batched paths only: a
@@ -628,7 +628,7 @@ int tl_model_prefill_rows(tl_model* m, const int* tokens_host, int num_tokens, i
 /* tensor-parallel wiring (one process per GPU): RCCL communicator over xGMI; unique_id is the ncclUniqueId (128 bytes)
  * produced by tl_tp_unique_id on rank 0 and broadcast by the host (torch.distributed). Call tl_model_tp_init on every
  * rank before tl_model_finalize: the decode step (incl. its 2 all-reduces per layer and the logits all-gather) is
- * captured into the graph there. Replaces distributed_coordinator.cpp's MPI request routing (SURVEY 8e). */
+ * captured into the graph there. Replaces distributed_coordinator.cpp's MPI request routing. */
 int tl_tp_unique_id(void* id_out_128);
 int tl_model_tp_init(tl_model* m, const void* unique_id_128);
 /* Peer-to-peer exchange for the decode step (no counterpart in the reference): the two f32[hidden] all-reduces per layer

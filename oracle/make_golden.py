@@ -103,7 +103,7 @@ def make_g4(ref):
 def main():
     os.makedirs(OUT, exist_ok=True)
     ref, orc = Ref(), Oracle()
-    if sys.argv[1:] == ["g4"]:  # only the GGUF fixture (the others are unchanged since round 1)
+    if sys.argv[1:] == ["g4"]:  # only the GGUF fixture (the others do not change with it)
         return make_g4(ref)
     rng = np.random.default_rng(20261110)
 

@@ -214,7 +214,7 @@ class Oracle:
 
 class OracleModel:
     """A model held by the oracle. `tensors`: dict name -> (type, uint8/float32 ndarray, rows, cols),
-    names as in GGUF (SURVEY A2). Arrays are kept alive here (the C side borrows them)."""
+    names as in GGUF. Arrays are kept alive here (the C side borrows them)."""
 
     KINDS = {"attn_q": T_ATTN_Q, "attn_k": T_ATTN_K, "attn_v": T_ATTN_V, "attn_output": T_ATTN_O,
              "ffn_gate": T_FFN_GATE, "ffn_up": T_FFN_UP, "ffn_down": T_FFN_DOWN,
@@ -331,7 +331,7 @@ class Ref:
         L.ref_rope_batch.argtypes = [_fp, _fp] + [C.c_int] * 5 + [_fp, C.c_int, C.c_int]
         L.ref_softmax.argtypes = [_fp, _fp, C.c_int]
         L.ref_silu.argtypes = [_fp, _fp, C.c_int]
-        if hasattr(L, "ref_gguf_open"):  # (a libtlref.so built before round 2 lacks the parser / timing doorways)
+        if hasattr(L, "ref_gguf_open"):  # (a libtlref.so of an older build lacks the parser / timing doorways)
             L.ref_last_error.restype = C.c_char_p
             L.ref_gguf_open.restype = C.c_long
             L.ref_gguf_open.argtypes = [C.c_char_p, C.c_int]

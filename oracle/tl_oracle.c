@@ -4,7 +4,7 @@
  * A restatement in plain C of what the reference computes on its CPU path; every function names
  * the reference file:line it follows. Float expressions keep the reference's evaluation order and
  * are compiled with -ffp-contract=off so that no multiply-add is fused (the reference's canonical
- * build is baseline x86-64 without FMA, SURVEY §8c).
+ * build is baseline x86-64 without FMA).
  */
 #include "tl_oracle.h"
 
@@ -669,7 +669,7 @@ void tlo_dequantize_whole_tensor(int type, const void* blocks, size_t nblocks, f
 }
 
 /* one projection y = W x through either the fused path or (ref_structure) ensure_*_dequantized +
- * matvec_f32_f32_vector_cpu — the two are bit-identical (SURVEY §8 a6) */
+ * matvec_f32_f32_vector_cpu — the two are bit-identical */
 static void project(tlo_model* m, tlo_tensor* t, const float* x, float* y) {
   if (m->ref_structure && t->type != TLO_F32) {
     if (!t->f32) {
@@ -789,7 +789,7 @@ void tlo_forward_batch(tlo_model* m, float* x, int T, int start_pos, float* logi
   free(xn); free(q); free(k); free(v); free(att); free(prj); free(g); free(u); free(h);
 }
 
-/* TinyLlamaSession::generate on token ids, greedy (api.cpp:585-813; SURVEY appendix A5) */
+/* TinyLlamaSession::generate on token ids, greedy (api.cpp:585-813) */
 int tlo_generate(tlo_model* m, const int* prompt, int n_prompt, int max_new, float penalty,
                  int eos_id, int* out_ids, float* logits_dump) {
   const int P = n_prompt, V = m->vocab, hs = m->hidden;

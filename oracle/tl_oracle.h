@@ -16,7 +16,7 @@
  * end-to-end composition is pinned only through its primitives.
  *
  * Build: gcc -O2 -ffp-contract=off -fopenmp (NO -march=native: FMA contraction changes the
- * dequantized bit patterns, SURVEY §8c).
+ * dequantized bit patterns).
  */
 #ifndef TL_ORACLE_H
 #define TL_ORACLE_H
@@ -131,7 +131,7 @@ void tlo_forward(tlo_model* m, float* x, int pos, float* logits, int n_layers_li
 /* forward_cpu_batch + forward_cpu_logits_batch, cpu_batch_processor.cpp:11-281, model.cpp:1094-1156.
  * x[T][hidden] in/out; logits[T][vocab] (may be NULL) */
 void tlo_forward_batch(tlo_model* m, float* x, int T, int start_pos, float* logits);
-/* generate() loop on token ids (api.cpp:585-813, SURVEY A5); greedy. Returns #generated.
+/* generate() loop on token ids (api.cpp:585-813); greedy. Returns #generated.
  * logits_dump (may be NULL): [max_new][vocab], the (pre-penalty) logits at each sampled position */
 int tlo_generate(tlo_model* m, const int* prompt, int n_prompt, int max_new, float penalty,
                  int eos_id, int* out_ids, float* logits_dump);

@@ -393,8 +393,8 @@ __device__ __forceinline__ void attn_split_body(const AttnArgs& a, const int kvh
   //      that the consumer (every workgroup of the attn_output GEMV re-reads the partials) finds one record per head.
   //      Hand-off: written-through record stores, vmcnt(0), barrier, one relaxed agent-scope counter add per workgroup;
   //      the last one reads the records with agent-scope loads. The counter is left at zero for the next launch.
-  //      What this rests on: it is the form MI355X_MICROARCH.md lists as measured valid on gfx950 without fences ("Valid
-  //      forms", table row 1: every stored byte sc1 and drained by its wave before the workgroup barrier, ONE lane adds to
+  //      What this rests on: a form that measures as valid on gfx950 without fences
+  //      (every stored byte sc1 and drained by its wave before the workgroup barrier, ONE lane adds to
   //      ONE unsharded counter, the workgroup whose add came last -- told by the returned value -- loads with sc1 loads after
   //      its add has returned, its other waves after a barrier that lane joins). It is a property of this chip's caches, not
   //      of the C++ memory model: an agent-scope release / acquire pair instead (buffer_wbl2 + buffer_inv, ~1.7 us each)

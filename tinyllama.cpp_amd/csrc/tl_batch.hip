@@ -1,4 +1,4 @@
-// tl_batch.hip — the position-dependent kernels of the MULTI-SEQUENCE decode step (SURVEY f4): B sequences advance one
+// tl_batch.hip — the position-dependent kernels of the MULTI-SEQUENCE decode step: B sequences advance one
 // token each per step; the projections run as skinny GEMMs on the matrix cores (tl_gemm.hip, the weights are read once
 // for all B tokens), and what depends on (sequence, position) lives here:
 //   - RoPE of q / k at each token's own position + K/V write into the SEQUENCE-MAJOR cache

@@ -57,7 +57,7 @@ struct GemvVec {
 // A chain launch is a 2-D grid (workgroups of a task, tasks): the workgroups of task j+1 are dispatched behind those of
 // task j and take a CU as soon as one has room, issue their first weight loads (constants) and only then wait for task j,
 // so that kernel boundary, argument fetch and the first HBM round trip of a launch overlap the tail of its predecessor.
-// Hand-off (MI355X_MICROARCH.md, "Valid forms", table row 1): every activation word that crosses a task edge is stored
+// Hand-off (measured as valid on gfx950 without fences): every activation word that crosses a task edge is stored
 // with an agent-scope (sc1, write-through) store and loaded with sc1 loads; every storing wave drains its stores
 // (s_waitcnt vmcnt(0)), the workgroup meets at a barrier, one lane adds 1 to the task's arrival counter (8 shards on
 // lines of their own: 256 arrivals on one word serialise at ~12 ns each); the consumer's wave 0 polls the shards with sc1
@@ -862,8 +862,8 @@ __device__ __forceinline__ void gemv_body(const GemvSeg& sg0, const GemvSeg& sg1
 
 // Since the launch geometry travels as explicit arguments these kernels have NO hidden argument block: their kernarg
 // segment would be exactly the 276 bytes of explicit arguments, not a multiple of 8. rocprofv3's dispatch callback faulted
-// twice in round 2 under dispatches of this kernel family (a memmove off the end of a mapping; profiles/README.md,
-// "profiler aborts": not explained by the argument block alone -- other kernels of the library share both properties and
+// twice under dispatches of this kernel family (a memmove off the end of a mapping;
+// not explained by the argument block alone -- other kernels of the library share both properties and
 // have run under the profiler -- but rounding the segment up to 320 bytes (5 x 64) with an unread tail argument costs
 // nothing).
 struct GemvPad {

@@ -122,7 +122,7 @@ struct tl_model {
   } pf;
   int prefill_terms = 0;     // MFMAs per product in the prefill GEMMs (0: tl_gemm_set_terms' process-wide value)
   int prefill_min_batch = 8; // prompts shorter than this replay the decode graph token by token
-  // multi-sequence decode (SURVEY f4): a second, SEQUENCE-MAJOR cache [layer][K|V][seq][max_pos][kv_dim] and the
+  // multi-sequence decode: a second, SEQUENCE-MAJOR cache [layer][K|V][seq][max_pos][kv_dim] and the
   // device-resident per-sequence state of the batched generation loop (tl_model_batch_init)
   struct Batch {
     int max_batch = 0;
@@ -201,7 +201,7 @@ extern "C" int tl_model_create(const tl_model_config* cfg, tl_model** out) {
   const int tp = cfg->tp_size <= 0 ? 1 : cfg->tp_size;
   const int hd = cfg->hidden_size / cfg->num_attention_heads;
   TL_REQUIRE(cfg->tp_rank >= 0 && cfg->tp_rank < tp, "tl_model_create: tp_rank %d outside [0,%d)", cfg->tp_rank, tp);
-  // Megatron-style shards (SURVEY 8e): q/k/v/gate/up/output by output rows (heads, intermediate columns, vocab rows),
+  // Megatron-style shards: q/k/v/gate/up/output by output rows (heads, intermediate columns, vocab rows),
   // attn_output/ffn_down by input columns, which must fall on 256-element super-block boundaries
   TL_REQUIRE(cfg->num_attention_heads % tp == 0 && cfg->num_key_value_heads % tp == 0 &&
                  cfg->intermediate_size % tp == 0 && cfg->vocab_size % tp == 0,
@@ -616,7 +616,7 @@ static int launch_proj(tl_model* m, const GemvArgs& a, hipStream_t s) {
     }                                                                                            \
   } while (0)
 
-// x = sum over ranks of xp (RCCL over xGMI; one f32[hidden_size] all-reduce per row-split projection, SURVEY 8e)
+// x = sum over ranks of xp (RCCL over xGMI; one f32[hidden_size] all-reduce per row-split projection)
 // (w: the row-split matrix whose launch produced xp; when that launch carried the exchange itself there is nothing to do)
 static int tp_all_reduce(tl_model* m, hipStream_t s, const tl_qweight* w = nullptr) {
   if (m->tp == 1 && !m->comm) return 0;
@@ -1246,7 +1246,7 @@ extern "C" int tl_model_generate_greedy(tl_model* m, int first_token, int start_
   return tp_check_peer(m);
 }
 
-// Sampled generation entirely on the device (SURVEY f2): the decode step with tl_sample.hip's top-k / top-p sampler as
+// Sampled generation entirely on the device: the decode step with tl_sample.hip's top-k / top-p sampler as
 // its tail. temperature < 0.05 samples greedily (api.cpp:134). The uniform variates come from a counter-based
 // generator keyed by `seed` (the reference seeds std::mt19937 from std::random_device: not reproducible either).
 extern "C" int tl_model_generate_sampled(tl_model* m, int first_token, int start_pos, int n_steps, float penalty,
@@ -1422,7 +1422,7 @@ static int ensure_prefill_ws(tl_model* m, bool all_logits) {
 // One chunk (tokens toks_dev[0..T) at positions start_pos.., T <= pf.cap) in pieces, so that a tensor-parallel group can
 // be driven in lockstep; the residual stream lives in pf.xb. tp > 1: the row-split GEMMs (attn_output, ffn_down) write
 // this rank's partial for the whole chunk into pf.xpart (rank 0 folds the residual in) and ONE all-reduce of T x hidden
-// floats per projection pair turns the partials into the new residual stream (SURVEY 8e).
+// floats per projection pair turns the partials into the new residual stream.
 static int prefill_embed(tl_model* m, const int* toks_dev, int T, hipStream_t s) {
   m->pf.pend = {nullptr, 0, 0};  // (a chunk that failed half-way must not leave its pending projection to the next one)
   return tl_launch_dequant_gather(m->tok, toks_dev, T, m->pf.xb, s);
@@ -1733,7 +1733,7 @@ extern "C" int tl_tp_local_group_prefill(tl_model* const* ms, int n, const int* 
 }
 
 
-// ---- multi-sequence decode (SURVEY f4; generate_batch api.cpp:836-1142, batch_generation_parallel :1423,
+// ---- multi-sequence decode (generate_batch api.cpp:836-1142, batch_generation_parallel :1423,
 //      forward_cpu_batch_generation model.cpp:1158-1523 / forward_device_batch_generation :1863-2114) -------------------
 // B sequences advance one token each per step. The projections of the B tokens run as skinny GEMMs on the matrix cores
 // (the batched-prefill kernels: the weights are streamed once per step for all sequences), RoPE / KV write / attention
@@ -2338,7 +2338,7 @@ extern "C" int tl_model_bytes_per_token(const tl_model* m, int pos, double* weig
     return 0;
   }
   if (weight_bytes) *weight_bytes = m->weight_bytes;
-  if (kv_bytes)  // read K and V of positions 0..pos, write one position (SURVEY §8d)
+  if (kv_bytes)  // read K and V of positions 0..pos, write one position
     *kv_bytes = (double)m->cfg.num_hidden_layers * 2.0 * ((double)pos + 2.0) * m->kv_dim * sizeof(float);
   return 0;
 }

@@ -16,13 +16,13 @@
 //     uncached allocations, so neither the writer's nor the reader's L2 (8 per GPU) ever holds a stale word;
 //   - every poll is bounded by a wall-clock deadline: a missing peer raises an error flag, never a hung GPU.
 // The kernels are plain launches: they are captured into the per-rank step graph like every other kernel of the step.
-// Folded form (VERDICT r1 item 5): the same protocol carried by the GEMV launches on the producing side of an exchange
+// Folded form: the same protocol carried by the GEMV launches on the producing side of an exchange
 // (tl_gemv.hip, PEER instantiations; the object they read is TlPeerDev): the lane that holds a finished row pushes its
 // word to every rank, and at the end of its work the wave polls this rank's area for its own rows of all ranks, sums them
 // in rank order (row-split projections) or files them (lm_head) and writes the result where the next launch reads it: no
 // exchange launch at all, 2 x layers + 1 fewer launches per token. These exchanges have areas and epochs of their own
 // (one epoch word per kind, advanced by the last workgroup of a launch), so both forms can be used side by side.
-// No counterpart in the reference (its multi-GPU story is a mock MPI coordinator, SURVEY 8e).
+// No counterpart in the reference (its multi-GPU story is a mock MPI coordinator).
 #include <hip/hip_runtime.h>
 
 #include <cstdlib>

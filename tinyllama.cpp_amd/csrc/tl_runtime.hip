@@ -1,6 +1,6 @@
 // tl_runtime.hip — device / memory / stream entry points of the C-ABI. They stand in for the raw
 // cudaSetDevice / cudaMalloc / cudaMemcpy / cudaFree / cudaStream* calls the reference's host files make
-// inline (model.cpp, gpu_initialization.cpp, weight_management.cpp, kv_cache.cpp, api.cpp; SURVEY §2.1).
+// inline (model.cpp, gpu_initialization.cpp, weight_management.cpp, kv_cache.cpp, api.cpp).
 #include <stdarg.h>
 #include <stdio.h>
 
@@ -90,7 +90,7 @@ extern "C" int tl_device_sync(void) {
 // tl_attention (split partials), tl_matmul_q (activation planes) and tl_sample_top_k_top_p (probabilities, parameters)
 // need device memory beyond their arguments. One lazily grown allocation per (device, slot), handed out under a mutex;
 // growing synchronises the device first (an earlier launch may still read the old block). Calls that share a slot must
-// not overlap on one device: one host thread per stream, as in the reference (SURVEY 8b.3). tl_shutdown() frees them.
+// not overlap on one device: one host thread per stream, as in the reference. tl_shutdown() frees them.
 namespace {
 std::mutex g_scratch_mu;
 std::map<std::pair<int, int>, std::pair<void*, size_t>> g_scratch;

@@ -1,4 +1,4 @@
-// tl_sample.hip — temperature / top-k / top-p sampling on the device (SURVEY f2), the non-greedy half of
+// tl_sample.hip — temperature / top-k / top-p sampling on the device, the non-greedy half of
 // sample_top_k_top_p_temperature (api.cpp:126-216) + apply_repetition_penalty (api.cpp:86-97).
 //
 // The reference copies vocab * 4 B to the host every token and sorts the whole vocabulary there (std::sort over

@@ -209,7 +209,7 @@ class Model:
         buf = (C.c_ubyte * 128).from_buffer_copy(bytes(unique_id))
         check(lib().tl_model_tp_init(self.h, buf), "tl_model_tp_init")
 
-    # ---- multi-sequence decode (SURVEY f4) -------------------------------------------------------------------------
+    # ---- multi-sequence decode -------------------------------------------------------------------------
     def batch_init(self, max_batch):
         check(lib().tl_model_batch_init(self.h, int(max_batch)), "tl_model_batch_init")
 
@@ -344,7 +344,7 @@ class Model:
         return (last, allb) if all_logits else last
 
     def generate(self, prompt, max_new, penalty=1.0, eos_id=-1):
-        """TinyLlamaSession::generate on token ids, greedy (api.cpp:585-813, SURVEY A5): prompts of >= 32
+        """TinyLlamaSession::generate on token ids, greedy (api.cpp:585-813): prompts of >= 32
         tokens go through tl_model_prefill, shorter ones are fed token by token; then device-side greedy steps."""
         prompt = [int(t) for t in prompt]
         P = len(prompt)

@@ -2,7 +2,7 @@
 // quantized super-blocks go from the page cache to the device without a typed host copy.
 //
 // Replaces gguf_parser.cpp:123-806 (load_gguf_meta: typed std::vector copies of every tensor) for the new backend.
-// Format facts as the reference parses them (SURVEY appendix A1): little-endian; header magic "GGUF", u32 version,
+// Format facts as the reference parses them: little-endian; header magic "GGUF", u32 version,
 // u64 tensor count, u64 kv count; strings are u64 length + bytes; tensor info = name, u32 n_dims (<= 4), u64 dims,
 // u32 ggml type, u64 offset relative to the data section, which starts at the next multiple of general.alignment
 // (default 32). dims[0] = columns (in_features), dims[1] = rows.

@@ -1,4 +1,4 @@
-// tl_tokenizer.hpp — the reference's tokenizer (tokenizer.cpp) without Boost: SURVEY §8 row f3.
+// tl_tokenizer.hpp — the reference's tokenizer (tokenizer.cpp) without Boost.
 //
 // What TinyLlamaSession needs from Tokenizer when the model comes from a GGUF file: the constructor from the file's
 // metadata (tokenizer.cpp:516-1048), encode (:1141-1410), decode (:1412-1652), apply_chat_template (:1663-1741), for the

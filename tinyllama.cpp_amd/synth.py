@@ -1,7 +1,7 @@
-"""Synthetic random-init models in the reference's on-disk formats (SURVEY §8d, appendix A1-A3).
+"""Synthetic random-init models in the reference's on-disk formats.
 
 Everything here is host-side numpy: random quantized super-blocks in the exact GGUF byte layouts
-(quantization.h:57-124), a model builder for the BASELINE.json shapes with the "Q4_K_M" tensor-type
+(quantization.h:57-124), a model builder for the benchmark's shapes with the "Q4_K_M" tensor-type
 mix, and a GGUF-v3 writer (gguf_parser.cpp:134-528 is the reader it targets).
 
 Scales are chosen so that dequantized weights have std ~= gain/sqrt(fan_in): activations stay O(1)
@@ -68,7 +68,7 @@ def edge_blocks(typ, rng):
     return b
 
 
-# ---- model shapes (SURVEY §8) -----------------------------------------------------------------
+# ---- model shapes -----------------------------------------------------------------
 SHAPES = {
     "tiny": dict(hidden=256, inter=512, n_heads=4, n_kv_heads=2, n_layers=3, vocab=64, max_pos=128,
                  eps=1e-5, rope_theta=10000.0),
@@ -88,7 +88,7 @@ SHAPES = {
 
 
 def tensor_plan(cfg, mix="q4_k_m"):
-    """[(name, type, rows, cols)] in file order. mix: 'q4_k_m' (SURVEY §8d: Q4_K except attn_v/ffn_down
+    """[(name, type, rows, cols)] in file order. mix: 'q4_k_m' (Q4_K except attn_v/ffn_down
     Q6_K on layers i<L/8 || i>=7L/8 || (i-L/8)%3==2, output Q6_K), 'q6_k', 'q8_0', 'q4_k'."""
     H, I, L, V = cfg["hidden"], cfg["inter"], cfg["n_layers"], cfg["vocab"]
     kvd = cfg["n_kv_heads"] * (H // cfg["n_heads"])
@@ -117,7 +117,7 @@ def tensor_plan(cfg, mix="q4_k_m"):
 
 
 def weight_bytes_per_token(cfg, mix="q4_k_m"):
-    """Algorithmic weight bytes one decoded token must read (SURVEY §8d B_tok without the KV terms):
+    """Algorithmic weight bytes one decoded token must read (without the KV terms):
     every projection + output.weight + ONE row of token_embd."""
     total = 0
     for name, typ, rows, cols in tensor_plan(cfg, mix):

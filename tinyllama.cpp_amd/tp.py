@@ -1,4 +1,4 @@
-"""Tensor-parallel sharding of the model's tensors (host side of SURVEY §8e).
+"""Tensor-parallel sharding of the model's tensors (host side).
 
 Megatron-style: attn_q/k/v, ffn_gate/up and output.weight are split by OUTPUT ROWS (rank r holds the r-th block of
 query heads / kv heads / intermediate columns / vocab rows); attn_output and ffn_down are split by INPUT COLUMNS
@@ -19,7 +19,7 @@ COL_SPLIT = ("attn_output", "ffn_down")
 
 
 def check(cfg, size):
-    """Raise ValueError unless `cfg` shards `size` ways (SURVEY §8e: heads, kv heads, 256-column boundaries)."""
+    """Raise ValueError unless `cfg` shards `size` ways (heads, kv heads, 256-column boundaries)."""
     H, I, nh, nkv, V = cfg["hidden"], cfg["inter"], cfg["n_heads"], cfg["n_kv_heads"], cfg["vocab"]
     hd = H // nh
     if size < 1 or nh % size or nkv % size or I % size or V % size:

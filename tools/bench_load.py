@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Load path (SURVEY f1): a synthetic GGUF file of the Llama-3-8B shapes (cut to --layers layers) is written to a scratch
+"""Load path: a synthetic GGUF file of the Llama-3-8B shapes (cut to --layers layers) is written to a scratch
 directory, then opened twice through the C++ host layer (mmap -> tl_model_set_tensor -> plane layout on the device):
 seconds and GB/s of quantized bytes from the mapping to HBM. The second open reads from a warm page cache."""
 import argparse

@@ -3,7 +3,7 @@
 
     python tools/bench_prefill.py [--workload llama-3-8b] [--lens 128,512,2048] [--terms 6,3,1] [--reps 3]
 
-Algorithmic GEMM flops per token = 2 * (weight elements of all layer projections) (SURVEY 8d; the lm_head runs for the
+Algorithmic GEMM flops per token = 2 * (weight elements of all layer projections) (the lm_head runs for the
 last token only, as a GEMV); executed bf16 MFMA flops = (MFMAs per product: 3 / 2 / 1 for terms 6 / 3 / 1 with the integer-plane GEMM) x that."""
 import argparse
 import json
