@@ -47,8 +47,8 @@ int tl_debug_gemm_px_launches(long long* count_out);
 int tl_debug_split_launches(long long* count_out);
 
 /* Test hook (no counterpart in the reference): tl_matmul_q through the f16 form that a model's chunks and multi-sequence steps
- * take (tl_hgemm.hip), any number of tokens, in a workgroup shape (0: 64 rows x 16 tokens, 1: 128 x 32, 2: 256 x 64, 3: 256 x 64 in
- * waves of 64 rows, Q4_K and Q8_K, 4: 128 x 64) and a number of K slices, none of them empty. */
+ * take (tl_hgemm.hip), any number of tokens, in a workgroup shape (0: 64 rows x 16 tokens, 1: 128 x 32, 2: 256 x 64, 3: in waves of 64
+ * rows, 512 x 64 in Q4_K and 256 x 64 in Q8_K, 4: 128 x 64) and a number of K slices, none of them empty. */
 int tl_debug_half_gemm(const tl_qweight* w, const float* x_dev, float* y_dev, int num_tokens, int shape, int slices, void* stream);
 
 /* Test hook (no counterpart in the reference): tl_dense_matmul's product with one term through the kernel that takes the items from a

@@ -423,6 +423,44 @@ def test_half_plane_gemm_shapes(E, pkg, shape, name, rows, cols, T, slices):
     w.free()
 
 
+@pytest.mark.parametrize("name,rows,cols,T,slices", [
+    ("q4_k", 255, 256, 63, 1), ("q4_k", 600, 2304, 129, 3), ("q6_k", 257, 768, 64, 1), ("q6_k", 255, 768, 65, 3), ("q6_k", 1, 256, 300, 1),
+    ("q8_0", 511, 1280, 130, 2), ("q8_0", 70, 256, 65, 1), ("q8_k", 257, 768, 65, 2), ("q8_k", 33, 2304, 64, 1)])
+def test_half_plane_gemm_lds_shape_has_the_sums_of_shape_4(E, pkg, name, rows, cols, T, slices):
+    """256 rows in eight waves with weights through LDS against 128 rows in four with weights through registers: the same bits. Rows and
+    tokens off the tiles, odd numbers of super-blocks (two rows' d in one dword, the last row's at the end of its plane), slices of
+    one super-block and a short last one."""
+    from tinyllama_cpp_amd.capi import check, lib
+    t, S = TYPES[name], pkg.synth
+    rng = np.random.default_rng(rows + 7 * cols + T)
+    w = E.QWeight(t, S.random_blocks(t, rows * cols // S.BLOCK_ELEMS[t], rng, w_std=1.0 / np.sqrt(cols)), rows, cols)
+    xb, yb = E.DeviceBuffer.from_numpy(rng.standard_normal((T, cols)).astype(np.float32)), E.DeviceBuffer(4 * T * rows)
+    got = []
+    for shape in (2, 4):
+        check(lib().tl_memset(yb.ptr, 0xff, yb.nbytes, None))
+        check(lib().tl_debug_half_gemm(w.h, xb.ptr, yb.ptr, T, shape, slices, None))
+        got.append(yb.to_numpy(np.uint32, (T, rows)))
+    assert np.array_equal(got[0], got[1])
+    w.free()
+
+
+@pytest.mark.parametrize("rows,cols,T,slices", [(511, 256, 64, 1), (513, 1280, 65, 2), (1030, 512, 63, 1)])
+def test_half_plane_gemm_waves_of_64_rows(E, pkg, rows, cols, T, slices):
+    """512 rows a workgroup around its tile. The bound of test_half_plane_gemm_edges."""
+    from tinyllama_cpp_amd.capi import check, lib
+    S = pkg.synth
+    rng = np.random.default_rng(rows)
+    w = E.QWeight(Q4_K, S.random_blocks(Q4_K, rows * cols // 256, rng, w_std=1.0 / np.sqrt(cols)), rows, cols)
+    x = rng.standard_normal((T, cols)).astype(np.float32)
+    xb, yb = E.DeviceBuffer.from_numpy(x), E.DeviceBuffer(4 * T * rows)
+    check(lib().tl_debug_half_gemm(w.h, xb.ptr, yb.ptr, T, 3, slices, None))
+    W = w.dequantize().astype(np.float64)
+    scale = np.abs(x).astype(np.float64) @ (np.abs(W) + 4.0 * np.abs(W).max(axis=1, keepdims=True)).T
+    y = yb.to_numpy(np.float32, (T, rows))
+    assert (np.abs(y - x.astype(np.float64) @ W.T) <= (2.0 ** -22 + 48 * 2.0 ** -24 + cols / 256 * 2.0 ** -24) * scale).all()
+    w.free()
+
+
 @pytest.mark.parametrize("shape", [2, 3, 4])
 @pytest.mark.parametrize("T", [512, 513, 1024, 1050, 1500])
 def test_half_plane_gemm_panels_of_token_tiles(E, pkg, shape, T):

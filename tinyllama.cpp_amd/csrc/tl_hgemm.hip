@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "tl_internal.h"
+#include "tl_lds.h"
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
@@ -194,6 +195,103 @@ struct HSegs {  // up to three matrices over the same activations (q | k | v, ga
   int mt_end[3];
 };
 
+// Which tile a workgroup computes.
+// consecutive workgroups go to the 8 XCDs in turn: each XCD walks a contiguous range, panels of `panel` token tiles one after another
+// and inside a panel token tiles fastest. The workgroups that read the same weights thereby share an L2, and the 32 or 64 that an
+// XCD runs at a time read 8 token tiles' activations and 4 or 8 row tiles' weights; with all token tiles side by side, 2048 tokens
+// (32 tiles, 32 MB of activations a round) fetched three times as much through the fabric, which costs time and clock: 28672 x 4096
+// in Q4_K times 2048 tokens 986 -> 967 us in waves of 64 rows and 1200 -> 1116 in shape 4, 16384 x 3072 in Q6_K 682 -> 648.
+struct Place {
+  int slice, nt, mt, seg;
+};
+__device__ __forceinline__ Place place_of(const HSegs& segs, int mtiles, int ntiles, int nslices, int panel) {
+  const int total = mtiles * ntiles * nslices, per8 = total >> 3, rem8 = total & 7;
+  const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+  const int v = xcd * per8 + (xcd < rem8 ? xcd : rem8) + at;
+  Place p;
+  p.slice = v / (mtiles * ntiles);
+  const int in_slice = v - p.slice * mtiles * ntiles;
+  p.nt = 0, p.mt = in_slice;
+  if (ntiles > 1) {  // (one tile of tokens: launches of 6 us, which need none of these divisions)
+    const int pi = in_slice / (panel * mtiles), in_panel = in_slice - pi * panel * mtiles;
+    const int width = ntiles - panel * pi < panel ? ntiles - panel * pi : panel;
+    p.mt = in_panel / width;
+    p.nt = panel * pi + in_panel - p.mt * width;
+  }
+  p.seg = (p.mt >= segs.mt_end[0]) + (p.mt >= segs.mt_end[1]);
+  if (p.seg) p.mt -= segs.mt_end[p.seg - 1];
+  return p;
+}
+
+// acc += a super-block's sums times the rows' factors and the tokens' powers of two. bs: its block sums [token][hi 8 | lo 8], then 2^-k
+// (APART: sums of the hi part's products t and of the small ones tl)
+template <int TYPE, int TK, int NI, int MI>
+__device__ __forceinline__ void add_superblock(typename Tile<TK>::Acc (&acc)[NI][MI], const typename Tile<TK>::Acc (&t)[NI][MI],
+                                               const typename Tile<TK>::Acc (&tl)[NI][MI], const typename Tile<TK>::Acc (&c8)[NI][MI],
+                                               const WHead<TYPE> (&H)[MI], const _Float16* ab, const _Float16* invs, int fr, int fg) {
+  typedef Tile<TK> TL;
+  typedef typename TL::Acc Acc;
+  constexpr bool APART = MI == 1;
+  const Acc zero = {};
+  float d[MI], dm[MI];
+  f16x8 mn[MI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    d[i] = TYPE == TL_Q4_K ? h2f(H[i].h[0] & 0xFFFFu) : TYPE == TL_Q6_K ? h2f(H[i].d) : TYPE == TL_Q8_K ? h2f_scale(H[i].d) : 1.f;
+    if (TYPE == TL_Q4_K) {
+      mn[i] = q4_minima(H[i].h[2], H[i].h[3]);
+      dm[i] = -h2f(H[i].h[0] >> 16);
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < NI; ++n) {
+    f16x8 bs;
+    if (TYPE == TL_Q4_K) {
+      bs = *reinterpret_cast<const f16x8*>(ab + (TK * n + fr) * 16 + (fg & 1) * 8);
+      if (TK == 16 && fg >= 2) bs = f16x8{};  // (the instruction's columns 16..31: nothing)
+    }
+    const float* inv = reinterpret_cast<const float*>(invs) + TK * n;
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      Acc s;
+      if (TYPE == TL_Q4_K) s = TL::mfma(bs, mn[i], zero);
+#pragma unroll
+      for (int q = 0; q < TL::E / 4; ++q) {
+        const f32x4 iv = *reinterpret_cast<const f32x4*>(inv + TL::quad(q, fg));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float x = TYPE == TL_Q8_0 ? c8[n][i][4 * q + e] : d[i] * (APART ? t[n][i][4 * q + e] + tl[n][i][4 * q + e] : t[n][i][4 * q + e]);
+          if (TYPE == TL_Q4_K) x = fmaf(dm[i], s[4 * q + e], x);
+          acc[n][i][4 * q + e] = fmaf(iv[e], x, acc[n][i][4 * q + e]);
+        }
+      }
+    }
+  }
+}
+template <int TK, int NI, int MI>
+__device__ __forceinline__ void store_tile(float* __restrict__ y, const float* __restrict__ resid, const typename Tile<TK>::Acc (&acc)[NI][MI],
+                                           int n0, int m0, int T, int M, int fr, int fg) {
+#pragma unroll
+  for (int n = 0; n < NI; ++n)
+#pragma unroll
+    for (int q = 0; q < Tile<TK>::E / 4; ++q) {
+      const int t0 = n0 + TK * n + Tile<TK>::quad(q, fg);
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        const int r = m0 + TK * i + fr;
+        if (r >= M) continue;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (t0 + e < T) {
+            const size_t o = (size_t)(t0 + e) * M + r;
+            const float val = acc[n][i][4 * q + e];
+            y[o] = resid ? resid[o] + val : val;
+          }
+        }
+      }
+    }
+}
+
 // Workgroup: NW waves of TK MI rows each x TK NI tokens. LDS: two buffers of a super-block's activation tile, [4 x 64
 // columns][2 parts][tokens][64] f16, the 16-byte pieces of a token's 128 bytes at piece ^ (token / 2 & 7): the 16
 // consecutive tokens of a fragment read and the 2 x 8 pieces of a staging write cover the 64 banks once; behind them the
@@ -211,26 +309,10 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
   constexpr bool CHUNKED = TYPE == TL_Q4_K || TYPE == TL_Q6_K;
   constexpr bool RINGED = BN > 32;                                // the tile goes through a ring of three 64-column steps
   extern __shared__ __attribute__((aligned(16))) _Float16 hlds[];
-  // consecutive workgroups go to the 8 XCDs in turn: each XCD walks a contiguous range, panels of `panel` token tiles one after another
-  // and inside a panel token tiles fastest. The workgroups that read the same weights thereby share an L2, and the 32 or 64 that an
-  // XCD runs at a time read 8 token tiles' activations and 4 or 8 row tiles' weights; with all token tiles side by side, 2048 tokens
-  // (32 tiles, 32 MB of activations a round) fetched three times as much through the fabric, which costs time and clock: 28672 x 4096
-  // in Q4_K times 2048 tokens 986 -> 967 us in shape 3 and 1200 -> 1116 in shape 4, 16384 x 3072 in Q6_K 682 -> 648.
-  const int total = mtiles * ntiles * nslices, per8 = total >> 3, rem8 = total & 7;
-  const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
-  const int v = xcd * per8 + (xcd < rem8 ? xcd : rem8) + at;
-  const int slice = v / (mtiles * ntiles), in_slice = v - slice * mtiles * ntiles;
-  int nt = 0, mt = in_slice;
-  if (ntiles > 1) {  // (one tile of tokens: launches of 6 us, which need none of these divisions)
-    const int pi = in_slice / (panel * mtiles), in_panel = in_slice - pi * panel * mtiles;
-    const int width = ntiles - panel * pi < panel ? ntiles - panel * pi : panel;
-    mt = in_panel / width;
-    nt = panel * pi + in_panel - mt * width;
-  }
-  const int seg = (mt >= segs.mt_end[0]) + (mt >= segs.mt_end[1]);
-  if (seg) mt -= segs.mt_end[seg - 1];
-  const QW w = segs.w[seg];
-  float* __restrict__ y = segs.y[seg];
+  const Place pl = place_of(segs, mtiles, ntiles, nslices, panel);
+  const QW w = segs.w[pl.seg];
+  float* __restrict__ y = segs.y[pl.seg];
+  const int slice = pl.slice, nt = pl.nt, mt = pl.mt;
   const int M = w.rows, K = w.cols;
   const int nsb_all = (K + 255) >> 8, per = (nsb_all + nslices - 1) / nslices;
   const int sb0 = slice * per, nsb = nsb_all - sb0 < per ? nsb_all - sb0 : per;
@@ -445,41 +527,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
           for (int r = 0; r < XR; ++r) *reinterpret_cast<f16x8*>(xn + c * STEP + xl[r]) = xr[c][r];
       }
     }
-    // the super-block's sums times the rows' factors and the tokens' powers of two
-    float d[MI], dm[MI];
-    f16x8 mn[MI];
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-      d[i] = TYPE == TL_Q4_K ? h2f(H[i].h[0] & 0xFFFFu) : TYPE == TL_Q6_K ? h2f(H[i].d) : TYPE == TL_Q8_K ? h2f_scale(H[i].d) : 1.f;
-      if (TYPE == TL_Q4_K) {
-        mn[i] = q4_minima(H[i].h[2], H[i].h[3]);
-        dm[i] = -h2f(H[i].h[0] >> 16);
-      }
-    }
-#pragma unroll
-    for (int n = 0; n < NI; ++n) {
-      f16x8 bs;
-      if (TYPE == TL_Q4_K) {
-        bs = *reinterpret_cast<const f16x8*>(ab + (TK * n + fr) * 16 + (fg & 1) * 8);
-        if (NG == 4 && fg >= 2) bs = f16x8{};  // (the instruction's columns 16..31: nothing)
-      }
-      const float* inv = reinterpret_cast<const float*>(ab + 16 * BN) + TK * n;
-#pragma unroll
-      for (int i = 0; i < MI; ++i) {
-        Acc s;
-        if (TYPE == TL_Q4_K) s = TL::mfma(bs, mn[i], zero);
-#pragma unroll
-        for (int q = 0; q < TL::E / 4; ++q) {
-          const f32x4 iv = *reinterpret_cast<const f32x4*>(inv + TL::quad(q, fg));
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            float x = TYPE == TL_Q8_0 ? c8[n][i][4 * q + e] : d[i] * (APART ? t[n][i][4 * q + e] + tl[n][i][4 * q + e] : t[n][i][4 * q + e]);
-            if (TYPE == TL_Q4_K) x = fmaf(dm[i], s[4 * q + e], x);
-            acc[n][i][4 * q + e] = fmaf(iv[e], x, acc[n][i][4 * q + e]);
-          }
-        }
-      }
-    }
+    add_superblock<TYPE, TK, NI, MI>(acc, t, tl, c8, H, ab, ab + 16 * BN, fr, fg);
     if (NEXT) {
 #pragma unroll
       for (int i = 0; i < MI; ++i) H[i] = Hn[i];
@@ -490,25 +538,289 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
   for (int b = 0; b + 1 < nsb; ++b) superblock(b, std::true_type{});
   superblock(nsb - 1, std::false_type{});
 
+  store_tile<TK, NI, MI>(y, resid, acc, n0, m0, T, M, fr, fg);
+}
+
+// The same product in workgroups of eight waves and 64 tokens, one on a CU, rows in whole super-blocks: activations and weights go from
+// memory to LDS directly (tl_lds_load16), the weights as they lie in memory, so that neither needs registers on the way. In the kernel
+// above every step's LDS stores wait for loads asked for one step before, and with them, since loads are counted in order, for the
+// weights asked for just before those; here whatever a step asks for has a step and a half to arrive. It also issues an eighth fewer
+// vector instructions. The same operands in the same order: the same bits. 28672 x 4096 in Q4_K, us at 128 / 512 / 2048 tokens: 256
+// rows 78 / 312 / 1057 -> 74 / 299 / 1006, waves of 64 rows 87 / 290 / 962 -> - / 266 / 892; 16384 x 3072 in Q6_K 72 / 179 / 634 -> 67
+// / 160 / 604; 28672 x 4096 in Q8_0 104 / 389 / 1361 -> 97 / 375 / 1272. What bounds it: power. The matrix instructions alone, at the clock
+// that they leave, take three quarters of the time at 2048 tokens; taking out the unpacking, the fragment reads or the loads gives 3 to 5 %
+// each.
+// LDS, in bytes: activations of four 64-column steps [part][64 tokens][64] f16; two halves of a super-block of the rows' nibbles (bytes),
+// behind them Q6_K's high bits; the rows' heads of two super-blocks (16 bytes and, Q6_K and Q8_K, the dword that d lies in); block sums and
+// powers of two of two super-blocks. 16-byte pieces of a row are exchanged so that the 16 rows of a fragment read cover the 64 banks once.
+template <int TYPE, int MI, int NW>
+struct LdsMap {
+  static constexpr int BM = 32 * MI * NW, XSLOT = 64 * 256;
+  static constexpr int QROW = TYPE == TL_Q4_K || TYPE == TL_Q6_K ? 64 : 128, HROW = TYPE == TL_Q6_K ? 32 : 0;  // bytes of half a super-block
+  static constexpr bool H16 = TYPE != TL_Q8_K, D4 = TYPE == TL_Q6_K || TYPE == TL_Q8_K;
+  static constexpr int W = 4 * XSLOT, WSLOT = BM * (QROW + HROW);
+  static constexpr int H = W + 2 * WSLOT, HSLOT = BM * ((H16 ? 16 : 0) + (D4 ? 4 : 0));
+  static constexpr int A = H + 2 * HSLOT, ASLOT = 64 * 32 + 1024;
+  static constexpr int BYTES = A + 2 * ASLOT;
+};
+template <int TYPE, int MI, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void hgemm_lds_kernel(HSegs segs, HAct act, const float* __restrict__ resid, int T, int mtiles,
+                                                             int ntiles, int nslices, int panel) {
+  typedef LdsMap<TYPE, MI, NW> L;
+  typedef Tile<32> TL;
+  typedef f32x16 Acc;
+  constexpr int NI = 2, US = 4, BN = 64, BM = L::BM;
+  constexpr bool CHUNKED = TYPE == TL_Q4_K || TYPE == TL_Q6_K, APART = MI == 1;
+  static_assert(NW == 8 && (MI == 1 || MI == 2), "");
+  extern __shared__ __attribute__((aligned(16))) _Float16 hlds[];
+  unsigned char* const lds = reinterpret_cast<unsigned char*>(hlds);
+  const Place pl = place_of(segs, mtiles, ntiles, nslices, panel);
+  const QW w = segs.w[pl.seg];
+  float* __restrict__ y = segs.y[pl.seg];
+  const int M = w.rows, K = w.cols;
+  const int nsb_all = K >> 8, per = (nsb_all + nslices - 1) / nslices;
+  const int sb0 = __builtin_amdgcn_readfirstlane(pl.slice * per), nsb = nsb_all - sb0 < per ? nsb_all - sb0 : per;
+  if (nslices > 1) y += (size_t)pl.slice * (size_t)T * (size_t)M;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fr = lane & 31, fg = lane >> 5;
+  const int n0 = pl.nt * BN, tile0 = pl.mt * BM, m0 = tile0 + wave * 32 * MI;
+  const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)lds;
+  auto row_at = [&](int r) { return (unsigned)(r < M ? r : M - 1); };  // (rows beyond the last: its values, never stored)
+  // what this lane fetches: 16-byte pieces of the activations, of the wave's rows, of 64 rows' heads (MI 1: two waves fetch the same)
+  constexpr int XI = 16 / NW, QI = MI * L::QROW / 32, HI = L::HROW ? MI : 0;
+  unsigned xoff[XI], qoff[QI], hoff[HI ? HI : 1];
+  const int xpart = wave >= NW / 2;  // (a wave's pieces are of one part)
+#pragma unroll
+  for (int i = 0; i < XI; ++i) {
+    const int tok = ((wave * XI + i) * 8 + (lane >> 3)) & (BN - 1);
+    const int t = n0 + tok < T ? n0 + tok : T - 1;
+    xoff[i] = ((unsigned)t * (unsigned)K + (((lane & 7) ^ ((tok >> 1) & 7)) << 3)) * 2u;
+  }
+  const char* xbase = tl_uniform(reinterpret_cast<const char*>(act.x + (xpart ? act.ps : 0)));
+#pragma unroll
+  for (int i = 0; i < QI; ++i) {
+    const int row = L::QROW == 64 ? i * 16 + (lane >> 2) : i * 8 + (lane >> 3);
+    const int piece = L::QROW == 64 ? (lane & 3) ^ ((row >> 2) & 3) : (lane & 7) ^ ((row >> 1) & 7);
+    qoff[i] = row_at(m0 + row) * (unsigned)(CHUNKED ? K >> 1 : K) + (piece << 4);
+  }
+#pragma unroll
+  for (int i = 0; i < HI; ++i) {
+    const int row = i * 32 + (lane >> 1);
+    hoff[i] = row_at(m0 + row) * (unsigned)(K >> 2) + (((lane & 1) ^ ((row >> 3) & 1)) << 4);
+  }
+  const int head64 = MI == 1 ? wave >> 1 : wave;
+  const unsigned hrow = row_at(tile0 + head64 * 64 + lane), headoff = hrow * (unsigned)(K >> 4), drow = hrow * (unsigned)nsb_all;
+  const unsigned char *q_base = tl_uniform(w.p0), *hi_base = tl_uniform(w.p1);
+  const unsigned char* head_base = tl_uniform(TYPE == TL_Q6_K ? w.p2 : w.p1);
+  const unsigned char* d_base = tl_uniform(TYPE == TL_Q6_K ? w.p3 : w.p1);
+  const int apiece = wave % 3;  // two of block sums, one of powers of two
+  const char* abase = tl_uniform(apiece < 2 ? reinterpret_cast<const char*>(act.bs + (size_t)n0 * 16) + apiece * 1024 : reinterpret_cast<const char*>(act.inv + n0));
+  const unsigned astride = __builtin_amdgcn_readfirstlane((unsigned)act.tpad * (apiece < 2 ? 32 : 4));
+  const unsigned aoff = (apiece < 2 ? lane : lane & 15) * 16;
+
+  auto fetch_x = [&](int sb, int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < XI; ++i) tl_lds_load16(lds0 + c * L::XSLOT + (wave * XI + i) * 1024, xoff[i], xbase + (size_t)(sb * 4 + c) * 128);
+  };
+  auto fetch_w = [&](int sb, int h) __attribute__((always_inline)) {
+    const unsigned b = lds0 + L::W + h * L::WSLOT;
+#pragma unroll
+    for (int i = 0; i < QI; ++i) tl_lds_load16(b + wave * (32 * MI * L::QROW) + i * 1024, qoff[i], q_base + (size_t)(2 * sb + h) * L::QROW);
+#pragma unroll
+    for (int i = 0; i < HI; ++i) tl_lds_load16(b + BM * L::QROW + (wave * MI + i) * 1024, hoff[i], hi_base + (size_t)(2 * sb + h) * L::HROW);
+  };
+  auto fetch_head = [&](int sb, int par) __attribute__((always_inline)) {
+    const unsigned b = lds0 + L::H + par * L::HSLOT;
+    if (L::H16) tl_lds_load16(b + head64 * 1024, headoff, head_base + (size_t)sb * 16);
+    // (the aligned dword around a 2-byte d: a plane is a whole number of 256 bytes)
+    if (L::D4) tl_lds_load4(b + (L::H16 ? BM * 16 : 0) + head64 * 256, ((drow + sb) & ~1u) * 2u, d_base);
+  };
+  auto fetch_aux = [&](int sb, int par) __attribute__((always_inline)) {
+    tl_lds_load16(lds0 + L::A + par * L::ASLOT + apiece * 1024, aoff, abase + (size_t)sb * astride);
+  };
+  constexpr int WLOADS = QI + HI, HLOADS = (L::H16 ? 1 : 0) + (L::D4 ? 1 : 0);
+  // what this lane reads: its eight columns of operand k in a step's activations, its weights of odd and even steps
+  int xo[4], qo[2][2], ho[2];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int piece = CHUNKED ? 4 * fg + k : 4 * (k >> 1) + 2 * fg + (k & 1);
+    xo[k] = (fr * 128 + ((piece ^ ((fr >> 1) & 7)) << 4)) / 2;
+  }
+#pragma unroll
+  for (int o = 0; o < 2; ++o) {
+    if (L::QROW == 64) {
+      qo[o][0] = fr * 64 + (((2 * o + fg) ^ ((fr >> 2) & 3)) << 4);
+      qo[o][1] = 0;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) qo[o][k] = fr * 128 + (((4 * o + 2 * k + fg) ^ ((fr >> 1) & 7)) << 4);
+    }
+    ho[o] = fr * 32 + ((o ^ ((fr >> 3) & 1)) << 4) + fg * 8;
+  }
+  auto read_w = [&](WStep<TYPE>(&g)[MI], int u) __attribute__((always_inline)) {
+    const unsigned char* b = lds + L::W + (u >> 1) * L::WSLOT;
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const unsigned char* r = b + (wave * MI + i) * (32 * L::QROW);
+      g[i].q = *reinterpret_cast<const u32x4*>(r + qo[u & 1][0]);
+      if (L::QROW == 128) g[i].q1 = *reinterpret_cast<const u32x4*>(r + qo[u & 1][1]);
+      if (L::HROW) g[i].hi = *reinterpret_cast<const u32x2*>(b + BM * L::QROW + (wave * MI + i) * 1024 + ho[u & 1]);
+    }
+  };
+  auto read_head = [&](WHead<TYPE>(&g)[MI], int sb, int par) __attribute__((always_inline)) {
+    const unsigned char* b = lds + L::H + par * L::HSLOT;
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const int row = (wave * MI + i) * 32 + fr;
+      if (L::H16) g[i].h = *reinterpret_cast<const u32x4*>(b + row * 16);
+      if (L::D4) {
+        const unsigned two = *reinterpret_cast<const unsigned*>(b + (L::H16 ? BM * 16 : 0) + row * 4);
+        g[i].d = (two >> (16 * ((row_at(tile0 + row) * (unsigned)nsb_all + sb) & 1))) & 0xFFFFu;
+      }
+    }
+  };
+
+  const Acc zero = {};
+  Acc acc[NI][MI];
 #pragma unroll
   for (int n = 0; n < NI; ++n)
 #pragma unroll
-    for (int q = 0; q < TL::E / 4; ++q) {
-      const int t0 = n0 + TK * n + TL::quad(q, fg);
+    for (int i = 0; i < MI; ++i) acc[n][i] = zero;
+  WStep<TYPE> W[2][MI];
+  WHead<TYPE> H[MI], Hn[MI];
+  fetch_head(sb0, 0);
+  fetch_w(sb0, 0);
+  fetch_x(sb0, 0);
+  fetch_x(sb0, 1);
+  fetch_aux(sb0, 0);
+  fetch_w(sb0, 1);
+  fetch_x(sb0, 2);
+  tl_lds_barrier<0>();
+  read_head(H, sb0, 0);
+  read_w(W[0], 0);
+
+  auto superblock = [&](int b, auto next_c) __attribute__((always_inline)) {
+    constexpr bool NEXT = decltype(next_c)::value;  // another super-block follows: fetch it on the way
+    const int sb = __builtin_amdgcn_readfirstlane(sb0 + b), cur = __builtin_amdgcn_readfirstlane(b & 1);  // (scalar: bases of loads)
+    const _Float16* ab = hlds + (L::A + cur * L::ASLOT) / 2;
+    Acc t[NI][MI], tl[NI][MI], c8[NI][MI];  // (as above)
+    unsigned h1[MI], h3[MI];
+    if (TYPE == TL_Q4_K) {
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
-        const int r = m0 + TK * i + fr;
-        if (r >= M) continue;
+        h1[i] = H[i].h[1] >> (4 * fg);
+        h3[i] = H[i].h[3] >> (2 * fg);
+      }
+    }
+    constexpr int RD = MI == 1 ? 2 : 1, RING = RD + 1, NF = 4 * US * NI;
+    f16x8 fa[RING][2];
+    auto read_frags = [&](int f) __attribute__((always_inline)) {  // operand f / NI of the super-block, token fragment f % NI
+      const int kk = f / NI, n = f % NI;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          if (t0 + e < T) {
-            const size_t o = (size_t)(t0 + e) * M + r;
-            const float val = acc[n][i][4 * q + e];
-            y[o] = resid ? resid[o] + val : val;
+      for (int p = 0; p < 2; ++p)
+        fa[f % RING][p] = *reinterpret_cast<const f16x8*>(hlds + ((kk >> 2) * L::XSLOT + (p * BN + 32 * n) * 128) / 2 + xo[kk & 3]);
+    };
+#pragma unroll
+    for (int f = 0; f < RD; ++f) read_frags(f);
+#pragma unroll
+    for (int u = 0; u < US; ++u) {
+      // Step u of the super-block lies in slot u and is read up to its barrier, the next step from its own start on. What a step asks for is
+      // there at the barrier of the step after: activations three steps ahead, into the slot of the step before; the next
+      // super-block's weights as soon as both steps of a half have been read into registers (a step ahead); heads and block sums
+      // where the other super-block's are long read
+      if (u == 0) fetch_x(sb, 3);
+      else if (NEXT) fetch_x(sb + 1, u - 1);
+      if (NEXT && u == 1) {
+        fetch_w(sb + 1, 0);
+        fetch_head(sb + 1, cur ^ 1);
+      }
+      if (NEXT && u == 2) fetch_aux(sb + 1, cur ^ 1);
+      if (NEXT && u == 3) fetch_w(sb + 1, 1);
+      if (NEXT || u < US - 1) read_w(W[(u + 1) & 1], (u + 1) & 3);
+      if (NEXT && u == 3) read_head(Hn, sb + 1, cur ^ 1);
+      __builtin_amdgcn_sched_barrier(0);
+      Scale4 sc[MI];
+      f16x2 s6[MI][2];
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        if (TYPE == TL_Q4_K) sc[i] = q4_scale(h1[i], h3[i], 2 * u);
+        if (TYPE == TL_Q6_K) {
+          const unsigned sw = H[i].h[u] >> (16 * fg);
+          const _Float16 a = (_Float16)(short)(signed char)(sw & 0xFFu), c = (_Float16)(short)(signed char)((sw >> 8) & 0xFFu);
+          s6[i][0] = f16x2{a, a};
+          s6[i][1] = f16x2{c, c};
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int kk = 4 * u + k;
+        f16x8 bh[MI], bl[MI];
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+          const WStep<TYPE>& g = W[u & 1][i];
+          if (TYPE == TL_Q4_K) bh[i] = q4_operand(g.q[k], sc[i]);
+          else if (TYPE == TL_Q6_K) q6_operand(g.q[k], g.hi[k >> 1], k & 1, s6[i][k >> 1], bh[i], bl[i]);
+          else bh[i] = k < 2 ? q8_operand(g.q[2 * (k & 1)], g.q[2 * (k & 1) + 1]) : q8_operand(g.q1[2 * (k & 1)], g.q1[2 * (k & 1) + 1]);
+        }
+        const bool fresh = TYPE == TL_Q8_0 ? (k & 1) == 0 : kk == 0;
+#pragma unroll
+        for (int n = 0; n < NI; ++n) {
+          const int f = kk * NI + n;
+          __builtin_amdgcn_sched_barrier(0);
+          if (f + RD < NF) read_frags(f + RD);
+          __builtin_amdgcn_sched_barrier(0);
+          const f16x8 a0 = fa[f % RING][0], a1 = fa[f % RING][1];
+#pragma unroll
+          for (int i = 0; i < MI; ++i) {
+            Acc& c = APART ? tl[n][i] : t[n][i];
+            c = TL::mfma(a1, bh[i], fresh ? zero : c);
+          }
+#pragma unroll
+          for (int i = 0; i < MI; ++i) t[n][i] = TL::mfma(a0, bh[i], APART && fresh ? zero : t[n][i]);
+          if (TYPE == TL_Q6_K) {
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+              Acc& c = APART ? tl[n][i] : t[n][i];
+              c = TL::mfma(a0, bl[i], c);
+            }
+          }
+        }
+        if (TYPE == TL_Q8_0 && (k & 1)) {
+#pragma unroll
+          for (int i = 0; i < MI; ++i) {
+            const float d = h2f_scale((H[i].h[u] >> (16 * (k >> 1))) & 0xFFFFu);
+#pragma unroll
+            for (int n = 0; n < NI; ++n) {
+#pragma unroll
+              for (int e = 0; e < 16; ++e) {
+                const float c = APART ? t[n][i][e] + tl[n][i][e] : t[n][i][e];
+                c8[n][i][e] = kk == 1 ? d * c : fmaf(d, c, c8[n][i][e]);
+              }
+              asm volatile("" : "+v"(c8[n][i]));
+            }
           }
         }
       }
+      __builtin_amdgcn_sched_barrier(0);
+      if (NEXT) {
+        if (u == 0) tl_lds_barrier<XI>();
+        if (u == 1) tl_lds_barrier<XI + WLOADS + HLOADS>();
+        if (u == 2) tl_lds_barrier<XI + 1>();
+        if (u == 3) tl_lds_barrier<XI + WLOADS>();
+      } else {
+        if (u == 0) tl_lds_barrier<XI>();
+        if (u == 1) tl_lds_barrier<0>();
+      }
     }
+    add_superblock<TYPE, 32, NI, MI>(acc, t, tl, c8, H, ab, ab + 16 * BN, fr, fg);
+    if (NEXT) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i) H[i] = Hn[i];
+    }
+  };
+  for (int b = 0; b + 1 < nsb; ++b) superblock(b, std::true_type{});
+  superblock(nsb - 1, std::false_type{});
+  store_tile<32, NI, MI>(y, resid, acc, n0, m0, T, M, fr, fg);
 }
 
 // ---- producer of the activation planes ----------------------------------------------------------------------------------
@@ -647,38 +959,41 @@ __global__ __launch_bounds__(256) void hsplit_kernel(const float* __restrict__ x
 // The shapes of a workgroup. Up to 16 tokens: 64 rows, four workgroups (sixteen waves) on a CU, which keeps the most weight
 // bytes in flight: a step of 16 sequences of the 8B shape (8 layers) 0.96 ms against 0.98 with the 32-token shape (Q8_0 of
 // 1.1B 0.58 against 0.63). Up to 64: 128 rows x 32 tokens, two on a CU (32 sequences 1.04 ms; 64: 1.46 against 1.49 with
-// 64-token tiles). More: 64-token tiles, each operand unpacked once for two token fragments. No one unit is full there: in shape 2
-// the matrix cores are busy in 36 % (28672 x 4096 in Q4_K, 128 tokens, 224 workgroups on 256 CUs), 42 % (512 tokens) and 50 %
-// (16384 x 3072 in Q6_K, 2048 tokens) of the cycles, at 2.1, 1.9 and 1.8 GHz, the two waves of a SIMD wait in 29 % of theirs for
-// data and barriers and in 37 % for their turn to issue. Without unpacking, fragment reads and scale FMAs a 512-token chunk is 20 %
-// shorter. Which of the three shapes is taken is a matter of filling the chip, so the plan below weighs them.
+// 64-token tiles). More: 64-token tiles, each operand unpacked once for two token fragments, in workgroups of 256 rows (2), of 512 in
+// waves of 64 (3; Q4_K: for others registers or LDS are short) and of 128, two on a CU (4). Which of them is taken is a matter of
+// filling the chip, so the plan below weighs them.
 // (8 layers of the 8B shape in ms, this kernel / the bf16 kernels it replaced: 8 sequences 0.86 / 1.56, 32: 1.05 / 1.62,
 // 64: 1.52 / 2.03, 128: 2.2 / 2.7; a prompt of 512: 5.3 / 7.0.)
 struct HShape {
   int tk, ni, mi, nw, wpe, percu;
+  bool lds;  // hgemm_lds_kernel
 };
-constexpr HShape SHAPE[] = {{16, 1, 1, 4, 4, 4}, {32, 1, 1, 4, 2, 2}, {32, 2, 1, 8, 2, 1}, {32, 2, 2, 4, 2, 2}, {32, 2, 1, 4, 2, 2}};
-// us of a super-block of a workgroup on a full chip (measured before the panels, which made long prompts 2 to 7 % cheaper)
-constexpr float HGEMM_US[] = {1.2f, 2.0f, 4.9f, 9.0f, 5.0f};
+constexpr HShape hgemm_shape(int type, int shape) {
+  constexpr HShape all[] = {{16, 1, 1, 4, 4, 4, false}, {32, 1, 1, 4, 2, 2, false}, {32, 2, 1, 8, 2, 1, true}, {32, 2, 2, 8, 2, 1, true}, {32, 2, 1, 4, 2, 2, false}};
+  if (shape == 3 && type != TL_Q4_K) return {32, 2, 2, 4, 2, 2, false};  // (Q8_K)
+  return all[shape];
+}
+// us of a super-block of a workgroup on a full chip. Shape 3 is priced so that, over the projections of the 1B, 3B and 8B shapes and 65 to
+// 2048 tokens, it is taken as often as where it ran in pairs of 256 rows (at its own 7.4 it would be taken in a sixth more of them, and its
+// single chain of sums rounds more: 2.1e-7 against 1.7e-7 at 2048 columns)
+constexpr float HGEMM_US[] = {1.2f, 2.0f, 4.25f, 7.8f, 5.0f}, HGEMM_US_3_Q8_K = 9.0f;
 // Price of a launch of n workgroups of `per` super-blocks, and of S slices' partial sums of `outputs` numbers.
 // Q4_K and Q8_K, and all formats up to 64 tokens: rounds over the chip x (super-blocks + start and end) + the partial sums written
 // and read once at about 4 TB/s. Q6_K (a third product, longer unpacking) and Q8_0 (16 additions and FMAs a block) beyond: the
 // time of the fullest CU, whose last workgroup takes 0.6 of a pair's time where two share it, and 0.16 of the way to what an even
 // share would take (clocks rise where CUs run dry). Over the projections of the 1B, 3B and 8B shapes and 100 to 2048 tokens that
-// picks within 0.5 % of the best shape and slices on average and 6 % at worst; rounds, which priced Q8_0 like Q4_K and left it one
-// shape, within 3 % and 20: 11264 x 2048 times 512 tokens in Q6_K 108 us, now 96; 3072 x 8192 in Q8_0 109, now 103. (For Q4_K it
-// would choose shape 3 more often, whose single chain of sums rounds more.)
+// picks within 0.7 % (Q6_K), 1 % (Q8_0) and 2 % (Q4_K) of the best shape and slices on average and 11, 11 and 20 % at worst.
 float hgemm_price(int cus, int type, int shape, long n, int per, int S, float outputs) {
-  const HShape& q = SHAPE[shape];
+  const HShape q = hgemm_shape(type, shape);
   if (shape >= 2 && (type == TL_Q6_K || type == TL_Q8_0)) {
-    const float us = type == TL_Q6_K ? (shape == 2 ? 6.4f : 6.85f) : (shape == 2 ? 5.6f : 6.0f), alone = q.percu == 2 ? 0.6f : 1.f;
+    const float us = type == TL_Q6_K ? (shape == 2 ? 6.3f : 6.85f) : (shape == 2 ? 5.5f : 6.0f), alone = q.percu == 2 ? 0.6f : 1.f;
     const long most = (n + cus - 1) / cus;
     const float fullest = q.percu == 2 ? (float)(most / 2) + (most & 1 ? alone : 0.f) : (float)most;
     const float even = (float)n / (float)cus / (float)q.percu;
     return (0.84f * fullest + 0.16f * (even > alone ? even : alone)) * ((float)per + 0.6f) * us + (S > 1 ? (float)S * (0.3f + outputs * 1.4e-6f) : 0.f);
   }
   const long slots = (long)cus * q.percu;
-  return (float)((n + slots - 1) / slots) * (float)(per + (shape < 2 ? 2 : 1)) * HGEMM_US[shape] * (type == TL_Q6_K ? 1.37f : 1.f) +
+  return (float)((n + slots - 1) / slots) * (float)(per + (shape < 2 ? 2 : 1)) * (shape == 3 && !q.lds ? HGEMM_US_3_Q8_K : HGEMM_US[shape]) * (type == TL_Q6_K ? 1.37f : 1.f) +
          (S > 1 ? (float)S * (0.3f + outputs * 2e-6f) : 0.f);
 }
 // the shape and the K slices of the least price
@@ -689,7 +1004,8 @@ HgemmPlan hgemm_plan(const QW* w, int n, int T) {
   float least = -1.f;
   for (int v = lo; v <= hi; ++v) {
     if (v == 3 && (type == TL_Q6_K || type == TL_Q8_0)) continue;  // (spills)
-    const HShape& q = SHAPE[v];
+    if (v == 2 && w[0].cols % 256) continue;                       // (rows that end inside a super-block)
+    const HShape q = hgemm_shape(type, v);
     const int bm = q.tk * q.mi * q.nw, bn = q.tk * q.ni, ntiles = (T + bn - 1) / bn;
     long tiles = 0, rows = 0;
     for (int i = 0; i < n; ++i) {
@@ -711,14 +1027,18 @@ HgemmPlan hgemm_plan(const QW* w, int n, int T) {
 
 template <int TYPE, int V>
 int hgemm_go(const HSegs& g, int mt, const HAct& act, const float* resid, int T, int S, hipStream_t s) {
-  constexpr HShape q = SHAPE[V];
+  constexpr HShape q = hgemm_shape(TYPE, V);
   constexpr int BN = q.tk * q.ni;
-  constexpr size_t lds = (size_t)(BN > 32 ? 3 * 2 * 64 + 2 * 18 : 2 * (4 * 2 * 64 + 18)) * BN * sizeof(_Float16);
+  constexpr size_t lds = q.lds ? (size_t)LdsMap<TYPE, q.mi, q.nw>::BYTES
+                               : (size_t)(BN > 32 ? 3 * 2 * 64 + 2 * 18 : 2 * (4 * 2 * 64 + 18)) * BN * sizeof(_Float16);
+  static_assert(lds <= 160 * 1024, "");
   static TlDeviceOnce lds_raised;
-  auto kernel = hgemm_kernel<TYPE, q.tk, q.ni, q.mi, q.nw, q.wpe>;
+  void (*kernel)(HSegs, HAct, const float*, int, int, int, int, int);
+  if constexpr (q.lds) kernel = hgemm_lds_kernel<TYPE, q.mi, q.nw>;
+  else kernel = hgemm_kernel<TYPE, q.tk, q.ni, q.mi, q.nw, q.wpe>;
   TL_TRY(tl_raise_lds_limit(kernel, (int)lds, lds_raised));
   // panels of eight token tiles and more, all alike: a panel of the one tile that is left over reads all weights again for it (28672 x
-  // 4096 in Q4_K times 513 tokens, nine tiles, 274 us in one panel of shape 3, 281 in eight and one)
+  // 4096 in Q4_K times 513 tokens, nine tiles, 274 us in one panel of shape 3 with 256 rows, 281 in eight and one)
   const int ntiles = (T + BN - 1) / BN, panels = ntiles < 16 ? 1 : ntiles / 8, panel = (ntiles + panels - 1) / panels;
   kernel<<<dim3((unsigned)(mt * ntiles * S)), dim3(64 * q.nw), lds, s>>>(g, act, resid, T, mt, ntiles, S, panel);
   TL_HIP(hipGetLastError());
@@ -728,7 +1048,8 @@ template <int TYPE>
 int hgemm_typed(const QW* w, int n, const HgemmPlan& p, const HAct& act, float* const* out, const float* resid, int T, hipStream_t s) {
   HSegs g = {};
   int mt = 0;
-  const int bm = SHAPE[p.shape].tk * SHAPE[p.shape].mi * SHAPE[p.shape].nw;
+  const int shape = p.shape == 2 && w[0].cols % 256 ? 4 : p.shape;  // (rows that end inside a super-block: shape 4's kernel has the same sums)
+  const int bm = hgemm_shape(TYPE, shape).tk * hgemm_shape(TYPE, shape).mi * hgemm_shape(TYPE, shape).nw;
   for (int i = 0; i < 3; ++i) {
     const int k = i < n ? i : n - 1;  // (unused slots repeat the last matrix; their tile range is empty)
     g.w[i] = w[k];
@@ -736,11 +1057,11 @@ int hgemm_typed(const QW* w, int n, const HgemmPlan& p, const HAct& act, float* 
     if (i < n) mt += (w[i].rows + bm - 1) / bm;
     g.mt_end[i] = mt;
   }
-  if (p.shape == 0) return hgemm_go<TYPE, 0>(g, mt, act, resid, T, p.S, s);
-  if (p.shape == 1) return hgemm_go<TYPE, 1>(g, mt, act, resid, T, p.S, s);
-  if (p.shape == 2) return hgemm_go<TYPE, 2>(g, mt, act, resid, T, p.S, s);
+  if (shape == 0) return hgemm_go<TYPE, 0>(g, mt, act, resid, T, p.S, s);
+  if (shape == 1) return hgemm_go<TYPE, 1>(g, mt, act, resid, T, p.S, s);
+  if (shape == 2) return hgemm_go<TYPE, 2>(g, mt, act, resid, T, p.S, s);
   if constexpr (TYPE == TL_Q4_K || TYPE == TL_Q8_K)
-    if (p.shape == 3) return hgemm_go<TYPE, 3>(g, mt, act, resid, T, p.S, s);
+    if (shape == 3) return hgemm_go<TYPE, 3>(g, mt, act, resid, T, p.S, s);
   return hgemm_go<TYPE, 4>(g, mt, act, resid, T, p.S, s);
 }
 
