@@ -35,61 +35,62 @@ typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
-// y = g * sigmoid(alpha * g) * (u + 1), g = min(gate, limit), u = clamp(up, -limit, limit)  (tl_moe.hip has the operator)
-__device__ __forceinline__ float dense_glu(float g, float u, float limit, float alpha, float up_add) {
-  g = fminf(g, limit);
-  u = fminf(fmaxf(u, -limit), limit);
-  return g / (1.0f + expf(-alpha * g)) * (u + up_add);
-}
-
-// The epilogue of a wave: WM x WN products of 32 x 32, features from f0 on, items from i0 on (items below hi are stored).
+// The epilogue of a wave: WM x WN products of 32 x 32, features from f0 on, items from i0 on (items below hi are stored). 32 items at a
+// time go through the wave's part of LDS (dense_store_floats, left by everybody before), out of which a short loop takes four features
+// a lane, 128 WM consecutive bytes of a row at a time. Out of the registers, whose numbers are fixed at compile time, the activations'
+// code stood there once per accumulator, and a launch's only pass through it waited for instructions: with xIELU behind it,
+// 4096 x 2048 times 1998 tokens took 82 us, 10304 x 2048 with tanh on some features 159, now 51 and 120. The same bits.
+constexpr int dense_store_floats(int wm) { return 32 * (32 * wm + 4); }
 template <int WM, int WN>
-__device__ __forceinline__ void dense_store(const DenseArgs& a, f32x16 (&acc)[WM][WN], float* Y, int f0, int i0, int hi, int lane) {
-  // C layout: lane holds token (lane & 31) of a 32 x 32 product, features (e / 4) * 8 + (lane >> 5) * 4 + (e & 3)
+__device__ __forceinline__ void dense_store(const DenseArgs& a, const f32x16 (&acc)[WM][WN], float* Y, int f0, int i0, int hi, int lane, float* st) {
+  constexpr int LD = 32 * WM + 4, Q = 8 * WM;  // (padded: 16 items' pieces meet no bank twice)
   const bool v4 = (a.ldy & 3) == 0 && ((size_t)Y & 15) == 0;
   const int act_to = a.act_to > 0 ? a.act_to : a.rows;
 #pragma unroll
   for (int j = 0; j < WN; ++j) {
-    const int it = i0 + j * 32 + (lane & 31);
-    if (it >= hi) continue;
-    const int orow = a.y_rows ? a.y_rows[it] : it;
-    float* yr = Y + (size_t)orow * a.ldy;
+    // C layout: lane holds token (lane & 31) of a 32 x 32 product, features (e / 4) * 8 + (lane >> 5) * 4 + (e & 3)
 #pragma unroll
-    for (int i = 0; i < WM; ++i) {
+    for (int i = 0; i < WM; ++i)
 #pragma unroll
-      for (int gq = 0; gq < 4; ++gq) {
-        const int f = f0 + i * 32 + gq * 8 + (lane >> 5) * 4;
-        if (a.glu) {  // (gate, up) pairs: features f, f + 1 -> unit f / 2; f + 2, f + 3 -> the next one
+      for (int gq = 0; gq < 4; ++gq)
+        *reinterpret_cast<f32x4*>(st + (lane & 31) * LD + i * 32 + gq * 8 + (lane >> 5) * 4) =
+            f32x4{acc[i][j][gq * 4], acc[i][j][gq * 4 + 1], acc[i][j][gq * 4 + 2], acc[i][j][gq * 4 + 3]};
+    __builtin_amdgcn_wave_barrier();  // (a wave's LDS operations run in order)
+#pragma unroll 1
+    for (int p = lane; p < 32 * Q; p += 64) {
+      const int tok = p / Q, it = i0 + j * 32 + tok, f = f0 + p % Q * 4;
+      if (it >= hi || f >= a.rows) continue;
+      f32x4 v = *reinterpret_cast<const f32x4*>(st + tok * LD + p % Q * 4);
+      float* yr = Y + (size_t)(a.y_rows ? a.y_rows[it] : it) * a.ldy;
+      if (a.glu) {  // (gate, up) pairs: features f, f + 1 -> unit f / 2; f + 2, f + 3 -> the next one
 #pragma unroll
-          for (int e = 0; e < 2; ++e)
-            if (f + 2 * e + 1 < a.rows)
-              yr[(f >> 1) + e] = tl_glu_apply(a.glu_kind, acc[i][j][gq * 4 + 2 * e], acc[i][j][gq * 4 + 2 * e + 1], a.glu_limit, a.glu_alpha, a.glu_up_add);
-          continue;
-        }
-        if (a.bias) {
+        for (int e = 0; e < 2; ++e)
+          if (f + 2 * e + 1 < a.rows) yr[(f >> 1) + e] = tl_glu_apply(a.glu_kind, v[2 * e], v[2 * e + 1], a.glu_limit, a.glu_alpha, a.glu_up_add);
+        continue;
+      }
+      if (a.bias) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (f + e < a.rows) acc[i][j][gq * 4 + e] += a.bias[f + e];
-        }
-        if (a.softcap > 0.0f) {
+        for (int e = 0; e < 4; ++e)
+          if (f + e < a.rows) v[e] += a.bias[f + e];
+      }
+      if (a.softcap > 0.0f) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[i][j][gq * 4 + e] = a.softcap * tanhf(acc[i][j][gq * 4 + e] / a.softcap);
-        }
-        if (a.act) {
+        for (int e = 0; e < 4; ++e) v[e] = a.softcap * tanhf(v[e] / a.softcap);
+      }
+      if (a.act && f + 4 > a.act_from && f < act_to) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (f + e >= a.act_from && f + e < act_to) acc[i][j][gq * 4 + e] = tl_act_apply(a.act, acc[i][j][gq * 4 + e], a.act_p, a.act_q);
-        }
-        if (v4 && f + 4 <= a.rows) {
-          *reinterpret_cast<float4*>(yr + f) =
-              make_float4(acc[i][j][gq * 4], acc[i][j][gq * 4 + 1], acc[i][j][gq * 4 + 2], acc[i][j][gq * 4 + 3]);
-        } else {
+        for (int e = 0; e < 4; ++e)
+          if (f + e >= a.act_from && f + e < act_to) v[e] = tl_act_apply(a.act, v[e], a.act_p, a.act_q);
+      }
+      if (v4 && f + 4 <= a.rows) {
+        *reinterpret_cast<f32x4*>(yr + f) = v;
+      } else {
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (f + e < a.rows) yr[f + e] = acc[i][j][gq * 4 + e];
-        }
+        for (int e = 0; e < 4; ++e)
+          if (f + e < a.rows) yr[f + e] = v[e];
       }
     }
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
@@ -105,8 +106,11 @@ __global__ __launch_bounds__(256) void dense_gemm_kernel(const DenseArgs a) {
   constexpr int NB = TERMS == 1 ? 2 : 1;               // steps in LDS (three terms in two would leave one workgroup a CU)
   constexpr int KP = BK / 8, RP = 256 / KP;            // 16-byte pieces of a row, rows that the workgroup stages at a time
   constexpr int PW = BM / RP, PX = BN / RP;            // pieces a thread stages
-  __shared__ __attribute__((aligned(16))) unsigned short Ws[NB][BM][LDK];
-  __shared__ __attribute__((aligned(16))) unsigned short Xs[NB][TERMS][BN][LDK];
+  constexpr int TILES = NB * (BM + TERMS * BN) * LDK * 2;
+  static_assert(TILES >= 4 * dense_store_floats(WM) * 4, "");
+  __shared__ __attribute__((aligned(16))) unsigned char tiles[TILES];  // (the waves' outputs at the end)
+  auto& Ws = *reinterpret_cast<unsigned short(*)[NB][BM][LDK]>(tiles);
+  auto& Xs = *reinterpret_cast<unsigned short(*)[NB][TERMS][BN][LDK]>(tiles + NB * BM * LDK * 2);
   __shared__ __attribute__((aligned(16))) unsigned short Xe[NB][FIRST ? 32 : 1][LDK];
   __shared__ int xrow[BN];
   const int tid = threadIdx.x, g = blockIdx.z;
@@ -256,7 +260,7 @@ __global__ __launch_bounds__(256) void dense_gemm_kernel(const DenseArgs a) {
       __syncthreads();
     }
   }
-  dense_store<WM, WN>(a, acc, Y, f0 + wm * WM * 32, t0 + wn * WN * 32, hi, lane);
+  dense_store<WM, WN>(a, acc, Y, f0 + wm * WM * 32, t0 + wn * WN * 32, hi, lane, reinterpret_cast<float*>(tiles) + wave * dense_store_floats(WM));
 }
 
 template <int N>
@@ -360,8 +364,10 @@ __global__ __launch_bounds__(64 * NWM * NWN, 2) void dense_plane_kernel(const De
     }
     slot = slot == NS - 1 ? 0 : slot + 1;
   }
+  static_assert(NS * STAGE >= NW * dense_store_floats(WM) * 4, "");
   dma_wait<0>();
-  dense_store<WM, WN>(a, acc, a.y, f0 + wm * WM * 32, t0 + wn * WN * 32, hi, lane);
+  __syncthreads();  // (the stages have been read and no piece is on its way)
+  dense_store<WM, WN>(a, acc, a.y, f0 + wm * WM * 32, t0 + wn * WN * 32, hi, lane, reinterpret_cast<float*>(dlds) + wave * dense_store_floats(WM));
 }
 
 // x[T][ldx] -> bf16 [T][cols], and behind it the second terms of the first `second` rows; eight columns a thread
