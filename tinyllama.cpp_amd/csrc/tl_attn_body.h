@@ -6,6 +6,7 @@
 #include <type_traits>
 
 #include "tl_chunk.h"
+#include "tl_lanes.h"
 
 namespace tl_attn {
 
@@ -43,11 +44,11 @@ __device__ __forceinline__ float max32(float v) {
   v = dpp_max<0x4E>(v);
   v = dpp_max<0x141>(v);
   v = dpp_max<0x140>(v);
-  return fmaxf(v, __shfl_xor(v, 16));
+  return fmaxf(v, tl_xor<16>(v));
 }
 __device__ __forceinline__ float sum32(float v) {
   v = row_sum16(v);
-  return v + __shfl_xor(v, 16);
+  return v + tl_xor<16>(v);
 }
 // agent-scope accesses for data handed between workgroups inside one launch (the L2s of the 8 XCDs are not coherent with
 // each other for ordinary accesses)

@@ -18,6 +18,7 @@
 
 #include "tl_chunk.h"
 #include "tl_internal.h"
+#include "tl_lanes.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -353,8 +354,8 @@ __global__ __launch_bounds__(256) void attn_batch_decode_kernel(BatchAttnArgs a)
       v[4 + e] = hi[e];
     }
     float bs = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-    bs += __shfl_xor(bs, 1);
-    bs += __shfl_xor(bs, 2);
+    bs += tl_xor<1>(bs);
+    bs += tl_xor<2>(bs);
     if ((tid & 3) == 0) a.xsum[(size_t)(i0 >> 5) * a.tpad + tok] = bs;
     for (int p = 0; p < a.np; ++p) {
       bf16x8 b;
@@ -412,15 +413,7 @@ __global__ __launch_bounds__(1024) void batch_argmax_advance_kernel(const float*
       }
     }
   }
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) {
-    const float ov = __shfl_xor(best, o);
-    const int oi = __shfl_xor(idx, o);
-    if (ov > best || (ov == best && oi < idx)) {
-      best = ov;
-      idx = oi;
-    }
-  }
+  tl_wave_best(best, idx);
   if ((threadIdx.x & 63) == 0) {
     bv[threadIdx.x >> 6] = best;
     bi[threadIdx.x >> 6] = idx;

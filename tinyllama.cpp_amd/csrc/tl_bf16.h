@@ -3,6 +3,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "tl_lanes.h"
+
 __device__ __forceinline__ float tl_bf2f(unsigned short h) { return __uint_as_float((unsigned)h << 16); }
 
 // 8 bf16 weights (one 16-byte load) against 8 FP32 values
@@ -31,12 +33,6 @@ __device__ __forceinline__ float tl_row16_sum(float x) {
   x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x141, 0xf, 0xf, false));  // row_half_mirror
   x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x140, 0xf, 0xf, false));  // row_mirror
   return x;
-}
-
-__device__ __forceinline__ float tl_wave_sum(float s) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o);
-  return s;
 }
 
 // R rows of a bf16 matrix (row r at w + r * stride; rows >= nrows read row 0 and are to be ignored by the caller) against

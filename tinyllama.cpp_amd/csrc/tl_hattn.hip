@@ -22,6 +22,7 @@
 #include <math.h>
 
 #include "tl_internal.h"
+#include "tl_lanes.h"
 #include "tl_lds.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -98,11 +99,8 @@ __global__ __launch_bounds__(256) void kv_planes_kernel(const HPlanesArgs a) {
     for (int t = 0; t < PV; ++t)
       if (fabsf(v[t][i]) < INFINITY) mv = fmaxf(mv, fabsf(v[t][i]));
   }
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) {
-    mk = fmaxf(mk, __shfl_xor(mk, o));
-    mv = fmaxf(mv, __shfl_xor(mv, o));
-  }
+  mk = tl_wave_max(mk);
+  mv = tl_wave_max(mv);
   if ((tid & 63) == 0) {
     red[tid >> 6] = mk;
     red[4 + (tid >> 6)] = mv;
@@ -227,7 +225,7 @@ __global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs a) {
         if (fabsf(x[s][i]) < INFINITY) mx = fmaxf(mx, fabsf(x[s][i]));
       }
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    mx = fmaxf(mx, tl_xor<32>(mx));
     const int k = scale_exp(mx);
     const float f = pow2i(k);
 #pragma unroll
@@ -362,7 +360,7 @@ __global__ __launch_bounds__(256, 2) void hattn_kernel(const HAttnArgs a) {
     ev = __builtin_amdgcn_readfirstlane(stage_ex.y);
     __syncthreads();
   }
-  float l = lrun + __shfl_xor(lrun, 32);
+  float l = lrun + tl_xor<32>(lrun);
   const float unit = 1.0f / HA_P_UNIT * pow2i(-krun);
   float* dst;
   float f = unit;

@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "tl_internal.h"
+#include "tl_lanes.h"
 #include "tl_lds.h"
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -850,8 +851,7 @@ __device__ __forceinline__ void hsplit8(const float* v, _Float16* __restrict__ p
   float top = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) top = fmaxf(top, fabsf(v[e]));
-#pragma unroll
-  for (int o = 16; o >= 1; o >>= 1) top = fmaxf(top, __shfl_xor(top, o));
+  top = tl_wave_max<16>(top);
   if (i0 >= K) return;  // (whole quads of threads: K is a multiple of 32)
   // top * 2^k in [512, 1024); k of zeros and of sub-normals keeps 2^k and 2^-k normal
   int ex = (int)((__builtin_bit_cast(unsigned, top) >> 23) & 255u) - 127;
@@ -865,8 +865,8 @@ __device__ __forceinline__ void hsplit8(const float* v, _Float16* __restrict__ p
 #pragma unroll
   for (int e = 0; e < 8; ++e) x[e] = v[e] * scale;
   float s = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));  // (scaled: below 2^15 whatever the row holds)
-  s += __shfl_xor(s, 1);
-  s += __shfl_xor(s, 2);
+  s += tl_xor<1>(s);
+  s += tl_xor<2>(s);
   if ((i0 & 31) == 0 && (K & 255) == 0) {  // sum of the 32-column block, at the place of its minimum in the operand
     const int j = (i0 >> 5) & 7, at = j < 4 ? 2 * j : 2 * (j - 4) + 1;
     _Float16* o = bs + ((size_t)sb * tpad + t) * 16 + at;
@@ -915,7 +915,7 @@ __global__ __launch_bounds__(HNORM_THREADS) void hsplit_norm_kernel(const float*
       }
     }
   }
-  for (int o = 32; o >= 1; o >>= 1) ssq += __shfl_xor(ssq, o);
+  ssq = tl_wave_sum(ssq);
   if ((tid & 63) == 0) red[tid >> 6] = ssq;
   __syncthreads();
   float sum = 0.f;

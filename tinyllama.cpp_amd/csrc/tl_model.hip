@@ -21,6 +21,7 @@
 #include <rccl/rccl.h>
 
 #include "tl_internal.h"
+#include "tl_lanes.h"
 #include "tl_stack.h"
 
 namespace {
@@ -383,12 +384,7 @@ __device__ __forceinline__ void better(float v, int i, float& best, int& idx) {
 }
 // workgroup-wide first-maximum; result valid in thread 0. bv/bi: >= 16 entries of LDS each
 __device__ __forceinline__ void block_argmax(float& best, int& idx, float* bv, int* bi) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) {
-    const float ov = __shfl_xor(best, o);
-    const int oi = __shfl_xor(idx, o);
-    better(ov, oi, best, idx);
-  }
+  tl_wave_best(best, idx);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) {
     bv[threadIdx.x >> 6] = best;

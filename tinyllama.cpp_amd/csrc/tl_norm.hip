@@ -15,8 +15,7 @@ namespace {
 constexpr int kMaxWaves = 16;
 
 __device__ __forceinline__ float block_sum(float v, float* red) {  // red: kMaxWaves floats of LDS; result in every thread
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+  v = tl_wave_sum(v);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
@@ -537,11 +536,8 @@ void launch_hyper(const HyperArgs& a, size_t lds, hipStream_t s) {
 // ---- two sublayers that read the same x: both outputs (normed on the way in, if asked for) join the residual, and the norms of the
 // two sublayers that read x next share one set of statistics. A thread holds its columns (PER pieces of V) in registers ----------
 __device__ __forceinline__ void block_sum2(float& p, float& q, float* red) {  // red: 2 kMaxWaves floats
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) {
-    p += __shfl_xor(p, o);
-    q += __shfl_xor(q, o);
-  }
+  p = tl_wave_sum(p);
+  q = tl_wave_sum(q);
   if ((threadIdx.x & 63) == 0) {
     red[threadIdx.x >> 6] = p;
     red[kMaxWaves + (threadIdx.x >> 6)] = q;

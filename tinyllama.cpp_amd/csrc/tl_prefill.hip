@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "tl_internal.h"
+#include "tl_lanes.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -214,7 +215,7 @@ __global__ __launch_bounds__(64 * PF_NW) void attn_prefill_mfma_kernel(const flo
       PF_FORCE(tmax);
       if (tcount == 0) PFS(3 + 12 * ph);
 #endif
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+      tmax = fmaxf(tmax, tl_xor<32>(tmax));
       const float mnew = fmaxf(mrun, tmax);  // may still be -inf: a wave's first tiles can lie wholly behind a query
       const float corr = mrun == -INFINITY ? 0.f : expf(mrun - mnew);
       mrun = mnew;
@@ -256,7 +257,7 @@ __global__ __launch_bounds__(64 * PF_NW) void attn_prefill_mfma_kernel(const flo
     }
     PFS(6 + 12 * ph);
     // ---- merge the active waves: M = max_w m_w, L = sum_w l_w e^(m_w - M), O = sum_w O_w e^(m_w - M), in wave order ----
-    const float ltot = lrun + __shfl_xor(lrun, 32);
+    const float ltot = lrun + tl_xor<32>(lrun);
     __syncthreads();  // (second tile of the pair: everybody is done reading the first tile's slots)
     PFS(7 + 12 * ph);
     // every wave is past its last K Q^T of this query tile: the pair's second query tile may replace it (loads issued
@@ -325,8 +326,8 @@ __global__ __launch_bounds__(64 * PF_NW) void attn_prefill_mfma_kernel(const flo
       }
       float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
       float bs = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-      bs += __shfl_xor(bs, 1);  // (the four threads of a block are neighbours of one row: all here together)
-      bs += __shfl_xor(bs, 2);
+      bs += tl_xor<1>(bs);  // (the four threads of a block are neighbours of one row: all here together)
+      bs += tl_xor<2>(bs);
       if (!live) continue;
       const int tok = t.q0 + row, K = nh * HD, i0 = head * HD + 8 * c8;
       if ((c8 & 3) == 0) pl.xsum[(size_t)(i0 >> 5) * pl.tpad + tok] = bs;
@@ -444,7 +445,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_pack_kernel(const PackArgs a)
     }
 #pragma unroll
     for (int e = 0; e < 16; ++e) tmax = fmaxf(tmax, s[e]);
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+    tmax = fmaxf(tmax, tl_xor<32>(tmax));
     const float mnew = fmaxf(mrun, tmax);
     const float corr = mrun == -INFINITY ? 0.f : expf(mrun - mnew);
     mrun = mnew;
@@ -479,12 +480,12 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_pack_kernel(const PackArgs a)
       for (int e = 0; e < 16; ++e) o[b][e] = fmaf(o[b][e], cr[e], u[0][e] + u[1][e]);
     }
   }
-  const float inv = 1.0f / (lrun + __shfl_xor(lrun, 32) + 1e-9f);
+  const float inv = 1.0f / (lrun + tl_xor<32>(lrun) + 1e-9f);
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
-    const int at = min(bad_at[b], __shfl_xor(bad_at[b], 32));
+    const int at = min(bad_at[b], tl_xor<32>(bad_at[b]));
     if (__any(at != 0x7fffffff)) {
-      const float x = bad[b] + __shfl_xor(bad[b], 32);
+      const float x = bad[b] + tl_xor<32>(bad[b]);
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int seen = it.start_pos + min(row0 + acc_row(e, h), rows - 1) / a.group;

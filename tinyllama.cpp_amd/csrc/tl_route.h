@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include "tl_lanes.h"
 #include "tlhip.h"
 
 // One wave (all 64 lanes) picks the `top` largest of z[experts] (LDS; overwritten), the lower index among equals, and writes
@@ -14,11 +15,9 @@ __device__ __forceinline__ void tl_route_select(float* z, int experts, int top, 
     if (over_all) {  // the sum over every expert, before the choices are taken out of z
       top_z = -INFINITY;
       for (int e = lane; e < experts; e += 64) top_z = fmaxf(top_z, z[e]);
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) top_z = fmaxf(top_z, __shfl_xor(top_z, o));
+      top_z = tl_wave_max(top_z);
       for (int e = lane; e < experts; e += 64) all += expf(z[e] - top_z);
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) all += __shfl_xor(all, o);
+      all = tl_wave_sum(all);
     }
     // `top` rounds: the lanes scan the experts not yet chosen for the largest logit (lower index wins among equals)
     float mx = 0.0f, denom = 0.0f, mine = 0.0f;
@@ -33,15 +32,7 @@ __device__ __forceinline__ void tl_route_select(float* z, int experts, int top, 
           bi = e;
         }
       }
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) {
-        const float ov = __shfl_xor(bv, o);
-        const int oi = __shfl_xor(bi, o);
-        if (ov > bv || (ov == bv && oi < bi)) {
-          bv = ov;
-          bi = oi;
-        }
-      }
+      tl_wave_best(bv, bi);
       if (bi == 0x7fffffff) bi = 0;  // only when every logit is NaN
       if (j == 0) mx = bv;
       const float p = expf(bv - mx);
@@ -81,16 +72,14 @@ __device__ __forceinline__ void tl_route_select_groups(float* z, float* key, flo
   };
   float mx = -INFINITY;
   for (int e = lane; e < experts; e += 64) mx = fmaxf(mx, z[e]);
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+  mx = tl_wave_max(mx);
   float sum = 0.0f;
   for (int e = lane; e < experts; e += 64) {
     const float p = expf(z[e] - mx);
     z[e] = p;
     sum += p;
   }
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o);
+  sum = tl_wave_sum(sum);
   const int per = experts / groups;
   for (int e = lane; e < experts; e += 64) {
     z[e] = z[e] / sum;
@@ -113,15 +102,7 @@ __device__ __forceinline__ void tl_route_select_groups(float* z, float* key, flo
         bi = g;
       }
     }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      const float ov = __shfl_xor(bv, o);
-      const int oi = __shfl_xor(bi, o);
-      if (ov > bv || (ov == bv && oi < bi)) {
-        bv = ov;
-        bi = oi;
-      }
-    }
+    tl_wave_best(bv, bi);
     if (bi == 0x7fffffff) bi = 0;
     for (int e = bi * per + lane; e < (bi + 1) * per; e += 64) key[e] = z[e];
     if (lane == 0) gs[bi] = -INFINITY;
@@ -138,15 +119,7 @@ __device__ __forceinline__ void tl_route_select_groups(float* z, float* key, flo
         bi = e;
       }
     }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      const float ov = __shfl_xor(bv, o);
-      const int oi = __shfl_xor(bi, o);
-      if (ov > bv || (ov == bv && oi < bi)) {
-        bv = ov;
-        bi = oi;
-      }
-    }
+    tl_wave_best(bv, bi);
     if (bi == 0x7fffffff) bi = 0;
     const float sc = z[bi];
     denom += sc;
@@ -204,15 +177,14 @@ __device__ __forceinline__ void tl_route_select_sigmoid_groups(float* z, float* 
         bi = g;
       }
     }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      const float ov = __shfl_xor(bv, o);
-      const int oi = __shfl_xor(bi, o);
+    tl_butterfly<32>([&](auto o) __attribute__((always_inline)) {
+      const float ov = tl_xor<decltype(o)::value>(bv);
+      const int oi = tl_xor<decltype(o)::value>(bi);
       if (oi != 0x7fffffff && (bi == 0x7fffffff || ov > bv || (ov == bv && oi < bi))) {
         bv = ov;
         bi = oi;
       }
-    }
+    });
     if (bi == 0x7fffffff) bi = 0;
     if (lane == 0) gs[bi] = INFINITY;
     wave_sync();
@@ -230,15 +202,7 @@ __device__ __forceinline__ void tl_route_select_sigmoid_groups(float* z, float* 
         bi = e;
       }
     }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      const float ov = __shfl_xor(bv, o);
-      const int oi = __shfl_xor(bi, o);
-      if (ov > bv || (ov == bv && oi < bi)) {
-        bv = ov;
-        bi = oi;
-      }
-    }
+    tl_wave_best(bv, bi);
     if (bi == 0x7fffffff) bi = 0;
     if (lane == 0) {
       ids[j] = bi;

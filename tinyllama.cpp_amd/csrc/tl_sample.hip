@@ -23,6 +23,7 @@
 #include <math.h>
 
 #include "tl_internal.h"
+#include "tl_lanes.h"
 
 namespace {
 
@@ -53,8 +54,7 @@ __device__ __forceinline__ int slice_len(int n) { return (n + SK_SLICES - 1) / S
 template <int NT>
 __device__ __forceinline__ float slices_max(const SampleWs* ws, float* sm) {
   float m = threadIdx.x < SK_SLICES ? ws->smax[threadIdx.x] : -INFINITY;
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+  m = tl_wave_max(m);
   if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = m;
   __syncthreads();
   m = sm[0];
@@ -95,8 +95,7 @@ __global__ __launch_bounds__(SK_SLICE_THREADS) void sample_max_kernel(float* __r
   }
   float m = -INFINITY;
   for (int i = lo + tid; i < hi; i += SK_SLICE_THREADS) m = fmaxf(m, logits[i]);
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+  m = tl_wave_max(m);
   if ((tid & 63) == 0) sm[tid >> 6] = m;
   __syncthreads();
   if (tid == 0) {
@@ -116,8 +115,7 @@ __global__ __launch_bounds__(SK_SLICE_THREADS) void sample_sum_kernel(const floa
   const float mx = slices_max<SK_SLICE_THREADS>(ws, sm), inv_t = 1.0f / temperature;
   double part = 0.0;
   for (int i = lo + tid; i < hi; i += SK_SLICE_THREADS) part += exp((double)((logits[i] - mx) * inv_t));
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) part += __shfl_xor(part, o);
+  part = tl_wave_sum(part);
   if ((tid & 63) == 0) sd[tid >> 6] = part;
   __syncthreads();
   if (tid == 0) {

@@ -75,8 +75,7 @@ __device__ __forceinline__ void swa_merge_records(const SwaArgs& a, int nsplit, 
 #pragma unroll
   for (int u = 0; u < 8; ++u) first[u] = lane < a.vdim ? swa_ld_agent(rec + (size_t)(u < nsplit ? u : nsplit - 1) * rs + 2 + lane) : 0.0f;
   float M = mz;
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
+  M = tl_wave_max(M);
   const float sv = a.sink && a.sink_val ? a.sink_val[h] : 0.0f;
   if (a.sink) M = fmaxf(M, sv);
   const float fz = mz == -INFINITY ? 0.0f : expf(mz - M);
@@ -238,14 +237,12 @@ __global__ __launch_bounds__(256) void swa_kernel(const SwaArgs a) {
       if (a.dist_r1) sc -= swa_dist(r1, r2, i - j);
     }
     float cm = sc;
-#pragma unroll
-    for (int w = 32; w >= 1; w >>= 1) cm = fmaxf(cm, __shfl_xor(cm, w));
+    cm = tl_wave_max(cm);
     const float mn = a.sigmoid ? 0.0f : fmaxf(m, cm);  // finite: lane 0 of a piece is always a visible key
     const float p = !valid ? 0.0f : a.sigmoid ? 1.0f / (1.0f + expf(-(sc + hb))) : expf(sc - mn);
     const float corr = expf(m - mn);  // m = -inf at the first piece: 0
     float ps = p;
-#pragma unroll
-    for (int w = 32; w >= 1; w >>= 1) ps += __shfl_xor(ps, w);
+    ps = tl_wave_sum(ps);
     l = l * corr + ps;
     m = mn;
     const int cnt = (jend - j0 + 1) < 64 ? (jend - j0 + 1) : 64;
@@ -363,8 +360,8 @@ __global__ __launch_bounds__(256) void swa_rows_kernel(const SwaArgs a) {
         s[u] = j <= jend ? d : -INFINITY;
         mx = fmaxf(mx, s[u]);
       }
-      mx = fmaxf(mx, __shfl_xor(mx, 16));
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      mx = fmaxf(mx, tl_xor<16>(mx));
+      mx = fmaxf(mx, tl_xor<32>(mx));
       const float mn = a.sigmoid ? 0.0f : fmaxf(m, mx);  // finite: the first key of a piece is a visible one
       const float corr = expf(m - mn);                   // m = -inf at the first piece: 0
       m = mn;
@@ -391,8 +388,8 @@ __global__ __launch_bounds__(256) void swa_rows_kernel(const SwaArgs a) {
       else add(std::false_type{});
     }
   }
-  l += __shfl_xor(l, 16);
-  l += __shfl_xor(l, 32);
+  l += tl_xor<16>(l);
+  l += tl_xor<32>(l);
   if (lane == 0) {
     ml[wave * 2] = m;
     ml[wave * 2 + 1] = l;
@@ -502,13 +499,11 @@ __global__ __launch_bounds__(512) void swa_shared_kernel(const SwaArgs a) {
         sc[u] = j0 + my_key + 16 * u <= i ? acc * a.scale : -INFINITY;
       }
       float cm = fmaxf(sc[0], sc[1]);
-#pragma unroll
-      for (int w = 8; w >= 1; w >>= 1) cm = fmaxf(cm, __shfl_xor(cm, w));
+      cm = tl_wave_max<8>(cm);
       const float mn = fmaxf(m, cm);  // finite: a tile's first key is visible
       const float corr = expf(m - mn), p0 = expf(sc[0] - mn), p1 = expf(sc[1] - mn);
       float sum = p0 + p1;
-#pragma unroll
-      for (int w = 8; w >= 1; w >>= 1) sum += __shfl_xor(sum, w);
+      tl_butterfly<8>([&](auto o) __attribute__((always_inline)) { sum += tl_xor<decltype(o)::value>(sum); });
       l = l * corr + sum;
       m = mn;
       ps[my_head * SH_LD + my_key] = p0;
@@ -564,12 +559,10 @@ __global__ __launch_bounds__(256) void swa_shared_combine_kernel(const SwaArgs a
   const float mz = lane < a.nsplit ? rec[(size_t)lane * rs] : -INFINITY;
   const float lz = lane < a.nsplit ? rec[(size_t)lane * rs + 1] : 0.0f;
   float M = mz;
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
+  M = tl_wave_max(M);
   const float fz = mz == -INFINITY ? 0.0f : expf(mz - M);
   float L = lz * fz;
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) L += __shfl_xor(L, o);
+  L = tl_wave_sum(L);
   float acc = 0.0f;
   for (int z0 = wave; z0 < a.nsplit; z0 += 32) {  // eight records' values in flight together
     float v[8];
@@ -752,7 +745,7 @@ __global__ __launch_bounds__(256, 2) void swa_mfma_kernel(const SwaArgs a) {  //
       s[e] = seen ? sc : -INFINITY;
       tmax = fmaxf(tmax, s[e]);
     }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+    tmax = fmaxf(tmax, tl_xor<32>(tmax));
     // sigmoid mode: the maximum is pinned to 0 once the query has seen a key, so that no factor ever differs from 1
     const float mnew = a.sigmoid ? (tmax == -INFINITY ? mrun : 0.0f) : fmaxf(mrun, tmax);  // may still be -inf: a tile can lie wholly outside one query's window
     const float corr = mrun == -INFINITY ? 0.0f : expf(mrun - mnew);
@@ -783,7 +776,7 @@ __global__ __launch_bounds__(256, 2) void swa_mfma_kernel(const SwaArgs a) {  //
 #pragma unroll
       for (int b = 0; b < DB; ++b) o[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(s[8 + e], vb[e][b], o[b], 0, 0, 0);
   }
-  const float ltot = lrun + __shfl_xor(lrun, 32);
+  const float ltot = lrun + tl_xor<32>(lrun);
   if (h == 0) {
     sm_m[wave * 32 + r] = mrun;
     sm_l[wave * 32 + r] = ltot;
