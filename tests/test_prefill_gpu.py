@@ -423,6 +423,17 @@ def test_half_plane_gemm_shapes(E, pkg, shape, name, rows, cols, T, slices):
     w.free()
 
 
+@pytest.mark.parametrize("shape", [5, 6, 7, 8])
+@pytest.mark.parametrize("name,rows,cols,T,slices", [
+    ("q4_k", 1, 256, 1, 1), ("q4_k", 63, 768, 7, 3), ("q4_k", 129, 2304, 9, 5), ("q4_k", 64, 512, 33, 1), ("q6_k", 65, 512, 8, 2),
+    ("q6_k", 127, 768, 17, 1), ("q6_k", 128, 1792, 31, 4), ("q8_0", 129, 64, 3, 1), ("q8_0", 65, 320, 16, 2), ("q8_0", 1, 1088, 8, 5),
+    ("q8_0", 255, 1984, 32, 3), ("q8_k", 130, 1280, 8, 3), ("q8_k", 63, 256, 15, 1)])
+def test_half_plane_gemm_shapes_of_few_tokens(E, pkg, shape, name, rows, cols, T, slices):
+    """Both parts of eight tokens in one instruction (5, 6), eight waves of 16 rows (6, 7), two fragments of 16 tokens (8): one token, one
+    more than a tile, rows around 64 and 128, slices. The bound of test_half_plane_gemm_edges."""
+    test_half_plane_gemm_shapes(E, pkg, shape, name, rows, cols, T, slices)
+
+
 @pytest.mark.parametrize("name,rows,cols,T,slices", [
     ("q4_k", 255, 256, 63, 1), ("q4_k", 600, 2304, 129, 3), ("q6_k", 257, 768, 64, 1), ("q6_k", 255, 768, 65, 3), ("q6_k", 1, 256, 300, 1),
     ("q8_0", 511, 1280, 130, 2), ("q8_0", 70, 256, 65, 1), ("q8_k", 257, 768, 65, 2), ("q8_k", 33, 2304, 64, 1)])

@@ -224,15 +224,24 @@ __device__ __forceinline__ Place place_of(const HSegs& segs, int mtiles, int nti
   return p;
 }
 
+// STACK: the upper half of the wave has the small sums of the lower half's tokens. The whole, in both halves (Q6_K: tl holds the
+// remainders' products, small in either half)
+template <int TYPE>
+__device__ __forceinline__ float stacked_sum(float t, float tl, int fg) {
+  float small = fg >= 2 ? t : 0.f;
+  if (TYPE == TL_Q6_K) small += tl;
+  const float big = fg >= 2 ? 0.f : t, other = tl_xor<32>(small);
+  return big + (TYPE == TL_Q6_K ? small + other : other);
+}
 // acc += a super-block's sums times the rows' factors and the tokens' powers of two. bs: its block sums [token][hi 8 | lo 8], then 2^-k
 // (APART: sums of the hi part's products t and of the small ones tl)
-template <int TYPE, int TK, int NI, int MI>
+template <int TYPE, int TK, int NI, int MI, bool STACK>
 __device__ __forceinline__ void add_superblock(typename Tile<TK>::Acc (&acc)[NI][MI], const typename Tile<TK>::Acc (&t)[NI][MI],
                                                const typename Tile<TK>::Acc (&tl)[NI][MI], const typename Tile<TK>::Acc (&c8)[NI][MI],
                                                const WHead<TYPE> (&H)[MI], const _Float16* ab, const _Float16* invs, int fr, int fg) {
   typedef Tile<TK> TL;
   typedef typename TL::Acc Acc;
-  constexpr bool APART = MI == 1;
+  constexpr bool APART = TK == 16 || MI == 1;
   const Acc zero = {};
   float d[MI], dm[MI];
   f16x8 mn[MI];
@@ -248,7 +257,7 @@ __device__ __forceinline__ void add_superblock(typename Tile<TK>::Acc (&acc)[NI]
   for (int n = 0; n < NI; ++n) {
     f16x8 bs;
     if (TYPE == TL_Q4_K) {
-      bs = *reinterpret_cast<const f16x8*>(ab + (TK * n + fr) * 16 + (fg & 1) * 8);
+      bs = *reinterpret_cast<const f16x8*>(ab + (TK * n + (STACK ? fr & 7 : fr)) * 16 + (fg & 1) * 8);
       if (TK == 16 && fg >= 2) bs = f16x8{};  // (the instruction's columns 16..31: nothing)
     }
     const float* inv = reinterpret_cast<const float*>(invs) + TK * n;
@@ -258,10 +267,14 @@ __device__ __forceinline__ void add_superblock(typename Tile<TK>::Acc (&acc)[NI]
       if (TYPE == TL_Q4_K) s = TL::mfma(bs, mn[i], zero);
 #pragma unroll
       for (int q = 0; q < TL::E / 4; ++q) {
-        const f32x4 iv = *reinterpret_cast<const f32x4*>(inv + TL::quad(q, fg));
+        const f32x4 iv = *reinterpret_cast<const f32x4*>(inv + TL::quad(q, STACK ? fg & 1 : fg));
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          float x = TYPE == TL_Q8_0 ? c8[n][i][4 * q + e] : d[i] * (APART ? t[n][i][4 * q + e] + tl[n][i][4 * q + e] : t[n][i][4 * q + e]);
+          float x;
+          if (TYPE == TL_Q8_0) x = c8[n][i][4 * q + e];
+          else if (STACK) x = d[i] * stacked_sum<TYPE>(t[n][i][4 * q + e], tl[n][i][4 * q + e], fg);
+          else x = d[i] * (APART ? t[n][i][4 * q + e] + tl[n][i][4 * q + e] : t[n][i][4 * q + e]);
+          if (TYPE == TL_Q8_0 && STACK) x += tl_xor<32>(x);
           if (TYPE == TL_Q4_K) x = fmaf(dm[i], s[4 * q + e], x);
           acc[n][i][4 * q + e] = fmaf(iv[e], x, acc[n][i][4 * q + e]);
         }
@@ -269,7 +282,7 @@ __device__ __forceinline__ void add_superblock(typename Tile<TK>::Acc (&acc)[NI]
     }
   }
 }
-template <int TK, int NI, int MI>
+template <int TK, int NI, int MI, bool STACK>
 __device__ __forceinline__ void store_tile(float* __restrict__ y, const float* __restrict__ resid, const typename Tile<TK>::Acc (&acc)[NI][MI],
                                            int n0, int m0, int T, int M, int fr, int fg) {
 #pragma unroll
@@ -277,6 +290,7 @@ __device__ __forceinline__ void store_tile(float* __restrict__ y, const float* _
 #pragma unroll
     for (int q = 0; q < Tile<TK>::E / 4; ++q) {
       const int t0 = n0 + TK * n + Tile<TK>::quad(q, fg);
+      if (STACK && fg >= 2) continue;
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
         const int r = m0 + TK * i + fr;
@@ -293,18 +307,21 @@ __device__ __forceinline__ void store_tile(float* __restrict__ y, const float* _
     }
 }
 
-// Workgroup: NW waves of TK MI rows each x TK NI tokens. LDS: two buffers of a super-block's activation tile, [4 x 64
-// columns][2 parts][tokens][64] f16, the 16-byte pieces of a token's 128 bytes at piece ^ (token / 2 & 7): the 16
-// consecutive tokens of a fragment read and the 2 x 8 pieces of a staging write cover the 64 banks once; behind them the
+// Workgroup: NW waves of TK MI rows each x TK NI tokens (STACK, for up to 8 tokens: x 8, whose hi parts are rows 0..7 of the instruction's
+// operand and whose lo parts are rows 8..15: half the matrix instructions, half the activations' way through LDS; 64 rows of Q4_K x 256
+// columns, four workgroups on a CU, 0.80 -> 0.67 us). LDS: two buffers of a super-block's activation tile, [4 x 64
+// columns][2 parts][tokens][64] f16, the 16-byte pieces of a token's 128 bytes at piece ^ (row / 2 & 7), row = part x tokens + token: the 16
+// consecutive rows of a fragment read and the 2 x 8 pieces of a staging write cover the 64 banks once; behind them the
 // super-block's block sums and powers of two.
-template <int TYPE, int TK, int NI, int MI, int NW, int WPE>
+template <int TYPE, int TK, int NI, int MI, int NW, int WPE, bool STACK>
 __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct act, const float* __restrict__ resid, int T, int mtiles,
                                                            int ntiles, int nslices, int panel) {
   typedef Tile<TK> TL;
   typedef typename TL::Acc Acc;
   constexpr int NG = 64 / TK, US = 8 / NG;                        // lane groups, steps of a super-block
-  constexpr int BN = TK * NI, NT = 64 * NW, STEP = 2 * BN * 64;   // STEP: halfs of 64 columns
-  constexpr int XR = 2 * BN * 8 / NT;                             // 16-byte pieces of 64 columns per thread
+  constexpr int BN = STACK ? 8 : TK * NI, NT = 64 * NW, STEP = 2 * BN * 64;  // STEP: halfs of 64 columns
+  constexpr int XP = 16 * BN, XR = (BN > 32 ? XP : 4 * XP) / NT;  // 16-byte pieces of 64 columns; per thread of a fetch (RINGED: 64 columns)
+  constexpr int PARTS = STACK ? 1 : 2;                            // fragments of an operand
   constexpr int AUXH = 18 * BN;                                   // halfs of a super-block's block sums and 2^-k (float)
   constexpr int BUF = 4 * STEP + AUXH;                            // !RINGED: halfs of a buffer
   constexpr bool CHUNKED = TYPE == TL_Q4_K || TYPE == TL_Q6_K;
@@ -333,12 +350,12 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
   int xl[XR];
 #pragma unroll
   for (int r = 0; r < XR; ++r) {
-    const int id = tid + r * NT, q = id & 7, row = id >> 3, tok = row % BN, part = row / BN;
+    const int id = (tid + r * NT) % XP, q = id & 7, row = id >> 3, tok = row % BN, part = row / BN;
     xg[r] = (unsigned)((size_t)part * act.ps + (size_t)(n0 + tok < T ? n0 + tok : T - 1) * K + q * 8);
-    xl[r] = row * 64 + ((q ^ ((tok >> 1) & 7)) << 3);
+    xl[r] = (tid + r * NT) / XP * STEP + row * 64 + ((q ^ ((row >> 1) & 7)) << 3);
   }
-  auto load_x = [&](int r, int sb, int c) {  // 64-column piece c of super-block sb
-    const int s = sb * 4 + c;
+  auto load_x = [&](int r, int sb, int c) {  // 64-column piece c (and on) of super-block sb
+    const int s = sb * 4 + c + (tid + r * NT) / XP;
     return *reinterpret_cast<const f16x8*>(act.x + (size_t)(xg[r] + (unsigned)((s < slast ? s : slast) * 64)));
   };
   // 16-byte pieces of a super-block's block sums (2 BN) and powers of two (BN / 4); spare threads copy a piece again
@@ -355,7 +372,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
     xo[k] = (col >> 6) * STEP + fr * 64 + ((((col & 63) >> 3) ^ ((fr >> 1) & 7)) << 3);
   }
 
-  constexpr bool APART = MI == 1;
+  constexpr bool APART = TK == 16 || MI == 1;
   constexpr int WD = US == 4 && NI * MI == 4 ? 2 : US;  // steps the weight loads run ahead: a super-block
   WStep<TYPE> W[MI][WD];
   WHead<TYPE> H[MI], Hn[MI];
@@ -364,7 +381,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
   for (int i = 0; i < MI; ++i) load_head<TYPE>(H[i], w, R[i], sb0);
   {
     const u32x4 aux = *reinterpret_cast<const u32x4*>(ag + (size_t)sb0 * astride);
-    constexpr int FIRST = RINGED ? 2 : 4;
+    constexpr int FIRST = RINGED ? 2 : 1;
     f16x8 xr[FIRST][XR];
 #pragma unroll
     for (int c = 0; c < FIRST; ++c)
@@ -408,7 +425,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
     // short, so that only the former's 16 additions round at the sum's own size, and as two chains. Q8_0: of a 32-column
     // block, c8 adds up the blocks
     Acc t[NI][MI], tl[NI][MI], c8[NI][MI];
-    f16x8 xr[RINGED ? 1 : 4][XR];
+    f16x8 xr[XR];
     unsigned h1[MI], h3[MI];
     if (TYPE == TL_Q4_K) {
 #pragma unroll
@@ -426,7 +443,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
       const _Float16* base = !RINGED ? xb + (kk >> 2) * (NG / 2) * STEP
                                      : hlds + ((kk >> 2) == u ? slot : slot == 2 ? 0 : slot + 1) * STEP;
 #pragma unroll
-      for (int p = 0; p < 2; ++p) fa[f % RING][p] = *reinterpret_cast<const f16x8*>(base + (p * BN + TK * n) * 64 + xo[kk & 3]);
+      for (int p = 0; p < PARTS; ++p) fa[f % RING][p] = *reinterpret_cast<const f16x8*>(base + (p * BN + TK * n) * 64 + xo[kk & 3]);
     };
 #pragma unroll
     for (int f = 0; f < RD; ++f) read_frags(f, 0);
@@ -434,12 +451,10 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
     for (int u = 0; u < US; ++u) {
       if (RINGED && (NEXT || u + 2 < US)) {  // two steps on
 #pragma unroll
-        for (int r = 0; r < XR; ++r) xr[0][r] = load_x(r, sb, u + 2);
+        for (int r = 0; r < XR; ++r) xr[r] = load_x(r, sb, u + 2);
       } else if (NEXT && u == 0) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-          for (int r = 0; r < XR; ++r) xr[c][r] = load_x(r, sb + 1, c);
+        for (int r = 0; r < XR; ++r) xr[r] = load_x(r, sb + 1, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
       Scale4 sc[MI];
@@ -474,11 +489,13 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
           __builtin_amdgcn_sched_barrier(0);
           if (f + RD < NF) read_frags(f + RD, u);
           __builtin_amdgcn_sched_barrier(0);
-          const f16x8 a0 = fa[f % RING][0], a1 = fa[f % RING][1];
+          const f16x8 a0 = fa[f % RING][0], a1 = fa[f % RING][PARTS - 1];
+          if (!STACK) {
 #pragma unroll
-          for (int i = 0; i < MI; ++i) {
-            Acc& c = APART ? tl[n][i] : t[n][i];
-            c = TL::mfma(a1, bh[i], fresh ? zero : c);
+            for (int i = 0; i < MI; ++i) {
+              Acc& c = APART ? tl[n][i] : t[n][i];
+              c = TL::mfma(a1, bh[i], fresh ? zero : c);
+            }
           }
 #pragma unroll
           for (int i = 0; i < MI; ++i) t[n][i] = TL::mfma(a0, bh[i], APART && fresh ? zero : t[n][i]);
@@ -486,7 +503,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
 #pragma unroll
             for (int i = 0; i < MI; ++i) {
               Acc& c = APART ? tl[n][i] : t[n][i];
-              c = TL::mfma(a0, bl[i], c);
+              c = TL::mfma(a0, bl[i], STACK && fresh ? zero : c);
             }
           }
         }
@@ -500,7 +517,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
             for (int n = 0; n < NI; ++n) {
 #pragma unroll
               for (int e = 0; e < TL::E; ++e) {
-                const float c = APART ? t[n][i][e] + tl[n][i][e] : t[n][i][e];
+                const float c = STACK ? t[n][i][e] : APART ? t[n][i][e] + tl[n][i][e] : t[n][i][e];
                 c8[n][i][e] = blk == 0 ? d * c : fmaf(d, c, c8[n][i][e]);
               }
               asm volatile("" : "+v"(c8[n][i]));  // here, not behind the loop (eight blocks' sums would stay live)
@@ -517,18 +534,16 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
       if (RINGED) {
         if (NEXT || u + 2 < US) {  // into the slot that everybody left at the last barrier
 #pragma unroll
-          for (int r = 0; r < XR; ++r) *reinterpret_cast<f16x8*>(hlds + (slot == 0 ? 2 : slot - 1) * STEP + xl[r]) = xr[0][r];
+          for (int r = 0; r < XR; ++r) *reinterpret_cast<f16x8*>(hlds + (slot == 0 ? 2 : slot - 1) * STEP + xl[r]) = xr[r];
         }
         slot = slot == 2 ? 0 : slot + 1;
         if (u < US - 1) __syncthreads();
       } else if (NEXT && u == US - 1) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-          for (int r = 0; r < XR; ++r) *reinterpret_cast<f16x8*>(xn + c * STEP + xl[r]) = xr[c][r];
+        for (int r = 0; r < XR; ++r) *reinterpret_cast<f16x8*>(xn + xl[r]) = xr[r];
       }
     }
-    add_superblock<TYPE, TK, NI, MI>(acc, t, tl, c8, H, ab, ab + 16 * BN, fr, fg);
+    add_superblock<TYPE, TK, NI, MI, STACK>(acc, t, tl, c8, H, ab, ab + 16 * BN, fr, fg);
     if (NEXT) {
 #pragma unroll
       for (int i = 0; i < MI; ++i) H[i] = Hn[i];
@@ -539,7 +554,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
   for (int b = 0; b + 1 < nsb; ++b) superblock(b, std::true_type{});
   superblock(nsb - 1, std::false_type{});
 
-  store_tile<TK, NI, MI>(y, resid, acc, n0, m0, T, M, fr, fg);
+  store_tile<TK, NI, MI, STACK>(y, resid, acc, n0, m0, T, M, fr, fg);
 }
 
 // The same product in workgroups of eight waves and 64 tokens, one on a CU, rows in whole super-blocks: activations and weights go from
@@ -813,7 +828,7 @@ __global__ __launch_bounds__(64 * NW, 2) void hgemm_lds_kernel(HSegs segs, HAct 
         if (u == 1) tl_lds_barrier<0>();
       }
     }
-    add_superblock<TYPE, 32, NI, MI>(acc, t, tl, c8, H, ab, ab + 16 * BN, fr, fg);
+    add_superblock<TYPE, 32, NI, MI, false>(acc, t, tl, c8, H, ab, ab + 16 * BN, fr, fg);
     if (NEXT) {
 #pragma unroll
       for (int i = 0; i < MI; ++i) H[i] = Hn[i];
@@ -821,7 +836,7 @@ __global__ __launch_bounds__(64 * NW, 2) void hgemm_lds_kernel(HSegs segs, HAct 
   };
   for (int b = 0; b + 1 < nsb; ++b) superblock(b, std::true_type{});
   superblock(nsb - 1, std::false_type{});
-  store_tile<32, NI, MI>(y, resid, acc, n0, m0, T, M, fr, fg);
+  store_tile<32, NI, MI, false>(y, resid, acc, n0, m0, T, M, fr, fg);
 }
 
 // ---- producer of the activation planes ----------------------------------------------------------------------------------
@@ -956,57 +971,79 @@ __global__ __launch_bounds__(256) void hsplit_kernel(const float* __restrict__ x
   hsplit8(v, planes, ps, t, K, i0, tpad);
 }
 
-// The shapes of a workgroup. Up to 16 tokens: 64 rows, four workgroups (sixteen waves) on a CU, which keeps the most weight
-// bytes in flight: a step of 16 sequences of the 8B shape (8 layers) 0.96 ms against 0.98 with the 32-token shape (Q8_0 of
-// 1.1B 0.58 against 0.63). Up to 64: 128 rows x 32 tokens, two on a CU (32 sequences 1.04 ms; 64: 1.46 against 1.49 with
-// 64-token tiles). More: 64-token tiles, each operand unpacked once for two token fragments, in workgroups of 256 rows (2), of 512 in
-// waves of 64 (3; Q4_K: for others registers or LDS are short) and of 128, two on a CU (4). Which of them is taken is a matter of
-// filling the chip, so the plan below weighs them.
+// The shapes of a workgroup. Up to 8 tokens: both parts of a token's activations in the 16 rows of one matrix instruction (stack), 64 or
+// 128 rows of weights a workgroup; up to 16: the same with an instruction for either part. Up to 32: 64 rows in 16-row waves, three
+// workgroups on a CU, or 128 in 32-row waves. Up to 64: these, or the 64-token tiles of long chunks. More: 64-token tiles, each operand
+// unpacked once for two token fragments, in workgroups of 256 rows (2), of 512 in waves of 64 (3; Q4_K: for others registers or LDS are
+// short) and of 128, two on a CU (4). Which of them is taken is a matter of filling the chip, so the plan below weighs them.
 // (8 layers of the 8B shape in ms, this kernel / the bf16 kernels it replaced: 8 sequences 0.86 / 1.56, 32: 1.05 / 1.62,
 // 64: 1.52 / 2.03, 128: 2.2 / 2.7; a prompt of 512: 5.3 / 7.0.)
 struct HShape {
   int tk, ni, mi, nw, wpe, percu;
-  bool lds;  // hgemm_lds_kernel
+  bool lds, stack;  // lds: hgemm_lds_kernel
 };
+constexpr int HGEMM_SHAPES = 9;
 constexpr HShape hgemm_shape(int type, int shape) {
-  constexpr HShape all[] = {{16, 1, 1, 4, 4, 4, false}, {32, 1, 1, 4, 2, 2, false}, {32, 2, 1, 8, 2, 1, true}, {32, 2, 2, 8, 2, 1, true}, {32, 2, 1, 4, 2, 2, false}};
-  if (shape == 3 && type != TL_Q4_K) return {32, 2, 2, 4, 2, 2, false};  // (Q8_K)
+  constexpr HShape all[HGEMM_SHAPES] = {
+      {16, 1, 1, 4, 4, 4, false, false}, {32, 1, 1, 4, 2, 2, false, false}, {32, 2, 1, 8, 2, 1, true, false},
+      {32, 2, 2, 8, 2, 1, true, false},  {32, 2, 1, 4, 2, 2, false, false}, {16, 1, 1, 4, 4, 4, false, true},
+      {16, 1, 1, 8, 4, 2, false, true},  {16, 1, 1, 8, 4, 2, false, false}, {16, 2, 1, 4, 3, 3, false, false}};
+  if (shape == 3 && type != TL_Q4_K) return {32, 2, 2, 4, 2, 2, false, false};  // (Q8_K)
   return all[shape];
 }
-// us of a super-block of a workgroup on a full chip. Shape 3 is priced so that, over the projections of the 1B, 3B and 8B shapes and 65 to
-// 2048 tokens, it is taken as often as where it ran in pairs of 256 rows (at its own 7.4 it would be taken in a sixth more of them, and its
-// single chain of sums rounds more: 2.1e-7 against 1.7e-7 at 2048 columns)
-constexpr float HGEMM_US[] = {1.2f, 2.0f, 4.25f, 7.8f, 5.0f}, HGEMM_US_3_Q8_K = 9.0f;
-// Price of a launch of n workgroups of `per` super-blocks, and of S slices' partial sums of `outputs` numbers.
-// Q4_K and Q8_K, and all formats up to 64 tokens: rounds over the chip x (super-blocks + start and end) + the partial sums written
-// and read once at about 4 TB/s. Q6_K (a third product, longer unpacking) and Q8_0 (16 additions and FMAs a block) beyond: the
+constexpr int hgemm_tokens(const HShape& q) { return q.stack ? 8 : q.tk * q.ni; }
+// Up to 64 tokens a launch takes, in us with weights that no cache holds, its start and end (a quarter of that again for every further
+// round over the chip) and, of the CU with the most workgroups, all their super-blocks one after another: co-resident ones share the issue
+// slots and the CU's way to memory, so none of them is free. Fitted to 2048 .. 28672 rows of 2048 .. 14336 columns times 8, 16, 24, 32 and
+// 48 tokens in 1 to 8 slices (rms 5 to 10 % a shape); the choice by it is within 1 % of the best of all on average (11 % at worst), and
+// against one shape and rounds over the chip a launch got 10 to 12 % shorter at 8 tokens, 8 to 10 at 16, 9 to 11 at 32, 11 to 14 at 48
+// (Q4_K, 8 tokens: 16384 x 3072 12.5 -> 11.0 us, 4096 x 14336 14.6 -> 12.6; 48 tokens: 28672 x 4096 51.5 -> 39.4).
+struct HFew {
+  float start, superblock[4];  // Q4_K, Q6_K, Q8_0, Q8_K
+};
+constexpr HFew HGEMM_FEW[HGEMM_SHAPES] = {
+    {4.0f, {0.80f, 1.15f, 1.54f, 1.26f}}, {5.7f, {1.43f, 2.20f, 2.46f, 1.72f}}, {9.0f, {3.18f, 4.65f, 4.58f, 3.09f}},
+    {},                                   {7.2f, {2.40f, 3.28f, 3.56f, 2.68f}}, {4.0f, {0.67f, 1.01f, 1.41f, 1.09f}},
+    {4.5f, {0.98f, 1.66f, 2.66f, 2.00f}}, {4.8f, {1.09f, 1.79f, 2.76f, 2.08f}}, {4.9f, {1.10f, 1.49f, 1.75f, 1.41f}}};
+// Beyond: us of a super-block of a workgroup on a full chip. Shape 3 is priced so that, over the projections of the 1B, 3B and 8B shapes
+// and 65 to 2048 tokens, it is taken as often as where it ran in pairs of 256 rows (at its own 7.4 it would be taken in a sixth more of
+// them, and its single chain of sums rounds more: 2.1e-7 against 1.7e-7 at 2048 columns)
+constexpr float HGEMM_US[] = {0.f, 0.f, 4.25f, 7.8f, 5.0f}, HGEMM_US_3_Q8_K = 9.0f;
+// Price of a launch over T tokens of n workgroups of `per` super-blocks, and of S slices' partial sums of `outputs` numbers.
+// Q4_K and Q8_K beyond 64 tokens: rounds over the chip x (super-blocks + start and end) + the partial sums written and read once at about
+// 4 TB/s. Q6_K (a third product, longer unpacking) and Q8_0 (16 additions and FMAs a block): the
 // time of the fullest CU, whose last workgroup takes 0.6 of a pair's time where two share it, and 0.16 of the way to what an even
 // share would take (clocks rise where CUs run dry). Over the projections of the 1B, 3B and 8B shapes and 100 to 2048 tokens that
 // picks within 0.7 % (Q6_K), 1 % (Q8_0) and 2 % (Q4_K) of the best shape and slices on average and 11, 11 and 20 % at worst.
-float hgemm_price(int cus, int type, int shape, long n, int per, int S, float outputs) {
+float hgemm_price(int cus, int type, int shape, int T, long n, int per, int S, float outputs) {
   const HShape q = hgemm_shape(type, shape);
-  if (shape >= 2 && (type == TL_Q6_K || type == TL_Q8_0)) {
+  const long most = (n + cus - 1) / cus, rounds = (most + q.percu - 1) / q.percu;
+  const float sums = S > 1 ? (float)S * (0.3f + outputs * 2e-6f) : 0.f;
+  if (T <= 64) {
+    const HFew& f = HGEMM_FEW[shape];
+    return f.start * (0.75f + 0.25f * (float)rounds) + (float)(most * per) * f.superblock[type == TL_Q4_K ? 0 : type == TL_Q6_K ? 1 : type == TL_Q8_0 ? 2 : 3] + sums;
+  }
+  if (type == TL_Q6_K || type == TL_Q8_0) {
     const float us = type == TL_Q6_K ? (shape == 2 ? 6.3f : 6.85f) : (shape == 2 ? 5.5f : 6.0f), alone = q.percu == 2 ? 0.6f : 1.f;
-    const long most = (n + cus - 1) / cus;
     const float fullest = q.percu == 2 ? (float)(most / 2) + (most & 1 ? alone : 0.f) : (float)most;
     const float even = (float)n / (float)cus / (float)q.percu;
     return (0.84f * fullest + 0.16f * (even > alone ? even : alone)) * ((float)per + 0.6f) * us + (S > 1 ? (float)S * (0.3f + outputs * 1.4e-6f) : 0.f);
   }
-  const long slots = (long)cus * q.percu;
-  return (float)((n + slots - 1) / slots) * (float)(per + (shape < 2 ? 2 : 1)) * (shape == 3 && !q.lds ? HGEMM_US_3_Q8_K : HGEMM_US[shape]) * (type == TL_Q6_K ? 1.37f : 1.f) +
-         (S > 1 ? (float)S * (0.3f + outputs * 2e-6f) : 0.f);
+  return (float)rounds * (float)(per + 1) * (shape == 3 && !q.lds ? HGEMM_US_3_Q8_K : HGEMM_US[shape]) + sums;
 }
 // the shape and the K slices of the least price
 HgemmPlan hgemm_plan(const QW* w, int n, int T) {
   const int nsb = (w[0].cols + 255) / 256, type = w[0].type, cus = tl_num_cus();  // (the call asks the runtime: once a plan)
-  const int lo = T <= 16 ? 0 : T <= 64 ? 1 : 2, hi = T <= 64 ? lo : 4;
-  HgemmPlan best = {lo, 1};
+  const unsigned few = T <= 8 ? 1u << 5 | 1u << 6 : T <= 16 ? 1u << 0 | 1u << 7 : 1u << 1 | 1u << 8, many = 1u << 2 | 1u << 4;
+  const unsigned shapes = T <= 32 ? few : T <= 64 ? few | many : many | 1u << 3;  // (shape 3 sums in one chain: not for few tokens)
+  HgemmPlan best = {};
   float least = -1.f;
-  for (int v = lo; v <= hi; ++v) {
+  for (int v = 0; v < HGEMM_SHAPES; ++v) {
+    if (!(shapes >> v & 1)) continue;
     if (v == 3 && (type == TL_Q6_K || type == TL_Q8_0)) continue;  // (spills)
     if (v == 2 && w[0].cols % 256) continue;                       // (rows that end inside a super-block)
     const HShape q = hgemm_shape(type, v);
-    const int bm = q.tk * q.mi * q.nw, bn = q.tk * q.ni, ntiles = (T + bn - 1) / bn;
+    const int bm = q.tk * q.mi * q.nw, bn = hgemm_tokens(q), ntiles = (T + bn - 1) / bn;
     long tiles = 0, rows = 0;
     for (int i = 0; i < n; ++i) {
       tiles += (long)((w[i].rows + bm - 1) / bm) * ntiles;
@@ -1015,7 +1052,7 @@ HgemmPlan hgemm_plan(const QW* w, int n, int T) {
     for (int S = 1; S <= 8 && S <= nsb; ++S) {
       const int per = (nsb + S - 1) / S;
       if ((nsb + per - 1) / per != S) continue;  // (no empty slice)
-      const float price = hgemm_price(cus, type, v, tiles * S, per, S, (float)T * (float)rows);
+      const float price = hgemm_price(cus, type, v, T, tiles * S, per, S, (float)T * (float)rows);
       if (least < 0.f || price < least) {
         least = price;
         best = {v, S};
@@ -1028,14 +1065,14 @@ HgemmPlan hgemm_plan(const QW* w, int n, int T) {
 template <int TYPE, int V>
 int hgemm_go(const HSegs& g, int mt, const HAct& act, const float* resid, int T, int S, hipStream_t s) {
   constexpr HShape q = hgemm_shape(TYPE, V);
-  constexpr int BN = q.tk * q.ni;
+  constexpr int BN = hgemm_tokens(q);
   constexpr size_t lds = q.lds ? (size_t)LdsMap<TYPE, q.mi, q.nw>::BYTES
                                : (size_t)(BN > 32 ? 3 * 2 * 64 + 2 * 18 : 2 * (4 * 2 * 64 + 18)) * BN * sizeof(_Float16);
   static_assert(lds <= 160 * 1024, "");
   static TlDeviceOnce lds_raised;
   void (*kernel)(HSegs, HAct, const float*, int, int, int, int, int);
   if constexpr (q.lds) kernel = hgemm_lds_kernel<TYPE, q.mi, q.nw>;
-  else kernel = hgemm_kernel<TYPE, q.tk, q.ni, q.mi, q.nw, q.wpe>;
+  else kernel = hgemm_kernel<TYPE, q.tk, q.ni, q.mi, q.nw, q.wpe, q.stack>;
   TL_TRY(tl_raise_lds_limit(kernel, (int)lds, lds_raised));
   // panels of eight token tiles and more, all alike: a panel of the one tile that is left over reads all weights again for it (28672 x
   // 4096 in Q4_K times 513 tokens, nine tiles, 274 us in one panel of shape 3 with 256 rows, 281 in eight and one)
@@ -1062,6 +1099,10 @@ int hgemm_typed(const QW* w, int n, const HgemmPlan& p, const HAct& act, float* 
   if (shape == 2) return hgemm_go<TYPE, 2>(g, mt, act, resid, T, p.S, s);
   if constexpr (TYPE == TL_Q4_K || TYPE == TL_Q8_K)
     if (shape == 3) return hgemm_go<TYPE, 3>(g, mt, act, resid, T, p.S, s);
+  if (shape == 5) return hgemm_go<TYPE, 5>(g, mt, act, resid, T, p.S, s);
+  if (shape == 6) return hgemm_go<TYPE, 6>(g, mt, act, resid, T, p.S, s);
+  if (shape == 7) return hgemm_go<TYPE, 7>(g, mt, act, resid, T, p.S, s);
+  if (shape == 8) return hgemm_go<TYPE, 8>(g, mt, act, resid, T, p.S, s);
   return hgemm_go<TYPE, 4>(g, mt, act, resid, T, p.S, s);
 }
 
@@ -1078,7 +1119,7 @@ int tl_launch_hgemm(const QW* w, int n, const void* planes, size_t ps, float* co
   for (int i = 0; i < n; ++i)
     TL_REQUIRE(tl_hgemm_supported(w[i]) && w[i].type == w[0].type && w[i].cols == w[0].cols, "half-plane GEMM: matrix %d does not fit", i);
   const int nsb = (w[0].cols + 255) / 256;
-  TL_REQUIRE(p.S >= 1 && (p.S - 1) * ((nsb + p.S - 1) / p.S) < nsb && p.shape >= 0 && p.shape <= 4 &&
+  TL_REQUIRE(p.S >= 1 && (p.S - 1) * ((nsb + p.S - 1) / p.S) < nsb && p.shape >= 0 && p.shape < HGEMM_SHAPES &&
                  !(p.shape == 3 && w[0].type != TL_Q4_K && w[0].type != TL_Q8_K),
              "half-plane GEMM: shape %d, %d K slices of %d super-blocks", p.shape, p.S, nsb);
   TL_REQUIRE(n >= 1 && n <= 3 && T > 0 && ps < ((size_t)1 << 31) && ps >= tl_gemm_padded_tokens(T) * (size_t)w[0].cols, "half-plane GEMM: bad argument");

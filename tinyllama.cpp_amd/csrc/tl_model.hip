@@ -1366,7 +1366,7 @@ static void half_part_floats(const tl_model* m, int most, size_t (&cap)[3]) {
   // between these numbers of tokens a plan's tiles stay and only the price of its partial sums rises: S is largest at the first
   for (const Group& g : groups)
     for (int T = 1, end; T <= most; T = end + 1) {
-      end = std::min(T == 1 ? 16 : T == 17 ? 32 : T + 63 - (T - 1) % 64, most);
+      end = std::min(T == 1 ? 8 : T == 9 ? 16 : T == 17 ? 32 : T + 63 - (T - 1) % 64, most);
       const int S = tl_hgemm_plan(g.w, g.n, T).S;
       for (int i = 0; i < g.n && S > 1; ++i) cap[g.at + i] = std::max(cap[g.at + i], (size_t)S * end * g.w[i].rows);
     }
