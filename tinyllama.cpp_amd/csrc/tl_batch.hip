@@ -19,6 +19,7 @@
 #include "tl_chunk.h"
 #include "tl_internal.h"
 #include "tl_lanes.h"
+#include "tl_parts.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -93,19 +94,6 @@ __global__ void batch_rope_kv_kernel(float* __restrict__ q, float* __restrict__ 
 // The same, element for element, where heads and rows are whole 16-byte pieces: four elements a thread, a row of the grid per token (the
 // general kernel divides by the token's elements and loads four bytes at a time): 512 tokens of 32 + 2 x 8 heads of 128 11.7 -> 9.3 us, 1650 of
 // 32 + 2 x 4 of 64 9.4 -> 7.4, 128 of the former in four K slices 6.4 -> 5.6.
-__device__ __forceinline__ f32x4 ld_parts4(const float* base, const GemmParts& g, size_t o) {
-  if (!g.S) return *reinterpret_cast<const f32x4*>(base + o);
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int z = 0; z < g.S; z += 4) {
-    f32x4 p[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) p[i] = *reinterpret_cast<const f32x4*>(g.part + (size_t)(z + i < g.S ? z + i : g.S - 1) * g.n + o);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (z + i < g.S) acc = z + i ? acc + p[i] : p[i];
-  }
-  return acc;
-}
 __global__ __launch_bounds__(256) void batch_rope_kv4_kernel(float* __restrict__ q, float* __restrict__ k, const float* __restrict__ v,
                                                              float* __restrict__ kc, float* __restrict__ vc, size_t seq_stride,
                                                              const float* __restrict__ table, const int* __restrict__ pos,
@@ -114,18 +102,21 @@ __global__ __launch_bounds__(256) void batch_rope_kv4_kernel(float* __restrict__
   const int t = blockIdx.y, e = (blockIdx.x * 256 + threadIdx.x) * 4, qd = nq * hd, kv_dim = nkv * hd;
   if (e >= qd + 2 * kv_dim) return;
   const int p = pos ? pos[t] : start_pos + t, sq = seq ? seq[t] : 0;
+  const bool isq = e < qd, isv = e >= qd + kv_dim;
+  const int d = isq ? e : isv ? e - qd - kv_dim : e - qd;
+  const size_t o = (size_t)t * (isq ? qd : kv_dim) + d;
+  const GemmParts g[1] = {isq ? pq : isv ? pv : pk};
+  f32x4 sum[1][1];
+  if (g[0].S) tl_parts_sum(g, o, sum);  // (asked for beside the position)
+  else sum[0][0] = *reinterpret_cast<const f32x4*>((isq ? q : isv ? v : k) + o);
+  const f32x4 x = sum[0][0];
   if (p < 0 || p >= max_seq || sq < 0 || sq >= n_seq) return;
   const size_t row = (size_t)sq * seq_stride + (size_t)p * kv_dim;
-  if (e >= qd + kv_dim) {
-    const int d = e - qd - kv_dim;
-    *reinterpret_cast<f32x4*>(vc + row + d) = ld_parts4(v, pv, (size_t)t * kv_dim + d);
+  if (isv) {
+    *reinterpret_cast<f32x4*>(vc + row + d) = x;
     return;
   }
-  const bool isq = e < qd;
-  const int d = isq ? e : e - qd;
   const f32x4 cs = *reinterpret_cast<const f32x4*>(table + (size_t)p * hd + d % hd);
-  const size_t o = (size_t)t * (isq ? qd : kv_dim) + d;
-  const f32x4 x = isq ? ld_parts4(q, pq, o) : ld_parts4(k, pk, o);
   float r[4];
   rot2(x[0], x[1], cs[0], cs[1], r[0], r[1]);
   rot2(x[2], x[3], cs[2], cs[3], r[2], r[3]);
