@@ -141,6 +141,27 @@ def test_batch_long_contexts_and_eight_head_groups(pkg, oracle):
     om.close()
 
 
+@pytest.mark.parametrize("heads,kv_heads,hd,B", [(6, 2, 128, 130), (12, 4, 64, 65), (4, 2, 64, 129), (8, 1, 64, 129), (4, 4, 128, 65)])
+def test_batched_attention_in_four_and_eight_waves(pkg, heads, kv_heads, hd, B):
+    """One step of B sequences (more workgroups than CUs: four waves each) against the same sequences seven at a time (eight waves), at
+    contexts around one and several steps of either. Both are within 2^-22 of the exact sums a layer and product, as in the packed tests."""
+    from tinyllama_cpp_amd import engine as E
+    E.init(0)
+    cfg = dict(pkg.synth.SHAPES["tiny-gqa"], hidden=heads * hd, n_heads=heads, n_kv_heads=kv_heads, n_layers=2, max_pos=320)
+    cfg, tensors = pkg.synth.build_model(cfg, "q4_k_m", seed=5)
+    m = E.Model(cfg).load(tensors)
+    m.batch_init(B)
+    rng = np.random.default_rng(heads + B)
+    lens = [(1, 31, 63, 64, 127, 128, 255, 256, 300, 16)[i] if i < 10 else int(rng.integers(1, 40)) for i in range(B)]
+    _, ids = m.batch_prefill_packed([rng.integers(0, cfg["vocab"], n).astype(np.int32) for n in lens], slots=list(range(B)))
+    toks = [int(x) for x in ids]
+    whole, _ = m.batch_decode(toks, lens, list(range(B)))
+    for i in range(0, min(B, 28), 7):
+        part, _ = m.batch_decode(toks[i:i + 7], lens[i:i + 7], list(range(i, i + 7)))
+        assert np.isfinite(part).all() and np.linalg.norm(part - whole[i:i + 7]) <= 4e-6 * np.linalg.norm(part), i
+    m.free()
+
+
 def test_packed_prefill_rejects_bad_batches(pkg):
     from tinyllama_cpp_amd import engine as E
     from tinyllama_cpp_amd.capi import TlError, check, lib

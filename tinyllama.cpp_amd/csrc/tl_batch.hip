@@ -156,11 +156,14 @@ __device__ __forceinline__ float batch_row_sum16(float v) {
   v = dpp_add<0x140, 0xf>(v);  // row_mirror
   return v;
 }
-template <int HD, int G>
-__global__ __launch_bounds__(256) void attn_batch_decode_kernel(BatchAttnArgs a) {
-  constexpr int NW = 4, LP = 16, NV = HD / 64, PP = 64 / LP, U = 8 / NV, RECL = HD + 4;
-  constexpr int NR = NW * PP;  // row groups per workgroup (= one DPP row of lanes in the weights phase)
-  static_assert(NR == 16, "the weights of a head's row groups are reduced inside one DPP row");
+// A wave alone on its SIMD issues an instruction every four cycles, and a step over 16 positions is some 700 of them: where the launch
+// leaves CUs idle, eight waves take the positions instead of four (NW): 8 sequences of 8 heads of 128 for 3 query heads each, about 95
+// positions, 8.0 -> 6.25 us (sixteen loads in flight in four waves: 8.05, the two steps were not what it waits for).
+template <int HD, int G, int NW>
+__global__ __launch_bounds__(64 * NW) void attn_batch_decode_kernel(BatchAttnArgs a) {
+  constexpr int LP = 16, NV = HD / 64, PP = 64 / LP, U = 8 / NV, RECL = HD + 4;
+  constexpr int NR = NW * PP;  // row groups per workgroup (= one or two DPP rows of lanes in the weights phase)
+  static_assert(NR == 16 || NR == 32, "the weights of a head's row groups are reduced inside one or two DPP rows");
   __shared__ __attribute__((aligned(16))) float part[NR * G * RECL];
   __shared__ float red[16], wts[G * NR];
   __shared__ __attribute__((aligned(16))) float outbuf[G * HD];
@@ -200,9 +203,10 @@ __global__ __launch_bounds__(256) void attn_batch_decode_kernel(BatchAttnArgs a)
         vv[u][v] = *reinterpret_cast<const f32x4*>(vbase + off + 64 * v);
       }
     }
-    if constexpr (G == 4) {
-      // the exps of the four heads once per quad (lane l: head l % 4, DPP quad broadcasts) instead of identically in all 16
-      // lanes of a row: as in tl_attn.hip's fold (same values, a quarter of the exps)
+    if constexpr (G > 1) {
+      // the exps of the heads once per quad (lane l: head l % 4, with fewer than four the spare lanes repeat the last; DPP quad
+      // broadcasts) instead of identically in all 16 lanes of a row: as in tl_attn.hip's fold (same values, 1 / G of the exps)
+      constexpr int G1 = 1, G2 = G > 2 ? 2 : G - 1, G3 = G - 1;
       float s[G][U], mx[G];
 #pragma unroll
       for (int g = 0; g < G; ++g) {
@@ -220,11 +224,11 @@ __global__ __launch_bounds__(256) void attn_batch_decode_kernel(BatchAttnArgs a)
       }
       const int gq = lane & 3;
       auto sel4 = [&](float x0, float x1, float x2, float x3) { return gq == 0 ? x0 : gq == 1 ? x1 : gq == 2 ? x2 : x3; };
-      const float mxs = sel4(mx[0], mx[1], mx[2], mx[3]);
-      const float cs = exp_diff(sel4(m[0], m[1], m[2], m[3]), mxs);  // (0 while nothing is valid: the state stays empty)
+      const float mxs = sel4(mx[0], mx[G1], mx[G2], mx[G3]);
+      const float cs = exp_diff(sel4(m[0], m[G1], m[G2], m[G3]), mxs);  // (0 while nothing is valid: the state stays empty)
       float ps[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) ps[u] = valid[u] ? expf(sel4(s[0][u], s[1][u], s[2][u], s[3][u]) - mxs) : 0.f;
+      for (int u = 0; u < U; ++u) ps[u] = valid[u] ? expf(sel4(s[0][u], s[G1][u], s[G2][u], s[G3][u]) - mxs) : 0.f;
       auto apply = [&](auto g_c) __attribute__((always_inline)) {
         constexpr int g = decltype(g_c)::value;
         constexpr int QP = g * 0x55;  // quad_perm: every lane of the quad reads lane g
@@ -248,8 +252,8 @@ __global__ __launch_bounds__(256) void attn_batch_decode_kernel(BatchAttnArgs a)
       };
       apply(std::integral_constant<int, 0>{});
       apply(std::integral_constant<int, 1>{});
-      apply(std::integral_constant<int, 2>{});
-      apply(std::integral_constant<int, 3>{});
+      if constexpr (G > 2) apply(std::integral_constant<int, 2>{});
+      if constexpr (G > 3) apply(std::integral_constant<int, 3>{});
       continue;
     }
 #pragma unroll
@@ -297,7 +301,7 @@ __global__ __launch_bounds__(256) void attn_batch_decode_kernel(BatchAttnArgs a)
     }
   }
   __syncthreads();
-  if (tid < G * NR) {  // lane 16 g + r: the weight exp(m_r - M) of row group r of head g, once; 1 / (L + 1e-9)
+  if (tid < G * NR) {  // lane NR g + r: the weight exp(m_r - M) of row group r of head g, once; 1 / (L + 1e-9)
     const int g = tid / NR, r = tid % NR;
     const float* rec = part + (size_t)(r * G + g) * RECL;
     const float mr = rec[HD];
@@ -310,13 +314,15 @@ __global__ __launch_bounds__(256) void attn_batch_decode_kernel(BatchAttnArgs a)
     M = dmax(M, std::integral_constant<int, 0x4E>{});
     M = dmax(M, std::integral_constant<int, 0x141>{});
     M = dmax(M, std::integral_constant<int, 0x140>{});
+    if (NR == 32) M = fmaxf(M, tl_xor<16>(M));
     const float w = exp_diff(mr, M);  // (0 for a row group without rows)
-    const float L = batch_row_sum16(rec[HD + 1] * w);
+    float L = batch_row_sum16(rec[HD + 1] * w);
+    if (NR == 32) L += tl_xor<16>(L);
     wts[tid] = w;
     if (r == 0) red[8 + g] = 1.0f / (L + 1e-9f);  // utils.cpp:692
   }
   __syncthreads();
-  for (int i = tid; i < G * (HD / 4); i += 256) {
+  for (int i = tid; i < G * (HD / 4); i += 64 * NW) {
     const int g = i / (HD / 4), c4 = i % (HD / 4);
     f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -365,7 +371,8 @@ int launch_attn_h(const BatchAttnArgs& a, int T, hipStream_t s) {
   const int grp = a.nh / a.nkv;
   auto go = [&](auto g_c, int parts) {
     constexpr int G = decltype(g_c)::value;
-    attn_batch_decode_kernel<HD, G><<<dim3(a.nkv, T, parts), 256, 0, s>>>(a);
+    if ((long)a.nkv * T * parts <= tl_num_cus()) attn_batch_decode_kernel<HD, G, 8><<<dim3(a.nkv, T, parts), 512, 0, s>>>(a);
+    else attn_batch_decode_kernel<HD, G, 4><<<dim3(a.nkv, T, parts), 256, 0, s>>>(a);
   };
   switch (grp) {
     case 1: go(std::integral_constant<int, 1>{}, 1); break;
