@@ -423,6 +423,31 @@ def test_half_plane_gemm_shapes(E, pkg, shape, name, rows, cols, T, slices):
     w.free()
 
 
+@pytest.mark.parametrize("heads,kv_heads,hd", [(8, 1, 64), (6, 2, 128), (4, 4, 64)])
+def test_short_prompts_attend_token_by_token(E, pkg, monkeypatch, heads, kv_heads, hd):
+    """Chunks of few tokens over few keys take the batched FP32 attention. Tokens and starts on both sides of its line (with a CU's 400 keys)
+    and around a workgroup a CU, against the FP32 prompt kernel (TL_HATTN=0): two layers, within 2^-22 a product and layer."""
+    E.init(0)
+    cfg = dict(pkg.synth.SHAPES["tiny-gqa"], hidden=heads * hd, n_heads=heads, n_kv_heads=kv_heads, n_layers=2, max_pos=640)
+    cfg, tensors = pkg.synth.build_model(cfg, "q4_k_m", seed=6)
+    m = E.Model(cfg).load(tensors)
+    toks = np.random.default_rng(hd).integers(0, cfg["vocab"], 620).astype(np.int32)
+    want = {}
+    cases = [(0, 9), (0, 31), (0, 65), (0, 129), (0, 257), (65, 17), (300, 40), (380, 20), (380, 21), (390, 64), (560, 10)]
+    for switch in ("0", "1"):
+        monkeypatch.setenv("TL_HATTN", switch)
+        for start, n in cases:
+            m.reset_kv()
+            if start:
+                m.prefill(toks[:start])
+            got = m.prefill(toks[start:start + n], start, all_logits=True)[1]
+            if switch == "0":
+                want[start, n] = got
+            else:
+                assert np.linalg.norm(got - want[start, n]) <= 4e-6 * np.linalg.norm(want[start, n]), (start, n)
+    m.free()
+
+
 @pytest.mark.parametrize("shape", [5, 6, 7, 8])
 @pytest.mark.parametrize("name,rows,cols,T,slices", [
     ("q4_k", 1, 256, 1, 1), ("q4_k", 63, 768, 7, 3), ("q4_k", 129, 2304, 9, 5), ("q4_k", 64, 512, 33, 1), ("q6_k", 65, 512, 8, 2),

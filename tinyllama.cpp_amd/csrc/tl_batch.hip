@@ -131,7 +131,7 @@ struct BatchAttnArgs {
   const float* vc;
   size_t seq_stride;
   float* out;       // [T][nh][hd]
-  const int* pos;
+  const int* pos;   // NULL (and seq): one sequence, tokens at start_pos and on
   const int* seq;
   int nh, nkv, max_seq, n_seq;
   float scale;
@@ -142,6 +142,7 @@ struct BatchAttnArgs {
   size_t plane_stride;
   float* xsum;
   int np, tpad;
+  int start_pos;
 };
 
 // One workgroup per (kv head, token, head-group part): the G query heads of the group share every K/V row read.
@@ -171,7 +172,7 @@ __global__ __launch_bounds__(64 * NW) void attn_batch_decode_kernel(BatchAttnArg
   const int head0 = (kvh * gridDim.z + blockIdx.z) * G;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int sub = lane / LP, ln = lane % LP;
-  const int pos = a.pos[tok], sq = a.seq[tok];
+  const int pos = a.pos ? a.pos[tok] : a.start_pos + tok, sq = a.seq ? a.seq[tok] : 0;
   if (pos < 0 || pos >= a.max_seq || sq < 0 || sq >= a.n_seq) return;  // uniform
   const int len = pos + 1;
   const int kv_dim = a.nkv * HD;
@@ -464,11 +465,12 @@ bool tl_batch_attn_supported(int nh, int nkv, int hd) {
 
 int tl_launch_batch_attn(const float* q, const float* kc, const float* vc, size_t seq_stride, float* out, const int* pos_dev,
                          const int* seq_dev, int T, int nh, int nkv, int hd, int max_seq, int n_seq, float scale,
-                         hipStream_t s, void* planes, size_t plane_stride, int terms) {
+                         hipStream_t s, void* planes, size_t plane_stride, int terms, int start_pos) {
   TL_REQUIRE(tl_batch_attn_supported(nh, nkv, hd), "batched decode attention: unsupported head configuration %d/%d/%d", nh,
              nkv, hd);
-  TL_REQUIRE(q && kc && vc && out && pos_dev && seq_dev && T > 0 && T <= 65535, "batched decode attention: bad argument");
-  BatchAttnArgs a = {q, kc, vc, seq_stride, out, pos_dev, seq_dev, nh, nkv, max_seq, n_seq, scale, nullptr, 0, nullptr, 0, 0};
+  TL_REQUIRE(q && kc && vc && out && ((pos_dev && seq_dev) || (!pos_dev && !seq_dev && start_pos >= 0)) && T > 0 && T <= 65535,
+             "batched decode attention: bad argument");
+  BatchAttnArgs a = {q, kc, vc, seq_stride, out, pos_dev, seq_dev, nh, nkv, max_seq, n_seq, scale, nullptr, 0, nullptr, 0, 0, start_pos};
   if (planes) {  // layout as tl_launch_split makes it: three bf16 planes, then the block sums
     TL_REQUIRE(plane_stride >= tl_gemm_padded_tokens(T) * (size_t)nh * hd, "batched decode attention: activation planes too small");
     a.planes = static_cast<__bf16*>(planes);

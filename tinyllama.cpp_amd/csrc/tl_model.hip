@@ -1507,6 +1507,15 @@ static bool half_attn_on() {  // TL_HATTN=0: the FP32 attention kernels everywhe
   const char* ha = getenv("TL_HATTN");
   return !(ha && atoi(ha) == 0);
 }
+// Few tokens over few keys: a workgroup a token and kv head (tl_batch.hip, FP32) instead of converted K/V tiles, their products and, over
+// many keys, the combination: one launch less, and none of them fills the chip. Its time goes with workgroups x keys beyond a workgroup a CU,
+// and the two are level at 600 keys a CU's workgroup (1.1B; 3B and 8B 700 to 1000). Prompts from the start / behind 200 tokens, the other
+// route's time over this one's: 1.1B Q8_0 of 23 tokens 1.06 / 1.10, 64 1.06 / 1.02, 100 1.04 / 0.96; 3B Q6_K of 9 to 64 tokens 1.09 to 1.11.
+static bool short_chunk(const tl_model* m, int T, int start_pos) {
+  if (!tl_batch_attn_supported(m->nh_l, m->nkv_l, m->head_dim)) return false;
+  const long groups = (long)T * m->nkv_l * (m->nh_l / m->nkv_l == 8 ? 2 : 1), cus = tl_num_cus();
+  return (groups > cus ? groups : cus) * (start_pos + T) <= 400 * cus;
+}
 static int half_attn_ws(tl_model* m) {
   tl_model::Prefill& p = m->pf;
   if (p.hattn) return 0;
@@ -1547,7 +1556,11 @@ static int prefill_attn_half(tl_model* m, int l, int T, int start_pos, hipStream
   // (no split launch; TL_ATTN_PLANES=0 keeps the launch, for A/B runs and the bit-identity test)
   const char* ap = getenv("TL_ATTN_PLANES");
   const TlHattn x = half_attn(m, m->kc(l), m->vc(l), T, start_pos);
-  if (terms == TL_TERMS_HALF && tl_hattn_supported(x) && half_attn_on()) {
+  if (terms == TL_TERMS_HALF && half_attn_on() && short_chunk(m, T, start_pos)) {
+    TL_TRY(tl_launch_batch_attn(p.qb, m->kc(l), m->vc(l), 0, p.ab, nullptr, nullptr, T, m->nh_l, m->nkv_l, hd, c.max_position_embeddings, 1, scale, s,
+                                nullptr, 0, 0, start_pos));
+    TL_TRY(tl_launch_split(0, p.ab, nullptr, p.planes, ps, T, m->qd_l, terms, 0.f, s));
+  } else if (terms == TL_TERMS_HALF && tl_hattn_supported(x) && half_attn_on()) {
     TL_TRY(half_attn_ws(m));
     TL_TRY(tl_launch_hattn(x, p.hattn, p.hattn_bytes, s));
     TL_TRY(tl_launch_split(0, p.ab, nullptr, p.planes, ps, T, m->qd_l, terms, 0.f, s));
