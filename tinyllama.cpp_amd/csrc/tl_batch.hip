@@ -17,6 +17,7 @@
 #include <type_traits>
 
 #include "tl_chunk.h"
+#include "tl_hsplit.h"
 #include "tl_internal.h"
 #include "tl_lanes.h"
 #include "tl_parts.h"
@@ -143,6 +144,8 @@ struct BatchAttnArgs {
   float* xsum;
   int np, tpad;
   int start_pos;
+  // the same for the f16 GEMM's planes (what hsplit_kernel would make of `out`): workgroups of whole super-blocks only
+  _Float16* hplanes;
 };
 
 // One workgroup per (kv head, token, head-group part): the G query heads of the group share every K/V row read.
@@ -334,11 +337,19 @@ __global__ __launch_bounds__(64 * NW) void attn_batch_decode_kernel(BatchAttnArg
     }
     const float inv = red[8 + g];
     o[0] *= inv; o[1] *= inv; o[2] *= inv; o[3] *= inv;
-    if (a.planes) *reinterpret_cast<f32x4*>(outbuf + g * HD + 4 * c4) = o;
+    if (a.planes || a.hplanes) *reinterpret_cast<f32x4*>(outbuf + g * HD + 4 * c4) = o;
     else *reinterpret_cast<f32x4*>(a.out + ((size_t)tok * a.nh + head0 + g) * HD + 4 * c4) = o;
   }
-  if (!a.planes) return;  // uniform
+  if (!a.planes && !a.hplanes) return;  // uniform
   __syncthreads();
+  if (G * HD % 256 == 0 && a.hplanes) {
+    if (tid >= G * HD / 8) return;  // (whole half waves, a super-block each)
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = outbuf[tid * 8 + e];
+    tl_hsplit8(v, a.hplanes, a.plane_stride, tok, a.nh * HD, head0 * HD + tid * 8, a.tpad);
+    return;
+  }
   // split_kernel<SPLIT_PLAIN>'s body for this workgroup's G * HD consecutive columns: 8 columns per thread, the sum of a
   // 32-column block over 4 neighbouring threads
   const int K = a.nh * HD;
@@ -463,6 +474,11 @@ bool tl_batch_attn_supported(int nh, int nkv, int hd) {
   return (hd == 64 || hd == 128) && (g == 1 || g == 2 || g == 3 || g == 4 || g == 8);
 }
 
+bool tl_batch_attn_half(int nh, int nkv, int hd) {
+  const int g = nh / nkv == 8 ? 4 : nh / nkv;  // heads of a workgroup
+  return tl_batch_attn_supported(nh, nkv, hd) && g * hd % 256 == 0;
+}
+
 int tl_launch_batch_attn(const float* q, const float* kc, const float* vc, size_t seq_stride, float* out, const int* pos_dev,
                          const int* seq_dev, int T, int nh, int nkv, int hd, int max_seq, int n_seq, float scale,
                          hipStream_t s, void* planes, size_t plane_stride, int terms, int start_pos) {
@@ -470,8 +486,14 @@ int tl_launch_batch_attn(const float* q, const float* kc, const float* vc, size_
              nkv, hd);
   TL_REQUIRE(q && kc && vc && out && ((pos_dev && seq_dev) || (!pos_dev && !seq_dev && start_pos >= 0)) && T > 0 && T <= 65535,
              "batched decode attention: bad argument");
-  BatchAttnArgs a = {q, kc, vc, seq_stride, out, pos_dev, seq_dev, nh, nkv, max_seq, n_seq, scale, nullptr, 0, nullptr, 0, 0, start_pos};
-  if (planes) {  // layout as tl_launch_split makes it: three bf16 planes, then the block sums
+  BatchAttnArgs a = {q, kc, vc, seq_stride, out, pos_dev, seq_dev, nh, nkv, max_seq, n_seq, scale, nullptr, 0, nullptr, 0, 0, start_pos, nullptr};
+  if (planes && terms == TL_TERMS_HALF) {
+    TL_REQUIRE(tl_batch_attn_half(nh, nkv, hd) && plane_stride >= tl_gemm_padded_tokens(T) * (size_t)nh * hd,
+               "batched decode attention: activation planes too small or heads of parts of a super-block");
+    a.hplanes = static_cast<_Float16*>(planes);
+    a.plane_stride = plane_stride;
+    a.tpad = (int)tl_gemm_padded_tokens(T);
+  } else if (planes) {  // layout as tl_launch_split makes it: three bf16 planes, then the block sums
     TL_REQUIRE(plane_stride >= tl_gemm_padded_tokens(T) * (size_t)nh * hd, "batched decode attention: activation planes too small");
     a.planes = static_cast<__bf16*>(planes);
     a.plane_stride = plane_stride;

@@ -360,6 +360,7 @@ int tl_launch_batch_rope_kv(float* q, float* k, const float* v, float* kc, float
                             hipStream_t s, const GemmParts* pq = nullptr, const GemmParts* pk = nullptr,
                             const GemmParts* pv = nullptr, int start_pos = 0);
 bool tl_batch_attn_supported(int nh, int nkv, int hd);
+bool tl_batch_attn_half(int nh, int nkv, int hd);  // planes of TL_TERMS_HALF come from the launch itself
 int tl_launch_batch_attn(const float* q, const float* kc, const float* vc, size_t seq_stride, float* out, const int* pos_dev,
                          const int* seq_dev, int T, int nh, int nkv, int hd, int max_seq, int n_seq, float scale,
                          hipStream_t s, void* planes = nullptr, size_t plane_stride = 0, int terms = 0, int start_pos = 0);

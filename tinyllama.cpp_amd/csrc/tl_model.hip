@@ -1516,6 +1516,12 @@ static bool short_chunk(const tl_model* m, int T, int start_pos) {
   const long groups = (long)T * m->nkv_l * (m->nh_l / m->nkv_l == 8 ? 2 : 1), cus = tl_num_cus();
   return (groups > cus ? groups : cus) * (start_pos + T) <= 400 * cus;
 }
+// the batched attention writes the f16 planes of the product that reads it (TL_ATTN_HALF_PLANES=0: a launch of its own does, for A/B runs and
+// the bit-identity test)
+static bool attn_half_planes(const tl_model* m) {
+  const char* e = getenv("TL_ATTN_HALF_PLANES");
+  return tl_batch_attn_half(m->nh_l, m->nkv_l, m->head_dim) && !(e && atoi(e) == 0);
+}
 static int half_attn_ws(tl_model* m) {
   tl_model::Prefill& p = m->pf;
   if (p.hattn) return 0;
@@ -1557,9 +1563,10 @@ static int prefill_attn_half(tl_model* m, int l, int T, int start_pos, hipStream
   const char* ap = getenv("TL_ATTN_PLANES");
   const TlHattn x = half_attn(m, m->kc(l), m->vc(l), T, start_pos);
   if (terms == TL_TERMS_HALF && half_attn_on() && short_chunk(m, T, start_pos)) {
+    const bool planes = attn_half_planes(m);
     TL_TRY(tl_launch_batch_attn(p.qb, m->kc(l), m->vc(l), 0, p.ab, nullptr, nullptr, T, m->nh_l, m->nkv_l, hd, c.max_position_embeddings, 1, scale, s,
-                                nullptr, 0, 0, start_pos));
-    TL_TRY(tl_launch_split(0, p.ab, nullptr, p.planes, ps, T, m->qd_l, terms, 0.f, s));
+                                planes ? p.planes : nullptr, ps, terms, start_pos));
+    if (!planes) TL_TRY(tl_launch_split(0, p.ab, nullptr, p.planes, ps, T, m->qd_l, terms, 0.f, s));
   } else if (terms == TL_TERMS_HALF && tl_hattn_supported(x) && half_attn_on()) {
     TL_TRY(half_attn_ws(m));
     TL_TRY(tl_launch_hattn(x, p.hattn, p.hattn_bytes, s));
@@ -1771,7 +1778,7 @@ static int batch_attn_half(tl_model* m, int l, int T, int packed, hipStream_t s)
   if (packed) {
     TL_TRY(tl_launch_attn_packed(p.qb, m->bkc(l), m->bvc(l), p.ab, m->kv_layer_elems, m->bt.pack, packed, m->nh_l, m->nkv_l, hd, scale, s));
     TL_TRY(tl_launch_split(0, p.ab, nullptr, p.planes, ps, T, m->qd_l, terms, 0.f, s));
-  } else if (terms == TL_TERMS_HALF || (ap && atoi(ap) == 0)) {
+  } else if (terms == TL_TERMS_HALF ? !attn_half_planes(m) : ap && atoi(ap) == 0) {
     TL_TRY(tl_launch_batch_attn(p.qb, m->bkc(l), m->bvc(l), m->kv_layer_elems, p.ab, m->bt.pos, m->bt.seq, T, m->nh_l,
                                 m->nkv_l, hd, c.max_position_embeddings, m->bt.max_batch, scale, s));
     TL_TRY(tl_launch_split(0, p.ab, nullptr, p.planes, ps, T, m->qd_l, terms, 0.f, s));
