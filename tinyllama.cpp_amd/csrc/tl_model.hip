@@ -136,7 +136,8 @@ struct tl_model {
     size_t ids_cap = 0;
     unsigned char* stage = nullptr;  // pinned, kCopyThreads x 2 pieces: many logits on their way to the caller (copy_to_caller)
     hipEvent_t staged[8] = {};
-    int gemv_max = 0;  // steps with at most this many sequences take the multi-vector GEMV route (0: never)
+    int gemv_max = 0;   // steps with at most this many sequences take the multi-vector GEMV route (0: never)
+    int gemv_half = 0;  // the same where the GEMMs would be the f16 form
   } bt;
   // Chain launches (tl_gemv.hip): the step's GEMVs between two attention launches -- attn_output, gate/up, ffn_down and the
   // next layer's QKV (the lm_head after the last layer) -- run as tasks of ONE launch, handed over through arrival counters
@@ -1789,7 +1790,7 @@ static int batch_attn_half(tl_model* m, int l, int T, int packed, hipStream_t s)
   return project_residual(m, L.q[TL_T_ATTN_OUTPUT], T, s);
 }
 
-// The same step for a FEW sequences (T <= batch_gemv_max, default 4): the projections as multi-vector GEMVs
+// The same step for a FEW sequences (T <= gemv_most): the projections as multi-vector GEMVs
 // (gemv_nv_kernel: one pass over the weights for up to four tokens, RMSNorm / residual / SwiGLU fused as in the
 // single-sequence step) instead of matrix-core GEMMs, whose cost per step does not fall below that of 128 tokens.
 static bool batch_gemv_ok(const tl_model* m) {
@@ -1802,6 +1803,19 @@ static bool batch_gemv_ok(const tl_model* m) {
       if (!ok(L.q[k])) return false;
   return true;
 }
+// The most sequences whose step is one GEMV pass of up to four vectors instead of f16 GEMMs. Four steps in ms, GEMV / GEMM: Q6_K 3B 6.4 /
+// 7.7 with 2 sequences, 9.3 / 7.9 with 3, 1.1B 5.5 / 4.9 with 3, 8B 14.0 / 12.2; Q8_0 8B 15.0 / 15.3 with 3 and 15.5 / 15.4 with 4, 1.1B 5.4 / 5.3
+// and 5.6 / 5.4. The GEMMs' error against 64 bits is the smaller one there (1.1B, 4 sequences: 6.1 and 7.1e-7, 5.2 and 7.8e-7). With Q4_K
+// matrices they are faster from 3 on too (1.1B 5.8 / 4.6), but 3 to 11 % further off: those keep the pass.
+static int batch_gemv_half(const tl_model* m) {
+  int most = 2;
+  auto see = [&](int type) { most = std::max(most, type == TL_Q6_K ? 2 : type == TL_Q8_0 ? 3 : 4); };
+  see(m->out->type);
+  for (const LayerW& L : m->layers)
+    for (int k = 0; k < 7; ++k) see(L.q[k]->type);
+  return most;
+}
+static int gemv_most(const tl_model* m) { return chunk_terms(m) == TL_TERMS_HALF ? m->bt.gemv_half : m->bt.gemv_max; }
 static int batch_layers_gemv(tl_model* m, int T, hipStream_t s) {
   const tl_model_config& c = m->cfg;
   tl_model::Prefill& p = m->pf;
@@ -1878,7 +1892,7 @@ static int batch_layers_gemv(tl_model* m, int T, hipStream_t s) {
 // all layers for the T tokens in bt.toks / bt.pos / bt.seq: the residual stream ends up in pf.xb [T][hidden]
 static int batch_layers(tl_model* m, int T, hipStream_t s, int packed = 0) {
   TL_REQUIRE(T >= 1 && T <= m->pf.cap, "tl_model: a batched step of %d tokens exceeds the chunk workspaces (%d)", T, m->pf.cap);
-  if (T <= m->bt.gemv_max) return batch_layers_gemv(m, T, s);
+  if (T <= gemv_most(m)) return batch_layers_gemv(m, T, s);
   TL_TRY(prefill_embed(m, m->bt.toks, T, s));
   for (int l = 0; l < m->cfg.num_hidden_layers; ++l) {
     TL_TRY(batch_attn_half(m, l, T, packed, s));
@@ -1892,7 +1906,7 @@ static int batch_head(tl_model* m, const float* hidden, int R, hipStream_t s) {
              m->pf.cap < kChunkRows ? m->pf.cap : kChunkRows);
   const tl_model_config& c = m->cfg;
   tl_model::Prefill& p = m->pf;
-  if (R <= m->bt.gemv_max) {
+  if (R <= gemv_most(m)) {
     GemvArgs f = {};
     f.seg[0] = {qw_view(m->out), p.logits_all};
     f.nseg = 1;
@@ -2017,11 +2031,11 @@ extern "C" int tl_model_batch_init(tl_model* m, int max_batch) {
     }
   }
   b.max_batch = max_batch;
-  b.gemv_max = batch_gemv_ok(m) ? 4 : 0;  // one pass of up to four vectors: 2.5 / 4.0 / 4.1 ms per step for 2 / 3 / 4 sequences; the
-                                          // direct small-token GEMM route costs 5.3 ms whatever the count (two GEMV passes: 6.1 - 7.8)
+  b.gemv_max = batch_gemv_ok(m) ? 4 : 0;  // one pass of up to four vectors
+  b.gemv_half = b.gemv_max ? batch_gemv_half(m) : 0;
   if (const char* e = getenv("TL_BATCH_GEMV_MAX")) {  // A/B runs: 0 = always the matrix-core GEMMs
     const int v = atoi(e);
-    if (v >= 0 && v <= 64 && b.gemv_max) b.gemv_max = v;
+    if (v >= 0 && v <= 64 && b.gemv_max) b.gemv_max = b.gemv_half = v;
   }
   TL_TRY(ensure_prefill_ws(m, true));
   TL_HIP(hipStreamSynchronize(m->stream));
@@ -2105,7 +2119,7 @@ extern "C" int tl_model_batch_prefill_packed(tl_model* m, int n_tokens, const in
   for (int c0 = 0; c0 < n_tokens; c0 += chunk) {
     const int T = n_tokens - c0 < chunk ? n_tokens - c0 : chunk;
     int packed = 0;
-    if (tiles && T > m->bt.gemv_max) {
+    if (tiles && T > gemv_most(m)) {
       try {
         if (m->bt.packs.size() <= (size_t)(c0 / chunk)) m->bt.packs.resize(c0 / chunk + 1);
         std::vector<TlAttnItem>& items = m->bt.packs[c0 / chunk];
