@@ -73,13 +73,6 @@ int tl_debug_packed_attention(const float* q_dev, const float* k_cache_dev, cons
                               const int* positions_host, const int* seq_idx_host, int num_tokens, int heads, int kv_heads, int dim,
                               float scale, void* stream);
 
-/* Test hook (no counterpart in the reference): tl_general_delta's recurrence in the chunks of 16 tokens that prompts take (tl_delta.hip);
- * head size 64 or 128, |decay_scale| at most 1, rows and addresses at 16 bytes. ws_dev: 81 dim + 1024
- * numbers a chunk and head. */
-int tl_debug_general_delta_chunks(const float* p_dev, int ld, const float* dw_dev, const float* w0_dev, const float* a_bias_dev,
-                                  float decay_scale, float* state_dev, float* o_dev, float* ws_dev, long long ws_floats,
-                                  int num_tokens, int heads, int dim, void* stream);
-
 /* Parity hook for layer-list models (no counterpart in the reference): cb(ctx, layer, x_dev, num_tokens, width) is called after
  * every layer of every forward pass, the stream synchronised, with the residual stream on the device. NULL switches it off.
  * With the hook set the decode step must run eagerly (TL_NO_GRAPH=1 at finalize): a captured step cannot call back. */

@@ -29,13 +29,11 @@
 //   gdelta_scan  the same column-per-16-lanes layout as delta_scan. With x = u . s and y = (w r) . s over the OLD column s,
 //                o_c = y - (r . a u) x + (r . k) v_c and s <- w s - (a u) x + k v_c: the two sums over the state are reduced
 //                together, so a token again costs one reduction latency.
-//   gdelta_chunk_pre, gdelta_chunks   the same recurrence sixteen tokens at a time, as matrix products (below).
 #include <math.h>
 
 #include <type_traits>
 
 #include "tl_bf16.h"
-#include "tl_lds.h"
 #include "tl_stack.h"
 
 namespace {
@@ -502,8 +500,8 @@ __global__ __launch_bounds__(256) void gdelta_scan_kernel(const GDeltaScanArgs a
 // The same for key sizes of exactly 16 E and rows at 16 bytes. One wave a SIMD walks the tokens, so what a token costs is the number of
 // its instructions: here five 16-byte LDS reads at constant offsets (a stage is unrolled), 5 E products and sums, and two row sums. (r w)
 // is formed once in staging; the lane whose number is the token's keeps x and y, and a stage's outputs are finished and stored together.
-// The new column is one rounding of w s + (k v - a u x). 32 heads of 64 times 1998 tokens 241 us. Models take it for few tokens and for
-// decays that gdelta_chunks does not take.
+// The new column is one rounding of w s + (k v - a u x). 32 heads of 64 times 1999 tokens: 239 us with a stage that is not unrolled and
+// an output stored per token; a layer-list prompt of eight such layers 8.5 -> 7.4 ms, about 100 us a launch.
 template <int E>
 __global__ __launch_bounds__(256) void gdelta_scan_wide_kernel(const GDeltaScanArgs a) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -595,414 +593,7 @@ __global__ __launch_bounds__(256) void gdelta_scan_wide_kernel(const GDeltaScanA
   }
 }
 
-// ---- the generalized delta rule in chunks of 16 tokens ---------------------------------------------------------------------------------
-// With W_t the product of a chunk's decays up to token t, the column after token t is W_t (s0 + sum_{j <= t} (k_j v_j - (a u)_j x_j) / W_j),
-// so that the chunk's sixteen x = u_t . s_{t-1} solve (I + D) x = U s0 + B v and everything else is a product:
-//     U_t = u_t W_{t-1},  R_t = r_t W_t,  K_j = k_j / W_j,  A_j = (a u)_j / W_j
-//     B = U K^T, D = U A^T (j < t);  E = R K^T, F = R A^T (j <= t);  T = (I + D)^-1
-//     z = U s0 + B v,  x = T z,  y = R s0 + E v - F x,  s <- W_16 (s0 + K^T v - A^T x)
-// All but s0 and v is the same for a head's columns and does not wait for the state: gdelta_chunk_pre forms it for all chunks at once,
-// gdelta_chunks walks the chunks. W shrinks by at most e a token here (tl_gdelta_chunks_take), so that 1 / W stays below e^16.
-// A chunk with a number that is not finite or beyond 1e12 would spread it to the tokens before: it is marked and walked token by token.
-constexpr int GC = 16;  // tokens of a chunk
-constexpr float GC_LARGE = 1e12f;
-// floats of a chunk of a head: U, R [D / 16][16 tokens][16 channels], (k times the decays behind it)^T, -(a u times those)^T [D][16], B, E, -F,
-// T [16][16], W_16 [D], decays [16][D]. Where the chunk is marked, the last number of B's first row, 0 otherwise, is 1, the first four
-// parts are u, r, k, a u [16][D] and the decays are there.
-__host__ __device__ constexpr int gc_floats(int D) { return 5 * GC * D + 4 * GC * GC + D; }
-__host__ __device__ constexpr int gc_mats(int D) { return 4 * GC * D; }
-__host__ __device__ constexpr int gc_w(int D) { return gc_mats(D) + 4 * GC * GC; }
-struct GDeltaChunkArgs {
-  const float* p;
-  int ld;
-  const float *dw, *w0, *a_bias;
-  float decay_scale;
-  float *ws, *state, *o;
-  int T, heads, nchunks;
-};
-
-typedef float gc4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ gc4 gc_mfma(float a, float b, gc4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-// a b of 16 x 16 numbers: lane (m, g) holds a[m][4 g ..] and b[4 g ..][m] (the layout that products leave). Two sums of eight: with one sum
-// over all of a chain's products the read-outs were 1.8 times as far from 64 bits as the token-by-token kernel's
-__device__ __forceinline__ gc4 gc_mul16(gc4 a, gc4 b) {
-  return gc_mfma(a[1], b[1], gc_mfma(a[0], b[0], gc4{})) + gc_mfma(a[3], b[3], gc_mfma(a[2], b[2], gc4{}));
-}
-
-// grid (chunks, heads): 16 lanes a token, E channels a lane
-template <int E>
-__global__ __launch_bounds__(256, 2) void gdelta_chunk_pre_kernel(const GDeltaChunkArgs a) {
-  constexpr int D = 16 * E, LD = D + 4;
-  __shared__ __attribute__((aligned(16))) float su[GC][LD], sr[GC][LD], sk[GC][LD], sa[GC][LD], sw[GC][LD];
-  __shared__ __attribute__((aligned(16))) float mat[4][GC][GC + 4];  // B, D, E, F
-  __shared__ float diag[2][GC];                                      // r . k, r . (a u)
-  __shared__ int marked;
-  const int tid = threadIdx.x, tt = tid >> 4, sub = tid & 15, h = blockIdx.y, t = blockIdx.x * GC + tt, hd = a.heads * D, d0 = sub * E;
-  const bool in = t < a.T;
-  const float* row = a.p + (size_t)(in ? t : a.T - 1) * a.ld + (size_t)h * D + d0;
-  const float* dwp = a.dw + (size_t)(in ? t : a.T - 1) * hd + (size_t)h * D + d0;
-  if (tid == 0) marked = 0;
-  float r[E], k[E], u[E], au[E], w[E];
-  float ss = 0.0f, top = 0.0f;
-  bool bad = false;
-#pragma unroll
-  for (int e = 0; e < E; e += 4) {
-    const gc4 rv = *reinterpret_cast<const gc4*>(row + e), kv = *reinterpret_cast<const gc4*>(row + hd + e);
-    const gc4 vv = *reinterpret_cast<const gc4*>(row + 2 * (size_t)hd + e), av = *reinterpret_cast<const gc4*>(row + 4 * (size_t)hd + e);
-    const gc4 dv = *reinterpret_cast<const gc4*>(dwp + e);
-    const gc4 ab = *reinterpret_cast<const gc4*>(a.a_bias + h * D + d0 + e), wb = *reinterpret_cast<const gc4*>(a.w0 + h * D + d0 + e);
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      r[e + c] = in ? rv[c] : 0.0f;
-      k[e + c] = in ? kv[c] : 0.0f;
-      au[e + c] = sigmoidf_(av[c] + ab[c]);
-      w[e + c] = in ? expf(-a.decay_scale * sigmoidf_(dv[c] + wb[c])) : 1.0f;
-      ss += k[e + c] * k[e + c];
-      top = fmaxf(top, fmaxf(fmaxf(fabsf(rv[c]), fabsf(kv[c])), fabsf(vv[c])));  // (fmaxf drops a NaN: the sum below does not)
-      bad |= !(rv[c] + kv[c] + vv[c] + au[e + c] + w[e + c] < INFINITY);
-    }
-  }
-  bad |= !(top <= GC_LARGE);
-  ss = tl_row16_sum(ss);
-  const float inv = 1.0f / sqrtf(ss + 1e-6f);
-  float rk = 0.0f, rau = 0.0f;
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    u[e] = k[e] * inv;
-    au[e] *= u[e];
-    rk += r[e] * k[e];
-    rau += r[e] * au[e];
-  }
-  rk = tl_row16_sum(rk);
-  rau = tl_row16_sum(rau);
-  if (sub == 0) {
-    diag[0][tt] = rk;
-    diag[1][tt] = rau;
-  }
-  __syncthreads();
-  if (in && bad) marked = 1;
-#pragma unroll
-  for (int e = 0; e < E; e += 4) *reinterpret_cast<gc4*>(&sw[tt][d0 + e]) = gc4{w[e], w[e + 1], w[e + 2], w[e + 3]};
-  __syncthreads();
-  float* ws = a.ws + ((size_t)blockIdx.x * a.heads + h) * gc_floats(D);
-  if (marked) {
-#pragma unroll
-    for (int e = 0; e < E; e += 4) {
-      float* o = ws + tt * D + d0 + e;
-      *reinterpret_cast<gc4*>(o) = gc4{u[e], u[e + 1], u[e + 2], u[e + 3]};
-      *reinterpret_cast<gc4*>(o + GC * D) = gc4{r[e], r[e + 1], r[e + 2], r[e + 3]};
-      *reinterpret_cast<gc4*>(o + 2 * GC * D) = gc4{k[e], k[e + 1], k[e + 2], k[e + 3]};
-      *reinterpret_cast<gc4*>(o + 3 * GC * D) = gc4{au[e], au[e + 1], au[e + 2], au[e + 3]};
-      *reinterpret_cast<gc4*>(o + gc_w(D) + D) = gc4{w[e], w[e + 1], w[e + 2], w[e + 3]};
-    }
-    if (tid == 0) ws[gc_mats(D) + GC - 1] = 1.0f;
-    return;
-  }
-  // the channels' k and a u times the decays behind their token, from the last one back: as often rounded as in the recurrence
-#pragma unroll
-  for (int e = 0; e < E; e += 4) {
-    *reinterpret_cast<gc4*>(&sk[tt][d0 + e]) = gc4{k[e], k[e + 1], k[e + 2], k[e + 3]};
-    *reinterpret_cast<gc4*>(&sa[tt][d0 + e]) = gc4{au[e], au[e + 1], au[e + 2], au[e + 3]};
-  }
-  __syncthreads();
-  if (tid < D) {
-    float c[GC], kc[GC], ac[GC], back = 1.0f;
-#pragma unroll
-    for (int i = GC - 1; i >= 0; --i) {
-      c[i] = sw[i][tid];
-      kc[i] = sk[i][tid] * back;
-      ac[i] = -(sa[i][tid] * back);
-      back *= c[i];
-    }
-#pragma unroll
-    for (int i = 0; i < GC; i += 4) {
-      *reinterpret_cast<gc4*>(ws + 2 * GC * D + tid * GC + i) = gc4{kc[i], kc[i + 1], kc[i + 2], kc[i + 3]};
-      *reinterpret_cast<gc4*>(ws + 3 * GC * D + tid * GC + i) = gc4{ac[i], ac[i + 1], ac[i + 2], ac[i + 3]};
-    }
-    ws[gc_w(D) + tid] = back;
-#pragma unroll
-    for (int i = 1; i < GC; ++i) c[i] *= c[i - 1];
-#pragma unroll
-    for (int i = 0; i < GC; ++i) sw[i][tid] = c[i];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int e = 0; e < E; e += 4) {
-    const gc4 now = *reinterpret_cast<const gc4*>(&sw[tt][d0 + e]);
-    gc4 before = gc4{1.0f, 1.0f, 1.0f, 1.0f};
-    if (tt) before = *reinterpret_cast<const gc4*>(&sw[tt - 1][d0 + e]);
-    gc4 U, R, K, A;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      U[c] = u[e + c] * before[c];
-      R[c] = r[e + c] * now[c];
-      K[c] = k[e + c] / now[c];
-      A[c] = au[e + c] / now[c];
-    }
-    *reinterpret_cast<gc4*>(&su[tt][d0 + e]) = U;
-    *reinterpret_cast<gc4*>(&sr[tt][d0 + e]) = R;
-    *reinterpret_cast<gc4*>(&sk[tt][d0 + e]) = K;
-    *reinterpret_cast<gc4*>(&sa[tt][d0 + e]) = A;
-    const int at = (d0 + e) / 16 * 256 + tt * 16 + (d0 + e) % 16;
-    *reinterpret_cast<gc4*>(ws + at) = U;
-    *reinterpret_cast<gc4*>(ws + GC * D + at) = R;
-  }
-  __syncthreads();
-  // a wave forms one of B, D, E, F
-  const int wave = tid >> 6, lane = tid & 63, m = lane & 15, g = lane >> 4;
-  {
-    const float* left = wave < 2 ? &su[m][0] : &sr[m][0];
-    const float* right = wave & 1 ? &sa[m][0] : &sk[m][0];
-    gc4 c = {};
-#pragma unroll
-    for (int i = 0; i < D / 16; ++i) c += gc_mul16(*reinterpret_cast<const gc4*>(left + 16 * i + 4 * g), *reinterpret_cast<const gc4*>(right + 16 * i + 4 * g));
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int t1 = 4 * g + e;
-      mat[wave][t1][m] = m < t1 ? c[e] : m == t1 && wave >= 2 ? diag[wave - 2][m] : 0.0f;
-    }
-  }
-  __syncthreads();
-  float* mw = ws + gc_mats(D);  // B, E, -F, T
-  if (wave) {
-    const gc4 c = *reinterpret_cast<const gc4*>(&mat[wave == 1 ? 0 : wave][m][4 * g]);
-    *reinterpret_cast<gc4*>(mw + (wave - 1) * GC * GC + m * GC + 4 * g) = wave == 3 ? -c : c;
-    return;
-  }
-  // T, column m a lane (every group of lanes all of it): T_t = e_t - sum_{j < t} D_tj T_j
-  float c[GC];
-#pragma unroll
-  for (int i = 0; i < GC; ++i) {
-    float x = i == m ? 1.0f : 0.0f;
-#pragma unroll
-    for (int j = 0; j < i; ++j) x = fmaf(-mat[1][i][j], c[j], x);
-    c[i] = x;
-    if (g == 0) mw[3 * GC * GC + i * GC + m] = x;
-  }
-}
-
-// A workgroup owns 16 columns of a head, each of its first four waves 16 KT of their key channels, as products leave them: lane (m, g)
-// column m, channels 4 g .. of each 16. What bounds it is the chain of a chunk: products with the wave's channels, a meeting of the
-// waves for z, T z, the update: 23 products of 32 cycles and a barrier a wave. A fifth wave moves the operands straight into LDS two chunks
-// ahead and adds up and stores y. The workgroups of a head run on one XCD and share the operands in its L2. 32 heads of 64 times 1998
-// tokens: 117 us and 39 for gdelta_chunk_pre, where the walk token by token took 241 and 46; with operands loaded by the four waves
-// themselves, into registers or LDS, 153 to 163.
-// LDS, in floats: U, R, K, A of the channels, W_16, B, E, F, T and v of four chunks; z and y of two.
-template <int KT>
-struct GcMap {
-  static constexpr int D = 64 * KT, PARTS = 4 * GC * D, W = PARTS, M = W + 64 * KT, V = M + 4 * GC * GC, SLOT = V + GC * GC;
-  static constexpr int NS = KT == 1 ? 4 : 3;  // (three: the fifth wave asks for a chunk behind the barrier, not in front of it)
-  static constexpr int Z = NS * SLOT, Y = Z + 2 * 4 * 256, FLOATS = Y + 2 * 4 * 256;
-};
-template <int KT>
-__global__ __launch_bounds__(320, 2) void gdelta_chunks_kernel(const GDeltaChunkArgs a) {
-  typedef GcMap<KT> L;
-  constexpr int D = L::D, CB = D / 16;
-  extern __shared__ __attribute__((aligned(16))) float gl[];
-  const int total = a.heads * CB, per8 = total >> 3, rem8 = total & 7, xcd = blockIdx.x & 7;
-  const int at = xcd * per8 + (xcd < rem8 ? xcd : rem8) + (blockIdx.x >> 3);
-  const int h = at / CB, col0 = at % CB * 16;
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, m = lane & 15, g = lane >> 4;
-  const int hd = a.heads * D, tile = m * 16 + 4 * g;
-  const float* vp = a.p + 2 * (size_t)hd + (size_t)h * D + col0;
-  float* op = a.o + (size_t)h * D + col0;
-  const float* base = tl_uniform(a.ws + (size_t)h * gc_floats(D));
-  auto meet = []() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-  auto is_marked = [&](const float* slot) { return __builtin_amdgcn_readfirstlane(__float_as_int(slot[L::M + GC - 1])) == 0x3f800000; };
-  if (wave == 4) {
-    const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) float*)gl;
-    const float* vbase = tl_uniform(vp);
-    constexpr int LOADS = 16 * KT + KT + 4 + 4;
-    auto fetch = [&](int c) __attribute__((always_inline)) {  // (beyond the last: the last one again, not walked)
-      const int cc = __builtin_amdgcn_readfirstlane(c < a.nchunks ? c : a.nchunks - 1);
-      const float* ws = base + (size_t)cc * a.heads * gc_floats(D);
-      const unsigned slot = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)c % L::NS * L::SLOT * 4);
-#pragma unroll
-      for (int j = 0; j < 16 * KT; ++j) tl_lds_load16(slot + j * 1024, lane * 16, ws + j * 256);
-#pragma unroll
-      for (int j = 0; j < KT; ++j) tl_lds_load4(slot + (L::W + 64 * j) * 4, lane * 4, ws + gc_w(D) + 64 * j);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        tl_lds_load16(slot + L::M * 4 + j * 1024, lane * 16, ws + gc_mats(D) + j * 256);
-        const int t = cc * GC + 4 * j + g;
-        tl_lds_load4(slot + (L::V + j * 64) * 4, ((unsigned)(t < a.T ? t : a.T - 1) * (unsigned)a.ld + m) * 4u, vbase);
-      }
-    };
-    // y of a chunk, out of the four waves' parts: four numbers a lane
-    auto store_y = [&](int c) __attribute__((always_inline)) {
-      const float* p = gl + L::Y + (c & 1) * 1024 + lane * 4;
-      auto part = [&](int w) { return *reinterpret_cast<const gc4*>(p + 256 * w); };
-      const gc4 y = (part(0) + part(1)) + (part(2) + part(3));
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int t = c * GC + 4 * g + e;
-        if (t < a.T) op[(size_t)t * hd + m] = y[e];
-      }
-    };
-    fetch(0);
-    fetch(1);
-    tl_lds_barrier<0>();
-    bool pending = false;
-    for (int c = 0; c < a.nchunks; ++c) {
-      const bool marked = is_marked(gl + (unsigned)c % L::NS * L::SLOT);
-      if (marked) {
-        meet();
-        if (pending) store_y(c - 1);
-        fetch(c + 2);
-        for (int i = 0; i < 4 * GC; ++i) meet();
-        tl_lds_barrier<0>();
-      } else if (L::NS == 4) {  // (stores are counted, too: those of the chunk before are older)
-        fetch(c + 2);
-        tl_lds_barrier<LOADS>();
-        if (pending) store_y(c - 1);
-      } else {
-        tl_lds_barrier<0>();
-        fetch(c + 2);
-        if (pending) store_y(c - 1);
-      }
-      pending = !marked;
-    }
-    meet();
-    if (pending) store_y(a.nchunks - 1);
-    return;
-  }
-  float* sp = a.state + ((size_t)h * D + col0 + m) * D + wave * 16 * KT + 4 * g;
-  gc4 s[KT];
-#pragma unroll
-  for (int i = 0; i < KT; ++i) s[i] = *reinterpret_cast<const gc4*>(sp + 16 * i);
-  // a marked chunk, token by token in the recurrence's own order, four meetings a token; z's place carries the two sums
-  auto walk = [&](int c) {
-    const float* ws = base + (size_t)c * a.heads * gc_floats(D);
-    float* zz = gl + L::Z;
-    for (int tt = 0; tt < GC; ++tt) {
-      const bool in = c * GC + tt < a.T;
-      const float v = in ? vp[(size_t)(c * GC + tt) * a.ld + m] : 0.0f;
-      float x = 0.0f, y = 0.0f;
-      for (int i = 0; i < KT; ++i) {
-        const gc4 u = *reinterpret_cast<const gc4*>(ws + tt * D + (wave * KT + i) * 16 + 4 * g);
-        x += (u[0] * s[i][0] + u[1] * s[i][1]) + (u[2] * s[i][2] + u[3] * s[i][3]);
-      }
-      x += __shfl_xor(x, 16);
-      x += __shfl_xor(x, 32);
-      meet();
-      zz[wave * 64 + lane] = x;
-      meet();
-      x = (zz[lane] + zz[64 + lane]) + (zz[128 + lane] + zz[192 + lane]);
-      for (int i = 0; i < KT; ++i) {
-        const float* q = ws + tt * D + (wave * KT + i) * 16 + 4 * g;
-        const gc4 r = *reinterpret_cast<const gc4*>(q + GC * D), k = *reinterpret_cast<const gc4*>(q + 2 * GC * D);
-        const gc4 n = *reinterpret_cast<const gc4*>(q + 3 * GC * D), w = *reinterpret_cast<const gc4*>(q + gc_w(D) + D);
-        for (int e = 0; e < 4; ++e) {
-          s[i][e] = in ? fmaf(w[e], s[i][e], fmaf(-n[e], x, k[e] * v)) : s[i][e];
-          y += r[e] * s[i][e];
-        }
-      }
-      y += __shfl_xor(y, 16);
-      y += __shfl_xor(y, 32);
-      meet();
-      zz[wave * 64 + lane] = y;
-      meet();
-      y = (zz[lane] + zz[64 + lane]) + (zz[128 + lane] + zz[192 + lane]);
-      if (in && wave == 0 && g == 0) op[(size_t)(c * GC + tt) * hd + m] = y;
-    }
-  };
-  // what a chunk's first products take, read a chunk ahead
-  struct Lead {
-    gc4 u[KT], r[KT], k[KT], v;
-    float vw, b, e;
-    bool marked;
-  };
-  auto lead = [&](Lead& q, int c) __attribute__((always_inline)) {
-    const float* slot = gl + (unsigned)c % L::NS * L::SLOT;
-    const float* own = slot + wave * KT * 256 + tile;
-#pragma unroll
-    for (int i = 0; i < KT; ++i) {
-      q.u[i] = *reinterpret_cast<const gc4*>(own + i * 256);
-      q.r[i] = *reinterpret_cast<const gc4*>(own + GC * D + i * 256);
-      q.k[i] = *reinterpret_cast<const gc4*>(own + 2 * GC * D + i * 256);
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) q.v[e] = slot[L::V + (4 * g + e) * GC + m];
-    q.vw = slot[L::V + (4 * g + wave) * GC + m];  // (a wave adds one of the four products with v to z and y, and of those with x to y)
-    q.b = slot[L::M + tile + wave];
-    q.e = slot[L::M + GC * GC + tile + wave];
-    q.marked = is_marked(slot);
-  };
-  meet();
-  Lead q;
-  lead(q, 0);
-  for (int c = 0; c < a.nchunks; ++c) {
-    if (q.marked) {
-      meet();
-      walk(c);
-      meet();
-      lead(q, c + 1);
-      continue;
-    }
-    const float* slot = gl + (unsigned)c % L::NS * L::SLOT;
-    float* zb = gl + L::Z + (c & 1) * 1024 + lane * 4;
-    if (c == a.nchunks - 1) {  // tokens beyond the last
-#pragma unroll
-      for (int e = 0; e < 4; ++e) q.v[e] = c * GC + 4 * g + e < a.T ? q.v[e] : 0.0f;
-      q.vw = c * GC + 4 * g + wave < a.T ? q.vw : 0.0f;
-    }
-    gc4 z = gc_mfma(q.b, q.vw, gc4{});
-#pragma unroll
-    for (int i = 0; i < KT; ++i) z += gc_mul16(q.u[i], s[i]);
-    *reinterpret_cast<gc4*>(zb + wave * 256) = z;
-    gc4 tm = *reinterpret_cast<const gc4*>(slot + L::M + 3 * GC * GC + tile), y = gc_mfma(q.e, q.vw, gc4{}), kv[KT], n[KT], w[KT];
-    const float f = slot[L::M + 2 * GC * GC + tile + wave];
-#pragma unroll
-    for (int i = 0; i < KT; ++i) {
-      n[i] = *reinterpret_cast<const gc4*>(slot + 3 * GC * D + (wave * KT + i) * 256 + tile);
-      w[i] = *reinterpret_cast<const gc4*>(slot + L::W + (wave * KT + i) * 16 + 4 * g);
-      y += gc_mul16(q.r[i], s[i]);
-      kv[i] = gc_mul16(q.k[i], q.v);
-    }
-    meet();
-    const gc4 zs = (*reinterpret_cast<const gc4*>(zb) + *reinterpret_cast<const gc4*>(zb + 256)) +
-                   (*reinterpret_cast<const gc4*>(zb + 512) + *reinterpret_cast<const gc4*>(zb + 768));
-    lead(q, c + 1);
-    const gc4 x = gc_mul16(tm, zs);
-#pragma unroll
-    for (int i = 0; i < KT; ++i) {
-      const gc4 d = kv[i] + gc_mul16(n[i], x);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s[i][e] = fmaf(w[i][e], s[i][e], d[e]);
-    }
-    const float xw = wave < 2 ? (wave ? x[1] : x[0]) : wave == 2 ? x[2] : x[3];
-    *reinterpret_cast<gc4*>(gl + L::Y + (c & 1) * 1024 + wave * 256 + lane * 4) = y + gc_mfma(f, xw, gc4{});
-  }
-  meet();
-#pragma unroll
-  for (int i = 0; i < KT; ++i) *reinterpret_cast<gc4*>(sp + 16 * i) = s[i];
-}
-template <int KT>
-int gdelta_chunks_go(const GDeltaChunkArgs& a, hipStream_t s) {
-  constexpr int lds = GcMap<KT>::FLOATS * 4;
-  static_assert(lds <= 160 * 1024, "");
-  static TlDeviceOnce lds_raised;
-  TL_TRY(tl_raise_lds_limit(gdelta_chunks_kernel<KT>, lds, lds_raised));
-  gdelta_chunk_pre_kernel<4 * KT><<<dim3(a.nchunks, a.heads), 256, 0, s>>>(a);
-  gdelta_chunks_kernel<KT><<<a.heads * 4 * KT, 320, lds, s>>>(a);
-  TL_HIP(hipGetLastError());
-  return 0;
-}
-
 }  // namespace
-
-bool tl_gdelta_chunks_take(int dim, float decay_scale) { return (dim == 64 || dim == 128) && fabsf(decay_scale) <= 1.0f; }
-size_t tl_gdelta_chunk_floats(int T, int heads, int dim) { return (size_t)((T + GC - 1) / GC) * heads * gc_floats(dim); }
-int tl_launch_gdelta_chunks(const GDeltaPreArgs& in, float* ws, float* state, float* o, hipStream_t s) {
-  TL_REQUIRE(in.p && in.dw && in.w0 && in.a_bias && ws && state && o && in.T > 0, "gdelta_chunks: bad arguments");
-  TL_REQUIRE(in.heads > 0 && in.heads <= 65535 && tl_gdelta_chunks_take(in.dim, in.decay_scale), "gdelta_chunks: %d heads of size %d, decay %g",
-             in.heads, in.dim, in.decay_scale);
-  TL_REQUIRE(in.ld >= 5 * in.heads * in.dim && in.ld % 4 == 0 && (size_t)in.T * in.ld < (1u << 30) &&
-                 (((size_t)in.p | (size_t)in.dw | (size_t)in.w0 | (size_t)in.a_bias | (size_t)ws | (size_t)state) & 15) == 0,
-             "gdelta_chunks: rows of %d floats or addresses off 16 bytes", in.ld);
-  const GDeltaChunkArgs a = {in.p, in.ld, in.dw, in.w0, in.a_bias, in.decay_scale, ws, state, o, in.T, in.heads, (in.T + GC - 1) / GC};
-  return in.dim == 64 ? gdelta_chunks_go<1>(a, s) : gdelta_chunks_go<2>(a, s);
-}
 
 int tl_launch_delta_pre(const DeltaPreArgs& a, hipStream_t s) {
   TL_REQUIRE(a.p && a.a && a.conv && a.a_log && a.dt_bias && a.qkv && a.beta && a.g && a.T > 0, "delta_pre: bad arguments");
@@ -1125,25 +716,6 @@ int tl_launch_gdelta_scan(const GDeltaScanArgs& a, hipStream_t s) {
   else gdelta_scan_kernel<16><<<grid, 256, 0, s>>>(a);
   TL_HIP(hipGetLastError());
   return 0;
-}
-
-extern "C" int tl_debug_general_delta_chunks(const float* p_dev, int ld, const float* dw_dev, const float* w0_dev, const float* a_bias_dev,
-                                             float decay_scale, float* state_dev, float* o_dev, float* ws_dev, long long ws_floats,
-                                             int num_tokens, int heads, int dim, void* stream) {
-  TL_REQUIRE(num_tokens > 0 && heads > 0 && heads <= 65535 && tl_gdelta_chunks_take(dim, decay_scale) &&
-                 ws_floats >= (long long)tl_gdelta_chunk_floats(num_tokens, heads, dim),
-             "tl_debug_general_delta_chunks: bad argument");
-  GDeltaPreArgs p = {};
-  p.p = p_dev;
-  p.ld = ld;
-  p.dw = dw_dev;
-  p.w0 = w0_dev;
-  p.a_bias = a_bias_dev;
-  p.decay_scale = decay_scale;
-  p.T = num_tokens;
-  p.heads = heads;
-  p.dim = dim;
-  return tl_launch_gdelta_chunks(p, ws_dev, state_dev, o_dev, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int tl_general_delta(const float* p_dev, int ld, const float* dw_dev, const float* w0_dev, const float* a_bias_dev,

@@ -534,12 +534,6 @@ struct GDeltaScanArgs {
   int T, heads, dim, vdim;
 };
 int tl_launch_gdelta_scan(const GDeltaScanArgs& a, hipStream_t s);
-// gdelta_pre and gdelta_scan of many tokens in one, sixteen tokens at a time on the matrix cores. in: p, ld, dw, w0, a_bias, decay_scale,
-// T, heads, dim of GDeltaPreArgs (its outputs are not used); v inside p (behind k), vdim == dim. ws: tl_gdelta_chunk_floats floats,
-// 16-byte aligned, as p, dw, w0, a_bias, state and rows of p are.
-bool tl_gdelta_chunks_take(int dim, float decay_scale);  // head sizes and decays that have this form
-size_t tl_gdelta_chunk_floats(int T, int heads, int dim);
-int tl_launch_gdelta_chunks(const GDeltaPreArgs& in, float* ws, float* state, float* o, hipStream_t s);
 
 // ---- tl_ssm.hip: S <- exp(-exp(a_log) dt) S + dt B x^T, y = S^T C + d x, y silu(z) per head; dt = softplus(raw + dt_bias) -----
 struct SsmScanArgs {

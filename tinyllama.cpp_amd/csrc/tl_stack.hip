@@ -178,7 +178,6 @@ struct TlStack {
   int max_lk = 0, max_lv = 0;
   int latent_expand = 64;                   // chunks of at least this many tokens expand (TL_STACK_LATENT_EXPAND; 0: never)
   float *gw = nullptr, *gu = nullptr, *gau = nullptr, *grau = nullptr, *grk = nullptr;  // generalized delta rule (gdelta_pre)
-  float* gchunk = nullptr;  // ... of many tokens (gdelta_chunks)
   int max_lq = 0, max_lqa = 0, max_gd = 0, gdelta_layers = 0;
   uint16_t* plane = nullptr;  // items of one product as bf16 (DenseArgs)
   size_t plane_room = 0;      // ... numbers: a chunk's tokens times the widest input of a product over them
@@ -256,13 +255,6 @@ namespace {
 int swa_bound(const tl_layer_spec& sp) {
   if (sp.chunk > 0 && (sp.window <= 0 || sp.chunk < sp.window)) return sp.chunk;
   return sp.window > 0 ? sp.window : 0;
-}
-
-// Whether a layer's generalized delta rule takes T tokens sixteen at a time (its rows and state at 16 bytes). 32 heads of 64, sixteen at a
-// time / one by one: 48 tokens 12.7 / 12.3 us, 64 13.9 / 14.6, 128 18.7 / 24.3, 512 48.5 / 76, 1998 147 / 268; 16 of 128, 1998: 189 / 465.
-constexpr int kGdeltaChunksFrom = 64;
-bool gdelta_in_chunks(const Layer& L, int T) {
-  return T >= kGdeltaChunksFrom && tl_gdelta_chunks_take(L.sp.dim, L.sp.decay_scale) && L.pd % 4 == 0 && ((size_t)L.state & 15) == 0;
 }
 
 int upload_frequencies(TlStack* st, Layer& L, const std::vector<double>& f) {
@@ -1197,19 +1189,11 @@ int tl_stack_finalize(TlStack* st, hipStream_t s) {
     TL_TRY(dev_alloc(st, &st->da, C * st->max_gd));
   }
   if (st->gdelta_layers) {
-    size_t rows = 1, chunk = 0;  // tokens that go through gdelta_pre at most
-    for (const Layer& L : st->layers) {
-      if (L.sp.mixer != TL_MIXER_GDELTA) continue;
-      const size_t most = gdelta_in_chunks(L, C) ? std::min<size_t>(C, kGdeltaChunksFrom - 1) : C;
-      rows = std::max(rows, most);
-      if (most < C) chunk = std::max(chunk, tl_gdelta_chunk_floats(C, L.sp.heads, L.sp.dim));
-    }
-    TL_TRY(dev_alloc(st, &st->gw, rows * st->max_gd));
-    TL_TRY(dev_alloc(st, &st->gu, rows * st->max_gd));
-    TL_TRY(dev_alloc(st, &st->gau, rows * st->max_gd));
-    TL_TRY(dev_alloc(st, &st->grau, rows * st->max_heads));
-    TL_TRY(dev_alloc(st, &st->grk, rows * st->max_heads));
-    if (chunk) TL_TRY(dev_alloc(st, &st->gchunk, chunk));
+    TL_TRY(dev_alloc(st, &st->gw, C * st->max_gd));
+    TL_TRY(dev_alloc(st, &st->gu, C * st->max_gd));
+    TL_TRY(dev_alloc(st, &st->gau, C * st->max_gd));
+    TL_TRY(dev_alloc(st, &st->grau, C * st->max_heads));
+    TL_TRY(dev_alloc(st, &st->grk, C * st->max_heads));
   }
   {
     size_t ws = 1;
@@ -2104,11 +2088,6 @@ int gdelta_mixer(TlStack* st, Layer& L, const float* in, int T, hipStream_t s) {
   p.T = T;
   p.heads = sp.heads;
   p.dim = sp.dim;
-  if (gdelta_in_chunks(L, T)) {
-    TL_TRY(tl_launch_gdelta_chunks(p, st->gchunk, L.state, st->att, s));
-    TL_TRY(tl_launch_gated_head_norm_rows(st->att, st->qkv + 3 * hd, ld, L.onorm, 1, T, sp.heads, sp.dim, st->cfg.norm_eps, s));
-    return project(st, L.wo, W, L.od, st->att, L.od, st->proj, W, T, s);
-  }
   p.w = st->gw;
   p.u = st->gu;
   p.au = st->gau;
