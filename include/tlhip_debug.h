@@ -73,6 +73,13 @@ int tl_debug_packed_attention(const float* q_dev, const float* k_cache_dev, cons
                               const int* positions_host, const int* seq_idx_host, int num_tokens, int heads, int kv_heads, int dim,
                               float scale, void* stream);
 
+/* Test hook (no counterpart in the reference): the attention of multi-sequence steps and of prompts of few tokens (tl_batch.hip) over q
+ * [T][heads][dim], token i at positions_dev[i] of sequence seq_idx_dev[i] (both NULL: at start_pos + i of sequence 0), whose caches
+ * [max_seq][kv_heads][dim] lie seq_stride floats apart; tokens elsewhere are left out. dim 64 or 128, 1, 2, 3, 4 or 8 heads a kv head. */
+int tl_debug_batch_attention(const float* q_dev, const float* k_cache_dev, const float* v_cache_dev, float* out_dev, long long seq_stride,
+                             const int* positions_dev, const int* seq_idx_dev, int start_pos, int num_tokens, int heads, int kv_heads,
+                             int dim, int max_seq, int num_seq, float scale, void* stream);
+
 /* Parity hook for layer-list models (no counterpart in the reference): cb(ctx, layer, x_dev, num_tokens, width) is called after
  * every layer of every forward pass, the stream synchronised, with the residual stream on the device. NULL switches it off.
  * With the hook set the decode step must run eagerly (TL_NO_GRAPH=1 at finalize): a captured step cannot call back. */

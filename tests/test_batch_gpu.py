@@ -187,6 +187,44 @@ def test_batched_attention_writes_the_products_input(pkg, monkeypatch, heads, kv
             assert all(np.isfinite(a).all() and np.array_equal(a, b) for a, b in zip(got, want))
 
 
+@pytest.mark.parametrize("heads,kv_heads,hd", [(3, 3, 64), (2, 1, 128), (4, 2, 64), (3, 1, 128), (6, 2, 64), (4, 1, 64), (8, 1, 128)])
+@pytest.mark.parametrize("T", [3, 300])
+def test_batched_attention_of_keys_out_of_range(pkg, heads, kv_heads, hd, T):
+    """Keys so large that their scores are -inf, at every 16th and 32nd position (all that a group of lanes of four or eight waves sees) and
+    in the first positions: weight 0, as if they were not there; a token that sees no others gets 0. Bound of
+    test_packed_attention_kernel. Three tokens take eight waves, 300 four."""
+    from tinyllama_cpp_amd import engine as E
+    from tinyllama_cpp_amd.capi import check, lib
+    E.init(0)
+    rng = np.random.default_rng(heads * hd + T)
+    S, group, start = 340, heads // kv_heads, 30
+    q = np.abs(rng.standard_normal((T, heads, hd))).astype(np.float32) + 0.5
+    k, v = (rng.standard_normal((S, kv_heads, hd)).astype(np.float32) for _ in range(2))
+    gone = np.zeros(S, bool)
+    gone[:2] = gone[5::32] = gone[7::16] = gone[16::16] = True
+    k[gone] = -3e38
+    scale = float(np.float32(1.0 / np.sqrt(hd)))
+    dev, out = [E.DeviceBuffer.from_numpy(a) for a in (q, k, v)], E.DeviceBuffer(4 * q.size)
+
+    def run(at):
+        check(lib().tl_memset(out.ptr, 0xff, out.nbytes, None))
+        check(lib().tl_debug_batch_attention(*(d.ptr for d in dev), out.ptr, 0, None, None, at, T, heads, kv_heads, hd, S, 1, scale, None))
+        return out.to_numpy(np.float32, q.shape)
+
+    got = run(start)
+    assert np.isfinite(got).all()
+    for i in range(T):
+        at = np.flatnonzero(~gone[:start + i + 1])
+        K, V = (np.repeat(a[at].astype(np.float64), group, 1) for a in (k, v))
+        sc = np.einsum("hd,jhd->hj", q[i].astype(np.float64), K) * scale
+        w = np.exp(sc - sc.max(1, keepdims=True))
+        w /= w.sum(1, keepdims=True)
+        want = np.einsum("hj,jhd->hd", w, V)
+        bound = 2.0 ** -24 * np.einsum("hj,jhd->hd", w * (12 + 8 * np.abs(sc).max()), np.abs(V))
+        assert (np.abs(got[i] - want) <= bound).all(), (i, float((np.abs(got[i] - want) / bound).max()))
+    assert not run(0)[:2].any()
+
+
 def test_packed_prefill_rejects_bad_batches(pkg):
     from tinyllama_cpp_amd import engine as E
     from tinyllama_cpp_amd.capi import TlError, check, lib

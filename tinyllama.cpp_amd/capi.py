@@ -200,6 +200,7 @@ DEBUG_SIGNATURES = {
     "tl_debug_dense_plane_taken": [C.c_int, C.c_int, C.c_int, C.c_longlong, C.c_int],
     "tl_debug_half_attention": [_fp, _fp, _fp, _fp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_float, _vp],
     "tl_debug_packed_attention": [_fp, _fp, _fp, _fp, C.c_longlong, _vp, _vp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_float, _vp],
+    "tl_debug_batch_attention": [_fp, _fp, _fp, _fp, C.c_longlong, _vp, _vp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_float, _vp],
     "tl_model_debug_layer_hook": [_vp, LAYER_HOOK, _vp],
 }
 

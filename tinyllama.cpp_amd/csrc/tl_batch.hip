@@ -230,9 +230,10 @@ __global__ __launch_bounds__(64 * NW) void attn_batch_decode_kernel(BatchAttnArg
       auto sel4 = [&](float x0, float x1, float x2, float x3) { return gq == 0 ? x0 : gq == 1 ? x1 : gq == 2 ? x2 : x3; };
       const float mxs = sel4(mx[0], mx[G1], mx[G2], mx[G3]);
       const float cs = exp_diff(sel4(m[0], m[G1], m[G2], m[G3]), mxs);  // (0 while nothing is valid: the state stays empty)
+      const float ref = mxs == -INFINITY ? 0.f : mxs;  // (rows whose scores are all -inf: weights of 0, not of exp(-inf + inf))
       float ps[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) ps[u] = valid[u] ? expf(sel4(s[0][u], s[G1][u], s[G2][u], s[G3][u]) - mxs) : 0.f;
+      for (int u = 0; u < U; ++u) ps[u] = valid[u] ? expf(sel4(s[0][u], s[G1][u], s[G2][u], s[G3][u]) - ref) : 0.f;
       auto apply = [&](auto g_c) __attribute__((always_inline)) {
         constexpr int g = decltype(g_c)::value;
         constexpr int QP = g * 0x55;  // quad_perm: every lane of the quad reads lane g
@@ -502,6 +503,14 @@ int tl_launch_batch_attn(const float* q, const float* kc, const float* vc, size_
     a.tpad = (int)tl_gemm_padded_tokens(T);
   }
   return hd == 64 ? launch_attn_h<64>(a, T, s) : launch_attn_h<128>(a, T, s);
+}
+// Test hook (tlhip_debug.h): the kernel above as an operator
+extern "C" int tl_debug_batch_attention(const float* q_dev, const float* k_cache_dev, const float* v_cache_dev, float* out_dev, long long seq_stride,
+                                        const int* positions_dev, const int* seq_idx_dev, int start_pos, int num_tokens, int heads, int kv_heads,
+                                        int dim, int max_seq, int num_seq, float scale, void* stream) {
+  TL_REQUIRE(heads > 0 && kv_heads > 0 && max_seq > 0 && num_seq > 0 && seq_stride >= 0, "tl_debug_batch_attention: bad argument");
+  return tl_launch_batch_attn(q_dev, k_cache_dev, v_cache_dev, (size_t)seq_stride, out_dev, positions_dev, seq_idx_dev, num_tokens, heads, kv_heads, dim,
+                              max_seq, num_seq, scale, static_cast<hipStream_t>(stream), nullptr, 0, 0, start_pos);
 }
 
 int tl_launch_batch_argmax_advance(const float* logits, int T, int V, int* tokens_dev, int* pos_dev, int* ids_out_dev,
