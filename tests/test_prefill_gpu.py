@@ -603,6 +603,31 @@ def test_split_products_of_long_chunks_stay_in_the_models_buffers(E, pkg, mix):
     m.free()
 
 
+@pytest.mark.parametrize("max_pos", [2048, 80])
+def test_short_first_prompts_make_the_workspaces_of_long_ones(E, pkg, max_pos):
+    """A first prompt of 20 tokens, whose attention needs no workspace, makes that of the f16 attention all the same (some 145 MB; with 80
+    positions no chunk ever takes it): longer prompts and a prompt behind another allocate no more than their token ids."""
+    import ctypes as C
+    hip = C.CDLL("libamdhip64.so")
+
+    def free_bytes():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    E.init(0)
+    cfg = dict(hidden=512, inter=512, n_heads=4, n_kv_heads=2, n_layers=1, vocab=64, max_pos=max_pos, eps=1e-5, rope_theta=10000.0)
+    _, tensors = pkg.synth.build_model(cfg, "q6_k", seed=2)
+    m = E.Model(cfg).load(tensors)
+    toks = np.random.default_rng(1).integers(0, cfg["vocab"], max_pos).astype(np.int32)
+    m.prefill(toks[:20], 0)
+    before = free_bytes()
+    for start, T in ((0, max_pos), (0, max_pos // 2), (max_pos // 2, max_pos // 2)):
+        m.prefill(toks[start:start + T], start)
+        assert before - free_bytes() <= (2 << 20), (start, T, before - free_bytes())
+    m.free()
+
+
 @pytest.mark.parametrize("T", [2048, 2049, 2600])
 def test_prefill_chunks_of_2048(E, pkg, T):
     """Prompts around the largest chunk: the last logits of the whole prompt against the last row of an all-logits prefill, which

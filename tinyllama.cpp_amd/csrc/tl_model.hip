@@ -1486,7 +1486,7 @@ static int qkv_deferred(tl_model* m, LayerW& L, int T, hipStream_t s) {
   TL_HIP(hipStreamWaitEvent(s, p.join, 0));
   return 0;
 }
-// the f16 attention over layer l's rows at kc / vc, and its workspace (made at the first use)
+// the f16 attention over layer l's rows at kc / vc
 static TlHattn half_attn(tl_model* m, const float* kc, const float* vc, int T, int start_pos) {
   TlHattn x = {};
   x.q = m->pf.qb;
@@ -1523,10 +1523,15 @@ static bool attn_half_planes(const tl_model* m) {
   const char* e = getenv("TL_ATTN_HALF_PLANES");
   return tl_batch_attn_half(m->nh_l, m->nkv_l, m->head_dim) && !(e && atoi(e) == 0);
 }
+// the f16 attention's workspace, before a prompt's first launch, whatever the prompt's length: a long prompt behind a short one makes no
+// memory in its midst. None where no chunk that the model can hold goes beyond short_chunk
 static int half_attn_ws(tl_model* m) {
   tl_model::Prefill& p = m->pf;
-  if (p.hattn) return 0;
-  const size_t bytes = tl_hattn_bytes(m->cfg.max_position_embeddings, m->nkv_l, m->head_dim, m->head_dim);
+  const int positions = m->cfg.max_position_embeddings, most = std::min(p.cap, positions);
+  if (p.hattn || chunk_terms(m) != TL_TERMS_HALF || !half_attn_on() || !tl_hattn_supported(half_attn(m, m->kc(0), m->vc(0), 1, 0)) ||
+      short_chunk(m, most, positions - most))
+    return 0;
+  const size_t bytes = tl_hattn_bytes(positions, m->nkv_l, m->head_dim, m->head_dim);
   TL_HIP(hipMalloc(&p.hattn, bytes));
   p.hattn_bytes = bytes;
   return 0;
@@ -1569,7 +1574,6 @@ static int prefill_attn_half(tl_model* m, int l, int T, int start_pos, hipStream
                                 planes ? p.planes : nullptr, ps, terms, start_pos));
     if (!planes) TL_TRY(tl_launch_split(0, p.ab, nullptr, p.planes, ps, T, m->qd_l, terms, 0.f, s));
   } else if (terms == TL_TERMS_HALF && tl_hattn_supported(x) && half_attn_on()) {
-    TL_TRY(half_attn_ws(m));
     TL_TRY(tl_launch_hattn(x, p.hattn, p.hattn_bytes, s));
     TL_TRY(tl_launch_split(0, p.ab, nullptr, p.planes, ps, T, m->qd_l, terms, 0.f, s));
   } else if (terms != TL_TERMS_HALF && tl_attn_prefill_mfma_supported(m->nh_l, m->nkv_l, hd) && !(ap && atoi(ap) == 0)) {
@@ -1638,6 +1642,7 @@ static int upload_tokens(tl_model* m, const int* tokens_host, int num_tokens, hi
 }
 static int prepare_prefill(tl_model* m, const int* tokens_host, int num_tokens, bool all_logits, hipStream_t s) {
   TL_TRY(ensure_prefill_ws(m, all_logits));
+  TL_TRY(half_attn_ws(m));
   return upload_tokens(m, tokens_host, num_tokens, s);
 }
 
