@@ -974,8 +974,8 @@ __global__ __launch_bounds__(256) void hsplit_kernel(const float* __restrict__ x
 }
 
 // The shapes of a workgroup. Up to 8 tokens: both parts of a token's activations in the 16 rows of one matrix instruction (stack), 64 or
-// 128 rows of weights a workgroup; up to 16: the same with an instruction for either part. Up to 32: 64 rows in 16-row waves, three
-// workgroups on a CU, or 128 in 32-row waves. Up to 64: these, or the 64-token tiles of long chunks. More: 64-token tiles, each operand
+// 128 rows of weights a workgroup; up to 16: the same with an instruction for either part. Up to 32: 64 rows in 16-row waves
+// (8) or 128 in 32-row waves (1), both two workgroups on a CU, whose LDS two super-blocks of 32 tokens fill. Up to 64: these, or the 64-token tiles of long chunks. More: 64-token tiles, each operand
 // unpacked once for two token fragments, in workgroups of 256 rows (2), of 512 in waves of 64 (3; Q4_K: for others registers or LDS are
 // short) and of 128, two on a CU (4). Which of them is taken is a matter of filling the chip, so the plan below weighs them.
 // (8 layers of the 8B shape in ms, this kernel / the bf16 kernels it replaced: 8 sequences 0.86 / 1.56, 32: 1.05 / 1.62,
@@ -989,7 +989,7 @@ constexpr HShape hgemm_shape(int type, int shape) {
   constexpr HShape all[HGEMM_SHAPES] = {
       {16, 1, 1, 4, 4, 4, false, false}, {32, 1, 1, 4, 2, 2, false, false}, {32, 2, 1, 8, 2, 1, true, false},
       {32, 2, 2, 8, 2, 1, true, false},  {32, 2, 1, 4, 2, 2, false, false}, {16, 1, 1, 4, 4, 4, false, true},
-      {16, 1, 1, 8, 4, 2, false, true},  {16, 1, 1, 8, 4, 2, false, false}, {16, 2, 1, 4, 3, 3, false, false}};
+      {16, 1, 1, 8, 4, 2, false, true},  {16, 1, 1, 8, 4, 2, false, false}, {16, 2, 1, 4, 3, 2, false, false}};
   if (shape == 3 && type != TL_Q4_K) return {32, 2, 2, 4, 2, 2, false, false};  // (Q8_K)
   return all[shape];
 }
@@ -1070,7 +1070,7 @@ int hgemm_go(const HSegs& g, int mt, const HAct& act, const float* resid, int T,
   constexpr int BN = hgemm_tokens(q);
   constexpr size_t lds = q.lds ? (size_t)LdsMap<TYPE, q.mi, q.nw>::BYTES
                                : (size_t)(BN > 32 ? 3 * 2 * 64 + 2 * 18 : 2 * (4 * 2 * 64 + 18)) * BN * sizeof(_Float16);
-  static_assert(lds <= 160 * 1024, "");
+  static_assert(q.percu * lds <= 160 * 1024, "hgemm_price counts on `percu` workgroups on a CU");
   static TlDeviceOnce lds_raised;
   void (*kernel)(HSegs, HAct, const float*, int, int, int, int, int);
   if constexpr (q.lds) kernel = hgemm_lds_kernel<TYPE, q.mi, q.nw>;
