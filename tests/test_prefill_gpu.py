@@ -426,26 +426,35 @@ def test_half_plane_gemm_shapes(E, pkg, shape, name, rows, cols, T, slices):
 @pytest.mark.parametrize("heads,kv_heads,hd", [(8, 1, 64), (6, 2, 128), (4, 4, 64)])
 def test_short_prompts_attend_token_by_token(E, pkg, monkeypatch, heads, kv_heads, hd):
     """Chunks of few tokens over few keys take the batched FP32 attention. Tokens and starts on both sides of its line (with a CU's 400 keys)
-    and around a workgroup a CU, against the FP32 prompt kernel (TL_HATTN=0): two layers, within 2^-22 a product and layer."""
+    and around a workgroup a CU, against the FP32 prompt kernel (TL_HATTN=0): two layers, within 2^-22 a product and layer. Which attention
+    ran is counted; where it is the batched one, the f16 kernel's logits (TL_ATTN_SHORT=0) are others, elsewhere the same."""
     E.init(0)
     cfg = dict(pkg.synth.SHAPES["tiny-gqa"], hidden=heads * hd, n_heads=heads, n_kv_heads=kv_heads, n_layers=2, max_pos=640)
     cfg, tensors = pkg.synth.build_model(cfg, "q4_k_m", seed=6)
     m = E.Model(cfg).load(tensors)
     toks = np.random.default_rng(hd).integers(0, cfg["vocab"], 620).astype(np.int32)
-    want = {}
+    cus, got = 256, {}  # (compute units of an MI355X)
     cases = [(0, 9), (0, 31), (0, 65), (0, 129), (0, 257), (65, 17), (300, 40), (380, 20), (380, 21), (390, 64), (560, 10)]
-    for switch in ("0", "1"):
-        monkeypatch.setenv("TL_HATTN", switch)
+    few = {(start, n) for start, n in cases if max(n * kv_heads * (2 if heads == 8 * kv_heads else 1), cus) * (start + n) <= 400 * cus}
+    assert few and len(few) < len(cases)
+    for route, hattn, short in (("fp32", "0", "1"), ("f16", "1", "0"), ("rule", "1", "1")):
         for start, n in cases:
             m.reset_kv()
+            monkeypatch.setenv("TL_HATTN", "0")  # (the same rows before the chunk)
             if start:
                 m.prefill(toks[:start])
-            got = m.prefill(toks[start:start + n], start, all_logits=True)[1]
-            if switch == "0":
-                want[start, n] = got
-            else:
-                assert np.linalg.norm(got - want[start, n]) <= 4e-6 * np.linalg.norm(want[start, n]), (start, n)
+            monkeypatch.setenv("TL_HATTN", hattn)
+            monkeypatch.setenv("TL_ATTN_SHORT", short)
+            before = _count("tl_debug_half_attention_launches")
+            got[route, start, n] = m.prefill(toks[start:start + n], start, all_logits=True)[1]
+            half = _count("tl_debug_half_attention_launches") - before
+            assert half == (0 if route == "fp32" or (route == "rule" and (start, n) in few) else 2), (route, start, n, half)
     m.free()
+    for at in cases:
+        want = got["fp32", at[0], at[1]]
+        for route in ("f16", "rule"):
+            assert np.linalg.norm(got[route, at[0], at[1]] - want) <= 4e-6 * np.linalg.norm(want), (route, at)
+        assert np.array_equal(got["rule", at[0], at[1]], got["f16", at[0], at[1]]) == (at not in few), at
 
 
 @pytest.mark.parametrize("shape", [5, 6, 7, 8])
@@ -551,7 +560,9 @@ def test_half_attention_edges(E, pkg, monkeypatch, heads, kv, hd, start, T):
     128 and 32, one and several pieces of the keys, tiles whose values are 2^-9 .. 2^9 apart (the common exponent of the running
     sum) and an all-zero tile. A score's error is at most 2^-21 |q| |k| scale from the parts and hd 2^-24 of it from the sums;
     with |q| |k| scale below 16 here, and as much again from the values, the outputs agree to 2 * 16 * (2^-21 + hd 2^-24) < 3e-4
-    at worst; errors are independent, so the L2 distance of the logits is held to 1e-5."""
+    at worst; errors are independent, so the L2 distance of the logits is held to 1e-5. (TL_ATTN_SHORT=0: the shorter ones would take
+    the batched attention.)"""
+    monkeypatch.setenv("TL_ATTN_SHORT", "0")
     cfg = dict(hidden=heads * hd, inter=256, n_heads=heads, n_kv_heads=kv, n_layers=1, vocab=64, max_pos=start + T, eps=1e-5,
                rope_theta=10000.0)
     _, tensors = pkg.synth.build_model(cfg, "q8_0", seed=heads + T)
@@ -569,7 +580,9 @@ def test_half_attention_edges(E, pkg, monkeypatch, heads, kv, hd, start, T):
         m.reset_kv()
         if start:
             m.set_kv_cache(0, K, V)
+        before = _count("tl_debug_half_attention_launches")
         got.append(np.array(m.prefill(toks, start, all_logits=True)[1], np.float64))
+        assert _count("tl_debug_half_attention_launches") - before == int(route)
     m.free()
     assert np.isfinite(got[1]).all() and not np.array_equal(got[0], got[1])
     assert np.linalg.norm(got[1] - got[0]) <= 1e-5 * np.linalg.norm(got[0]), np.linalg.norm(got[1] - got[0]) / np.linalg.norm(got[0])

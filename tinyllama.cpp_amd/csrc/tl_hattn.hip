@@ -21,6 +21,8 @@
 //   3. hattn_combine_kernel sums the pieces of a row tile that has more than one, in order.
 #include <math.h>
 
+#include <atomic>
+
 #include "tl_internal.h"
 #include "tl_lanes.h"
 #include "tl_lds.h"
@@ -484,6 +486,7 @@ size_t tl_hattn_bytes(int max_keys, int kv_heads, int dim, int vdim) {
 }
 
 // ws: tl_hattn_bytes of at least the positions that the tokens see
+static std::atomic<long long> g_hattn_launches{0};
 int tl_launch_hattn(const TlHattn& x, void* ws, size_t ws_bytes, hipStream_t s) {
   if (x.T == 0) return 0;
   TL_REQUIRE(tl_hattn_supported(x) && x.T > 0 && x.start_pos >= 0, "tl_launch_hattn: unsupported shapes");
@@ -511,9 +514,16 @@ int tl_launch_hattn(const TlHattn& x, void* ws, size_t ws_bytes, hipStream_t s) 
   else if (x.dim == 96) launch<96, 64>(p, a, s);
   else launch<64, 64>(p, a, s);
   TL_HIP(hipGetLastError());
+  g_hattn_launches.fetch_add(1, std::memory_order_relaxed);
   return 0;
 }
 
+// Diagnostic hook (tlhip_debug.h): calls of the function above so far in this process
+extern "C" int tl_debug_half_attention_launches(long long* count_out) {
+  TL_REQUIRE(count_out, "tl_debug_half_attention_launches: null argument");
+  *count_out = g_hattn_launches.load();
+  return 0;
+}
 // Measurement and test hook: the kernels above as an operator (tlhip_debug.h)
 extern "C" int tl_debug_half_attention(const float* q_dev, const float* k_cache_dev, const float* v_cache_dev, float* out_dev, int num_tokens,
                                        int start_pos, int heads, int kv_heads, int dim, int vdim, int window, float scale, void* stream) {

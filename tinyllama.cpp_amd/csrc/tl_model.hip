@@ -1512,8 +1512,10 @@ static bool half_attn_on() {  // TL_HATTN=0: the FP32 attention kernels everywhe
 // many keys, the combination: one launch less, and none of them fills the chip. Its time goes with workgroups x keys beyond a workgroup a CU,
 // and the two are level at 600 keys a CU's workgroup (1.1B; 3B and 8B 700 to 1000). Prompts from the start / behind 200 tokens, the other
 // route's time over this one's: 1.1B Q8_0 of 23 tokens 1.06 / 1.10, 64 1.06 / 1.02, 100 1.04 / 0.96; 3B Q6_K of 9 to 64 tokens 1.09 to 1.11.
+// (TL_ATTN_SHORT=0: never, for A/B runs and the tests of the other route)
 static bool short_chunk(const tl_model* m, int T, int start_pos) {
-  if (!tl_batch_attn_supported(m->nh_l, m->nkv_l, m->head_dim)) return false;
+  const char* e = getenv("TL_ATTN_SHORT");
+  if ((e && atoi(e) == 0) || !tl_batch_attn_supported(m->nh_l, m->nkv_l, m->head_dim)) return false;
   const long groups = (long)T * m->nkv_l * (m->nh_l / m->nkv_l == 8 ? 2 : 1), cus = tl_num_cus();
   return (groups > cus ? groups : cus) * (start_pos + T) <= 400 * cus;
 }
