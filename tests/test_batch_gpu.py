@@ -165,26 +165,42 @@ def test_batched_attention_in_four_and_eight_waves(pkg, heads, kv_heads, hd, B):
 @pytest.mark.parametrize("heads,kv_heads,hd", [(8, 1, 64), (8, 2, 128), (8, 4, 64), (4, 2, 128)])
 def test_batched_attention_writes_the_products_input(pkg, monkeypatch, heads, kv_heads, hd):
     """A step of 7 and of 130 sequences and a prompt of 9 tokens, whose attention writes the two f16 parts itself where a workgroup's heads
-    are whole super-blocks (64 x 2: they are not), bit for bit with the split in a launch of its own (TL_ATTN_HALF_PLANES=0)."""
+    are whole super-blocks (64 x 2: they are not), bit for bit with the split in a launch of its own (TL_ATTN_HALF_PLANES=0): one launch
+    a layer and call less, which are counted."""
+    import ctypes as C
     from tinyllama_cpp_amd import engine as E
+    from tinyllama_cpp_amd.capi import check, lib
     E.init(0)
+
+    def splits():
+        n = C.c_longlong()
+        check(lib().tl_debug_split_launches(C.byref(n)))
+        return n.value
+
     cfg = dict(pkg.synth.SHAPES["tiny-gqa"], hidden=heads * hd, n_heads=heads, n_kv_heads=kv_heads, n_layers=2, max_pos=320)
     cfg, tensors = pkg.synth.build_model(cfg, "q4_k_m", seed=8)
     rng = np.random.default_rng(heads)
     prompts = [rng.integers(0, cfg["vocab"], n).astype(np.int32) for n in rng.integers(1, 12, 130)]
-    want = None
+    want, launches = None, []
     for switch in ("0", "1"):
         monkeypatch.setenv("TL_ATTN_HALF_PLANES", switch)
         m = E.Model(cfg).load(tensors)
         m.batch_init(130)
         first, ids = m.batch_prefill_packed(prompts, slots=list(range(130)))
         toks, lens = [int(x) for x in ids], [len(p) for p in prompts]
-        got = [m.batch_decode(toks, lens, list(range(130)))[0], m.batch_decode(toks[:7], lens[:7], list(range(7)))[0], m.prefill(np.arange(9, dtype=np.int32))]
+        got, counts = [], [splits()]
+        for call in (lambda: m.batch_decode(toks, lens, list(range(130)))[0], lambda: m.batch_decode(toks[:7], lens[:7], list(range(7)))[0],
+                     lambda: m.prefill(np.arange(9, dtype=np.int32))):
+            got.append(call())
+            counts.append(splits())
+        launches.append(np.diff(counts))
         m.free()
         if want is None:
             want = got
         else:
             assert all(np.isfinite(a).all() and np.array_equal(a, b) for a, b in zip(got, want))
+    group = min(heads // kv_heads, 4)
+    assert (launches[0] - launches[1] == (2 if group * hd % 256 == 0 else 0)).all(), launches
 
 
 @pytest.mark.parametrize("heads,kv_heads,hd", [(3, 3, 64), (2, 1, 128), (4, 2, 64), (3, 1, 128), (6, 2, 64), (4, 1, 64), (8, 1, 128)])
