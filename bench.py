@@ -2,8 +2,8 @@
 """bench.py — greedy decode throughput of the quantized forward pass on MI355X.
 
 A "step" is one decoded token: one pass of the hot path (embedding lookup, L transformer layers over the
-device-resident KV cache, lm_head, on-device greedy sampling) for one sequence. The default workload is the one
-the north star's target is quoted on and that fits one GPU: Llama-3-8B-shaped synthetic random-init Q4_K_M
+device-resident KV cache, lm_head, on-device greedy sampling) for one sequence. The default workload is
+the largest of the reference's headline models that fits one GPU: Llama-3-8B-shaped synthetic random-init Q4_K_M
 (the Q4_K_M tensor mix; 4.62 GB of quantized weights per token), weights resident in HBM before the timed region.
 
     python bench.py --gpus 1 --steps 128 --warmup 16 [--workload llama-3-8b|tinyllama-1.1b|llama-3.2-3b|tiny]

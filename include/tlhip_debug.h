@@ -50,7 +50,9 @@ int tl_debug_half_attention_launches(long long* count_out);
 
 /* Test hook (no counterpart in the reference): tl_matmul_q through the f16 form that a model's chunks and multi-sequence steps
  * take (tl_hgemm.hip), any number of tokens, in a workgroup shape (0: 64 rows x 16 tokens, 1: 128 x 32, 2: 256 x 64, 3: in waves of 64
- * rows, 512 x 64 in Q4_K and 256 x 64 in Q8_K, 4: 128 x 64) and a number of K slices, none of them empty. */
+ * rows, 512 x 64 in Q4_K and 256 x 64 in Q8_K, 4: 128 x 64, 5 and 6: 64 and 128 rows x 8 tokens, whose two parts share an instruction, 7:
+ * 128 x 16 in waves of 16 rows, 8: 64 x 32 in the same) and a number of K slices, none of them empty. Rows that are not whole super-blocks
+ * (Q8_0) run shape 4 where 2 is asked for: the same sums, and no plan chooses 2 for them. */
 int tl_debug_half_gemm(const tl_qweight* w, const float* x_dev, float* y_dev, int num_tokens, int shape, int slices, void* stream);
 
 /* Test hook (no counterpart in the reference): tl_dense_matmul's product with one term through the kernel that takes the items from a

@@ -1,4 +1,4 @@
-"""Multi-sequence decode (SURVEY f4; generate_batch api.cpp:836, forward_cpu_batch_generation model.cpp:1158) on MI355X:
+"""Multi-sequence decode (generate_batch api.cpp:836, forward_cpu_batch_generation model.cpp:1158) on MI355X:
 B sequences with prompts of different lengths share every step's weight stream (skinny GEMMs on the matrix cores) over a
 sequence-major KV cache. The bar is the reference's sequential fallback: every sequence must decode exactly as it does
 alone -- logits within the decode tolerance of the single-sequence CPU oracle, identical greedy ids -- whatever else is

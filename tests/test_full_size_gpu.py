@@ -1,4 +1,4 @@
-"""Full-size checks on MI355X at BASELINE.json's headline shape (Llama-3-8B, 32 layers, vocabulary 128256, Q4_K_M
+"""Full-size checks on MI355X at the benchmark's shape (Llama-3-8B, 32 layers, vocabulary 128256, Q4_K_M
 mix, synthetic weights), where the CPU oracle would need minutes per token: size-independent properties instead.
 
   * two independent device implementations agree: the batched prefill (MFMA GEMMs over bf16 planes, FP32-MFMA attention)
@@ -123,7 +123,7 @@ def test_multi_sequence_decode_agrees_with_single_sequence_at_full_size(big):
             assert np.array_equal(np.concatenate([[first[j]], more[:, j]]), ids), (len(members), i)
 
 
-# ---- BASELINE.json configs[4]: the Llama-3-70B-shaped model on ONE GPU (the N = 1 anchor of its tensor-parallel curve) ----
+# ---- the Llama-3-70B-shaped model on ONE GPU (the N = 1 anchor of its tensor-parallel curve) ----
 @pytest.fixture(scope="module")
 def big70(pkg):
     """The 70B layer shape (H 8192, I 28672, 64 / 8 heads of 128) and its full vocabulary at 4 layers: every launch has

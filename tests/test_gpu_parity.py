@@ -2,7 +2,7 @@
 CPU oracle on the same seeded inputs and against the committed golden vectors (outputs of the reference's
 own code, oracle/make_golden.py).
 
-Bars (SURVEY §8d):
+Bars:
   * dequantized weights: BIT-EXACT (NaN positions must coincide; NaN payloads are not compared);
   * RoPE: bit-exact (unfused FP32 mul/sub in the reference's order);
   * GEMV / logits: |delta| <= GEMV_TOL * max(1, |ref|) vs the Kahan-double oracle — FP32 accumulation over
@@ -91,7 +91,7 @@ def test_gemv_golden(E, golden, name):
     ("q4_k", 16390, 3072), ("q6_k", 16385, 3072), ("q8_0", 16387, 2304), ("q4_k", 16384, 5632), ("q8_k", 16388, 3072),
     ("q4_k", 37, 3072), ("q6_k", 10, 11008), ("q8_0", 5, 2304), ("q4_k", 1, 5632)])
 def test_gemv_vs_oracle_model_shapes(E, pkg, oracle, name, rows, cols):
-    """Shapes of the BASELINE configs (H x H, I x H, H x I, ragged row counts, one row, max K)."""
+    """Shapes of the benchmarked models (H x H, I x H, H x I, ragged row counts, one row, max K)."""
     t = TYPES[name]
     S = pkg.synth
     rng = np.random.default_rng(rows * 7 + cols)
@@ -314,9 +314,9 @@ def test_model_kv_cache_and_prefill_vs_oracle(E, pkg, oracle):
 
 @pytest.mark.parametrize("mix", ["q4_k_m", "q8_0"])
 def test_model_tinyllama_shape_two_layers(E, pkg, oracle, mix):
-    """Real TinyLlama-1.1B H/I/heads (SURVEY G4) at 2 layers and a cut vocabulary: logits + greedy stream. q8_0 is
-    BASELINE.json's configs[0] (TinyLlama-1.1B-Chat Q8_0: every matrix dequantize_q8_0_block's format,
-    quantization.cpp:1047-1052), q4_k_m its configs[1]."""
+    """Real TinyLlama-1.1B H/I/heads at 2 layers and a cut vocabulary: logits + greedy stream. q8_0 is
+    TinyLlama-1.1B-Chat Q8_0 (every matrix dequantize_q8_0_block's format, quantization.cpp:1047-1052), q4_k_m the same
+    model's Q4_K_M mix."""
     cfg = dict(pkg.synth.SHAPES["tinyllama-1.1b"], n_layers=2, vocab=2048, max_pos=64)
     cfg, tensors = pkg.synth.build_model(cfg, mix, seed=11)
     m = E.Model(cfg).load(tensors)
@@ -333,7 +333,7 @@ def test_model_tinyllama_shape_two_layers(E, pkg, oracle, mix):
 
 
 def test_model_tinyllama_q8_0_prefill_then_decode(E, pkg, oracle):
-    """configs[0] through the generate loop's other branch (api.cpp:601-694): a 40-token prompt goes through the batched
+    """TinyLlama-1.1B Q8_0 through the generate loop's other branch (api.cpp:601-694): a 40-token prompt goes through the batched
     prefill, then greedy decode with the default penalty 1.3; ids and the first sampled position's logits vs the oracle."""
     cfg = dict(pkg.synth.SHAPES["tinyllama-1.1b"], n_layers=2, vocab=2048, max_pos=128)
     cfg, tensors = pkg.synth.build_model(cfg, "q8_0", seed=12)

@@ -128,7 +128,7 @@ def test_end_to_end_golden(oracle, pkg, golden, tag):
         assert np.array_equal(ids, g[f"{tag}_p{plen}_pen1.0_ids"])
         assert np.array_equal(logits, g[f"{tag}_p{plen}_logits"])
         assert np.array_equal(m.generate(prompt, 12, penalty=1.3), g[f"{tag}_p{plen}_pen1.3_ids"])
-    # ref_structure (whole-tensor dequant + f32 mat-vec + l-2 eviction) is bit-identical (SURVEY a6)
+    # ref_structure (whole-tensor dequant + f32 mat-vec + l-2 eviction) is bit-identical
     m.set_ref_structure(True)
     ids2, logits2 = m.generate(g[f"{tag}_p4_prompt"], 12, penalty=1.0, dump_logits=True)
     assert np.array_equal(ids2, g[f"{tag}_p4_pen1.0_ids"]) and np.array_equal(logits2, g[f"{tag}_p4_logits"])
@@ -136,7 +136,7 @@ def test_end_to_end_golden(oracle, pkg, golden, tag):
 
 
 def test_prefill_matches_stepwise(oracle, pkg):
-    """Batched prefill reproduces token-by-token logits to <= 1e-6 (SURVEY §8c probe)."""
+    """Batched prefill reproduces token-by-token logits to <= 1e-6."""
     cfg, tensors = pkg.synth.build_model("tiny", "q4_k_m", seed=7)
     m = OracleModel(oracle, cfg, tensors)
     toks = np.random.default_rng(0).integers(0, cfg["vocab"], 9)

@@ -1,4 +1,4 @@
-"""the C++ tokenizer (host/tl_tokenizer.cpp over include/tlhost.h) against oracle/tokenizer_oracle.py.
+"""The C++ tokenizer (host/tl_tokenizer.cpp over include/tlhost.h) against oracle/tokenizer_oracle.py.
 
 PARITY UNPINNED: the reference's tokenizer.cpp cannot be built here (Boost, nlohmann/json) and the reference holds no
 tokenizer vectors, so nothing in this file has been compared with the reference running. Two kinds of test:

@@ -106,7 +106,7 @@ def test_shard_shapes_and_bytes():
     for size in (1, 2, 4, 8):
         tp.check(cfg, size)
     with pytest.raises(ValueError):
-        tp.check(S.SHAPES["llama-3.2-3b"], 8)  # 3072 / 8 = 384 is not a multiple of 256 (SURVEY 8e)
+        tp.check(S.SHAPES["llama-3.2-3b"], 8)  # 3072 / 8 = 384 is not a multiple of 256
     with pytest.raises(ValueError):
         tp.check(S.SHAPES["tinyllama-1.1b"], 8)  # 4 kv heads
     cfg, tensors = S.build_model("tiny-tp", "q4_k_m", seed=1)

@@ -111,7 +111,7 @@ def test_tp_local_group_prefill_matches_oracle(pkg, oracle, shape, mix, tp, T):
 
 
 def test_tp8_at_the_70b_shard_shapes(pkg, oracle):
-    """BASELINE config 5 (Llama-3-70B-shaped, TP = 8) at its real per-rank shapes — hidden 8192, 8 query heads + 1 kv head
+    """The Llama-3-70B-shaped model (TP = 8) at its real per-rank shapes — hidden 8192, 8 query heads + 1 kv head
     and 3584 intermediate columns per rank — cut to 2 layers and a 4096-token vocabulary so that the CPU oracle can
     follow: decode in lockstep over all 8 shards on one GPU, then a batched prefill."""
     from tinyllama_cpp_amd import engine as E

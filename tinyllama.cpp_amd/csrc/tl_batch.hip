@@ -162,7 +162,7 @@ __device__ __forceinline__ float batch_row_sum16(float v) {
 }
 // A wave alone on its SIMD issues an instruction every four cycles, and a step over 16 positions is some 700 of them: where the launch
 // leaves CUs idle, eight waves take the positions instead of four (NW): 8 sequences of 8 heads of 128 for 3 query heads each, about 95
-// positions, 8.0 -> 6.25 us (sixteen loads in flight in four waves: 8.05, the two steps were not what it waits for).
+// positions, 8.19 -> 6.43 us in a whole call (sixteen loads in flight in four waves gained nothing: the two steps were not what it waits for).
 template <int HD, int G, int NW>
 __global__ __launch_bounds__(64 * NW) void attn_batch_decode_kernel(BatchAttnArgs a) {
   constexpr int LP = 16, NV = HD / 64, PP = 64 / LP, U = 8 / NV, RECL = HD + 4;

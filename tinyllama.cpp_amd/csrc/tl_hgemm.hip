@@ -13,8 +13,10 @@
 //     super-block's factor to it: 16 FMAs per 33 matrix instructions (Q4_K) where integer operands need 16 per 3;
 //   - Q4_K's minima: sum_j m_j * (sum of x over sub-block j) is one more K = 16 matrix instruction per super-block, with
 //     the eight sub-block sums' two f16 parts side by side along K and the same eight m_j against either half.
-// Weights go from HBM straight into registers (a super-block ahead), are unpacked there and never touch LDS; the
-// activation tile is staged through LDS, a super-block ahead as well, with one barrier per super-block.
+// hgemm_kernel (tiles of up to 128 rows, Q8_K 256): weights go from HBM straight into registers (a super-block ahead), are unpacked
+// there and never touch LDS; the activation tile is staged through LDS, up to 32 tokens a super-block ahead with one barrier
+// per super-block, 64 tokens in a ring of three 64-column steps. hgemm_lds_kernel (256 and 512 rows): activations and
+// weights are both copied from memory to LDS as they lie there, with a barrier per 64-column step, and unpacked behind it.
 //
 // The order of the columns inside an operand is free as long as both sides agree. Lane half h of a Q4_K / Q6_K step takes
 // the 32-weight chunk 2 s + h (one 16-byte load), of a Q8 step 16 of the 32 bytes of a chunk; the eight columns of an
@@ -565,9 +567,10 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
 // weights asked for just before those; here whatever a step asks for has a step and a half to arrive. It also issues an eighth fewer
 // vector instructions. The same operands in the same order: the same bits. 28672 x 4096 in Q4_K, us at 128 / 512 / 2048 tokens: 256
 // rows 78 / 312 / 1057 -> 74 / 299 / 1006, waves of 64 rows 87 / 290 / 962 -> - / 266 / 892; 16384 x 3072 in Q6_K 72 / 179 / 634 -> 67
-// / 160 / 604; 28672 x 4096 in Q8_0 104 / 389 / 1361 -> 97 / 375 / 1272. What bounds it: power. The matrix instructions alone, at the clock
-// that they leave, take three quarters of the time at 2048 tokens; taking out the unpacking, the fragment reads or the loads gives 3 to 5 %
-// each.
+// / 160 / 604; 28672 x 4096 in Q8_0 104 / 389 / 1361 -> 97 / 375 / 1272. What bounds it (counters of single launches): the clock falls as
+// the matrix cores fill, 28672 x 4096 in Q4_K at 128 / 512 / 2048 tokens 2.2 / 1.9 / 1.6 GHz with the cores busy in 39 / 50 / 60 % of the
+// cycles, 16384 x 3072 in Q6_K at 2048 1.7 GHz and 53 %; the two waves of a SIMD wait in 26 to 29 % of theirs for data and barriers and in
+// 33 to 42 % for their turn to issue. In Q8_0 (16 additions and FMAs a block) the cores are busy in 30 %, at 2.0 GHz.
 // LDS, in bytes: activations of four 64-column steps [part][64 tokens][64] f16; two halves of a super-block of the rows' nibbles (bytes),
 // behind them Q6_K's high bits; the rows' heads of two super-blocks (16 bytes and, Q6_K and Q8_K, the dword that d lies in); block sums and
 // powers of two of two super-blocks. 16-byte pieces of a row are exchanged so that the 16 rows of a fragment read cover the 64 banks once.
@@ -865,8 +868,8 @@ __device__ __forceinline__ f32x4 hparts4(const GemmParts& g, size_t o) {
 }
 constexpr int HNORM_THREADS = 512, HMAX_COLS = 8 * 8 * HNORM_THREADS;
 // WIDE (a piece a thread; launches whose workgroups are all on the chip at once, so that registers cost nothing): the row, the weights and
-// all slices in one round trip. 8 rows of 3072, 2 to 8 slices, 4.81 -> 4.05 us on average, 128 of 4096 7.3 -> 6.6; gate and up of 8 x 8192
-// (hsplit_kernel) 4.46 -> 3.64.
+// all slices in one round trip. In whole calls: 8 rows of 3072, 2 to 8 slices, 4.97 -> 4.10 us on average, 128 of 4096 7.74 -> 7.29; gate and
+// up of 8 x 8192 (hsplit_kernel) 4.46 -> 3.78.
 template <int NIT, bool WIDE>
 __global__ __launch_bounds__(HNORM_THREADS) void hsplit_norm_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                     _Float16* __restrict__ planes, size_t ps, int K, float eps,
