@@ -143,8 +143,8 @@ def test_batch_long_contexts_and_eight_head_groups(pkg, oracle):
 
 @pytest.mark.parametrize("heads,kv_heads,hd,B", [(6, 2, 128, 130), (12, 4, 64, 65), (4, 2, 64, 129), (8, 1, 64, 129), (4, 4, 128, 65)])
 def test_batched_attention_in_four_and_eight_waves(pkg, heads, kv_heads, hd, B):
-    """One step of B sequences (more workgroups than CUs: four waves each) against the same sequences seven at a time (eight waves), at
-    contexts around one and several steps of either. Both are within 2^-22 of the exact sums a layer and product, as in the packed tests."""
+    """One step of B sequences (more workgroups than CUs: four waves each) against the same sequences seven at a time (eight waves beyond a
+    step of four), at contexts around one and several steps of either. Both are within 2^-22 of the exact sums a layer and product, as in the packed tests."""
     from tinyllama_cpp_amd import engine as E
     E.init(0)
     cfg = dict(pkg.synth.SHAPES["tiny-gqa"], hidden=heads * hd, n_heads=heads, n_kv_heads=kv_heads, n_layers=2, max_pos=320)
@@ -239,6 +239,29 @@ def test_batched_attention_of_keys_out_of_range(pkg, heads, kv_heads, hd, T):
         bound = 2.0 ** -24 * np.einsum("hj,jhd->hd", w * (12 + 8 * np.abs(sc).max()), np.abs(V))
         assert (np.abs(got[i] - want) <= bound).all(), (i, float((np.abs(got[i] - want) / bound).max()))
     assert not run(0)[:2].any()
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd", [(3, 3, 64), (2, 1, 128), (3, 1, 128), (4, 1, 64), (8, 1, 128)])
+def test_batched_attention_of_one_step_takes_four_waves(pkg, heads, kv_heads, hd):
+    """Positions that four waves take in one step (64 of 128 columns, 128 of 64) are theirs however few tokens there are: the bits of the same
+    tokens in a launch of 300, which has four waves throughout. One position more, and eight waves sum in another order."""
+    from tinyllama_cpp_amd import engine as E
+    from tinyllama_cpp_amd.capi import check, lib
+    E.init(0)
+    rng = np.random.default_rng(heads * hd)
+    S, T, step = 340, 300, 4096 * 2 // hd
+    q = rng.standard_normal((T, heads, hd)).astype(np.float32)
+    pos = np.resize(np.array([0, 1, 15, 16, 31, 33, step - 2, step - 1, step, step + 40], np.int32), T)
+    dev = [E.DeviceBuffer.from_numpy(a) for a in (q, *(rng.standard_normal((S, kv_heads, hd)).astype(np.float32) for _ in range(2)))]
+    posd, seqd, out = E.DeviceBuffer.from_numpy(pos), E.DeviceBuffer.from_numpy(np.zeros(T, np.int32)), E.DeviceBuffer(4 * q.size)
+
+    def run(n):
+        check(lib().tl_debug_batch_attention(*(d.ptr for d in dev), out.ptr, 0, posd.ptr, seqd.ptr, 0, n, heads, kv_heads, hd, S, 1, 0.125, None))
+        return out.to_numpy(np.float32, q.shape)[:n]
+
+    many, few = run(T)[:10], run(10)
+    assert np.isfinite(many).all() and np.array_equal(many[:8], few[:8]) and not np.array_equal(many[8:], few[8:])
+    assert np.linalg.norm(many[8:] - few[8:]) <= 2e-6 * np.linalg.norm(many[8:])
 
 
 def test_packed_prefill_rejects_bad_batches(pkg):

@@ -160,9 +160,10 @@ __device__ __forceinline__ float batch_row_sum16(float v) {
   v = dpp_add<0x140, 0xf>(v);  // row_mirror
   return v;
 }
-// A wave alone on its SIMD issues an instruction every four cycles, and a step over 16 positions is some 700 of them: where the launch
-// leaves CUs idle, eight waves take the positions instead of four (NW): 8 sequences of 8 heads of 128 for 3 query heads each, about 95
-// positions, 8.19 -> 6.43 us in a whole call (sixteen loads in flight in four waves gained nothing: the two steps were not what it waits for).
+// A wave alone on its SIMD issues an instruction every four cycles, and a step of four waves (64 positions of 128 columns, 128 of 64) is some
+// 700 of them: where the launch leaves CUs idle and a token needs more than one such step, eight waves take its positions (NW, W). 8
+// sequences of 8 heads of 128 for 3 query heads each, at 20 / 100 / 500 / 4000 positions, four -> eight waves 4.9 / 6.3 / 16.3 / 106 -> 4.9 /
+// 6.0 / 12.7 / 75 us (20 with all eight at work: 5.7, whose fold of 32 records and second wave a SIMD are then all that is gained).
 template <int HD, int G, int NW>
 __global__ __launch_bounds__(64 * NW) void attn_batch_decode_kernel(BatchAttnArgs a) {
   constexpr int LP = 16, NV = HD / 64, PP = 64 / LP, U = 8 / NV, RECL = HD + 4;
@@ -178,6 +179,8 @@ __global__ __launch_bounds__(64 * NW) void attn_batch_decode_kernel(BatchAttnArg
   const int pos = a.pos ? a.pos[tok] : a.start_pos + tok, sq = a.seq ? a.seq[tok] : 0;
   if (pos < 0 || pos >= a.max_seq || sq < 0 || sq >= a.n_seq) return;  // uniform
   const int len = pos + 1;
+  // the waves that take positions: four where these need no second step
+  const int W = NW > 4 && len > 4 * PP * U ? NW : 4, rows = W * PP;
   const int kv_dim = a.nkv * HD;
   const float* kbase = a.kc + (size_t)sq * a.seq_stride + (size_t)kvh * HD + 4 * ln;
   const float* vbase = a.vc + (size_t)sq * a.seq_stride + (size_t)kvh * HD + 4 * ln;
@@ -193,12 +196,12 @@ __global__ __launch_bounds__(64 * NW) void attn_batch_decode_kernel(BatchAttnArg
     m[g] = -INFINITY;
     l[g] = 0.f;
   }
-  for (int base = 0; base < len; base += NW * PP * U) {
+  for (int base = 0; base < (wave < W ? len : 0); base += rows * U) {
     f32x4 kk[U][NV], vv[U][NV];
     bool valid[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {  // unconditional, clamped loads: the whole batch in flight together
-      const int idx = base + (u * NW + wave) * PP + sub;
+      const int idx = base + (u * W + wave) * PP + sub;
       valid[u] = idx < len;
       const size_t off = (size_t)(valid[u] ? idx : len - 1) * kv_dim;
 #pragma unroll
@@ -295,21 +298,23 @@ __global__ __launch_bounds__(64 * NW) void attn_batch_decode_kernel(BatchAttnArg
   // every row group's state -> an LDS record (folding the four groups of a wave in registers first is 2 x 10 LDS-path
   // shuffles per head and lane, and four exps per output element on top: as in tl_attn_body.h)
   const int rg = wave * PP + sub;
+  if (rg < rows) {
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    float* rec = part + (size_t)(rg * G + g) * RECL;
+    for (int g = 0; g < G; ++g) {
+      float* rec = part + (size_t)(rg * G + g) * RECL;
 #pragma unroll
-    for (int v = 0; v < NV; ++v) *reinterpret_cast<f32x4*>(rec + 64 * v + 4 * ln) = acc[g][v];
-    if (ln == 0) {
-      rec[HD] = m[g];
-      rec[HD + 1] = l[g];
+      for (int v = 0; v < NV; ++v) *reinterpret_cast<f32x4*>(rec + 64 * v + 4 * ln) = acc[g][v];
+      if (ln == 0) {
+        rec[HD] = m[g];
+        rec[HD + 1] = l[g];
+      }
     }
   }
   __syncthreads();
   if (tid < G * NR) {  // lane NR g + r: the weight exp(m_r - M) of row group r of head g, once; 1 / (L + 1e-9)
     const int g = tid / NR, r = tid % NR;
     const float* rec = part + (size_t)(r * G + g) * RECL;
-    const float mr = rec[HD];
+    const float mr = r < rows ? rec[HD] : -INFINITY, lr = r < rows ? rec[HD + 1] : 0.f;
     auto dmax = [](float v, auto ctrl_c) {
       constexpr int CTRL = decltype(ctrl_c)::value;
       const int t = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false);
@@ -321,7 +326,7 @@ __global__ __launch_bounds__(64 * NW) void attn_batch_decode_kernel(BatchAttnArg
     M = dmax(M, std::integral_constant<int, 0x140>{});
     if (NR == 32) M = fmaxf(M, tl_xor<16>(M));
     const float w = exp_diff(mr, M);  // (0 for a row group without rows)
-    float L = batch_row_sum16(rec[HD + 1] * w);
+    float L = batch_row_sum16(lr * w);
     if (NR == 32) L += tl_xor<16>(L);
     wts[tid] = w;
     if (r == 0) red[8 + g] = 1.0f / (L + 1e-9f);  // utils.cpp:692
@@ -330,11 +335,13 @@ __global__ __launch_bounds__(64 * NW) void attn_batch_decode_kernel(BatchAttnArg
   for (int i = tid; i < G * (HD / 4); i += 64 * NW) {
     const int g = i / (HD / 4), c4 = i % (HD / 4);
     f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int r0 = 0; r0 < rows; r0 += 16) {  // row-group order
 #pragma unroll
-    for (int r = 0; r < NR; ++r) {  // row-group order
-      const f32x4 x = *reinterpret_cast<const f32x4*>(part + (size_t)(r * G + g) * RECL + 4 * c4);
-      const float w = wts[g * NR + r];
-      o[0] = fmaf(x[0], w, o[0]); o[1] = fmaf(x[1], w, o[1]); o[2] = fmaf(x[2], w, o[2]); o[3] = fmaf(x[3], w, o[3]);
+      for (int r = r0; r < r0 + 16; ++r) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(part + (size_t)(r * G + g) * RECL + 4 * c4);
+        const float w = wts[g * NR + r];
+        o[0] = fmaf(x[0], w, o[0]); o[1] = fmaf(x[1], w, o[1]); o[2] = fmaf(x[2], w, o[2]); o[3] = fmaf(x[3], w, o[3]);
+      }
     }
     const float inv = red[8 + g];
     o[0] *= inv; o[1] *= inv; o[2] *= inv; o[3] *= inv;
@@ -384,7 +391,8 @@ int launch_attn_h(const BatchAttnArgs& a, int T, hipStream_t s) {
   const int grp = a.nh / a.nkv;
   auto go = [&](auto g_c, int parts) {
     constexpr int G = decltype(g_c)::value;
-    if ((long)a.nkv * T * parts <= tl_num_cus()) attn_batch_decode_kernel<HD, G, 8><<<dim3(a.nkv, T, parts), 512, 0, s>>>(a);
+    // 16, 24 and 28 workgroups of 32 CUs, 4 heads of 128 a workgroup, 4000 positions, four -> eight waves 148 -> 109, 149 -> 137, 153 -> 157 us
+    if ((long)a.nkv * T * parts * 4 <= tl_num_cus() * 3l) attn_batch_decode_kernel<HD, G, 8><<<dim3(a.nkv, T, parts), 512, 0, s>>>(a);
     else attn_batch_decode_kernel<HD, G, 4><<<dim3(a.nkv, T, parts), 256, 0, s>>>(a);
   };
   switch (grp) {
