@@ -30,7 +30,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
-HBM_PEAK_GBPS = 8000.0  # /opt/skills/guides/MI355X_MICROARCH.md: HBM3E 8.0 TB/s spec
+HBM_PEAK_GBPS = 8000.0  # HBM3E's 8.0 TB/s, nominal
 MIX = {"llama-3-8b": "q4_k_m", "tinyllama-1.1b": "q4_k_m", "llama-3.2-3b": "q6_k", "tiny": "q4_k_m",
        "tiny-gqa": "q4_k_m"}
 
@@ -835,7 +835,7 @@ def main():
         # the timed decode step, whose bytes are the quantized planes counted above
         "prefill_planes_bytes_per_gpu": int(model.prefill_planes_bytes()),
     }
-    if world > 1:  # the multi-rank line describes itself at the top level (the driver keeps only this line)
+    if world > 1:  # the multi-rank line describes itself at the top level (its caller may keep only this line)
         ar = kern.get("tp_all_reduce", {})
         out["ranks"] = world
         out["via"] = "replicas (tensor-parallel set-up failed)" if tp_fallback else ar.get("via", "rccl")

@@ -868,8 +868,8 @@ __device__ __forceinline__ f32x4 hparts4(const GemmParts& g, size_t o) {
 }
 constexpr int HNORM_THREADS = 512, HMAX_COLS = 8 * 8 * HNORM_THREADS;
 // WIDE (a piece a thread; launches whose workgroups are all on the chip at once, so that registers cost nothing): the row, the weights and
-// all slices in one round trip. In whole calls: 8 rows of 3072, 2 to 8 slices, 4.97 -> 4.10 us on average, 128 of 4096 7.74 -> 7.29; gate and
-// up of 8 x 8192 (hsplit_kernel) 4.46 -> 3.78.
+// all slices in one round trip. In whole calls: 8 rows of 3072, 2 to 8 slices, 5.06 -> 4.03 us on average, 128 of 4096 7.47 -> 6.53; gate and
+// up of 8 x 8192 (hsplit_kernel) 4.50 -> 3.65.
 template <int NIT, bool WIDE>
 __global__ __launch_bounds__(HNORM_THREADS) void hsplit_norm_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                     _Float16* __restrict__ planes, size_t ps, int K, float eps,

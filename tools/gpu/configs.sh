@@ -1,4 +1,4 @@
-# The other BASELINE.json configurations on one GPU (decode), plus long-context decode of the headline workload.
+# The other benchmarked shapes on one GPU (decode), plus long-context decode of the headline workload.
 cd $GRAFT_REPO_ROOT
 for w in tinyllama-1.1b llama-3.2-3b; do
   timeout -k 10 300 python bench.py --workload $w --steps 128 --warmup 16 --no-cpu-baseline > gpurun_out/cfg_$w.json 2> gpurun_out/cfg_$w.err || exit 1
