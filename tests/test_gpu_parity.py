@@ -332,6 +332,27 @@ def test_model_tinyllama_shape_two_layers(E, pkg, oracle, mix):
     om.close()
 
 
+@pytest.mark.parametrize("hidden,heads,kv,inter,mix", [
+    (2048, 32, 4, 1024, "q4_k_m"), (2048, 32, 4, 4096, "q8_0"), (2304, 36, 4, 2560, "q6_k"), (4096, 32, 8, 256, "q4_k_m"), (5120, 40, 8, 256, "q4_k_m"),
+    (256, 4, 2, 8448, "q4_k_m"), (256, 4, 2, 16640, "q6_k"), (768, 12, 4, 6144, "q8_0")])
+def test_decode_stages_its_input_in_any_number_of_pieces(E, pkg, oracle, hidden, heads, kv, inter, mix):
+    """A step's launches read their input in one, two, up to four or more pieces of 16 bytes a thread, with a norm or without, in as many
+    waves as they have rows or in more: widths and feed-forward sizes on both sides of each of these lines, in logits."""
+    cfg = dict(pkg.synth.SHAPES["tiny"], hidden=hidden, n_heads=heads, n_kv_heads=kv, inter=inter, n_layers=2, vocab=512, max_pos=160)
+    cfg, tensors = pkg.synth.build_model(cfg, mix, seed=hidden + inter)
+    m = E.Model(cfg).load(tensors)
+    om = OracleModel(oracle, cfg, tensors)
+    prompt = np.random.default_rng(inter).integers(0, cfg["vocab"], 132).astype(np.int32)  # (up to three records of the attention)
+    want = om.generate(prompt[:5], 1, penalty=1.0, dump_logits=True)[1][0], om.generate(prompt, 1, penalty=1.0, dump_logits=True)[1][0]
+    for pos, tok in enumerate(prompt):
+        logits, _ = m.decode(int(tok), pos)
+        if pos in (4, prompt.size - 1):
+            w = want[pos > 4]
+            assert close(logits, w, LOGIT_TOL).all(), (pos, np.abs(logits - w).max())
+    m.free()
+    om.close()
+
+
 def test_model_tinyllama_q8_0_prefill_then_decode(E, pkg, oracle):
     """TinyLlama-1.1B Q8_0 through the generate loop's other branch (api.cpp:601-694): a 40-token prompt goes through the batched
     prefill, then greedy decode with the default penalty 1.3; ids and the first sampled position's logits vs the oracle."""

@@ -10,7 +10,7 @@
 //   - grid (kv head, sequence split, head-group part): one workgroup serves the query heads of a kv head (GQA group), so
 //     every K/V byte is read once; groups of 8 heads (TinyLlama, the 70B shape) are served by two workgroups of 4 (their
 //     K/V rows are read twice, the per-row softmax work per workgroup halves: +11 % tokens/s on TinyLlama-1.1B); a split
-//     is max(64, pow2(len / 32)) positions (tl_attn_split_len): at most 32 splits, so that 8 kv heads fill 256 CUs from
+//     is max(64, pow2(len / 32)) positions (tl_attn_split_shift): at most 32 splits, so that 8 kv heads fill 256 CUs from
 //     2048 positions on while short contexts still spread over tens of CUs;
 //   - a K/V row is read by 16 lanes (one DPP row) x 16 B x hd/64 loads, four rows per wave load; the dot's reduction is
 //     four DPP adds (quad_perm, row_half_mirror, row_mirror) and every lane of the row ends up with the score. (The first

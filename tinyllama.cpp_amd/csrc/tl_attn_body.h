@@ -83,8 +83,7 @@ __device__ __forceinline__ void attn_split_body(const AttnArgs& a, const int kvh
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int pos = a.pos_dev ? *a.pos_dev : a.seq_len - 1;
   const int len = pos + 1;
-  const int SL = tl_attn_split_len(len);
-  const int active = (len + SL - 1) / SL;
+  const int sh = tl_attn_split_shift(len), SL = 1 << sh, active = (len + SL - 1) >> sh;
   if (split >= active || pos < 0 || pos >= a.max_seq) return;  // (the combine only reads splits < active)
   const int kv_dim = a.kv_row;
   const size_t hoff = (size_t)kvh * (size_t)a.kv_head;

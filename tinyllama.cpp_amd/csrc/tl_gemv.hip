@@ -111,7 +111,7 @@ __device__ __forceinline__ void fused_attention_phase(const ChainWait& cw, int w
   const FusedAttn& f = *cw.fa;
   const int pos = *f.at.pos_dev;  // (uniform: a scalar load)
   const int len = pos + 1;
-  const int SL = tl_attn_split_len(len), active = (len + SL - 1) / SL;
+  const int active = tl_attn_records(len, false);
   const int per = f.at.nkv * f.at.zparts;
   const int ntasks = (pos >= 0 && pos < f.at.max_seq) ? per * active : 0;
   if (ntasks == 0) return;  // (the position is out of range: the step's other kernels ignore it too)
@@ -194,51 +194,54 @@ __device__ __forceinline__ void stx1(float* p, float v) {
 // ---- x staging: (optional RMSNorm, utils.cpp:648-673) -> strided LDS image + per-chunk half sums --------------
 // Split in two so that the x loads are the FIRST loads a wave issues: loads return in order, and staging must not
 // wait behind the first weight loads (an HBM round trip) that are issued in between.
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+// SX, what a launch says about its input at compile time: 0 nothing (up to four pieces of 16 bytes a thread in registers, the rest in a
+// loop, a norm or none); SX > 0: RMSNorm, at most SX pieces a thread; SX < 0: no norm, at most -SX pieces.
+constexpr int stage_pieces(int sx) { return sx == 0 ? 4 : sx < 0 ? -sx : sx; }
+template <int SX, bool XATTN>
 struct XRegs {
-  f32x4 v[4];  // the first four float4 of a thread (covers cols <= 16 * blockDim)
-  f32x4 g[2];  // norm weights of the first two (norm launches have cols = hidden_size <= 8 * blockDim in practice)
+  f32x4 v[XATTN ? 1 : stage_pieces(SX)];
+  f32x4 g[XATTN || SX < 0 ? 1 : SX == 0 ? 2 : SX];  // norm weights (SX 0: of the first two pieces)
   // XATTN: the first XA_CHUNK split partials of the thread's first float4: out, (max, sum); and the active split count
-  f32x4 ao[6];
-  float am[6], al[6];
+  f32x4 ao[XATTN ? 6 : 1];
+  f32x2 aml[XATTN ? 6 : 1];
   int active;
 };
 
 constexpr int XA_CHUNK = 6;
-// issue the loads of splits [s0, s0 + XA_CHUNK) (clamped to the active ones) of float4 index i
+// issue the loads of splits [s0, s0 + XA_CHUNK) (clamped to the active ones) of float4 index i. Head sizes are powers of two (gemv_plan):
+// a lane's record is a 32-bit offset, a split's a scalar base
 template <bool CHAIN = false>
-__device__ __forceinline__ void xattn_issue(const GemvVec& a, int i, int s0, int active, f32x4* ao, float* am, float* al) {
-  const int hd = a.attn_hd, recl = hd + 4;
-  const int e = i << 2, h = e / hd, d = e - h * hd;
-  const float* rec0 = a.attn_ws + (size_t)h * TL_ATTN_MAX_SPLITS * recl;
+__device__ __forceinline__ void xattn_issue(const GemvVec& a, int i, int s0, int active, f32x4* ao, f32x2* aml) {
+  const unsigned hd = (unsigned)a.attn_hd, recl = hd + 4, e = (unsigned)i << 2;
+  const unsigned head = (e >> (31 - __builtin_clz(hd))) * (TL_ATTN_MAX_SPLITS * recl * 4u);
+  const unsigned oo = head + (e & (hd - 1)) * 4u, om = head + hd * 4u;
 #pragma unroll
   for (int k = 0; k < XA_CHUNK; ++k) {
     const int s = s0 + k < active ? s0 + k : active - 1;  // unconditional loads (counted waits), clamped
-    const float* rec = rec0 + (size_t)s * recl;
-    if constexpr (CHAIN) {  // the records may have been written in THIS launch (attention folded in): sc1 loads
-      const unsigned ro = (unsigned)((h * TL_ATTN_MAX_SPLITS + s) * recl);  // (wave-uniform base, per-lane offset)
-      ao[k] = ldx4<true>(a.attn_ws, (ro + (unsigned)d) * 4u);
-      am[k] = ldx1<true>(a.attn_ws + ro + hd);
-      al[k] = ldx1<true>(a.attn_ws + ro + hd + 1);
+    const float* rec = a.attn_ws + (unsigned)s * recl;
+    ao[k] = ldx4<CHAIN>(rec, oo);  // (CHAIN: the records may have been written in THIS launch, attention folded in: sc1 loads)
+    if constexpr (CHAIN) {
+      const float* ml = a.attn_ws + (om >> 2) + (unsigned)s * recl;
+      aml[k] = f32x2{ldx1<true>(ml), ldx1<true>(ml + 1)};
     } else {
-      ao[k] = *reinterpret_cast<const f32x4*>(rec + d);
-      am[k] = rec[hd];
-      al[k] = rec[hd + 1];
+      aml[k] = ldc<f32x2>(rec, om);  // (records are whole 16-byte pieces)
     }
   }
 }
-// fold a chunk into the running (M, L, O) of a float4
-__device__ __forceinline__ void xattn_fold(int s0, int active, const f32x4* ao, const float* am, const float* al, float& M,
-                                           float& L, f32x4& O) {
+// fold a chunk into the running (M, L, O) of a float4 (one straight line: a branch around the exps of records that are not there has the
+// compiler wait for the first weights in front of it)
+__device__ __forceinline__ void xattn_fold(int s0, int active, const f32x4* ao, const f32x2* aml, float& M, float& L, f32x4& O) {
   float mx = M;
 #pragma unroll
-  for (int k = 0; k < XA_CHUNK; ++k) mx = fmaxf(mx, s0 + k < active ? am[k] : -INFINITY);
+  for (int k = 0; k < XA_CHUNK; ++k) mx = fmaxf(mx, s0 + k < active ? aml[k][0] : -INFINITY);
   const float corr = M == -INFINITY ? 0.f : expf(M - mx);
   L *= corr;
   O[0] *= corr; O[1] *= corr; O[2] *= corr; O[3] *= corr;
 #pragma unroll
   for (int k = 0; k < XA_CHUNK; ++k) {
-    const float w = s0 + k < active ? expf(am[k] - mx) : 0.f;
-    L = fmaf(al[k], w, L);
+    const float w = s0 + k < active ? expf(aml[k][0] - mx) : 0.f;
+    L = fmaf(aml[k][1], w, L);
     O[0] = fmaf(ao[k][0], w, O[0]); O[1] = fmaf(ao[k][1], w, O[1]);
     O[2] = fmaf(ao[k][2], w, O[2]); O[3] = fmaf(ao[k][3], w, O[3]);
   }
@@ -246,103 +249,114 @@ __device__ __forceinline__ void xattn_fold(int s0, int active, const f32x4* ao, 
 }
 // Unconditional (index-clamped) loads: a load under a branch makes the compiler wait with vmcnt(0) at the join,
 // which would also wait for the weight loads issued after these.
-template <bool XATTN, bool CHAIN = false>
-__device__ __forceinline__ void stage_x_issue(const GemvVec& a, XRegs& r) {
+template <int SX, bool XATTN, bool CHAIN = false>
+__device__ __forceinline__ void stage_x_issue(const GemvVec& a, XRegs<SX, XATTN>& r) {
   const int n4 = a.cols >> 2;
-  if (XATTN) {
+  if constexpr (XATTN) {
     int pos;  // scalar load: its own counter, so the partial loads below need not wait behind anything
     asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(pos) : "s"(a.attn_pos) : "memory");
     r.active = tl_attn_records(pos + 1, a.attn_merged != 0);
     const int i = threadIdx.x < (unsigned)n4 ? threadIdx.x : n4 - 1;
-    xattn_issue<CHAIN>(a, i, 0, r.active, r.ao, r.am, r.al);
+    xattn_issue<CHAIN>(a, i, 0, r.active, r.ao, r.aml);
     return;
   }
-  const void* wbase = a.norm_w ? a.norm_w : a.x;
+  const void* wbase = SX > 0 || a.norm_w ? a.norm_w : a.x;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
+  for (int k = 0; k < stage_pieces(SX); ++k) {
     const int i = threadIdx.x + k * a.nthr;
     r.v[k] = ldx4<CHAIN>(a.x, (unsigned)(i < n4 ? i : n4 - 1) * 16u);
   }
+  if constexpr (SX >= 0) {
 #pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int i = threadIdx.x + k * a.nthr;
-    r.g[k] = ldc<f32x4>(wbase, (unsigned)(i < n4 ? i : n4 - 1) * 16u);
+    for (int k = 0; k < (SX == 0 ? 2 : SX); ++k) {
+      const int i = threadIdx.x + k * a.nthr;
+      r.g[k] = ldc<f32x4>(wbase, (unsigned)(i < n4 ? i : n4 - 1) * 16u);
+    }
   }
 }
 __device__ __forceinline__ float ssq4(f32x4 t) { return (t[0] * t[0] + t[1] * t[1]) + (t[2] * t[2] + t[3] * t[3]); }
-template <bool XATTN, bool CHAIN = false>
-__device__ __forceinline__ void stage_x_finish(const GemvVec& a, const XRegs& r, float* smem) {
+// Returns the RMS factor of the row (1 without a norm). It multiplies a finished row sum instead of every staged value: the launch needs
+// one barrier instead of two, and the factor's chain of instructions lies where the first weights are waited for. (One rounding less
+// per value; the sums' range moves by the factor, 1e19 at most below which its own sum of squares overflows.)
+template <int SX, bool XATTN, bool CHAIN = false>
+__device__ __forceinline__ float stage_x_finish(const GemvVec& a, const XRegs<SX, XATTN>& r, float* smem) {
   float* xs = smem + XS_SCRATCH;
   const int tid = threadIdx.x, nthr = a.nthr;
   const int n4 = a.cols >> 2;
-  if (XATTN) {
+  // four values of the image; a chunk's half sums behind its 32 values (n4 is a multiple of 8 and blockDim of 64, so quads of threads are
+  // all-in or all-out of every branch)
+  auto put = [&](int i, f32x4 t) __attribute__((always_inline)) {
+    float* dst = xs + (i >> 3) * XS_STRIDE;
+    *reinterpret_cast<f32x4*>(dst + ((i & 7) << 2)) = t;
+    float s = (t[0] + t[1]) + (t[2] + t[3]);
+    s = dpp_add<0x4E, 0xf>(dpp_add<0xB1, 0xf>(s));  // quad sum in every lane of the quad (DPP, no LDS path)
+    if ((i & 3) == 0) dst[32 + ((i >> 2) & 1)] = s;
+  };
+  if constexpr (XATTN) {
     // x = combined attention output: out = sum_s o_s e^(m_s - M) / (sum_s l_s e^(m_s - M) + 1e-9), utils.cpp:692
     for (int i = tid; i < n4; i += nthr) {
       float M = -INFINITY, L = 0.f;
       f32x4 O = {0.f, 0.f, 0.f, 0.f};
       if (i == tid) {
-        xattn_fold(0, r.active, r.ao, r.am, r.al, M, L, O);
+        xattn_fold(0, r.active, r.ao, r.aml, M, L, O);
       } else {
         f32x4 ao[XA_CHUNK];
-        float am[XA_CHUNK], al[XA_CHUNK];
-        xattn_issue<CHAIN>(a, i, 0, r.active, ao, am, al);
-        xattn_fold(0, r.active, ao, am, al, M, L, O);
+        f32x2 aml[XA_CHUNK];
+        xattn_issue<CHAIN>(a, i, 0, r.active, ao, aml);
+        xattn_fold(0, r.active, ao, aml, M, L, O);
       }
       for (int s0 = XA_CHUNK; s0 < r.active; s0 += XA_CHUNK) {
         f32x4 ao[XA_CHUNK];
-        float am[XA_CHUNK], al[XA_CHUNK];
-        xattn_issue<CHAIN>(a, i, s0, r.active, ao, am, al);
-        xattn_fold(s0, r.active, ao, am, al, M, L, O);
+        f32x2 aml[XA_CHUNK];
+        xattn_issue<CHAIN>(a, i, s0, r.active, ao, aml);
+        xattn_fold(s0, r.active, ao, aml, M, L, O);
       }
       const float inv = 1.0f / (L + 1e-9f);
-      f32x4 t = {O[0] * inv, O[1] * inv, O[2] * inv, O[3] * inv};
-      const int idx = i << 2;
-      float* dst = xs + (idx >> 5) * XS_STRIDE;
-      *reinterpret_cast<f32x4*>(dst + (idx & 31)) = t;
-      float sm4 = (t[0] + t[1]) + (t[2] + t[3]);
-      sm4 = dpp_add<0x4E, 0xf>(dpp_add<0xB1, 0xf>(sm4));  // quad sum in every lane of the quad (DPP, no LDS path)
-      if ((i & 3) == 0) dst[32 + ((i >> 2) & 1)] = sm4;
+      put(i, f32x4{O[0] * inv, O[1] * inv, O[2] * inv, O[3] * inv});
     }
     __syncthreads();
-    return;
-  }
-  const f32x4* x4 = reinterpret_cast<const f32x4*>(a.x);
-  const f32x4* w4 = reinterpret_cast<const f32x4*>(a.norm_w);
-  float nf = 1.0f;
-  if (a.norm_w) {
+    return 1.0f;
+  } else {
+    const f32x4* x4 = reinterpret_cast<const f32x4*>(a.x);
+    const f32x4* w4 = reinterpret_cast<const f32x4*>(a.norm_w);
+    const bool norm = SX > 0 || (SX == 0 && a.norm_w);
     float ssq = 0.f;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) ssq += (tid + k * nthr < n4) ? ssq4(r.v[k]) : 0.f;
-    for (int i = tid + 4 * nthr; i < n4; i += nthr) ssq += ssq4(CHAIN ? ldx4<CHAIN>(a.x, (unsigned)i * 16u) : x4[i]);
-    ssq = wave_sum_lane63(ssq);  // DPP only (the xor butterfly is six dependent LDS-path shuffles here)
-    if ((tid & 63) == 63) smem[tid >> 6] = ssq;
-    __syncthreads();
-    float tot = 0.f;
-    for (int w = 0; w < (nthr >> 6); ++w) tot += smem[w];
-    const float e = a.eps < 1e-5f ? 1e-5f : a.eps;  // SAFE_MAX(eps, MIN_NORM_EPS)
-    nf = 1.0f / sqrtf(tot / (float)a.cols + e);
-  }
-  auto put = [&](int i, f32x4 t, f32x4 g) {
-    if (a.norm_w) {
-      t[0] = t[0] * nf * g[0]; t[1] = t[1] * nf * g[1]; t[2] = t[2] * nf * g[2]; t[3] = t[3] * nf * g[3];
+    for (int k = 0; k < stage_pieces(SX); ++k) {
+      const int i = tid + k * nthr;
+      if (i < n4) {
+        f32x4 t = r.v[k];
+        if (norm) {
+          ssq += ssq4(t);
+          if (SX > 0 || k < 2) t *= r.g[SX < 0 ? 0 : k < (SX == 0 ? 2 : SX) ? k : 0];
+          else t *= w4[i];
+        }
+        put(i, t);
+      }
     }
-    const int idx = i << 2;
-    float* dst = xs + (idx >> 5) * XS_STRIDE;
-    *reinterpret_cast<f32x4*>(dst + (idx & 31)) = t;
-    // 4 consecutive threads cover 16 consecutive x: their sum is one of the chunk's two half sums
-    float s = (t[0] + t[1]) + (t[2] + t[3]);
-    s = dpp_add<0x4E, 0xf>(dpp_add<0xB1, 0xf>(s));  // quad sum in every lane of the quad (DPP, no LDS path)
-    if ((i & 3) == 0) dst[32 + ((i >> 2) & 1)] = s;
-  };
-  // n4 is a multiple of 8 and blockDim of 64, so quads of threads are all-in or all-out of every branch
-  const f32x4 one = {1.f, 1.f, 1.f, 1.f};
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int i = tid + k * nthr;
-    if (i < n4) put(i, r.v[k], k < 2 ? r.g[k] : (a.norm_w ? w4[i] : one));
+    if constexpr (SX == 0) {
+      for (int i = tid + 4 * nthr; i < n4; i += nthr) {
+        f32x4 t = CHAIN ? ldx4<CHAIN>(a.x, (unsigned)i * 16u) : x4[i];
+        if (norm) {
+          ssq += ssq4(t);
+          t *= w4[i];
+        }
+        put(i, t);
+      }
+    }
+    if (norm) {
+      ssq = wave_sum_lane63(ssq);  // DPP only (the xor butterfly is six dependent LDS-path shuffles here)
+      if ((tid & 63) == 63) smem[tid >> 6] = ssq;
+    }
+    __syncthreads();
+    if (!norm) return 1.0f;
+    const int w = tid & 15;  // at most 16 waves: every row of 16 lanes adds their sums up
+    float tot = smem[w];
+    tot = w < (nthr >> 6) ? tot : 0.f;
+    tot = dpp_add<0x140, 0xf>(dpp_add<0x141, 0xf>(dpp_add<0x4E, 0xf>(dpp_add<0xB1, 0xf>(tot))));
+    const float e = a.eps < 1e-5f ? 1e-5f : a.eps;  // SAFE_MAX(eps, MIN_NORM_EPS)
+    return 1.0f / sqrtf(tot / (float)a.cols + e);
   }
-  for (int i = tid + 4 * nthr; i < n4; i += nthr) put(i, CHAIN ? ldx4<CHAIN>(a.x, (unsigned)i * 16u) : x4[i], a.norm_w ? w4[i] : one);
-  __syncthreads();
 }
 
 // ---- the kernel ------------------------------------------------------------------------------------------------
@@ -355,10 +369,16 @@ struct Segs {
 };
 
 // row group `rg` of a class: rows (2*lt, 2*lt+1) of one of its segments, or row lt of the gate/up pair
-template <bool PAIR>
+// (ONE: the launch is one matrix)
+template <bool PAIR, bool ONE>
 __device__ __forceinline__ void group_of(const Segs& g, int rg, QW& wa, QW& wb, int& ra, int& rb, float*& out) {
   if (PAIR) {  // wa / wb / out were set once by the caller and never change
     ra = rb = rg;
+    return;
+  }
+  if (ONE) {
+    ra = 2 * rg;
+    rb = ra + 1 < wa.rows ? ra + 1 : wa.rows - 1;
     return;
   }
   int seg = 0, lt = rg;
@@ -479,14 +499,21 @@ struct StepMeta {
 // CHAIN (a task of a chain launch): x and the first residual values are loaded only AFTER the wait for the predecessor
 // task, which follows the first weight loads; activation loads and stores take their sc1 forms.
 // AHD > 0 (with CHAIN): the launch carries its layer's attention (fused_attention_phase<AHD, AG>) in place of the wait.
-template <int TYPE, bool PAIR, bool RESID, bool XATTN, bool STAMP, bool PEER = false, bool CHAIN = false, int AHD = 0,
-          int AG = 0>
-__device__ __forceinline__ void run_class(const Segs& g, const GemvVec& a, XRegs& xr, float* smem, int first,
+// KS: a wave has one row group at most and of that the spans sp0 .. sp1 - 1 only; the waves of a row group, `rows_waves` apart, leave their
+// sums in LDS (one matrix with a residual, no norm: the reduction scratch in front of the x image is free) and the first of them adds
+// them up.
+struct KPart {
+  int sp0, sp1, wave, row_waves, parts;
+};
+template <int TYPE, bool PAIR, bool ONE, bool RESID, int SX, bool XATTN, bool STAMP, bool PEER = false, bool CHAIN = false, int AHD = 0,
+          int AG = 0, bool KS = false>
+__device__ __forceinline__ void run_class(const Segs& g, const GemvVec& a, XRegs<SX, XATTN>& xr, float* smem, int first,
                                           int stride, int total, int lane, unsigned long long* ts, unsigned pe = 0,
-                                          int peer_wave = 0, const ChainWait* cw = nullptr) {
+                                          int peer_wave = 0, const ChainWait* cw = nullptr, const KPart kp = {}) {
+  static_assert(!KS || (ONE && RESID && !PEER && !CHAIN && !STAMP && (XATTN || SX < 0)), "");
   const float* xs = smem + XS_SCRATCH;
   const int nchunks = a.cols >> 5;
-  const int nspans = (nchunks + 63) >> 6;
+  const int nspans = KS ? kp.sp1 : (nchunks + 63) >> 6;
   // PEER: this wave's slice of the stash behind the x image, and the row groups it has finished
   float* stash = smem + XS_SCRATCH + nchunks * XS_STRIDE + 2 * peer_wave * a.peer_gpw;
   int ndone = 0;
@@ -495,18 +522,20 @@ __device__ __forceinline__ void run_class(const Segs& g, const GemvVec& a, XRegs
     if constexpr (CHAIN) {
       if constexpr (AHD > 0) fused_attention_phase<AHD, AG>(*cw, peer_wave, lane);
       else chain_wait(*cw, peer_wave, lane);
-      stage_x_issue<XATTN, CHAIN>(a, xr);
+      stage_x_issue<SX, XATTN, CHAIN>(a, xr);
     }
-    stage_x_finish<XATTN, CHAIN>(a, xr, smem);
+    stage_x_finish<SX, XATTN, CHAIN>(a, xr, smem);
     if (STAMP) ts[4] = __builtin_readcyclecounter();
+    if (KS) __syncthreads();
     return;
   }
-  int irg = first, isp = 0;
+  int irg = first, isp = KS ? kp.sp0 : 0;
   QW wa = g.w0, wb = PAIR ? g.w1 : g.w0;
   int ra = 0, rb = 0;
   float* out = g.o0;
-  group_of<PAIR>(g, irg, wa, wb, ra, rb, out);
-  float acc0 = 0.f, acc1 = 0.f;
+  group_of<PAIR, ONE>(g, irg, wa, wb, ra, rb, out);
+  float acc0 = 0.f, acc1 = 0.f, nf = 1.0f;
+  constexpr bool NORM = SX >= 0 && !XATTN;
   bool with_resid = !CHAIN;  // (CHAIN: the first step's residual values follow the wait)
 
   auto issue = [&](Step<TYPE>& st, StepMeta& m) {
@@ -525,7 +554,7 @@ __device__ __forceinline__ void run_class(const Segs& g, const GemvVec& a, XRegs
     if (++isp == nspans) {  // advance the issue cursor (scalar work, overlaps the loads)
       isp = 0;
       irg += stride;
-      if (irg < total) group_of<PAIR>(g, irg, wa, wb, ra, rb, out);
+      if (!KS && irg < total) group_of<PAIR, ONE>(g, irg, wa, wb, ra, rb, out);
     }
   };
   auto consume = [&](const Step<TYPE>& st, const StepMeta& m) {
@@ -545,10 +574,17 @@ __device__ __forceinline__ void run_class(const Segs& g, const GemvVec& a, XRegs
     acc0 += act ? d0 : 0.0f;
     acc1 += act ? d1 : 0.0f;
     if (m.sp == nspans - 1) {  // row group complete: reduce, epilogue, store
-      const float y0 = wave_sum_lane63(acc0);
-      const float y1 = wave_sum_lane63(acc1);
+      float y0 = wave_sum_lane63(acc0);
+      float y1 = wave_sum_lane63(acc1);
+      if (NORM) {
+        y0 *= nf;
+        y1 *= nf;
+      }
       if (lane == 63) {
-        if (PAIR) {
+        if (KS) {
+          smem[2 * kp.wave] = y0;
+          smem[2 * kp.wave + 1] = y1;
+        } else if (PAIR) {
           const float sg = 1.0f / (1.0f + expf(-y0));  // silu_cpu (utils.cpp:700-707), then * up (model.cpp:735)
           stx1<CHAIN>(m.out + m.ra, (y0 * sg) * y1);
         } else if (PEER) {  // into the wave's stash; pushed and collected at the end of the wave's work (peer_collect)
@@ -585,14 +621,14 @@ __device__ __forceinline__ void run_class(const Segs& g, const GemvVec& a, XRegs
     if constexpr (AHD > 0) fused_attention_phase<AHD, AG>(*cw, peer_wave, lane);
     else chain_wait(*cw, peer_wave, lane);
     chain_stamp(cw, 2);
-    stage_x_issue<XATTN, CHAIN>(a, xr);
+    stage_x_issue<SX, XATTN, CHAIN>(a, xr);
     if (RESID) {
       cur.r0 = ldx1<CHAIN>(a.resid + ra0);
       cur.r1 = ldx1<CHAIN>(a.resid + rb0);
     }
     with_resid = true;
   }
-  stage_x_finish<XATTN, CHAIN>(a, xr, smem);
+  nf = stage_x_finish<SX, XATTN, CHAIN>(a, xr, smem);
   if constexpr (CHAIN) chain_stamp(cw, 3);
   if (STAMP) ts[4] = __builtin_readcyclecounter();
   while (irg < total) {
@@ -606,6 +642,14 @@ __device__ __forceinline__ void run_class(const Segs& g, const GemvVec& a, XRegs
   if constexpr (CHAIN) chain_stamp(cw, 4);
   consume(cur, mc);
   if (STAMP && ts[5] == 0) ts[5] = __builtin_readcyclecounter();
+  if constexpr (KS) {
+    __syncthreads();
+    if (kp.wave < kp.row_waves && lane < 2 && ra0 + lane < wa.rows) {
+      float y = smem[2 * kp.wave + lane];
+      for (int p = 1; p < kp.parts; ++p) y += smem[2 * (kp.wave + p * kp.row_waves) + lane];
+      stg_f32(out + ra0 + lane, (lane ? cur.r1 : cur.r0) + y);
+    }
+  }
   if (PEER) peer_collect<RESID>(a.peer, pe, g.o0, g.w0.rows, first, stride, ndone, stash, lane);
 }
 
@@ -629,9 +673,9 @@ struct StepMetaF {
   float* out;
 };
 
-template <bool PAIR, int RPG>
+template <bool PAIR, bool ONE, int RPG>
 __device__ __forceinline__ void group_of_flat(const Segs& g, int rg, QW& wa, QW& wb, int& ra, float*& out) {
-  if (PAIR) {  // wa / wb / out were set once by the caller and never change
+  if (PAIR || ONE) {  // wa / wb / out were set once by the caller and never change
     ra = rg * RPG;
     return;
   }
@@ -658,22 +702,24 @@ __device__ __forceinline__ void group_of_flat(const Segs& g, int rg, QW& wa, QW&
   ra = RPG * lt;
 }
 
-template <int TYPE, bool PAIR, bool RESID, bool XATTN, int RA>
-__device__ __forceinline__ void run_class_flat(const Segs& g, const GemvVec& a, const XRegs& xr, float* smem, int first,
+template <int TYPE, bool PAIR, bool ONE, bool RESID, int SX, bool XATTN, int RA>
+__device__ __forceinline__ void run_class_flat(const Segs& g, const GemvVec& a, const XRegs<SX, XATTN>& xr, float* smem, int first,
                                                int stride, int total, int lane) {
   constexpr int RPG = PAIR ? RA : 2 * RA;  // output rows per group
   const float* xs = smem + XS_SCRATCH;
   const int nchunks = a.cols >> 5;                  // > 64 (host)
   const int nsteps = (RA * nchunks + 63) >> 6;
   if (first >= total) {
-    stage_x_finish<XATTN>(a, xr, smem);
+    stage_x_finish<SX, XATTN>(a, xr, smem);
     return;
   }
+  constexpr bool NORM = SX >= 0 && !XATTN;
+  float nf = 1.0f;
   int irg = first, is = 0, ij0 = 0, ioff0 = 0;  // issue cursor: group, step, first row / chunk offset of the step
   QW wa = g.w0, wb = PAIR ? g.w1 : g.w0;
   int ra = 0;
   float* out = g.o0;
-  group_of_flat<PAIR, RPG>(g, irg, wa, wb, ra, out);
+  group_of_flat<PAIR, ONE, RPG>(g, irg, wa, wb, ra, out);
   float acc[2 * RA];
 #pragma unroll
   for (int k = 0; k < 2 * RA; ++k) acc[k] = 0.f;
@@ -712,7 +758,7 @@ __device__ __forceinline__ void run_class_flat(const Segs& g, const GemvVec& a, 
       ij0 = 0;
       ioff0 = 0;
       irg += stride;
-      if (irg < total) group_of_flat<PAIR, RPG>(g, irg, wa, wb, ra, out);
+      if (irg < total) group_of_flat<PAIR, ONE, RPG>(g, irg, wa, wb, ra, out);
     }
   };
   auto consume = [&](const StepF<TYPE, RA>& st, const StepMetaF& m) {
@@ -743,6 +789,7 @@ __device__ __forceinline__ void run_class_flat(const Segs& g, const GemvVec& a, 
 #pragma unroll
       for (int k = 0; k < 2 * RA; ++k) {
         y[k] = wave_sum_lane63(acc[k]);
+        if (NORM) y[k] *= nf;
         acc[k] = 0.f;
       }
       if (lane == 63) {
@@ -764,7 +811,7 @@ __device__ __forceinline__ void run_class_flat(const Segs& g, const GemvVec& a, 
   StepF<TYPE, RA> cur, nxt;  // depth-one software pipeline in the copy form (see run_class)
   StepMetaF mc, mn;
   issue(cur, mc);
-  stage_x_finish<XATTN>(a, xr, smem);
+  nf = stage_x_finish<SX, XATTN>(a, xr, smem);
   while (irg < total) {
     issue(nxt, mn);
     consume(cur, mc);
@@ -783,13 +830,14 @@ __device__ __forceinline__ void run_class_flat(const Segs& g, const GemvVec& a, 
 // The body of a launch; `bid` is the workgroup's index among the a.grid workgroups of the launch (blockIdx.x), or of its
 // task in a chain launch (CHAIN; cw says what to wait for; RA = 0, no PEER).
 template <int TA, int TB, bool PAIR, int ROLE, bool STAMP = false, int RA = 0, bool PEER = false, bool CHAIN = false,
-          int AHD = 0, int AG = 0>
+          int AHD = 0, int AG = 0, int SX = 0, bool KS = false>
 __device__ __forceinline__ void gemv_body(const GemvSeg& sg0, const GemvSeg& sg1, const GemvSeg& sg2, const GemvVec& a,
                                           int t0, int t1, int t2, int nsegA, int wavesA, int bid, float* smem,
                                           const ChainWait* cw = nullptr) {
   // the roles launched with a residual / with x still in attention partials
   constexpr bool RESID = ROLE == GEMV_ATTN_OUT || ROLE == GEMV_DOWN || ROLE == GEMV_ATTN_OUT_COMBINE;
   constexpr bool XATTN = ROLE == GEMV_ATTN_OUT_COMBINE;
+  constexpr bool ONE = !PAIR && (RESID || ROLE == GEMV_LM_HEAD);  // (gemv_plan: one matrix)
   unsigned long long ts[8] = {0, 0, 0, 0, 0, 0, 0, 0}, rt0 = 0;
   if (STAMP) {
     ts[0] = __builtin_readcyclecounter();
@@ -812,8 +860,8 @@ __device__ __forceinline__ void gemv_body(const GemvSeg& sg0, const GemvSeg& sg1
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nwaves = a.nthr >> 6;
-  XRegs xr;
-  if constexpr (!CHAIN) stage_x_issue<XATTN>(a, xr);  // (CHAIN: after the wait for the predecessor task, in run_class)
+  XRegs<SX, XATTN> xr;
+  if constexpr (!CHAIN) stage_x_issue<SX, XATTN>(a, xr);  // (CHAIN: after the wait for the predecessor task, in run_class)
   if (STAMP) ts[2] = __builtin_readcyclecounter();
   unsigned pe = 0;  // the epoch this launch's words carry: one more than the exchanges completed (0 = cleared area)
   if (PEER) {
@@ -822,12 +870,17 @@ __device__ __forceinline__ void gemv_body(const GemvSeg& sg0, const GemvSeg& sg1
   }
   if (TB == TL_NONE || wave < wavesA) {
     const int wA = TB == TL_NONE ? nwaves : wavesA;
-    const int total = PAIR ? t0 : (nsegA == 1 ? t0 : (nsegA == 2 ? t0 + t1 : t0 + t1 + t2));
+    const int total = PAIR || ONE ? t0 : (nsegA == 1 ? t0 : (nsegA == 2 ? t0 + t1 : t0 + t1 + t2));
     const Segs g = {sg0.w, sg1.w, sg2.w, sg0.out, sg1.out, sg2.out, t0, nsegA >= 2 ? t1 : 0x3fffffff};
-    if constexpr (RA > 0)
-      run_class_flat<TA, PAIR, RESID, XATTN, RA>(g, a, xr, smem, wave * a.grid + bid, a.grid * wA, total, lane);
+    if constexpr (KS) {  // wavesA: waves of a part; t1: 4096 / wavesA rounded up; t2: parts
+      const int part = (int)((unsigned)(wave * t1) >> 12), spans = ((a.cols >> 5) + 63) >> 6;
+      const KPart kp = {part * spans / t2, (part + 1) * spans / t2, wave, wavesA, t2};
+      run_class<TA, PAIR, ONE, RESID, SX, XATTN, false, false, false, 0, 0, true>(
+          g, a, xr, smem, part < t2 ? (wave - part * wavesA) * a.grid + bid : total, total, total, lane, ts, 0, wave, nullptr, kp);
+    } else if constexpr (RA > 0)
+      run_class_flat<TA, PAIR, ONE, RESID, SX, XATTN, RA>(g, a, xr, smem, wave * a.grid + bid, a.grid * wA, total, lane);
     else
-      run_class<TA, PAIR, RESID, XATTN, STAMP, PEER, CHAIN, AHD, AG>(g, a, xr, smem, wave * a.grid + bid, a.grid * wA, total,
+      run_class<TA, PAIR, ONE, RESID, SX, XATTN, STAMP, PEER, CHAIN, AHD, AG>(g, a, xr, smem, wave * a.grid + bid, a.grid * wA, total,
                                                                      lane, ts, pe, wave, cw);
   } else if (TB != TL_NONE) {
     constexpr int TBB = TB == TL_NONE ? TA : TB;
@@ -835,10 +888,10 @@ __device__ __forceinline__ void gemv_body(const GemvSeg& sg0, const GemvSeg& sg1
     const int tb = nsegA == 1 ? t1 : t2;
     const Segs g = {sb.w, sb.w, sb.w, sb.out, sb.out, sb.out, 0x3fffffff, 0x3fffffff};
     if constexpr (RA > 0)
-      run_class_flat<TBB, false, false, XATTN, RA>(g, a, xr, smem, (wave - wavesA) * a.grid + bid,
+      run_class_flat<TBB, false, true, false, SX, XATTN, RA>(g, a, xr, smem, (wave - wavesA) * a.grid + bid,
                                                    a.grid * (nwaves - wavesA), tb, lane);
     else
-      run_class<TBB, false, false, XATTN, STAMP, false, CHAIN>(g, a, xr, smem, (wave - wavesA) * a.grid + bid,
+      run_class<TBB, false, true, false, SX, XATTN, STAMP, false, CHAIN>(g, a, xr, smem, (wave - wavesA) * a.grid + bid,
                                                                a.grid * (nwaves - wavesA), tb, lane, ts, 0, wave, cw);
   }
   if (PEER) {  // every wave has read the epoch and collected its rows: the last workgroup through advances the epoch
@@ -869,11 +922,11 @@ __device__ __forceinline__ void gemv_body(const GemvSeg& sg0, const GemvSeg& sg1
 struct GemvPad {
   int unused[11];
 };
-template <int TA, int TB, bool PAIR, int ROLE, bool STAMP = false, int RA = 0, bool PEER = false>
+template <int TA, int TB, bool PAIR, int ROLE, bool STAMP = false, int RA = 0, bool PEER = false, int SX = 0, bool KS = false>
 __global__ __launch_bounds__(GEMV_MAX_THREADS) void gemv_kernel(GemvSeg sg0, GemvSeg sg1, GemvSeg sg2, GemvVec a,
                                                                 int t0, int t1, int t2, int nsegA, int wavesA, GemvPad) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
-  gemv_body<TA, TB, PAIR, ROLE, STAMP, RA, PEER>(sg0, sg1, sg2, a, t0, t1, t2, nsegA, wavesA, blockIdx.x, smem);
+  gemv_body<TA, TB, PAIR, ROLE, STAMP, RA, PEER, false, 0, 0, SX, KS>(sg0, sg1, sg2, a, t0, t1, t2, nsegA, wavesA, blockIdx.x, smem);
 }
 
 // ---- the attn_output launch that carries its layer's attention (RoPE + KV write + split attention, tl_attn_body.h) -------
@@ -1023,19 +1076,50 @@ struct Launch {
   int nsegA, wavesA;
   int grid, threads;
   size_t lds;
+  int parts;  // > 1: the spans of a row group are dealt to so many waves, wavesA apart
   int ra;  // 0: span steps; 2 / 4: flattened steps with that many rows per stream and group
 };
 
-template <int TA, int TB, bool PAIR, int ROLE, bool STAMP = false, int RA = 0, bool PEER = false>
-static int gemv_launch_ra(const Launch& L, hipStream_t s) {
+template <int TA, int TB, bool PAIR, int ROLE, bool STAMP, int RA, bool PEER, int SX, bool KS = false>
+static int gemv_launch_sx(const Launch& L, hipStream_t s) {
   static TlDeviceOnce lds_raised;  // per kernel instantiation, per device
-  TL_TRY(tl_raise_lds_limit(gemv_kernel<TA, TB, PAIR, ROLE, STAMP, RA, PEER>, 160 * 1024, lds_raised));
+  TL_TRY(tl_raise_lds_limit(gemv_kernel<TA, TB, PAIR, ROLE, STAMP, RA, PEER, SX, KS>, 160 * 1024, lds_raised));
   GemvVec v = L.v;
   v.nthr = L.threads;
   v.grid = L.grid;
-  gemv_kernel<TA, TB, PAIR, ROLE, STAMP, RA, PEER><<<L.grid, L.threads, L.lds, s>>>(L.seg[0], L.seg[1], L.seg[2], v, L.t[0],
-                                                                                     L.t[1], L.t[2], L.nsegA, L.wavesA, GemvPad{});
+  gemv_kernel<TA, TB, PAIR, ROLE, STAMP, RA, PEER, SX, KS><<<L.grid, L.threads, L.lds, s>>>(L.seg[0], L.seg[1], L.seg[2], v, L.t[0],
+                                                                                         L.t[1], L.t[2], L.nsegA, L.wavesA, GemvPad{});
   return 0;
+}
+// The step's own launches know their input: how many pieces a thread stages, a norm or none (other sizes, Q8_K and launches that carry an
+// exchange take the general form). A launch's prologue is bound by its instructions, sixteen waves sharing four SIMDs: with four clamped
+// pieces a thread, both cases of the norm, two IEEE divisions and a root in front of the staged values, and a second barrier, 270 a wave; now 110.
+// us with a norm, before / after: 1.1B Q4_K_M q | k | v 4.0 / 3.45, gate and up 6.9 / 5.9, 3B Q6_K 7.05 / 6.05 and 11.1 / 10.4, 8B Q4_K_M 6.9 /
+// 5.6 and 15.5 / 14.8; attn_output with 32-bit record addresses and one matrix at compile time 4.65 / 4.1, 6.7 / 6.4, 6.95 / 6.5
+template <int TA, int TB, bool PAIR, int ROLE, bool STAMP = false, int RA = 0, bool PEER = false>
+static int gemv_launch_ra(const Launch& L, hipStream_t s) {
+  const int pieces = (L.v.cols / 4 + L.threads - 1) / L.threads;
+  if constexpr (!STAMP && !PEER && TA != TL_Q8_K) {
+    if constexpr (PAIR || ROLE == GEMV_QKV || ROLE == GEMV_LM_HEAD) {
+      if (L.v.norm_w && pieces <= 1) return gemv_launch_sx<TA, TB, PAIR, ROLE, STAMP, RA, PEER, 1>(L, s);
+      if (L.v.norm_w && pieces <= 2) return gemv_launch_sx<TA, TB, PAIR, ROLE, STAMP, RA, PEER, 2>(L, s);
+    }
+    if constexpr (RA == 0 && (ROLE == GEMV_DOWN || ROLE == GEMV_ATTN_OUT_COMBINE)) {
+      if (L.parts > 1) {
+        Launch K = L;
+        K.t[1] = (4096 + L.wavesA - 1) / L.wavesA;
+        K.t[2] = L.parts;
+        if constexpr (ROLE == GEMV_ATTN_OUT_COMBINE) return gemv_launch_sx<TA, TB, PAIR, ROLE, STAMP, RA, PEER, 0, true>(K, s);
+        else return pieces <= 2 ? gemv_launch_sx<TA, TB, PAIR, ROLE, STAMP, RA, PEER, -2, true>(K, s)
+                                : gemv_launch_sx<TA, TB, PAIR, ROLE, STAMP, RA, PEER, -4, true>(K, s);
+      }
+    }
+    if constexpr (ROLE == GEMV_DOWN) {
+      if (!L.v.norm_w && pieces <= 2) return gemv_launch_sx<TA, TB, PAIR, ROLE, STAMP, RA, PEER, -2>(L, s);
+      if (!L.v.norm_w && pieces <= 4) return gemv_launch_sx<TA, TB, PAIR, ROLE, STAMP, RA, PEER, -4>(L, s);
+    }
+  }
+  return gemv_launch_sx<TA, TB, PAIR, ROLE, STAMP, RA, PEER, 0>(L, s);
 }
 template <int TA, int TB, bool PAIR, int ROLE, bool STAMP = false>
 static int gemv_launch_one(const Launch& L, hipStream_t s) {
@@ -1108,11 +1192,16 @@ static int gemv_flat_rows(int cols, bool allowed, long total_rows, bool pair) {
   return best;
 }
 
-static int gemv_geometry(Launch& L, int total) {
+// Waves that share the rows: twelve of Q4_K and Q6_K. A launch's prologue is the instructions of its waves, which share the SIMDs' issue
+// slots, and three waves a SIMD ask for enough. A token in us in sixteen / twelve: 1.1B Q4_K_M 513 / 503, Q6_K 584 / 573, 3B Q4_K_M 910
+// / 887, Q6_K 1005 / 991, 8B Q4_K_M 1419 / 1406, Q6_K 1663 / 1648; of Q8_0, which has more bytes a row, 1.1B 560 / 557, but 3B 1073 / 1082
+// and 8B 1963 / 1970 (eight waves: 1 to 7 % behind the better one in 3B and 8B).
+static int gemv_row_waves(int type) { return (type == TL_Q4_K || type == TL_Q6_K) && g_max_waves > 12 ? 12 : g_max_waves; }
+static int gemv_geometry(Launch& L, int total, int most_waves) {
   // one workgroup per CU, all resident at once; small problems use fewer CUs / fewer waves per workgroup
   L.grid = total < g_num_cus ? total : g_num_cus;
   int waves = (total + L.grid - 1) / L.grid;
-  if (waves > g_max_waves) waves = g_max_waves;
+  if (waves > most_waves) waves = most_waves;
   if (waves < 4) waves = 4;  // the x staging pass wants a few waves
   L.threads = waves * 64;
   return waves;
@@ -1136,6 +1225,7 @@ static int gemv_plan(const GemvArgs& a, Launch& L, int* role_out, bool* classB_o
   for (int i = 0; i < a.nseg; ++i)
     if (a.seg[i].w.type == TL_F32) return 0;
   L = Launch{};
+  L.parts = 1;
   L.lds = sizeof(float) * (XS_SCRATCH + (size_t)(a.cols / 32) * XS_STRIDE);
   TL_REQUIRE(L.lds <= 160 * 1024, "gemv: cols %d needs %zu B of LDS (> 160 KiB)", a.cols, L.lds);
   L.v = GemvVec{a.x, a.norm_w, a.resid, a.eps, a.cols, nullptr, a.attn_ws, a.attn_pos, a.attn_hd, a.attn_merged, 0, 0, a.peer, 0};
@@ -1154,7 +1244,7 @@ static int gemv_plan(const GemvArgs& a, Launch& L, int* role_out, bool* classB_o
     if (a.seg[1].w.type != ta) return 0;  // gate and up in different formats: unfused
     L.t[0] = L.ra ? (a.seg[0].w.rows + L.ra - 1) / L.ra : a.seg[0].w.rows;
     L.nsegA = 2;
-    L.wavesA = gemv_geometry(L, L.t[0]);
+    L.wavesA = gemv_geometry(L, L.t[0], gemv_row_waves(ta));
     *role_out = GEMV_GATE_UP;
     *plain = true;
     return 0;
@@ -1179,7 +1269,7 @@ static int gemv_plan(const GemvArgs& a, Launch& L, int* role_out, bool* classB_o
   }
   L.nsegA = nsegA;
   const int total = classB ? totalA + L.t[nsegA] : totalA;
-  const int waves = gemv_geometry(L, total);
+  const int waves = gemv_geometry(L, total, gemv_row_waves(ta));
   L.wavesA = waves;
   if (a.peer) {  // the waves' stashes of finished rows behind the x image
     L.v.peer_gpw = (total + L.grid * waves - 1) / (L.grid * waves);
@@ -1200,11 +1290,32 @@ static int gemv_plan(const GemvArgs& a, Launch& L, int* role_out, bool* classB_o
   int role = a.role;  // the residual epilogue is compiled into the ATTN_OUT / DOWN instantiations only
   if (a.resid && role != GEMV_ATTN_OUT && role != GEMV_DOWN) role = GEMV_ATTN_OUT;
   if (!a.resid && (role == GEMV_ATTN_OUT || role == GEMV_DOWN)) role = GEMV_GENERIC;
+  if (role == GEMV_LM_HEAD && a.nseg != 1) role = GEMV_GENERIC;  // (that instantiation is one matrix too)
   if (a.attn_ws) {
-    TL_REQUIRE(a.resid && a.attn_pos && !a.norm_w && a.nseg == 1 && a.attn_hd > 0 && a.attn_hd % 4 == 0 &&
+    TL_REQUIRE(a.resid && a.attn_pos && !a.norm_w && a.nseg == 1 && a.attn_hd > 0 && a.attn_hd % 4 == 0 && (a.attn_hd & (a.attn_hd - 1)) == 0 &&
                    a.cols % a.attn_hd == 0,
                "gemv: attention-partials input needs a single residual launch without norm");
     role = GEMV_ATTN_OUT_COMBINE;
+  }
+  // Few rows of many columns: waves that only help staging x, until a thread has two pieces of it (its loads are one round trip and its
+  // values few instructions). ffn_down in us: 2048 x 5632 in 4 waves 5.4 (Q4_K / Q6_K mix), 6.2 (Q8_0), in 8 4.9 and 5.4, 11 4.65 and
+  // 5.1; 3072 x 8192 (Q6_K) in 6 7.4, in 16 7.0; 4096 x 14336 in 8 10.5, in 16 10.0.
+  // Row groups of a few spans and few of them: each span to a wave of its own, so that all loads of the launch are in flight at once (1.1B
+  // ffn_down, 3 spans, 4 -> 12 waves: Q4_K_M 4.65 -> 4.5 us, Q8_0 5.1 -> 4.95; 3B attn_output in Q6_K, 2 spans, 6 -> 12 waves: 6.45 -> 6.1; not
+  // in sixteen waves: 8B attn_output 6.5 -> 6.75; nor in parts of several spans: 8B ffn_down 10.2 -> 10.5, 3B's 6.95 either way)
+  const int spans = (a.cols / 32 + 63) / 64;
+  const int most_parts = gemv_row_waves(TL_Q4_K) / waves;
+  if ((role == GEMV_DOWN || role == GEMV_ATTN_OUT_COMBINE) && !a.peer && !a.norm_w && L.ra == 0 && ta != TL_Q8_K && total <= L.grid * waves &&
+      spans >= 2 && spans <= most_parts) {
+    L.parts = spans;
+    L.threads = spans * waves * 64;
+  }
+  if (role == GEMV_DOWN && !a.peer && L.parts <= 1) {
+    const int want = (a.cols / 4 + 127) / 128, most = want < g_max_waves ? want : g_max_waves;
+    if (most > waves) {
+      L.threads = most * 64;
+      L.wavesA = most;
+    }
   }
   *role_out = role;
   *plain = true;
@@ -1390,9 +1501,8 @@ int tl_chain_plan(const GemvArgs& a, void* task_out, size_t* lds_out, int pred_n
     t.t[i] = L.t[i];
   }
   t.a = L.v;
-  // every wave of the persistent workgroup takes part in every task (same barriers for all). A launch of its own with
-  // fewer waves has at most one row group per wave, and wave w takes the same one here (the others only help staging
-  // x); a row's sum does not depend on the wave that forms it
+  // every wave of the persistent workgroup takes part in every task (same barriers for all), whatever a launch of its own
+  // would take; a row's sum does not depend on the wave that forms it
   t.a.nthr = GEMV_MAX_THREADS;
   t.a.grid = L.grid;
   t.nsegA = L.nsegA;
@@ -1460,7 +1570,7 @@ extern "C" int tl_debug_gemv_stamps(const tl_qweight* w, const float* x_dev, flo
   for (int i = 0; i < 3; ++i) L.seg[i] = GemvSeg{qw_view(w), y_dev};
   L.t[0] = (w->rows + 1) / 2;
   L.nsegA = 1;
-  L.wavesA = gemv_geometry(L, L.t[0]);
+  L.wavesA = gemv_geometry(L, L.t[0], g_max_waves);
   TL_HIP(hipMemsetAsync(stamps_dev, 0, sizeof(unsigned long long) * 10 * (size_t)L.grid * (L.threads / 64), s));
   if (w->type == TL_Q4_K) TL_TRY((gemv_launch_one<TL_Q4_K, TL_NONE, false, GEMV_GENERIC, true>(L, s)));
   else TL_TRY((gemv_launch_one<TL_Q6_K, TL_NONE, false, GEMV_GENERIC, true>(L, s)));
@@ -1696,7 +1806,7 @@ __global__ __launch_bounds__(NV <= 2 ? GEMV_MAX_THREADS : GEMV_MAX_THREADS / 2) 
   QW wa = g.w0, wb = PAIR ? g.w1 : g.w0;
   int ra = 0, rb = 0;
   float* out = g.o0;
-  group_of<PAIR>(g, irg, wa, wb, ra, rb, out);
+  group_of<PAIR, false>(g, irg, wa, wb, ra, rb, out);
   float acc[2 * NV];
 #pragma unroll
   for (int k = 0; k < 2 * NV; ++k) acc[k] = 0.f;
@@ -1721,7 +1831,7 @@ __global__ __launch_bounds__(NV <= 2 ? GEMV_MAX_THREADS : GEMV_MAX_THREADS / 2) 
     if (++isp == nspans) {
       isp = 0;
       irg += stride;
-      if (irg < total) group_of<PAIR>(g, irg, wa, wb, ra, rb, out);
+      if (irg < total) group_of<PAIR, false>(g, irg, wa, wb, ra, rb, out);
     }
   };
   auto consume = [&](const StepNv<TYPE, NV>& st, const StepMeta& m) {
@@ -1834,7 +1944,7 @@ int tl_launch_gemv_nv(const GemvArgs& a, int nv, hipStream_t s) {
       L.t[i] = a.pair ? sg.w.rows : (sg.w.rows + 1) / 2;
       if (i < a.nseg && !(a.pair && i > 0)) total += L.t[i];
     }
-    gemv_geometry(L, total);
+    gemv_geometry(L, total, g_max_waves);
     if (nvt > 2 && L.threads > GEMV_MAX_THREADS / 2) L.threads = GEMV_MAX_THREADS / 2;
     const NvVec vec = {a.x + (size_t)v0 * a.cols, a.norm_w, a.resid ? a.resid + (size_t)v0 * a.seg[0].w.rows : nullptr,
                        a.eps, a.cols, n};

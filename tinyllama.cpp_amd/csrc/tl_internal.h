@@ -180,10 +180,10 @@ constexpr int TL_ATTN_MAX_SPLITS = 32;
 // positions per split for a sequence of `len` positions: max(64, pow2ceil(len / 32)) -> at most 32 splits. 64 rows are
 // two row slots per wave of the split kernel, the smallest unit it issues anyway; 32-row splits only doubled the records
 // the consumer has to combine (len 500: attention + attn_output 22.8 -> 20.3 us per layer).
-__host__ __device__ inline int tl_attn_split_len(int len) {
-  int sl = 64;
-  while (sl * TL_ATTN_MAX_SPLITS < len) sl <<= 1;
-  return sl;
+// (its logarithm: the splits that hold positions follow by a shift)
+__host__ __device__ inline int tl_attn_split_shift(int len) {
+  const int s = len > 1 ? 32 - __builtin_clz((unsigned)len - 1u) - 5 : 0;  // 32 splits: pow2ceil(len) / 32
+  return s > 6 ? s : 6;
 }
 // Number of splits from which the split kernel merges its own partials (the last workgroup of a head group to finish
 // does it, when AttnArgs::done_cnt is set) instead of leaving `active` records per head to the consumer: the attn_output
@@ -192,8 +192,7 @@ __host__ __device__ inline int tl_attn_split_len(int len) {
 constexpr int TL_ATTN_MERGE_MIN = 17;
 // records per head the consumer of the partials has to combine for a sequence of `len` positions
 __host__ __device__ inline int tl_attn_records(int len, bool merged) {
-  const int sl = tl_attn_split_len(len);
-  const int active = (len + sl - 1) / sl;
+  const int sh = tl_attn_split_shift(len), active = (len + (1 << sh) - 1) >> sh;
   return merged && active >= TL_ATTN_MERGE_MIN ? 1 : active;
 }
 struct AttnArgs {
