@@ -651,3 +651,23 @@ def test_projections_and_router_rows_of_every_length(env, heads, dim, width):
     got = np.concatenate([m.prefill_rows(toks[:5], 0), m.prefill_rows(toks[5:37], 5), np.stack([m.decode(int(toks[i]), i)[0] for i in (37, 38, 39)])])
     assert rel_rms(got, want) < FP32_TOL
     m.free()
+
+
+@pytest.mark.parametrize("width,heads,n_layers", [(1024, 5, 1), (1024, 16, 2), (2048, 9, 3), (4096, 40, 4), (1536, 4, 3)])
+def test_residual_sum_in_front_of_the_next_product(env, width, heads, n_layers):
+    """One token's residual norm carried by the next layer's product, at every width that takes it and one that does not: none to three
+    moves of the residual row (a layer without feed-forward among them), few rows and more rows than waves, single tokens from the captured
+    step and as a portion of one, both against the float64 oracle and against the launches of their own."""
+    S = env["synth"]
+    L = S.stack_layer
+    layers = [L(heads, 1, 64, 32, 50, v_mix=True, experts=4, top=2, ff=64, shared_ff=32, mlp=l != 1) for l in range(n_layers)]
+    cfg = S.stack_config(width, 211, layers)
+    toks = np.random.default_rng(width).integers(0, cfg["vocab"], 30).astype(np.int32)
+    got = []
+    for fuse in (1, 0):
+        m, _, orc = make(env, cfg, seed=9, max_pos=64, TL_STACK_FUSE_RESID=fuse)
+        got.append(np.concatenate([m.prefill_rows(toks[:20], 0), np.stack([m.decode(int(toks[i]), i)[0] for i in range(20, 25)]),
+                                   m.prefill_rows(toks[25:26], 25), np.stack([m.decode(int(toks[i]), i)[0] for i in range(26, 30)])]))
+        assert rel_rms(got[-1], orc.forward(list(toks))) < FP32_TOL
+        m.free()
+    assert rel_rms(got[0], got[1]) < FP32_TOL

@@ -198,6 +198,10 @@ struct ResidNormArgs {
   RouterArgs route;
 };
 int tl_launch_resid_norm(const ResidNormArgs& a, hipStream_t s);
+// one token: x_out = x + y / rms(y) * (1 + norm_w) and out = W x_out in one launch (tl_dense.hip); x_out is not x
+bool tl_dense_gemv_resid_fits(const uint16_t* w, int rows, int cols);
+int tl_launch_dense_gemv_resid(const uint16_t* w, int rows, int cols, const float* x, const float* y, const float* norm_w, float eps, float* x_out,
+                               float* out, hipStream_t s);
 // pre-norm blocks with an RMS norm: x[t] += a_scale a[t] + b_scale b[t] + sum_j slot_w[j] slots[j]; then, when w is set,
 // h[t] = x[t] / sqrt(mean(x[t]^2) + eps) * w (one_plus: * (1 + w)): the norm in front of the sublayer that reads x next
 struct ResidRmsArgs {

@@ -153,6 +153,7 @@ struct TlStack {
   int exact_items = 0;      // ... of the forward call that is being enqueued
   bool gemv_decode = true;
   bool fuse_router = true;  // TL_STACK_FUSE_ROUTER=0: the router as a launch of its own (A/B, tests)
+  bool fuse_resid = true;   // TL_STACK_FUSE_RESID=0: one token's residual norms as launches of their own (A/B, tests)
   bool fuse_steps = true;   // TL_STACK_FUSE_STEPS=0: one token of a recurrence in as many launches as a chunk takes (A/B, tests)
   bool fuse_canon = true;   // TL_STACK_FUSE_CANON=0: the convolution on what a sublayer reads as a launch of its own also for one token
   // One token through a parallel block: mixer and feed-forward read the same h and meet only in the residual sum, so the
@@ -162,7 +163,9 @@ struct TlStack {
   hipStream_t side = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   // workspaces for one chunk
-  float *x = nullptr, *qkv = nullptr, *att = nullptr, *proj = nullptr, *v_first = nullptr, *xn = nullptr;
+  float *x = nullptr, *x_main = nullptr, *x_next = nullptr;  // the residual stream; one token's may change to a row of its own and back
+  const float* late_norm = nullptr;  // the norm weights of a residual sum that the next layer's first product carries (its addend: proj)
+  float *qkv = nullptr, *att = nullptr, *proj = nullptr, *v_first = nullptr, *xn = nullptr;
   float* att_side = nullptr;                // one token of a pair's second mixer on the second stream
   float *att2 = nullptr, *proj2 = nullptr;  // the second score map of differential attention; the second mixer of a pair
   float* hn = nullptr;      // the norm of x before the convolution on what a sublayer reads
@@ -787,6 +790,7 @@ int tl_stack_create(const tl_stack_config* cfg, TlStack** out) {
   st->need_globals = 1 | 2 | 8 | (cfg->embed_norm ? 4 : 0) | (cfg->norm == TL_NORM_DYT ? 16 | 32 : 0) |
                      (cfg->norm == TL_NORM_LAYER ? 16 | (cfg->embed_norm ? 64 : 0) : 0);
   if (const char* e = getenv("TL_STACK_GEMV")) st->gemv_decode = atoi(e) != 0;
+  if (const char* e = getenv("TL_STACK_FUSE_RESID")) st->fuse_resid = atoi(e) != 0;
   if (const char* e = getenv("TL_STACK_FUSE_ROUTER")) st->fuse_router = atoi(e) != 0;
   if (const char* e = getenv("TL_STACK_FORK")) st->fork = atoi(e) != 0;
   if (const char* e = getenv("TL_STACK_FUSE_STEPS")) st->fuse_steps = atoi(e) != 0;
@@ -1162,7 +1166,9 @@ int tl_stack_finalize(TlStack* st, hipStream_t s) {
   if (st->cfg.canon_taps > 0) TL_TRY(dev_alloc(st, &st->hn, C * W));
   if (st->cfg.streams > 0) TL_TRY(dev_alloc(st, &st->xs, C * W * st->cfg.streams));
   if (st->max_gram) TL_TRY(dev_alloc(st, &st->gram, st->max_gram));
-  TL_TRY(dev_alloc(st, &st->x, C * W));
+  TL_TRY(dev_alloc(st, &st->x_main, C * W));
+  TL_TRY(dev_alloc(st, &st->x_next, W));
+  st->x = st->x_main;
   TL_TRY(dev_alloc(st, &st->h, C * W));
   if (st->layers[0].sp.block == TL_BLOCK_PARALLEL_NORMS) TL_TRY(dev_alloc(st, &st->h2, C * W));
   TL_TRY(dev_alloc(st, &st->qkv, C * st->max_qkv));
@@ -1430,6 +1436,13 @@ int project_act(TlStack* st, const uint16_t* w, int rows, int cols, const float*
 // with the biases of its columns and the activation of a constant-decay mixer's
 int first_product(TlStack* st, const Layer& L, const Layer& Wt, const float* in, int T, hipStream_t s) {
   const int W = st->cfg.width, rows = L.pd + (L.side ? L.side->pd : 0);
+  if (st->late_norm) {  // (late_product said so: one plain matrix on x, in front of which the residual sum of the layer before is still to come)
+    const float* nw = st->late_norm;
+    st->late_norm = nullptr;
+    TL_TRY(tl_launch_dense_gemv_resid(Wt.wqkv, rows, W, st->x, st->proj, nw, st->cfg.norm_eps, st->x_next, st->qkv, s));
+    std::swap(st->x, st->x_next);
+    return 0;
+  }
   GemvActArgs act = {};
   act.bias = Wt.prod_b;
   if (L.sp.mixer == TL_MIXER_LIGHTNING) {
@@ -1558,8 +1571,16 @@ RouterArgs router_args(TlStack* st, const Layer& L, const Layer& Wt, const float
   return r;
 }
 
+// A post-norm block whose last residual sum the first product of the block behind it can carry (one token)
+bool late_product(const TlStack* st, size_t li, int T) {
+  if (T != 1 || !st->gemv_decode || !st->fuse_resid || st->hook || li + 1 >= st->layers.size()) return false;
+  const Layer &L = st->layers[li], &N = st->layers[li + 1];
+  auto post = [](const Layer& l) { return l.sp.block != TL_BLOCK_PARALLEL && l.sp.block != TL_BLOCK_PARALLEL_NORMS && l.sp.block != TL_BLOCK_PRE_NORM; };
+  const Layer& Wn = st->layers[N.wsrc];
+  return post(L) && post(N) && N.sp.mixer == TL_MIXER_SWA && !N.side && !Wn.prod_b && tl_dense_gemv_resid_fits(Wn.wqkv, N.pd, st->cfg.width);
+}
 // x += norm2(ff(x)) of a post-norm block
-int moe_layer(TlStack* st, Layer& L, int T, hipStream_t s) {
+int moe_layer(TlStack* st, Layer& L, int T, hipStream_t s, bool late) {
   const tl_layer_spec& sp = L.sp;
   const Layer& Wt = st->layers[L.wsrc];
   const int W = st->cfg.width;
@@ -1573,6 +1594,10 @@ int moe_layer(TlStack* st, Layer& L, int T, hipStream_t s) {
   n.eps = st->cfg.norm_eps;
   TL_REQUIRE(!sp.shared_gate, "layer-list engine: a gated shared expert runs in parallel blocks only");
   TL_TRY(moe_experts(st, L, Wt, st->x, T, st->proj, s));
+  if (late) {
+    st->late_norm = Wt.norm2;
+    return 0;
+  }
   if (T == 1 && st->gemv_decode) {
     n.a = st->proj;
     return tl_launch_resid_norm(n, s);
@@ -2557,6 +2582,13 @@ int tl_stack_forward(TlStack* st, const int* tokens_dev, int T, int start_pos, c
   const int W = c.width;
   const bool dyt = c.norm == TL_NORM_DYT, lnorm = c.norm == TL_NORM_LAYER || c.norm == TL_NORM_LAYER_PLAIN;
   st->exact_items = !pos_dev && start_pos == 0 ? st->exact_first : 0;
+  // every late residual sum moves the stream to the other buffer: it starts where it will end in x_main
+  float* const row = st->x == st->x_main ? st->x_next : st->x;
+  size_t moves = 0;
+  for (size_t li = 0; li < st->layers.size(); ++li) moves += late_product(st, li, T);
+  st->late_norm = nullptr;
+  st->x = moves & 1 ? row : st->x_main;
+  st->x_next = moves & 1 ? st->x_main : row;
   if (lnorm && !c.embed_norm) {
     HyperArgs r = {};  // every stream starts as the (scaled) embedding row
     hyper_next(st, r, &st->layers[0], 1, T, nullptr);
@@ -2608,8 +2640,10 @@ int tl_stack_forward(TlStack* st, const int* tokens_dev, int T, int start_pos, c
         n.route.ids = st->ids;
         n.route.wts = st->wts;
       }
-      TL_TRY(tl_launch_resid_norm(n, s));
-      if (sp.mlp == TL_MLP_MOE) TL_TRY(moe_layer(st, L, T, s));
+      const bool late = late_product(st, li, T);
+      if (late && sp.mlp != TL_MLP_MOE) st->late_norm = n.w;
+      else TL_TRY(tl_launch_resid_norm(n, s));
+      if (sp.mlp == TL_MLP_MOE) TL_TRY(moe_layer(st, L, T, s, late));
     }
     if (st->hook) {
       TL_HIP(hipStreamSynchronize(s));
