@@ -194,10 +194,30 @@ __device__ __forceinline__ f16x8 q8_operand(unsigned a, unsigned b) {
               as_h2(pick(y, 0x00FF00FFu)) - off, as_h2(pick(y >> 8, 0x00FF00FFu)) - off);
 }
 
-struct HSegs {  // up to three matrices over the same activations (q | k | v, gate | up): row tiles follow each other
+// v / d of 31-bit v by one multiplication: m = floor(2^(31 + l) / d) + 1 with l = ceil(log2 d) fits 32 bits, and v m / 2^(31 + l) exceeds v / d
+// by less than 1 / d
+struct Div {
+  unsigned m, l;
+  static Div by(unsigned d) {
+    unsigned l = 0;
+    while ((1ull << l) < d) ++l;
+    return Div{(unsigned)((1ull << (31 + l)) / d + 1), l};
+  }
+  __device__ __forceinline__ int of(int v) const { return (int)(__umulhi(2u * (unsigned)v, m) >> l); }
+};
+// A launch: up to three matrices over the same activations (q | k | v, gate | up), whose row tiles follow each other, and the grid's
+// division into slices, panels and tiles. What every workgroup would otherwise work out for itself is worked out here: in a launch of few
+// tokens the instructions in front of the first load are a part of its time (eight tokens in Q4_K: 313 and six waits for arguments, each
+// asked for when the one before had come; now 161 and three. 0.4 us of 7: steps of 8 sequences over 28 layers of 3072 1.86 -> 1.80 ms)
+struct HSegs {
+  int T, K, nsb, per;                          // tokens, columns, super-blocks of a row and of a slice
+  int per8, rem8, slice_tiles, panel_tiles;    // workgroups of an XCD (and how many XCDs have one more), of a slice, of a panel
+  Div by_slice, by_panel, by_width, by_last;   // ... and divisions by the tiles of a slice and of a panel, and by the token tiles of a panel and of the last one
+  int panel, width_last, last_panel, mt_end[2];
+  const float* resid;
+  HAct act;
   QW w[3];
   float* y[3];
-  int mt_end[3];
 };
 
 // Which tile a workgroup computes.
@@ -209,22 +229,21 @@ struct HSegs {  // up to three matrices over the same activations (q | k | v, ga
 struct Place {
   int slice, nt, mt, seg;
 };
-__device__ __forceinline__ Place place_of(const HSegs& segs, int mtiles, int ntiles, int nslices, int panel) {
-  const int total = mtiles * ntiles * nslices, per8 = total >> 3, rem8 = total & 7;
+__device__ __forceinline__ Place place_of(const HSegs& g) {
   const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
-  const int v = xcd * per8 + (xcd < rem8 ? xcd : rem8) + at;
+  const int v = xcd * g.per8 + (xcd < g.rem8 ? xcd : g.rem8) + at;
   Place p;
-  p.slice = v / (mtiles * ntiles);
-  const int in_slice = v - p.slice * mtiles * ntiles;
-  p.nt = 0, p.mt = in_slice;
-  if (ntiles > 1) {  // (one tile of tokens: launches of 6 us, which need none of these divisions)
-    const int pi = in_slice / (panel * mtiles), in_panel = in_slice - pi * panel * mtiles;
-    const int width = ntiles - panel * pi < panel ? ntiles - panel * pi : panel;
-    p.mt = in_panel / width;
-    p.nt = panel * pi + in_panel - p.mt * width;
-  }
-  p.seg = (p.mt >= segs.mt_end[0]) + (p.mt >= segs.mt_end[1]);
-  if (p.seg) p.mt -= segs.mt_end[p.seg - 1];
+  p.slice = g.by_slice.of(v);
+  const int in_slice = v - p.slice * g.slice_tiles, pi = g.by_panel.of(in_slice), in_panel = in_slice - pi * g.panel_tiles;
+  const bool last = pi == g.last_panel;
+  int wl = g.width_last, wp = g.panel;
+  Div dl = g.by_last, dp = g.by_width;
+  asm("" : "+s"(wl), "+s"(wp), "+s"(dl.m), "+s"(dl.l), "+s"(dp.m), "+s"(dp.l));  // (loads of both, not one whose address is chosen first)
+  const int width = last ? wl : wp;
+  p.mt = Div{last ? dl.m : dp.m, last ? dl.l : dp.l}.of(in_panel);
+  p.nt = g.panel * pi + in_panel - p.mt * width;
+  p.seg = (p.mt >= g.mt_end[0]) + (p.mt >= g.mt_end[1]);
+  p.mt -= p.seg == 0 ? 0 : p.seg == 1 ? g.mt_end[0] : g.mt_end[1];
   return p;
 }
 
@@ -318,8 +337,7 @@ __device__ __forceinline__ void store_tile(float* __restrict__ y, const float* _
 // consecutive rows of a fragment read and the 2 x 8 pieces of a staging write cover the 64 banks once; behind them the
 // super-block's block sums and powers of two.
 template <int TYPE, int TK, int NI, int MI, int NW, int WPE, bool STACK>
-__global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct act, const float* __restrict__ resid, int T, int mtiles,
-                                                           int ntiles, int nslices, int panel) {
+__global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(const HSegs segs) {
   typedef Tile<TK> TL;
   typedef typename TL::Acc Acc;
   constexpr int NG = 64 / TK, US = 8 / NG;                        // lane groups, steps of a super-block
@@ -331,15 +349,14 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
   constexpr bool CHUNKED = TYPE == TL_Q4_K || TYPE == TL_Q6_K;
   constexpr bool RINGED = BN > 32;                                // the tile goes through a ring of three 64-column steps
   extern __shared__ __attribute__((aligned(16))) _Float16 hlds[];
-  const Place pl = place_of(segs, mtiles, ntiles, nslices, panel);
-  const QW w = segs.w[pl.seg];
-  float* __restrict__ y = segs.y[pl.seg];
-  const int slice = pl.slice, nt = pl.nt, mt = pl.mt;
-  const int M = w.rows, K = w.cols;
-  const int nsb_all = (K + 255) >> 8, per = (nsb_all + nslices - 1) / nslices;
-  const int sb0 = slice * per, nsb = nsb_all - sb0 < per ? nsb_all - sb0 : per;
-  const int slast = K / 64 - 1;
-  if (nslices > 1) y += (size_t)slice * (size_t)T * (size_t)M;
+  const Place pl = place_of(segs);
+  QW w = segs.w[pl.seg];
+  const HAct act = segs.act;
+  const int nt = pl.nt, mt = pl.mt, T = segs.T;
+  const int M = w.rows, K = segs.K;
+  w.cols = K;  // (known before the matrix is)
+  const int sb0 = pl.slice * segs.per, nsb = segs.nsb - sb0 < segs.per ? segs.nsb - sb0 : segs.per;
+  const int slast = (K >> 6) - 1;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int fr = lane & (TK - 1), fg = lane / TK;
   const int n0 = nt * BN, m0 = mt * (TK * MI * NW) + wave * (TK * MI);
@@ -365,9 +382,10 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
   // 16-byte pieces of a super-block's block sums (2 BN) and powers of two (BN / 4); spare threads copy a piece again
   constexpr int AUX = 2 * BN + BN / 4;
   const int ap = tid % AUX;
-  const unsigned char* ag = ap < 2 * BN ? reinterpret_cast<const unsigned char*>(act.bs + (size_t)n0 * 16) + ap * 16
-                                        : reinterpret_cast<const unsigned char*>(act.inv + n0) + (ap - 2 * BN) * 16;
-  const size_t astride = (size_t)act.tpad * (ap < 2 * BN ? 32 : 4);
+  const unsigned char* const abase = reinterpret_cast<const unsigned char*>(act.bs);  // (the powers of two lie ps / 8 bytes behind)
+  const unsigned ashift = ap < 2 * BN ? 5u : 2u;
+  const unsigned ag = ((unsigned)n0 << ashift) + (unsigned)ap * 16u + (ap < 2 * BN ? 0u : (unsigned)(act.ps >> 3) - 32u * BN);
+  const unsigned astride = (unsigned)act.tpad << ashift;
   // fragment reads: where the lane's eight columns of operand k lie in a step's part of the tile
   int xo[4];
 #pragma unroll
@@ -384,7 +402,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
 #pragma unroll
   for (int i = 0; i < MI; ++i) load_head<TYPE>(H[i], w, R[i], sb0);
   {
-    const u32x4 aux = *reinterpret_cast<const u32x4*>(ag + (size_t)sb0 * astride);
+    const u32x4 aux = *reinterpret_cast<const u32x4*>(abase + (ag + (unsigned)sb0 * astride));
     constexpr int FIRST = RINGED ? 2 : 1;
     f16x8 xr[FIRST][XR];
 #pragma unroll
@@ -421,7 +439,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
     _Float16* an = RINGED ? hlds + 3 * STEP + (cur ^ 1) * AUXH : xn + 4 * STEP;
     u32x4 aux;
     if (NEXT) {
-      aux = *reinterpret_cast<const u32x4*>(ag + (size_t)(sb + 1) * astride);
+      aux = *reinterpret_cast<const u32x4*>(abase + (ag + (unsigned)(sb + 1) * astride));
 #pragma unroll
       for (int i = 0; i < MI; ++i) load_head<TYPE>(Hn[i], w, R[i], sb + 1);
     }
@@ -558,7 +576,8 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(HSegs segs, HAct ac
   for (int b = 0; b + 1 < nsb; ++b) superblock(b, std::true_type{});
   superblock(nsb - 1, std::false_type{});
 
-  store_tile<TK, NI, MI, STACK>(y, resid, acc, n0, m0, T, M, fr, fg);
+  float* const y = segs.y[pl.seg] + (size_t)pl.slice * (size_t)T * (size_t)M;  // (slices beyond the first only where there are several)
+  store_tile<TK, NI, MI, STACK>(y, segs.resid, acc, n0, m0, T, M, fr, fg);
 }
 
 // The same product in workgroups of eight waves and 64 tokens, one on a CU, rows in whole super-blocks: activations and weights go from
@@ -585,8 +604,7 @@ struct LdsMap {
   static constexpr int BYTES = A + 2 * ASLOT;
 };
 template <int TYPE, int MI, int NW>
-__global__ __launch_bounds__(64 * NW, 2) void hgemm_lds_kernel(HSegs segs, HAct act, const float* __restrict__ resid, int T, int mtiles,
-                                                             int ntiles, int nslices, int panel) {
+__global__ __launch_bounds__(64 * NW, 2) void hgemm_lds_kernel(const HSegs segs) {
   typedef LdsMap<TYPE, MI, NW> L;
   typedef Tile<32> TL;
   typedef f32x16 Acc;
@@ -595,13 +613,12 @@ __global__ __launch_bounds__(64 * NW, 2) void hgemm_lds_kernel(HSegs segs, HAct 
   static_assert(NW == 8 && (MI == 1 || MI == 2), "");
   extern __shared__ __attribute__((aligned(16))) _Float16 hlds[];
   unsigned char* const lds = reinterpret_cast<unsigned char*>(hlds);
-  const Place pl = place_of(segs, mtiles, ntiles, nslices, panel);
+  const Place pl = place_of(segs);
   const QW w = segs.w[pl.seg];
-  float* __restrict__ y = segs.y[pl.seg];
-  const int M = w.rows, K = w.cols;
-  const int nsb_all = K >> 8, per = (nsb_all + nslices - 1) / nslices;
-  const int sb0 = __builtin_amdgcn_readfirstlane(pl.slice * per), nsb = nsb_all - sb0 < per ? nsb_all - sb0 : per;
-  if (nslices > 1) y += (size_t)pl.slice * (size_t)T * (size_t)M;
+  const HAct act = segs.act;
+  const int M = w.rows, K = segs.K, T = segs.T;
+  const int nsb_all = segs.nsb;
+  const int sb0 = __builtin_amdgcn_readfirstlane(pl.slice * segs.per), nsb = nsb_all - sb0 < segs.per ? nsb_all - sb0 : segs.per;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 31, fg = lane >> 5;
   const int n0 = pl.nt * BN, tile0 = pl.mt * BM, m0 = tile0 + wave * 32 * MI;
@@ -841,7 +858,8 @@ __global__ __launch_bounds__(64 * NW, 2) void hgemm_lds_kernel(HSegs segs, HAct 
   };
   for (int b = 0; b + 1 < nsb; ++b) superblock(b, std::true_type{});
   superblock(nsb - 1, std::false_type{});
-  store_tile<32, NI, MI, false>(y, resid, acc, n0, m0, T, M, fr, fg);
+  float* const y = segs.y[pl.seg] + (size_t)pl.slice * (size_t)T * (size_t)M;
+  store_tile<32, NI, MI, false>(y, segs.resid, acc, n0, m0, T, M, fr, fg);
 }
 
 // ---- producer of the activation planes ----------------------------------------------------------------------------------
@@ -1068,27 +1086,44 @@ HgemmPlan hgemm_plan(const QW* w, int n, int T) {
 }
 
 template <int TYPE, int V>
-int hgemm_go(const HSegs& g, int mt, const HAct& act, const float* resid, int T, int S, hipStream_t s) {
+int hgemm_go(HSegs& g, int mt, int S, hipStream_t s) {
   constexpr HShape q = hgemm_shape(TYPE, V);
   constexpr int BN = hgemm_tokens(q);
   constexpr size_t lds = q.lds ? (size_t)LdsMap<TYPE, q.mi, q.nw>::BYTES
                                : (size_t)(BN > 32 ? 3 * 2 * 64 + 2 * 18 : 2 * (4 * 2 * 64 + 18)) * BN * sizeof(_Float16);
   static_assert(q.percu * lds <= 160 * 1024, "hgemm_price counts on `percu` workgroups on a CU");
   static TlDeviceOnce lds_raised;
-  void (*kernel)(HSegs, HAct, const float*, int, int, int, int, int);
+  void (*kernel)(HSegs);
   if constexpr (q.lds) kernel = hgemm_lds_kernel<TYPE, q.mi, q.nw>;
   else kernel = hgemm_kernel<TYPE, q.tk, q.ni, q.mi, q.nw, q.wpe, q.stack>;
   TL_TRY(tl_raise_lds_limit(kernel, (int)lds, lds_raised));
   // panels of eight token tiles and more, all alike: a panel of the one tile that is left over reads all weights again for it (28672 x
   // 4096 in Q4_K times 513 tokens, nine tiles, 274 us in one panel of shape 3 with 256 rows, 281 in eight and one)
-  const int ntiles = (T + BN - 1) / BN, panels = ntiles < 16 ? 1 : ntiles / 8, panel = (ntiles + panels - 1) / panels;
-  kernel<<<dim3((unsigned)(mt * ntiles * S)), dim3(64 * q.nw), lds, s>>>(g, act, resid, T, mt, ntiles, S, panel);
+  const int ntiles = (g.T + BN - 1) / BN, panels = ntiles < 16 ? 1 : ntiles / 8, panel = (ntiles + panels - 1) / panels;
+  g.per = (g.nsb + S - 1) / S;
+  g.per8 = mt * ntiles * S / 8;
+  g.rem8 = mt * ntiles * S % 8;
+  g.slice_tiles = mt * ntiles;
+  g.panel = panel;
+  g.panel_tiles = panel * mt;
+  g.last_panel = (ntiles - 1) / panel;
+  g.width_last = ntiles - g.last_panel * panel;
+  g.by_slice = Div::by(g.slice_tiles);
+  g.by_panel = Div::by(g.panel_tiles);
+  g.by_width = Div::by(panel);
+  g.by_last = Div::by(g.width_last);
+  kernel<<<dim3((unsigned)(mt * ntiles * S)), dim3(64 * q.nw), lds, s>>>(g);
   TL_HIP(hipGetLastError());
   return 0;
 }
 template <int TYPE>
 int hgemm_typed(const QW* w, int n, const HgemmPlan& p, const HAct& act, float* const* out, const float* resid, int T, hipStream_t s) {
   HSegs g = {};
+  g.T = T;
+  g.K = w[0].cols;
+  g.nsb = (w[0].cols + 255) / 256;
+  g.resid = resid;
+  g.act = act;
   int mt = 0;
   const int shape = p.shape == 2 && w[0].cols % 256 ? 4 : p.shape;  // (rows that end inside a super-block: shape 4's kernel has the same sums)
   const int bm = hgemm_shape(TYPE, shape).tk * hgemm_shape(TYPE, shape).mi * hgemm_shape(TYPE, shape).nw;
@@ -1097,18 +1132,18 @@ int hgemm_typed(const QW* w, int n, const HgemmPlan& p, const HAct& act, float* 
     g.w[i] = w[k];
     g.y[i] = out[k];
     if (i < n) mt += (w[i].rows + bm - 1) / bm;
-    g.mt_end[i] = mt;
+    if (i < 2) g.mt_end[i] = mt;
   }
-  if (shape == 0) return hgemm_go<TYPE, 0>(g, mt, act, resid, T, p.S, s);
-  if (shape == 1) return hgemm_go<TYPE, 1>(g, mt, act, resid, T, p.S, s);
-  if (shape == 2) return hgemm_go<TYPE, 2>(g, mt, act, resid, T, p.S, s);
+  if (shape == 0) return hgemm_go<TYPE, 0>(g, mt, p.S, s);
+  if (shape == 1) return hgemm_go<TYPE, 1>(g, mt, p.S, s);
+  if (shape == 2) return hgemm_go<TYPE, 2>(g, mt, p.S, s);
   if constexpr (TYPE == TL_Q4_K || TYPE == TL_Q8_K)
-    if (shape == 3) return hgemm_go<TYPE, 3>(g, mt, act, resid, T, p.S, s);
-  if (shape == 5) return hgemm_go<TYPE, 5>(g, mt, act, resid, T, p.S, s);
-  if (shape == 6) return hgemm_go<TYPE, 6>(g, mt, act, resid, T, p.S, s);
-  if (shape == 7) return hgemm_go<TYPE, 7>(g, mt, act, resid, T, p.S, s);
-  if (shape == 8) return hgemm_go<TYPE, 8>(g, mt, act, resid, T, p.S, s);
-  return hgemm_go<TYPE, 4>(g, mt, act, resid, T, p.S, s);
+    if (shape == 3) return hgemm_go<TYPE, 3>(g, mt, p.S, s);
+  if (shape == 5) return hgemm_go<TYPE, 5>(g, mt, p.S, s);
+  if (shape == 6) return hgemm_go<TYPE, 6>(g, mt, p.S, s);
+  if (shape == 7) return hgemm_go<TYPE, 7>(g, mt, p.S, s);
+  if (shape == 8) return hgemm_go<TYPE, 8>(g, mt, p.S, s);
+  return hgemm_go<TYPE, 4>(g, mt, p.S, s);
 }
 
 }  // namespace
