@@ -383,6 +383,29 @@ def test_merged_and_separate_launches_round_alike(pkg, monkeypatch, mix, n):
     assert np.array_equal(got[0], got[1]), np.abs(got[0].astype(np.float64) - got[1]).max()
 
 
+@pytest.mark.parametrize("heads,kv", [(8, 4), (4, 4)])
+def test_two_formats_in_one_launch(pkg, monkeypatch, heads, kv):
+    """q | k in Q4_K and v in Q6_K share a launch, in every workgroup shape (tokens around 8, 16, 32 and 64, and so many that waves take 64
+    rows), with rows that end inside a tile and K slices: the same bits as a launch of each with the shared launch's shapes and slices
+    (TL_GEMM_MERGE=0), whose products are held against float64 elsewhere."""
+    from tinyllama_cpp_amd import engine as E
+    E.init(0)
+    cfg, tensors = pkg.synth.build_model(dict(hidden=heads * 128, inter=512, n_heads=heads, n_kv_heads=kv, n_layers=1, vocab=64, max_pos=2048, eps=1e-5,
+                                              rope_theta=10000.0), "q4_k_m", seed=16)
+    assert [tensors["blk.0.attn_%s.weight" % n][0] for n in "qkv"] == [pkg.synth.Q4_K, pkg.synth.Q4_K, pkg.synth.Q6_K]
+    m = E.Model(cfg).load(tensors)
+    rng = np.random.default_rng(heads)
+    for n in (1, 8, 9, 16, 17, 31, 33, 64, 65, 130, 520, 1999):
+        toks = rng.integers(0, cfg["vocab"], n).astype(np.int32)
+        got = []
+        for merge in ("0", "1"):
+            monkeypatch.setenv("TL_GEMM_MERGE", merge)
+            m.reset_kv()
+            got.append(np.array(m.prefill(toks, 0, all_logits=True)[1]))
+        assert np.array_equal(got[0], got[1]), (n, np.abs(got[0].astype(np.float64) - got[1]).max())
+    m.free()
+
+
 def test_packed_prompts_longer_than_a_sequence(pkg):
     """A packed batch of more tokens than a sequence has positions goes through as one chunk: every prompt's last logits are those
     of its own prefill, up to the order of 32-bit sums (2^-22 a layer and product)."""

@@ -1723,7 +1723,7 @@ static int launch_gemm_dispatch(const QW& w, const __bf16* xp, size_t plane_stri
 }
 
 // Up to three matrices over the same activation planes (q | k | v, gate | up) in one launch of the f16 kernel or of the
-// integer-plane kernel. All matrices of one format and width. The integer-plane kernel: taken only when that changes no bit, with
+// integer-plane kernel. All matrices of one width and format (or, in the f16 form, two in Q4_K and a third in Q6_K). The integer-plane kernel: taken only when that changes no bit, with
 // the number of K slices that each matrix's own launch would use. The f16 kernel: the shape and slices are the group's, also where
 // its matrices have to be launched one after another, so the sums do not depend on whether they could be merged. Outputs: with one
 // slice y[i] directly; with more, the partial tiles go to defer[i] (required) for the consumer to sum. *merged = false: nothing was
@@ -1738,14 +1738,21 @@ int tl_launch_gemm_q_multi(const QW* w, int n, const void* planes, size_t plane_
   if (n < 2 || n > 3 || T <= 0 || terms == 1) return 0;
   const bool half = terms == TL_TERMS_HALF;
   if (!half && q && atoi(q) == 0) return 0;
-  for (int i = 0; i < n; ++i)
+  // two matrices in Q4_K and a third in Q6_K: plans of their own for one launch, where that is the better price
+  HgemmPlan plan4 = {}, plan6 = {};
+  const bool pair = half && n == 3 && w[1].type == w[0].type && w[2].type != w[0].type &&
+                    tl_hgemm_pair_plan(w, 2, w[2], T, ksplit_enabled() ? 8 : 1, &plan4, &plan6);
+  for (int i = 0; i < n && !pair; ++i)
     if (w[i].type != w[0].type || w[i].cols != w[0].cols || w[i].cols % 64 != 0 || w[i].rows <= 0) return 0;
   if (!half && (!on || (bm && atoi(bm) == 64))) return 0;  // (the merged integer-plane launch exists for 128-row tiles only)
   const int BN = (T <= 64 || qi_narrow_always()) ? 64 : GB_N;
   const int ntiles = (T + BN - 1) / BN;
   int S[3] = {1, 1, 1};
   HgemmPlan plan = {0, 1};
-  if (half) {  // one shape and slice count for the group, from the tiles of the whole launch
+  if (pair) {
+    S[0] = S[1] = plan4.S;
+    S[2] = plan6.S;
+  } else if (half) {  // one shape and slice count for the group, from the tiles of the whole launch
     plan = half_plan(w, n, T);
     S[0] = S[1] = S[2] = plan.S;
   } else {     // K slices of every matrix as its own launch would choose them
@@ -1769,7 +1776,7 @@ int tl_launch_gemm_q_multi(const QW* w, int n, const void* planes, size_t plane_
     if (!half) return 0;  // (integer-plane route: every matrix keeps its own slice count, the caller's launches are the same)
     // the f16 form one matrix at a time, with the group's shape and slices: the same sums as the merged launch
     for (int i = 0; i < n; ++i) {
-      t_group_plan = plan;
+      t_group_plan = !pair ? plan : i < 2 ? plan4 : plan6;
       const int rc1 = tl_launch_gemm_q(w[i], planes, plane_stride, y[i], nullptr, T, terms, s, defer ? defer[i] : nullptr);
       t_group_plan = {0, 0};
       if (rc1) return rc1;
@@ -1780,7 +1787,8 @@ int tl_launch_gemm_q_multi(const QW* w, int n, const void* planes, size_t plane_
   const __bf16* xp = static_cast<const __bf16*>(planes);
   int rc = 0;
   if (half) {
-    TL_TRY(tl_launch_hgemm(w, n, planes, plane_stride, out, nullptr, T, plan, s));
+    if (pair) TL_TRY(tl_launch_hgemm_pair(w, 2, w[2], planes, plane_stride, out, out[2], T, plan4, plan6, s));
+    else TL_TRY(tl_launch_hgemm(w, n, planes, plane_stride, out, nullptr, T, plan, s));
     for (int i = 0; i < n; ++i)
       if (defer && defer[i]) defer[i]->got = S[i] > 1 ? GemmParts{out[i], (size_t)T * w[i].rows, S[i]} : GemmParts{nullptr, 0, 0};
     *merged = true;

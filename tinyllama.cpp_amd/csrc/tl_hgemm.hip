@@ -15,7 +15,7 @@
 //     the eight sub-block sums' two f16 parts side by side along K and the same eight m_j against either half.
 // hgemm_kernel (tiles of up to 128 rows, Q8_K 256): weights go from HBM straight into registers (a super-block ahead), are unpacked
 // there and never touch LDS; the activation tile is staged through LDS, up to 32 tokens a super-block ahead with one barrier
-// per super-block, 64 tokens in a ring of three 64-column steps. hgemm_lds_kernel (256 and 512 rows): activations and
+// per super-block, 64 tokens in a ring of three 64-column steps. hgemm_lds_body (256 and 512 rows): activations and
 // weights are both copied from memory to LDS as they lie there, with a barrier per 64-column step, and unpacked behind it.
 //
 // The order of the columns inside an operand is free as long as both sides agree. Lane half h of a Q4_K / Q6_K step takes
@@ -229,8 +229,8 @@ struct HSegs {
 struct Place {
   int slice, nt, mt, seg;
 };
-__device__ __forceinline__ Place place_of(const HSegs& g) {
-  const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+__device__ __forceinline__ Place place_of(const HSegs& g, int block) {
+  const int xcd = block & 7, at = block >> 3;
   const int v = xcd * g.per8 + (xcd < g.rem8 ? xcd : g.rem8) + at;
   Place p;
   p.slice = g.by_slice.of(v);
@@ -336,8 +336,8 @@ __device__ __forceinline__ void store_tile(float* __restrict__ y, const float* _
 // columns][2 parts][tokens][64] f16, the 16-byte pieces of a token's 128 bytes at piece ^ (row / 2 & 7), row = part x tokens + token: the 16
 // consecutive rows of a fragment read and the 2 x 8 pieces of a staging write cover the 64 banks once; behind them the
 // super-block's block sums and powers of two.
-template <int TYPE, int TK, int NI, int MI, int NW, int WPE, bool STACK>
-__global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(const HSegs segs) {
+template <int TYPE, int TK, int NI, int MI, int NW, bool STACK>
+__device__ __forceinline__ void hgemm_body(const HSegs& segs, int block) {
   typedef Tile<TK> TL;
   typedef typename TL::Acc Acc;
   constexpr int NG = 64 / TK, US = 8 / NG;                        // lane groups, steps of a super-block
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void hgemm_kernel(const HSegs segs) {
   constexpr bool CHUNKED = TYPE == TL_Q4_K || TYPE == TL_Q6_K;
   constexpr bool RINGED = BN > 32;                                // the tile goes through a ring of three 64-column steps
   extern __shared__ __attribute__((aligned(16))) _Float16 hlds[];
-  const Place pl = place_of(segs);
+  const Place pl = place_of(segs, block);
   QW w = segs.w[pl.seg];
   const HAct act = segs.act;
   const int nt = pl.nt, mt = pl.mt, T = segs.T;
@@ -604,7 +604,7 @@ struct LdsMap {
   static constexpr int BYTES = A + 2 * ASLOT;
 };
 template <int TYPE, int MI, int NW>
-__global__ __launch_bounds__(64 * NW, 2) void hgemm_lds_kernel(const HSegs segs) {
+__device__ __forceinline__ void hgemm_lds_body(const HSegs& segs, int block) {
   typedef LdsMap<TYPE, MI, NW> L;
   typedef Tile<32> TL;
   typedef f32x16 Acc;
@@ -613,7 +613,7 @@ __global__ __launch_bounds__(64 * NW, 2) void hgemm_lds_kernel(const HSegs segs)
   static_assert(NW == 8 && (MI == 1 || MI == 2), "");
   extern __shared__ __attribute__((aligned(16))) _Float16 hlds[];
   unsigned char* const lds = reinterpret_cast<unsigned char*>(hlds);
-  const Place pl = place_of(segs);
+  const Place pl = place_of(segs, block);
   const QW w = segs.w[pl.seg];
   const HAct act = segs.act;
   const int M = w.rows, K = segs.K, T = segs.T;
@@ -1003,7 +1003,7 @@ __global__ __launch_bounds__(256) void hsplit_kernel(const float* __restrict__ x
 // 64: 1.52 / 2.03, 128: 2.2 / 2.7; a prompt of 512: 5.3 / 7.0.)
 struct HShape {
   int tk, ni, mi, nw, wpe, percu;
-  bool lds, stack;  // lds: hgemm_lds_kernel
+  bool lds, stack;  // lds: hgemm_lds_body
 };
 constexpr int HGEMM_SHAPES = 9;
 constexpr HShape hgemm_shape(int type, int shape) {
@@ -1015,6 +1015,38 @@ constexpr HShape hgemm_shape(int type, int shape) {
   return all[shape];
 }
 constexpr int hgemm_tokens(const HShape& q) { return q.stack ? 8 : q.tk * q.ni; }
+template <int TYPE, int V>
+constexpr size_t hgemm_lds_bytes() {
+  constexpr HShape q = hgemm_shape(TYPE, V);
+  constexpr int BN = hgemm_tokens(q);
+  constexpr size_t lds = q.lds ? (size_t)LdsMap<TYPE, q.mi, q.nw>::BYTES
+                               : (size_t)(BN > 32 ? 3 * 2 * 64 + 2 * 18 : 2 * (4 * 2 * 64 + 18)) * BN * sizeof(_Float16);
+  static_assert(q.percu * lds <= 160 * 1024, "hgemm_price counts on `percu` workgroups on a CU");
+  return lds;
+}
+template <int TYPE, int V>
+__device__ __forceinline__ void hgemm_any(const HSegs& g, int block) {
+  constexpr HShape q = hgemm_shape(TYPE, V);
+  if constexpr (q.lds) hgemm_lds_body<TYPE, q.mi, q.nw>(g, block);
+  else hgemm_body<TYPE, q.tk, q.ni, q.mi, q.nw, q.stack>(g, block);
+}
+template <int TYPE, int V>
+__global__ __launch_bounds__(64 * hgemm_shape(TYPE, V).nw, hgemm_shape(TYPE, V).wpe) void hgemm_kernel(const HSegs g) {
+  hgemm_any<TYPE, V>(g, blockIdx.x);
+}
+// Matrices of two formats over the same activations (Q4_K files hold v as Q6_K in some layers, q and k as Q4_K): the longer workgroups
+// first, and the others fill up what they leave of the chip. A launch of v's 1024 x 3072 alone is 48 workgroups and 6 us for 8 tokens. Steps of
+// 8 sequences, 3B, half of whose layers hold v so, 1.79 -> 1.74 ms; 128 sequences, 8B, 7.5 -> 7.3; whole prompts of 9 to 1900 tokens, 1.1B, 3B
+// and 8B, 0 to 4 % less.
+struct HPair {
+  HSegs q6, q4;
+  int first;  // workgroups of q6
+};
+template <int V6, int V4>
+__global__ __launch_bounds__(64 * hgemm_shape(TL_Q4_K, V4).nw, hgemm_shape(TL_Q4_K, V4).wpe) void hgemm_pair_kernel(const HPair p) {
+  if ((int)blockIdx.x < p.first) hgemm_any<TL_Q6_K, V6>(p.q6, blockIdx.x);
+  else hgemm_any<TL_Q4_K, V4>(p.q4, blockIdx.x - p.first);
+}
 // Up to 64 tokens a launch takes, in us with weights that no cache holds, its start and end (a quarter of that again for every further
 // round over the chip) and, of the CU with the most workgroups, all their super-blocks one after another: co-resident ones share the issue
 // slots and the CU's way to memory, so none of them is free. Fitted to 2048 .. 28672 rows of 2048 .. 14336 columns times 8, 16, 24, 32 and
@@ -1054,8 +1086,8 @@ float hgemm_price(int cus, int type, int shape, int T, long n, int per, int S, f
   }
   return (float)rounds * (float)(per + 1) * (shape == 3 && !q.lds ? HGEMM_US_3_Q8_K : HGEMM_US[shape]) + sums;
 }
-// the shape and the K slices of the least price
-HgemmPlan hgemm_plan(const QW* w, int n, int T) {
+// the shape and the K slices of the least price, which is added to *sum
+HgemmPlan hgemm_plan(const QW* w, int n, int T, float* sum = nullptr) {
   const int nsb = (w[0].cols + 255) / 256, type = w[0].type, cus = tl_num_cus();  // (the call asks the runtime: once a plan)
   const unsigned few = T <= 8 ? 1u << 5 | 1u << 6 : T <= 16 ? 1u << 0 | 1u << 7 : 1u << 1 | 1u << 8, many = 1u << 2 | 1u << 4;
   const unsigned shapes = T <= 32 ? few : T <= 64 ? few | many : many | 1u << 3;  // (shape 3 sums in one chain: not for few tokens)
@@ -1082,24 +1114,64 @@ HgemmPlan hgemm_plan(const QW* w, int n, int T) {
       }
     }
   }
+  if (sum) *sum += least;
   return best;
 }
 
-template <int TYPE, int V>
-int hgemm_go(HSegs& g, int mt, int S, hipStream_t s) {
-  constexpr HShape q = hgemm_shape(TYPE, V);
-  constexpr int BN = hgemm_tokens(q);
-  constexpr size_t lds = q.lds ? (size_t)LdsMap<TYPE, q.mi, q.nw>::BYTES
-                               : (size_t)(BN > 32 ? 3 * 2 * 64 + 2 * 18 : 2 * (4 * 2 * 64 + 18)) * BN * sizeof(_Float16);
-  static_assert(q.percu * lds <= 160 * 1024, "hgemm_price counts on `percu` workgroups on a CU");
-  static TlDeviceOnce lds_raised;
-  void (*kernel)(HSegs);
-  if constexpr (q.lds) kernel = hgemm_lds_kernel<TYPE, q.mi, q.nw>;
-  else kernel = hgemm_kernel<TYPE, q.tk, q.ni, q.mi, q.nw, q.wpe, q.stack>;
-  TL_TRY(tl_raise_lds_limit(kernel, (int)lds, lds_raised));
+// Price of one launch over both (HPair), as hgemm_price for its workgroups: their super-blocks one after another on the CU that has most of
+// them, the longer workgroups dealt first
+float hgemm_pair_price(int cus, int v6, int v4, int T, long n6, int per6, int S6, long n4, int per4, int S4, float outputs6, float outputs4) {
+  const bool few = v4 != 2 && v4 != 3;
+  const HFew& f = HGEMM_FEW[v4];
+  const float t6 = few || T <= 64 ? (float)per6 * f.superblock[1] : ((float)per6 + 0.6f) * 6.3f;
+  const float t4 = few || T <= 64 ? (float)per4 * f.superblock[0] : (float)(per4 + 1) * HGEMM_US[v4];
+  // the CUs' loads: `more` of them at `high`, the others at `low`
+  const bool six = t6 >= t4;
+  const float tb = six ? t6 : t4, ts = six ? t4 : t6;
+  const long nb = six ? n6 : n4;
+  long ns = six ? n4 : n6, more = nb % cus;
+  float low = (float)(nb / cus) * tb, high = more ? low + tb : low;
+  if (!more) more = cus;
+  float top = high;
+  while (ns > 0) {  // a shorter one for each of the CUs with the least
+    const long least = low < high ? cus - more : more;
+    float& at = low < high ? low : high;
+    if (ns < least || more == cus) {
+      const long rounds = more == cus ? (ns + cus - 1) / cus : 1;
+      at += (float)rounds * ts;
+      ns = 0;
+    } else {
+      at += ts;
+      ns -= least;
+    }
+    top = at > top ? at : top;
+  }
+  const int S = S6 > S4 ? S6 : S4;
+  const float sums = (S > 1 ? 0.3f * (float)S : 0.f) + 2e-6f * ((S6 > 1 ? (float)S6 * outputs6 : 0.f) + (S4 > 1 ? (float)S4 * outputs4 : 0.f));
+  if (!few && T > 64) return top + sums;
+  const long most = (n6 + n4 + cus - 1) / cus, percu = hgemm_shape(TL_Q4_K, v4).percu, rounds = (most + percu - 1) / percu;
+  return f.start * (0.75f + 0.25f * (float)rounds) + top + sums;
+}
+
+// tiles and constants of the launch's division into workgroups; returns their number
+int hgemm_grid(HSegs& g, const QW* w, int n, const HShape& q, const HAct& act, float* const* out, const float* resid, int T, int S) {
+  const int bm = q.tk * q.mi * q.nw, BN = hgemm_tokens(q);
+  int mt = 0;
+  g.T = T;
+  g.K = w[0].cols;
+  g.nsb = (w[0].cols + 255) / 256;
+  g.resid = resid;
+  g.act = act;
+  for (int i = 0; i < 3; ++i) {
+    const int k = i < n ? i : n - 1;  // (unused slots repeat the last matrix; their tile range is empty)
+    g.w[i] = w[k];
+    g.y[i] = out[k];
+    if (i < n) mt += (w[i].rows + bm - 1) / bm;
+    if (i < 2) g.mt_end[i] = mt;
+  }
   // panels of eight token tiles and more, all alike: a panel of the one tile that is left over reads all weights again for it (28672 x
   // 4096 in Q4_K times 513 tokens, nine tiles, 274 us in one panel of shape 3 with 256 rows, 281 in eight and one)
-  const int ntiles = (g.T + BN - 1) / BN, panels = ntiles < 16 ? 1 : ntiles / 8, panel = (ntiles + panels - 1) / panels;
+  const int ntiles = (T + BN - 1) / BN, panels = ntiles < 16 ? 1 : ntiles / 8, panel = (ntiles + panels - 1) / panels;
   g.per = (g.nsb + S - 1) / S;
   g.per8 = mt * ntiles * S / 8;
   g.rem8 = mt * ntiles * S % 8;
@@ -1112,38 +1184,42 @@ int hgemm_go(HSegs& g, int mt, int S, hipStream_t s) {
   g.by_panel = Div::by(g.panel_tiles);
   g.by_width = Div::by(panel);
   g.by_last = Div::by(g.width_last);
-  kernel<<<dim3((unsigned)(mt * ntiles * S)), dim3(64 * q.nw), lds, s>>>(g);
+  return mt * ntiles * S;
+}
+template <int TYPE, int V>
+int hgemm_go(const HSegs& g, int blocks, hipStream_t s) {
+  static TlDeviceOnce lds_raised;
+  constexpr size_t lds = hgemm_lds_bytes<TYPE, V>();
+  TL_TRY(tl_raise_lds_limit(hgemm_kernel<TYPE, V>, (int)lds, lds_raised));
+  hgemm_kernel<TYPE, V><<<dim3((unsigned)blocks), dim3(64 * hgemm_shape(TYPE, V).nw), lds, s>>>(g);
   TL_HIP(hipGetLastError());
   return 0;
 }
 template <int TYPE>
 int hgemm_typed(const QW* w, int n, const HgemmPlan& p, const HAct& act, float* const* out, const float* resid, int T, hipStream_t s) {
   HSegs g = {};
-  g.T = T;
-  g.K = w[0].cols;
-  g.nsb = (w[0].cols + 255) / 256;
-  g.resid = resid;
-  g.act = act;
-  int mt = 0;
   const int shape = p.shape == 2 && w[0].cols % 256 ? 4 : p.shape;  // (rows that end inside a super-block: shape 4's kernel has the same sums)
-  const int bm = hgemm_shape(TYPE, shape).tk * hgemm_shape(TYPE, shape).mi * hgemm_shape(TYPE, shape).nw;
-  for (int i = 0; i < 3; ++i) {
-    const int k = i < n ? i : n - 1;  // (unused slots repeat the last matrix; their tile range is empty)
-    g.w[i] = w[k];
-    g.y[i] = out[k];
-    if (i < n) mt += (w[i].rows + bm - 1) / bm;
-    if (i < 2) g.mt_end[i] = mt;
-  }
-  if (shape == 0) return hgemm_go<TYPE, 0>(g, mt, p.S, s);
-  if (shape == 1) return hgemm_go<TYPE, 1>(g, mt, p.S, s);
-  if (shape == 2) return hgemm_go<TYPE, 2>(g, mt, p.S, s);
+  const int blocks = hgemm_grid(g, w, n, hgemm_shape(TYPE, shape), act, out, resid, T, p.S);
+  if (shape == 0) return hgemm_go<TYPE, 0>(g, blocks, s);
+  if (shape == 1) return hgemm_go<TYPE, 1>(g, blocks, s);
+  if (shape == 2) return hgemm_go<TYPE, 2>(g, blocks, s);
   if constexpr (TYPE == TL_Q4_K || TYPE == TL_Q8_K)
-    if (shape == 3) return hgemm_go<TYPE, 3>(g, mt, p.S, s);
-  if (shape == 5) return hgemm_go<TYPE, 5>(g, mt, p.S, s);
-  if (shape == 6) return hgemm_go<TYPE, 6>(g, mt, p.S, s);
-  if (shape == 7) return hgemm_go<TYPE, 7>(g, mt, p.S, s);
-  if (shape == 8) return hgemm_go<TYPE, 8>(g, mt, p.S, s);
-  return hgemm_go<TYPE, 4>(g, mt, p.S, s);
+    if (shape == 3) return hgemm_go<TYPE, 3>(g, blocks, s);
+  if (shape == 5) return hgemm_go<TYPE, 5>(g, blocks, s);
+  if (shape == 6) return hgemm_go<TYPE, 6>(g, blocks, s);
+  if (shape == 7) return hgemm_go<TYPE, 7>(g, blocks, s);
+  if (shape == 8) return hgemm_go<TYPE, 8>(g, blocks, s);
+  return hgemm_go<TYPE, 4>(g, blocks, s);
+}
+template <int V6, int V4>
+int hgemm_pair_go(const HPair& g, int blocks, hipStream_t s) {
+  static TlDeviceOnce lds_raised;
+  constexpr size_t l6 = hgemm_lds_bytes<TL_Q6_K, V6>(), l4 = hgemm_lds_bytes<TL_Q4_K, V4>(), lds = l6 > l4 ? l6 : l4;
+  static_assert(hgemm_shape(TL_Q6_K, V6).nw == hgemm_shape(TL_Q4_K, V4).nw && hgemm_shape(TL_Q6_K, V6).wpe == hgemm_shape(TL_Q4_K, V4).wpe, "");
+  TL_TRY(tl_raise_lds_limit(hgemm_pair_kernel<V6, V4>, (int)lds, lds_raised));
+  hgemm_pair_kernel<V6, V4><<<dim3((unsigned)blocks), dim3(64 * hgemm_shape(TL_Q4_K, V4).nw), lds, s>>>(g);
+  TL_HIP(hipGetLastError());
+  return 0;
 }
 
 }  // namespace
@@ -1154,6 +1230,77 @@ bool tl_hgemm_supported(const QW& w) {
          (size_t)w.rows * w.cols < ((size_t)1 << 32);  // (32-bit byte offsets)
 }
 HgemmPlan tl_hgemm_plan(const QW* w, int n, int T) { return hgemm_plan(w, n, T); }
+bool tl_hgemm_pair_plan(const QW* w4, int n4, const QW& w6, int T, int most_slices, HgemmPlan* p4, HgemmPlan* p6) {
+  if (w4[0].type != TL_Q4_K || w6.type != TL_Q6_K || w4[0].cols != w6.cols || n4 < 1 || n4 > 3) return false;
+  for (int i = 0; i < n4; ++i)
+    if (!tl_hgemm_supported(w4[i]) || w4[i].type != TL_Q4_K || w4[i].cols != w6.cols) return false;
+  if (!tl_hgemm_supported(w6)) return false;
+  const int nsb = w6.cols / 256, cus = tl_num_cus(), slices = most_slices < nsb ? most_slices : nsb;
+  long rows4 = 0;
+  for (int i = 0; i < n4; ++i) rows4 += w4[i].rows;
+  const float out4 = (float)T * (float)rows4, out6 = (float)T * (float)w6.rows;
+  const unsigned few = T <= 8 ? 1u << 5 | 1u << 6 : T <= 16 ? 1u << 0 | 1u << 7 : 1u << 1 | 1u << 8, many = 1u << 2;
+  const unsigned shapes = T <= 32 ? few : T <= 64 ? few | many : many | 1u << 3;
+  float least = -1.f;
+  for (int v = 0; v < HGEMM_SHAPES; ++v) {
+    if (!(shapes >> v & 1)) continue;
+    const int v6 = v == 3 ? 2 : v;
+    const HShape q4 = hgemm_shape(TL_Q4_K, v), q6 = hgemm_shape(TL_Q6_K, v6);
+    const int ntiles = (T + hgemm_tokens(q4) - 1) / hgemm_tokens(q4), bm4 = q4.tk * q4.mi * q4.nw, bm6 = q6.tk * q6.mi * q6.nw;
+    long t4 = 0;
+    for (int i = 0; i < n4; ++i) t4 += (long)((w4[i].rows + bm4 - 1) / bm4) * ntiles;
+    const long t6 = (long)((w6.rows + bm6 - 1) / bm6) * ntiles;
+    for (int a = 1; a <= 8 && a <= slices; ++a) {
+      const int per4 = (nsb + a - 1) / a;
+      if ((nsb + per4 - 1) / per4 != a) continue;
+      for (int b = 1; b <= 8 && b <= slices; ++b) {
+        const int per6 = (nsb + b - 1) / b;
+        if ((nsb + per6 - 1) / per6 != b) continue;
+        const float price = hgemm_pair_price(cus, v6, v, T, t6 * b, per6, b, t4 * a, per4, a, out6, out4);
+        if (least < 0.f || price < least) {
+          least = price;
+          *p4 = {v, a};
+          *p6 = {v6, b};
+        }
+      }
+    }
+  }
+  // (two launches: each at its own best)
+  float apart = 0.f;
+  const HgemmPlan s4 = hgemm_plan(w4, n4, T, &apart), s6 = hgemm_plan(&w6, 1, T, &apart);
+  if (least <= (T > 64 ? 0.96f : 1.f) * apart) return true;  // (the prices of long chunks are right to a few per cent)
+  *p4 = s4;
+  *p6 = s6;
+  return false;
+}
+int tl_launch_hgemm_pair(const QW* w4, int n4, const QW& w6, const void* planes, size_t ps, float* const* out4, float* out6, int T,
+                         const HgemmPlan& p4, const HgemmPlan& p6, hipStream_t s) {
+  const int nsb = w6.cols / 256;
+  for (int i = 0; i < n4; ++i)
+    TL_REQUIRE(tl_hgemm_supported(w4[i]) && w4[i].type == TL_Q4_K && w4[i].cols == w6.cols, "half-plane GEMM: matrix %d does not fit", i);
+  TL_REQUIRE(n4 >= 1 && n4 <= 3 && T > 0 && tl_hgemm_supported(w6) && w6.type == TL_Q6_K && ps < ((size_t)1 << 31) &&
+                 ps >= tl_gemm_padded_tokens(T) * (size_t)w6.cols, "half-plane GEMM: bad argument of a launch of two formats");
+  for (const HgemmPlan& p : {p4, p6})
+    TL_REQUIRE(p.S >= 1 && (p.S - 1) * ((nsb + p.S - 1) / p.S) < nsb && p.shape >= 0 && p.shape < HGEMM_SHAPES && p6.shape == (p4.shape == 3 ? 2 : p4.shape),
+               "half-plane GEMM: shape %d, %d K slices of %d super-blocks", p.shape, p.S, nsb);
+  const HAct act = hact(planes, ps, T);
+  HPair g = {};
+  g.first = hgemm_grid(g.q6, &w6, 1, hgemm_shape(TL_Q6_K, p6.shape), act, &out6, nullptr, T, p6.S);
+  const int blocks = g.first + hgemm_grid(g.q4, w4, n4, hgemm_shape(TL_Q4_K, p4.shape), act, out4, nullptr, T, p4.S);
+  switch (p4.shape) {
+    case 0: return hgemm_pair_go<0, 0>(g, blocks, s);
+    case 1: return hgemm_pair_go<1, 1>(g, blocks, s);
+    case 2: return hgemm_pair_go<2, 2>(g, blocks, s);
+    case 3: return hgemm_pair_go<2, 3>(g, blocks, s);
+    case 5: return hgemm_pair_go<5, 5>(g, blocks, s);
+    case 6: return hgemm_pair_go<6, 6>(g, blocks, s);
+    case 7: return hgemm_pair_go<7, 7>(g, blocks, s);
+    case 8: return hgemm_pair_go<8, 8>(g, blocks, s);
+    default: break;
+  }
+  TL_REQUIRE(false, "half-plane GEMM: shape %d has no launch of two formats", p4.shape);
+  return 0;
+}
 int tl_launch_hgemm(const QW* w, int n, const void* planes, size_t ps, float* const* out, const float* resid, int T, const HgemmPlan& p,
                     hipStream_t s) {
   for (int i = 0; i < n; ++i)

@@ -280,6 +280,10 @@ struct HgemmPlan {
 HgemmPlan tl_hgemm_plan(const QW* w, int n, int T);  // of one launch over w[0 .. n - 1]; fewer slices than its S only as S = 1
 int tl_launch_hgemm(const QW* w, int n, const void* planes, size_t plane_stride, float* const* out, const float* resid, int T,
                     const HgemmPlan& plan, hipStream_t s);
+// n4 matrices in Q4_K and one in Q6_K in one launch: true where that is the better price than a launch of each; the plans of either way
+bool tl_hgemm_pair_plan(const QW* w4, int n4, const QW& w6, int T, int most_slices, HgemmPlan* p4, HgemmPlan* p6);
+int tl_launch_hgemm_pair(const QW* w4, int n4, const QW& w6, const void* planes, size_t plane_stride, float* const* out4, float* out6, int T,
+                         const HgemmPlan& p4, const HgemmPlan& p6, hipStream_t s);
 int tl_launch_hsplit(int mode, const float* x, const float* aux, void* planes, size_t plane_stride, int T, int K, float eps,
                      hipStream_t s, const GemmParts& a, const GemmParts& b, float* xout);
 // y = (resid ? resid : 0) + the pending sums (what the GEMM launch would have run itself)

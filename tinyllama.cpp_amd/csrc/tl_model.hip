@@ -1354,6 +1354,7 @@ static void half_part_floats(const tl_model* m, int most, size_t (&cap)[3]) {
         add(L, {TL_T_ATTN_K}, 1);
       }
       add(L, {TL_T_ATTN_V}, 2);
+      if (tq == tk) add(L, {TL_T_ATTN_Q, TL_T_ATTN_K, TL_T_ATTN_V}, 0);
     }
     add(L, {TL_T_ATTN_OUTPUT}, 0);
     if (L.q[TL_T_FFN_GATE]->type == L.q[TL_T_FFN_UP]->type) {
@@ -1368,8 +1369,14 @@ static void half_part_floats(const tl_model* m, int most, size_t (&cap)[3]) {
   for (const Group& g : groups)
     for (int T = 1, end; T <= most; T = end + 1) {
       end = std::min(T == 1 ? 8 : T == 9 ? 16 : T == 17 ? 32 : T + 63 - (T - 1) % 64, most);
-      const int S = tl_hgemm_plan(g.w, g.n, T).S;
-      for (int i = 0; i < g.n && S > 1; ++i) cap[g.at + i] = std::max(cap[g.at + i], (size_t)S * end * g.w[i].rows);
+      HgemmPlan p4 = {}, p6 = {};  // (two formats: the plans of a launch over both, where there is one)
+      const bool pair = g.n == 3 && g.w[2].type != g.w[0].type;
+      if (pair && !tl_hgemm_pair_plan(g.w, 2, g.w[2], T, 8, &p4, &p6)) continue;
+      const int S = pair ? 0 : tl_hgemm_plan(g.w, g.n, T).S;
+      for (int i = 0; i < g.n; ++i) {
+        const int Si = !pair ? S : i < 2 ? p4.S : p6.S;
+        if (Si > 1) cap[g.at + i] = std::max(cap[g.at + i], (size_t)Si * end * g.w[i].rows);
+      }
     }
 }
 static int ensure_prefill_ws(tl_model* m, bool all_logits) {
@@ -1465,14 +1472,20 @@ static int qkv_deferred(tl_model* m, LayerW& L, int T, hipStream_t s) {
   p.dk = {p.part[1], p.part_cap[1], {nullptr, 0, 0}};
   p.dv = {p.part[2], p.part_cap[2], {nullptr, 0, 0}};
   const bool defer = p.part_cap[0] != 0;
-  // one launch where the formats are equal (Q4_K_M files hold v as Q6_K in some layers)
+  // one launch where the formats are equal, and also where two in Q4_K and v in Q6_K (some layers of Q4_K_M files) are better off in one
   bool merged = false;
   const QW w3[3] = {qw_view(L.q[TL_T_ATTN_Q]), qw_view(L.q[TL_T_ATTN_K]), qw_view(L.q[TL_T_ATTN_V])};
   float* const y3[3] = {p.qb, p.kb, p.vb};
   GemmDefer* const d3[3] = {&p.dq, &p.dk, &p.dv};
-  const int same = w3[2].type == w3[0].type ? 3 : 2;
   GemmDefer* const* d3p = defer ? d3 : nullptr;
-  if (w3[1].type == w3[0].type) TL_TRY(tl_launch_gemm_q_multi(w3, same, p.planes, ps, y3, T, terms, s, d3p, &merged));
+  int same = 3;
+  if (w3[1].type == w3[0].type) {
+    TL_TRY(tl_launch_gemm_q_multi(w3, 3, p.planes, ps, y3, T, terms, s, d3p, &merged));
+    if (!merged && w3[2].type != w3[0].type) {
+      same = 2;
+      TL_TRY(tl_launch_gemm_q_multi(w3, same, p.planes, ps, y3, T, terms, s, d3p, &merged));
+    }
+  }
   if (merged) {
     if (same == 2) TL_TRY(tl_launch_gemm_q(w3[2], p.planes, ps, p.vb, nullptr, T, terms, s, defer ? &p.dv : nullptr));
     return 0;
