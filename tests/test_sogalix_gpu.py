@@ -631,7 +631,7 @@ def test_configurations_drawn_at_random(env, seed, tmp_path):
     s.close()
 
 
-@pytest.mark.parametrize("heads,dim", [(3, 64), (2, 128)])
+@pytest.mark.parametrize("heads,dim", [(3, 64), (2, 128), (33, 64), (17, 128)])  # (33 and 17: more than half the chip's CUs with 16 lanes a column)
 def test_generalized_delta_rule_of_aligned_rows(env, heads, dim):
     """Rows at 16 bytes take the unrolled scan: portions below, at and above its stages of 16 and 8 tokens, against the recurrence
     in 64 bits (a few 32-bit roundings a token, decayed by w >= 0.54: some 1e-6 of the outputs' size)."""

@@ -497,31 +497,35 @@ __global__ __launch_bounds__(256) void gdelta_scan_kernel(const GDeltaScanArgs a
   }
 }
 
-// The same for key sizes of exactly 16 E and rows at 16 bytes. One wave a SIMD walks the tokens, so what a token costs is the number of
-// its instructions: here five 16-byte LDS reads at constant offsets (a stage is unrolled), 5 E products and sums, and two row sums. (r w)
-// is formed once in staging; the lane whose number is the token's keeps x and y, and a stage's outputs are finished and stored together.
-// The new column is one rounding of w s + (k v - a u x). 32 heads of 64 times 1999 tokens: 239 us with a stage that is not unrolled and
-// an output stored per token; a layer-list prompt of eight such layers 8.5 -> 7.4 ms, about 100 us a launch.
-template <int E>
+// The same for key sizes of 64 and 128 and rows at 16 bytes. One wave a SIMD walks the tokens, so what a token costs is the number of
+// its instructions: here five LDS reads at constant offsets (a stage is unrolled), five products and sums per key channel of a lane, and two
+// row sums. (r w) is formed once in staging; the lane whose number is the token's keeps x and y, and a stage's outputs are finished and
+// stored together. The new column is one rounding of w s + (k v - a u x).
+// LC lanes share a column, 16 or 32: with 32 a lane has half the key channels and a workgroup half the columns, so twice as many CUs are at
+// work: a rule on whether all of those workgroups then have a CU of their own (two waves a SIMD walk 32 instructions a token each, one 42).
+// 32 heads of 64 times 1999 tokens: 239 us with 16 lanes and operands read where they are used, 224 with them read ahead, 212 with 32 lanes
+// as well. What is left is the chain from a token's column to the next one's.
+template <int DP, int LC>
 __global__ __launch_bounds__(256) void gdelta_scan_wide_kernel(const GDeltaScanArgs a) {
+  constexpr int E = DP / LC, VE = E < 4 ? E : 4, NV = E / VE, COLS = 256 / LC, TB = 1024 / DP;  // tokens per stage: a 16-byte piece of each vector per thread
   typedef float f32x4 __attribute__((ext_vector_type(4)));
-  constexpr int DP = 16 * E, TB = 1024 / DP;  // tokens per stage: a 16-byte piece of each vector per thread
-  static_assert(TB <= 16, "a token of a stage per lane of a column");
+  typedef float vec __attribute__((ext_vector_type(VE)));
+  static_assert(TB <= 16 && (LC == 16 || LC == 32), "a token of a stage per lane of a row of 16");
   constexpr int RW = 0, K = 1, W = 2, U = 3, A = 4;
   __shared__ __attribute__((aligned(16))) float st[2][5][TB][DP];
-  __shared__ float sv[2][TB][16], sc[2][TB][2];
-  const int tid = threadIdx.x, sub = tid & 15, cl = tid >> 4, h = blockIdx.y;
-  const int col = blockIdx.x * 16 + cl, d0 = sub * E;
+  __shared__ float sv[2][TB][COLS], sc[2][TB][2];
+  const int tid = threadIdx.x, sub = tid & 15, cl = tid / LC, h = blockIdx.y;
+  const int col = blockIdx.x * COLS + cl, d0 = tid % LC * E;
   const bool live = col < a.vdim;  // lanes of a column beyond vdim compute on the first one's numbers and store nothing
   float* sp = a.state + ((size_t)h * a.vdim + (live ? col : 0)) * DP + d0;
-  f32x4 s[E / 4];
+  vec s[NV];
 #pragma unroll
-  for (int e = 0; e < E / 4; ++e) s[e] = *reinterpret_cast<const f32x4*>(sp + 4 * e);
+  for (int e = 0; e < NV; ++e) s[e] = *reinterpret_cast<const vec*>(sp + VE * e);
   const int hd = a.heads * DP, ft = tid / (DP / 4), fd = tid % (DP / 4) * 4;
   const float* rp = a.r + (size_t)h * DP + fd;
   const float* kp = a.k + (size_t)h * DP + fd;
   const size_t c0 = (size_t)h * DP + fd;
-  const int vt = tid >> 4, vcol = blockIdx.x * 16 + sub;
+  const int vt = tid / COLS, vs = tid % COLS, vcol = blockIdx.x * COLS + vs;
   const float* vp = a.v + (size_t)h * a.vdim + (vcol < a.vdim ? vcol : 0);
   const float* cp = (tid & 1 ? a.rk : a.rau) + h;
   f32x4 g[5];
@@ -540,35 +544,57 @@ __global__ __launch_bounds__(256) void gdelta_scan_wide_kernel(const GDeltaScanA
     g[RW] *= g[W];
 #pragma unroll
     for (int i = 0; i < 5; ++i) *reinterpret_cast<f32x4*>(&st[b][i][ft][fd]) = g[i];
-    if (vt < TB) sv[b][vt][sub] = gv;
+    if (vt < TB) sv[b][vt][vs] = gv;
     if (tid < 2 * TB) sc[b][tid >> 1][tid & 1] = gc;
   };
-  float xk = 0.0f, yk = 0.0f;
-  auto token = [&](int b, int tt) __attribute__((always_inline)) {
-    f32x4 q[5][E / 4];
+  auto dot = [](vec p, vec q) __attribute__((always_inline)) {
+    const float x = fmaf(p[0], q[0], p[1] * q[1]);
+    if constexpr (VE == 4) return x + fmaf(p[2], q[2], p[3] * q[3]);
+    else return x;
+  };
+  float xk = 0.0f, yk = 0.0f;  // (LC 32: x in the even rows of 16 lanes and y in the odd ones, in xk)
+  struct Token {
+    vec q[5][NV];
+    float vc;
+  };
+  auto read = [&](Token& n, int b, int tt) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 5; ++i)
 #pragma unroll
-      for (int e = 0; e < E / 4; ++e) q[i][e] = *reinterpret_cast<const f32x4*>(&st[b][i][tt][d0 + 4 * e]);
-    const float vc = sv[b][tt][cl];
-    float x = 0.0f, y = 0.0f;
+      for (int e = 0; e < NV; ++e) n.q[i][e] = *reinterpret_cast<const vec*>(&st[b][i][tt][d0 + VE * e]);
+    n.vc = sv[b][tt][cl];
+  };
+  auto token = [&](const Token& n, int tt) __attribute__((always_inline)) {
+    const vec(&q)[5][NV] = n.q;
+    const float vc = n.vc;
+    float x = dot(q[U][0], s[0]), y = dot(q[RW][0], s[0]);
 #pragma unroll
-    for (int e = 0; e < E / 4; ++e) {
-      x += fmaf(q[U][e][0], s[e][0], q[U][e][1] * s[e][1]) + fmaf(q[U][e][2], s[e][2], q[U][e][3] * s[e][3]);
-      y += fmaf(q[RW][e][0], s[e][0], q[RW][e][1] * s[e][1]) + fmaf(q[RW][e][2], s[e][2], q[RW][e][3] * s[e][3]);
+    for (int e = 1; e < NV; ++e) {
+      x += dot(q[U][e], s[e]);
+      y += dot(q[RW][e], s[e]);
     }
     x = tl_row16_sum(x);
     y = tl_row16_sum(y);
+    if constexpr (LC == 32) {
+      // x's odd rows change places with y's even ones: one addition forms x's sum in the even rows and y's in the odd ones, which take x from
+      // the last lane of the row below them (row_bcast:15)
+      const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+      const float z = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+      x = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(z), __float_as_int(z), 0x142, 0xa, 0xf, false));
+      xk = sub == tt ? z : xk;
+    } else {
+      xk = sub == tt ? x : xk;
+      yk = sub == tt ? y : yk;
+    }
 #pragma unroll
-    for (int e = 0; e < E / 4; ++e)
+    for (int e = 0; e < NV; ++e)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s[e][j] = fmaf(q[W][e][j], s[e][j], fmaf(-q[A][e][j], x, q[K][e][j] * vc));
-    xk = sub == tt ? x : xk;
-    yk = sub == tt ? y : yk;
+      for (int j = 0; j < VE; ++j) s[e][j] = fmaf(q[W][e][j], s[e][j], fmaf(-q[A][e][j], x, q[K][e][j] * vc));
   };
   float* op = a.o + (size_t)h * a.vdim + col;
   auto finish = [&](int b, int t0, int nt) __attribute__((always_inline)) {
-    if (live && sub < nt) op[(size_t)(t0 + sub) * a.heads * a.vdim] = yk - sc[b][sub][0] * xk + sc[b][sub][1] * sv[b][sub][cl];
+    const float yf = LC == 32 ? tl_xor<16>(xk) : yk;
+    if (live && sub < nt && tid % LC < 16) op[(size_t)(t0 + sub) * a.heads * a.vdim] = yf - sc[b][sub][0] * xk + sc[b][sub][1] * sv[b][sub][cl];
   };
   fetch(0);
   stash(0);
@@ -577,20 +603,44 @@ __global__ __launch_bounds__(256) void gdelta_scan_wide_kernel(const GDeltaScanA
   for (; t0 + TB <= a.T; t0 += TB, b ^= 1) {
     const bool more = t0 + TB < a.T;
     if (more) fetch(t0 + TB);  // in flight under this stage's tokens
+    // two tokens' operands are read while the two in front of them are walked: without the barriers the compiler reads a pair where it is
+    // used, and a round trip to LDS is as long as a token
+    Token n[2][2];
+    read(n[0][0], b, 0);
+    read(n[0][1], b, 1);
 #pragma unroll
-    for (int tt = 0; tt < TB; ++tt) token(b, tt);
+    for (int tt = 0; tt < TB; tt += 2) {
+      const int k = tt >> 1 & 1;
+      __builtin_amdgcn_sched_barrier(0);
+      if (tt + 2 < TB) {
+        read(n[k ^ 1][0], b, tt + 2);
+        read(n[k ^ 1][1], b, tt + 3);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      token(n[k][0], tt);
+      token(n[k][1], tt + 1);
+    }
     finish(b, t0, TB);
     if (more) stash(b ^ 1);  // the other buffer: its last readers passed the barrier at the end of the stage before
     __syncthreads();
   }
   if (t0 < a.T) {
-    for (int tt = 0; tt < a.T - t0; ++tt) token(b, tt);
+    for (int tt = 0; tt < a.T - t0; ++tt) {
+      Token n;
+      read(n, b, tt);
+      token(n, tt);
+    }
     finish(b, t0, a.T - t0);
   }
   if (live) {
 #pragma unroll
-    for (int e = 0; e < E / 4; ++e) *reinterpret_cast<f32x4*>(sp + 4 * e) = s[e];
+    for (int e = 0; e < NV; ++e) *reinterpret_cast<vec*>(sp + VE * e) = s[e];
   }
+}
+template <int DP>
+void gdelta_scan_wide(const GDeltaScanArgs& a, hipStream_t s) {
+  if (2 * (long)((a.vdim + 15) / 16) * a.heads <= tl_num_cus()) gdelta_scan_wide_kernel<DP, 32><<<dim3((a.vdim + 7) / 8, a.heads), 256, 0, s>>>(a);
+  else gdelta_scan_wide_kernel<DP, 16><<<dim3((a.vdim + 15) / 16, a.heads), 256, 0, s>>>(a);
 }
 
 }  // namespace
@@ -707,8 +757,8 @@ int tl_launch_gdelta_scan(const GDeltaScanArgs& a, hipStream_t s) {
   const dim3 grid((a.vdim + 15) / 16, a.heads);
   const int e = (a.dim + 15) / 16;
   const bool wide = (a.ld & 3) == 0 && (((size_t)a.r | (size_t)a.k | (size_t)a.w | (size_t)a.u | (size_t)a.au | (size_t)a.state) & 15) == 0;
-  if (wide && a.dim == 64) gdelta_scan_wide_kernel<4><<<grid, 256, 0, s>>>(a);
-  else if (wide && a.dim == 128) gdelta_scan_wide_kernel<8><<<grid, 256, 0, s>>>(a);
+  if (wide && a.dim == 64) gdelta_scan_wide<64>(a, s);
+  else if (wide && a.dim == 128) gdelta_scan_wide<128>(a, s);
   else if (e <= 1) gdelta_scan_kernel<1><<<grid, 256, 0, s>>>(a);
   else if (e <= 2) gdelta_scan_kernel<2><<<grid, 256, 0, s>>>(a);
   else if (e <= 4) gdelta_scan_kernel<4><<<grid, 256, 0, s>>>(a);
