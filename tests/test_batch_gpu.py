@@ -406,6 +406,38 @@ def test_two_formats_in_one_launch(pkg, monkeypatch, heads, kv):
     m.free()
 
 
+def test_packed_output_rows_in_any_order(pkg):
+    """Output rows of a packed batch that come in no order, from two chunks in turn, twice, and more of them than one gather takes: each is the
+    logits row of its own sequence's prefill, up to the order of 32-bit sums (2^-22 a layer and product)."""
+    from tinyllama_cpp_amd import engine as E
+    from tinyllama_cpp_amd.capi import check, lib
+    E.init(0)
+    cfg, tensors = pkg.synth.build_model(dict(pkg.synth.SHAPES["tiny-gqa"], max_pos=96), "q4_k_m", seed=18)
+    m = E.Model(cfg).load(tensors)
+    n_seq = 96
+    m.batch_init(n_seq)
+    rng = np.random.default_rng(18)
+    prompts = [rng.integers(0, cfg["vocab"], n).astype(np.int32) for n in rng.integers(9, 48, n_seq)]
+    toks, pos = np.concatenate(prompts), np.concatenate([np.arange(p.size, dtype=np.int32) for p in prompts])
+    seq = np.concatenate([np.full(p.size, i, np.int32) for i, p in enumerate(prompts)])
+    assert toks.size > 2048 + 64
+    want = []
+    for p in prompts:
+        m.reset_kv()
+        want.append(m.prefill(p, 0, all_logits=True)[1])
+    want = np.concatenate(want)
+    for rows in (rng.integers(0, toks.size, n_seq), np.arange(toks.size - n_seq, toks.size), np.array([2047, 2048, 0, 2048, toks.size - 1]), np.arange(64)):
+        rows = np.ascontiguousarray(rows, np.int32)
+        logits, ids = np.empty((rows.size, cfg["vocab"]), np.float32), np.empty(rows.size, np.int32)
+        check(lib().tl_model_batch_prefill_packed(m.h, toks.size, toks.ctypes.data, pos.ctypes.data, seq.ctypes.data, rows.size, rows.ctypes.data,
+                                                  logits.ctypes.data, ids.ctypes.data), "tl_model_batch_prefill_packed")
+        # (the bound of the next test, which is one of all rows together; another row's logits are as far off as their size)
+        assert np.linalg.norm(logits - want[rows]) <= 4e-6 * np.linalg.norm(want[rows])
+        assert all(np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(b) for a, b in zip(logits, want[rows]))
+        assert np.array_equal(ids, logits.argmax(1))
+    m.free()
+
+
 def test_packed_prompts_longer_than_a_sequence(pkg):
     """A packed batch of more tokens than a sequence has positions goes through as one chunk: every prompt's last logits are those
     of its own prefill, up to the order of 32-bit sums (2^-22 a layer and product)."""

@@ -1909,7 +1909,7 @@ static int batch_layers_gemv(tl_model* m, int T, hipStream_t s) {
 
 // one step for the T tokens in bt.toks / bt.pos / bt.seq; ids_dev: [T] next ids (first maximum of each logits row);
 // advance: the ids become the next tokens and the positions move on (device-resident loop)
-// all layers for the T tokens in bt.toks / bt.pos / bt.seq: the residual stream ends up in pf.xb [T][hidden]
+// all layers for the T tokens in bt.toks / bt.pos / bt.seq: the residual stream ends up in pf.xb [T][hidden], its last projection maybe pending
 static int batch_layers(tl_model* m, int T, hipStream_t s, int packed = 0) {
   TL_REQUIRE(T >= 1 && T <= m->pf.cap, "tl_model: a batched step of %d tokens exceeds the chunk workspaces (%d)", T, m->pf.cap);
   if (T <= gemv_most(m)) return batch_layers_gemv(m, T, s);
@@ -1918,15 +1918,16 @@ static int batch_layers(tl_model* m, int T, hipStream_t s, int packed = 0) {
     TL_TRY(batch_attn_half(m, l, T, packed, s));
     TL_TRY(prefill_mlp_half(m, l, T, s));
   }
-  return flush_residual(m, s);
+  return 0;
 }
-// final RMSNorm + lm_head of R hidden rows -> pf.logits_all [R][vocab]
+// final RMSNorm + lm_head of R hidden rows (pf.xb: with what is pending) -> pf.logits_all [R][vocab]
 static int batch_head(tl_model* m, const float* hidden, int R, hipStream_t s) {
   TL_REQUIRE(R >= 1 && R <= m->pf.cap && R <= kChunkRows, "tl_model: %d logits rows exceed the chunk workspaces (%d)", R,
              m->pf.cap < kChunkRows ? m->pf.cap : kChunkRows);
   const tl_model_config& c = m->cfg;
   tl_model::Prefill& p = m->pf;
   if (R <= gemv_most(m)) {
+    if (hidden == p.xb) TL_TRY(flush_residual(m, s));
     GemvArgs f = {};
     f.seg[0] = {qw_view(m->out), p.logits_all};
     f.nseg = 1;
@@ -1937,7 +1938,8 @@ static int batch_head(tl_model* m, const float* hidden, int R, hipStream_t s) {
     return tl_launch_gemv_nv(f, R, s);
   }
   const int terms = chunk_terms(m);
-  TL_TRY(tl_launch_split(1, hidden, m->out_norm, p.planes, p.plane_stride, R, c.hidden_size, terms, c.rms_norm_eps, s));
+  if (hidden == p.xb) TL_TRY(split_residual(m, m->out_norm, R, s));
+  else TL_TRY(tl_launch_split(1, hidden, m->out_norm, p.planes, p.plane_stride, R, c.hidden_size, terms, c.rms_norm_eps, s));
   return tl_launch_gemm_q(qw_view(m->out), p.planes, p.plane_stride, p.logits_all, nullptr, R, terms, s);
 }
 
@@ -2131,6 +2133,12 @@ extern "C" int tl_model_batch_prefill_packed(tl_model* m, int n_tokens, const in
                last_rows_host[j]);
   hipStream_t s = m->stream;
   const size_t H = c.hidden_size;
+  std::vector<int> rows;
+  try {
+    rows.reserve(n_last);
+  } catch (const std::bad_alloc&) {
+    TL_REQUIRE(false, "tl_model_batch_prefill_packed: no memory for %d output rows", n_last);
+  }
   const int chunk = chunk_tokens(m);
   TL_REQUIRE(chunk >= 1 && chunk <= kPrefillChunk, "tl_model_batch_prefill_packed: workspaces are missing");
   const char* ha = getenv("TL_HATTN");  // 0: every chunk token by token, any other number: by row tiles (A/B runs and tests)
@@ -2152,11 +2160,17 @@ extern "C" int tl_model_batch_prefill_packed(tl_model* m, int n_tokens, const in
     TL_HIP(hipMemcpyAsync(m->bt.pos, positions_host + c0, sizeof(int) * T, hipMemcpyHostToDevice, s));
     TL_HIP(hipMemcpyAsync(m->bt.seq, seq_idx_host + c0, sizeof(int) * T, hipMemcpyHostToDevice, s));
     TL_TRY(batch_layers(m, T, s, packed));
+    rows.clear();  // runs of output rows that are in this chunk
     for (int j = 0; j < n_last; ++j) {
       const int r = last_rows_host[j] - c0;
-      if (r >= 0 && r < T)
-        TL_HIP(hipMemcpyAsync(m->bt.last_h + (size_t)j * H, m->pf.xb + (size_t)r * H, sizeof(float) * H, hipMemcpyDeviceToDevice, s));
+      const bool here = r >= 0 && r < T;
+      if (here) rows.push_back(r);
+      if (!rows.empty() && (!here || j + 1 == n_last)) {
+        TL_TRY(tl_launch_gather_rows(m->pf.xb, m->pf.pend, rows.data(), (int)rows.size(), (int)H, m->bt.last_h + (j + (here ? 1 : 0) - rows.size()) * H, s));
+        rows.clear();
+      }
     }
+    m->pf.pend = {nullptr, 0, 0};
   }
   if (n_last > 0) {
     TL_TRY(batch_ids(m, (size_t)n_last));
