@@ -666,3 +666,34 @@ def test_many_logits_into_memory_that_the_runtime_knows(pkg):
     assert np.array_equal(on_device.to_numpy(np.float32, want.shape), want)
     assert hip.hipHostFree(pinned) == 0
     m.free()
+
+
+@pytest.mark.parametrize("heads,kv,hd", [(4, 4, 64), (4, 2, 128), (6, 2, 128), (8, 2, 64), (16, 2, 64), (16, 2, 128), (12, 4, 64)])
+def test_step_attention_takes_new_keys(pkg, monkeypatch, heads, kv, hd):
+    """A step whose attention rotates, sums and stores the new queries, keys and values itself against the same step with a launch of its own
+    for that (TL_ATTN_STEP=0): every group size and head size, sequences at their first position, at the edges of a wave's and a
+    workgroup's rows and beyond, slots out of order, four and eight waves; three steps, so that what was stored is read. Both sum the same
+    numbers in another order (the new position last): 2^-22 a layer and product, as packed prompts."""
+    from tinyllama_cpp_amd import engine as E
+    E.init(0)
+    cfg, tensors = pkg.synth.build_model(dict(hidden=heads * hd, inter=512, n_heads=heads, n_kv_heads=kv, n_layers=2, vocab=64, max_pos=320, eps=1e-5,
+                                              rope_theta=10000.0), "q4_k_m", seed=26)
+    lengths = [0, 1, 3, 4, 15, 16, 31, 32, 33, 63, 64, 65, 127, 128, 129, 200, 255, 256, 257, 300]
+    m = E.Model(cfg).load(tensors)
+    m.batch_init(140)
+    rng = np.random.default_rng(heads)
+    for n in (len(lengths), 140):  # (140 sequences: four waves a workgroup)
+        lens = (lengths * 7)[:n]
+        slots = rng.permutation(140)[:n].astype(np.int32)
+        prompts = [rng.integers(0, cfg["vocab"], k).astype(np.int32) for k in lens]
+        first = rng.integers(0, cfg["vocab"], n).astype(np.int32)
+        got = []
+        for step in ("0", "1"):
+            monkeypatch.setenv("TL_ATTN_STEP", step)
+            for s, p in zip(slots, prompts):
+                if p.size:
+                    m.batch_prefill(int(s), p)
+            out = [m.batch_decode(first, np.array(lens, np.int32) + i, slots)[0] for i in range(3)]
+            got.append(np.concatenate(out).astype(np.float64))
+        assert np.isfinite(got[1]).all() and np.linalg.norm(got[1] - got[0]) <= 4e-6 * np.linalg.norm(got[0])
+    m.free()

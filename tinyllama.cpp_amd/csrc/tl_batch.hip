@@ -146,6 +146,12 @@ struct BatchAttnArgs {
   int start_pos;
   // the same for the f16 GEMM's planes (what hsplit_kernel would make of `out`): workgroups of whole super-blocks only
   _Float16* hplanes;
+  // table != NULL (a token a sequence): q, k and v of the tokens are as the projections leave them, each maybe still the partial tiles of a
+  // K-split GEMM; they are summed and rotated here and written to the cache
+  const float* table;
+  const float *k, *v;
+  float *kw, *vw;
+  GemmParts pq, pk, pv;
 };
 
 // One workgroup per (kv head, token, head-group part): the G query heads of the group share every K/V row read.
@@ -164,52 +170,97 @@ __device__ __forceinline__ float batch_row_sum16(float v) {
 // 700 of them: where the launch leaves CUs idle and a token needs more than one such step, eight waves take its positions (NW, W). 8
 // sequences of 8 heads of 128 for 3 query heads each, at 20 / 100 / 500 / 4000 positions, four -> eight waves 4.9 / 6.3 / 16.3 / 106 -> 4.9 /
 // 6.0 / 12.7 / 75 us (20 with all eight at work: 5.7, whose fold of 32 records and second wave a SIMD are then all that is gained).
-template <int HD, int G, int NW>
+// FUSE (a step: every sequence has one token, at the end of its cache): a thread sums and rotates four numbers of the workgroup's query heads, the
+// new key or value on their way through LDS, while the cache's first rows are on theirs; the new position is folded from LDS, one of the
+// workgroups of a kv head writes it to the cache. A launch of its own for that is 3.8 us: steps of 8 sequences at 90 positions, 3B, 28 layers, 1.80
+// -> 1.74 ms; of 128 sequences, 8B, where it is a small part, level.
+template <int HD, int G, int NW, bool FUSE>
 __global__ __launch_bounds__(64 * NW) void attn_batch_decode_kernel(BatchAttnArgs a) {
   constexpr int LP = 16, NV = HD / 64, PP = 64 / LP, U = 8 / NV, RECL = HD + 4;
   constexpr int NR = NW * PP;  // row groups per workgroup (= one or two DPP rows of lanes in the weights phase)
   static_assert(NR == 16 || NR == 32, "the weights of a head's row groups are reduced inside one or two DPP rows");
   __shared__ __attribute__((aligned(16))) float part[NR * G * RECL];
   __shared__ float red[16], wts[G * NR];
-  __shared__ __attribute__((aligned(16))) float outbuf[G * HD];
+  __shared__ __attribute__((aligned(16))) float outbuf[G * HD];  // (FUSE: the query heads until they are in registers)
+  __shared__ __attribute__((aligned(16))) float knew[FUSE ? 2 * HD : 4];
   const int kvh = blockIdx.x, tok = blockIdx.y;
   const int head0 = (kvh * gridDim.z + blockIdx.z) * G;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int sub = lane / LP, ln = lane % LP;
-  const int pos = a.pos ? a.pos[tok] : a.start_pos + tok, sq = a.seq ? a.seq[tok] : 0;
-  if (pos < 0 || pos >= a.max_seq || sq < 0 || sq >= a.n_seq) return;  // uniform
+  const int pos = FUSE || a.pos ? a.pos[tok] : a.start_pos + tok, sq = FUSE || a.seq ? a.seq[tok] : 0;  // (a step has both)
+  if ((pos < 0) | (pos >= a.max_seq) | (sq < 0) | (sq >= a.n_seq)) return;  // uniform (and one wait for both numbers)
   const int len = pos + 1;
   // the waves that take positions: four where these need no second step
   const int W = NW > 4 && len > 4 * PP * U ? NW : 4, rows = W * PP;
   const int kv_dim = a.nkv * HD;
   const float* kbase = a.kc + (size_t)sq * a.seq_stride + (size_t)kvh * HD + 4 * ln;
   const float* vbase = a.vc + (size_t)sq * a.seq_stride + (size_t)kvh * HD + 4 * ln;
-  f32x4 qf[G][NV], acc[G][NV];
-  float m[G], l[G];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      qf[g][v] = *reinterpret_cast<const f32x4*>(a.q + ((size_t)tok * a.nh + head0 + g) * HD + 64 * v + 4 * ln);
-      acc[g][v] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    m[g] = -INFINITY;
-    l[g] = 0.f;
-  }
-  for (int base = 0; base < (wave < W ? len : 0); base += rows * U) {
-    f32x4 kk[U][NV], vv[U][NV];
-    bool valid[U];
+  const int ncache = FUSE ? pos : len;  // positions that come from the cache
+  f32x4 kk[U][NV], vv[U][NV];
+  bool valid[U];
+  auto issue = [&](int base) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {  // unconditional, clamped loads: the whole batch in flight together
       const int idx = base + (u * W + wave) * PP + sub;
-      valid[u] = idx < len;
-      const size_t off = (size_t)(valid[u] ? idx : len - 1) * kv_dim;
+      valid[u] = idx < ncache;
+      const size_t off = (size_t)(valid[u] ? idx : ncache > 0 ? ncache - 1 : 0) * kv_dim;
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
         kk[u][v] = *reinterpret_cast<const f32x4*>(kbase + off + 64 * v);
         vv[u][v] = *reinterpret_cast<const f32x4*>(vbase + off + 64 * v);
       }
     }
+  };
+  f32x4 qf[G][NV], acc[G][NV], kn[1][NV], vn[1][NV];
+  float m[G], l[G];
+  if constexpr (FUSE) {
+    static_assert((G + 2) * HD / 4 <= 64 * NW, "four numbers a thread");
+    const int part_of = tid / (HD / 4), d = tid % (HD / 4) * 4;  // head of the group, then key, then value
+    const bool isq = part_of < G, isk = part_of == G, there = part_of < G + 2;
+    const size_t o = isq ? ((size_t)tok * a.nh + head0 + part_of) * HD + d : ((size_t)tok * a.nkv + kvh) * HD + d;
+    f32x4 x = {}, cs = {};
+    GemmParts pq = a.pq, pk = a.pk, pv = a.pv;
+    asm("" : "+s"(pq.part), "+s"(pq.n), "+s"(pq.S), "+s"(pk.part), "+s"(pk.n), "+s"(pk.S), "+s"(pv.part), "+s"(pv.n), "+s"(pv.S));  // (values, not a place to load from)
+    if (there) {
+      const GemmParts g[1] = {{isq ? pq.part : isk ? pk.part : pv.part, isq ? pq.n : isk ? pk.n : pv.n, isq ? pq.S : isk ? pk.S : pv.S}};
+      cs = *reinterpret_cast<const f32x4*>(a.table + (size_t)pos * HD + d);
+      f32x4 sum[1][1];
+      if (g[0].S) tl_parts_sum(g, o, sum);
+      else sum[0][0] = *reinterpret_cast<const f32x4*>((isq ? a.q : isk ? a.k : a.v) + o);
+      x = sum[0][0];
+    }
+    issue(0);
+    if (there) {
+      if (isq || isk) {
+        float r[4];
+        rot2(x[0], x[1], cs[0], cs[1], r[0], r[1]);
+        rot2(x[2], x[3], cs[2], cs[3], r[2], r[3]);
+        x = f32x4{r[0], r[1], r[2], r[3]};
+      }
+      *reinterpret_cast<f32x4*>(isq ? outbuf + part_of * HD + d : knew + (isk ? 0 : HD) + d) = x;
+      if (!isq && blockIdx.z == 0)
+        *reinterpret_cast<f32x4*>((isk ? a.kw : a.vw) + (size_t)sq * a.seq_stride + (size_t)pos * kv_dim + (size_t)kvh * HD + d) = x;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      kn[0][v] = *reinterpret_cast<const f32x4*>(knew + 64 * v + 4 * ln);
+      vn[0][v] = *reinterpret_cast<const f32x4*>(knew + HD + 64 * v + 4 * ln);
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      qf[g][v] = *reinterpret_cast<const f32x4*>(FUSE ? outbuf + g * HD + 64 * v + 4 * ln : a.q + ((size_t)tok * a.nh + head0 + g) * HD + 64 * v + 4 * ln);
+      acc[g][v] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    m[g] = -INFINITY;
+    l[g] = 0.f;
+  }
+  // cnt rows a lane group into the running state
+  auto fold = [&](const auto& kk, const auto& vv, const auto& valid, auto cnt_c) __attribute__((always_inline)) {
+    constexpr int U = decltype(cnt_c)::value;
     if constexpr (G > 1) {
       // the exps of the heads once per quad (lane l: head l % 4, with fewer than four the spare lanes repeat the last; DPP quad
       // broadcasts) instead of identically in all 16 lanes of a row: as in tl_attn.hip's fold (same values, 1 / G of the exps)
@@ -262,7 +313,7 @@ __global__ __launch_bounds__(64 * NW) void attn_batch_decode_kernel(BatchAttnArg
       apply(std::integral_constant<int, 1>{});
       if constexpr (G > 2) apply(std::integral_constant<int, 2>{});
       if constexpr (G > 3) apply(std::integral_constant<int, 3>{});
-      continue;
+      return;
     }
 #pragma unroll
     for (int g = 0; g < G; ++g) {
@@ -294,6 +345,14 @@ __global__ __launch_bounds__(64 * NW) void attn_batch_decode_kernel(BatchAttnArg
           for (int e = 0; e < 4; ++e) acc[g][v][e] = fmaf(p, vv[u][v][e], acc[g][v][e]);
       }
     }
+  };
+  for (int base = 0; base < (wave < W ? ncache : 0); base += rows * U) {
+    if (!FUSE || base > 0) issue(base);
+    fold(kk, vv, valid, std::integral_constant<int, U>{});
+  }
+  if constexpr (FUSE) {
+    const bool one[1] = {sub == 0};
+    if (wave == W - 1) fold(kn, vn, one, std::integral_constant<int, 1>{});
   }
   // every row group's state -> an LDS record (folding the four groups of a wave in registers first is 2 x 10 LDS-path
   // shuffles per head and lane, and four exps per output element on top: as in tl_attn_body.h)
@@ -392,8 +451,12 @@ int launch_attn_h(const BatchAttnArgs& a, int T, hipStream_t s) {
   auto go = [&](auto g_c, int parts) {
     constexpr int G = decltype(g_c)::value;
     // 16, 24 and 28 workgroups of 32 CUs, 4 heads of 128 a workgroup, 4000 positions, four -> eight waves 148 -> 109, 149 -> 137, 153 -> 157 us
-    if ((long)a.nkv * T * parts * 4 <= tl_num_cus() * 3l) attn_batch_decode_kernel<HD, G, 8><<<dim3(a.nkv, T, parts), 512, 0, s>>>(a);
-    else attn_batch_decode_kernel<HD, G, 4><<<dim3(a.nkv, T, parts), 256, 0, s>>>(a);
+    const bool eight = (long)a.nkv * T * parts * 4 <= tl_num_cus() * 3l;
+    const dim3 grid(a.nkv, T, parts);
+    if (eight && a.table) attn_batch_decode_kernel<HD, G, 8, true><<<grid, 512, 0, s>>>(a);
+    else if (eight) attn_batch_decode_kernel<HD, G, 8, false><<<grid, 512, 0, s>>>(a);
+    else if (a.table) attn_batch_decode_kernel<HD, G, 4, true><<<grid, 256, 0, s>>>(a);
+    else attn_batch_decode_kernel<HD, G, 4, false><<<grid, 256, 0, s>>>(a);
   };
   switch (grp) {
     case 1: go(std::integral_constant<int, 1>{}, 1); break;
@@ -510,12 +573,30 @@ bool tl_batch_attn_half(int nh, int nkv, int hd) {
 
 int tl_launch_batch_attn(const float* q, const float* kc, const float* vc, size_t seq_stride, float* out, const int* pos_dev,
                          const int* seq_dev, int T, int nh, int nkv, int hd, int max_seq, int n_seq, float scale,
-                         hipStream_t s, void* planes, size_t plane_stride, int terms, int start_pos) {
+                         hipStream_t s, void* planes, size_t plane_stride, int terms, int start_pos, const BatchAttnNew* fresh) {
   TL_REQUIRE(tl_batch_attn_supported(nh, nkv, hd), "batched decode attention: unsupported head configuration %d/%d/%d", nh,
              nkv, hd);
   TL_REQUIRE(q && kc && vc && out && ((pos_dev && seq_dev) || (!pos_dev && !seq_dev && start_pos >= 0)) && T > 0 && T <= 65535,
              "batched decode attention: bad argument");
   BatchAttnArgs a = {q, kc, vc, seq_stride, out, pos_dev, seq_dev, nh, nkv, max_seq, n_seq, scale, nullptr, 0, nullptr, 0, 0, start_pos, nullptr};
+  if (fresh) {
+    const size_t kn = (size_t)T * nkv * hd;
+    size_t at = (size_t)q | (size_t)fresh->k | (size_t)fresh->v | (size_t)fresh->kc | (size_t)fresh->vc | (size_t)fresh->table;
+    for (const GemmParts* g : {&fresh->pq, &fresh->pk, &fresh->pv}) {
+      at |= g->S ? (size_t)g->part : 0;
+      TL_REQUIRE(!g->S || g->n == (g == &fresh->pq ? (size_t)T * nh * hd : kn), "batched decode attention: pending sums of another shape");
+    }
+    TL_REQUIRE(pos_dev && seq_dev && fresh->k && fresh->v && fresh->table && fresh->kc == kc && fresh->vc == vc && (at & 15) == 0 && (seq_stride & 3) == 0,
+               "batched decode attention: bad argument of a step's keys and values");
+    a.table = fresh->table;
+    a.k = fresh->k;
+    a.v = fresh->v;
+    a.kw = fresh->kc;
+    a.vw = fresh->vc;
+    a.pq = fresh->pq;
+    a.pk = fresh->pk;
+    a.pv = fresh->pv;
+  }
   if (planes && terms == TL_TERMS_HALF) {
     TL_REQUIRE(tl_batch_attn_half(nh, nkv, hd) && plane_stride >= tl_gemm_padded_tokens(T) * (size_t)nh * hd,
                "batched decode attention: activation planes too small or heads of parts of a super-block");

@@ -364,9 +364,17 @@ int tl_launch_batch_rope_kv(float* q, float* k, const float* v, float* kc, float
                             const GemmParts* pv = nullptr, int start_pos = 0);
 bool tl_batch_attn_supported(int nh, int nkv, int hd);
 bool tl_batch_attn_half(int nh, int nkv, int hd);  // planes of TL_TERMS_HALF come from the launch itself
+// a step's new keys and values, for tokens of a sequence each: q, k and v (or their pending sums) as the projections leave them; the attention
+// rotates them and writes the caches kc, vc itself (what tl_launch_batch_rope_kv does in front of it otherwise)
+struct BatchAttnNew {
+  const float *k, *v, *table;
+  float *kc, *vc;
+  GemmParts pq, pk, pv;
+};
 int tl_launch_batch_attn(const float* q, const float* kc, const float* vc, size_t seq_stride, float* out, const int* pos_dev,
                          const int* seq_dev, int T, int nh, int nkv, int hd, int max_seq, int n_seq, float scale,
-                         hipStream_t s, void* planes = nullptr, size_t plane_stride = 0, int terms = 0, int start_pos = 0);
+                         hipStream_t s, void* planes = nullptr, size_t plane_stride = 0, int terms = 0, int start_pos = 0,
+                         const BatchAttnNew* fresh = nullptr);
 // out[j] = x[rows_host[j]] + the pending sums there, rows of `width` floats (a multiple of 4)
 int tl_launch_gather_rows(const float* x, const GemmParts& pend, const int* rows_host, int n, int width, float* out, hipStream_t s);
 int tl_launch_batch_argmax_advance(const float* logits, int T, int V, int* tokens_dev, int* pos_dev, int* ids_out_dev,

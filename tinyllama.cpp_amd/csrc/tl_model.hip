@@ -1779,7 +1779,8 @@ extern "C" int tl_tp_local_group_prefill(tl_model* const* ms, int n, const int* 
 // generation loop needs no host round trip per step. Every sequence decodes exactly as it would alone (see tl_batch.hip
 // on the reference's history_len quirk). tp_size 1 only.
 // packed: that many row tiles of a packed chunk in bt.pack (0: token by token)
-static int batch_attn_half(tl_model* m, int l, int T, int packed, hipStream_t s) {
+// step: every token is a sequence's only one
+static int batch_attn_half(tl_model* m, int l, int T, int packed, bool step, hipStream_t s) {
   const tl_model_config& c = m->cfg;
   tl_model::Prefill& p = m->pf;
   LayerW& L = m->layers[l];
@@ -1790,9 +1791,14 @@ static int batch_attn_half(tl_model* m, int l, int T, int packed, hipStream_t s)
   (void)H;
   TL_TRY(split_residual(m, L.attn_norm, T, s));
   TL_TRY(qkv_deferred(m, L, T, s));
-  TL_TRY(tl_launch_batch_rope_kv(p.qb, p.kb, p.vb, m->bkc(l), m->bvc(l), m->kv_layer_elems, m->rope, m->bt.pos, m->bt.seq, T,
-                                 m->nh_l, m->nkv_l, hd, c.max_position_embeddings, m->bt.max_batch, s, &p.dq.got, &p.dk.got,
-                                 &p.dv.got));
+  // a step's attention rotates and stores what is new itself (TL_ATTN_STEP=0: a launch in front of it does, for A/B runs and tests)
+  const char* as = getenv("TL_ATTN_STEP");
+  const bool fused = step && !packed && tl_batch_attn_supported(m->nh_l, m->nkv_l, hd) && !(as && atoi(as) == 0);
+  const BatchAttnNew fresh = {p.kb, p.vb, m->rope, m->bkc(l), m->bvc(l), p.dq.got, p.dk.got, p.dv.got};
+  if (!fused)
+    TL_TRY(tl_launch_batch_rope_kv(p.qb, p.kb, p.vb, m->bkc(l), m->bvc(l), m->kv_layer_elems, m->rope, m->bt.pos, m->bt.seq, T,
+                                   m->nh_l, m->nkv_l, hd, c.max_position_embeddings, m->bt.max_batch, s, &p.dq.got, &p.dk.got,
+                                   &p.dv.got));
   // the attention output goes straight into the planes of the attn_output GEMM (no split launch; TL_ATTN_PLANES=0 keeps
   // the launch, for A/B runs and the bit-identity test)
   const char* ap = getenv("TL_ATTN_PLANES");
@@ -1801,11 +1807,12 @@ static int batch_attn_half(tl_model* m, int l, int T, int packed, hipStream_t s)
     TL_TRY(tl_launch_split(0, p.ab, nullptr, p.planes, ps, T, m->qd_l, terms, 0.f, s));
   } else if (terms == TL_TERMS_HALF ? !attn_half_planes(m) : ap && atoi(ap) == 0) {
     TL_TRY(tl_launch_batch_attn(p.qb, m->bkc(l), m->bvc(l), m->kv_layer_elems, p.ab, m->bt.pos, m->bt.seq, T, m->nh_l,
-                                m->nkv_l, hd, c.max_position_embeddings, m->bt.max_batch, scale, s));
+                                m->nkv_l, hd, c.max_position_embeddings, m->bt.max_batch, scale, s, nullptr, 0, 0, 0, fused ? &fresh : nullptr));
     TL_TRY(tl_launch_split(0, p.ab, nullptr, p.planes, ps, T, m->qd_l, terms, 0.f, s));
   } else {
     TL_TRY(tl_launch_batch_attn(p.qb, m->bkc(l), m->bvc(l), m->kv_layer_elems, p.ab, m->bt.pos, m->bt.seq, T, m->nh_l,
-                                m->nkv_l, hd, c.max_position_embeddings, m->bt.max_batch, scale, s, p.planes, ps, terms));
+                                m->nkv_l, hd, c.max_position_embeddings, m->bt.max_batch, scale, s, p.planes, ps, terms, 0,
+                                fused ? &fresh : nullptr));
   }
   return project_residual(m, L.q[TL_T_ATTN_OUTPUT], T, s);
 }
@@ -1910,12 +1917,12 @@ static int batch_layers_gemv(tl_model* m, int T, hipStream_t s) {
 // one step for the T tokens in bt.toks / bt.pos / bt.seq; ids_dev: [T] next ids (first maximum of each logits row);
 // advance: the ids become the next tokens and the positions move on (device-resident loop)
 // all layers for the T tokens in bt.toks / bt.pos / bt.seq: the residual stream ends up in pf.xb [T][hidden], its last projection maybe pending
-static int batch_layers(tl_model* m, int T, hipStream_t s, int packed = 0) {
+static int batch_layers(tl_model* m, int T, hipStream_t s, int packed, bool step) {
   TL_REQUIRE(T >= 1 && T <= m->pf.cap, "tl_model: a batched step of %d tokens exceeds the chunk workspaces (%d)", T, m->pf.cap);
   if (T <= gemv_most(m)) return batch_layers_gemv(m, T, s);
   TL_TRY(prefill_embed(m, m->bt.toks, T, s));
   for (int l = 0; l < m->cfg.num_hidden_layers; ++l) {
-    TL_TRY(batch_attn_half(m, l, T, packed, s));
+    TL_TRY(batch_attn_half(m, l, T, packed, step, s));
     TL_TRY(prefill_mlp_half(m, l, T, s));
   }
   return 0;
@@ -1999,7 +2006,7 @@ static int batch_step(tl_model* m, int T, int* ids_dev, bool advance, float* log
   const tl_model_config& c = m->cfg;
   tl_model::Prefill& p = m->pf;
   hipStream_t s = m->stream;
-  TL_TRY(batch_layers(m, T, s));
+  TL_TRY(batch_layers(m, T, s, 0, true));
   TL_TRY(batch_head(m, p.xb, T, s));
   TL_TRY(tl_launch_batch_argmax_advance(p.logits_all, T, c.vocab_size, advance ? m->bt.toks : nullptr, advance ? m->bt.pos : nullptr, ids_dev, s));
   return logits_host ? copy_to_caller(m, logits_host, p.logits_all, sizeof(float) * (size_t)T * c.vocab_size, s) : 0;
@@ -2159,7 +2166,7 @@ extern "C" int tl_model_batch_prefill_packed(tl_model* m, int n_tokens, const in
     TL_HIP(hipMemcpyAsync(m->bt.toks, tokens_host + c0, sizeof(int) * T, hipMemcpyHostToDevice, s));
     TL_HIP(hipMemcpyAsync(m->bt.pos, positions_host + c0, sizeof(int) * T, hipMemcpyHostToDevice, s));
     TL_HIP(hipMemcpyAsync(m->bt.seq, seq_idx_host + c0, sizeof(int) * T, hipMemcpyHostToDevice, s));
-    TL_TRY(batch_layers(m, T, s, packed));
+    TL_TRY(batch_layers(m, T, s, packed, false));
     rows.clear();  // runs of output rows that are in this chunk
     for (int j = 0; j < n_last; ++j) {
       const int r = last_rows_host[j] - c0;
