@@ -671,3 +671,31 @@ def test_residual_sum_in_front_of_the_next_product(env, width, heads, n_layers):
         assert rel_rms(got[-1], orc.forward(list(toks))) < FP32_TOL
         m.free()
     assert rel_rms(got[0], got[1]) < FP32_TOL
+
+
+@pytest.mark.parametrize("experts", [1, 2, 15, 16, 17, 33, 64, 65, 130])
+def test_router_choice_among_equals_and_without_numbers(env, experts):
+    """Choices of a row of lanes, of a wave and of more: logits that are their biases, with equal ones (the lower index first),
+    numbers that are none (never chosen while others are left) and as many choices as there are experts; softmax over the chosen in 64 bits
+    (an exp's and a quotient's roundings: some 1e-6)."""
+    capi, synth = env["capi"], env["synth"]
+    rng = np.random.default_rng(experts)
+    for kind in ("distinct", "equal", "none"):
+        for top in sorted({1, min(4, experts), min(16, experts), experts}):
+            b = rng.permutation(experts).astype(np.float32) / 8
+            if kind == "equal":
+                b = np.round(b).astype(np.float32)
+            if kind == "none":
+                if top > max(1, experts - 2) or experts < 2:
+                    continue
+                b[rng.integers(experts)] = np.nan
+            xd, wd, bd = dev(env, np.ones((2, 16), np.float32)), dev(env, synth.to_bf16(np.zeros((experts, 16), np.float32))), dev(env, b)
+            idd, wtd = env["engine"].DeviceBuffer(8 * top), env["engine"].DeviceBuffer(8 * top)
+            capi.check(capi.lib().tl_moe_route(xd.ptr, 2, 16, wd.ptr, bd.ptr, experts, top, idd.ptr, wtd.ptr, None), "tl_moe_route")
+            capi.check(capi.lib().tl_device_sync(), "sync")
+            order = np.lexsort((np.arange(experts), -np.where(np.isnan(b), -np.inf, b).astype(np.float64)))[:top]
+            z = b[order].astype(np.float64)
+            p = np.exp(z - z[0])
+            for t in range(2):
+                assert np.array_equal(idd.to_numpy(np.int32, (2, top))[t], order), (kind, top)
+                assert np.allclose(wtd.to_numpy(np.float32, (2, top))[t], p / p.sum(), rtol=4e-6, atol=1e-30), (kind, top)

@@ -60,9 +60,10 @@ __device__ __forceinline__ float tl_wave_max(float m) {
   tl_butterfly<FROM>([&](auto o) __attribute__((always_inline)) { m = fmaxf(m, tl_xor<decltype(o)::value>(m)); });
   return m;
 }
-// the largest value of a wave and its index, the lower index among equals, as seen from each lane
-__device__ __forceinline__ void tl_wave_best(float& v, int& i) {
-  tl_butterfly<32>([&](auto o) __attribute__((always_inline)) {
+// the largest value of a wave (FROM 32; 8: of each row of 16) and its index, the lower index among equals, as seen from each lane
+template <int FROM>
+__device__ __forceinline__ void tl_lanes_best(float& v, int& i) {
+  tl_butterfly<FROM>([&](auto o) __attribute__((always_inline)) {
     const float ov = tl_xor<decltype(o)::value>(v);
     const int oi = tl_xor<decltype(o)::value>(i);
     if (ov > v || (ov == v && oi < i)) {
@@ -71,3 +72,4 @@ __device__ __forceinline__ void tl_wave_best(float& v, int& i) {
     }
   });
 }
+__device__ __forceinline__ void tl_wave_best(float& v, int& i) { tl_lanes_best<32>(v, i); }

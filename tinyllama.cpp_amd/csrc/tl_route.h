@@ -19,6 +19,36 @@ __device__ __forceinline__ void tl_route_select(float* z, int experts, int top, 
       for (int e = lane; e < experts; e += 64) all += expf(z[e] - top_z);
       all = tl_wave_sum(all);
     }
+    // A lane an expert (up to 64): the rounds stay in registers, over one row of 16 lanes where these hold all experts, and the weights' exps come
+    // behind them. Through LDS a round was a store, a load and an exp more: 4 of 16 experts chosen behind a residual norm of 2048, 6.6 us, here 5.6
+    if (experts <= 64) {
+      auto choose = [&](auto from_c) __attribute__((always_inline)) {
+        constexpr int FROM = decltype(from_c)::value;
+        float v = lane < experts ? z[lane] : NAN, mine_z = 0.0f, largest = 0.0f;
+        int id = -1;
+        for (int j = 0; j < top; ++j) {
+          float bv = v > -INFINITY ? v : -INFINITY;
+          int bi = v == v ? lane : 0x7fffffff;
+          tl_lanes_best<FROM>(bv, bi);
+          if (bi == 0x7fffffff) bi = 0;  // only when every logit is NaN
+          if (j == 0) largest = bv;
+          mine_z = lane == j ? bv : mine_z;
+          id = lane == j ? bi : id;
+          v = lane == bi ? -INFINITY : v;  // chosen: out of the next rounds
+        }
+        const float p = expf(mine_z - largest);
+        float sum = 0.0f;
+        for (int j = 0; j < top; ++j) sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), j));
+        if (over_all) sum = all;  // (the first choice is the largest logit)
+        if (lane < top) {
+          ids[lane] = id;
+          wts[lane] = p / sum * scale;
+        }
+      };
+      if (experts <= 16) choose(std::integral_constant<int, 8>{});
+      else choose(std::integral_constant<int, 32>{});
+      return;
+    }
     // `top` rounds: the lanes scan the experts not yet chosen for the largest logit (lower index wins among equals)
     float mx = 0.0f, denom = 0.0f, mine = 0.0f;
     int my_id = -1;
