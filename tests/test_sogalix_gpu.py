@@ -631,7 +631,7 @@ def test_configurations_drawn_at_random(env, seed, tmp_path):
     s.close()
 
 
-@pytest.mark.parametrize("heads,dim", [(3, 64), (2, 128), (33, 64), (17, 128)])  # (33 and 17: more than half the chip's CUs with 16 lanes a column)
+@pytest.mark.parametrize("heads,dim", [(3, 64), (2, 128)])
 def test_generalized_delta_rule_of_aligned_rows(env, heads, dim):
     """Rows at 16 bytes take the unrolled scan: portions below, at and above its stages of 16 and 8 tokens, against the recurrence
     in 64 bits (a few 32-bit roundings a token, decayed by w >= 0.54: some 1e-6 of the outputs' size)."""
@@ -749,3 +749,10 @@ def test_large_products_give_the_same_bits_from_a_plane(env, monkeypatch):
     m.reset_kv()
     assert np.isfinite(got).all() and np.array_equal(got, m.prefill_rows(toks, 0))
     m.free()
+
+
+@pytest.mark.parametrize("heads,dim", [(32, 64), (33, 64), (16, 128), (17, 128)])
+def test_generalized_delta_rule_on_both_sides_of_half_the_chip(env, heads, dim):
+    """With 16 lanes a column, 32 heads of 64 and 16 of 128 are 128 workgroups, half of 256 CUs: the last that take 32 lanes, and the first that
+    take 16. The portions and bounds of test_generalized_delta_rule_of_aligned_rows."""
+    test_generalized_delta_rule_of_aligned_rows(env, heads, dim)
