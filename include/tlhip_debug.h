@@ -47,6 +47,8 @@ int tl_debug_gemm_px_launches(long long* count_out);
 int tl_debug_split_launches(long long* count_out);
 /* ... and attentions by the two-part f16 kernels (tl_hattn.hip): one a layer of a prompt's chunk that takes them */
 int tl_debug_half_attention_launches(long long* count_out);
+/* ... and GEMV launches with a norm whose input is not staged from registers as a whole (graph captures count once) */
+int tl_debug_gemv_general_norms(long long* count_out);
 
 /* Test hook (no counterpart in the reference): tl_matmul_q through the f16 form that a model's chunks and multi-sequence steps
  * take (tl_hgemm.hip), any number of tokens, in a workgroup shape (0: 64 rows x 16 tokens, 1: 128 x 32, 2: 256 x 64, 3: in waves of 64

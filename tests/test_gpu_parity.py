@@ -353,6 +353,34 @@ def test_decode_stages_its_input_in_any_number_of_pieces(E, pkg, oracle, hidden,
     om.close()
 
 
+@pytest.mark.parametrize("hidden,heads,mix,general", [
+    (6144, 48, "q4_k_m", 0), (8192, 64, "q4_k_m", 0), (8192, 64, "q6_k", 0), (8192, 64, "q8_0", 0), (9216, 72, "q4_k_m", 0), (9472, 74, "q6_k", 1)])
+def test_wide_norms_are_staged_from_registers(E, pkg, oracle, hidden, heads, mix, general):
+    """A step's launches with a norm hold up to three pieces of their input and its weights a thread in registers (9216 columns in the twelve
+    waves of Q4_K and Q6_K); wider ones take the general form. Which form ran, and its logits."""
+    import ctypes as C
+    from tinyllama_cpp_amd.capi import check, lib
+    count = C.c_longlong()
+
+    def general_norms():
+        check(lib().tl_debug_gemv_general_norms(C.byref(count)))
+        return count.value
+
+    cfg = dict(pkg.synth.SHAPES["tiny"], hidden=hidden, n_heads=heads, n_kv_heads=2, inter=3072, n_layers=1, vocab=6144, max_pos=16)
+    cfg, tensors = pkg.synth.build_model(cfg, mix, seed=hidden)
+    before = general_norms()
+    m = E.Model(cfg).load(tensors)  # (the step may be captured here)
+    om = OracleModel(oracle, cfg, tensors)
+    prompt = np.array([5, 4096, 77], np.int32)
+    want = om.generate(prompt, 1, penalty=1.0, dump_logits=True)[1][0]
+    for pos, tok in enumerate(prompt):
+        logits, _ = m.decode(int(tok), pos)
+    assert (general_norms() > before) == bool(general)
+    assert close(logits, want, LOGIT_TOL).all(), np.abs(logits - want).max()
+    m.free()
+    om.close()
+
+
 def test_model_tinyllama_q8_0_prefill_then_decode(E, pkg, oracle):
     """TinyLlama-1.1B Q8_0 through the generate loop's other branch (api.cpp:601-694): a 40-token prompt goes through the batched
     prefill, then greedy decode with the default penalty 1.3; ids and the first sampled position's logits vs the oracle."""

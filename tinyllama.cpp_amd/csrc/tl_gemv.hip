@@ -29,6 +29,8 @@
 
 #include "tl_internal.h"
 
+#include <atomic>
+
 #include "tl_chunk.h"
 #include "tl_attn_body.h"
 
@@ -1091,11 +1093,17 @@ static int gemv_launch_sx(const Launch& L, hipStream_t s) {
                                                                                          L.t[1], L.t[2], L.nsegA, L.wavesA, GemvPad{});
   return 0;
 }
-// The step's own launches know their input: how many pieces a thread stages, a norm or none (other sizes, Q8_K and launches that carry an
-// exchange take the general form). A launch's prologue is bound by its instructions, sixteen waves sharing four SIMDs: with four clamped
-// pieces a thread, both cases of the norm, two IEEE divisions and a root in front of the staged values, and a second barrier, 270 a wave; now 110.
+// The step's own launches know their input: how many pieces a thread stages (with a norm up to three: 9216 columns in twelve waves, 12288 in
+// sixteen), a norm or none (other sizes, Q8_K and launches that carry an exchange take the general form). A launch's prologue is bound by its
+// instructions, sixteen waves sharing four SIMDs: with four clamped pieces a thread, both cases of the norm, two IEEE divisions and a root in
+// front of the staged values, and a second barrier, 270 a wave; now 110.
 // us with a norm, before / after: 1.1B Q4_K_M q | k | v 4.0 / 3.45, gate and up 6.9 / 5.9, 3B Q6_K 7.05 / 6.05 and 11.1 / 10.4, 8B Q4_K_M 6.9 /
 // 5.6 and 15.5 / 14.8; attn_output with 32-bit record addresses and one matrix at compile time 4.65 / 4.1, 6.7 / 6.4, 6.95 / 6.5
+// The general form holds norm weights of two pieces and loads a third's behind the first weights. Four layers of 8192 columns, all launches in
+// the general form and sixteen waves / the third piece in the general form / in registers, us a token: Q4_K_M (three pieces in twelve waves) 490
+// / 484 / 480, Q6_K 595 / 580 / 578; three of 12288 in Q8_0 (three pieces in sixteen), the last two, 670 / 663. (Two pieces in sixteen waves, 8192
+// columns: Q4_K_M 479, Q6_K 586.)
+static std::atomic<long long> g_gemv_general_norms{0};  // tl_debug_gemv_general_norms
 template <int TA, int TB, bool PAIR, int ROLE, bool STAMP = false, int RA = 0, bool PEER = false>
 static int gemv_launch_ra(const Launch& L, hipStream_t s) {
   const int pieces = (L.v.cols / 4 + L.threads - 1) / L.threads;
@@ -1103,6 +1111,7 @@ static int gemv_launch_ra(const Launch& L, hipStream_t s) {
     if constexpr (PAIR || ROLE == GEMV_QKV || ROLE == GEMV_LM_HEAD) {
       if (L.v.norm_w && pieces <= 1) return gemv_launch_sx<TA, TB, PAIR, ROLE, STAMP, RA, PEER, 1>(L, s);
       if (L.v.norm_w && pieces <= 2) return gemv_launch_sx<TA, TB, PAIR, ROLE, STAMP, RA, PEER, 2>(L, s);
+      if (L.v.norm_w && pieces <= 3) return gemv_launch_sx<TA, TB, PAIR, ROLE, STAMP, RA, PEER, 3>(L, s);
     }
     if constexpr (RA == 0 && (ROLE == GEMV_DOWN || ROLE == GEMV_ATTN_OUT_COMBINE)) {
       if (L.parts > 1) {
@@ -1119,6 +1128,7 @@ static int gemv_launch_ra(const Launch& L, hipStream_t s) {
       if (!L.v.norm_w && pieces <= 4) return gemv_launch_sx<TA, TB, PAIR, ROLE, STAMP, RA, PEER, -4>(L, s);
     }
   }
+  if (L.v.norm_w) g_gemv_general_norms.fetch_add(1, std::memory_order_relaxed);
   return gemv_launch_sx<TA, TB, PAIR, ROLE, STAMP, RA, PEER, 0>(L, s);
 }
 template <int TA, int TB, bool PAIR, int ROLE, bool STAMP = false>
@@ -1550,6 +1560,12 @@ __global__ void chain_gen_bump_kernel(unsigned* gen) { *gen = *gen + 1u; }
 int tl_launch_chain_gen_bump(unsigned* gen, hipStream_t s) {
   chain_gen_bump_kernel<<<1, 1, 0, s>>>(gen);
   TL_HIP(hipGetLastError());
+  return 0;
+}
+
+extern "C" int tl_debug_gemv_general_norms(long long* count_out) {
+  TL_REQUIRE(count_out, "tl_debug_gemv_general_norms: null argument");
+  *count_out = g_gemv_general_norms.load(std::memory_order_relaxed);
   return 0;
 }
 
