@@ -501,11 +501,10 @@ struct StepMeta {
 // CHAIN (a task of a chain launch): x and the first residual values are loaded only AFTER the wait for the predecessor
 // task, which follows the first weight loads; activation loads and stores take their sc1 forms.
 // AHD > 0 (with CHAIN): the launch carries its layer's attention (fused_attention_phase<AHD, AG>) in place of the wait.
-// KS: a wave has one row group at most and of that the spans sp0 .. sp1 - 1 only; the waves of a row group, `rows_waves` apart, leave their
-// sums in LDS (one matrix with a residual, no norm: the reduction scratch in front of the x image is free) and the first of them adds
-// them up.
+// KS: a wave has one row group at most and of that one span; the waves of a row group, `row_waves` apart, leave their sums in LDS (one matrix
+// with a residual, no norm: the reduction scratch in front of the x image is free) and the first of them adds them up.
 struct KPart {
-  int sp0, sp1, wave, row_waves, parts;
+  int span, wave, row_waves, spans;
 };
 template <int TYPE, bool PAIR, bool ONE, bool RESID, int SX, bool XATTN, bool STAMP, bool PEER = false, bool CHAIN = false, int AHD = 0,
           int AG = 0, bool KS = false>
@@ -515,7 +514,7 @@ __device__ __forceinline__ void run_class(const Segs& g, const GemvVec& a, XRegs
   static_assert(!KS || (ONE && RESID && !PEER && !CHAIN && !STAMP && (XATTN || SX < 0)), "");
   const float* xs = smem + XS_SCRATCH;
   const int nchunks = a.cols >> 5;
-  const int nspans = KS ? kp.sp1 : (nchunks + 63) >> 6;
+  const int nspans = (nchunks + 63) >> 6;
   // PEER: this wave's slice of the stash behind the x image, and the row groups it has finished
   float* stash = smem + XS_SCRATCH + nchunks * XS_STRIDE + 2 * peer_wave * a.peer_gpw;
   int ndone = 0;
@@ -531,7 +530,7 @@ __device__ __forceinline__ void run_class(const Segs& g, const GemvVec& a, XRegs
     if (KS) __syncthreads();
     return;
   }
-  int irg = first, isp = KS ? kp.sp0 : 0;
+  int irg = first, isp = KS ? kp.span : 0;
   QW wa = g.w0, wb = PAIR ? g.w1 : g.w0;
   int ra = 0, rb = 0;
   float* out = g.o0;
@@ -553,10 +552,10 @@ __device__ __forceinline__ void run_class(const Segs& g, const GemvVec& a, XRegs
     }
     st.c0.load(wa, ra, cc);
     st.c1.load(wb, rb, cc);
-    if (++isp == nspans) {  // advance the issue cursor (scalar work, overlaps the loads)
+    if (!KS && ++isp == nspans) {  // advance the issue cursor (scalar work, overlaps the loads)
       isp = 0;
       irg += stride;
-      if (!KS && irg < total) group_of<PAIR, ONE>(g, irg, wa, wb, ra, rb, out);
+      if (irg < total) group_of<PAIR, ONE>(g, irg, wa, wb, ra, rb, out);
     }
   };
   auto consume = [&](const Step<TYPE>& st, const StepMeta& m) {
@@ -575,7 +574,7 @@ __device__ __forceinline__ void run_class(const Segs& g, const GemvVec& a, XRegs
     const float d1 = st.c1.dot(x, sums[0], sums[1], cc & 7);
     acc0 += act ? d0 : 0.0f;
     acc1 += act ? d1 : 0.0f;
-    if (m.sp == nspans - 1) {  // row group complete: reduce, epilogue, store
+    if (KS || m.sp == nspans - 1) {  // row group complete: reduce, epilogue, store
       float y0 = wave_sum_lane63(acc0);
       float y1 = wave_sum_lane63(acc1);
       if (NORM) {
@@ -633,7 +632,7 @@ __device__ __forceinline__ void run_class(const Segs& g, const GemvVec& a, XRegs
   nf = stage_x_finish<SX, XATTN, CHAIN>(a, xr, smem);
   if constexpr (CHAIN) chain_stamp(cw, 3);
   if (STAMP) ts[4] = __builtin_readcyclecounter();
-  while (irg < total) {
+  while (!KS && irg < total) {
     issue(nxt, mn);
     consume(cur, mc);
     if (STAMP && ts[5] == 0) ts[5] = __builtin_readcyclecounter();
@@ -648,7 +647,7 @@ __device__ __forceinline__ void run_class(const Segs& g, const GemvVec& a, XRegs
     __syncthreads();
     if (kp.wave < kp.row_waves && lane < 2 && ra0 + lane < wa.rows) {
       float y = smem[2 * kp.wave + lane];
-      for (int p = 1; p < kp.parts; ++p) y += smem[2 * (kp.wave + p * kp.row_waves) + lane];
+      for (int p = 1; p < kp.spans; ++p) y += smem[2 * (kp.wave + p * kp.row_waves) + lane];
       stg_f32(out + ra0 + lane, (lane ? cur.r1 : cur.r0) + y);
     }
   }
@@ -874,11 +873,11 @@ __device__ __forceinline__ void gemv_body(const GemvSeg& sg0, const GemvSeg& sg1
     const int wA = TB == TL_NONE ? nwaves : wavesA;
     const int total = PAIR || ONE ? t0 : (nsegA == 1 ? t0 : (nsegA == 2 ? t0 + t1 : t0 + t1 + t2));
     const Segs g = {sg0.w, sg1.w, sg2.w, sg0.out, sg1.out, sg2.out, t0, nsegA >= 2 ? t1 : 0x3fffffff};
-    if constexpr (KS) {  // wavesA: waves of a part; t1: 4096 / wavesA rounded up; t2: parts
-      const int part = (int)((unsigned)(wave * t1) >> 12), spans = ((a.cols >> 5) + 63) >> 6;
-      const KPart kp = {part * spans / t2, (part + 1) * spans / t2, wave, wavesA, t2};
+    if constexpr (KS) {  // wavesA: waves of a span; t1: 4096 / wavesA rounded up; t2: spans
+      const int span = (int)((unsigned)(wave * t1) >> 12);
+      const KPart kp = {span, wave, wavesA, t2};
       run_class<TA, PAIR, ONE, RESID, SX, XATTN, false, false, false, 0, 0, true>(
-          g, a, xr, smem, part < t2 ? (wave - part * wavesA) * a.grid + bid : total, total, total, lane, ts, 0, wave, nullptr, kp);
+          g, a, xr, smem, span < t2 ? (wave - span * wavesA) * a.grid + bid : total, total, total, lane, ts, 0, wave, nullptr, kp);
     } else if constexpr (RA > 0)
       run_class_flat<TA, PAIR, ONE, RESID, SX, XATTN, RA>(g, a, xr, smem, wave * a.grid + bid, a.grid * wA, total, lane);
     else
@@ -1078,7 +1077,7 @@ struct Launch {
   int nsegA, wavesA;
   int grid, threads;
   size_t lds;
-  int parts;  // > 1: the spans of a row group are dealt to so many waves, wavesA apart
+  int parts;  // > 1: a row group's spans, so many, go to a wave each, wavesA apart
   int ra;  // 0: span steps; 2 / 4: flattened steps with that many rows per stream and group
 };
 
@@ -1118,9 +1117,8 @@ static int gemv_launch_ra(const Launch& L, hipStream_t s) {
         Launch K = L;
         K.t[1] = (4096 + L.wavesA - 1) / L.wavesA;
         K.t[2] = L.parts;
-        if constexpr (ROLE == GEMV_ATTN_OUT_COMBINE) return gemv_launch_sx<TA, TB, PAIR, ROLE, STAMP, RA, PEER, 0, true>(K, s);
-        else return pieces <= 2 ? gemv_launch_sx<TA, TB, PAIR, ROLE, STAMP, RA, PEER, -2, true>(K, s)
-                                : gemv_launch_sx<TA, TB, PAIR, ROLE, STAMP, RA, PEER, -4, true>(K, s);
+        // (four waves a span and more, of 512 pieces: two a thread at most)
+        return gemv_launch_sx<TA, TB, PAIR, ROLE, STAMP, RA, PEER, ROLE == GEMV_DOWN ? -2 : 0, true>(K, s);
       }
     }
     if constexpr (ROLE == GEMV_DOWN) {
@@ -1311,7 +1309,7 @@ static int gemv_plan(const GemvArgs& a, Launch& L, int* role_out, bool* classB_o
   // values few instructions). ffn_down in us: 2048 x 5632 in 4 waves 5.4 (Q4_K / Q6_K mix), 6.2 (Q8_0), in 8 4.9 and 5.4, 11 4.65 and
   // 5.1; 3072 x 8192 (Q6_K) in 6 7.4, in 16 7.0; 4096 x 14336 in 8 10.5, in 16 10.0.
   // Row groups of a few spans and few of them: each span to a wave of its own, so that all loads of the launch are in flight at once (1.1B
-  // ffn_down, 3 spans, 4 -> 12 waves: Q4_K_M 4.65 -> 4.5 us, Q8_0 5.1 -> 4.95; 3B attn_output in Q6_K, 2 spans, 6 -> 12 waves: 6.45 -> 6.1; not
+  // ffn_down, 3 spans, 4 -> 12 waves: Q4_K_M 4.65 -> 4.15 us, Q8_0 5.1 -> 4.85; 3B attn_output in Q6_K, 2 spans, 6 -> 12 waves: 6.45 -> 6.0; not
   // in sixteen waves: 8B attn_output 6.5 -> 6.75; nor in parts of several spans: 8B ffn_down 10.2 -> 10.5, 3B's 6.95 either way)
   const int spans = (a.cols / 32 + 63) / 64;
   const int most_parts = gemv_row_waves(TL_Q4_K) / waves;
@@ -1511,8 +1509,8 @@ int tl_chain_plan(const GemvArgs& a, void* task_out, size_t* lds_out, int pred_n
     t.t[i] = L.t[i];
   }
   t.a = L.v;
-  // every wave of the persistent workgroup takes part in every task (same barriers for all), whatever a launch of its own
-  // would take; a row's sum does not depend on the wave that forms it
+  // every wave of the persistent workgroup takes part in every task (same barriers for all), whatever a launch of its own would take. A row's
+  // sum is the same whichever wave forms it, but a launch of its own that deals a row group's spans to waves adds them in another order
   t.a.nthr = GEMV_MAX_THREADS;
   t.a.grid = L.grid;
   t.nsegA = L.nsegA;
