@@ -385,8 +385,8 @@ def test_merged_and_separate_launches_round_alike(pkg, monkeypatch, mix, n):
 
 @pytest.mark.parametrize("heads,kv", [(8, 4), (4, 4)])
 def test_two_formats_in_one_launch(pkg, monkeypatch, heads, kv):
-    """q | k in Q4_K and v in Q6_K share a launch, in every workgroup shape (tokens around 8, 16, 32 and 64, and so many that waves take 64
-    rows), with rows that end inside a tile and K slices: the same bits as a launch of each with the shared launch's shapes and slices
+    """q | k in Q4_K and v in Q6_K share a launch, tokens around 8, 16, 32 and 64 and many more, in the workgroup shapes of narrow matrices (the
+    next test has those of wide ones), with rows that end inside a tile and K slices: the same bits as a launch of each with the shared launch's shapes and slices
     (TL_GEMM_MERGE=0), whose products are held against float64 elsewhere."""
     from tinyllama_cpp_amd import engine as E
     E.init(0)
@@ -402,6 +402,40 @@ def test_two_formats_in_one_launch(pkg, monkeypatch, heads, kv):
             monkeypatch.setenv("TL_GEMM_MERGE", merge)
             m.reset_kv()
             got.append(np.array(m.prefill(toks, 0, all_logits=True)[1]))
+        assert np.array_equal(got[0], got[1]), (n, np.abs(got[0].astype(np.float64) - got[1]).max())
+    m.free()
+
+
+@pytest.mark.parametrize("heads,tokens", [(32, {8: 5, 20: 1, 40: 1, 63: 1, 844: 3, 900: 3, 1200: 3, 1350: 3}), (40, {8: 6, 9: 7, 16: 7, 130: 3, 650: 3}),
+                                          (64, {8: 6, 9: 7, 16: 7, 17: 1, 32: 1, 33: 2, 200: 3, 450: 3})])
+def test_two_formats_in_one_launch_of_wide_matrices(pkg, monkeypatch, heads, tokens):
+    """As above in the shapes that wide matrices take: 128 rows x 32 tokens (1), waves of 64 rows in Q4_K with twice the rows of a Q6_K tile
+    beside them (3), 128 rows x 8 and x 16 tokens (6 and 7), one and several K slices of either format; the shape that ran is counted."""
+    import ctypes as C
+    from tinyllama_cpp_amd import engine as E
+    from tinyllama_cpp_amd.capi import check, lib
+    E.init(0)
+    cfg, tensors = pkg.synth.build_model(dict(hidden=heads * 128, inter=512, n_heads=heads, n_kv_heads=8, n_layers=1, vocab=64, max_pos=1408, eps=1e-5,
+                                              rope_theta=10000.0), "q4_k_m", seed=16)
+    m = E.Model(cfg).load(tensors)
+    rng = np.random.default_rng(heads)
+    counts = (C.c_longlong * 9)()
+
+    def launches():
+        check(lib().tl_debug_half_pair_launches(counts))
+        return np.array(counts)
+
+    for n, shape in tokens.items():
+        toks = rng.integers(0, cfg["vocab"], n).astype(np.int32)
+        got = []
+        for merge in ("0", "1"):
+            monkeypatch.setenv("TL_GEMM_MERGE", merge)
+            m.reset_kv()
+            before = launches()
+            every = n <= 512  # (chunks whose logits are all asked for end there)
+            logits = m.prefill(toks, 0, all_logits=True)[1] if every else m.prefill(toks, 0)
+            got.append(np.concatenate([np.ravel(logits)] + [np.ravel(x) for i in range(0, n, 5) for x in m.kv_cache(0, i)]))  # (in every column of a tile)
+            assert np.array_equal(np.flatnonzero(launches() - before), [shape] if merge == "1" else []), (n, merge)
         assert np.array_equal(got[0], got[1]), (n, np.abs(got[0].astype(np.float64) - got[1]).max())
     m.free()
 

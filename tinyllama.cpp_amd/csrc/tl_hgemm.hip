@@ -22,6 +22,7 @@
 // the 32-weight chunk 2 s + h (one 16-byte load), of a Q8 step 16 of the 32 bytes of a chunk; the eight columns of an
 // operand are in the order [0 2 1 3 4 6 5 7], which is what masking a dword into 16-bit halves gives without moving a
 // byte, and which the activation planes are written in.
+#include <atomic>
 #include <type_traits>
 
 #include "tl_internal.h"
@@ -1211,6 +1212,7 @@ int hgemm_typed(const QW* w, int n, const HgemmPlan& p, const HAct& act, float* 
   if (shape == 8) return hgemm_go<TYPE, 8>(g, blocks, s);
   return hgemm_go<TYPE, 4>(g, blocks, s);
 }
+std::atomic<long long> g_pair_launches[HGEMM_SHAPES];  // of either shape of Q4_K (tl_debug_half_pair_launches)
 template <int V6, int V4>
 int hgemm_pair_go(const HPair& g, int blocks, hipStream_t s) {
   static TlDeviceOnce lds_raised;
@@ -1283,6 +1285,7 @@ int tl_launch_hgemm_pair(const QW* w4, int n4, const QW& w6, const void* planes,
   for (const HgemmPlan& p : {p4, p6})
     TL_REQUIRE(p.S >= 1 && (p.S - 1) * ((nsb + p.S - 1) / p.S) < nsb && p.shape >= 0 && p.shape < HGEMM_SHAPES && p6.shape == (p4.shape == 3 ? 2 : p4.shape),
                "half-plane GEMM: shape %d, %d K slices of %d super-blocks", p.shape, p.S, nsb);
+  g_pair_launches[p4.shape].fetch_add(1, std::memory_order_relaxed);
   const HAct act = hact(planes, ps, T);
   HPair g = {};
   g.first = hgemm_grid(g.q6, &w6, 1, hgemm_shape(TL_Q6_K, p6.shape), act, &out6, nullptr, T, p6.S);
@@ -1299,6 +1302,11 @@ int tl_launch_hgemm_pair(const QW* w4, int n4, const QW& w6, const void* planes,
     default: break;
   }
   TL_REQUIRE(false, "half-plane GEMM: shape %d has no launch of two formats", p4.shape);
+  return 0;
+}
+extern "C" int tl_debug_half_pair_launches(long long* counts_out) {
+  TL_REQUIRE(counts_out, "tl_debug_half_pair_launches: null argument");
+  for (int i = 0; i < HGEMM_SHAPES; ++i) counts_out[i] = g_pair_launches[i].load(std::memory_order_relaxed);
   return 0;
 }
 int tl_launch_hgemm(const QW* w, int n, const void* planes, size_t ps, float* const* out, const float* resid, int T, const HgemmPlan& p,
