@@ -1065,6 +1065,10 @@ constexpr HFew HGEMM_FEW[HGEMM_SHAPES] = {
 // and 65 to 2048 tokens, it is taken as often as where it ran in pairs of 256 rows (at its own 7.4 it would be taken in a sixth more of
 // them, and its single chain of sums rounds more: 2.1e-7 against 1.7e-7 at 2048 columns)
 constexpr float HGEMM_US[] = {0.f, 0.f, 4.25f, 7.8f, 5.0f}, HGEMM_US_3_Q8_K = 9.0f;
+constexpr float HGEMM_US_Q6_K[] = {0.f, 0.f, 6.3f, 0.f, 6.85f}, HGEMM_US_Q8_0[] = {0.f, 0.f, 5.5f, 0.f, 6.0f};
+constexpr float HGEMM_ENDS = 0.6f;  // start and end of a workgroup of these two, in its super-blocks
+// partial sums: of a slice, and of a number of it (Q6_K and Q8_0 beyond 64 tokens: 1.4e-6)
+constexpr float HGEMM_SLICE_US = 0.3f, HGEMM_SUM_US = 2e-6f;
 // Price of a launch over T tokens of n workgroups of `per` super-blocks, and of S slices' partial sums of `outputs` numbers.
 // Q4_K and Q8_K beyond 64 tokens: rounds over the chip x (super-blocks + start and end) + the partial sums written and read once at about
 // 4 TB/s. Q6_K (a third product, longer unpacking) and Q8_0 (16 additions and FMAs a block): the
@@ -1074,16 +1078,16 @@ constexpr float HGEMM_US[] = {0.f, 0.f, 4.25f, 7.8f, 5.0f}, HGEMM_US_3_Q8_K = 9.
 float hgemm_price(int cus, int type, int shape, int T, long n, int per, int S, float outputs) {
   const HShape q = hgemm_shape(type, shape);
   const long most = (n + cus - 1) / cus, rounds = (most + q.percu - 1) / q.percu;
-  const float sums = S > 1 ? (float)S * (0.3f + outputs * 2e-6f) : 0.f;
+  const float sums = S > 1 ? (float)S * (HGEMM_SLICE_US + outputs * HGEMM_SUM_US) : 0.f;
   if (T <= 64) {
     const HFew& f = HGEMM_FEW[shape];
     return f.start * (0.75f + 0.25f * (float)rounds) + (float)(most * per) * f.superblock[type == TL_Q4_K ? 0 : type == TL_Q6_K ? 1 : type == TL_Q8_0 ? 2 : 3] + sums;
   }
   if (type == TL_Q6_K || type == TL_Q8_0) {
-    const float us = type == TL_Q6_K ? (shape == 2 ? 6.3f : 6.85f) : (shape == 2 ? 5.5f : 6.0f), alone = q.percu == 2 ? 0.6f : 1.f;
+    const float us = (type == TL_Q6_K ? HGEMM_US_Q6_K : HGEMM_US_Q8_0)[shape], alone = q.percu == 2 ? 0.6f : 1.f;
     const float fullest = q.percu == 2 ? (float)(most / 2) + (most & 1 ? alone : 0.f) : (float)most;
     const float even = (float)n / (float)cus / (float)q.percu;
-    return (0.84f * fullest + 0.16f * (even > alone ? even : alone)) * ((float)per + 0.6f) * us + (S > 1 ? (float)S * (0.3f + outputs * 1.4e-6f) : 0.f);
+    return (0.84f * fullest + 0.16f * (even > alone ? even : alone)) * ((float)per + HGEMM_ENDS) * us + (S > 1 ? (float)S * (HGEMM_SLICE_US + outputs * 1.4e-6f) : 0.f);
   }
   return (float)rounds * (float)(per + 1) * (shape == 3 && !q.lds ? HGEMM_US_3_Q8_K : HGEMM_US[shape]) + sums;
 }
@@ -1120,12 +1124,19 @@ HgemmPlan hgemm_plan(const QW* w, int n, int T, float* sum = nullptr) {
 }
 
 // Price of one launch over both (HPair), as hgemm_price for its workgroups: their super-blocks one after another on the CU that has most of
-// them, the longer workgroups dealt first
-float hgemm_pair_price(int cus, int v6, int v4, int T, long n6, int per6, int S6, long n4, int per4, int S4, float outputs6, float outputs4) {
+// them, the longer workgroups dealt first. A launch takes no less than an even share of all super-blocks and its partial sums: where that is
+// more than `most_price` it is the answer (a plan weighs some 36 pairs of slices a shape, in front of a prompt's first launches: a host's time
+// for a plan of 4096 columns with 8 / 64 / 2000 tokens 1.5 / 2.4 / 2.5 us without, 1.5 / 1.8 / 1.2 with; of 8192 2.5 / 4.6 / 6.6 and 1.7 / 2.3 / 1.5)
+float hgemm_pair_price(int cus, int v6, int v4, int T, long n6, int per6, int S6, long n4, int per4, int S4, float outputs6, float outputs4,
+                       float most_price) {
   const bool few = v4 != 2 && v4 != 3;
   const HFew& f = HGEMM_FEW[v4];
-  const float t6 = few || T <= 64 ? (float)per6 * f.superblock[1] : ((float)per6 + 0.6f) * 6.3f;
+  const float t6 = few || T <= 64 ? (float)per6 * f.superblock[1] : ((float)per6 + HGEMM_ENDS) * HGEMM_US_Q6_K[v6];
   const float t4 = few || T <= 64 ? (float)per4 * f.superblock[0] : (float)(per4 + 1) * HGEMM_US[v4];
+  const int S = S6 > S4 ? S6 : S4;
+  const float sums = (S > 1 ? HGEMM_SLICE_US * (float)S : 0.f) + HGEMM_SUM_US * ((S6 > 1 ? (float)S6 * outputs6 : 0.f) + (S4 > 1 ? (float)S4 * outputs4 : 0.f));
+  const float even = 0.999f * ((float)n6 * t6 + (float)n4 * t4) / (float)cus + sums + (few || T <= 64 ? f.start : 0.f);  // (0.999: roundings of the loads below)
+  if (even > most_price) return even;
   // the CUs' loads: `more` of them at `high`, the others at `low`
   const bool six = t6 >= t4;
   const float tb = six ? t6 : t4, ts = six ? t4 : t6;
@@ -1147,8 +1158,6 @@ float hgemm_pair_price(int cus, int v6, int v4, int T, long n6, int per6, int S6
     }
     top = at > top ? at : top;
   }
-  const int S = S6 > S4 ? S6 : S4;
-  const float sums = (S > 1 ? 0.3f * (float)S : 0.f) + 2e-6f * ((S6 > 1 ? (float)S6 * outputs6 : 0.f) + (S4 > 1 ? (float)S4 * outputs4 : 0.f));
   if (!few && T > 64) return top + sums;
   const long most = (n6 + n4 + cus - 1) / cus, percu = hgemm_shape(TL_Q4_K, v4).percu, rounds = (most + percu - 1) / percu;
   return f.start * (0.75f + 0.25f * (float)rounds) + top + sums;
@@ -1243,7 +1252,12 @@ bool tl_hgemm_pair_plan(const QW* w4, int n4, const QW& w6, int T, int most_slic
   const float out4 = (float)T * (float)rows4, out6 = (float)T * (float)w6.rows;
   const unsigned few = T <= 8 ? 1u << 5 | 1u << 6 : T <= 16 ? 1u << 0 | 1u << 7 : 1u << 1 | 1u << 8, many = 1u << 2;
   const unsigned shapes = T <= 32 ? few : T <= 64 ? few | many : many | 1u << 3;
-  float least = -1.f;
+  // (two launches: each at its own best. The prices of long chunks are right to a few per cent)
+  float apart = 0.f;
+  *p4 = hgemm_plan(w4, n4, T, &apart);
+  *p6 = hgemm_plan(&w6, 1, T, &apart);
+  float least = (T > 64 ? 0.96f : 1.f) * apart;
+  bool joint = false;
   for (int v = 0; v < HGEMM_SHAPES; ++v) {
     if (!(shapes >> v & 1)) continue;
     const int v6 = v == 3 ? 2 : v;
@@ -1258,22 +1272,17 @@ bool tl_hgemm_pair_plan(const QW* w4, int n4, const QW& w6, int T, int most_slic
       for (int b = 1; b <= 8 && b <= slices; ++b) {
         const int per6 = (nsb + b - 1) / b;
         if ((nsb + per6 - 1) / per6 != b) continue;
-        const float price = hgemm_pair_price(cus, v6, v, T, t6 * b, per6, b, t4 * a, per4, a, out6, out4);
-        if (least < 0.f || price < least) {
+        const float price = hgemm_pair_price(cus, v6, v, T, t6 * b, per6, b, t4 * a, per4, a, out6, out4, least);
+        if (price < least) {
           least = price;
+          joint = true;
           *p4 = {v, a};
           *p6 = {v6, b};
         }
       }
     }
   }
-  // (two launches: each at its own best)
-  float apart = 0.f;
-  const HgemmPlan s4 = hgemm_plan(w4, n4, T, &apart), s6 = hgemm_plan(&w6, 1, T, &apart);
-  if (least <= (T > 64 ? 0.96f : 1.f) * apart) return true;  // (the prices of long chunks are right to a few per cent)
-  *p4 = s4;
-  *p6 = s6;
-  return false;
+  return joint;
 }
 int tl_launch_hgemm_pair(const QW* w4, int n4, const QW& w6, const void* planes, size_t ps, float* const* out4, float* out6, int T,
                          const HgemmPlan& p4, const HgemmPlan& p6, hipStream_t s) {
