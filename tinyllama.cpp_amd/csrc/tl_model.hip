@@ -1365,7 +1365,10 @@ static void half_part_floats(const tl_model* m, int most, size_t (&cap)[3]) {
     }
     add(L, {TL_T_FFN_DOWN}, 0);
   }
-  // between these numbers of tokens a plan's tiles stay and only the price of its partial sums rises: S is largest at the first
+  // Between these numbers of tokens a plan's tiles stay and only the price of its partial sums rises: S is largest at the first. That is not
+  // sure of the plans of two formats, whose slices are chosen together and against two launches (2048 columns, q 2048 rows, k and v 256: shared at
+  // 21 numbers of tokens whose range's first is not). What they leave there has room in ensure_prefill_ws's own floor for the 1B, 3B, 8B
+  // and 70B shapes; where it had none, the matrices would go out one by one with the same slices and sums.
   for (const Group& g : groups)
     for (int T = 1, end; T <= most; T = end + 1) {
       end = std::min(T == 1 ? 8 : T == 9 ? 16 : T == 17 ? 32 : T + 63 - (T - 1) % 64, most);
