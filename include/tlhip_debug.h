@@ -51,6 +51,8 @@ int tl_debug_half_attention_launches(long long* count_out);
 int tl_debug_gemv_general_norms(long long* count_out);
 /* ... and f16 products of Q4_K and Q6_K matrices in one launch, counts_out[9] by the Q4_K tiles' workgroup shape (tl_debug_half_gemm) */
 int tl_debug_half_pair_launches(long long* counts_out);
+/* ... and one-token products of a layer list that carry the residual norm in front of them (graph captures count once) */
+int tl_debug_resid_products(long long* count_out);
 
 /* Test hook (no counterpart in the reference): tl_matmul_q through the f16 form that a model's chunks and multi-sequence steps
  * take (tl_hgemm.hip), any number of tokens, in a workgroup shape (0: 64 rows x 16 tokens, 1: 128 x 32, 2: 256 x 64, 3: in waves of 64

@@ -4,6 +4,7 @@ Every test builds its own small configuration and random weights (synth.build_st
 (operators, engine, decode graph) and, for generation, the C++ host (Session over a checkpoint folder). Exact mode
 (three-term chunk GEMMs, FP32 GEMVs) is compared at FP32 tolerances; the bf16-activation mode at bf16 tolerances, and its
 GEMM operator exactly against a product with bf16-rounded activations."""
+import ctypes
 import os
 
 import numpy as np
@@ -655,9 +656,9 @@ def test_projections_and_router_rows_of_every_length(env, heads, dim, width):
 
 @pytest.mark.parametrize("width,heads,n_layers", [(1024, 5, 1), (1024, 16, 2), (2048, 9, 3), (4096, 40, 4), (1536, 4, 3)])
 def test_residual_sum_in_front_of_the_next_product(env, width, heads, n_layers):
-    """One token's residual norm carried by the next layer's product, at every width that takes it and one that does not: none to three
-    moves of the residual row (a layer without feed-forward among them), few rows and more rows than waves, single tokens from the captured
-    step and as a portion of one, both against the float64 oracle and against the launches of their own."""
+    """One token's residual norm carried by the next layer's product: none to three moves of the residual row (a layer without feed-forward
+    among them), few rows and more rows than waves, single tokens from the captured step and as a portion of one, both against the float64 oracle
+    and against the launches of their own."""
     S = env["synth"]
     L = S.stack_layer
     layers = [L(heads, 1, 64, 32, 50, v_mix=True, experts=4, top=2, ff=64, shared_ff=32, mlp=l != 1) for l in range(n_layers)]
@@ -671,6 +672,29 @@ def test_residual_sum_in_front_of_the_next_product(env, width, heads, n_layers):
         assert rel_rms(got[-1], orc.forward(list(toks))) < FP32_TOL
         m.free()
     assert rel_rms(got[0], got[1]) < FP32_TOL
+
+
+@pytest.mark.parametrize("width,carried", [(512, 1), (520, 0), (1536, 1), (2560, 1), (3072, 1), (3584, 1), (4608, 1), (5120, 1), (5632, 0)])
+def test_widths_whose_residual_sum_rides_in_the_next_product(env, width, carried):
+    """Every width of one to ten whole 512-column pieces takes the product that carries the residual norm, others do not (the launches are
+    counted): single tokens against the float64 oracle."""
+    S, capi = env["synth"], env["capi"]
+    layers = [S.stack_layer(6, 1, 64, 32, 50, v_mix=True, experts=4, top=2, ff=64, shared_ff=32) for _ in range(2)]
+    cfg = S.stack_config(width, 211, layers)
+    toks = np.random.default_rng(width).integers(0, cfg["vocab"], 12).astype(np.int32)
+    count = ctypes.c_longlong()
+
+    def carried_products():
+        capi.check(capi.lib().tl_debug_resid_products(ctypes.byref(count)))
+        return count.value
+
+    before = carried_products()
+    m, _, orc = make(env, cfg, seed=11, max_pos=32)  # (the step may be captured here)
+    m.prefill_rows(toks[:4], 0, np.array([3], np.int32))
+    got = np.stack([m.decode(int(toks[i]), i)[0] for i in range(4, 12)])
+    assert (carried_products() > before) == bool(carried)
+    assert rel_rms(got, orc.forward(list(toks))[4:]) < FP32_TOL
+    m.free()
 
 
 @pytest.mark.parametrize("experts", [1, 2, 15, 16, 17, 33, 64, 65, 130])

@@ -198,6 +198,7 @@ DEBUG_SIGNATURES = {
     "tl_debug_half_attention_launches": [C.POINTER(C.c_longlong)],
     "tl_debug_gemv_general_norms": [C.POINTER(C.c_longlong)],
     "tl_debug_half_pair_launches": [C.POINTER(C.c_longlong)],
+    "tl_debug_resid_products": [C.POINTER(C.c_longlong)],
     "tl_debug_half_gemm": [_vp, _fp, _fp, C.c_int, C.c_int, C.c_int, _vp],
     "tl_debug_dense_plane": [_vp, C.c_int, C.c_int, _fp, C.c_int, _fp, C.c_int, C.c_int, C.c_int, _vp, _vp],
     "tl_debug_dense_plane_taken": [C.c_int, C.c_int, C.c_int, C.c_longlong, C.c_int],

@@ -24,6 +24,8 @@
 #include <math.h>
 #include <stdlib.h>
 
+#include <atomic>
+
 #include "tl_bf16.h"
 #include "tl_lds.h"
 #include "tl_stack.h"
@@ -416,7 +418,11 @@ __global__ __launch_bounds__(256) void dense_gemv_kernel(const unsigned short* _
 
 // One token: x_out = x + y / rms(y) * (1 + norm_w) in every workgroup (one of them writes it), out = W x_out, columns 512 NP. A row a wave
 // (more where a launch has more rows than waves), its NP 16-byte pieces asked for with the vectors. A residual norm of its own is a launch of
-// one workgroup that the product waits for: 3072 x 2048 4.9 + 4.4 us, here 4.8.
+// one workgroup that the product waits for: 3072 x 2048 4.9 + 4.4 us, here 4.8. A token of six layers, us, with launches of their own / carried:
+// 512 columns 201 / 193, 1024 216 / 203, 1536 249 / 241, 2048 268 / 255, 2560 317 / 302, 3072 328 / 319, 3584 388 / 372, 4096 413 / 394, 4608 495 /
+// 468, 5120 533 / 502. Ten pieces are 124 of the 128 registers that a thread of sixteen waves has, eleven spill: wider rows keep the two
+// launches, and so do rows that end inside a piece (the kernel has no tail).
+constexpr int RESID_PIECES = 10;
 template <int NP>
 __global__ __launch_bounds__(1024) void dense_gemv_resid_kernel(const unsigned short* __restrict__ W, const float* __restrict__ x, const float* __restrict__ y,
                                                                 const float* __restrict__ nw, float* __restrict__ x_out, float* __restrict__ out,
@@ -598,8 +604,17 @@ int tl_launch_dense_gemv_heads(const uint16_t* w, int groups, int rows, int cols
   return launch_gemv(w, groups, rows, cols, x, x_stride, y, y_stride, 0.0f, GemvActArgs{}, s);
 }
 
+namespace {
+std::atomic<long long> g_resid_products{0};  // tl_debug_resid_products
+template <int NP = RESID_PIECES>
+void gemv_resid_go(const uint16_t* w, int rows, int cols, const float* x, const float* y, const float* norm_w, float eps, float* x_out, float* out, int grid,
+                   int waves, hipStream_t s) {
+  if (cols == 512 * NP) dense_gemv_resid_kernel<NP><<<grid, 64 * waves, 0, s>>>(w, x, y, norm_w, x_out, out, rows, eps, 64 * waves, grid);
+  else if constexpr (NP > 1) gemv_resid_go<NP - 1>(w, rows, cols, x, y, norm_w, eps, x_out, out, grid, waves, s);
+}
+}  // namespace
 bool tl_dense_gemv_resid_fits(const uint16_t* w, int rows, int cols) {
-  return rows > 0 && (cols == 1024 || cols == 2048 || cols == 4096) && ((size_t)w & 15) == 0;
+  return rows > 0 && cols > 0 && cols % 512 == 0 && cols <= 512 * RESID_PIECES && ((size_t)w & 15) == 0;
 }
 int tl_launch_dense_gemv_resid(const uint16_t* w, int rows, int cols, const float* x, const float* y, const float* norm_w, float eps, float* x_out,
                                float* out, hipStream_t s) {
@@ -611,11 +626,14 @@ int tl_launch_dense_gemv_resid(const uint16_t* w, int rows, int cols, const floa
   waves = waves < least ? least : waves > 16 ? 16 : waves;
   int grid = (rows + waves - 1) / waves;
   if (grid > cus) grid = cus;
-  const int nthr = 64 * waves;
-  if (cols == 1024) dense_gemv_resid_kernel<2><<<grid, nthr, 0, s>>>(w, x, y, norm_w, x_out, out, rows, eps, nthr, grid);
-  else if (cols == 2048) dense_gemv_resid_kernel<4><<<grid, nthr, 0, s>>>(w, x, y, norm_w, x_out, out, rows, eps, nthr, grid);
-  else dense_gemv_resid_kernel<8><<<grid, nthr, 0, s>>>(w, x, y, norm_w, x_out, out, rows, eps, nthr, grid);
+  gemv_resid_go(w, rows, cols, x, y, norm_w, eps, x_out, out, grid, waves, s);
   TL_HIP(hipGetLastError());
+  g_resid_products.fetch_add(1, std::memory_order_relaxed);
+  return 0;
+}
+extern "C" int tl_debug_resid_products(long long* count_out) {
+  TL_REQUIRE(count_out, "tl_debug_resid_products: null argument");
+  *count_out = g_resid_products.load(std::memory_order_relaxed);
   return 0;
 }
 
